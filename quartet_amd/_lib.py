@@ -7,6 +7,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libquartet_hip.so")
+HOST_PATH = os.path.join(_HERE, "_quartet_host.so")
 
 QM_BF16, QM_F32 = 0, 1
 QM_QUEST_RTN, QM_ABSMAX_RTN, QM_ABSMAX_SR, QM_QUEST_SR = 0, 1, 2, 3
@@ -129,6 +130,29 @@ def lib():
     L.qm_linear_backward_seeded.argtypes = L.qm_linear_backward.argtypes[:-1] + [vp, vp]
     _lib = L
     return L
+
+
+_host = None
+
+
+def host():
+    """The native host side of the layers (csrc/host_ext.cpp): autograd functions over the same C ABI."""
+    global _host
+    if _host is None:
+        if not os.path.exists(HOST_PATH):
+            raise QuartetHipError(f"{HOST_PATH} is missing: build it with `make -C quartet_amd/csrc` (or __graft_entry__.build())")
+        lib()
+        import importlib.util
+
+        import torch  # noqa: F401  (its libraries must be loaded before the extension's)
+
+        from .linear import _gradient_draws
+        spec = importlib.util.spec_from_file_location("_quartet_host", HOST_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        module.bind(QuartetHipError, _gradient_draws)
+        _host = module
+    return _host
 
 
 def check(rc, what):

@@ -14,6 +14,7 @@ import weakref
 
 import torch
 
+from .. import _lib
 from .. import kernels as K
 from .base import BaseQuantizer
 
@@ -161,10 +162,8 @@ class _HadamardQuantizer(BaseQuantizer):
     def re_randomize(self):
         if self.rerotate == "signs":
             # H <- H @ diag(+-1) (mxfp4.py:53-60): flips accumulate, so they xor into the mask
-            flips = torch.randint(0, 2, (self.hadamard_dim,))
-            for j, f in enumerate(flips.tolist()):
-                if f == 0:  # randint*2-1 == -1
-                    self.sign_bits ^= 1 << j
+            # column j flips where torch.randint(0, 2, (hd,)) draws 0: randint*2-1 == -1
+            self.sign_bits ^= _lib.host().sign_flips(self.hadamard_dim)
         elif self.rerotate == "O32":
             # H <- U V^T of the SVD of a Gaussian matrix (mxfp4.py:61-64): Haar-distributed up to signs
             u, _, vh = torch.linalg.svd(torch.randn(self.hadamard_dim, self.hadamard_dim))
@@ -222,58 +221,19 @@ class DenseRotationQuantizerFn(torch.autograd.Function):
         return out.view(ctx.x_shape).to(ctx.x_dtype), None, None, None, None
 
 
-class QuestMXFP4QuantizerFn(torch.autograd.Function):
-    """mxfp4.py:127-146: quest-scaled RTN forward with clip mask, masked straight-through backward."""
-
-    @staticmethod
-    def forward(ctx, x, hadamard_dim, sign_bits):
-        x2 = _as_2d(x, hadamard_dim)
-        _, _, maskbits, deq = K.quantize_mxfp4(x2, hadamard_dim, sign_bits, K.QM_QUEST_RTN, want_mask=True,
-                                               want_dequant=True)
-        ctx.save_for_backward(maskbits)
-        ctx.hd, ctx.sign_bits, ctx.x_shape, ctx.x_dtype = hadamard_dim, sign_bits, x.shape, x.dtype
-        return deq.view(x.shape)
-
-    @staticmethod
-    def backward(ctx, grad_output):
-        (maskbits,) = ctx.saved_tensors
-        g = grad_output.contiguous().view(maskbits.shape[0], -1)
-        # under bf16 autocast the reference's `g @ H.T` runs with H cast to bf16 and a bf16 result
-        low = _autocast_bf16() or g.dtype == torch.bfloat16
-        sd = torch.bfloat16 if low else ctx.x_dtype
-        out = K.masked_hadamard_bwd(g, ctx.hd, sd, ctx.sign_bits, maskbits, torch.bfloat16 if low else g.dtype)
-        return out.view(ctx.x_shape).to(ctx.x_dtype), None, None
-
-
 class QuestMXFP4Quantizer(_HadamardQuantizer):
     def forward(self, x):
         self._note_input(x)
         if self.is_dense:
             return DenseRotationQuantizerFn.apply(x, self.hadamard_matrix, K.QM_QUEST_RTN, True, 1.0)
-        return QuestMXFP4QuantizerFn.apply(x, self.hadamard_dim, self.sign_bits)
+        # quest-scaled RTN forward with clip mask, masked straight-through backward (mxfp4.py:127-146)
+        return _lib.host().quantizer(x, self.hadamard_dim, self.sign_bits, K.QM_QUEST_RTN, 0, 1.0)
 
 
-class AlbertTsengQuantizerFn(torch.autograd.Function):
+def _absmax_quantize(x, hadamard_dim, sign_bits, stochastic, post_scale):
     """mxfp4.py:15-34: absmax/(3/4)-scaled RTN or SR forward, unmasked straight-through backward."""
-
-    @staticmethod
-    def forward(ctx, x, hadamard_dim, sign_bits, stochastic_round, post_scale):
-        x2 = _as_2d(x, hadamard_dim)
-        mode = K.QM_ABSMAX_SR if stochastic_round else K.QM_ABSMAX_RTN
-        _, _, _, deq = K.quantize_mxfp4(x2, hadamard_dim, sign_bits, mode,
-                                        seed=_fresh_seed() if stochastic_round else 0, want_dequant=True)
-        if post_scale != 1.0:
-            deq *= post_scale
-        ctx.hd, ctx.sign_bits, ctx.x_shape, ctx.x_dtype = hadamard_dim, sign_bits, x.shape, x.dtype
-        return deq.view(x.shape)
-
-    @staticmethod
-    def backward(ctx, grad_output):
-        g = grad_output.contiguous().view(-1, ctx.x_shape[-1] if ctx.x_shape[-1] % ctx.hd == 0 else ctx.hd)
-        low = _autocast_bf16() or g.dtype == torch.bfloat16
-        sd = torch.bfloat16 if low else ctx.x_dtype
-        out = K.masked_hadamard_bwd(g, ctx.hd, sd, ctx.sign_bits, None, torch.bfloat16 if low else g.dtype)
-        return out.view(ctx.x_shape).to(ctx.x_dtype), None, None, None, None
+    mode, seed = (K.QM_ABSMAX_SR, _fresh_seed()) if stochastic else (K.QM_ABSMAX_RTN, 0)
+    return _lib.host().quantizer(x, hadamard_dim, sign_bits, mode, seed, post_scale)
 
 
 class AlbertTsengQuantizer(_HadamardQuantizer):
@@ -286,7 +246,7 @@ class AlbertTsengQuantizer(_HadamardQuantizer):
         if self.is_dense:
             mode = K.QM_ABSMAX_SR if self.stochastic else K.QM_ABSMAX_RTN
             return DenseRotationQuantizerFn.apply(x, self.hadamard_matrix, mode, False, 1.0)
-        return AlbertTsengQuantizerFn.apply(x, self.hadamard_dim, self.sign_bits, self.stochastic, 1.0)
+        return _absmax_quantize(x, self.hadamard_dim, self.sign_bits, self.stochastic, 1.0)
 
 
 class AlignedAlbertTsengQuantizer(_HadamardQuantizer):
@@ -296,4 +256,4 @@ class AlignedAlbertTsengQuantizer(_HadamardQuantizer):
         self._note_input(x)
         if self.is_dense:
             return DenseRotationQuantizerFn.apply(x, self.hadamard_matrix, K.QM_ABSMAX_RTN, False, 1.009276)
-        return AlbertTsengQuantizerFn.apply(x, self.hadamard_dim, self.sign_bits, False, 1.009276)
+        return _absmax_quantize(x, self.hadamard_dim, self.sign_bits, False, 1.009276)
