@@ -36,8 +36,10 @@ enum { QM_BF16 = 0, QM_F32 = 1 };
  * (AlbertTsengQuantizer); RTN = ties toward zero, SR = stochastic rounding */
 enum { QM_QUEST_RTN = 0, QM_ABSMAX_RTN = 1, QM_ABSMAX_SR = 2, QM_QUEST_SR = 3 };
 
-/* layout of a packed tensor's code bytes (see above); producers and consumers must agree per tensor */
-enum { QM_LAYOUT_ROWMAJOR = 0, QM_LAYOUT_TILED = 1 };
+/* layout of a packed tensor's code bytes (see above); producers and consumers must agree per tensor.  QM_LAYOUT_PADDED, taken by
+ * the whole-layer entry points and the fused producers: QM_LAYOUT_TILED for any extents -- rows padded to 16 and columns to
+ * 128 in the code and scale arrays of a packed operand buffer, the padding columns zero codes and zero scale bytes. */
+enum { QM_LAYOUT_ROWMAJOR = 0, QM_LAYOUT_TILED = 1, QM_LAYOUT_PADDED = 2 };
 /* qm_linear_forward: which packed operand buffers already hold their operand on entry */
 enum { QM_W_IS_PACKED = 1, QM_X_IS_PACKED = 2 };
 /* rotated_flags of qm_linear_backward */
@@ -233,8 +235,8 @@ int qm_dequantize_mxfp4(const uint8_t* codes, const uint8_t* scales, int64_t R, 
  * per-kernel entry points above, in order), so the host pays one foreign call instead of three / eight.
  *
  * A packed operand is one caller-owned, 256-byte aligned buffer of qm_packed_operand_bytes(rows, cols) bytes holding,
- * at the offsets qm_packed_operand_offsets reports, the codes [rows, cols/2], E8M0 scales [rows, cols/32] and
- * clip-mask bits [rows, cols/8] of a quantized [rows, cols] tensor -- the three tensors per operand that
+ * at the offsets qm_packed_operand_offsets reports, the codes [rows, cols/2], E8M0 scales [rows, cols/32] (in the padded
+ * layout: of the padded extents) and clip-mask bits [rows, cols/8] of a quantized [rows, cols] tensor -- the three tensors per operand that
  * notebooks/benchmark_mxfp4.ipynb's CudaGemm keeps for backward (ctx.save_for_backward in its forward).
  *
  * qm_linear_forward = QuestMXFP4QuantizerFn.forward on x and W (quantizers/mxfp4.py:129-140) followed by
@@ -262,13 +264,14 @@ int qm_dequantize_mxfp4(const uint8_t* codes, const uint8_t* scales, int64_t R, 
  *                     next kernel (maskbits argument of qm_rmsnorm_backward / qm_swiglu_backward) or, for a forward
  *                     quantizer that holds a dense rotation, applies mask and transposed matrix itself; needs hd_x == 32.
  *                     QM_GW_ROTATED: the same for gw and the weight quantizer (second product, B6; gw_dtype == mid_dtype)
- * codes_layout applies to every packed tensor inside; QM_LAYOUT_TILED needs T, I, O multiples of 128 and at
- * least 256, and all Hadamard blocks 32.  T, I, O must be multiples of 32 for the backward pass.
- * Where a gradient product runs as qm_gemm_fuses_rotation describes (bf16 mid_dtype, Hadamard block 32, for gw also
- * gw_dtype == mid_dtype), the forward quantizer's masked inverse rotation is applied in that product's epilogue
- * (qm_gemm_mxfp4_tn_rotated) and the product is not staged in the workspace.  Where a gradient product is cut into K
- * ranges (Hadamard block 32, any mid_dtype / gw_dtype), the rotation is applied by the ordered reduction of the ranges,
- * with the arithmetic and roundings of the separate launches.  Elsewhere it is a launch of its own.
+ * codes_layout applies to every packed tensor inside; QM_LAYOUT_TILED needs T, I, O multiples of 128 (forward: T and O
+ * multiples of 16, I of 128), QM_LAYOUT_PADDED takes any; both need O % 8 == 0.  T, I, O must be multiples of 32, and of the
+ * Hadamard blocks along them, for the backward pass.
+ * The forward quantizer's masked inverse rotation is applied by the gradient product that feeds it where the kernel serving
+ * the shape can: in the epilogue of the 256 x 256 kernel (bf16 mid_dtype, Hadamard block 32, for gw also gw_dtype ==
+ * mid_dtype; see qm_gemm_mxfp4_tn_rotated), in the epilogue of the smaller tile kernels (bf16 mid_dtype, any Hadamard block,
+ * any gw_dtype), or in the ordered reduction of a product cut into K ranges (Hadamard block 32, any mid_dtype / gw_dtype);
+ * the last two with the arithmetic and roundings of the separate launches.  Elsewhere it is a launch of its own.
  */
 size_t qm_packed_operand_bytes(int64_t rows, int64_t cols);
 /* offsets: HOST array of three (codes, scales, mask bits); returns 0, or QM_ERR_INVALID unless cols % 32 == 0 */
@@ -326,7 +329,8 @@ int qm_linear_backward_seeded(const void* e, int e_dtype, int64_t T, int64_t I, 
  *   layer's activation quantizer (qm_linear_backward with QM_GX_ROTATED): then maskbits [rows, cols/8] (the mask region of
  *   the layer's packed_x; 4-byte aligned for qm_rmsnorm_backward), sign_bits and scale_dtype describe that quantizer, and the masked inverse rotation of
  *   qm_masked_hadamard_bwd (same operations, same bits, rounded to the gradient's dtype) is applied on the fly.
- * codes_layout QM_LAYOUT_TILED needs rows % 16 == 0 and cols (hidden) % 128 == 0; cols (hidden) % 32 == 0 always.
+ * codes_layout QM_LAYOUT_TILED needs rows % 16 == 0 and cols (hidden) % 128 == 0, QM_LAYOUT_PADDED takes any; cols (hidden)
+ * % 32 == 0 always.
  */
 int qm_rmsnorm_quantize_mxfp4(const void* x, int x_dtype, const void* add, int add_dtype, void* x_sum,
                               const float* gain, float eps, int64_t rows, int64_t cols, const uint32_t* sign_bits,

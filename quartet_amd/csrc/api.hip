@@ -8,6 +8,7 @@
 
 #include "../../include/quartet_hip.h"
 #include "qm_kernels.h"
+#include "qm_math.h"
 
 namespace {
 
@@ -32,6 +33,7 @@ bool valid_hd(int hd) { return hd == 32 || hd == 64 || hd == 128; }
 bool valid_dtype(int d) { return d == QM_BF16 || d == QM_F32; }
 bool valid_mode(int m) { return m >= QM_QUEST_RTN && m <= QM_QUEST_SR; }
 bool valid_layout(int l) { return l == QM_LAYOUT_ROWMAJOR || l == QM_LAYOUT_TILED; }
+bool valid_layer_layout(int l) { return valid_layout(l) || l == QM_LAYOUT_PADDED; }
 
 qm::SignBits make_signs(const uint32_t* sign_bits, int hd) {
     qm::SignBits sb{{0u, 0u, 0u, 0u}};
@@ -297,7 +299,7 @@ int qm_gemm_fuses_rotation(const uint8_t* a_scales, const uint8_t* b_scales, int
     if (M <= 0 || N <= 0 || K <= 0 || K % 32) return 0;
     // offered the workspace the plain product would use: a shape it would cut into K ranges is not served
     const size_t ws = qm::gemm_workspace_bytes(M, N, K);
-    return ws == 0 && qm::gemm_will_rotate(a_scales, b_scales, M, N, K, QM_BF16, QM_BF16, nullptr, 0) ? 1 : 0;
+    return ws == 0 && qm::gemm_persistent_rotates(a_scales, b_scales, M, N, K) ? 1 : 0;
 }
 
 int qm_gemm_mxfp4_tn_rotated(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes, const uint8_t* b_scales,
@@ -315,12 +317,11 @@ int qm_gemm_mxfp4_tn_rotated(const uint8_t* a_codes, const uint8_t* a_scales, co
                     (long long)M, (long long)N, (long long)K);
     if (!aligned(a_codes, 16) || !aligned(b_codes, 16) || !aligned(a_scales, 4) || !aligned(b_scales, 4) || !aligned(c, 16) || !aligned(maskbits, 4))
         return fail(QM_ERR_UNALIGNED, "qm_gemm_mxfp4_tn_rotated: codes and c need 16-byte, scales and mask bits 4-byte alignment");
-    bool rotated = false;
-    const int rc = from_hip(qm::gemm_mxfp4_tn_rotated(a_codes, a_scales, b_codes, b_scales, M, N, K, alpha, c, QM_BF16, a_layout, b_layout,
-                                                      nullptr, 0, maskbits, sign_bits ? sign_bits[0] : 0u, scale_dtype, QM_BF16, &rotated,
-                                                      reinterpret_cast<hipStream_t>(stream)), "qm_gemm_mxfp4_tn_rotated");
-    if (rc) return rc;
-    return rotated ? 0 : fail(QM_ERR_INVALID, "qm_gemm_mxfp4_tn_rotated: the product did not run as planned");
+    qm::TileProduct p = qm::make_product(a_codes, a_scales, b_codes, b_scales, M, N, K, alpha, c, a_layout, b_layout);
+    p.mask = maskbits;
+    p.signs = make_signs(sign_bits, 32);
+    p.rot_c = qm::hadamard_scale(32, scale_dtype);
+    return from_hip(qm::gemm_persistent_rotated(p, reinterpret_cast<hipStream_t>(stream)), "qm_gemm_mxfp4_tn_rotated");
 }
 
 int qm_dequantize_mxfp4(const uint8_t* codes, const uint8_t* scales, int64_t R, int64_t C, float post, void* out,
@@ -341,15 +342,18 @@ namespace {
 size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
 size_t esize(int dtype) { return dtype == QM_BF16 ? 2 : 4; }
 
-// one packed operand: codes, scales, mask bits, each region 256-byte aligned
+// one packed operand: codes, scales, mask bits, each region 256-byte aligned.  The code and scale regions hold the tiled
+// layout with its rows padded to 16 and its columns to 128; a row-major operand occupies the front of each region.
+size_t code_bytes(int64_t rows, int64_t cols) { return up256((size_t)qm::padded_rows(rows) * qm::padded_cols(cols) / 2); }
+size_t scale_bytes(int64_t rows, int64_t cols) { return up256((size_t)qm::padded_rows(rows) * qm::padded_cols(cols) / 32); }
 struct PackedLayout {
     size_t c, s, m, total;
 };
 PackedLayout packed_layout(int64_t rows, int64_t cols) {
     PackedLayout l;
     size_t o = 0;
-    l.c = o; o += up256((size_t)rows * cols / 2);
-    l.s = o; o += up256((size_t)rows * cols / 32);
+    l.c = o; o += code_bytes(rows, cols);
+    l.s = o; o += scale_bytes(rows, cols);
     l.m = o; o += up256((size_t)rows * cols / 8);
     l.total = o;
     return l;
@@ -360,26 +364,32 @@ struct WorkLayout {
 WorkLayout work_layout(int64_t T, int64_t I, int64_t O, int mid_dtype) {
     WorkLayout l;
     size_t o = 0;
-    l.ec = o; o += up256((size_t)T * O / 2);
-    l.es = o; o += up256((size_t)T * O / 32);
-    l.wtc = o; o += up256((size_t)I * O / 2);
-    l.wts = o; o += up256((size_t)I * O / 32);
+    l.ec = o; o += code_bytes(T, O);
+    l.es = o; o += scale_bytes(T, O);
+    l.wtc = o; o += code_bytes(I, O);
+    l.wts = o; o += scale_bytes(I, O);
     l.gxq = o; o += up256((size_t)T * I * esize(mid_dtype));
-    l.etc = o; o += up256((size_t)O * T / 2);
-    l.ets = o; o += up256((size_t)O * T / 32);
-    l.xtc = o; o += up256((size_t)I * T / 2);
-    l.xts = o; o += up256((size_t)I * T / 32);
+    l.etc = o; o += code_bytes(O, T);
+    l.ets = o; o += scale_bytes(O, T);
+    l.xtc = o; o += code_bytes(I, T);
+    l.xts = o; o += scale_bytes(I, T);
     l.gwq = o; o += up256((size_t)O * I * esize(mid_dtype));
-    const size_t g1 = qm::gemm_workspace_bytes(T, I, O), g2 = qm::gemm_workspace_bytes(O, I, T);
-    l.gemm_ws_bytes = g1 > g2 ? g1 : g2;  // split-K scratch, shared by the two products (they run one after the other)
+    // split-K scratch, shared by the two products (they run one after the other), for either layout's contraction length
+    const int64_t Op = qm::padded_cols(O), Tp = qm::padded_cols(T);
+    const size_t need[] = {qm::gemm_workspace_bytes(T, I, O), qm::gemm_workspace_bytes(O, I, T), qm::gemm_workspace_bytes(T, I, Op),
+                           qm::gemm_workspace_bytes(O, I, Tp)};
+    l.gemm_ws_bytes = 0;
+    for (size_t n : need) l.gemm_ws_bytes = n > l.gemm_ws_bytes ? n : l.gemm_ws_bytes;
     l.gemm_ws = o; o += up256(l.gemm_ws_bytes);
     l.total = o;
     return l;
 }
-// The whole-layer calls issue independent launches two to a grid when all of them run on the Hadamard-32 kernels with
-// tiled codes (which needs every extent to be a multiple of 128).
-bool pair_launches(int codes_layout, int64_t T, int64_t I, int64_t O, int hd_a, int hd_b, int hd_c) {
-    return codes_layout == QM_LAYOUT_TILED && hd_a == 32 && hd_b == 32 && hd_c == 32 && T % 128 == 0 && I % 128 == 0 &&
+bool tiled_layout(int codes_layout) { return codes_layout != QM_LAYOUT_ROWMAJOR; }
+// the layout the kernels of a single operation are told
+int kernel_layout(int codes_layout) { return tiled_layout(codes_layout) ? QM_LAYOUT_TILED : QM_LAYOUT_ROWMAJOR; }
+// a device seed base is read by the kernels of the tiled layer path, and offered for the extents the interface promises it for
+bool seed_base_served(int codes_layout, int64_t T, int64_t I, int64_t O, int hd_a, int hd_b, int hd_c) {
+    return tiled_layout(codes_layout) && hd_a == 32 && hd_b == 32 && hd_c == 32 && T % 128 == 0 && I % 128 == 0 &&
            O % 128 == 0;
 }
 }  // namespace
@@ -408,6 +418,7 @@ int qm_linear_forward(const void* x, int x_dtype, const void* w, int w_dtype, in
                       void* packed_w, size_t packed_w_bytes, int packed_flags, void* y, int y_dtype, int codes_layout,
                       void* stream) {
     if (T < 0 || I < 0 || O < 0) return fail(QM_ERR_INVALID, "qm_linear_forward: negative extent");
+    if (!valid_layer_layout(codes_layout)) return fail(QM_ERR_INVALID, "qm_linear_forward: unknown codes_layout %d", codes_layout);
     if (T == 0 || O == 0 || I == 0) return 0;
     if (I % 32) return fail(QM_ERR_INVALID, "qm_linear_forward: in_features %lld not a multiple of 32", (long long)I);
     const PackedLayout lx = packed_layout(T, I), lw = packed_layout(O, I);
@@ -419,27 +430,40 @@ int qm_linear_forward(const void* x, int x_dtype, const void* w, int w_dtype, in
     uint8_t* pw = static_cast<uint8_t*>(packed_w);
     if (packed_flags & ~(QM_W_IS_PACKED | QM_X_IS_PACKED)) return fail(QM_ERR_INVALID, "qm_linear_forward: unknown packed_flags %d", packed_flags);
     const bool w_is_packed = packed_flags & QM_W_IS_PACKED, x_is_packed = packed_flags & QM_X_IS_PACKED;
+    if (!y || !aligned(y, 4)) return fail(QM_ERR_INVALID, "qm_linear_forward: y must be non-null and 4-byte aligned");
+    hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
     int rc = 0;
-    if (!w_is_packed && !x_is_packed && pair_launches(codes_layout, T, I, O, hd_x, hd_w, 32) && x && w && y && valid_dtype(x_dtype) &&
-        valid_dtype(w_dtype) && aligned(x, 16) && aligned(w, 16)) {
-        // both forward quantizers in one grid
-        const qm::RowmajorArgs ax{x, x_dtype, T, I, signs_x ? signs_x[0] : 0u, px + lx.c, px + lx.s, px + lx.m};
-        const qm::RowmajorArgs aw{w, w_dtype, O, I, signs_w ? signs_w[0] : 0u, pw + lw.c, pw + lw.s, pw + lw.m};
-        rc = from_hip(qm::quantize_rowmajor_hd32_tiled_pair(ax, aw, reinterpret_cast<hipStream_t>(stream)), "qm_linear_forward");
-        if (rc) return rc;
+    int64_t K = I;
+    if (tiled_layout(codes_layout)) {
+        if (O % 8 || !aligned(y, 16)) return fail(QM_ERR_INVALID, "qm_linear_forward: tiled codes need out_features %% 8 == 0 and a 16-byte aligned y");
+        if (codes_layout == QM_LAYOUT_TILED && (T % 16 || O % 16 || I % 128))
+            return fail(QM_ERR_INVALID, "qm_linear_forward: tiled codes need tokens and out_features %% 16 == 0 and in_features %% 128 == 0 (QM_LAYOUT_PADDED takes any)");
+        const qm::RowmajorArgs ax{x, x_dtype, T, I, make_signs(signs_x, hd_x), px + lx.c, px + lx.s, px + lx.m};
+        const qm::RowmajorArgs aw{w, w_dtype, O, I, make_signs(signs_w, hd_w), pw + lw.c, pw + lw.s, pw + lw.m};
+        const auto bad = [&](const qm::RowmajorArgs& a, int hd) {
+            return !a.x || !aligned(a.x, 16) || !valid_dtype(a.dtype) || !valid_hd(hd) || a.cols % hd || a.rows >= (1ll << 31) - 16;
+        };
+        if ((!x_is_packed && bad(ax, hd_x)) || (!w_is_packed && bad(aw, hd_w)))
+            return fail(QM_ERR_INVALID, "qm_linear_forward: x and w must be non-null, 16-byte aligned, of a valid dtype, in_features a multiple of the Hadamard block");
+        if (!x_is_packed && !w_is_packed && hd_x == hd_w) {
+            rc = from_hip(qm::quantize_layer_forward(ax, &aw, hd_x, hs), "qm_linear_forward");   // both forward quantizers in one grid
+        } else {
+            if (!x_is_packed) rc = from_hip(qm::quantize_layer_forward(ax, nullptr, hd_x, hs), "qm_linear_forward");
+            if (!rc && !w_is_packed) rc = from_hip(qm::quantize_layer_forward(aw, nullptr, hd_w, hs), "qm_linear_forward");
+        }
+        K = qm::padded_cols(I);
     } else {
         if (!x_is_packed)
             rc = qm_quantize_mxfp4(x, x_dtype, T, I, hd_x, signs_x, QM_QUEST_RTN, 0, nullptr, 0, px + lx.c, px + lx.s, px + lx.m,
                                    nullptr, codes_layout, stream);
-        if (rc) return rc;
-        if (!w_is_packed) {
+        if (!rc && !w_is_packed)
             rc = qm_quantize_mxfp4(w, w_dtype, O, I, hd_w, signs_w, QM_QUEST_RTN, 0, nullptr, 0, pw + lw.c, pw + lw.s, pw + lw.m,
                                    nullptr, codes_layout, stream);
-            if (rc) return rc;
-        }
     }
-    return qm_gemm_mxfp4_tn(px + lx.c, px + lx.s, pw + lw.c, pw + lw.s, T, O, I, 1.0f, y, y_dtype, codes_layout, codes_layout, nullptr,
-                            0, stream);
+    if (rc) return rc;
+    if (!valid_dtype(y_dtype)) return fail(QM_ERR_INVALID, "qm_linear_forward: y_dtype %d", y_dtype);
+    return from_hip(qm::gemm_mxfp4_tn(px + lx.c, px + lx.s, pw + lw.c, pw + lw.s, T, O, K, 1.0f, y, y_dtype, kernel_layout(codes_layout), kernel_layout(codes_layout), nullptr, 0, hs),
+                    "qm_linear_forward");
 }
 
 int qm_linear_backward(const void* e, int e_dtype, int64_t T, int64_t I, int64_t O, const void* packed_x, const void* packed_w,
@@ -459,7 +483,8 @@ int qm_linear_backward_seeded(const void* e, int e_dtype, int64_t T, int64_t I, 
                               void* gw, int gw_dtype, int codes_layout, int rotated_flags, const float* g_matrix,
                               const uint64_t* seed_base, void* stream) {
     if (T < 0 || I < 0 || O < 0) return fail(QM_ERR_INVALID, "qm_linear_backward: negative extent");
-    if (seed_base && (!aligned(seed_base, 8) || g_matrix || !pair_launches(codes_layout, T, I, O, hd_x, hd_w, hd_g)))
+    if (!valid_layer_layout(codes_layout)) return fail(QM_ERR_INVALID, "qm_linear_backward: unknown codes_layout %d", codes_layout);
+    if (seed_base && (!aligned(seed_base, 8) || g_matrix || !seed_base_served(codes_layout, T, I, O, hd_x, hd_w, hd_g)))
         return fail(QM_ERR_INVALID, "qm_linear_backward_seeded: a device seed base needs the tiled layout with Hadamard blocks 32, "
                                     "T, I, O multiples of 128, no dense rotation, and an 8-byte aligned pointer");
     if (T == 0 || O == 0 || I == 0) return 0;
@@ -506,48 +531,59 @@ int qm_linear_backward_seeded(const void* e, int e_dtype, int64_t T, int64_t I, 
                                                 gw_dtype, true, hs), "qm_linear_backward");
     };
     if (gx_rotated && hd_x != 32) return fail(QM_ERR_INVALID, "qm_linear_backward: gx_rotated needs hd_x == 32");
-    // B3 + B7 and B6 + B8: where a gradient product runs on the persistent kernel's bf16 epilogue, the masked inverse
-    // rotation of the forward quantizer is applied to the tile before it is stored and the product lands in gx / gw
-    // directly (`fused` reports it); otherwise the product goes to the workspace and the rotation is a kernel of its own.
-    const auto grad_product = [&](const uint8_t* ac, const uint8_t* as, const uint8_t* bc, const uint8_t* bs, int64_t M, int64_t N,
-                                  int64_t K, void* plain_dst, void* final_dst, bool want_rotation, int hd, int final_dtype,
-                                  const uint8_t* mask, const uint32_t* signs, int scale_dtype, bool& fused) -> int {
-        fused = want_rotation && hd == 32 && final_dst && aligned(final_dst, 16) && valid_dtype(scale_dtype) && mask &&
-                qm::gemm_will_rotate(as, bs, M, N, K, mid_dtype, final_dtype, gws, wl.gemm_ws_bytes);
-        if (!fused)
-            return qm_gemm_mxfp4_tn(ac, as, bc, bs, M, N, K, alpha, plain_dst, mid_dtype, codes_layout, codes_layout, gws, wl.gemm_ws_bytes, stream);
-        bool done = false;
-        const int r = from_hip(qm::gemm_mxfp4_tn_rotated(ac, as, bc, bs, M, N, K, alpha, final_dst, mid_dtype, codes_layout, codes_layout, gws,
-                                                         wl.gemm_ws_bytes, mask, signs ? signs[0] : 0u, scale_dtype, final_dtype, &done, hs),
-                               "qm_linear_backward");
-        if (r) return r;
-        return done ? 0 : fail(QM_ERR_INVALID, "qm_linear_backward: a gradient product did not run as planned");
+    // B3 + B7 and B6 + B8: where the kernel that serves a gradient product applies the masked inverse rotation of the forward
+    // quantizer before it stores the result (choose_product tells), the product lands in gx / gw directly; otherwise it goes
+    // to the workspace and the rotation is a kernel of its own.
+    const bool tiled = tiled_layout(codes_layout);
+    if (codes_layout == QM_LAYOUT_TILED && (T % 128 || I % 128 || O % 128))
+        return fail(QM_ERR_INVALID, "qm_linear_backward: QM_LAYOUT_TILED needs T, I, O multiples of 128 (QM_LAYOUT_PADDED takes any multiples of 32)");
+    const int64_t Kx = tiled ? qm::padded_cols(O) : O, Kw = tiled ? qm::padded_cols(T) : T;
+    struct GradProduct {
+        qm::TileProduct p;
+        qm::ProductChoice choice;
+        int out_dtype;
     };
-    bool gx_fused = false, gw_fused = false;
-    const auto product_gx = [&]() {
-        return grad_product(k + wl.ec, k + wl.es, k + wl.wtc, k + wl.wts, T, I, O, gx_product, gx, !gx_rotated, hd_x, mid_dtype, px + lx.m,
-                            signs_x, x_scale_dtype, gx_fused);
+    const auto plan_product = [&](size_t ac, size_t as, size_t bc, size_t bs, int64_t M, int64_t N, int64_t K, void* plain_dst, void* final_dst,
+                                  bool want_rotation, int hd, int final_dtype, const uint8_t* mask, const uint32_t* signs, int scale_dtype) {
+        GradProduct g{qm::make_product(k + ac, k + as, k + bc, k + bs, M, N, K, alpha, plain_dst, kernel_layout(codes_layout), kernel_layout(codes_layout)), {}, mid_dtype};
+        if (want_rotation && final_dst && aligned(final_dst, 16) && valid_dtype(scale_dtype) && valid_hd(hd) && N % hd == 0) {
+            qm::TileProduct r = g.p;
+            r.c = final_dst;
+            r.mask = mask;
+            r.hd = hd;
+            r.signs = make_signs(signs, hd);
+            r.rot_c = qm::hadamard_scale(hd, scale_dtype);
+            const qm::ProductChoice c = qm::choose_product(r, mid_dtype, final_dtype, gws, wl.gemm_ws_bytes);
+            if (c.rotates) return GradProduct{r, c, final_dtype};
+        }
+        g.choice = qm::choose_product(g.p, mid_dtype, mid_dtype, gws, wl.gemm_ws_bytes);
+        return g;
     };
-    const auto product_gw = [&]() {
-        return grad_product(k + wl.etc, k + wl.ets, k + wl.xtc, k + wl.xts, O, I, T, gw_product, gw, !gw_rotated, hd_w, gw_dtype, pw + lw.m,
-                            signs_w, w_scale_dtype, gw_fused);
+    const GradProduct gx_plan = plan_product(wl.ec, wl.es, wl.wtc, wl.wts, T, I, Kx, gx_product, gx, !gx_rotated, hd_x, mid_dtype, px + lx.m, signs_x, x_scale_dtype);
+    const GradProduct gw_plan = plan_product(wl.etc, wl.ets, wl.xtc, wl.xts, O, I, Kw, gw_product, gw, !gw_rotated, hd_w, gw_dtype, pw + lw.m, signs_w, w_scale_dtype);
+    const bool gx_fused = gx_plan.choice.rotates, gw_fused = gw_plan.choice.rotates;
+    const auto run = [&](const GradProduct& g) {
+        return from_hip(qm::run_product(g.choice, g.p, mid_dtype, g.out_dtype, gws, hs), "qm_linear_backward");
     };
+    const auto product_gx = [&]() { return run(gx_plan); };
+    const auto product_gw = [&]() { return run(gw_plan); };
     if (g_matrix) {
+        const int kl = kernel_layout(codes_layout);
         // a dense rotation in the gradient quantizer (rerotate="O32"): the same eight steps on the dense-rotation kernels
         if (hd_g != 32 || T % 128 || I % 128 || O % 128)
             return fail(QM_ERR_INVALID, "qm_linear_backward: a dense gradient rotation needs hd_g == 32 and T, I, O multiples of 128 "
                                         "(T=%lld I=%lld O=%lld)", (long long)T, (long long)I, (long long)O);
-        rc = qm_quantize_mxfp4_dense(e, e_dtype, T, O, g_matrix, g_mode, 0, seeds[0], k + wl.ec, k + wl.es, nullptr, nullptr, codes_layout, stream);
+        rc = qm_quantize_mxfp4_dense(e, e_dtype, T, O, g_matrix, g_mode, 0, seeds[0], k + wl.ec, k + wl.es, nullptr, nullptr, kl, stream);
         if (rc) return rc;
         rc = qm_requantize_transposed_mxfp4_dense(pw + lw.c, pw + lw.s, O, I, 1.0f, w_val_dtype, g_matrix, g_mode, seeds[1], k + wl.wtc,
-                                                  k + wl.wts, nullptr, codes_layout, codes_layout, stream);
+                                                  k + wl.wts, nullptr, kl, kl, stream);
         if (rc) return rc;
         rc = product_gx();
         if (rc) return rc;
-        rc = qm_quantize_mxfp4_dense(e, e_dtype, O, T, g_matrix, g_mode, 1, seeds[2], k + wl.etc, k + wl.ets, nullptr, nullptr, codes_layout, stream);
+        rc = qm_quantize_mxfp4_dense(e, e_dtype, O, T, g_matrix, g_mode, 1, seeds[2], k + wl.etc, k + wl.ets, nullptr, nullptr, kl, stream);
         if (rc) return rc;
         rc = qm_requantize_transposed_mxfp4_dense(px + lx.c, px + lx.s, T, I, 1.0f, x_val_dtype, g_matrix, g_mode, seeds[3], k + wl.xtc,
-                                                  k + wl.xts, nullptr, codes_layout, codes_layout, stream);
+                                                  k + wl.xts, nullptr, kl, kl, stream);
         if (rc) return rc;
         rc = product_gw();
         if (rc) return rc;
@@ -557,17 +593,16 @@ int qm_linear_backward_seeded(const void* e, int e_dtype, int64_t T, int64_t I, 
         }
         return gw_fused ? 0 : rotate_gw();
     }
-    if (pair_launches(codes_layout, T, I, O, hd_x, hd_w, hd_g) && e && gx && gw && valid_dtype(e_dtype) && aligned(e, 16) &&
-        aligned(gx, 16) && aligned(gw, 16) && valid_dtype(x_val_dtype) && valid_dtype(w_val_dtype) &&
-        valid_dtype(x_scale_dtype) && valid_dtype(w_scale_dtype)) {
-        // seven launches: Q(e) with Q(e^T), Q(Q(W)^T) with Q(Q(x)^T), the two products, the two inverse rotations
-        const uint32_t sg = signs_g ? signs_g[0] : 0u;
-        rc = from_hip(qm::quantize_both_orientations_hd32_tiled(e, e_dtype, T, O, sg, g_mode, seeds[0], seeds[2], k + wl.ec, k + wl.es,
-                                                                k + wl.etc, k + wl.ets, seed_base, hs), "qm_linear_backward");
-        if (rc) return rc;
+    if (tiled) {
+        // the gradient quantizers (Q(e), Q(e^T), Q(Q(W)^T), Q(Q(x)^T)), the two products, the inverse rotations they do not carry
+        if (!valid_hd(hd_g) || !valid_hd(hd_x) || !valid_hd(hd_w) || T % hd_g || O % hd_g || I % hd_x || I % hd_w || !e || !gx || !gw || !valid_dtype(e_dtype) ||
+            !aligned(e, 16) || !aligned(gx, 16) || !aligned(gw, 16) || !valid_dtype(x_val_dtype) || !valid_dtype(w_val_dtype) ||
+            !valid_dtype(x_scale_dtype) || !valid_dtype(w_scale_dtype))
+            return fail(QM_ERR_INVALID, "qm_linear_backward: null, misaligned or ill-typed tensors, or extents that are not multiples of the Hadamard blocks");
         const qm::RequantArgs rw{pw + lw.c, pw + lw.s, O, I, w_val_dtype, seeds[1], k + wl.wtc, k + wl.wts};
         const qm::RequantArgs rx{px + lx.c, px + lx.s, T, I, x_val_dtype, seeds[3], k + wl.xtc, k + wl.xts};
-        rc = from_hip(qm::requantize_transposed_hd32_tiled_pair(rx, rw, sg, g_mode, seed_base, hs), "qm_linear_backward");
+        rc = from_hip(qm::quantize_layer_backward(e, e_dtype, T, O, hd_g, make_signs(signs_g, hd_g), g_mode, seeds[0], seeds[2], k + wl.ec, k + wl.es,
+                                                  k + wl.etc, k + wl.ets, rx, rw, seed_base, hs), "qm_linear_backward");
         if (rc) return rc;
         rc = product_gx();
         if (rc) return rc;
@@ -575,8 +610,10 @@ int qm_linear_backward_seeded(const void* e, int e_dtype, int64_t T, int64_t I, 
         if (rc) return rc;
         const bool need_x = !gx_rotated && !gx_fused, need_w = !gw_rotated && !gw_fused;
         if (!need_x) return need_w ? rotate_gw() : 0;
-        if (!need_w)
-            return qm_masked_hadamard_bwd(k + wl.gxq, mid_dtype, T, I, hd_x, x_scale_dtype, signs_x, px + lx.m, gx, mid_dtype, stream);
+        if (!need_w || hd_x != 32 || hd_w != 32) {
+            rc = qm_masked_hadamard_bwd(k + wl.gxq, mid_dtype, T, I, hd_x, x_scale_dtype, signs_x, px + lx.m, gx, mid_dtype, stream);
+            return rc ? rc : need_w ? rotate_gw() : 0;
+        }
         return from_hip(qm::masked_hadamard_bwd_hd32_pair(k + wl.gxq, T * I, x_scale_dtype,
                                                           signs_x ? signs_x[0] : 0u, px + lx.m, gx, k + wl.gwq, O * I,
                                                           w_scale_dtype, signs_w ? signs_w[0] : 0u,
@@ -609,7 +646,7 @@ int qm_linear_backward_seeded(const void* e, int e_dtype, int64_t T, int64_t I, 
 int qm_rmsnorm_quantize_mxfp4(const void* x, int x_dtype, const void* add, int add_dtype, void* x_sum, const float* gain, float eps,
                               int64_t rows, int64_t cols, const uint32_t* sign_bits, void* packed, size_t packed_bytes,
                               float* factor, int codes_layout, void* stream) {
-    if (!valid_layout(codes_layout)) return fail(QM_ERR_INVALID, "qm_rmsnorm_quantize_mxfp4: unknown codes_layout %d", codes_layout);
+    if (!valid_layer_layout(codes_layout)) return fail(QM_ERR_INVALID, "qm_rmsnorm_quantize_mxfp4: unknown codes_layout %d", codes_layout);
     if (!valid_dtype(x_dtype)) return fail(QM_ERR_INVALID, "qm_rmsnorm_quantize_mxfp4: x_dtype %d is not QM_BF16/QM_F32", x_dtype);
     if (rows < 0 || cols <= 0 || cols % 32)
         return fail(QM_ERR_INVALID, "qm_rmsnorm_quantize_mxfp4: need rows >= 0 and cols a positive multiple of 32 (got [%lld, %lld])",
@@ -627,13 +664,13 @@ int qm_rmsnorm_quantize_mxfp4(const void* x, int x_dtype, const void* add, int a
         return fail(QM_ERR_INVALID, "qm_rmsnorm_quantize_mxfp4: a residual summand needs an fp32 x, a valid add_dtype and x_sum");
     uint8_t* p = static_cast<uint8_t*>(packed);
     return from_hip(qm::rmsnorm_quantize_hd32(x, x_dtype, add, add_dtype, x_sum, gain, eps, rows, cols, sign_bits ? sign_bits[0] : 0u, p + l.c, p + l.s,
-                                              p + l.m, factor, codes_layout == QM_LAYOUT_TILED, reinterpret_cast<hipStream_t>(stream)),
+                                              p + l.m, factor, tiled_layout(codes_layout), reinterpret_cast<hipStream_t>(stream)),
                     "qm_rmsnorm_quantize_mxfp4");
 }
 
 int qm_swiglu_quantize_mxfp4(const void* h12, int dtype, int64_t rows, int64_t hidden, const uint32_t* sign_bits, void* packed,
                              size_t packed_bytes, int codes_layout, void* stream) {
-    if (!valid_layout(codes_layout)) return fail(QM_ERR_INVALID, "qm_swiglu_quantize_mxfp4: unknown codes_layout %d", codes_layout);
+    if (!valid_layer_layout(codes_layout)) return fail(QM_ERR_INVALID, "qm_swiglu_quantize_mxfp4: unknown codes_layout %d", codes_layout);
     if (!valid_dtype(dtype)) return fail(QM_ERR_INVALID, "qm_swiglu_quantize_mxfp4: dtype %d is not QM_BF16/QM_F32", dtype);
     if (rows < 0 || hidden <= 0 || hidden % 32)
         return fail(QM_ERR_INVALID, "qm_swiglu_quantize_mxfp4: need rows >= 0 and hidden a positive multiple of 32 (got [%lld, %lld])",
@@ -649,7 +686,7 @@ int qm_swiglu_quantize_mxfp4(const void* h12, int dtype, int64_t rows, int64_t h
         return fail(QM_ERR_UNALIGNED, "qm_swiglu_quantize_mxfp4: h12 needs 16-byte, packed 256-byte alignment");
     uint8_t* p = static_cast<uint8_t*>(packed);
     return from_hip(qm::swiglu_quantize_hd32(h12, dtype, rows, hidden, sign_bits ? sign_bits[0] : 0u, p + l.c, p + l.s, p + l.m,
-                                             codes_layout == QM_LAYOUT_TILED, reinterpret_cast<hipStream_t>(stream)),
+                                             tiled_layout(codes_layout), reinterpret_cast<hipStream_t>(stream)),
                     "qm_swiglu_quantize_mxfp4");
 }
 

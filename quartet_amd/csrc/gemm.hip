@@ -14,37 +14,27 @@
 // in the two successive MFMAs; both operands use the same assignment, which is all the
 // instruction needs.
 //
-// Three kernels, picked by shape in gemm_mxfp4_tn() at the end of the file:
-//   gemm_mxfp4_tn_big4_kernel  M, N multiples of 64 and >= 256, K > 768 and K % 512 == 0, or another multiple of 128 whose
-//                              last block of four K steps repeats (muted) at most a third as many steps as K has.
+// Kernels, picked by choose_product() at the end of the file:
+//   gemm_mxfp4_tn_big4_kernel  any M >= 256, N a multiple of 64 and >= 256, K a multiple of 128 whose last block of four K steps
+//                              repeats (muted) at most a third as many steps as K has.
 //                              Persistent, 256x256 macro tile, 4 waves x 128x128, operands global -> LDS directly into a
 //                              4-stage ring, scales in blocks of four K steps, row-major or tiled code bytes, optional split-K.
-//   gemm_mxfp4_tn_duo_kernel   same M, N, K % 128 == 0 and K <= 768, or K % 128 == 64 (row-major operands, any K >= 192):
-//                              256x128 tiles, two workgroups per CU hiding each other's tile boundaries, scales per K step.
+//   gemm_tile.hip              tiles from 256x128 down to 64x32 for everything too small or too short for that one.
 //   gemm_mxfp4_tn_kernel       any M, N and K % 32 == 0: 128x128 macro tile, 4 waves x 64x64, operands staged
 //                              global -> registers -> LDS (rows padded from 64 to 80 bytes so the 16-byte fragment
 //                              reads of 16 consecutive rows hit 64 distinct banks), double buffered.
 // All keep fp32 accumulators in registers, use one barrier per K step and apply alpha in the epilogue.
 #include <hip/hip_runtime.h>
-#include <hip/hip_ext.h>
 #include <stdint.h>
 
-#include <atomic>
 #include <type_traits>
-#include <utility>
 
-#include "qm_kernels.h"
-#include "qm_math.h"
+#include "gemm_common.h"
 
 namespace qm {
 
 namespace {
 
-typedef int v8i __attribute__((ext_vector_type(8)));
-typedef float v16f __attribute__((ext_vector_type(16)));
-
-constexpr int kBK = 128;             // K elements per step
-constexpr int kRowBytes = kBK / 2;   // 64 bytes of codes per row per step
 constexpr int kPitchDw = 20;         // 80-byte LDS row pitch, in dwords
 
 template <int BM, int BN>
@@ -226,80 +216,9 @@ __global__ __launch_bounds__(256) void gemm_mxfp4_tn_kernel(const uint8_t* __res
 // a tile is requested three K steps before it is consumed.  LDS rows are 64 bytes; the 16-byte column
 // of (row, c) is stored at c ^ ((row >> 2) & 3), applied on the global-address side of the load and on
 // the fragment read, which keeps the 16-byte fragment reads of 32 consecutive rows off each other's banks.
-typedef float v2f __attribute__((ext_vector_type(2)));
-typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
-
-// acc element e of a 32x32 tile is row 8*(e/4) + 4*half + e%4, column lane%32: per store instruction the
-// two half-waves each write one 64-byte (bf16) row segment.  (Making a lane's 4 values contiguous along n by
-// swapping the MFMA operand roles was measured slower: 64 scattered 8-byte pieces per instruction.)
-// One accumulator register into a vector register, in program order: left to itself the compiler copies ten blocks of
-// sixteen ahead of the first pass, and the 160 registers that takes push values the K loop needs out to scratch memory,
-// whose reloads then wait for every operand load in flight (loads return in order).
-__device__ __forceinline__ float acc_read(float a) {
-    float v;
-    asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(a));
-    return v;
-}
-// The hazard recogniser does not look inside assembly statements: a matrix instruction's result may be read by a vector
-// instruction only a number of wait states after it issued (19 for the sixteen-pass forms).  Every epilogue that reads
-// accumulators through acc_read() starts with this, whatever the scheduler has put between the last product and it.
-__device__ __forceinline__ void acc_settle() { asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory"); }
-template <typename OutT, bool IN_ORDER = false>
-__device__ __forceinline__ void store_tile(const v16f& t, float alpha, OutT* __restrict__ c, int64_t row0, int64_t col,
-                                           int64_t N, int half) {
-#pragma unroll
-    for (int e = 0; e < 16; e += 2) {
-        const int64_t r = row0 + 8 * (e / 4) + 4 * half + (e & 3);
-        const float v0 = (IN_ORDER ? acc_read(t[e]) : t[e]) * alpha, v1 = (IN_ORDER ? acc_read(t[e + 1]) : t[e + 1]) * alpha;
-        if constexpr (sizeof(OutT) == 2) {
-            // v_cvt_pk_bf16_f32: round-to-nearest-even, two values per instruction
-            const v2bf p = __builtin_convertvector(v2f{v0, v1}, v2bf);
-            const uint32_t bits = __builtin_bit_cast(uint32_t, p);
-            c[r * N + col] = (uint16_t)(bits & 0xffffu);
-            c[(r + 1) * N + col] = (uint16_t)(bits >> 16);
-        } else {
-            c[r * N + col] = v0;
-            c[(r + 1) * N + col] = v1;
-        }
-    }
-}
-
 constexpr int kBigM = 256, kBigN = 256;
 constexpr int kStages = 4;
 constexpr int kBOff = kBigM * kRowBytes;
-
-// Tile order: workgroup ids are dealt round-robin to the 8 XCDs by the hardware; give each XCD a
-// contiguous run of tiles in an order that walks 4-row groups column by column, so the tiles that
-// share an L2 also share A and B panels.
-__device__ __forceinline__ void tile_of_block(int bid, int tiles_m, int tiles_n, int& tm, int& tn) {
-    const int total = tiles_m * tiles_n;
-    int t = bid;
-    if ((total & 7) == 0) t = (bid & 7) * (total >> 3) + (bid >> 3);
-    constexpr int GM = 4;
-    const int per_group = GM * tiles_n;
-    const int group = t / per_group;
-    const int first_m = group * GM;
-    const int gm = (tiles_m - first_m) < GM ? (tiles_m - first_m) : GM;
-    const int r = t - group * per_group;
-    tm = first_m + r % gm;
-    tn = r / gm;
-}
-
-// global -> LDS without passing through registers.  Written as inline assembly on purpose: the
-// compiler's wait-count insertion treats every LDS read as possibly aliasing an outstanding
-// global_load_lds and would drain all loads (vmcnt(0)) before each fragment read, which defeats the
-// prefetch ring; the kernel waits explicitly for the one tile it is about to read instead.
-// LDS destination = lds_base (wave-uniform, via M0) + lane * size.  The "memory" clobber tells the compiler what it cannot
-// see in the statement: that it writes LDS, so no fragment read may be moved across it (costs nothing measurable).
-// addressed as uniform 64-bit base (SGPR pair) + per-lane 32-bit byte offset: no 64-bit VGPR address math
-__device__ __forceinline__ void load_lds_b128_s(const uint8_t* base, uint32_t lane_off, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(base), "s"(lds_base) : "memory");
-}
-// s_waitcnt immediate that waits for the vector-memory counter only
-constexpr int vmcnt_imm(int n) { return 0x0f70 | (n & 0xf) | ((n >> 4) << 14); }
-__device__ __forceinline__ void load_lds_b32(const uint8_t* gsrc, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(gsrc), "s"(lds_base) : "memory");
-}
 
 struct SubFrags {
     uint4 a[4], b[4];  // one K sub-step (64 values): four A tiles, four B tiles
@@ -342,261 +261,6 @@ __device__ __forceinline__ void big_mfma_sub(const SubFrags& f, const uint32_t (
     }
 }
 
-// one MFMA, then one memory instruction of the given class, n times: keeps the matrix pipe fed while the
-// wave issues its LDS / VMEM instructions
-#define QM_SCHED_PAIR(mask, n)                                   \
-    for (int _i = 0; _i < (n); ++_i) {                           \
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);       \
-        __builtin_amdgcn_sched_group_barrier((mask), 1, 0);      \
-    }
-
-// ---- two workgroups per CU: 256 x 128 tiles for short contractions -------------------------------------------------
-// With a short K the tile boundary dominates: the 256 x 256 kernels spend about 7.5 k cycles per tile converting, staging
-// and storing the result while no matrix instruction runs, against 1.3 k cycles per K step.  Here a workgroup owns a
-// 256 x 128 tile with four waves of 128 x 64 (128 accumulator registers, at most 256 registers per wave), so a SIMD holds
-// one wave of each of two workgroups: while one of them waits at its barrier, requests operands, or converts and stores
-// its tile, the other's matrix instructions keep the pipe busy.  The price is 1.5 x the operand traffic per flop (LDS
-// fragment reads and global -> LDS bytes), which is why long contractions stay on the 256 x 256 kernel.
-// Three-stage ring per workgroup (3 x 25.5 KiB: codes of 256 + 128 rows and one scale dword per row and K step); the
-// ring doubles as the epilogue's staging area, so nothing is prefetched across tiles -- the neighbour workgroup covers
-// the gap.  Persistent: the grid is two workgroups per CU.  M, N multiples of 64, M >= 256, N >= 128, K % 128 == 0, or
-// K % 128 == 64 with row-major operands (a final half step, see duo_issue).
-constexpr int kDuoM = 256, kDuoN = 128, kDuoStages = 3;
-constexpr int kDuoBOff = kDuoM * kRowBytes;                                   // 16 KiB of A codes
-constexpr int kDuoSAOff = (kDuoM + kDuoN) * kRowBytes;                        // 24 KiB of codes
-constexpr int kDuoSBOff = kDuoSAOff + kDuoM * 4;
-constexpr int kDuoStageBytes = kDuoSBOff + kDuoN * 4;                         // 25.5 KiB
-constexpr int kDuoSmemBytes = kDuoStages * kDuoStageBytes;                    // 76.5 KiB
-constexpr int kDuoEpiPitch = 144;   // bytes per staged row of 64 bf16: 128 rows x 144 B = 18 KiB per wave
-#ifndef QM_DUO_MAX_K
-#define QM_DUO_MAX_K 768
-#endif
-constexpr int kDuoMaxK = QM_DUO_MAX_K;  // longest contraction served by this kernel
-constexpr int kDuoLoads = 8;        // VMEM instructions per wave per K step: 4 (A) + 2 (B) + 2 (scales)
-static_assert(4 * 128 * kDuoEpiPitch <= kDuoSmemBytes, "the epilogue stages through the operand ring");
-
-struct DuoFrags {
-    uint4 a[4], b[2];
-};
-struct DuoPlan {
-    const uint8_t* a;   // uniform: this wave's 64 A rows of the tile, K step 0
-    const uint8_t* b;   // uniform: this wave's 32 B rows
-    const uint8_t* sa;  // this lane's A scale dword source at K step 0 (+ ks * 4 bytes)
-    const uint8_t* sb;
-    int64_t row16_bytes;
-    uint32_t lane_codes_a, lane_codes_b;
-    uint32_t half_codes_a, half_codes_b;  // the same for a final half step (K % 128 == 64): the row's last 32 bytes twice
-    int kstep_a, kstep_b;
-    uint32_t lds_a, lds_b, lds_sa, lds_sb;  // wave-uniform LDS addresses (stage 0)
-};
-// half: the step covers only 64 contraction indices (the last step of a K with K % 128 == 64, row-major operands).  Its
-// lanes request the row's final two 16-byte pieces in place of all four, and the scale dword that ends with the row's last
-// byte (two bytes early), so that no request leaves the row; the consumer shifts that dword down by 16 bits, which puts
-// the two real scale bytes first and zeros (2^-127: products vanish) where the missing half of the step would be.
-__device__ __forceinline__ void duo_issue(const DuoPlan& p, int stage, int ks, bool half) {
-    const uint32_t off = (uint32_t)stage * kDuoStageBytes;
-    const uint32_t la = half ? p.half_codes_a : p.lane_codes_a, lb = half ? p.half_codes_b : p.lane_codes_b;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) load_lds_b128_s(p.a + j * p.row16_bytes + ks * p.kstep_a, la, p.lds_a + off + j * 1024);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) load_lds_b128_s(p.b + j * p.row16_bytes + ks * p.kstep_b, lb, p.lds_b + off + j * 1024);
-    const int sback = half ? 2 : 0;
-    load_lds_b32(p.sa + ks * 4 - sback, p.lds_sa + off);
-    load_lds_b32(p.sb + ks * 4 - sback, p.lds_sb + off);
-}
-__device__ __forceinline__ void duo_read_sub(const uint8_t* __restrict__ stage, int a_off, int b_off, DuoFrags& f) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) f.a[i] = *reinterpret_cast<const uint4*>(stage + a_off + i * 32 * kRowBytes);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) f.b[j] = *reinterpret_cast<const uint4*>(stage + b_off + j * 32 * kRowBytes);
-}
-template <int SUB, bool SWAP, bool ZERO>
-__device__ __forceinline__ void duo_mfma_sub(const DuoFrags& f, const uint32_t (&sca)[4], const uint32_t (&scb)[2], v16f (&acc)[4][2]) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const v8i av = v8i{(int)f.a[i].x, (int)f.a[i].y, (int)f.a[i].z, (int)f.a[i].w, 0, 0, 0, 0};
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const v8i bv = v8i{(int)f.b[j].x, (int)f.b[j].y, (int)f.b[j].z, (int)f.b[j].w, 0, 0, 0, 0};
-            v16f cin;
-            if constexpr (ZERO) {
-#pragma unroll
-                for (int e = 0; e < 16; ++e) cin[e] = 0.0f;
-            } else {
-                cin = acc[i][j];
-            }
-            if constexpr (SWAP)
-                acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bv, av, cin, 4, 4, SUB, (int)scb[j], SUB, (int)sca[i]);
-            else
-                acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(av, bv, cin, 4, 4, SUB, (int)sca[i], SUB, (int)scb[j]);
-        }
-    }
-}
-
-template <typename OutT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_mxfp4_tn_duo_kernel(
-    const uint8_t* __restrict__ a_codes, const uint8_t* __restrict__ a_scales, const uint8_t* __restrict__ b_codes,
-    const uint8_t* __restrict__ b_scales, int M, int N, int K, float alpha, OutT* __restrict__ c, int a_tiled, int b_tiled) {
-    extern __shared__ uint32_t smem[];
-    uint8_t* smem_bytes = reinterpret_cast<uint8_t*>(smem);
-    const uint32_t smem_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint32_t*)smem;
-    constexpr bool SWAP = sizeof(OutT) == 2;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 1, wn = wave & 1;
-    const int lrow = lane & 31, half = lane >> 5;
-    const int tiles_m = (M + kDuoM - 1) / kDuoM, tiles_n = (N + kDuoN - 1) / kDuoN, total = tiles_m * tiles_n;
-    const int code_pitch = K / 2, groups = K / 32;
-    const int nk = (K + kBK - 1) / kBK;
-    const int half_step = (K % kBK) ? nk - 1 : -1;  // the K step that covers only 64 indices (K % 128 == 64), or none
-
-    const int swz = (lrow >> 2) & 3;
-    const int a_off0 = (wm * 128 + lrow) * kRowBytes + (((2 * half) ^ swz) * 16);
-    const int a_off1 = (wm * 128 + lrow) * kRowBytes + (((2 * half + 1) ^ swz) * 16);
-    const int b_off0 = kDuoBOff + (wn * 64 + lrow) * kRowBytes + (((2 * half) ^ swz) * 16);
-    const int b_off1 = kDuoBOff + (wn * 64 + lrow) * kRowBytes + (((2 * half + 1) ^ swz) * 16);
-    // scales in LDS: A dword p holds row (p >> 7) * 128 + (p & 3) * 32 + ((p >> 2) & 31), so one 16-byte read fetches the
-    // scale dwords of a lane's four A tiles; B dword p holds row (p >> 6) * 64 + (p & 1) * 32 + ((p >> 1) & 31): one 8-byte read
-    const int a_sc_off = kDuoSAOff + (wm * 32 + lrow) * 16;
-    const int b_sc_off = kDuoSBOff + (wn * 32 + lrow) * 8;
-    const int sh = 16 * half;
-
-    DuoPlan plan;
-    plan.row16_bytes = (int64_t)16 * code_pitch;
-    {
-        const int prow = lane >> 2;
-        const int pcv = (lane & 3) ^ ((prow >> 2) & 3);
-        const uint32_t rowmajor_off = (uint32_t)(prow * code_pitch + pcv * 16);
-        const uint32_t tiled_off = (uint32_t)(prow * 64 + pcv * 16);
-        plan.lane_codes_a = a_tiled ? tiled_off : rowmajor_off;
-        plan.lane_codes_b = b_tiled ? tiled_off : rowmajor_off;
-        // a half step exists for row-major operands only: pieces 2 and 3 of the step lie beyond the row, their LDS slots
-        // receive pieces 0 and 1 again (and zero scales)
-        plan.half_codes_a = plan.half_codes_b = (uint32_t)(prow * code_pitch + (pcv & 1) * 16);
-        plan.kstep_a = a_tiled ? 1024 : kRowBytes;
-        plan.kstep_b = b_tiled ? 1024 : kRowBytes;
-        plan.lds_a = (uint32_t)__builtin_amdgcn_readfirstlane((int)(smem_base + wave * 4096));
-        plan.lds_b = (uint32_t)__builtin_amdgcn_readfirstlane((int)(smem_base + kDuoBOff + wave * 2048));
-        plan.lds_sa = (uint32_t)__builtin_amdgcn_readfirstlane((int)(smem_base + kDuoSAOff + wave * 256));
-        // 128 B scale dwords: waves 2 and 3 repeat the requests of waves 0 and 1 (same bytes to the same place), which
-        // keeps every wave's count of outstanding loads the same
-        plan.lds_sb = (uint32_t)__builtin_amdgcn_readfirstlane((int)(smem_base + kDuoSBOff + (wave & 1) * 256));
-    }
-    // operand rows behind the scale dwords this lane requests
-    const int pa = wave * 64 + lane, pb = (wave & 1) * 64 + lane;
-    const int srow_a = (pa >> 7) * 128 + (pa & 3) * 32 + ((pa >> 2) & 31);
-    const int srow_b = (pb >> 6) * 64 + (pb & 1) * 32 + ((pb >> 1) & 31);
-
-    for (int t = (int)blockIdx.x; t < total; t += (int)gridDim.x) {
-        int tm, tn;
-        tile_of_block(t, tiles_m, tiles_n, tm, tn);
-        const int64_t m0 = (int64_t)tm * kDuoM, n0 = (int64_t)tn * kDuoN;
-        {
-            // M and N are multiples of 64 (32 for a wave's share of B): a wave's share of a panel lies inside the matrix or
-            // outside it as a whole; an outside share reads the matrix's last rows instead (its products are dropped below)
-            int64_t ma = m0 + wave * 64, nb = n0 + wave * 32;
-            ma = ma < M ? ma : (int64_t)M - 64;
-            nb = nb < N ? nb : (int64_t)N - 32;
-            plan.a = a_codes + ma * code_pitch;
-            plan.b = b_codes + nb * code_pitch;
-            plan.sa = a_scales + (m0 + srow_a < M ? m0 + srow_a : (int64_t)M - 1) * groups;
-            plan.sb = b_scales + (n0 + srow_b < N ? n0 + srow_b : (int64_t)N - 1) * groups;
-        }
-        const int rows_valid = (int)(M - m0) - wm * 128, cols_valid = (int)(N - n0) - wn * 64;
-
-        const auto issue = [&](int stage, int ks) { duo_issue(plan, stage, ks, ks == half_step); };
-        // the scale dwords of a half step arrive two bytes early (see duo_issue).  Without a branch: a K step is one basic
-        // block, which is what holds its instruction order in place.
-        const auto settle_scales = [&](uint4& a, uint2& b, int ks) {
-            const uint32_t down = ks == half_step ? 16u : 0u;
-            a.x >>= down; a.y >>= down; a.z >>= down; a.w >>= down;
-            b.x >>= down; b.y >>= down;
-        };
-        issue(0, 0);
-        issue(1, nk > 1 ? 1 : 0);
-        issue(2, nk > 2 ? 2 : nk - 1);
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * kDuoLoads));  // step 0 is in; steps 1, 2 may be pending
-        __syncthreads();
-        DuoFrags f0, f1;
-        uint4 sa4 = *reinterpret_cast<const uint4*>(smem_bytes + a_sc_off);
-        uint2 sb2 = *reinterpret_cast<const uint2*>(smem_bytes + b_sc_off);
-        settle_scales(sa4, sb2, 0);
-        duo_read_sub(smem_bytes, a_off0, b_off0, f0);
-
-        v16f acc[4][2];
-        int stage = 0;
-        // one K step: `stage` is the ring slot it consumes and then refills with step s + 3
-        auto step = [&](auto first_tag, int s) {
-            constexpr bool FIRST = decltype(first_tag)::value;
-            const int nstage = stage == kDuoStages - 1 ? 0 : stage + 1;
-            const uint8_t* cur = smem_bytes + stage * kDuoStageBytes;
-            const uint8_t* nxt = smem_bytes + nstage * kDuoStageBytes;
-            const uint32_t sca[4] = {__builtin_amdgcn_ubfe(sa4.x, (uint32_t)sh, 16u), __builtin_amdgcn_ubfe(sa4.y, (uint32_t)sh, 16u),
-                                     __builtin_amdgcn_ubfe(sa4.z, (uint32_t)sh, 16u), __builtin_amdgcn_ubfe(sa4.w, (uint32_t)sh, 16u)};
-            const uint32_t scb[2] = {__builtin_amdgcn_ubfe(sb2.x, (uint32_t)sh, 16u), __builtin_amdgcn_ubfe(sb2.y, (uint32_t)sh, 16u)};
-            duo_read_sub(cur, a_off1, b_off1, f1);
-            duo_mfma_sub<0, SWAP, FIRST>(f0, sca, scb, acc);
-            QM_SCHED_PAIR(0x100, 6)
-            __builtin_amdgcn_sched_barrier(0);
-            // younger than the loads of step s + 1: those of step s + 2
-            __builtin_amdgcn_s_waitcnt(vmcnt_imm(kDuoLoads));
-            __syncthreads();
-            __builtin_amdgcn_sched_barrier(0);
-            // past the end: a repeat nobody reads keeps the counts of outstanding loads uniform
-            issue(stage, s + 3 < nk ? s + 3 : nk - 1);
-            sa4 = *reinterpret_cast<const uint4*>(nxt + a_sc_off);
-            sb2 = *reinterpret_cast<const uint2*>(nxt + b_sc_off);
-            settle_scales(sa4, sb2, s + 1);
-            duo_read_sub(nxt, a_off0, b_off0, f0);
-            duo_mfma_sub<1, SWAP, false>(f1, sca, scb, acc);
-            QM_SCHED_PAIR(0x100, 6)
-            __builtin_amdgcn_sched_barrier(0);
-            stage = nstage;
-        };
-        step(std::true_type{}, 0);
-        for (int ks = 1; ks < nk; ++ks) step(std::false_type{}, ks);
-        // every request has landed and every wave has read its last fragments: the ring becomes the staging area
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-        __syncthreads();
-        if constexpr (SWAP) {
-            uint8_t* region = smem_bytes + wave * (128 * kDuoEpiPitch);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-#pragma unroll
-                    for (int b = 0; b < 4; ++b) {
-                        const v16f& v = acc[i][j];
-                        const v2bf p0 = __builtin_convertvector(v2f{v[4 * b] * alpha, v[4 * b + 1] * alpha}, v2bf);
-                        const v2bf p1 = __builtin_convertvector(v2f{v[4 * b + 2] * alpha, v[4 * b + 3] * alpha}, v2bf);
-                        *reinterpret_cast<uint2*>(region + (i * 32 + lrow) * kDuoEpiPitch + (j * 32 + 8 * b + 4 * half) * 2) =
-                            make_uint2(__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1));
-                    }
-            // the region is private to the wave; LDS operations of one wave complete in order
-            const int chunk = lane & 7, rsub = lane >> 3;
-            uint8_t* out = reinterpret_cast<uint8_t*>(reinterpret_cast<uint16_t*>(c) + (m0 + wm * 128 + rsub) * N + n0 + wn * 64) + chunk * 16;
-            const int64_t pitch8 = (int64_t)N * 16;  // eight rows of bf16
-            if (cols_valid > 0) {
-#pragma unroll
-                for (int r8 = 0; r8 < 16; ++r8) {
-                    const uint4 v = *reinterpret_cast<const uint4*>(region + (r8 * 8 + rsub) * kDuoEpiPitch + chunk * 16);
-                    typedef uint32_t u4v __attribute__((ext_vector_type(4)));
-                    if (r8 * 8 < rows_valid) __builtin_nontemporal_store(u4v{v.x, v.y, v.z, v.w}, reinterpret_cast<u4v*>(out + r8 * pitch8));
-                }
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    if (i * 32 < rows_valid && j * 32 < cols_valid)
-                        store_tile<OutT>(acc[i][j], alpha, c, m0 + wm * 128 + i * 32, n0 + wn * 64 + j * 32 + lrow, N, half);
-        }
-        __syncthreads();  // the staging area is the next tile's ring
-    }
-}
-
 // ---- persistent variant: scales travel in blocks of four K steps ------------------------------------
 // Fetching one scale dword per row per K step costs as many L2 requests as the codes themselves (each
 // row's 4 bytes sit in a different cache line).  Here a wave-load brings 16 bytes per row = the scales of
@@ -614,13 +278,11 @@ struct Big4Plan {
     const uint8_t* b;
     const uint8_t* sa;  // uniform: first scale byte of this tile's A panel
     const uint8_t* sb;
-    int64_t row16_bytes;    // 16 rows of codes
-    uint32_t lane_codes_a;  // this lane's byte offset inside a wave-load's source: row lane/4 + swizzled 16-byte column of a
-    uint32_t lane_codes_b;  //   row-major panel, or the same pick inside the 1 KiB tile of a tiled one
     int kstep_a, kstep_b;   // bytes from one K step to the next: 64 row-major, 1024 tiled
-    uint32_t voff_a[4];     // lane_codes_a + i * (row16_bytes - 1024): wave-load i of a K step, issued with instruction
-    uint32_t voff_b[4];     //   offset i * 1024, which moves its LDS destination by as much (and the source back in place)
-    uint32_t lane_scales;   // this lane's byte offset inside a panel's scales: row wave*64 + lane
+    uint32_t voff_a[4];     // wave-load i of a K step, issued with instruction offset i * 1024, which moves its LDS destination
+    uint32_t voff_b[4];     //   by as much (and the source back in place): row offset - i * 1024
+    uint32_t lane_scales_a;   // this lane's byte offset inside a panel's scales: row wave*64 + lane
+    uint32_t lane_scales_b;
     uint32_t lds_codes;     // wave-uniform LDS address of this wave's first A wave-load in stage 0
     uint32_t lds_scales;    // wave-uniform LDS address of this wave's A scale wave-load in buffer 0
 };
@@ -629,15 +291,15 @@ __device__ __forceinline__ void big4_issue_codes(const Big4Plan& p, int stage, i
     const uint32_t base = p.lds_codes + stage * kCodeStageBytes;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        load_lds_b128_s(p.a + j * p.row16_bytes + ks * p.kstep_a, p.lane_codes_a, base + j * 1024);
-        load_lds_b128_s(p.b + j * p.row16_bytes + ks * p.kstep_b, p.lane_codes_b, base + kBOff + j * 1024);
+        load_lds_b128_s(p.a + j * 1024 + ks * p.kstep_a, p.voff_a[j], base + j * 1024);
+        load_lds_b128_s(p.b + j * 1024 + ks * p.kstep_b, p.voff_b[j], base + kBOff + j * 1024);
     }
 }
 // soff: byte offset, within a row's scales, of the 16 bytes (four K steps) to request
 __device__ __forceinline__ void big4_issue_scales(const Big4Plan& p, int soff, int buf) {
     const uint32_t base = p.lds_scales + buf * kScaleBufBytes;
-    load_lds_b128_s(p.sa + soff, p.lane_scales, base);
-    load_lds_b128_s(p.sb + soff, p.lane_scales, base + kBigM * 16);
+    load_lds_b128_s(p.sa + soff, p.lane_scales_a, base);
+    load_lds_b128_s(p.sb + soff, p.lane_scales_b, base + kBigM * 16);
 }
 
 // The LDS destination of a global->LDS load is M0 + the instruction's offset + lane * 16, and the same offset is added
@@ -758,7 +420,7 @@ struct RotEpilogue {
 };
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-template <bool ROT = false>
+template <bool ROT = false, bool RAGGED = false>
 __device__ __forceinline__ void big4_epilogue_bf16(v16f (&acc)[4][4], float alpha, uint16_t* __restrict__ c, int64_t m0,
                                                    int64_t n0, int64_t N, int wm, int wn, int wave, int lane_in,
                                                    uint8_t* smem_bytes, int rows_valid, int cols_valid,
@@ -873,14 +535,16 @@ __device__ __forceinline__ void big4_epilogue_bf16(v16f (&acc)[4][4], float alph
                 else emit(std::true_type{});
             }
             // the region is private to the wave; LDS operations of one wave complete in order
-#pragma unroll
-            for (int r8 = 0; r8 < 4; ++r8) {
+            const auto put = [&](int r8) {
                 const uint4 v = *reinterpret_cast<const uint4*>(rd + r8 * 1024);
                 // streaming store: the tile is not read again by this kernel, and keeping it out of the L2 leaves the
                 // operand panels there (measured: -1.3 % on the product alone, -3 % on the whole layer step)
                 typedef uint32_t u4v __attribute__((ext_vector_type(4)));
                 __builtin_nontemporal_store(u4v{v.x, v.y, v.z, v.w}, reinterpret_cast<u4v*>(out + r8 * pitch8 + jp * 128));
-            }
+            };
+#pragma unroll
+            for (int r8 = 0; r8 < 4; ++r8)
+                if (!RAGGED || i * 32 + r8 * 8 + rsub < rows_valid) put(r8);
             // keeps the passes apart: a scheduler that reads many passes' accumulators into vector registers ahead of time
             // pushes the K loop's live values out to scratch memory, and their reloads wait for every operand load in flight
             __builtin_amdgcn_sched_barrier(0);
@@ -903,7 +567,8 @@ __device__ __forceinline__ unsigned long long shader_clock() {
 // Persistent: the grid is one workgroup per CU (or fewer); each workgroup walks tiles bid, bid + grid, ... as one
 // flat stream of K steps.  The loads that refill a freed ring stage simply continue into the next tile, so the
 // pipeline never drains between tiles and the epilogue runs while the next tile's first four stages arrive.
-template <typename OutT, bool STAMP = false, bool ROT = false>
+// RAGGED: M is not a multiple of 64 (an instantiation of its own: the row tests cost the others 2 to 8 % in registers).
+template <typename OutT, bool STAMP = false, bool ROT = false, bool RAGGED = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_mxfp4_tn_big4_kernel(
     const uint8_t* __restrict__ a_codes, const uint8_t* __restrict__ a_scales, const uint8_t* __restrict__ b_codes,
     const uint8_t* __restrict__ b_scales, int M, int N, int K, float alpha, OutT* __restrict__ c, int a_tiled,
@@ -952,25 +617,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     const int sh = 16 * half;
 
     Big4Plan plan;
-    plan.row16_bytes = (int64_t)16 * code_pitch;
     plan.lds_codes = (uint32_t)__builtin_amdgcn_readfirstlane((int)(smem_base + wave * 4096));
     plan.lds_scales = (uint32_t)__builtin_amdgcn_readfirstlane((int)(smem_base + kScaleAreaOff + wave * 1024));
-    {
-        const int prow = lane >> 2;  // the wave's 64-row offset is folded into the uniform part below
-        const int pcv = (lane & 3) ^ ((prow >> 2) & 3);
-        const uint32_t rowmajor_off = (uint32_t)(prow * code_pitch + pcv * 16);
-        const uint32_t tiled_off = (uint32_t)(prow * 64 + pcv * 16);  // same (row, swizzled slot) pick inside the 1 KiB tile
-        plan.lane_codes_a = a_tiled ? tiled_off : rowmajor_off;
-        plan.lane_codes_b = b_tiled ? tiled_off : rowmajor_off;
-        plan.kstep_a = a_tiled ? 1024 : kRowBytes;
-        plan.kstep_b = b_tiled ? 1024 : kRowBytes;
-        plan.lane_scales = (uint32_t)(lane * groups);
-        const uint32_t step16 = (uint32_t)plan.row16_bytes - 1024u;  // 16 rows are 8 K bytes in either layout, K >= 512
+    const int row16 = 16 * code_pitch;   // 16 rows are 8 K bytes in either layout, K >= 512
+    // the offsets of clamped rows may fall below i * 1024: RAGGED takes them from a base that much further back
+    constexpr uint32_t kLoadBias = RAGGED ? 3 * 1024 : 0;
+    // source of this lane in wave-load i: row 16 i + lane / 4 of the wave's 64 (at most `last`), swizzled 16-byte column
+    const auto lane_source = [&](int i, int last, int tiled) {
+        const int prow = lane >> 2, pcv = (lane & 3) ^ ((prow >> 2) & 3);
+        int r = 16 * i + prow;
+        r = r < last ? r : last;
+        const uint32_t off = tiled ? (uint32_t)((r >> 4) * row16 + (r & 15) * 64) : (uint32_t)(r * code_pitch);
+        return off + pcv * 16 + kLoadBias - 1024u * i;
+    };
+    plan.kstep_a = a_tiled ? 1024 : kRowBytes;
+    plan.kstep_b = b_tiled ? 1024 : kRowBytes;
+    plan.lane_scales_a = plan.lane_scales_b = (uint32_t)(lane * groups);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            plan.voff_a[i] = plan.lane_codes_a + (uint32_t)i * step16;
-            plan.voff_b[i] = plan.lane_codes_b + (uint32_t)i * step16;
-        }
+    for (int i = 0; i < 4; ++i) {
+        plan.voff_a[i] = lane_source(i, 63, a_tiled);
+        plan.voff_b[i] = lane_source(i, 63, b_tiled);
     }
     const int wave_u = wave;
     int load_tm, load_tn, load_split;  // work item the load stream is in
@@ -978,14 +644,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         const int t = item / splits;
         load_split = item - t * splits;
         tile_of_block(t, tiles_m, tiles_n, load_tm, load_tn);
-        // M and N are multiples of 64: a wave's 64-row share of a panel is inside the matrix or outside it as a whole;
-        // an outside share reads the matrix's last 64 rows instead (its products are dropped by the epilogue)
+        // N, and but for RAGGED M, is a multiple of 64: a wave's 64-row share of a panel is inside the matrix or outside it as a
+        // whole; an outside share reads the matrix's last 64 rows instead (its products are dropped by the epilogue).
+        // RAGGED: A's rows past the end read the last row (of the last block of 16 in a tiled operand).
         int64_t m0 = (int64_t)load_tm * kBigM + wave_u * 64, n0 = (int64_t)load_tn * kBigN + wave_u * 64;
-        m0 = m0 < M ? m0 : (int64_t)M - 64;
+        m0 = m0 < M ? m0 : RAGGED ? (int64_t)((M - 1) & ~63) : (int64_t)M - 64;
         n0 = n0 < N ? n0 : (int64_t)N - 64;
         const int64_t k0 = (int64_t)load_split * nk_real;  // first K step of the item
-        plan.a = a_codes + m0 * code_pitch + k0 * plan.kstep_a;
-        plan.b = b_codes + n0 * code_pitch + k0 * plan.kstep_b;
+        plan.a = a_codes + m0 * code_pitch + k0 * plan.kstep_a - kLoadBias;
+        plan.b = b_codes + n0 * code_pitch + k0 * plan.kstep_b - kLoadBias;
+        if constexpr (RAGGED) {   // otherwise the lane offsets never change
+            const int last = M - 1 - (int)m0, last_code = a_tiled ? last | 15 : last;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) plan.voff_a[i] = lane_source(i, last_code, a_tiled);
+            plan.lane_scales_a = (uint32_t)((lane < last ? lane : last) * groups);
+        }
         plan.sa = a_scales + m0 * groups + k0 * 4;
         plan.sb = b_scales + n0 * groups + k0 * 4;
     };
@@ -1068,7 +741,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         for (int ks = 4; ks < nk; ks += 4) block4(ks, std::false_type{});
         stamp();
         if constexpr (sizeof(OutT) == 2) {
-            big4_epilogue_bf16<ROT>(acc, alpha, reinterpret_cast<uint16_t*>(c), m0, n0, N, wm, wn, wave, lane, smem_bytes,
+            big4_epilogue_bf16<ROT, RAGGED>(acc, alpha, reinterpret_cast<uint16_t*>(c), m0, n0, N, wm, wn, wave, lane, smem_bytes,
                                     rows_valid, cols_valid, rot, keep, keep_shifted);
         } else {
             OutT* dst = splits > 1 ? c + (int64_t)cur_split * M * N : c;
@@ -1078,8 +751,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             for (int i = 0; i < 4; ++i)
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                    if (i * 32 < rows_valid && j * 32 < cols_valid)
-                        store_tile<OutT, true>(acc[i][j], a_eff, dst, m0 + wm * 128 + i * 32, n0 + wn * 128 + j * 32 + lrow, N, half);
+                    if (i * 32 < rows_valid && j * 32 < cols_valid) {
+                        const int64_t row0 = m0 + wm * 128 + i * 32, col = n0 + wn * 128 + j * 32 + lrow;
+                        store_tile<OutT, true>(acc[i][j], a_eff, dst, row0, col, N, half, RAGGED ? rows_valid - i * 32 : 32);
+                    }
         }
         stamp();
     }
@@ -1150,35 +825,50 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     sink[(size_t)blockIdx.x * 256 + tid] = sum;
 }
 
-// hipFuncSetAttribute(MaxDynamicSharedMemorySize) once per kernel and device instead of on every launch
-constexpr int kMaxDevices = 64;
-template <typename Kern>
-hipError_t allow_dynamic_lds(Kern kern, int bytes, std::atomic<bool> (&done)[kMaxDevices]) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    if (dev >= 0 && dev < kMaxDevices && done[dev].load(std::memory_order_acquire)) return hipSuccess;
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    if (e == hipSuccess && dev >= 0 && dev < kMaxDevices) done[dev].store(true, std::memory_order_release);
-    return e;
+// ---- which kernel serves a product ----------------------------------------------------------------------------------
+// Estimated durations in microseconds, fitted to 110 shapes of 0.2 to 900 GF (tiled operands; each kernel that serves the
+// shape was timed): mean error 13 %, and the fastest kernel is the one chosen but for 0.3 % of the time on average.  All
+// kernels give the same bits except a cut into K ranges, so nothing but time hangs on the choice.
+struct KernelCost {
+    int bm, bn, per_cu;              // tile, resident workgroups per CU
+    double step, shared, boundary;   // one K step of a workgroup alone on its CU; with n of them: n * shared; per tile
+};
+constexpr KernelCost kTileCosts[] = {{256, 128, 2, 0.726, 0.648, 2.4}, {128, 128, 3, 0.198, 0.373, 1.5}, {128, 64, 3, 0.170, 0.277, 0.9},
+                                     {64, 64, 4, 0.129, 0.207, 0.63}, {64, 32, 4, 0.176, 0.139, 0.71}};
+constexpr double kLaunch = 2.3, kPersistentStep = 0.88, kPersistentBoundary = 3.7, kMemory = 3.2e6;   // bytes per us of a reduction pass
+
+double tile_cost(const KernelCost& k, int64_t M, int64_t N, int64_t K, int cus) {
+    const int64_t tiles = ((M + k.bm - 1) / k.bm) * ((N + k.bn - 1) / k.bn), steps = (K + kBK - 1) / kBK;
+    const auto round = [&](int64_t n) {   // n workgroups of one CU side by side
+        const double step = k.step > n * k.shared ? k.step : n * k.shared;
+        return steps * step + k.boundary * __builtin_sqrt((double)n);
+    };
+    const int64_t full = tiles / (k.per_cu * cus), rest = tiles % (k.per_cu * cus);
+    return kLaunch + full * round(k.per_cu) + (rest ? round((rest + cus - 1) / cus) : 0.0);
+}
+double persistent_cost(int64_t M, int64_t N, int64_t K, int splits, int cus) {
+    const int64_t items = ((M + kBigM - 1) / kBigM) * ((N + kBigN - 1) / kBigN) * splits;
+    const int64_t steps = (K / kBK / splits + 3) & ~(int64_t)3;
+    const double t = kLaunch + (double)((items + cus - 1) / cus) * (steps * kPersistentStep + kPersistentBoundary);
+    return splits == 1 ? t : t + kLaunch + (4.0 * splits + 2.0) * (double)M * (double)N / kMemory;
 }
 
-int device_cus() {
-    static int cached = 0;  // one GPU model per process
-    if (cached > 0) return cached;
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-        n > 0)
-        return cached = n;
-    return 256;
+// The persistent kernel: M any, N a multiple of 64, at least one tile; it walks K in blocks of four steps: K % 512 == 0
+// directly (scale rows are then 16-byte aligned like their base), other multiples of 128 with up to three muted steps in
+// the last block when those are at most a third of the real ones; their 16-byte scale requests start at 4-byte aligned
+// addresses.
+bool persistent_serves(int64_t M, int64_t N, int64_t K, const void* a_scales, const void* b_scales, const void* c) {
+    const int64_t steps = K / kBK, pad = ((steps + 3) & ~(int64_t)3) - steps;
+    if (N % 64 || M < kBigM || N < kBigN || K % kBK || steps < 4 || pad * 3 > steps || M >= (1 << 30) || N >= (1 << 30) || K >= (1 << 24)) return false;
+    if (K % 512 == 0 && ((reinterpret_cast<uintptr_t>(a_scales) | reinterpret_cast<uintptr_t>(b_scales)) & 15)) return false;
+    return (reinterpret_cast<uintptr_t>(c) & 15) == 0;
 }
-
-// How many K ranges to cut a GEMM into so that its (tile, range) items fill the CUs: the divisor s of K/512 that
+// How many K ranges to cut a product into so that its (tile, range) items fill the CUs: the divisor s of K / 512 that
 // minimises rounds(s) * steps(s) plus a per-item overhead, each range keeping at least eight K steps.  1 = no split.
 int choose_splits(int64_t M, int64_t N, int64_t K, int cus) {
     const int64_t tiles = ((M + kBigM - 1) / kBigM) * ((N + kBigN - 1) / kBigN);
     const int64_t nblk = K / 512;
-    if (tiles * 4 >= cus * 3 || nblk < 4) return 1;
+    if (K % 512 || tiles * 4 >= cus * 3 || nblk < 4) return 1;
     int best = 1;
     double best_cost = 1e30;
     for (int sp = 1; sp <= nblk && sp <= 64; ++sp) {
@@ -1197,38 +887,31 @@ int choose_splits(int64_t M, int64_t N, int64_t K, int cus) {
 // item, where the tile boundary is a third or more of a tile; longer ones neither gain nor lose (within 0.7 %)
 int big4_late_start(int64_t K, int splits) { return K / kBK / splits <= 16 ? 6 : 0; }
 
-template <typename OutT, bool ROT = false>
-hipError_t launch_big4(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
-                       const uint8_t* b_scales, int64_t M, int64_t N, int64_t K, float alpha, void* c, int a_tiled,
-                       int b_tiled, int splits, int cus, hipStream_t stream, const RotEpilogue& rot = RotEpilogue{}) {
-    auto kern = gemm_mxfp4_tn_big4_kernel<OutT, false, ROT>;
+template <typename OutT, bool ROT, bool RAGGED>
+hipError_t launch_big4_as(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
+                          const uint8_t* b_scales, int64_t M, int64_t N, int64_t K, float alpha, void* c, int a_tiled,
+                          int b_tiled, int splits, int cus, hipStream_t stream, const RotEpilogue& rot) {
+    auto kern = gemm_mxfp4_tn_big4_kernel<OutT, false, ROT, RAGGED>;
     static std::atomic<bool> lds_allowed[kMaxDevices];
     hipError_t e = allow_dynamic_lds(kern, kBig4SmemBytes, lds_allowed);
     if (e != hipSuccess) return e;
     const int64_t items = ((M + kBigM - 1) / kBigM) * ((N + kBigN - 1) / kBigN) * splits;
-    // one workgroup per CU, and a grid that is a multiple of 8 so that item t and t + grid land on the same XCD
+    // one workgroup per CU, and where a workgroup walks several items a grid that is a multiple of 8, so that item t and
+    // t + grid land on the same XCD
     int64_t g = items < cus ? items : cus;
-    if (g > 8) g -= g % 8;
+    if (g > 8 && g < items) g -= g % 8;
     dim3 grid((unsigned)g), block(256);
     kern<<<grid, block, kBig4SmemBytes, stream>>>(a_codes, a_scales, b_codes, b_scales, (int)M, (int)N, (int)K, alpha,
                                                   reinterpret_cast<OutT*>(c), a_tiled, b_tiled, splits, big4_late_start(K, splits), nullptr, rot);
     return hipGetLastError();
 }
-
-template <typename OutT>
-hipError_t launch_duo(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes, const uint8_t* b_scales,
-                      int64_t M, int64_t N, int64_t K, float alpha, void* c, int a_tiled, int b_tiled, int cus, hipStream_t stream) {
-    auto kern = gemm_mxfp4_tn_duo_kernel<OutT>;
-    static std::atomic<bool> lds_allowed[kMaxDevices];
-    hipError_t e = allow_dynamic_lds(kern, kDuoSmemBytes, lds_allowed);
-    if (e != hipSuccess) return e;
-    const int64_t tiles = ((M + kDuoM - 1) / kDuoM) * ((N + kDuoN - 1) / kDuoN);
-    // two workgroups per CU, and a grid that is a multiple of 8 so that tile t and t + grid land on the same XCD
-    int64_t g = tiles < 2 * cus ? tiles : 2 * cus;
-    if (g > 8) g -= g % 8;
-    kern<<<dim3((unsigned)g), dim3(256), kDuoSmemBytes, stream>>>(a_codes, a_scales, b_codes, b_scales, (int)M, (int)N, (int)K, alpha,
-                                                                  reinterpret_cast<OutT*>(c), a_tiled, b_tiled);
-    return hipGetLastError();
+template <typename OutT, bool ROT = false>
+hipError_t launch_big4(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
+                       const uint8_t* b_scales, int64_t M, int64_t N, int64_t K, float alpha, void* c, int a_tiled,
+                       int b_tiled, int splits, int cus, hipStream_t stream, const RotEpilogue& rot = RotEpilogue{}) {
+    if (M % 64)
+        return launch_big4_as<OutT, ROT, true>(a_codes, a_scales, b_codes, b_scales, M, N, K, alpha, c, a_tiled, b_tiled, splits, cus, stream, rot);
+    return launch_big4_as<OutT, ROT, false>(a_codes, a_scales, b_codes, b_scales, M, N, K, alpha, c, a_tiled, b_tiled, splits, cus, stream, rot);
 }
 
 template <int BM, int BN, int WM, int WN>
@@ -1299,104 +982,114 @@ bool gemm_supports_tiled(int64_t M, int64_t N, int64_t K) {
            K < (1 << 30);
 }
 
-// bytes of scratch with which gemm_mxfp4_tn cuts this shape into K ranges (0: it would not)
+// bytes of scratch with which gemm_mxfp4_tn may cut this shape into K ranges (0: it would not)
 size_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-    if (!gemm_supports_tiled(M, N, K) || K % 512 || K <= kDuoMaxK) return 0;
+    if (!persistent_serves(M, N, K, nullptr, nullptr, nullptr)) return 0;
     const int sp = choose_splits(M, N, K, device_cus());
     return sp > 1 ? (size_t)sp * (size_t)M * (size_t)N * sizeof(float) : 0;
+}
+
+// The kernel that serves product p.  p.mask: the caller wants the masked inverse rotation applied to the result (mid dtype
+// c_dtype, stored in rot_out_dtype); `rotates` tells whether the chosen kernel does it.  Where it does not, the rotation is
+// a kernel of its own that reads and writes the result, which the comparison accounts for.
+ProductChoice choose_product(const TileProduct& p, int c_dtype, int rot_out_dtype, const void* workspace, size_t workspace_bytes) {
+    const int cus = device_cus();
+    const int64_t M = p.M, N = p.N, K = p.K;
+    const bool rotate = p.mask != nullptr;
+    const double separate = rotate ? kLaunch + (double)M * N * ((c_dtype == BF16 ? 2 : 4) + (rot_out_dtype == BF16 ? 2 : 4)) / kMemory : 0.0;
+    ProductChoice best{ProductChoice::GENERIC, 0, 1, false};
+    double best_cost = 1e30, best_plain = 1e30;   // with the rotation, and of the product alone
+    const auto consider = [&](ProductChoice c, double cost) {
+        best_plain = cost < best_plain ? cost : best_plain;
+        if (rotate && !c.rotates) cost += separate;
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = c;
+        }
+    };
+    const bool persistent = persistent_serves(M, N, K, p.a_scales, p.b_scales, p.c);
+    if (persistent) {
+        const bool bf16 = c_dtype == BF16 && rot_out_dtype == BF16;
+        consider({ProductChoice::PERSISTENT, 0, 1, rotate && bf16 && p.hd == 32}, persistent_cost(M, N, K, 1, cus));
+    }
+    if (gemm_tile_serves(M, N, K, p.a_tiled, p.b_tiled, p.c))
+        for (int kind = TILE_256x128; kind <= TILE_64x32; ++kind)
+            consider({ProductChoice::TILE, kind, 1, rotate && c_dtype == BF16 && kTileCosts[kind].bn >= p.hd},
+                     tile_cost(kTileCosts[kind], M, N, K, cus));
+    // a cut into K ranges rounds differently: whether to make it is decided on the product alone, so that a product and the
+    // same product with the rotation agree
+    if (persistent && workspace) {
+        const int sp = choose_splits(M, N, K, cus);
+        if (sp > 1 && (size_t)sp * M * N * sizeof(float) <= workspace_bytes && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
+            persistent_cost(M, N, K, sp, cus) < best_plain)
+            return {ProductChoice::PERSISTENT, 0, sp, rotate && p.hd == 32};
+    }
+    return best;
+}
+
+// Runs product p on the chosen kernel.  Rotated (c.rotates): p.c receives rot_out_dtype elements; otherwise the plain product
+// in c_dtype.  workspace as offered to choose_product.
+hipError_t run_product(const ProductChoice& c, const TileProduct& p, int c_dtype, int rot_out_dtype, void* workspace, hipStream_t stream) {
+    const int64_t M = p.M, N = p.N, K = p.K;
+    const int cus = device_cus();
+    if (c.path == ProductChoice::TILE) {
+        TileProduct q = p;
+        if (!c.rotates) q.mask = nullptr;
+        q.out_f32 = c_dtype == BF16 && rot_out_dtype == F32;
+        return gemm_tile(c.kind, q, nullptr, c_dtype, stream);
+    }
+    if (c.path == ProductChoice::GENERIC) {
+        if (p.a_tiled || p.b_tiled) return hipErrorInvalidValue;
+        return launch_gemm<128, 128, 64, 64>(p.a_codes, p.a_scales, p.b_codes, p.b_scales, M, N, K, p.alpha, p.c, c_dtype, stream);
+    }
+    if (c.splits > 1) {
+        // partial sums per K range in fp32 (plain accumulator layout), then one ordered reduction
+        hipError_t e = launch_big4<float>(p.a_codes, p.a_scales, p.b_codes, p.b_scales, M, N, K, 1.0f, workspace, p.a_tiled, p.b_tiled, c.splits,
+                                          cus, stream);
+        if (e != hipSuccess) return e;
+        const int64_t mn = M * N;
+        const float* part = static_cast<const float*>(workspace);
+        if (c.rotates)
+            return splitk_reduce_rotated(part, c.splits, mn, p.alpha, c_dtype, p.mask, p.signs.w[0], p.rot_c, p.c, rot_out_dtype, stream);
+        dim3 grid((unsigned)((mn / 4 + 255) / 256)), block(256);
+        if (c_dtype == BF16)
+            splitk_reduce_kernel<uint16_t><<<grid, block, 0, stream>>>(part, c.splits, mn, p.alpha, static_cast<uint16_t*>(p.c));
+        else
+            splitk_reduce_kernel<float><<<grid, block, 0, stream>>>(part, c.splits, mn, p.alpha, static_cast<float*>(p.c));
+        return hipGetLastError();
+    }
+    if (c.rotates)
+        return launch_big4<uint16_t, true>(p.a_codes, p.a_scales, p.b_codes, p.b_scales, M, N, K, p.alpha, p.c, p.a_tiled, p.b_tiled, 1, cus, stream,
+                                           RotEpilogue{p.mask, p.signs.w[0], p.rot_c});
+    if (c_dtype == BF16)
+        return launch_big4<uint16_t>(p.a_codes, p.a_scales, p.b_codes, p.b_scales, M, N, K, p.alpha, p.c, p.a_tiled, p.b_tiled, 1, cus, stream);
+    return launch_big4<float>(p.a_codes, p.a_scales, p.b_codes, p.b_scales, M, N, K, p.alpha, p.c, p.a_tiled, p.b_tiled, 1, cus, stream);
+}
+
+TileProduct make_product(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes, const uint8_t* b_scales, int64_t M, int64_t N,
+                         int64_t K, float alpha, void* c, int a_layout, int b_layout) {
+    TileProduct p{};
+    p.a_codes = a_codes; p.a_scales = a_scales; p.b_codes = b_codes; p.b_scales = b_scales; p.c = c;
+    p.M = (int)M; p.N = (int)N; p.K = (int)K; p.alpha = alpha; p.hd = 32;
+    p.a_tiled = a_layout == LAYOUT_TILED; p.b_tiled = b_layout == LAYOUT_TILED;
+    return p;
 }
 
 hipError_t gemm_mxfp4_tn(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
                          const uint8_t* b_scales, int64_t M, int64_t N, int64_t K, float alpha, void* c, int c_dtype,
                          int a_layout, int b_layout, void* workspace, size_t workspace_bytes, hipStream_t stream) {
-    return gemm_mxfp4_tn_rotated(a_codes, a_scales, b_codes, b_scales, M, N, K, alpha, c, c_dtype, a_layout, b_layout, workspace,
-                                 workspace_bytes, nullptr, 0u, F32, c_dtype, nullptr, stream);
-}
-
-// whether gemm_mxfp4_tn_rotated would apply the rotation itself for these arguments: in the epilogue of an uncut product
-// (bf16 in and out), or in the reduction of a product it cuts into K ranges
-bool gemm_will_rotate(const uint8_t* a_scales, const uint8_t* b_scales, int64_t M, int64_t N, int64_t K, int c_dtype, int rot_out_dtype,
-                      const void* workspace, size_t workspace_bytes) {
-    if (!gemm_supports_tiled(M, N, K) || K <= kDuoMaxK) return false;
-    if (rot_out_dtype != c_dtype && !(c_dtype == BF16 && rot_out_dtype == F32)) return false;
-    const int64_t nk_real = K / kBK, nk_pad = (nk_real + 3) & ~(int64_t)3;
-    const bool persistent_ok = K % 512 == 0 ? ((reinterpret_cast<uintptr_t>(a_scales) | reinterpret_cast<uintptr_t>(b_scales)) & 15) == 0
-                                            : (nk_real >= 4 && (nk_pad - nk_real) * 3 <= nk_real);
-    if (!persistent_ok) return false;
-    int sp = workspace && K % 512 == 0 ? choose_splits(M, N, K, device_cus()) : 1;
-    if (sp > 1 && ((size_t)sp * M * N * sizeof(float) > workspace_bytes || (reinterpret_cast<uintptr_t>(workspace) & 15))) sp = 1;
-    return sp > 1 || (c_dtype == BF16 && rot_out_dtype == BF16);
-}
-
-// The product, with the layer's masked inverse Hadamard rotation (blocks of 32 along N) applied to the result before it is
-// stored when `rot_mask` is given and gemm_will_rotate() holds: in the persistent kernel's bf16 epilogue, or in the ordered
-// reduction of the K ranges.  *rotated tells which (true: c holds the rotated result in rot_out_dtype; false: c holds the
-// plain product in c_dtype and the caller runs the rotation as a kernel of its own).
-hipError_t gemm_mxfp4_tn_rotated(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
-                                 const uint8_t* b_scales, int64_t M, int64_t N, int64_t K, float alpha, void* c, int c_dtype,
-                                 int a_layout, int b_layout, void* workspace, size_t workspace_bytes, const uint8_t* rot_mask,
-                                 uint32_t rot_signs, int rot_scale_dtype, int rot_out_dtype, bool* rotated, hipStream_t stream) {
-    if (rotated) *rotated = false;
     if (M == 0 || N == 0) return hipSuccess;
-    const int at = a_layout == LAYOUT_TILED, bt = b_layout == LAYOUT_TILED;
-    const bool big_ok = gemm_supports_tiled(M, N, K);
-    if ((at || bt) && !big_ok) return hipErrorInvalidValue;
-    // The persistent kernel walks K in blocks of four steps: K % 512 == 0 directly (scale rows are then 16-byte aligned
-    // like their base), other multiples of 128 with up to three muted steps in the last block when those are at most a
-    // third of the real ones (K = 1152 and 1664 gain 3-5 % over a kernel without muted steps); their 16-byte scale
-    // requests start at 4-byte aligned addresses.  Every multiple of 128 above 768 qualifies; up to 768 the contraction is
-    // so short that the tile boundary dominates and the two-workgroups-per-CU kernel is faster (measured at 32768 tokens:
-    // 640 x 640 15 against 23 us, 3456 x 640 70 against 82 us; at K = 1536 it is 13-25 % slower than the persistent kernel).
-    const int64_t nk_real = K / kBK, nk_pad = (nk_real + 3) & ~(int64_t)3;
-    const bool persistent_ok = K % 512 == 0 ? ((reinterpret_cast<uintptr_t>(a_scales) | reinterpret_cast<uintptr_t>(b_scales)) & 15) == 0
-                                            : (nk_real >= 4 && (nk_pad - nk_real) * 3 <= nk_real);
-    // K % 128 == 64 (the 30 M Llama's hidden width 1728): the two-workgroup kernel closes such a contraction with a half
-    // step.  Row-major operands (the tiled layout does not exist for these K); a c that is only 4-byte aligned, which the
-    // interface accepts at these shapes, stays on the generic kernel.
-    const bool half_ok = !at && !bt && K % kBK == 64 && K >= 192 && gemm_supports_tiled(M, N, K - 64) &&
-                         (reinterpret_cast<uintptr_t>(c) & 15) == 0;
-    if (half_ok) {
-        const int cus = device_cus();
-        if (c_dtype == BF16) return launch_duo<uint16_t>(a_codes, a_scales, b_codes, b_scales, M, N, K, alpha, c, 0, 0, cus, stream);
-        return launch_duo<float>(a_codes, a_scales, b_codes, b_scales, M, N, K, alpha, c, 0, 0, cus, stream);
-    }
-    if (big_ok && (K <= kDuoMaxK || !persistent_ok)) {
-        // short contraction: two 256 x 128 workgroups per CU hide each other's tile boundaries (also the fallback for scale
-        // arrays that are not 16-byte aligned, which the persistent kernel's 16-byte scale requests need when K % 512 == 0)
-        const int cus = device_cus();
-        if (c_dtype == BF16) return launch_duo<uint16_t>(a_codes, a_scales, b_codes, b_scales, M, N, K, alpha, c, at, bt, cus, stream);
-        return launch_duo<float>(a_codes, a_scales, b_codes, b_scales, M, N, K, alpha, c, at, bt, cus, stream);
-    }
-    if (big_ok && persistent_ok) {
-        const int cus = device_cus();
-        int sp = workspace && K % 512 == 0 ? choose_splits(M, N, K, cus) : 1;  // K ranges are whole blocks of four steps
-        if (sp > 1 && ((size_t)sp * M * N * sizeof(float) > workspace_bytes || (reinterpret_cast<uintptr_t>(workspace) & 15))) sp = 1;
-        if (sp > 1) {
-            // partial sums per K range in fp32 (plain accumulator layout), then one ordered reduction
-            hipError_t e = launch_big4<float>(a_codes, a_scales, b_codes, b_scales, M, N, K, 1.0f, workspace, at, bt, sp, cus, stream);
-            if (e != hipSuccess) return e;
-            const int64_t mn = M * N;
-            if (rot_mask && rotated && (rot_out_dtype == c_dtype || (c_dtype == BF16 && rot_out_dtype == F32))) {
-                *rotated = true;
-                return splitk_reduce_rotated(static_cast<const float*>(workspace), sp, mn, alpha, c_dtype, rot_mask, rot_signs, rot_scale_dtype,
-                                             c, rot_out_dtype, stream);
-            }
-            dim3 grid((unsigned)((mn / 4 + 255) / 256)), block(256);
-            if (c_dtype == BF16)
-                splitk_reduce_kernel<uint16_t><<<grid, block, 0, stream>>>(static_cast<const float*>(workspace), sp, mn, alpha, static_cast<uint16_t*>(c));
-            else
-                splitk_reduce_kernel<float><<<grid, block, 0, stream>>>(static_cast<const float*>(workspace), sp, mn, alpha, static_cast<float*>(c));
-            return hipGetLastError();
-        }
-        if (c_dtype == BF16 && rot_out_dtype == BF16 && rot_mask && rotated) {
-            *rotated = true;
-            const RotEpilogue rot{rot_mask, rot_signs, hadamard_scale(32, rot_scale_dtype)};
-            return launch_big4<uint16_t, true>(a_codes, a_scales, b_codes, b_scales, M, N, K, alpha, c, at, bt, 1, cus, stream, rot);
-        }
-        if (c_dtype == BF16) return launch_big4<uint16_t>(a_codes, a_scales, b_codes, b_scales, M, N, K, alpha, c, at, bt, 1, cus, stream);
-        return launch_big4<float>(a_codes, a_scales, b_codes, b_scales, M, N, K, alpha, c, at, bt, 1, cus, stream);
-    }
-    return launch_gemm<128, 128, 64, 64>(a_codes, a_scales, b_codes, b_scales, M, N, K, alpha, c, c_dtype, stream);
+    if (M >= (1ll << 31) || N >= (1ll << 31) || K >= (1ll << 31)) return hipErrorInvalidValue;
+    const TileProduct p = make_product(a_codes, a_scales, b_codes, b_scales, M, N, K, alpha, c, a_layout, b_layout);
+    return run_product(choose_product(p, c_dtype, c_dtype, workspace, workspace_bytes), p, c_dtype, c_dtype, workspace, stream);
+}
+
+// The product with the rotation in the persistent kernel's epilogue (bf16, Hadamard block 32)
+bool gemm_persistent_rotates(const uint8_t* a_scales, const uint8_t* b_scales, int64_t M, int64_t N, int64_t K) {
+    return gemm_supports_tiled(M, N, K) && K > 768 && persistent_serves(M, N, K, a_scales, b_scales, nullptr);
+}
+hipError_t gemm_persistent_rotated(TileProduct p, hipStream_t stream) {
+    return run_product({ProductChoice::PERSISTENT, 0, 1, true}, p, BF16, BF16, nullptr, stream);
 }
 
 }  // namespace qm

@@ -1,0 +1,427 @@
+// FP4 x FP4 "TN" product on tiles from 64 x 32 to 256 x 128: everything that the persistent 256 x 256 kernel of gemm.hip
+// is too coarse for -- short contractions, matrices with few tiles, and any number of rows and (multiples of eight) columns.
+//
+// One design, five tile shapes.  A workgroup of W waves owns a BM x BN tile, each wave WM x WN of it in 32 x 32 blocks of
+// v_mfma_scale_f32_32x32x64_f8f6f4.  Operands go global -> LDS directly (16 bytes per lane, XOR-swizzled 16-byte slots)
+// into a ring of STAGES K steps of 128, scales as one dword per row and step; one barrier per step.  Rows past the end of a
+// matrix are requested as its last row (their products are dropped), so no request leaves the operands.  bf16 results pass
+// through the ring's LDS and leave as 16-byte pieces of whole rows; on that way a lane holds eight consecutive columns,
+// which is what the masked inverse Hadamard rotation of the layer's backward pass works on: it is applied there (blocks of
+// 32, 64 or 128 along N), with the arithmetic of the stand-alone kernel, bit for bit, and the rotated-basis gradient never
+// travels through memory.  Two independent products of the same element types can share a grid (the two gradient products
+// of a small layer: neither fills the chip alone).
+//
+// What bounds it: at 256 x 128 the LDS reads of the K loop (1.5 x the 256 x 256 kernel's bytes per flop) and, for short
+// contractions, the tile boundary, which the neighbour workgroup on the same CU covers; the smaller tiles are latency-bound
+// and exist to put more workgroups on the chip.  Accumulation order over K is the same in every shape (and in gemm.hip's
+// kernels): results do not depend on the choice.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include <type_traits>
+
+#include "gemm_common.h"
+#include "hadamard_octet.h"
+
+namespace qm {
+
+namespace {
+
+template <int BM_, int BN_, int WM_, int WN_, int STAGES_, int OCC_>
+struct TileShape {
+    static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, STAGES = STAGES_, OCC = OCC_;   // OCC: workgroups per CU
+    static constexpr int kWavesN = BN / WN, kWaves = (BM / WM) * kWavesN, kThreads = kWaves * 64;
+    static constexpr int TM = WM / 32, TN = WN / 32;
+    static constexpr int kALoads = BM / 16 / kWaves, kBLoads = BN / 16 / kWaves;   // 1 KiB wave-loads per wave and K step
+    static constexpr int kAUnits = (BM + 63) / 64, kUnits = kAUnits + (BN + 63) / 64;   // 64 scale dwords each
+    static constexpr int kSLoads = (kUnits + kWaves - 1) / kWaves;
+    static constexpr int kLoads = kALoads + kBLoads + kSLoads;   // requests per wave and K step
+    static constexpr int kBOff = BM * kRowBytes, kSAOff = (BM + BN) * kRowBytes, kSBOff = kSAOff + kAUnits * 256;
+    static constexpr int kStageBytes = kSAOff + kUnits * 256;
+    static constexpr int kRingBytes = STAGES * kStageBytes;
+    static constexpr int kMUnits = BM * BN / 2048, kMLoads = (kMUnits + kWaves - 1) / kWaves;   // mask words of the tile, 64 at a time
+    static constexpr bool kMaskEarly = BM < 256;                 // 256 x 128: no room beside the ring for two workgroups per CU
+    static constexpr int kPitch = BN * 2 + 16;                   // bytes per staged row of the bf16 tile
+    static constexpr int kChunks = BN / 8;                       // 16-byte pieces per row
+    static constexpr int kRowsPerPass = kThreads / kChunks, kPasses = BM / kRowsPerPass;
+    static_assert(kALoads * 16 * kWaves == BM && kBLoads * 16 * kWaves == BN, "whole wave-loads per wave");
+    static constexpr int kMaskOff = kMaskEarly ? kRingBytes : (BM * kPitch + 255) / 256 * 256;
+    static constexpr int kSmemBytes = kRingBytes + (kMaskEarly ? kMUnits * 256 : 0);
+    static_assert(kMaskOff + kMUnits * 256 <= kSmemBytes && kSmemBytes * OCC <= 160 * 1024, "LDS of the resident workgroups");
+    static_assert(BM * kPitch <= kRingBytes, "the epilogue stages through the operand ring");
+    static_assert(TM == 1 || TM == 2 || TM == 4, "scale dwords of a lane are read as one vector");
+    static_assert(TN == 1 || TN == 2, "scale dwords of a lane are read as one vector");
+};
+
+template <int N>
+__device__ __forceinline__ void read_dwords(const uint8_t* p, uint32_t (&v)[N]) {
+    if constexpr (N == 4) {
+        const uint4 q = *reinterpret_cast<const uint4*>(p);
+        v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+    } else if constexpr (N == 2) {
+        const uint2 q = *reinterpret_cast<const uint2*>(p);
+        v[0] = q.x; v[1] = q.y;
+    } else {
+        v[0] = *reinterpret_cast<const uint32_t*>(p);
+    }
+}
+
+template <class S>
+struct TilePlan {
+    const uint8_t* a;   // uniform: first code byte of the tile's panels (K step 0)
+    const uint8_t* b;
+    const uint8_t* s[S::kSLoads];      // uniform: scale array behind this wave's scale requests
+    uint32_t voff_a[S::kALoads];       // this lane's byte offset from it: a row of the wave-load (clamped to the matrix) and
+    uint32_t voff_b[S::kBLoads];       //   the swizzled 16-byte column
+    uint32_t voff_s[S::kSLoads];
+    uint32_t half_back;                // pieces 2 and 3 of a half step re-read pieces 0 and 1
+    int kstep_a, kstep_b;              // bytes from one K step to the next: 64 row-major, 1024 tiled
+    uint32_t lds_a, lds_b, lds_s[S::kSLoads];   // wave-uniform LDS addresses (stage 0)
+};
+
+// half: the step covers only 64 contraction indices (the last step of a K with K % 128 == 64, row-major operands).  Its
+// lanes request the row's final two 16-byte pieces in place of all four, and the scale dword that ends with the row's last
+// byte (two bytes early), so that no request leaves the row; the consumer shifts that dword down by 16 bits, which puts
+// the two real scale bytes first and zeros (2^-127: products vanish) where the missing half of the step would be.
+template <class S>
+__device__ __forceinline__ void tile_issue(const TilePlan<S>& p, int stage, int ks, bool half) {
+    const uint32_t off = (uint32_t)stage * S::kStageBytes;
+    const uint32_t back = half ? p.half_back : 0u;
+    const uint8_t* a = p.a + (int64_t)ks * p.kstep_a;
+    const uint8_t* b = p.b + (int64_t)ks * p.kstep_b;
+#pragma unroll
+    for (int j = 0; j < S::kALoads; ++j) load_lds_b128_s(a, p.voff_a[j] - back, p.lds_a + off + j * 1024);
+#pragma unroll
+    for (int j = 0; j < S::kBLoads; ++j) load_lds_b128_s(b, p.voff_b[j] - back, p.lds_b + off + j * 1024);
+    const int sback = half ? 2 : 0;
+#pragma unroll
+    for (int u = 0; u < S::kSLoads; ++u) load_lds_b32_s(p.s[u] + ks * 4 - sback, p.voff_s[u], p.lds_s[u] + off);
+}
+
+template <class S>
+struct TileFrags {
+    uint4 a[S::TM], b[S::TN];
+};
+template <class S>
+__device__ __forceinline__ void tile_read(const uint8_t* __restrict__ stage, int a_off, int b_off, TileFrags<S>& f) {
+#pragma unroll
+    for (int i = 0; i < S::TM; ++i) f.a[i] = *reinterpret_cast<const uint4*>(stage + a_off + i * 32 * kRowBytes);
+#pragma unroll
+    for (int j = 0; j < S::TN; ++j) f.b[j] = *reinterpret_cast<const uint4*>(stage + b_off + j * 32 * kRowBytes);
+}
+// SWAP: B's rows (n) are the instruction's first operand, so a lane ends up with quads of consecutive n of one m
+template <class S, int SUB, bool SWAP, bool ZERO>
+__device__ __forceinline__ void tile_mfma(const TileFrags<S>& f, const uint32_t (&sca)[S::TM], const uint32_t (&scb)[S::TN],
+                                          v16f (&acc)[S::TM][S::TN]) {
+#pragma unroll
+    for (int i = 0; i < S::TM; ++i) {
+        const v8i av = v8i{(int)f.a[i].x, (int)f.a[i].y, (int)f.a[i].z, (int)f.a[i].w, 0, 0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < S::TN; ++j) {
+            const v8i bv = v8i{(int)f.b[j].x, (int)f.b[j].y, (int)f.b[j].z, (int)f.b[j].w, 0, 0, 0, 0};
+            v16f cin;
+            if constexpr (ZERO) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) cin[e] = 0.0f;
+            } else {
+                cin = acc[i][j];
+            }
+            if constexpr (SWAP)
+                acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bv, av, cin, 4, 4, SUB, (int)scb[j], SUB, (int)sca[i]);
+            else
+                acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(av, bv, cin, 4, 4, SUB, (int)sca[i], SUB, (int)scb[j]);
+        }
+    }
+}
+
+template <class S, typename OutT>
+__device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* smem, uint32_t smem_base) {
+    constexpr bool SWAP = sizeof(OutT) == 2;
+    uint8_t* smem_bytes = reinterpret_cast<uint8_t*>(smem);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / S::kWavesN, wn = wave % S::kWavesN;
+    const int lrow = lane & 31, half = lane >> 5;
+    const int M = g.M, N = g.N, K = g.K;
+    const int tiles_m = (M + S::BM - 1) / S::BM, tiles_n = (N + S::BN - 1) / S::BN;
+    const int code_pitch = K / 2, groups = K / 32;
+    const int nk = (K + kBK - 1) / kBK;
+    const int half_step = (K % kBK) ? nk - 1 : -1;  // the K step that covers only 64 indices (K % 128 == 64), or none
+    int tm, tn;
+    tile_of_block<(S::BM >= 256 ? 4 : 8)>(t, tiles_m, tiles_n, tm, tn);
+    const int m0 = tm * S::BM, n0 = tn * S::BN;
+
+    const int swz = (lrow >> 2) & 3;
+    const int a_off0 = (wm * S::WM + lrow) * kRowBytes + (((2 * half) ^ swz) * 16);
+    const int a_off1 = (wm * S::WM + lrow) * kRowBytes + (((2 * half + 1) ^ swz) * 16);
+    const int b_off0 = S::kBOff + (wn * S::WN + lrow) * kRowBytes + (((2 * half) ^ swz) * 16);
+    const int b_off1 = S::kBOff + (wn * S::WN + lrow) * kRowBytes + (((2 * half + 1) ^ swz) * 16);
+    // scales in LDS: A dword p holds row (p / (32 TM)) * WM + (p % TM) * 32 + (p / TM) % 32, so one read fetches the scale
+    // dwords of a lane's TM blocks; B likewise with TN and WN
+    const int a_sc_off = S::kSAOff + (wm * 32 + lrow) * (4 * S::TM);
+    const int b_sc_off = S::kSBOff + (wn * 32 + lrow) * (4 * S::TN);
+    const int sh = 16 * half;
+
+    TilePlan<S> plan;
+    {
+        const int prow = lane >> 2;
+        const int pcv = (lane & 3) ^ ((prow >> 2) & 3);
+        const int64_t row16 = (int64_t)16 * code_pitch;
+        const int last_a = (g.a_tiled ? (M + 15) & ~15 : M) - 1 - m0, last_b = (g.b_tiled ? (N + 15) & ~15 : N) - 1 - n0;
+        const auto row_off = [&](int r, int tiled) {
+            return tiled ? (uint32_t)((r >> 4) * row16) + (uint32_t)((r & 15) * 64 + pcv * 16) : (uint32_t)(r * code_pitch + pcv * 16);
+        };
+        plan.a = g.a_codes + (int64_t)m0 * code_pitch;   // m0, n0 are multiples of 16: the same expression in both layouts
+        plan.b = g.b_codes + (int64_t)n0 * code_pitch;
+#pragma unroll
+        for (int j = 0; j < S::kALoads; ++j) {
+            const int r = (wave * S::kALoads + j) * 16 + prow;
+            plan.voff_a[j] = row_off(r < last_a ? r : last_a, g.a_tiled);
+        }
+#pragma unroll
+        for (int j = 0; j < S::kBLoads; ++j) {
+            const int r = (wave * S::kBLoads + j) * 16 + prow;
+            plan.voff_b[j] = row_off(r < last_b ? r : last_b, g.b_tiled);
+        }
+        plan.half_back = (uint32_t)(pcv & 2) * 16u;
+        plan.kstep_a = g.a_tiled ? 1024 : kRowBytes;
+        plan.kstep_b = g.b_tiled ? 1024 : kRowBytes;
+        plan.lds_a = (uint32_t)__builtin_amdgcn_readfirstlane((int)(smem_base + wave * S::kALoads * 1024));
+        plan.lds_b = (uint32_t)__builtin_amdgcn_readfirstlane((int)(smem_base + S::kBOff + wave * S::kBLoads * 1024));
+#pragma unroll
+        for (int u = 0; u < S::kSLoads; ++u) {
+            // unit of 64 scale dwords this wave requests; a wave without one of its own repeats another's (same bytes to the
+            // same place), which keeps every wave's count of outstanding requests the same
+            const int unit = (wave + u * S::kWaves) % S::kUnits;
+            const bool is_a = unit < S::kAUnits;
+            const int p = (is_a ? unit : unit - S::kAUnits) * 64 + lane;
+            const int ra = (p / (32 * S::TM)) * S::WM + (p % S::TM) * 32 + (p / S::TM) % 32;
+            const int rb = (p / (32 * S::TN)) * S::WN + (p % S::TN) * 32 + (p / S::TN) % 32;
+            const int la = M - 1 - m0, lb = N - 1 - n0;
+            const int r = is_a ? (ra < la ? ra : la) : (rb < lb ? rb : lb);
+            plan.s[u] = is_a ? g.a_scales + (int64_t)m0 * groups : g.b_scales + (int64_t)n0 * groups;
+            plan.voff_s[u] = (uint32_t)(r * groups);
+            plan.lds_s[u] = (uint32_t)__builtin_amdgcn_readfirstlane((int)(smem_base + S::kSAOff + unit * 256));
+        }
+    }
+    // The rotation's mask words of the tile, [BM][BN / 32] in LDS: with room beside the ring they are requested ahead of
+    // the operands, otherwise into the ring's free end once the K loop is done.
+    const auto issue_mask = [&](uint32_t at) {
+        const int64_t pitch = N / 8;   // N is a multiple of 32 with a mask: whole words
+        const uint8_t* base = g.mask + (int64_t)m0 * pitch;
+#pragma unroll
+        for (int u = 0; u < S::kMLoads; ++u) {
+            const int unit = (wave + u * S::kWaves) % S::kMUnits;
+            const int p = unit * 64 + lane, r = p / (S::BN / 32);
+            const int col = n0 / 32 + p % (S::BN / 32);
+            const int rr = r < M - 1 - m0 ? r : M - 1 - m0, cc = col < N / 32 ? col : N / 32 - 1;
+            load_lds_b32_s(base, (uint32_t)(rr * (int)pitch + cc * 4),
+                           (uint32_t)__builtin_amdgcn_readfirstlane((int)(smem_base + at + unit * 256)));
+        }
+    };
+    if (SWAP && S::kMaskEarly && g.mask) issue_mask(S::kMaskOff);
+
+    const auto issue = [&](int stage, int ks) { tile_issue<S>(plan, stage, ks, ks == half_step); };
+    // the scale dwords of a half step arrive two bytes early (see tile_issue).  Without a branch: a K step is one basic block.
+    const auto settle_scales = [&](uint32_t (&a)[S::TM], uint32_t (&b)[S::TN], int ks) {
+        const uint32_t down = ks == half_step ? 16u : 0u;
+#pragma unroll
+        for (int i = 0; i < S::TM; ++i) a[i] >>= down;
+#pragma unroll
+        for (int j = 0; j < S::TN; ++j) b[j] >>= down;
+    };
+#pragma unroll
+    for (int s = 0; s < S::STAGES; ++s) issue(s, s < nk ? s : nk - 1);
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm((S::STAGES - 1) * S::kLoads));  // step 0 is in; later ones may be pending
+    __syncthreads();
+    TileFrags<S> f0, f1;
+    uint32_t sa[S::TM], sb[S::TN];
+    read_dwords<S::TM>(smem_bytes + a_sc_off, sa);
+    read_dwords<S::TN>(smem_bytes + b_sc_off, sb);
+    settle_scales(sa, sb, 0);
+    tile_read<S>(smem_bytes, a_off0, b_off0, f0);
+
+    v16f acc[S::TM][S::TN];
+    int stage = 0;
+    // one K step: `stage` is the ring slot it consumes and then refills with step s + STAGES
+    auto step = [&](auto first_tag, int s) {
+        constexpr bool FIRST = decltype(first_tag)::value;
+        const int nstage = stage == S::STAGES - 1 ? 0 : stage + 1;
+        const uint8_t* cur = smem_bytes + stage * S::kStageBytes;
+        const uint8_t* nxt = smem_bytes + nstage * S::kStageBytes;
+        uint32_t sca[S::TM], scb[S::TN];
+#pragma unroll
+        for (int i = 0; i < S::TM; ++i) sca[i] = __builtin_amdgcn_ubfe(sa[i], (uint32_t)sh, 16u);
+#pragma unroll
+        for (int j = 0; j < S::TN; ++j) scb[j] = __builtin_amdgcn_ubfe(sb[j], (uint32_t)sh, 16u);
+        tile_read<S>(cur, a_off1, b_off1, f1);
+        tile_mfma<S, 0, SWAP, FIRST>(f0, sca, scb, acc);
+        if constexpr (S::TM * S::TN >= S::TM + S::TN) { QM_SCHED_PAIR(0x100, S::TM + S::TN) }
+        __builtin_amdgcn_sched_barrier(0);
+        // younger than the requests of step s + 1: those of the STAGES - 2 steps after it
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm((S::STAGES - 2) * S::kLoads));
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
+        // past the end: a repeat nobody reads keeps the counts of outstanding requests uniform
+        issue(stage, s + S::STAGES < nk ? s + S::STAGES : nk - 1);
+        read_dwords<S::TM>(nxt + a_sc_off, sa);
+        read_dwords<S::TN>(nxt + b_sc_off, sb);
+        settle_scales(sa, sb, s + 1);
+        tile_read<S>(nxt, a_off0, b_off0, f0);
+        tile_mfma<S, 1, SWAP, false>(f1, sca, scb, acc);
+        if constexpr (S::TM * S::TN >= S::TM + S::TN) { QM_SCHED_PAIR(0x100, S::TM + S::TN) }
+        __builtin_amdgcn_sched_barrier(0);
+        stage = nstage;
+    };
+    step(std::true_type{}, 0);
+    for (int ks = 1; ks < nk; ++ks) step(std::false_type{}, ks);
+    // every request has landed and every wave has read its last fragments: the ring becomes the staging area
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+    __syncthreads();
+    const float alpha = g.alpha;
+    if (SWAP && !S::kMaskEarly && g.mask) issue_mask(S::kMaskOff);
+    if constexpr (SWAP) {
+#pragma unroll
+        for (int i = 0; i < S::TM; ++i)
+#pragma unroll
+            for (int j = 0; j < S::TN; ++j)
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    const v16f& v = acc[i][j];
+                    const v2bf p0 = __builtin_convertvector(v2f{v[4 * b] * alpha, v[4 * b + 1] * alpha}, v2bf);
+                    const v2bf p1 = __builtin_convertvector(v2f{v[4 * b + 2] * alpha, v[4 * b + 3] * alpha}, v2bf);
+                    *reinterpret_cast<uint2*>(smem_bytes + (wm * S::WM + i * 32 + lrow) * S::kPitch + (wn * S::WN + j * 32 + 8 * b + 4 * half) * 2) =
+                        make_uint2(__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1));
+                }
+        if constexpr (!S::kMaskEarly) __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+        __syncthreads();
+        const int chunk = tid % S::kChunks, rsub = tid / S::kChunks;
+        const int out_col = n0 + chunk * 8;
+        typedef uint32_t u4v __attribute__((ext_vector_type(4)));
+        typedef float f4v __attribute__((ext_vector_type(4)));
+        const bool col_ok = out_col < N;   // N is a multiple of 8
+        if (!g.mask) {
+            uint16_t* out = reinterpret_cast<uint16_t*>(g.c) + (int64_t)(m0 + rsub) * N + out_col;
+#pragma unroll
+            for (int r = 0; r < S::kPasses; ++r) {
+                const uint4 v = *reinterpret_cast<const uint4*>(smem_bytes + (r * S::kRowsPerPass + rsub) * S::kPitch + chunk * 16);
+                if (col_ok && m0 + r * S::kRowsPerPass + rsub < M)
+                    __builtin_nontemporal_store(u4v{v.x, v.y, v.z, v.w}, reinterpret_cast<u4v*>(out + (int64_t)r * S::kRowsPerPass * N));
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < S::kPasses; ++r) {
+                const uint4 raw = *reinterpret_cast<const uint4*>(smem_bytes + (r * S::kRowsPerPass + rsub) * S::kPitch + chunk * 16);
+                const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+                float v[8];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    v[2 * i] = u2f(w[i] << 16);
+                    v[2 * i + 1] = u2f(w[i] & 0xffff0000u);
+                }
+                const uint32_t kb = smem_bytes[S::kMaskOff + (r * S::kRowsPerPass + rsub) * (S::BN / 8) + chunk];
+                // whole Hadamard blocks lie in neighbouring lanes (N is a multiple of the block); lanes past N work along
+                if (g.hd == 32) octet_inverse_rotation<32>(v, kb, chunk & 3, g.signs);
+                else if (g.hd == 64) { if constexpr (S::BN >= 64) octet_inverse_rotation<64>(v, kb, chunk & 7, g.signs); }
+                else { if constexpr (S::BN >= 128) octet_inverse_rotation<128>(v, kb, chunk & 15, g.signs); }
+                uint32_t o[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    o[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{v[2 * i] * g.rot_c, v[2 * i + 1] * g.rot_c}, v2bf));
+                const int row = m0 + r * S::kRowsPerPass + rsub;
+                if (col_ok && row < M) {
+                    const int64_t at = (int64_t)row * N + out_col;
+                    if (!g.out_f32) {
+                        __builtin_nontemporal_store(u4v{o[0], o[1], o[2], o[3]}, reinterpret_cast<u4v*>(reinterpret_cast<uint16_t*>(g.c) + at));
+                    } else {   // the bf16-rounded result, widened
+                        f4v* dst = reinterpret_cast<f4v*>(reinterpret_cast<float*>(g.c) + at);
+                        __builtin_nontemporal_store(f4v{u2f(o[0] << 16), u2f(o[0] & 0xffff0000u), u2f(o[1] << 16), u2f(o[1] & 0xffff0000u)}, dst);
+                        __builtin_nontemporal_store(f4v{u2f(o[2] << 16), u2f(o[2] & 0xffff0000u), u2f(o[3] << 16), u2f(o[3] & 0xffff0000u)}, dst + 1);
+                    }
+                }
+            }
+        }
+    } else {
+        float* c = reinterpret_cast<float*>(g.c);
+#pragma unroll
+        for (int i = 0; i < S::TM; ++i)
+#pragma unroll
+            for (int j = 0; j < S::TN; ++j) {
+                const int col = n0 + wn * S::WN + j * 32 + lrow;
+                if (col >= N) continue;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    const int row = m0 + wm * S::WM + i * 32 + 8 * (e / 4) + 4 * half + (e & 3);
+                    if (row < M) c[(int64_t)row * N + col] = acc[i][j][e] * alpha;
+                }
+            }
+    }
+    __syncthreads();  // the staging area is the next tile's ring
+}
+
+// Persistent over the tiles of g, then of h (h.M == 0: none)
+template <class S, typename OutT>
+__global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu((S::OCC * S::kWaves + 3) / 4))) void gemm_mxfp4_tn_tile_kernel(
+    TileProduct g, TileProduct h, int tiles_g, int tiles) {
+    extern __shared__ uint32_t smem[];
+    const uint32_t smem_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint32_t*)smem;
+    for (int t = (int)blockIdx.x; t < tiles; t += (int)gridDim.x) {
+        const bool first = t < tiles_g;   // uniform: every field below is a scalar select
+        TileProduct p;
+#define QM_PICK(f) p.f = first ? g.f : h.f
+        QM_PICK(a_codes); QM_PICK(a_scales); QM_PICK(b_codes); QM_PICK(b_scales); QM_PICK(c); QM_PICK(mask); QM_PICK(M); QM_PICK(N);
+        QM_PICK(K); QM_PICK(a_tiled); QM_PICK(b_tiled); QM_PICK(alpha); QM_PICK(hd); QM_PICK(signs.w[0]); QM_PICK(signs.w[1]);
+        QM_PICK(signs.w[2]); QM_PICK(signs.w[3]); QM_PICK(rot_c); QM_PICK(out_f32);
+#undef QM_PICK
+        tile_run<S, OutT>(p, first ? t : t - tiles_g, smem, smem_base);
+    }
+}
+
+template <class S>
+int tiles_of(const TileProduct& p) { return p.M == 0 ? 0 : ((p.M + S::BM - 1) / S::BM) * ((p.N + S::BN - 1) / S::BN); }
+
+template <class S, typename OutT>
+hipError_t launch_tiles(const TileProduct& g, const TileProduct& h, hipStream_t stream) {
+    auto kern = gemm_mxfp4_tn_tile_kernel<S, OutT>;
+    static std::atomic<bool> lds_allowed[kMaxDevices];
+    hipError_t e = allow_dynamic_lds(kern, S::kSmemBytes, lds_allowed);
+    if (e != hipSuccess) return e;
+    const int tg = tiles_of<S>(g), tiles = tg + tiles_of<S>(h);
+    // a grid that is a multiple of 8 so that tile t and t + grid land on the same XCD
+    int grid = tiles < S::OCC * device_cus() ? tiles : S::OCC * device_cus();
+    if (grid > 8 && grid < tiles) grid -= grid % 8;
+    kern<<<dim3((unsigned)grid), dim3(S::kThreads), S::kSmemBytes, stream>>>(g, h, tg, tiles);
+    return hipGetLastError();
+}
+
+using Tile256x128 = TileShape<256, 128, 128, 64, 3, 2>;
+using Tile128x128 = TileShape<128, 128, 64, 64, 3, 3>;
+using Tile128x64 = TileShape<128, 64, 64, 32, 4, 3>;
+using Tile64x64 = TileShape<64, 64, 32, 32, 4, 4>;
+using Tile64x32 = TileShape<64, 32, 32, 32, 6, 4>;
+
+}  // namespace
+
+bool gemm_tile_serves(int64_t M, int64_t N, int64_t K, int a_tiled, int b_tiled, const void* c) {
+    const bool k_ok = K % kBK == 0 || (K % kBK == 64 && K >= 192 && !a_tiled && !b_tiled);
+    return M > 0 && N >= 8 && N % 8 == 0 && K > 0 && k_ok && M < (1 << 30) && N < (1 << 30) && K < (1 << 23) &&
+           (reinterpret_cast<uintptr_t>(c) & 15) == 0;
+}
+
+hipError_t gemm_tile(int shape, const TileProduct& g, const TileProduct* second, int c_dtype, hipStream_t stream) {
+    TileProduct h{};
+    if (second) h = *second;
+    const auto go = [&](auto s) {
+        using S = decltype(s);
+        return c_dtype == BF16 ? launch_tiles<S, uint16_t>(g, h, stream) : launch_tiles<S, float>(g, h, stream);
+    };
+    switch (shape) {
+        case TILE_256x128: return go(Tile256x128{});
+        case TILE_128x128: return go(Tile128x128{});
+        case TILE_128x64: return go(Tile128x64{});
+        case TILE_64x64: return go(Tile64x64{});
+        default: return go(Tile64x32{});
+    }
+}
+
+}  // namespace qm

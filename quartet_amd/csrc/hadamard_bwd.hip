@@ -10,6 +10,7 @@
 
 #include <type_traits>
 
+#include "hadamard_octet.h"
 #include "qm_jobs.h"
 #include "qm_kernels.h"
 #include "qm_math.h"
@@ -21,58 +22,13 @@ namespace {
 typedef float v2f __attribute__((ext_vector_type(2)));
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 
-__device__ __forceinline__ float dpp_quad_xor1(float v) {
-    return u2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2u(v), 0xB1, 0xF, 0xF, true));
-}
-__device__ __forceinline__ float dpp_quad_xor2(float v) {
-    return u2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2u(v), 0x4E, 0xF, 0xF, true));
-}
-template <int LANE_MASK>
-__device__ __forceinline__ float lane_xor(float v) {
-    if constexpr (LANE_MASK == 1) return dpp_quad_xor1(v);
-    else if constexpr (LANE_MASK == 2) return dpp_quad_xor2(v);
-    else return __shfl_xor(v, LANE_MASK, 64);
-}
-template <int LANE_MASK>
-__device__ __forceinline__ void cross_lane_stage(float (&v)[8], int lane_in_chunk) {
-    // lower lane of a butterfly: own + partner; upper lane: partner - own = partner + (-own)
-    const uint32_t flip = (lane_in_chunk & LANE_MASK) ? 0x80000000u : 0u;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const float p = lane_xor<LANE_MASK>(v[i]);
-        v[i] = p + u2f(f2u(v[i]) ^ flip);
-    }
-}
-
 // Eight values of one octet (already loaded into v) -> mask, sign flips, butterfly within the Hadamard block (whose other
 // octets sit in the neighbouring lanes), c, store.  ROUND_OUT (fp32 out): the result is rounded to bf16 and then widened --
 // what a bf16 result converted to fp32 afterwards holds, without the separate conversion pass.
 template <typename TOut, int HD, bool ROUND_OUT>
 __device__ __forceinline__ void rotate_octet(float (&v)[8], uint32_t keep, int64_t octet, float c, const SignBits& sb, TOut* __restrict__ out) {
     const int lic = (int)(octet & (HD / 8 - 1));
-    const int j0 = lic * 8;
-    const uint32_t sign8 = (sb.w[j0 >> 5] >> (j0 & 31)) & 0xffu;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        // g * mask as the reference multiplies: the factor is the float 1.0 or 0.0 built from the bit
-        const uint32_t all = (uint32_t)__builtin_amdgcn_sbfe((int)keep, i, 1);  // 0 or ~0
-        const float x = v[i] * u2f(all & 0x3f800000u);
-        v[i] = u2f(f2u(x) ^ (((sign8 >> i) & 1u) << 31));
-    }
-#pragma unroll
-    for (int h = 1; h < 8; h <<= 1) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            if (i & h) continue;
-            float a = v[i], b = v[i + h];
-            v[i] = a + b;
-            v[i + h] = a - b;
-        }
-    }
-    cross_lane_stage<1>(v, lic);
-    cross_lane_stage<2>(v, lic);
-    if constexpr (HD >= 64) cross_lane_stage<4>(v, lic);
-    if constexpr (HD >= 128) cross_lane_stage<8>(v, lic);
+    octet_inverse_rotation<HD>(v, keep, lic, sb);
     if constexpr (sizeof(TOut) == 2) {
         uint32_t w[4];
 #pragma unroll
@@ -102,6 +58,8 @@ __device__ __forceinline__ void rotate_octet(float (&v)[8], uint32_t keep, int64
 // ROUND_IN (bf16 in, fp32 out): the result is rounded to bf16 before it is widened.
 template <typename TIn, typename TOut, int HD, bool ROUND_IN = false>
 struct HadamardBwdJob {
+    static constexpr int kLds = 0;
+    static constexpr int kWaves = 1;
     const TIn* g;
     int64_t n_octets;
     float c;
@@ -143,6 +101,8 @@ struct HadamardBwdJob {
 // dtype is bf16 (MID_BF16).  One pass in place of the reduction followed by the rotation, with the same arithmetic.
 template <bool MID_BF16, typename TOut>
 struct SplitKRotateJob {
+    static constexpr int kLds = 0;
+    static constexpr int kWaves = 1;
     const float* partial;
     int splits;
     int64_t mn;
@@ -240,25 +200,24 @@ hipError_t masked_hadamard_bwd_hd32_pair(const void* ga, int64_t na, int scale_d
     const SignBits sa{{sign_a, 0, 0, 0}}, sb{{sign_b, 0, 0, 0}};
     const float ca = hadamard_scale(32, scale_dtype_a), cb = hadamard_scale(32, scale_dtype_b);
     if (dtype == BF16 && out_dtype_b == F32) {
-        launch_job_pair(HadamardBwdJob<uint16_t, uint16_t, 32>(ga, na, ca, sa, mask_a, out_a),
-                        HadamardBwdJob<uint16_t, float, 32, true>(gb, nb, cb, sb, mask_b, out_b), stream);
+        launch_jobs(stream, HadamardBwdJob<uint16_t, uint16_t, 32>(ga, na, ca, sa, mask_a, out_a),
+                    HadamardBwdJob<uint16_t, float, 32, true>(gb, nb, cb, sb, mask_b, out_b));
     } else if (dtype == BF16) {
         using J = HadamardBwdJob<uint16_t, uint16_t, 32>;
-        launch_job_pair(J(ga, na, ca, sa, mask_a, out_a), J(gb, nb, cb, sb, mask_b, out_b), stream);
+        launch_jobs(stream, J(ga, na, ca, sa, mask_a, out_a), J(gb, nb, cb, sb, mask_b, out_b));
     } else {
         using J = HadamardBwdJob<float, float, 32>;
-        launch_job_pair(J(ga, na, ca, sa, mask_a, out_a), J(gb, nb, cb, sb, mask_b, out_b), stream);
+        launch_jobs(stream, J(ga, na, ca, sa, mask_a, out_a), J(gb, nb, cb, sb, mask_b, out_b));
     }
     return hipGetLastError();
 }
 
 // c = masked inverse rotation (blocks of 32 along the rows) of the reduced product alpha * sum_s partial[s]; see SplitKRotateJob
 hipError_t splitk_reduce_rotated(const float* partial, int splits, int64_t mn, float alpha, int mid_dtype, const uint8_t* maskbits,
-                                 uint32_t sign_word, int scale_dtype, void* out, int out_dtype, hipStream_t stream) {
+                                 uint32_t sign_word, float c, void* out, int out_dtype, hipStream_t stream) {
     if (mn == 0) return hipSuccess;
     if (mn % 32 || !maskbits || splits < 1 || (mid_dtype == F32 && out_dtype != F32)) return hipErrorInvalidValue;
     const SignBits sb{{sign_word, 0, 0, 0}};
-    const float c = hadamard_scale(32, scale_dtype);
     if (mid_dtype == BF16 && out_dtype == BF16) launch_job(SplitKRotateJob<true, uint16_t>(partial, splits, mn, alpha, c, sb, maskbits, out), stream);
     else if (mid_dtype == BF16) launch_job(SplitKRotateJob<true, float>(partial, splits, mn, alpha, c, sb, maskbits, out), stream);
     else launch_job(SplitKRotateJob<false, float>(partial, splits, mn, alpha, c, sb, maskbits, out), stream);

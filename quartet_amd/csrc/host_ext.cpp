@@ -114,6 +114,7 @@ struct Layer : torch::CustomClassHolder {
     Tensor x_dense, w_dense;   // dense rotations of the forward quantizers (rerotate="O32"), or undefined
     int64_t T = 0, I = 0, O = 0;
     int layout = QM_LAYOUT_ROWMAJOR;
+    bool seed_base_ok = false;
     at::ScalarType x_dtype{}, w_dtype{};
     std::vector<int64_t> x_shape;
     explicit Layer(py::handle q) : g_q(q) {}
@@ -132,10 +133,13 @@ LayerPtr make_layer(int a_hd, py::handle a_signs, int w_hd, py::handle w_signs, 
 void set_extents(Layer& l, int64_t T, const Tensor& weight) {
     l.T = T; l.I = weight.size(1); l.O = weight.size(0);
     l.w_dtype = weight.scalar_type();
-    // Tiled code bytes (16 rows x 128 elements contiguous) when every operand of the three products qualifies: all three
-    // extents multiples of 128 and at least 256, Hadamard block 32 throughout; row-major codes otherwise.
-    const auto ok = [](int64_t d) { return d % 128 == 0 && d >= 256; };
-    l.layout = ok(l.T) && ok(l.I) && ok(l.O) && l.a_hd == 32 && l.w_hd == 32 && l.g_hd == 32 ? QM_LAYOUT_TILED : QM_LAYOUT_ROWMAJOR;
+    // Tiled code bytes (16 rows x 128 elements contiguous, extents padded with zeros).  Row-major where the padding is not
+    // available: rows of y that are not whole 16-byte pieces, and dense forward rotations off the multiples of 128.
+    const bool dense = l.x_dense.defined() || l.w_dense.defined();
+    const bool classic = l.T % 128 == 0 && l.I % 128 == 0 && l.O % 128 == 0;
+    l.layout = l.O % 8 || (dense && !classic) ? QM_LAYOUT_ROWMAJOR : QM_LAYOUT_PADDED;
+    // the extents for which a device seed base is promised (set_device_seed_base)
+    l.seed_base_ok = classic && l.T >= 256 && l.I >= 256 && l.O >= 256 && l.a_hd == 32 && l.w_hd == 32 && l.g_hd == 32;
 }
 
 Tensor packed_buffer(int64_t rows, int64_t cols, const Tensor& like) { return bytes((int64_t)qm_packed_operand_bytes(rows, cols), like); }
@@ -156,7 +160,7 @@ Tensor quantize_dense_into_packed(const Tensor& x2, const Tensor& dense, int lay
     check(qm_packed_operand_offsets(rows, cols, off), "qm_packed_operand_offsets");
     uint8_t* base = packed.data_ptr<uint8_t>();
     check(qm_quantize_mxfp4_dense(x2.data_ptr(), dtype_code(x2.scalar_type()), rows, cols, m.data_ptr<float>(), QM_QUEST_RTN, 0, 0,
-                                  base + off[0], base + off[1], base + off[2], nullptr, layout, stream_of(x2)),
+                                  base + off[0], base + off[1], base + off[2], nullptr, layout == QM_LAYOUT_PADDED ? QM_LAYOUT_TILED : layout, stream_of(x2)),
           "qm_quantize_mxfp4_dense");
     return packed;
 }
@@ -216,7 +220,7 @@ Gradients backward_products(const Layer& l, const Tensor& e, const Tensor& packe
         py::gil_scoped_acquire gil;
         try {
             const py::tuple drawn = py::reinterpret_steal<py::object>(PyObject_CallFunction(
-                g_draw, "OOLLL", l.g_q.p, l.layout == QM_LAYOUT_TILED ? Py_True : Py_False, (long long)l.T, (long long)l.I, (long long)l.O));
+                g_draw, "OOLLL", l.g_q.p, l.seed_base_ok ? Py_True : Py_False, (long long)l.T, (long long)l.I, (long long)l.O));
             if (!drawn.ptr()) throw py::error_already_set();
             g_signs = signs_of(drawn[0]);
             const py::tuple s = drawn[1];

@@ -1,6 +1,6 @@
 // Job kernels.  A job is the work of one kernel launch as a struct: its arguments, `blocks` (how many 256-thread
-// workgroups it needs) and `run(block)`, the body of one workgroup.  `job_kernel` runs one job; `job_pair_kernel`
-// runs two independent jobs in a single grid, the first job's blocks first: the second job's blocks fill the machine
+// workgroups it needs) and `run(block)`, the body of one workgroup.  `job_kernel` runs one job or
+// several independent ones in a single grid, the first job's blocks first: the next job's blocks fill the machine
 // while the first one drains, and the pause between two dependent launches of a stream is paid once.
 //
 // Wave priorities.  A job's workgroup computes its addresses, requests its input, works on it for a few thousand
@@ -22,27 +22,44 @@ __device__ __forceinline__ void job_requests_issued() { __builtin_amdgcn_s_setpr
 // before the final stores: a wave that is about to leave makes room for the next one sooner
 __device__ __forceinline__ void job_stores_next() { __builtin_amdgcn_s_setprio(3); }
 
-template <class A>
-__global__ __launch_bounds__(256) void job_kernel(A a) {
-    job_starts();
-    a.run(blockIdx.x);
+// Workgroup scratch of a job: dynamic LDS, sized for the largest job of the launch (J::kLds bytes).  As a static array in
+// each job's body, two jobs of one kernel would be given the sum of their needs.
+extern __shared__ uint4 job_lds[];
+
+template <class A, class... Rest>
+__device__ __forceinline__ void run_job(unsigned bid, const A& a, const Rest&... rest) {
+    if constexpr (sizeof...(Rest) == 0) {
+        a.run(bid);
+    } else {
+        if (bid < a.blocks) a.run(bid);
+        else run_job(bid - a.blocks, rest...);
+    }
 }
 
-template <class A, class B>
-__global__ __launch_bounds__(256) void job_pair_kernel(A a, B b) {
-    job_starts();
-    if (blockIdx.x < a.blocks) a.run(blockIdx.x);
-    else b.run(blockIdx.x - a.blocks);
+constexpr int least(int a) { return a; }
+template <typename... Ts>
+constexpr int least(int a, Ts... rest) {
+    const int r = least(rest...);
+    return a < r ? a : r;
 }
 
+// J::kWaves: resident waves per SIMD the job is to be compiled for (1: no wish), for the job of a launch that wants fewest
+template <class... Jobs>
+__global__ __launch_bounds__(256, least(Jobs::kWaves...)) void job_kernel(Jobs... jobs) {
+    job_starts();
+    run_job(blockIdx.x, jobs...);
+}
+
+// independent jobs in one grid, the first job's blocks first
+template <class... Jobs>
+void launch_jobs(hipStream_t stream, const Jobs&... jobs) {
+    unsigned lds = 0;
+    ((lds = (unsigned)Jobs::kLds > lds ? (unsigned)Jobs::kLds : lds), ...);
+    job_kernel<Jobs...><<<dim3((jobs.blocks + ...)), dim3(256), lds, stream>>>(jobs...);
+}
 template <class A>
 void launch_job(const A& job, hipStream_t stream) {
-    job_kernel<<<dim3(job.blocks), dim3(256), 0, stream>>>(job);
-}
-
-template <class A, class B>
-void launch_job_pair(const A& a, const B& b, hipStream_t stream) {
-    job_pair_kernel<<<dim3(a.blocks + b.blocks), dim3(256), 0, stream>>>(a, b);
+    launch_jobs(stream, job);
 }
 
 }  // namespace qm

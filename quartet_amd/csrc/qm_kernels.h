@@ -15,6 +15,11 @@ struct SignBits {
 // [R/16][C/128][16 rows][64 bytes] -- the 16 rows x 128 elements one GEMM wave-load fetches are 1 KiB contiguous.
 enum CodeLayout : int { LAYOUT_ROWMAJOR = 0, LAYOUT_TILED = 1 };
 
+// A tiled operand of any extents is stored with its rows padded to 16 and its columns to 128: the padding columns hold zero
+// codes and zero scale bytes (they add exact zeros to a product), the padding rows are never consumed.
+__host__ __device__ inline int64_t padded_rows(int64_t r) { return (r + 15) & ~(int64_t)15; }
+__host__ __device__ inline int64_t padded_cols(int64_t c) { return (c + 127) & ~(int64_t)127; }
+
 // byte offset of the 64-byte piece (row r, column block kb) in the tiled layout
 __host__ __device__ inline int64_t tiled_code_offset(int64_t r, int64_t kb, int64_t kblocks) {
     return (((r >> 4) * kblocks + kb) << 10) + ((r & 15) << 6);
@@ -63,12 +68,13 @@ hipError_t requantize_transposed_mxfp4_dense(const uint8_t* codes_in, const uint
                                              uint8_t* codes_out, uint8_t* scales_out, void* dequant, int in_layout,
                                              int out_layout, hipStream_t stream);
 
-// Pairs of independent quantizer launches issued as one grid (Hadamard block 32, tiled codes in and out).
+// The quantizer launches of one layer, several independent ones per grid: tiled codes of any extents (see padded_cols),
+// Hadamard block 32, 64 or 128.
 struct RowmajorArgs {
     const void* x;
     int dtype;
-    int64_t rows, cols;
-    uint32_t sign_word;
+    int64_t rows, cols;   // cols % hd == 0
+    SignBits signs;
     uint8_t* codes;
     uint8_t* scales;
     uint8_t* maskbits;
@@ -76,20 +82,20 @@ struct RowmajorArgs {
 struct RequantArgs {
     const uint8_t* codes_in;
     const uint8_t* scales_in;
-    int64_t R, C;
+    int64_t R, C;         // R % hd == 0, C % 32 == 0
     int val_dtype;
     uint64_t seed;
     uint8_t* codes;
     uint8_t* scales;
 };
-hipError_t quantize_rowmajor_hd32_tiled_pair(const RowmajorArgs& a, const RowmajorArgs& b, hipStream_t stream);
-hipError_t quantize_both_orientations_hd32_tiled(const void* e, int dtype, int64_t T, int64_t O, uint32_t sign_word, int mode,
-                                                 uint64_t seed_rows, uint64_t seed_transposed, uint8_t* codes_rows,
-                                                 uint8_t* scales_rows, uint8_t* codes_transposed, uint8_t* scales_transposed,
-                                                 const uint64_t* seed_base, hipStream_t stream);
-// seed_base: null, or device memory holding a value the kernels add to every seed when they run
-hipError_t requantize_transposed_hd32_tiled_pair(const RequantArgs& a, const RequantArgs& b, uint32_t sign_word, int mode,
-                                                 const uint64_t* seed_base, hipStream_t stream);
+// forward quantizers (quest RTN + clip mask) of x and, unless w is null, of the weight
+hipError_t quantize_layer_forward(const RowmajorArgs& x, const RowmajorArgs* w, int hd, hipStream_t stream);
+// backward: absmax quantizer of e [T, O] along its rows and of its transpose along T, and the transposed, re-quantized
+// packed x and W.  seed_base: null, or device memory holding a value the kernels add to every seed when they run.
+hipError_t quantize_layer_backward(const void* e, int dtype, int64_t T, int64_t O, int hd, const SignBits& signs, int mode,
+                                   uint64_t seed_rows, uint64_t seed_transposed, uint8_t* codes_rows, uint8_t* scales_rows,
+                                   uint8_t* codes_transposed, uint8_t* scales_transposed, const RequantArgs& x, const RequantArgs& w,
+                                   const uint64_t* seed_base, hipStream_t stream);
 hipError_t masked_hadamard_bwd_hd32_pair(const void* ga, int64_t na, int scale_dtype_a, uint32_t sign_a, const uint8_t* mask_a, void* out_a,
                                          const void* gb, int64_t nb, int scale_dtype_b, uint32_t sign_b, const uint8_t* mask_b, void* out_b,
                                          int dtype, int out_dtype_b, hipStream_t stream);
@@ -122,21 +128,52 @@ hipError_t requantize_transposed_mxfp4(const uint8_t* codes_in, const uint8_t* s
 hipError_t gemm_mxfp4_tn(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
                          const uint8_t* b_scales, int64_t M, int64_t N, int64_t K, float alpha, void* c, int c_dtype,
                          int a_layout, int b_layout, void* workspace, size_t workspace_bytes, hipStream_t stream);
-// the same product with the masked inverse Hadamard rotation of the layer's backward pass (hd 32, along N) fused into the
-// store of the result where the kernel serving the shape can do it: in the persistent kernel's bf16 epilogue (c_dtype and
-// rot_out_dtype both BF16), or in the ordered reduction of a product cut into K ranges (the product rounded to c_dtype,
-// the rotated result stored in rot_out_dtype: c_dtype, or F32 holding the bf16-rounded result).  *rotated reports whether
-// it was; c then holds rot_out_dtype elements, otherwise the plain product in c_dtype.
-bool gemm_will_rotate(const uint8_t* a_scales, const uint8_t* b_scales, int64_t M, int64_t N, int64_t K, int c_dtype, int rot_out_dtype,
-                      const void* workspace, size_t workspace_bytes);
-hipError_t gemm_mxfp4_tn_rotated(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
-                                 const uint8_t* b_scales, int64_t M, int64_t N, int64_t K, float alpha, void* c, int c_dtype,
-                                 int a_layout, int b_layout, void* workspace, size_t workspace_bytes, const uint8_t* rot_mask,
-                                 uint32_t rot_signs, int rot_scale_dtype, int rot_out_dtype, bool* rotated, hipStream_t stream);
 // the reduction of a product cut into K ranges with that rotation applied to the reduced values (hadamard_bwd.hip)
 hipError_t splitk_reduce_rotated(const float* partial, int splits, int64_t mn, float alpha, int mid_dtype, const uint8_t* maskbits,
-                                 uint32_t sign_word, int scale_dtype, void* out, int out_dtype, hipStream_t stream);
+                                 uint32_t sign_word, float c, void* out, int out_dtype, hipStream_t stream);
 size_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
+
+// The product on small and middle-sized tiles (gemm_tile.hip).  Any M; N % 8 == 0; K % 128 == 0, or K % 128 == 64 with
+// row-major operands; c 16-byte aligned.  A tiled operand's last block of 16 rows exists in memory whatever its row count.
+// mask: null, or the clip-mask bits [M, N / 8] of the masked inverse Hadamard rotation (block hd in {32, 64, 128} along N,
+// N % hd == 0, column signs, factor rot_c) that is then applied to the bf16-rounded product; out_f32 stores its bf16
+// result widened to fp32.  bf16 c_dtype only.
+struct TileProduct {
+    const uint8_t* a_codes;
+    const uint8_t* a_scales;
+    const uint8_t* b_codes;
+    const uint8_t* b_scales;
+    void* c;
+    const uint8_t* mask;
+    int M, N, K;
+    int a_tiled, b_tiled;
+    float alpha;
+    int hd;
+    SignBits signs;
+    float rot_c;
+    int out_f32;
+};
+enum TileKind : int { TILE_256x128 = 0, TILE_128x128 = 1, TILE_128x64 = 2, TILE_64x64 = 3, TILE_64x32 = 4 };
+bool gemm_tile_serves(int64_t M, int64_t N, int64_t K, int a_tiled, int b_tiled, const void* c);
+// one product, or two independent ones of the same element type in one grid
+hipError_t gemm_tile(int kind, const TileProduct& g, const TileProduct* second, int c_dtype, hipStream_t stream);
+
+// The kernel a product runs on (gemm.hip).  Products with p.mask set ask for the masked inverse rotation; `rotates` tells
+// whether that kernel applies it (p.c then holds rot_out_dtype elements: c_dtype, or F32 holding the bf16-rounded result)
+// or the caller has to (p.c then holds the plain product in c_dtype).
+struct ProductChoice {
+    enum Path : int { GENERIC = 0, PERSISTENT = 1, TILE = 2 } path;
+    int kind;      // TileKind
+    int splits;    // K ranges of the persistent kernel
+    bool rotates;
+};
+TileProduct make_product(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes, const uint8_t* b_scales, int64_t M, int64_t N,
+                         int64_t K, float alpha, void* c, int a_layout, int b_layout);
+ProductChoice choose_product(const TileProduct& p, int c_dtype, int rot_out_dtype, const void* workspace, size_t workspace_bytes);
+hipError_t run_product(const ProductChoice& c, const TileProduct& p, int c_dtype, int rot_out_dtype, void* workspace, hipStream_t stream);
+// the rotation in the persistent kernel's bf16 epilogue (Hadamard block 32)
+bool gemm_persistent_rotates(const uint8_t* a_scales, const uint8_t* b_scales, int64_t M, int64_t N, int64_t K);
+hipError_t gemm_persistent_rotated(TileProduct p, hipStream_t stream);
 // C = alpha * A (packed MXFP4 [M, K]) x B (bf16 [K, N] row-major): K % 64 == 0, N % 8 == 0
 bool gemm_fp4_bf16_nn_supported(int64_t M, int64_t N, int64_t K);
 hipError_t gemm_fp4_bf16_nn(const uint8_t* a_codes, const uint8_t* a_scales, const void* b, int64_t M, int64_t N, int64_t K,

@@ -315,6 +315,84 @@ __device__ __forceinline__ void dense_rotate(float (&v)[32], const DenseFrag& f)
     }
 }
 
+// ---- Hadamard blocks 64 and 128 ---------------------------------------------------------------------------
+// Same one-group-per-lane layout; a Hadamard chunk is HD/32 consecutive lanes (a lane pair or a quad).  The
+// five in-register stages are followed by the stride-32 (and stride-64) stages across the lanes of the chunk, one
+// DPP-fed multiply-add per element: own + partner in the lower lane of a butterfly, own - partner in the upper one.
+// The upper lane's exact value is partner - own = -(own - partner): rounding is symmetric, so the negation commutes
+// with it, and it is folded into the column sign applied at the end (a lane's values are negated once per stage in
+// which it is the upper lane).  The column signs differ per lane of the chunk; they are applied as lane masks held in
+// scalar registers (bit l of mask j: negate element j in lane l), one select per element.
+template <int CTRL>
+__device__ __forceinline__ void cross_lane_stage(float (&v)[32], float s) {
+    // s = +1 in the lower lane, -1 in the upper one.  An instruction reads its own destination register from the
+    // partner lane; the leading s_nop keeps the two wait states a DPP read needs after a vector write to that register
+    // (the compiler does not look into assembly statements).
+#define QM_X(N) "v_fmac_f32_dpp %" #N ", %" #N ", %16 quad_perm:[%17,%18,%19,%20] row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+#define QM_STAGE16(B)                                                                                                   \
+    asm volatile("s_nop 1\n\t" QM_X(0) QM_X(1) QM_X(2) QM_X(3) QM_X(4) QM_X(5) QM_X(6) QM_X(7) QM_X(8) QM_X(9) QM_X(10) QM_X(11)  \
+                 QM_X(12) QM_X(13) QM_X(14) QM_X(15)                                                                     \
+                 : "+v"(v[(B)]), "+v"(v[(B) + 1]), "+v"(v[(B) + 2]), "+v"(v[(B) + 3]), "+v"(v[(B) + 4]), "+v"(v[(B) + 5]),  \
+                   "+v"(v[(B) + 6]), "+v"(v[(B) + 7]), "+v"(v[(B) + 8]), "+v"(v[(B) + 9]), "+v"(v[(B) + 10]),             \
+                   "+v"(v[(B) + 11]), "+v"(v[(B) + 12]), "+v"(v[(B) + 13]), "+v"(v[(B) + 14]), "+v"(v[(B) + 15])          \
+                 : "v"(s), "n"(CTRL & 3), "n"((CTRL >> 2) & 3), "n"((CTRL >> 4) & 3), "n"((CTRL >> 6) & 3))
+    QM_STAGE16(0);
+    QM_STAGE16(16);
+#undef QM_STAGE16
+#undef QM_X
+}
+
+// Per-element negation fields of the wide kernel: bit p of field j = column sign of rotated element 32 p + j, xor 1 for
+// the lanes of a chunk whose index has an odd number of set bits (their values come out of the cross-lane stages negated).
+template <int HD>
+SignBits wide_sign_fields(const SignBits& sb) {
+    constexpr int P = HD / 32;
+    SignBits sf{{0u, 0u, 0u, 0u}};
+    for (int j = 0; j < 32; ++j) {
+        uint32_t field = 0u;
+        for (int p = 0; p < P; ++p) field |= (((sb.w[p] >> j) & 1u) ^ (uint32_t)(__builtin_popcount((unsigned)p) & 1)) << p;
+        sf.w[(j * P) >> 5] |= field << ((j * P) & 31);
+    }
+    return sf;
+}
+
+
+// What a quantizer's rotation needs at run time: the factor hd^-1/2 and its column signs (HD = 32: one word; wider blocks:
+// the per-element fields of wide_sign_fields)
+struct Rotation {
+    float c;
+    SignBits signs;
+};
+template <int HD>
+Rotation make_rotation(int dtype, const SignBits& sb) {
+    if constexpr (HD == 32) return Rotation{hadamard_scale(32, dtype), sb};
+    else return Rotation{hadamard_scale(HD, dtype), wide_sign_fields<HD>(sb)};
+}
+// x @ H for a lane's group of 32; a block of 64 or 128 spans the lane pair or quad whose lanes hold its groups in order
+template <int HD>
+__device__ __forceinline__ void rotate_block(float (&v)[32], const Rotation& r) {
+    if constexpr (HD == 32) {
+        rotate_group(v, r.c, r.signs.w[0]);
+    } else {
+        butterfly32(v);
+        const int part = (int)threadIdx.x & (HD / 32 - 1);
+        cross_lane_stage<0xB1>(v, (part & 1) ? -1.0f : 1.0f);                           // quad_perm [1,0,3,2]: stride 32
+        if constexpr (HD == 128) cross_lane_stage<0x4E>(v, (part & 2) ? -1.0f : 1.0f);  // quad_perm [2,3,0,1]: stride 64
+        // the fields hold, per element j, HD/32 bits: bit p = negate element j in the chunk's lane p (column sign xor the
+        // stage negations above).  field * 0x5555... (or 0x1111...) spreads it over the wave's chunks.
+        constexpr int P = HD / 32;
+        constexpr uint32_t kUnit = P == 2 ? 0x55555555u : 0x11111111u;
+#pragma unroll
+        for (int j = 0; j < 32; ++j) {
+            const uint32_t field = (r.signs.w[(j * P) >> 5] >> ((j * P) & 31)) & ((1u << P) - 1u);  // wave-uniform: scalar registers
+            const uint32_t half = field * kUnit;
+            const uint64_t m = ((uint64_t)half << 32) | half;
+            const float scaled = v[j] * r.c;
+            asm("v_cndmask_b32_e64 %0, %1, -%1, %2" : "=v"(v[j]) : "v"(scaled), "s"(m));
+        }
+    }
+}
+
 // rotate (hd = 32) + quantize the group in v; gi is its logical (row-major) group index, which also keys the
 // random stream; ci is the index of its 16 code bytes in the code buffer (= gi for row-major codes)
 template <typename T, int MODE, bool WANT_MASK>
@@ -393,47 +471,56 @@ void launch_rowmajor_dense(int mode, const void* x, int64_t rows, int64_t cols, 
 // b % chunks of 512 columns (four code tiles); wave w owns rows 4w..4w+3 of the block, lane l its row l / 16 and
 // group l % 16 of the run: the wave reads four contiguous KiB (bf16) and writes, per tile, four rows' 64-byte pieces
 // = 256 contiguous bytes.  The four scale bytes of four adjacent groups are gathered into one dword store.
-template <typename T, int MODE, bool WANT_MASK>
+// PADDED: any number of rows; columns that are not a multiple of 128 are completed with zero codes and scales.  (Whole tiles
+// have instantiations of their own: the edge tests cost the kernel 5 to 10 %.)
+template <typename T, int MODE, bool WANT_MASK, int HD = 32, bool PADDED = false>
 struct RowmajorTiledJob {
+    static constexpr int kLds = 0;
+    static constexpr int kWaves = 1;
     const T* x;
-    int64_t cols;
-    int chunks;
-    float c;
-    uint32_t sign_word;
+    int rows, groups, groups_p, chunks;   // groups of 32 per row: of the tensor, of its padded code tiles
+    Rotation rot;
     uint64_t seed;
     const uint64_t* seed_base = nullptr;  // device memory, or null: a value the kernel adds to `seed` when it runs
     GroupOut out;
     unsigned blocks;
 
-    RowmajorTiledJob(const void* x_, int64_t rows, int64_t cols_, float c_, uint32_t sign_word_, uint64_t seed_,
-                     const GroupOut& out_)
-        : x(reinterpret_cast<const T*>(x_)), cols(cols_), chunks((int)((cols_ / 128 + 3) / 4)), c(c_),
-          sign_word(sign_word_), seed(seed_), out(out_), blocks((unsigned)((rows / 16) * ((cols_ / 128 + 3) / 4))) {}
+    RowmajorTiledJob(const void* x_, int64_t rows_, int64_t cols_, const Rotation& rot_, uint64_t seed_, const GroupOut& out_)
+        : x(reinterpret_cast<const T*>(x_)), rows((int)rows_), groups((int)(cols_ / 32)), groups_p((int)(padded_cols(cols_) / 32)),
+          chunks((groups_p + 15) / 16), rot(rot_), seed(seed_), out(out_), blocks((unsigned)(padded_rows(rows_) / 16 * chunks)) {}
 
     __device__ __forceinline__ void run(unsigned bid) const {
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        const int groups = (int)(cols / 32);  // per row
         const unsigned rb = bid / (unsigned)chunks;
         const int g = (int)(bid - rb * chunks) * 16 + (lane & 15);  // group within the row
-        if (g >= groups) return;  // cols % 128 == 0: quads of lanes leave together, the gather below sees full quads
         const int rin = wave * 4 + (lane >> 4);  // row within the block
+        // groups_p is a multiple of four: quads of lanes leave together, but for the padding lanes of a row's last quad
+        if (g >= (PADDED ? groups_p : groups)) return;
+        if (PADDED && (int)rb * 16 + rin >= rows) return;
         // uniform 64-bit block bases + small per-lane offsets
+        const int pitch = PADDED ? groups_p : groups;   // groups per row of the code and scale arrays
         const int64_t gi = (int64_t)rb * 16 * groups + (rin * groups + g);
-        const int64_t ci = (int64_t)rb * 16 * groups + ((g >> 2) * 64 + rin * 4 + (g & 3));
+        const int64_t ci = (int64_t)rb * 16 * pitch + ((g >> 2) * 64 + rin * 4 + (g & 3));
+        if (PADDED && g >= groups) {
+            out.codes[ci] = make_uint4(0u, 0u, 0u, 0u);
+            return;
+        }
         float v[32];
         load_group<T>(x + gi * 32, v);
         job_requests_issued();
-        rotate_group(v, c, sign_word);
+        rotate_block<HD>(v, rot);
         GroupCodes o;
         quantize_group_regs<MODE, WANT_MASK>(v, seed_base ? seed + *seed_base : seed, gi, o);
         job_stores_next();
         out.codes[ci] = make_uint4(o.w[0], o.w[1], o.w[2], o.w[3]);
-        // quad_perm broadcasts of lanes 1, 2, 3 of each quad
+        // quad_perm broadcasts of lanes 1, 2, 3 of each quad (0 from a padding lane: it has left)
         const uint32_t s1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)o.scale_byte, 0x55, 0xf, 0xf, false);
         const uint32_t s2 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)o.scale_byte, 0xAA, 0xf, 0xf, false);
         const uint32_t s3 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)o.scale_byte, 0xFF, 0xf, 0xf, false);
-        if ((lane & 3) == 0)
-            *reinterpret_cast<uint32_t*>(out.scales + gi) = o.scale_byte | (s1 << 8) | (s2 << 16) | (s3 << 24);
+        if ((lane & 3) == 0) {
+            const int64_t si = PADDED ? (int64_t)rb * 16 * pitch + (rin * pitch + g) : gi;
+            *reinterpret_cast<uint32_t*>(out.scales + si) = o.scale_byte | (s1 << 8) | (s2 << 16) | (s3 << 24);
+        }
         if constexpr (WANT_MASK) out.maskbits[gi] = o.keep;
         if (out.dequant) store_dequant<T>(reinterpret_cast<T*>(out.dequant) + gi * 32, o);
     }
@@ -446,10 +533,10 @@ void launch_rowmajor_g32(int mode, const void* x, int64_t rows, int64_t cols, bo
     if (tiled) {
         const auto go = [&](auto job) { launch_job(job, stream); };
         switch (mode) {
-            case QUEST_RTN: go(RowmajorTiledJob<T, QUEST_RTN, WANT_MASK>(x, rows, cols, c, sign_word, seed, out)); break;
-            case ABSMAX_RTN: go(RowmajorTiledJob<T, ABSMAX_RTN, WANT_MASK>(x, rows, cols, c, sign_word, seed, out)); break;
-            case ABSMAX_SR: go(RowmajorTiledJob<T, ABSMAX_SR, WANT_MASK>(x, rows, cols, c, sign_word, seed, out)); break;
-            default: go(RowmajorTiledJob<T, QUEST_SR, WANT_MASK>(x, rows, cols, c, sign_word, seed, out)); break;
+            case QUEST_RTN: go(RowmajorTiledJob<T, QUEST_RTN, WANT_MASK>(x, rows, cols, Rotation{c, {{sign_word, 0, 0, 0}}}, seed, out)); break;
+            case ABSMAX_RTN: go(RowmajorTiledJob<T, ABSMAX_RTN, WANT_MASK>(x, rows, cols, Rotation{c, {{sign_word, 0, 0, 0}}}, seed, out)); break;
+            case ABSMAX_SR: go(RowmajorTiledJob<T, ABSMAX_SR, WANT_MASK>(x, rows, cols, Rotation{c, {{sign_word, 0, 0, 0}}}, seed, out)); break;
+            default: go(RowmajorTiledJob<T, QUEST_SR, WANT_MASK>(x, rows, cols, Rotation{c, {{sign_word, 0, 0, 0}}}, seed, out)); break;
         }
         return;
     }
@@ -463,33 +550,6 @@ void launch_rowmajor_g32(int mode, const void* x, int64_t rows, int64_t cols, bo
     }
 }
 
-// ---- Hadamard blocks 64 and 128, row-major ---------------------------------------------------------------
-// Same one-group-per-lane layout; a Hadamard chunk is HD/32 consecutive lanes (a lane pair or a quad).  The
-// five in-register stages are followed by the stride-32 (and stride-64) stages across the lanes of the chunk, one
-// DPP-fed multiply-add per element: own + partner in the lower lane of a butterfly, own - partner in the upper one.
-// The upper lane's exact value is partner - own = -(own - partner): rounding is symmetric, so the negation commutes
-// with it, and it is folded into the column sign applied at the end (a lane's values are negated once per stage in
-// which it is the upper lane).  The column signs differ per lane of the chunk; they are applied as lane masks held in
-// scalar registers (bit l of mask j: negate element j in lane l), one select per element.
-template <int CTRL>
-__device__ __forceinline__ void cross_lane_stage(float (&v)[32], float s) {
-    // s = +1 in the lower lane, -1 in the upper one.  An instruction reads its own destination register from the
-    // partner lane; the leading s_nop keeps the two wait states a DPP read needs after a vector write to that register
-    // (the compiler does not look into assembly statements).
-#define QM_X(N) "v_fmac_f32_dpp %" #N ", %" #N ", %16 quad_perm:[%17,%18,%19,%20] row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-#define QM_STAGE16(B)                                                                                                   \
-    asm volatile("s_nop 1\n\t" QM_X(0) QM_X(1) QM_X(2) QM_X(3) QM_X(4) QM_X(5) QM_X(6) QM_X(7) QM_X(8) QM_X(9) QM_X(10) QM_X(11)  \
-                 QM_X(12) QM_X(13) QM_X(14) QM_X(15)                                                                     \
-                 : "+v"(v[(B)]), "+v"(v[(B) + 1]), "+v"(v[(B) + 2]), "+v"(v[(B) + 3]), "+v"(v[(B) + 4]), "+v"(v[(B) + 5]),  \
-                   "+v"(v[(B) + 6]), "+v"(v[(B) + 7]), "+v"(v[(B) + 8]), "+v"(v[(B) + 9]), "+v"(v[(B) + 10]),             \
-                   "+v"(v[(B) + 11]), "+v"(v[(B) + 12]), "+v"(v[(B) + 13]), "+v"(v[(B) + 14]), "+v"(v[(B) + 15])          \
-                 : "v"(s), "n"(CTRL & 3), "n"((CTRL >> 2) & 3), "n"((CTRL >> 4) & 3), "n"((CTRL >> 6) & 3))
-    QM_STAGE16(0);
-    QM_STAGE16(16);
-#undef QM_STAGE16
-#undef QM_X
-}
-
 template <typename T, int MODE, bool WANT_MASK, int HD>
 __global__ __launch_bounds__(256) void quantize_rowmajor_wide_kernel(const T* __restrict__ x, int64_t n_groups, float c,
                                                                      SignBits sf, uint64_t seed, GroupOut out) {
@@ -500,22 +560,7 @@ __global__ __launch_bounds__(256) void quantize_rowmajor_wide_kernel(const T* __
     float v[32];
     load_group<T>(x + gi * 32, v);
     job_requests_issued();
-    butterfly32(v);
-    const int part = (int)threadIdx.x & (HD / 32 - 1);
-    cross_lane_stage<0xB1>(v, (part & 1) ? -1.0f : 1.0f);                           // quad_perm [1,0,3,2]: stride 32
-    if constexpr (HD == 128) cross_lane_stage<0x4E>(v, (part & 2) ? -1.0f : 1.0f);  // quad_perm [2,3,0,1]: stride 64
-    // sf holds, per element j, a field of HD/32 bits: bit p = negate element j in the chunk's lane p (column sign
-    // xor the stage negations above).  field * 0x5555... (or 0x1111...) spreads it over the wave's chunks.
-    constexpr int P = HD / 32;
-    constexpr uint32_t kUnit = P == 2 ? 0x55555555u : 0x11111111u;
-#pragma unroll
-    for (int j = 0; j < 32; ++j) {
-        const uint32_t field = (sf.w[(j * P) >> 5] >> ((j * P) & 31)) & ((1u << P) - 1u);  // wave-uniform: scalar registers
-        const uint32_t half = field * kUnit;
-        const uint64_t m = ((uint64_t)half << 32) | half;
-        const float scaled = v[j] * c;
-        asm("v_cndmask_b32_e64 %0, %1, -%1, %2" : "=v"(v[j]) : "v"(scaled), "s"(m));
-    }
+    rotate_block<HD>(v, Rotation{c, sf});
     GroupCodes o;
     quantize_group_regs<MODE, WANT_MASK>(v, seed, gi, o);
     job_stores_next();
@@ -523,20 +568,6 @@ __global__ __launch_bounds__(256) void quantize_rowmajor_wide_kernel(const T* __
     out.scales[gi] = (uint8_t)o.scale_byte;
     if constexpr (WANT_MASK) out.maskbits[gi] = o.keep;
     if (out.dequant) store_dequant<T>(reinterpret_cast<T*>(out.dequant) + gi * 32, o);
-}
-
-// Per-element negation fields of the wide kernel: bit p of field j = column sign of rotated element 32 p + j, xor 1 for
-// the lanes of a chunk whose index has an odd number of set bits (their values come out of the cross-lane stages negated).
-template <int HD>
-SignBits wide_sign_fields(const SignBits& sb) {
-    constexpr int P = HD / 32;
-    SignBits sf{{0u, 0u, 0u, 0u}};
-    for (int j = 0; j < 32; ++j) {
-        uint32_t field = 0u;
-        for (int p = 0; p < P; ++p) field |= (((sb.w[p] >> j) & 1u) ^ (uint32_t)(__builtin_popcount((unsigned)p) & 1)) << p;
-        sf.w[(j * P) >> 5] |= field << ((j * P) & 31);
-    }
-    return sf;
 }
 
 template <typename T, bool WANT_MASK, int HD>
@@ -567,47 +598,55 @@ struct TrTile {
 };
 constexpr int kTrP = 128;
 
-template <typename T, int MODE, bool DENSE = false>
+// Hadamard blocks 64 and 128 span two or four p-groups of a column.  Those groups then sit in neighbouring lanes (the lane
+// pair or quad of rotate_block) instead of in different waves: a wave covers fewer columns and all p-groups of the block.
+// PADDED: tiled codes of a P that is not a multiple of 128, completed with zero codes and scales.
+template <typename T, int MODE, bool DENSE = false, int HD = 32, bool PADDED = false>
 struct TransposedJob {
+    static constexpr int kLds = TrTile<T>::kQ * (4 * 16 + 4);
+    static constexpr int kWaves = 1;
     const T* x;
     int64_t P, Q;
-    float c;
-    uint32_t sign_word;
+    Rotation rot;
     uint64_t seed;
     const uint64_t* seed_base = nullptr;  // device memory, or null: a value the kernel adds to `seed` when it runs
     uint8_t* codes;
     uint8_t* scales;
     void* dequant;
     bool tiled_out;
-    const float* matrix;  // DENSE: the rotation, [32][32] fp32 (c and sign_word are then unused)
+    const float* matrix;  // DENSE: the rotation, [32][32] fp32 (rot is then unused)
     unsigned grid_p, blocks;
 
-    TransposedJob(const void* x_, int64_t P_, int64_t Q_, float c_, uint32_t sign_word_, uint64_t seed_, uint8_t* codes_,
-                  uint8_t* scales_, void* dequant_, bool tiled_out_, const float* matrix_ = nullptr)
-        : x(reinterpret_cast<const T*>(x_)), P(P_), Q(Q_), c(c_), sign_word(sign_word_), seed(seed_), codes(codes_),
+    TransposedJob(const void* x_, int64_t P_, int64_t Q_, const Rotation& rot_, uint64_t seed_, uint8_t* codes_, uint8_t* scales_,
+                  void* dequant_, bool tiled_out_, const float* matrix_ = nullptr)
+        : x(reinterpret_cast<const T*>(x_)), P(P_), Q(Q_), rot(rot_), seed(seed_), codes(codes_),
           scales(scales_), dequant(dequant_), tiled_out(tiled_out_), matrix(matrix_), grid_p((unsigned)((P_ + kTrP - 1) / kTrP)),
           blocks((unsigned)(((P_ + kTrP - 1) / kTrP) * ((Q_ + TrTile<T>::kQ - 1) / TrTile<T>::kQ))) {}
 
     __device__ __forceinline__ void run(unsigned bid) const {
         constexpr int TQ = TrTile<T>::kQ;
         constexpr int GPL = TrTile<T>::kGroupsPerLane;
-        __shared__ uint4 ocodes[TQ * 4];      // [q][4 groups x 16 B]
-        __shared__ uint32_t oscales[TQ];      // [q][4 B]
+        uint4* ocodes = job_lds;                                               // [q][4 groups x 16 B]
+        uint8_t* oscales = reinterpret_cast<uint8_t*>(job_lds + TQ * 4);       // [q][4 B]
         const int tid = threadIdx.x, lane = tid & 63;
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // tells the compiler it is wave-uniform
         const unsigned bq = bid / grid_p;
         const int64_t p0 = (int64_t)(bid - bq * grid_p) * kTrP, q0 = (int64_t)bq * TQ;
-        const int64_t pbase = p0 + wave * 32;       // this wave's group along p
-        const int64_t qa = q0 + lane * GPL;         // this lane's first column
-        const bool active = pbase < P && qa < Q;    // P % 32 == 0 and Q % 8 == 0: all of a lane's groups or none
+        // this lane's p-group within the strip's four and its load column (GPL adjacent columns)
+        const int pg = HD == 32 ? wave : HD == 64 ? (wave >> 1) * 2 + (lane & 1) : (lane & 3);
+        const int cd = HD == 32 ? lane : HD == 64 ? (wave & 1) * 32 + (lane >> 1) : wave * 16 + (lane >> 2);
+        const int64_t pbase = p0 + pg * 32;
+        const int64_t qa = q0 + cd * GPL;           // this lane's first column
+        const bool active = pbase < P && qa < Q;    // P % HD == 0 and Q % 8 == 0: all of a lane's (and of a chunk's) groups or none
         float v[GPL][32];
         if (active) {
             // uniform row pointers (scalar unit) + the lane's 32-bit dword offset: no per-lane 64-bit address math
-            const uint32_t* row = reinterpret_cast<const uint32_t*>(x + pbase * Q + q0);
             const int64_t row_dw = Q * (int64_t)sizeof(T) / 4;
+            const uint32_t* row = reinterpret_cast<const uint32_t*>(x + (HD == 32 ? pbase : p0) * Q + q0);
+            const uint32_t off = HD == 32 ? (uint32_t)lane : (uint32_t)(pg * 32 * row_dw + cd);
 #pragma unroll
             for (int i = 0; i < 32; ++i) {
-                const uint32_t w = (row + i * row_dw)[(uint32_t)lane];
+                const uint32_t w = (row + i * row_dw)[off];
                 if constexpr (sizeof(T) == 2) {
                     v[0][i] = u2f(w << 16);
                     v[1][i] = u2f(w & 0xffff0000u);
@@ -633,28 +672,34 @@ struct TransposedJob {
             for (int gq = 0; gq < GPL; ++gq) {
                 const int64_t gi = (qa + gq) * (P / 32) + pbase / 32;
                 GroupCodes res;
-                if constexpr (!DENSE) rotate_group(v[gq], c, sign_word);
+                if constexpr (!DENSE) rotate_block<HD>(v[gq], rot);
                 quantize_group_regs<MODE, false>(v[gq], seed_base ? seed + *seed_base : seed, gi, res);
                 if (dequant) store_dequant<T>(reinterpret_cast<T*>(dequant) + gi * 32, res);
-                ocodes[(lane * GPL + gq) * 4 + wave] = make_uint4(res.w[0], res.w[1], res.w[2], res.w[3]);
-                reinterpret_cast<uint8_t*>(oscales)[(lane * GPL + gq) * 4 + wave] = (uint8_t)res.scale_byte;
+                ocodes[(cd * GPL + gq) * 4 + pg] = make_uint4(res.w[0], res.w[1], res.w[2], res.w[3]);
+                oscales[(cd * GPL + gq) * 4 + pg] = (uint8_t)res.scale_byte;
+            }
+        } else if constexpr (PADDED) {
+#pragma unroll
+            for (int gq = 0; gq < GPL; ++gq) {
+                ocodes[(cd * GPL + gq) * 4 + pg] = make_uint4(0u, 0u, 0u, 0u);
+                oscales[(cd * GPL + gq) * 4 + pg] = 0;
             }
         }
         __syncthreads();
-        const int64_t code_pitch = P / 2, scale_pitch = P / 32;
+        const int64_t code_pitch = P / 2, P_p = PADDED ? padded_cols(P) : P, scale_pitch = P_p / 32;
         for (int idx = tid; idx < TQ * 4; idx += 256) {
             const int ql = idx >> 2, part = idx & 3;
-            if (q0 + ql < Q && p0 + part * 32 < P) {
+            if (q0 + ql < Q && p0 + part * 32 < P_p) {
                 // tiled: this workgroup's 128 p are one 64-byte column block, so 16 consecutive q rows form one 1 KiB tile
-                const int64_t off = tiled_out ? tiled_code_offset(q0 + ql, p0 / 128, P / 128) + part * 16
+                const int64_t off = tiled_out ? tiled_code_offset(q0 + ql, p0 / 128, P_p / 128) + part * 16
                                               : (q0 + ql) * code_pitch + p0 / 2 + part * 16;
                 *reinterpret_cast<uint4*>(codes + off) = ocodes[idx];
             }
         }
         if (tid < TQ && q0 + tid < Q) {
-            const uint32_t sw = oscales[tid];
+            const uint32_t sw = reinterpret_cast<const uint32_t*>(oscales)[tid];
             uint8_t* dst = scales + (q0 + tid) * scale_pitch + p0 / 32;
-            if (p0 + kTrP <= P) {
+            if (p0 + kTrP <= P_p) {
                 *reinterpret_cast<uint32_t*>(dst) = sw;
             } else {
                 for (int b = 0; b < 4; ++b)
@@ -674,26 +719,31 @@ struct TransposedJob {
 // 16-byte piece; codes leave through LDS as whole 64-byte row pieces (tiled output: four contiguous 1 KiB tiles per wave).
 constexpr int kRqR = 512, kRqC = 64;
 
-template <int VAL_DTYPE, int MODE, bool DENSE = false>
+// Hadamard blocks 64 and 128 span row groups 2k, 2k + 1 or all four of the wave's: lane l then handles row group l % 4 of
+// column quad l / 4, so that a block's groups sit in neighbouring lanes (rotate_block).  PADDED: tiled codes of extents that are
+// not multiples of 128, read and completed with the padding of zero codes and scales.
+template <int VAL_DTYPE, int MODE, bool DENSE = false, int HD = 32, bool PADDED = false>
 struct RequantJob {
+    static constexpr int kLds = 4 * kRqC * 4 * 16 + kRqC * 16;
+    static constexpr int kWaves = 1;
     const uint8_t* codes_in;
     const uint8_t* scales_in;
     int64_t R, C;
-    float post, c;
-    uint32_t sign_word;
+    float post;
+    Rotation rot;
     uint64_t seed;
     const uint64_t* seed_base = nullptr;  // device memory, or null: a value the kernel adds to `seed` when it runs
     uint8_t* codes;
     uint8_t* scales;
     void* dequant;
     bool tiled_in, tiled_out;
-    const float* matrix;  // DENSE: the rotation, [32][32] fp32 (c and sign_word are then unused)
+    const float* matrix;  // DENSE: the rotation, [32][32] fp32 (rot is then unused)
     unsigned grid_r, blocks;
 
-    RequantJob(const uint8_t* codes_in_, const uint8_t* scales_in_, int64_t R_, int64_t C_, float post_, float c_,
-               uint32_t sign_word_, uint64_t seed_, uint8_t* codes_, uint8_t* scales_, void* dequant_, bool tiled_in_,
-               bool tiled_out_, const float* matrix_ = nullptr)
-        : codes_in(codes_in_), scales_in(scales_in_), R(R_), C(C_), post(post_), c(c_), sign_word(sign_word_), seed(seed_),
+    RequantJob(const uint8_t* codes_in_, const uint8_t* scales_in_, int64_t R_, int64_t C_, float post_, const Rotation& rot_,
+               uint64_t seed_, uint8_t* codes_, uint8_t* scales_, void* dequant_, bool tiled_in_, bool tiled_out_,
+               const float* matrix_ = nullptr)
+        : codes_in(codes_in_), scales_in(scales_in_), R(R_), C(C_), post(post_), rot(rot_), seed(seed_),
           codes(codes_), scales(scales_), dequant(dequant_), tiled_in(tiled_in_), tiled_out(tiled_out_), matrix(matrix_),
           grid_r((unsigned)((R_ + kRqR - 1) / kRqR)),
           blocks((unsigned)(((R_ + kRqR - 1) / kRqR) * ((C_ + kRqC - 1) / kRqC))) {}
@@ -727,12 +777,22 @@ struct RequantJob {
             dense_rotate(v[0], frag);
             dense_rotate(v[1], frag);
         }
-        if (!active) return;
+        if (!active) {
+            if constexpr (PADDED) {
+#pragma unroll
+                for (int gq = 0; gq < 2; ++gq) {
+                    const int cl = 4 * cq + 2 * P + gq;
+                    ocodes[cl * 4 + rg] = make_uint4(0u, 0u, 0u, 0u);
+                    oscales[cl * 16 + wave * 4 + rg] = 0;
+                }
+            }
+            return;
+        }
 #pragma unroll
         for (int gq = 0; gq < 2; ++gq) {
             const int64_t gi = (ca + 2 * P + gq) * (R / 32) + rbase / 32;
             GroupCodes res;
-            if constexpr (!DENSE) rotate_group(v[gq], c, sign_word);
+            if constexpr (!DENSE) rotate_block<HD>(v[gq], rot);
             quantize_group_regs<MODE, false>(v[gq], seed_base ? seed + *seed_base : seed, gi, res);
             if (dequant) store_dequant<T>(reinterpret_cast<T*>(dequant) + gi * 32, res);
             const int cl = 4 * cq + 2 * P + gq;
@@ -742,15 +802,15 @@ struct RequantJob {
     }
 
     __device__ __forceinline__ void run(unsigned bid) const {
-        __shared__ uint4 ocodes_all[4][kRqC * 4];  // per wave: [c][4 row groups x 16 B]
-        __shared__ uint4 oscales_all[kRqC];        // [c][16 scale bytes: wave-major, then row group]
+        uint4* ocodes_all = job_lds;                        // per wave: [c][4 row groups x 16 B]
+        uint4* oscales_all = job_lds + 4 * kRqC * 4;        // [c][16 scale bytes: wave-major, then row group]
         const int tid = threadIdx.x, lane = tid & 63;
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // tells the compiler it is wave-uniform
         const unsigned bc = bid / grid_r;
         const int64_t r0 = (int64_t)(bid - bc * grid_r) * kRqR, c0 = (int64_t)bc * kRqC;
-        const int64_t in_code_pitch = C / 2, in_scale_pitch = C / 32;
+        const int64_t in_code_pitch = C / 2, C_p = PADDED ? padded_cols(C) : C, in_scale_pitch = C_p / 32, R_p = PADDED ? padded_cols(R) : R;
         const int64_t rw = r0 + wave * 128;          // this wave's first row
-        const int rg = lane >> 4, cq = lane & 15;    // row group within the wave, column quad
+        const int rg = HD == 32 ? lane >> 4 : lane & 3, cq = HD == 32 ? lane & 15 : lane >> 2;   // row group within the wave, column quad
         const int64_t rbase = rw + 32 * rg;
         const int64_t ca = c0 + 4 * cq;              // this lane's first column
         const bool active = rbase < R && ca < C;     // R % 32 == 0 and C % 32 == 0: all of a lane's groups or none
@@ -759,8 +819,8 @@ struct RequantJob {
         if (active) {
             // Uniform row pointers (scalar unit) + the lane's 32-bit byte offset: no per-lane 64-bit address math.
             // Tiled input: rows are 64 bytes apart inside a 16-row block, blocks (C / 128) KiB apart.
-            const int64_t blk = (C / 128) * 1024;
-            const uint8_t* cu = tiled_in ? codes_in + tiled_code_offset(rw, c0 / 128, C / 128) + (c0 & 127) / 2
+            const int64_t blk = (C_p / 128) * 1024;
+            const uint8_t* cu = tiled_in ? codes_in + tiled_code_offset(rw, c0 / 128, C_p / 128) + (c0 & 127) / 2
                                          : codes_in + rw * in_code_pitch + c0 / 2;
             const uint32_t lane_off = (uint32_t)((tiled_in ? 2 * rg * blk : 32 * rg * in_code_pitch) + 2 * cq);
             const int64_t row_step = tiled_in ? 64 : in_code_pitch;                 // next row of a 16-row block
@@ -784,18 +844,18 @@ struct RequantJob {
         job_requests_issued();
         DenseFrag frag;
         if constexpr (DENSE) load_dense_frag(matrix, VAL_DTYPE, frag);
-        uint4* ocodes = ocodes_all[wave];
+        uint4* ocodes = ocodes_all + wave * (kRqC * 4);
         uint8_t* oscales = reinterpret_cast<uint8_t*>(oscales_all);
         column_pair<0>(cw, sc, frag, active, ca, rbase, cq, rg, wave, ocodes, oscales);
         column_pair<1>(cw, sc, frag, active, ca, rbase, cq, rg, wave, ocodes, oscales);
         __syncthreads();
-        const int64_t code_pitch = R / 2, scale_pitch = R / 32;
+        const int64_t code_pitch = R / 2, scale_pitch = R_p / 32;
         // codes: each wave writes its own 64 x 64-byte tile
 #pragma unroll
         for (int it = 0; it < 4; ++it) {
             const int idx = it * 64 + lane, cl = idx >> 2, part = idx & 3;
-            if (c0 + cl < C && rw + part * 32 < R) {
-                const int64_t off = tiled_out ? tiled_code_offset(c0 + cl, rw / 128, R / 128) + part * 16
+            if (c0 + cl < C && rw + part * 32 < R_p) {
+                const int64_t off = tiled_out ? tiled_code_offset(c0 + cl, rw / 128, R_p / 128) + part * 16
                                               : (c0 + cl) * code_pitch + rw / 2 + part * 16;
                 *reinterpret_cast<uint4*>(codes + off) = ocodes[idx];
             }
@@ -808,33 +868,39 @@ struct RequantJob {
                 *reinterpret_cast<uint4*>(dst) = sw;
             } else {
                 const uint32_t w4[4] = {sw.x, sw.y, sw.z, sw.w};
-                for (int b = 0; b < 16; ++b)
-                    if (r0 + b * 32 < R) dst[b] = (uint8_t)(w4[b >> 2] >> (8 * (b & 3)));
+                if constexpr (PADDED) {   // whole dwords: the row count is padded to 128
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        if (r0 + j * 128 < R) *reinterpret_cast<uint32_t*>(dst + 4 * j) = w4[j];
+                } else {
+                    for (int b = 0; b < 16; ++b)
+                        if (r0 + b * 32 < R) dst[b] = (uint8_t)(w4[b >> 2] >> (8 * (b & 3)));
+                }
             }
         }
     }
 };
 
 template <typename T, bool DENSE>
-void launch_transposed_g32(int mode, const void* x, int64_t P, int64_t Q, float c, uint32_t sign_word, uint64_t seed,
+void launch_transposed_g32(int mode, const void* x, int64_t P, int64_t Q, const Rotation& rot, uint64_t seed,
                            uint8_t* codes, uint8_t* scales, void* dequant, bool tiled, const float* matrix, hipStream_t stream) {
     switch (mode) {
-        case QUEST_RTN: launch_job(TransposedJob<T, QUEST_RTN, DENSE>(x, P, Q, c, sign_word, seed, codes, scales, dequant, tiled, matrix), stream); break;
-        case ABSMAX_RTN: launch_job(TransposedJob<T, ABSMAX_RTN, DENSE>(x, P, Q, c, sign_word, seed, codes, scales, dequant, tiled, matrix), stream); break;
-        case ABSMAX_SR: launch_job(TransposedJob<T, ABSMAX_SR, DENSE>(x, P, Q, c, sign_word, seed, codes, scales, dequant, tiled, matrix), stream); break;
-        default: launch_job(TransposedJob<T, QUEST_SR, DENSE>(x, P, Q, c, sign_word, seed, codes, scales, dequant, tiled, matrix), stream); break;
+        case QUEST_RTN: launch_job(TransposedJob<T, QUEST_RTN, DENSE>(x, P, Q, rot, seed, codes, scales, dequant, tiled, matrix), stream); break;
+        case ABSMAX_RTN: launch_job(TransposedJob<T, ABSMAX_RTN, DENSE>(x, P, Q, rot, seed, codes, scales, dequant, tiled, matrix), stream); break;
+        case ABSMAX_SR: launch_job(TransposedJob<T, ABSMAX_SR, DENSE>(x, P, Q, rot, seed, codes, scales, dequant, tiled, matrix), stream); break;
+        default: launch_job(TransposedJob<T, QUEST_SR, DENSE>(x, P, Q, rot, seed, codes, scales, dequant, tiled, matrix), stream); break;
     }
 }
 
 template <int VAL_DTYPE, bool DENSE>
 void launch_requant_g32(int mode, const uint8_t* codes_in, const uint8_t* scales_in, int64_t R, int64_t C, float post,
-                        float c, uint32_t sign_word, uint64_t seed, uint8_t* codes, uint8_t* scales, void* dequant,
+                        const Rotation& rot, uint64_t seed, uint8_t* codes, uint8_t* scales, void* dequant,
                         bool tiled_in, bool tiled_out, const float* matrix, hipStream_t stream) {
     switch (mode) {
-        case QUEST_RTN: launch_job(RequantJob<VAL_DTYPE, QUEST_RTN, DENSE>(codes_in, scales_in, R, C, post, c, sign_word, seed, codes, scales, dequant, tiled_in, tiled_out, matrix), stream); break;
-        case ABSMAX_RTN: launch_job(RequantJob<VAL_DTYPE, ABSMAX_RTN, DENSE>(codes_in, scales_in, R, C, post, c, sign_word, seed, codes, scales, dequant, tiled_in, tiled_out, matrix), stream); break;
-        case ABSMAX_SR: launch_job(RequantJob<VAL_DTYPE, ABSMAX_SR, DENSE>(codes_in, scales_in, R, C, post, c, sign_word, seed, codes, scales, dequant, tiled_in, tiled_out, matrix), stream); break;
-        default: launch_job(RequantJob<VAL_DTYPE, QUEST_SR, DENSE>(codes_in, scales_in, R, C, post, c, sign_word, seed, codes, scales, dequant, tiled_in, tiled_out, matrix), stream); break;
+        case QUEST_RTN: launch_job(RequantJob<VAL_DTYPE, QUEST_RTN, DENSE>(codes_in, scales_in, R, C, post, rot, seed, codes, scales, dequant, tiled_in, tiled_out, matrix), stream); break;
+        case ABSMAX_RTN: launch_job(RequantJob<VAL_DTYPE, ABSMAX_RTN, DENSE>(codes_in, scales_in, R, C, post, rot, seed, codes, scales, dequant, tiled_in, tiled_out, matrix), stream); break;
+        case ABSMAX_SR: launch_job(RequantJob<VAL_DTYPE, ABSMAX_SR, DENSE>(codes_in, scales_in, R, C, post, rot, seed, codes, scales, dequant, tiled_in, tiled_out, matrix), stream); break;
+        default: launch_job(RequantJob<VAL_DTYPE, QUEST_SR, DENSE>(codes_in, scales_in, R, C, post, rot, seed, codes, scales, dequant, tiled_in, tiled_out, matrix), stream); break;
     }
 }
 
@@ -885,18 +951,18 @@ hipError_t quantize_rowmajor_wide(const void* x, int dtype, int64_t n, int hd, c
 hipError_t quantize_transposed_hd32(const void* x, int dtype, int64_t P, int64_t Q, uint32_t sign_word, int mode,
                                     uint64_t seed, uint8_t* codes, uint8_t* scales, void* dequant, bool tiled,
                                     hipStream_t stream) {
-    const float c = hadamard_scale(32, dtype);
-    if (dtype == BF16) launch_transposed_g32<uint16_t, false>(mode, x, P, Q, c, sign_word, seed, codes, scales, dequant, tiled, nullptr, stream);
-    else launch_transposed_g32<float, false>(mode, x, P, Q, c, sign_word, seed, codes, scales, dequant, tiled, nullptr, stream);
+    const Rotation rot{hadamard_scale(32, dtype), {{sign_word, 0, 0, 0}}};
+    if (dtype == BF16) launch_transposed_g32<uint16_t, false>(mode, x, P, Q, rot, seed, codes, scales, dequant, tiled, nullptr, stream);
+    else launch_transposed_g32<float, false>(mode, x, P, Q, rot, seed, codes, scales, dequant, tiled, nullptr, stream);
     return hipGetLastError();
 }
 
 hipError_t requantize_transposed_hd32(const uint8_t* codes_in, const uint8_t* scales_in, int64_t R, int64_t C, float post,
                                       int val_dtype, uint32_t sign_word, int mode, uint64_t seed, uint8_t* codes,
                                       uint8_t* scales, void* dequant, bool tiled_in, bool tiled_out, hipStream_t stream) {
-    const float c = hadamard_scale(32, val_dtype);
-    if (val_dtype == BF16) launch_requant_g32<BF16, false>(mode, codes_in, scales_in, R, C, post, c, sign_word, seed, codes, scales, dequant, tiled_in, tiled_out, nullptr, stream);
-    else launch_requant_g32<F32, false>(mode, codes_in, scales_in, R, C, post, c, sign_word, seed, codes, scales, dequant, tiled_in, tiled_out, nullptr, stream);
+    const Rotation rot{hadamard_scale(32, val_dtype), {{sign_word, 0, 0, 0}}};
+    if (val_dtype == BF16) launch_requant_g32<BF16, false>(mode, codes_in, scales_in, R, C, post, rot, seed, codes, scales, dequant, tiled_in, tiled_out, nullptr, stream);
+    else launch_requant_g32<F32, false>(mode, codes_in, scales_in, R, C, post, rot, seed, codes, scales, dequant, tiled_in, tiled_out, nullptr, stream);
     return hipGetLastError();
 }
 
@@ -919,16 +985,16 @@ hipError_t quantize_rowmajor_dense(const void* x, int dtype, int64_t rows, int64
 hipError_t quantize_transposed_dense(const void* x, int dtype, int64_t P, int64_t Q, const float* matrix, int mode,
                                      uint64_t seed, uint8_t* codes, uint8_t* scales, void* dequant, bool tiled,
                                      hipStream_t stream) {
-    if (dtype == BF16) launch_transposed_g32<uint16_t, true>(mode, x, P, Q, 1.0f, 0u, seed, codes, scales, dequant, tiled, matrix, stream);
-    else launch_transposed_g32<float, true>(mode, x, P, Q, 1.0f, 0u, seed, codes, scales, dequant, tiled, matrix, stream);
+    if (dtype == BF16) launch_transposed_g32<uint16_t, true>(mode, x, P, Q, Rotation{}, seed, codes, scales, dequant, tiled, matrix, stream);
+    else launch_transposed_g32<float, true>(mode, x, P, Q, Rotation{}, seed, codes, scales, dequant, tiled, matrix, stream);
     return hipGetLastError();
 }
 
 hipError_t requantize_transposed_dense(const uint8_t* codes_in, const uint8_t* scales_in, int64_t R, int64_t C, float post,
                                        int val_dtype, const float* matrix, int mode, uint64_t seed, uint8_t* codes,
                                        uint8_t* scales, void* dequant, bool tiled_in, bool tiled_out, hipStream_t stream) {
-    if (val_dtype == BF16) launch_requant_g32<BF16, true>(mode, codes_in, scales_in, R, C, post, 1.0f, 0u, seed, codes, scales, dequant, tiled_in, tiled_out, matrix, stream);
-    else launch_requant_g32<F32, true>(mode, codes_in, scales_in, R, C, post, 1.0f, 0u, seed, codes, scales, dequant, tiled_in, tiled_out, matrix, stream);
+    if (val_dtype == BF16) launch_requant_g32<BF16, true>(mode, codes_in, scales_in, R, C, post, Rotation{}, seed, codes, scales, dequant, tiled_in, tiled_out, matrix, stream);
+    else launch_requant_g32<F32, true>(mode, codes_in, scales_in, R, C, post, Rotation{}, seed, codes, scales, dequant, tiled_in, tiled_out, matrix, stream);
     return hipGetLastError();
 }
 
@@ -954,6 +1020,7 @@ struct RmsNormProducer {
     static constexpr int kOutDtype = F32;  // bf16-or-fp32 normalised value times the fp32 gain is fp32
     static constexpr bool kAdd = !std::is_void<TA>::value;
     using TAdd = typename std::conditional<kAdd, TA, T>::type;
+    static constexpr int kLds = kAdd ? 4 * 512 * 16 : 0;
     const T* x;
     const float* gain;
     float* factor;  // [rows]: 1 / sqrt(mean(x^2) + eps), kept for the backward pass
@@ -963,8 +1030,7 @@ struct RmsNormProducer {
 
     // 8 KiB of LDS per wave of the workgroup: staging of the residual sum on its way out
     __device__ __forceinline__ static float4* xsum_area() {
-        __shared__ float4 xbuf[4][512];
-        return xbuf[threadIdx.x >> 6];
+        return reinterpret_cast<float4*>(job_lds) + (threadIdx.x >> 6) * 512;
     }
 
     // The row's factor; `first` leaves with the raw elements of the lane's first group (if it has one).
@@ -1053,6 +1119,7 @@ struct RmsNormProducer {
 template <typename T>
 struct SwiGluProducer {
     static constexpr int kOutDtype = sizeof(T) == 2 ? BF16 : F32;
+    static constexpr int kLds = 0;
     const T* h12;  // [rows, 2 cols]: up, then gate
 
     template <int W = 64>
@@ -1080,6 +1147,8 @@ struct SwiGluProducer {
 // W: lanes per row (64, or 32 / 16 for rows of at most that many groups: two / four rows per wave)
 template <typename P, bool TILED, int W = 64>
 struct ProducedRowsJob {
+    static constexpr int kLds = P::kLds;
+    static constexpr int kWaves = 1;
     P prod;
     int64_t rows, cols;
     float c;
@@ -1100,10 +1169,13 @@ struct ProducedRowsJob {
         const int groups = (int)(cols / 32);
         float v[32];
         const float state = prod.template prepare<W>(row, lane, groups, cols, v, seg);
-        // TILED: cols % 128 == 0, so the four lanes of a quad run the same number of iterations
+        // TILED: the row's groups padded to a multiple of four with zero codes and scales; the padding lanes of the last quad
+        // are inactive in the loop, so that the scale gather reads zeros from them
+        const int groups_p = TILED ? (groups + 3) & ~3 : groups;
+        const auto tile_slot = [&](int g) { return (row >> 4) * 16 * groups_p + ((g >> 2) * 64 + (int)(row & 15) * 4 + (g & 3)); };
         for (int g = lane; g < groups; g += W) {
             const int64_t gi = row * groups + g;
-            const int64_t ci = TILED ? (row >> 4) * 16 * groups + ((g >> 2) * 64 + (int)(row & 15) * 4 + (g & 3)) : gi;
+            const int64_t ci = TILED ? tile_slot(g) : gi;
             prod.load(row, g, cols, state, g == lane, v);
             rotate_group(v, c, sign_word);
             GroupCodes o;
@@ -1114,12 +1186,13 @@ struct ProducedRowsJob {
                 const uint32_t s2 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)o.scale_byte, 0xAA, 0xf, 0xf, false);
                 const uint32_t s3 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)o.scale_byte, 0xFF, 0xf, 0xf, false);
                 if ((lane & 3) == 0)
-                    *reinterpret_cast<uint32_t*>(out.scales + gi) = o.scale_byte | (s1 << 8) | (s2 << 16) | (s3 << 24);
+                    *reinterpret_cast<uint32_t*>(out.scales + row * groups_p + g) = o.scale_byte | (s1 << 8) | (s2 << 16) | (s3 << 24);
             } else {
                 out.scales[gi] = (uint8_t)o.scale_byte;
             }
             out.maskbits[gi] = o.keep;
         }
+        if (TILED && lane < groups_p - groups) out.codes[tile_slot(groups + lane)] = make_uint4(0u, 0u, 0u, 0u);
     }
 };
 
@@ -1180,7 +1253,7 @@ hipError_t swiglu_quantize_hd32(const void* h12, int dtype, int64_t rows, int64_
     return hipGetLastError();
 }
 
-// ---- two independent jobs per launch (the whole-layer entry points) ---------------------------------------------
+// ---- the quantizer launches of one layer ------------------------------------------------------------------------
 
 namespace {
 template <typename F>
@@ -1193,58 +1266,69 @@ void with_absmax_mode(int mode, F&& f) {
     if (mode == ABSMAX_SR) f(std::integral_constant<int, ABSMAX_SR>{});
     else f(std::integral_constant<int, ABSMAX_RTN>{});
 }
+template <typename F>
+void with_flag(bool on, F&& f) {
+    if (on) f(std::true_type{});
+    else f(std::false_type{});
+}
+template <typename F>
+void with_hadamard(int hd, F&& f) {
+    if (hd == 32) f(std::integral_constant<int, 32>{});
+    else if (hd == 64) f(std::integral_constant<int, 64>{});
+    else f(std::integral_constant<int, 128>{});
+}
 }  // namespace
 
-// forward quantizer (quest RTN + clip mask, tiled codes) of two tensors, e.g. the activations and the weight of a layer
-hipError_t quantize_rowmajor_hd32_tiled_pair(const RowmajorArgs& a, const RowmajorArgs& b, hipStream_t stream) {
-    const GroupOut oa{reinterpret_cast<uint4*>(a.codes), a.scales, reinterpret_cast<uint32_t*>(a.maskbits), nullptr};
-    const GroupOut ob{reinterpret_cast<uint4*>(b.codes), b.scales, reinterpret_cast<uint32_t*>(b.maskbits), nullptr};
-    const float ca = hadamard_scale(32, a.dtype), cb = hadamard_scale(32, b.dtype);
-    with_elem_type(a.dtype, [&](auto ta) {
-        with_elem_type(b.dtype, [&](auto tb) {
-            launch_job_pair(RowmajorTiledJob<decltype(ta), QUEST_RTN, true>(a.x, a.rows, a.cols, ca, a.sign_word, 0, oa),
-                            RowmajorTiledJob<decltype(tb), QUEST_RTN, true>(b.x, b.rows, b.cols, cb, b.sign_word, 0, ob), stream);
-        });
-    });
-    return hipGetLastError();
-}
-
-// absmax quantizer of e [T, O] along its rows and of its transpose along T, tiled codes, one pass of launches
-hipError_t quantize_both_orientations_hd32_tiled(const void* e, int dtype, int64_t T, int64_t O, uint32_t sign_word, int mode,
-                                                 uint64_t seed_rows, uint64_t seed_transposed, uint8_t* codes_rows,
-                                                 uint8_t* scales_rows, uint8_t* codes_transposed, uint8_t* scales_transposed,
-                                                 const uint64_t* seed_base, hipStream_t stream) {
-    const GroupOut orow{reinterpret_cast<uint4*>(codes_rows), scales_rows, nullptr, nullptr};
-    const float c = hadamard_scale(32, dtype);
-    with_elem_type(dtype, [&](auto t) {
-        with_absmax_mode(mode, [&](auto m) {
-            using T_ = decltype(t);
-            constexpr int M = decltype(m)::value;
-            TransposedJob<T_, M> jt(e, T, O, c, sign_word, seed_transposed, codes_transposed, scales_transposed, nullptr, true);
-            RowmajorTiledJob<T_, M, false> jr(e, T, O, c, sign_word, seed_rows, orow);
-            jt.seed_base = jr.seed_base = seed_base;
-            launch_job_pair(jt, jr, stream);
-        });
-    });
-    return hipGetLastError();
-}
-
-// transpose + rotate + re-quantize two packed tensors (tiled codes in and out), e.g. Q(W) and Q(x) of a layer
-hipError_t requantize_transposed_hd32_tiled_pair(const RequantArgs& a, const RequantArgs& b, uint32_t sign_word, int mode,
-                                                 const uint64_t* seed_base, hipStream_t stream) {
-    const float ca = hadamard_scale(32, a.val_dtype), cb = hadamard_scale(32, b.val_dtype);
-    const auto with_val = [](int dt, auto&& f) {
-        if (dt == BF16) f(std::integral_constant<int, BF16>{});
-        else f(std::integral_constant<int, F32>{});
+hipError_t quantize_layer_forward(const RowmajorArgs& x, const RowmajorArgs* w, int hd, hipStream_t stream) {
+    const auto out_of = [](const RowmajorArgs& a) {
+        return GroupOut{reinterpret_cast<uint4*>(a.codes), a.scales, reinterpret_cast<uint32_t*>(a.maskbits), nullptr};
     };
-    with_val(a.val_dtype, [&](auto va) {
-        with_val(b.val_dtype, [&](auto vb) {
-            with_absmax_mode(mode, [&](auto m) {
-                constexpr int M = decltype(m)::value;
-                RequantJob<decltype(va)::value, M> ja(a.codes_in, a.scales_in, a.R, a.C, 1.0f, ca, sign_word, a.seed, a.codes, a.scales, nullptr, true, true);
-                RequantJob<decltype(vb)::value, M> jb(b.codes_in, b.scales_in, b.R, b.C, 1.0f, cb, sign_word, b.seed, b.codes, b.scales, nullptr, true, true);
-                ja.seed_base = jb.seed_base = seed_base;
-                launch_job_pair(ja, jb, stream);
+    const auto ragged = [](const RowmajorArgs& a) { return a.rows % 16 != 0 || a.cols % 128 != 0; };
+    with_hadamard(hd, [&](auto h) {
+        with_flag(ragged(x) || (w && ragged(*w)), [&](auto p) {
+            constexpr int HD = decltype(h)::value;
+            const auto job_of = [&](const RowmajorArgs& a, auto t) {
+                return RowmajorTiledJob<decltype(t), QUEST_RTN, true, HD, decltype(p)::value>(a.x, a.rows, a.cols, make_rotation<HD>(a.dtype, a.signs),
+                                                                                              0, out_of(a));
+            };
+            with_elem_type(x.dtype, [&](auto tx) {
+                if (!w) launch_jobs(stream, job_of(x, tx));
+                else with_elem_type(w->dtype, [&](auto tw) { launch_jobs(stream, job_of(x, tx), job_of(*w, tw)); });
+            });
+        });
+    });
+    return hipGetLastError();
+}
+
+hipError_t quantize_layer_backward(const void* e, int dtype, int64_t T, int64_t O, int hd, const SignBits& signs, int mode,
+                                   uint64_t seed_rows, uint64_t seed_transposed, uint8_t* codes_rows, uint8_t* scales_rows,
+                                   uint8_t* codes_transposed, uint8_t* scales_transposed, const RequantArgs& x, const RequantArgs& w,
+                                   const uint64_t* seed_base, hipStream_t stream) {
+    const GroupOut orow{reinterpret_cast<uint4*>(codes_rows), scales_rows, nullptr, nullptr};
+    with_absmax_mode(mode, [&](auto m) {
+        with_hadamard(hd, [&](auto h) {
+            constexpr int M = decltype(m)::value, HD = decltype(h)::value;
+            with_elem_type(dtype, [&](auto t) {
+                with_flag(T % 128 != 0 || O % 128 != 0, [&](auto p) {
+                    using T_ = decltype(t);
+                    constexpr bool PADDED = decltype(p)::value;
+                    const Rotation rot = make_rotation<HD>(dtype, signs);
+                    TransposedJob<T_, M, false, HD, PADDED> jt(e, T, O, rot, seed_transposed, codes_transposed, scales_transposed, nullptr, true);
+                    RowmajorTiledJob<T_, M, false, HD, PADDED> jr(e, T, O, rot, seed_rows, orow);
+                    jt.seed_base = jr.seed_base = seed_base;
+                    launch_jobs(stream, jt, jr);
+                });
+            });
+            const auto ragged = [](const RequantArgs& a) { return a.R % 128 != 0 || a.C % 128 != 0; };
+            with_flag(ragged(x) || ragged(w), [&](auto p) {
+                // a quest-coded operand (post = 1, no de-quantized output): its value type only picks the rounding of hd^-1/2
+                const auto requant = [&](const RequantArgs& a) {
+                    return RequantJob<BF16, M, false, HD, decltype(p)::value>(a.codes_in, a.scales_in, a.R, a.C, 1.0f, make_rotation<HD>(a.val_dtype, signs),
+                                                                              a.seed, a.codes, a.scales, nullptr, true, true);
+                };
+                auto jx = requant(x), jw = requant(w);
+                jx.seed_base = jw.seed_base = seed_base;
+                launch_jobs(stream, jx, jw);
             });
         });
     });

@@ -34,7 +34,7 @@ def set_device_seed_base(tensor):
     _SEED_BASE = tensor
 
 
-def _gradient_draws(g_q, tiled, T, I, O):
+def _gradient_draws(g_q, seed_base_ok, T, I, O):
     """What the backward pass of one layer draws on the host, called by it once: fresh column signs, then one seed per
     stochastic quantization in the order e, W^T, e^T, x^T.  Returns (column signs, seeds, stochastic, dense rotation or
     None, device seed base or None)."""
@@ -42,7 +42,7 @@ def _gradient_draws(g_q, tiled, T, I, O):
     stochastic, dense = g_q.stochastic, g_q._dense is not None
     seeds = (_fresh_seed(), _fresh_seed(), _fresh_seed(), _fresh_seed()) if stochastic else (0, 0, 0, 0)
     base = _SEED_BASE if stochastic else None
-    if base is not None and (dense or not tiled):
+    if base is not None and (dense or not seed_base_ok):
         # the device seed base is read by the pair launches of the tiled layout only: on any other path a captured replay
         # would silently repeat this launch's random streams
         raise _lib.QuartetHipError(
@@ -53,21 +53,14 @@ def _gradient_draws(g_q, tiled, T, I, O):
     return g_q.sign_bits, seeds, stochastic, g_q._dense, base
 
 
-def _use_tiled_codes(T, I, O, a_q, w_q, g_q):
-    """Tiled code bytes (16 rows x 128 elements contiguous) when every operand of the three products qualifies: all
-    three extents multiples of 128 and at least 256, Hadamard block 32 throughout; row-major codes otherwise."""
-    return (all(d % 128 == 0 and d >= 256 for d in (T, I, O)) and
-            a_q.hadamard_dim == 32 and w_q.hadamard_dim == 32 and g_q.hadamard_dim == 32)
-
-
 def _cached_weight(x, weight, a_q, w_q, g_q, weight_cache):
     """(cache key, packed Q(W) or None): Q(W) of an unchanged weight (the micro-steps of one accumulation) is quantized
-    once and kept by the layer."""
+    once and kept by the layer.  The last two entries of the key stand for the code layout, which csrc/host_ext.cpp picks."""
     if weight_cache is None:
         return None, None
-    O, I = weight.shape
-    key = (weight.data_ptr(), weight._version, weight.dtype, O, I, w_q.hadamard_dim, w_q.sign_bits,
-           _use_tiled_codes(x.numel() // x.shape[-1], I, O, a_q, w_q, g_q), None if w_q._dense is None else w_q._dense_epoch)
+    dense = a_q._dense is not None or w_q._dense is not None
+    key = (weight.data_ptr(), weight._version, weight.dtype, weight.shape, w_q.hadamard_dim, w_q.sign_bits,
+           None if w_q._dense is None else w_q._dense_epoch, dense and x.numel() // x.shape[-1] % 128 == 0)
     return key, weight_cache.get(key)
 
 

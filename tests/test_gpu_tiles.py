@@ -1,0 +1,82 @@
+"""The product on every tile size and the whole layer on padded operands, at the extents where tiles and padding can go
+wrong: below one tile, one row or column past a tile, contractions of one step and of half a step, token counts and widths
+that are multiples of 32 only, Hadamard blocks of 32, 64 and 128.  Everything against the oracle."""
+import random
+
+import numpy as np
+import pytest
+import torch
+
+from tests.util import make_input, to_oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    a, b = np.asarray(a, dtype=np.float64), np.asarray(b, dtype=np.float64)
+    return float(np.linalg.norm(a - b) / np.linalg.norm(b))
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 8, 128), (33, 72, 384), (64, 32, 128), (65, 64, 640), (130, 264, 640), (300, 384, 1792),   # 64-row tiles
+                                   (1000, 520, 256), (513, 1096, 1152), (1025, 2056, 128),                                       # larger tiles
+                                   (1063, 576, 1024), (2049, 1024, 1664),                                                        # persistent, ragged rows
+                                   (64, 640, 192), (300, 264, 1728)])                                                            # half steps
+def test_product_on_ragged_extents(oracle, M, N, K):
+    """Row-major operands of any M and N % 8 == 0: fp32 result within accumulation order of the oracle's float64 sums, bf16
+    result the rounding of the fp32 one bit for bit (the same sums in the same order)."""
+    print(f"case product {M}x{N}x{K}", flush=True)
+    from quartet_amd import kernels as Kn
+    g = torch.Generator().manual_seed(M + N + K)
+    mk = lambda r: (torch.randint(0, 256, (r, K // 2), generator=g, dtype=torch.uint8),
+                    torch.randint(120, 131, (r, K // 32), generator=g, dtype=torch.uint8))
+    (ac, as_), (bc, bs) = mk(M), mk(N)
+    dev = [t.to("cuda:0") for t in (ac, as_, bc, bs)]
+    c32 = Kn.gemm_mxfp4_tn(*dev, 1.5, torch.float32, split_k=False)
+    c16 = Kn.gemm_mxfp4_tn(*dev, 1.5, torch.bfloat16, split_k=False)
+    want = 1.5 * oracle.gemm_tn(ac.numpy(), as_.numpy(), bc.numpy(), bs.numpy())
+    assert rel(c32.cpu().numpy(), want) < 1e-5
+    assert torch.equal(c16, c32.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("T,I,O,hd", [(32, 32, 32, 32), (96, 160, 96, 32), (288, 192, 320, 32), (544, 1728, 352, 32), (1056, 640, 1088, 32),
+                                      (64, 64, 64, 64), (192, 320, 128, 64), (128, 128, 128, 128), (384, 256, 640, 128), (1280, 384, 896, 128)])
+def test_layer_on_padded_operands(oracle, T, I, O, hd):
+    """Forward and backward of the production layer against the oracle pipeline (same seeds and signs).  bf16 results: each
+    stored tensor adds one rounding of relative size 2^-9."""
+    print(f"case padded layer T={T} I={I} O={O} hd={hd}", flush=True)
+    import quartet_amd as q
+    x = make_input(T, I, torch.bfloat16, seed=1, outlier_frac=0.01)
+    w = make_input(O, I, torch.bfloat16, seed=2, outlier_frac=0, scale=0.02)
+    dy = make_input(T, O, torch.bfloat16, seed=3, outlier_frac=0, scale=1e-3)
+    layer = q.QuantizedLinear(I, O, bias=False, weight_quantizer=q.QuestMXFP4Quantizer(hadamard_dim=hd),
+                              activation_quantizer=q.QuestMXFP4Quantizer(hadamard_dim=hd),
+                              gradient_quantizer=q.AlbertTsengQuantizer(hadamard_dim=hd, stochastic=True, rerotate="signs"),
+                              backward_scheme=q.BACKWARD_SCHEMES["Q(E)Q(Wt)t_Q(Et)Q(Xt)t"]()).to("cuda:0", torch.bfloat16)
+    with torch.no_grad():
+        layer.weight.copy_(w.to("cuda:0"))
+    xd = x.to("cuda:0").requires_grad_(True)
+    torch.manual_seed(5)
+    random.seed(5)
+    y = layer(xd)
+    y.backward(dy.to("cuda:0"))
+    torch.cuda.synchronize()
+
+    torch.manual_seed(5)
+    random.seed(5)
+    o = oracle
+    signs = np.where(torch.randint(0, 2, (hd,)).numpy() == 0, -1, 1)
+    seeds = [random.getrandbits(63) for _ in range(4)]
+    d = float(o.FOUR_THIRDS)
+    qx = o.quantize(to_oracle(x), hd, mode=o.QUEST_RTN, want_mask=True)
+    qw = o.quantize(to_oracle(w), hd, mode=o.QUEST_RTN, want_mask=True)
+    y_ref = o.gemm_tn(qx["codes"], qx["scales"], qw["codes"], qw["scales"])
+    qe = o.quantize(to_oracle(dy), hd, signs=signs, mode=o.ABSMAX_SR, seed=seeds[0])
+    qwt = o.requantize_transposed(qw["codes"], qw["scales"], hd=hd, signs=signs, mode=o.ABSMAX_SR, seed=seeds[1])
+    gxq = o.gemm_tn(qe["codes"], qe["scales"], qwt["codes"], qwt["scales"], a_post=d, b_post=d)
+    qet = o.quantize(to_oracle(dy), hd, signs=signs, mode=o.ABSMAX_SR, transposed_in=True, seed=seeds[2])
+    qxt = o.requantize_transposed(qx["codes"], qx["scales"], hd=hd, signs=signs, mode=o.ABSMAX_SR, seed=seeds[3])
+    gwq = o.gemm_tn(qet["codes"], qet["scales"], qxt["codes"], qxt["scales"], a_post=d, b_post=d)
+    ste = lambda g, qd: o.masked_hadamard_bwd(g.astype(np.float32), hd, o.BF16, None, qd["mask"], out_dtype=o.F32)
+    assert rel(y.detach().float().cpu().numpy(), y_ref) <= 3e-3
+    assert rel(xd.grad.float().cpu().numpy(), ste(gxq, qx)) <= 5e-3
+    assert rel(layer.weight.grad.float().cpu().numpy(), ste(gwq, qw)) <= 5e-3
