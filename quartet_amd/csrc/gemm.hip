@@ -827,30 +827,47 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 
 // ---- which kernel serves a product ----------------------------------------------------------------------------------
 // Estimated durations in microseconds, fitted to 110 shapes of 0.2 to 900 GF (tiled operands; each kernel that serves the
-// shape was timed): mean error 13 %, and the fastest kernel is the one chosen but for 0.3 % of the time on average.  All
-// kernels give the same bits except a cut into K ranges, so nothing but time hangs on the choice.
+// shape was timed): mean error 13 %, and the fastest kernel is the one chosen but for 0.3 % of the time on average; with cuts
+// into K ranges (60 shapes, 2 to 16 ranges) but for 1.2 %.  All kernels give the same bits except a cut into K ranges, so
+// nothing but time hangs on the choice.
 struct KernelCost {
     int bm, bn, per_cu;              // tile, resident workgroups per CU
     double step, shared, boundary;   // one K step of a workgroup alone on its CU; with n of them: n * shared; per tile
+    double rotate[3];                // what the rotation (blocks of 32, 64, 128) adds to a round of per_cu tiles; 0: not served
 };
-constexpr KernelCost kTileCosts[] = {{256, 128, 2, 0.726, 0.648, 2.4}, {128, 128, 3, 0.198, 0.373, 1.5}, {128, 64, 3, 0.170, 0.277, 0.9},
-                                     {64, 64, 4, 0.129, 0.207, 0.63}, {64, 32, 4, 0.176, 0.139, 0.71}};
-constexpr double kLaunch = 2.3, kPersistentStep = 0.88, kPersistentBoundary = 3.7, kMemory = 3.2e6;   // bytes per us of a reduction pass
+constexpr KernelCost kTileCosts[] = {{256, 128, 2, 0.726, 0.648, 2.4, {5.6, 8.5, 9.6}},
+                                     {128, 128, 3, 0.198, 0.373, 1.5, {2.7, 4.4, 5.0}},
+                                     {128, 64, 3, 0.170, 0.277, 0.9, {1.5, 2.1, 0.0}},
+                                     {64, 64, 4, 0.129, 0.207, 0.63, {0.8, 1.1, 0.0}},
+                                     {64, 32, 4, 0.176, 0.139, 0.71, {0.7, 0.0, 0.0}}};
+constexpr double kLaunch = 2.3, kPersistentStep = 0.88, kPersistentBoundary = 3.7, kPersistentRotate = 3.5;
+constexpr double kMemory = 3.2e6, kRotateMemory = 6.6e6;   // bytes per us of the reduction and of a rotation pass of its own
 
-double tile_cost(const KernelCost& k, int64_t M, int64_t N, int64_t K, int cus) {
-    const int64_t tiles = ((M + k.bm - 1) / k.bm) * ((N + k.bn - 1) / k.bn), steps = (K + kBK - 1) / kBK;
+double ranges_cost(int64_t M, int64_t N, int splits) {   // writing, reading and reducing the partial sums of a cut product
+    return splits == 1 ? 0.0 : kLaunch + (4.0 * splits + 2.0) * (double)M * (double)N / kMemory;
+}
+double tile_cost(const KernelCost& k, int64_t M, int64_t N, int64_t K, int splits, int cus) {
+    const int64_t tiles = ((M + k.bm - 1) / k.bm) * ((N + k.bn - 1) / k.bn) * splits, all = (K + kBK - 1) / kBK, steps = (all + splits - 1) / splits;
     const auto round = [&](int64_t n) {   // n workgroups of one CU side by side
         const double step = k.step > n * k.shared ? k.step : n * k.shared;
         return steps * step + k.boundary * __builtin_sqrt((double)n);
     };
     const int64_t full = tiles / (k.per_cu * cus), rest = tiles % (k.per_cu * cus);
-    return kLaunch + full * round(k.per_cu) + (rest ? round((rest + cus - 1) / cus) : 0.0);
+    return kLaunch + full * round(k.per_cu) + (rest ? round((rest + cus - 1) / cus) : 0.0) + ranges_cost(M, N, splits);
+}
+// the masked inverse rotation in the epilogue of a tile kernel, and as a kernel of its own
+double tile_rotate_cost(const KernelCost& k, int64_t M, int64_t N, int hd, int cus) {
+    const int64_t tiles = ((M + k.bm - 1) / k.bm) * ((N + k.bn - 1) / k.bn);
+    const double rounds = (double)((tiles + cus - 1) / cus) / k.per_cu;
+    return k.rotate[hd == 32 ? 0 : hd == 64 ? 1 : 2] * (rounds > 1.0 ? rounds : 1.0);
+}
+double separate_rotate_cost(int64_t M, int64_t N, int in_bytes, int out_bytes) {
+    return kLaunch + 0.5 + (double)M * (double)N * (in_bytes + out_bytes) / kRotateMemory;
 }
 double persistent_cost(int64_t M, int64_t N, int64_t K, int splits, int cus) {
     const int64_t items = ((M + kBigM - 1) / kBigM) * ((N + kBigN - 1) / kBigN) * splits;
     const int64_t steps = (K / kBK / splits + 3) & ~(int64_t)3;
-    const double t = kLaunch + (double)((items + cus - 1) / cus) * (steps * kPersistentStep + kPersistentBoundary);
-    return splits == 1 ? t : t + kLaunch + (4.0 * splits + 2.0) * (double)M * (double)N / kMemory;
+    return kLaunch + (double)((items + cus - 1) / cus) * (steps * kPersistentStep + kPersistentBoundary) + ranges_cost(M, N, splits);
 }
 
 // The persistent kernel: M any, N a multiple of 64, at least one tile; it walks K in blocks of four steps: K % 512 == 0
@@ -863,22 +880,25 @@ bool persistent_serves(int64_t M, int64_t N, int64_t K, const void* a_scales, co
     if (K % 512 == 0 && ((reinterpret_cast<uintptr_t>(a_scales) | reinterpret_cast<uintptr_t>(b_scales)) & 15)) return false;
     return (reinterpret_cast<uintptr_t>(c) & 15) == 0;
 }
-// How many K ranges to cut a product into so that its (tile, range) items fill the CUs: the divisor s of K / 512 that
-// minimises rounds(s) * steps(s) plus a per-item overhead, each range keeping at least eight K steps.  1 = no split.
-int choose_splits(int64_t M, int64_t N, int64_t K, int cus) {
-    const int64_t tiles = ((M + kBigM - 1) / kBigM) * ((N + kBigN - 1) / kBigN);
-    const int64_t nblk = K / 512;
-    if (K % 512 || tiles * 4 >= cus * 3 || nblk < 4) return 1;
-    int best = 1;
-    double best_cost = 1e30;
-    for (int sp = 1; sp <= nblk && sp <= 64; ++sp) {
-        if (nblk % sp || (nblk / sp) * 4 < 8) continue;
-        const int64_t rounds = (tiles * sp + cus - 1) / cus;
-        const double cost = (double)rounds * ((double)(nblk / sp) * 4 + 6.0) + (sp > 1 ? 4.0 + 0.5 * sp : 0.0);
-        if (cost < best_cost - 1e-9) {
-            best_cost = cost;
-            best = sp;
-        }
+
+// The cheapest cut of a product into K ranges (splits == 1: none is possible): each range keeps at least four K steps, on the
+// persistent kernel whole blocks of four steps and at least two of them.  Few tiles and a long K leave CUs idle: 640 x 1728 x
+// 16512 took 49 us whole and 32 us in three ranges of 128 x 128 tiles, 1536 x 4096 x 16384 110 us and 71 us in two ranges.
+struct Cut {
+    ProductChoice choice;
+    double cost;
+};
+Cut cheapest_cut(int64_t M, int64_t N, int64_t K, bool persistent, bool tiles_ok, int cus) {
+    Cut best{{ProductChoice::GENERIC, 0, 1, false}, 1e30};
+    const int64_t steps = (K + kBK - 1) / kBK;
+    const auto consider = [&](ProductChoice::Path path, int kind, int sp, double cost) {
+        if (cost < best.cost) best = Cut{{path, kind, sp, false}, cost};
+    };
+    for (int sp = 2; sp <= 32 && steps / sp >= 4; ++sp) {
+        if (persistent && K % 512 == 0 && (K / 512) % sp == 0 && K / 512 / sp >= 2)
+            consider(ProductChoice::PERSISTENT, 0, sp, persistent_cost(M, N, K, sp, cus));
+        if (tiles_ok)
+            for (int kind = TILE_256x128; kind <= TILE_64x64; ++kind) consider(ProductChoice::TILE, kind, sp, tile_cost(kTileCosts[kind], M, N, K, sp, cus));
     }
     return best;
 }
@@ -982,47 +1002,95 @@ bool gemm_supports_tiled(int64_t M, int64_t N, int64_t K) {
            K < (1 << 30);
 }
 
+// The candidates of one shape, worked out once and remembered (per thread, a fixed table: 160 estimates take the host
+// several microseconds)
+struct ShapePlan {
+    int64_t M = -1, N = 0, K = 0;
+    int flags = -1;
+    double persistent = 1e30, tile[5] = {};
+    Cut cut{};
+    size_t cut_bytes = 0;       // scratch of the cut, 0 if it would not be made
+    size_t scratch_bytes = 0;   // what a caller is asked to provide: at least cut_bytes
+};
+// Few tiles of the persistent kernel and a long K: callers hold room for the ranges that would fill its CUs, whether or not
+// a cut on smaller tiles, or none, turns out cheaper
+size_t scratch_of_few_tiles(int64_t M, int64_t N, int64_t K, int cus) {
+    const int64_t tiles = ((M + kBigM - 1) / kBigM) * ((N + kBigN - 1) / kBigN), nblk = K / 512;
+    if (K % 512 || tiles * 4 >= cus * 3 || nblk < 4) return 0;
+    double best = 1e30;
+    int splits = 1;
+    for (int sp = 1; sp <= nblk && sp <= 64; ++sp) {
+        if (nblk % sp || (nblk / sp) * 4 < 8) continue;
+        const double cost = (double)((tiles * sp + cus - 1) / cus) * ((double)(nblk / sp) * 4 + 6.0) + (sp > 1 ? 4.0 + 0.5 * sp : 0.0);
+        if (cost < best - 1e-9) {
+            best = cost;
+            splits = sp;
+        }
+    }
+    return splits > 1 ? (size_t)splits * (size_t)M * (size_t)N * sizeof(float) : 0;
+}
+const ShapePlan& plan_of_shape(int64_t M, int64_t N, int64_t K, bool persistent, bool tiles_ok) {
+    static thread_local ShapePlan table[64];
+    const int flags = (persistent ? 1 : 0) | (tiles_ok ? 2 : 0);
+    ShapePlan& e = table[(size_t)(M * 31 + N * 17 + K * 7 + flags) % 64];
+    if (e.M == M && e.N == N && e.K == K && e.flags == flags) return e;
+    const int cus = device_cus();
+    ShapePlan p;
+    p.M = M; p.N = N; p.K = K; p.flags = flags;
+    double best = 1e30;
+    if (persistent) best = p.persistent = persistent_cost(M, N, K, 1, cus);
+    for (int kind = TILE_256x128; kind <= TILE_64x32; ++kind) {
+        p.tile[kind] = tiles_ok ? tile_cost(kTileCosts[kind], M, N, K, 1, cus) : 1e30;
+        best = p.tile[kind] < best ? p.tile[kind] : best;
+    }
+    p.cut = cheapest_cut(M, N, K, persistent, tiles_ok, cus);
+    p.cut_bytes = p.cut.cost < best ? (size_t)p.cut.choice.splits * (size_t)M * (size_t)N * sizeof(float) : 0;
+    p.scratch_bytes = persistent ? scratch_of_few_tiles(M, N, K, cus) : 0;
+    if (p.cut_bytes > p.scratch_bytes) p.scratch_bytes = p.cut_bytes;
+    return e = p;
+}
+
 // bytes of scratch with which gemm_mxfp4_tn may cut this shape into K ranges (0: it would not)
 size_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-    if (!persistent_serves(M, N, K, nullptr, nullptr, nullptr)) return 0;
-    const int sp = choose_splits(M, N, K, device_cus());
-    return sp > 1 ? (size_t)sp * (size_t)M * (size_t)N * sizeof(float) : 0;
+    const bool persistent = persistent_serves(M, N, K, nullptr, nullptr, nullptr), tiles_ok = gemm_tile_serves(M, N, K, 0, 0, nullptr);
+    return persistent || tiles_ok ? plan_of_shape(M, N, K, persistent, tiles_ok).scratch_bytes : 0;
 }
 
 // The kernel that serves product p.  p.mask: the caller wants the masked inverse rotation applied to the result (mid dtype
 // c_dtype, stored in rot_out_dtype); `rotates` tells whether the chosen kernel does it.  Where it does not, the rotation is
 // a kernel of its own that reads and writes the result, which the comparison accounts for.
 ProductChoice choose_product(const TileProduct& p, int c_dtype, int rot_out_dtype, const void* workspace, size_t workspace_bytes) {
-    const int cus = device_cus();
     const int64_t M = p.M, N = p.N, K = p.K;
     const bool rotate = p.mask != nullptr;
-    const double separate = rotate ? kLaunch + (double)M * N * ((c_dtype == BF16 ? 2 : 4) + (rot_out_dtype == BF16 ? 2 : 4)) / kMemory : 0.0;
+    const bool persistent = persistent_serves(M, N, K, p.a_scales, p.b_scales, p.c), tiles_ok = gemm_tile_serves(M, N, K, p.a_tiled, p.b_tiled, p.c);
+    if (!persistent && !tiles_ok) return {ProductChoice::GENERIC, 0, 1, false};
+    const ShapePlan& plan = plan_of_shape(M, N, K, persistent, tiles_ok);
+    // a cut into K ranges rounds differently: whether to make it is decided on the product alone, so that a product and the
+    // same product with the rotation agree
+    if (plan.cut_bytes && workspace && plan.cut_bytes <= workspace_bytes && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0) {
+        ProductChoice c = plan.cut.choice;
+        c.rotates = rotate;
+        return c;
+    }
+    const double separate = rotate ? separate_rotate_cost(M, N, c_dtype == BF16 ? 2 : 4, rot_out_dtype == BF16 ? 2 : 4) : 0.0;
     ProductChoice best{ProductChoice::GENERIC, 0, 1, false};
-    double best_cost = 1e30, best_plain = 1e30;   // with the rotation, and of the product alone
+    double best_cost = 1e30;
     const auto consider = [&](ProductChoice c, double cost) {
-        best_plain = cost < best_plain ? cost : best_plain;
-        if (rotate && !c.rotates) cost += separate;
         if (cost < best_cost) {
             best_cost = cost;
             best = c;
         }
     };
-    const bool persistent = persistent_serves(M, N, K, p.a_scales, p.b_scales, p.c);
+    const bool bf16 = c_dtype == BF16;
+    const int cus = device_cus();
     if (persistent) {
-        const bool bf16 = c_dtype == BF16 && rot_out_dtype == BF16;
-        consider({ProductChoice::PERSISTENT, 0, 1, rotate && bf16 && p.hd == 32}, persistent_cost(M, N, K, 1, cus));
+        if (rotate && bf16 && rot_out_dtype == BF16 && p.hd == 32) consider({ProductChoice::PERSISTENT, 0, 1, true}, plan.persistent + kPersistentRotate);
+        consider({ProductChoice::PERSISTENT, 0, 1, false}, plan.persistent + separate);
     }
-    if (gemm_tile_serves(M, N, K, p.a_tiled, p.b_tiled, p.c))
-        for (int kind = TILE_256x128; kind <= TILE_64x32; ++kind)
-            consider({ProductChoice::TILE, kind, 1, rotate && c_dtype == BF16 && kTileCosts[kind].bn >= p.hd},
-                     tile_cost(kTileCosts[kind], M, N, K, cus));
-    // a cut into K ranges rounds differently: whether to make it is decided on the product alone, so that a product and the
-    // same product with the rotation agree
-    if (persistent && workspace) {
-        const int sp = choose_splits(M, N, K, cus);
-        if (sp > 1 && (size_t)sp * M * N * sizeof(float) <= workspace_bytes && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
-            persistent_cost(M, N, K, sp, cus) < best_plain)
-            return {ProductChoice::PERSISTENT, 0, sp, rotate && p.hd == 32};
+    for (int kind = TILE_256x128; tiles_ok && kind <= TILE_64x32; ++kind) {
+        const KernelCost& k = kTileCosts[kind];
+        if (rotate && bf16 && k.bn >= p.hd) consider({ProductChoice::TILE, kind, 1, true}, plan.tile[kind] + tile_rotate_cost(k, M, N, p.hd, cus));
+        consider({ProductChoice::TILE, kind, 1, false}, plan.tile[kind] + separate);
     }
     return best;
 }
@@ -1032,31 +1100,40 @@ ProductChoice choose_product(const TileProduct& p, int c_dtype, int rot_out_dtyp
 hipError_t run_product(const ProductChoice& c, const TileProduct& p, int c_dtype, int rot_out_dtype, void* workspace, hipStream_t stream) {
     const int64_t M = p.M, N = p.N, K = p.K;
     const int cus = device_cus();
-    if (c.path == ProductChoice::TILE) {
-        TileProduct q = p;
-        if (!c.rotates) q.mask = nullptr;
-        q.out_f32 = c_dtype == BF16 && rot_out_dtype == F32;
-        return gemm_tile(c.kind, q, nullptr, c_dtype, stream);
-    }
     if (c.path == ProductChoice::GENERIC) {
         if (p.a_tiled || p.b_tiled) return hipErrorInvalidValue;
         return launch_gemm<128, 128, 64, 64>(p.a_codes, p.a_scales, p.b_codes, p.b_scales, M, N, K, p.alpha, p.c, c_dtype, stream);
     }
     if (c.splits > 1) {
         // partial sums per K range in fp32 (plain accumulator layout), then one ordered reduction
-        hipError_t e = launch_big4<float>(p.a_codes, p.a_scales, p.b_codes, p.b_scales, M, N, K, 1.0f, workspace, p.a_tiled, p.b_tiled, c.splits,
-                                          cus, stream);
+        hipError_t e;
+        if (c.path == ProductChoice::TILE) {
+            TileProduct q = p;
+            q.c = workspace;
+            q.splits = c.splits;
+            q.mask = nullptr;
+            e = gemm_tile(c.kind, q, nullptr, F32, stream);
+        } else {
+            e = launch_big4<float>(p.a_codes, p.a_scales, p.b_codes, p.b_scales, M, N, K, 1.0f, workspace, p.a_tiled, p.b_tiled, c.splits, cus, stream);
+        }
         if (e != hipSuccess) return e;
         const int64_t mn = M * N;
         const float* part = static_cast<const float*>(workspace);
         if (c.rotates)
-            return splitk_reduce_rotated(part, c.splits, mn, p.alpha, c_dtype, p.mask, p.signs.w[0], p.rot_c, p.c, rot_out_dtype, stream);
+            return splitk_reduce_rotated(part, c.splits, mn, p.alpha, c_dtype, p.mask, p.hd, p.signs, p.rot_c, p.c, rot_out_dtype, stream);
         dim3 grid((unsigned)((mn / 4 + 255) / 256)), block(256);
         if (c_dtype == BF16)
             splitk_reduce_kernel<uint16_t><<<grid, block, 0, stream>>>(part, c.splits, mn, p.alpha, static_cast<uint16_t*>(p.c));
         else
             splitk_reduce_kernel<float><<<grid, block, 0, stream>>>(part, c.splits, mn, p.alpha, static_cast<float*>(p.c));
         return hipGetLastError();
+    }
+    if (c.path == ProductChoice::TILE) {
+        TileProduct q = p;
+        q.splits = 1;
+        if (!c.rotates) q.mask = nullptr;
+        q.out_f32 = c_dtype == BF16 && rot_out_dtype == F32;
+        return gemm_tile(c.kind, q, nullptr, c_dtype, stream);
     }
     if (c.rotates)
         return launch_big4<uint16_t, true>(p.a_codes, p.a_scales, p.b_codes, p.b_scales, M, N, K, p.alpha, p.c, p.a_tiled, p.b_tiled, 1, cus, stream,
@@ -1070,7 +1147,7 @@ TileProduct make_product(const uint8_t* a_codes, const uint8_t* a_scales, const 
                          int64_t K, float alpha, void* c, int a_layout, int b_layout) {
     TileProduct p{};
     p.a_codes = a_codes; p.a_scales = a_scales; p.b_codes = b_codes; p.b_scales = b_scales; p.c = c;
-    p.M = (int)M; p.N = (int)N; p.K = (int)K; p.alpha = alpha; p.hd = 32;
+    p.M = (int)M; p.N = (int)N; p.K = (int)K; p.alpha = alpha; p.hd = 32; p.splits = 1;
     p.a_tiled = a_layout == LAYOUT_TILED; p.b_tiled = b_layout == LAYOUT_TILED;
     return p;
 }

@@ -145,10 +145,14 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
     const int M = g.M, N = g.N, K = g.K;
     const int tiles_m = (M + S::BM - 1) / S::BM, tiles_n = (N + S::BN - 1) / S::BN;
     const int code_pitch = K / 2, groups = K / 32;
-    const int nk = (K + kBK - 1) / kBK;
-    const int half_step = (K % kBK) ? nk - 1 : -1;  // the K step that covers only 64 indices (K % 128 == 64), or none
+    // a work item is (tile, K range): range r covers steps [r * all / splits, (r + 1) * all / splits) and, with splits > 1 (fp32
+    // instantiation only), stores its partial sums, unscaled, into slab r of c = [splits][M][N]
+    const int tiles = tiles_m * tiles_n, range = t / tiles;
+    const int nk_all = (K + kBK - 1) / kBK;
+    const int k_first = range * nk_all / g.splits, nk = (range + 1) * nk_all / g.splits - k_first;
+    const int half_step = (K % kBK) && range == g.splits - 1 ? nk - 1 : -1;  // the K step that covers only 64 indices (K % 128 == 64), or none
     int tm, tn;
-    tile_of_block<(S::BM >= 256 ? 4 : 8)>(t, tiles_m, tiles_n, tm, tn);
+    tile_of_block<(S::BM >= 256 ? 4 : 8)>(t - range * tiles, tiles_m, tiles_n, tm, tn);
     const int m0 = tm * S::BM, n0 = tn * S::BN;
 
     const int swz = (lrow >> 2) & 3;
@@ -171,8 +175,10 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
         const auto row_off = [&](int r, int tiled) {
             return tiled ? (uint32_t)((r >> 4) * row16) + (uint32_t)((r & 15) * 64 + pcv * 16) : (uint32_t)(r * code_pitch + pcv * 16);
         };
-        plan.a = g.a_codes + (int64_t)m0 * code_pitch;   // m0, n0 are multiples of 16: the same expression in both layouts
-        plan.b = g.b_codes + (int64_t)n0 * code_pitch;
+        plan.kstep_a = g.a_tiled ? 1024 : kRowBytes;
+        plan.kstep_b = g.b_tiled ? 1024 : kRowBytes;
+        plan.a = g.a_codes + (int64_t)m0 * code_pitch + (int64_t)k_first * plan.kstep_a;   // m0, n0 are multiples of 16: the same
+        plan.b = g.b_codes + (int64_t)n0 * code_pitch + (int64_t)k_first * plan.kstep_b;   //   expression in both layouts
 #pragma unroll
         for (int j = 0; j < S::kALoads; ++j) {
             const int r = (wave * S::kALoads + j) * 16 + prow;
@@ -184,8 +190,6 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
             plan.voff_b[j] = row_off(r < last_b ? r : last_b, g.b_tiled);
         }
         plan.half_back = (uint32_t)(pcv & 2) * 16u;
-        plan.kstep_a = g.a_tiled ? 1024 : kRowBytes;
-        plan.kstep_b = g.b_tiled ? 1024 : kRowBytes;
         plan.lds_a = (uint32_t)__builtin_amdgcn_readfirstlane((int)(smem_base + wave * S::kALoads * 1024));
         plan.lds_b = (uint32_t)__builtin_amdgcn_readfirstlane((int)(smem_base + S::kBOff + wave * S::kBLoads * 1024));
 #pragma unroll
@@ -199,7 +203,7 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
             const int rb = (p / (32 * S::TN)) * S::WN + (p % S::TN) * 32 + (p / S::TN) % 32;
             const int la = M - 1 - m0, lb = N - 1 - n0;
             const int r = is_a ? (ra < la ? ra : la) : (rb < lb ? rb : lb);
-            plan.s[u] = is_a ? g.a_scales + (int64_t)m0 * groups : g.b_scales + (int64_t)n0 * groups;
+            plan.s[u] = (is_a ? g.a_scales + (int64_t)m0 * groups : g.b_scales + (int64_t)n0 * groups) + k_first * 4;
             plan.voff_s[u] = (uint32_t)(r * groups);
             plan.lds_s[u] = (uint32_t)__builtin_amdgcn_readfirstlane((int)(smem_base + S::kSAOff + unit * 256));
         }
@@ -278,7 +282,7 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
     // every request has landed and every wave has read its last fragments: the ring becomes the staging area
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
     __syncthreads();
-    const float alpha = g.alpha;
+    const float alpha = g.splits > 1 ? 1.0f : g.alpha;
     if (SWAP && !S::kMaskEarly && g.mask) issue_mask(S::kMaskOff);
     if constexpr (SWAP) {
 #pragma unroll
@@ -342,7 +346,7 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
             }
         }
     } else {
-        float* c = reinterpret_cast<float*>(g.c);
+        float* c = reinterpret_cast<float*>(g.c) + (int64_t)range * M * N;
 #pragma unroll
         for (int i = 0; i < S::TM; ++i)
 #pragma unroll
@@ -370,7 +374,7 @@ __global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu((S:
         TileProduct p;
 #define QM_PICK(f) p.f = first ? g.f : h.f
         QM_PICK(a_codes); QM_PICK(a_scales); QM_PICK(b_codes); QM_PICK(b_scales); QM_PICK(c); QM_PICK(mask); QM_PICK(M); QM_PICK(N);
-        QM_PICK(K); QM_PICK(a_tiled); QM_PICK(b_tiled); QM_PICK(alpha); QM_PICK(hd); QM_PICK(signs.w[0]); QM_PICK(signs.w[1]);
+        QM_PICK(K); QM_PICK(splits); QM_PICK(a_tiled); QM_PICK(b_tiled); QM_PICK(alpha); QM_PICK(hd); QM_PICK(signs.w[0]); QM_PICK(signs.w[1]);
         QM_PICK(signs.w[2]); QM_PICK(signs.w[3]); QM_PICK(rot_c); QM_PICK(out_f32);
 #undef QM_PICK
         tile_run<S, OutT>(p, first ? t : t - tiles_g, smem, smem_base);
@@ -378,7 +382,7 @@ __global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu((S:
 }
 
 template <class S>
-int tiles_of(const TileProduct& p) { return p.M == 0 ? 0 : ((p.M + S::BM - 1) / S::BM) * ((p.N + S::BN - 1) / S::BN); }
+int tiles_of(const TileProduct& p) { return p.M == 0 ? 0 : ((p.M + S::BM - 1) / S::BM) * ((p.N + S::BN - 1) / S::BN) * p.splits; }
 
 template <class S, typename OutT>
 hipError_t launch_tiles(const TileProduct& g, const TileProduct& h, hipStream_t stream) {

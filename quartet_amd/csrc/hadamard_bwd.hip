@@ -99,7 +99,7 @@ struct HadamardBwdJob {
 // The same rotation on a product that was cut into K ranges: the input element is alpha * (p[0][i] + p[1][i] + ...)
 // summed in slab order (what the ordered reduction of the partial sums stores), rounded to bf16 when the product's own
 // dtype is bf16 (MID_BF16).  One pass in place of the reduction followed by the rotation, with the same arithmetic.
-template <bool MID_BF16, typename TOut>
+template <bool MID_BF16, typename TOut, int HD>
 struct SplitKRotateJob {
     static constexpr int kLds = 0;
     static constexpr int kWaves = 1;
@@ -136,7 +136,7 @@ struct SplitKRotateJob {
 #pragma unroll
             for (int i = 0; i < 8; ++i) v[i] = u2f((uint32_t)f32_to_bf16(v[i]) << 16);
         }
-        rotate_octet<TOut, 32, MID_BF16 && sizeof(TOut) == 4>(v, keep, octet, c, sb, out);
+        rotate_octet<TOut, HD, MID_BF16 && sizeof(TOut) == 4>(v, keep, octet, c, sb, out);
     }
 };
 
@@ -212,15 +212,20 @@ hipError_t masked_hadamard_bwd_hd32_pair(const void* ga, int64_t na, int scale_d
     return hipGetLastError();
 }
 
-// c = masked inverse rotation (blocks of 32 along the rows) of the reduced product alpha * sum_s partial[s]; see SplitKRotateJob
+// c = masked inverse rotation (blocks of hd along the rows) of the reduced product alpha * sum_s partial[s]; see SplitKRotateJob
 hipError_t splitk_reduce_rotated(const float* partial, int splits, int64_t mn, float alpha, int mid_dtype, const uint8_t* maskbits,
-                                 uint32_t sign_word, float c, void* out, int out_dtype, hipStream_t stream) {
+                                 int hd, const SignBits& signs, float c, void* out, int out_dtype, hipStream_t stream) {
     if (mn == 0) return hipSuccess;
-    if (mn % 32 || !maskbits || splits < 1 || (mid_dtype == F32 && out_dtype != F32)) return hipErrorInvalidValue;
-    const SignBits sb{{sign_word, 0, 0, 0}};
-    if (mid_dtype == BF16 && out_dtype == BF16) launch_job(SplitKRotateJob<true, uint16_t>(partial, splits, mn, alpha, c, sb, maskbits, out), stream);
-    else if (mid_dtype == BF16) launch_job(SplitKRotateJob<true, float>(partial, splits, mn, alpha, c, sb, maskbits, out), stream);
-    else launch_job(SplitKRotateJob<false, float>(partial, splits, mn, alpha, c, sb, maskbits, out), stream);
+    if (mn % hd || !maskbits || splits < 1 || (mid_dtype == F32 && out_dtype != F32)) return hipErrorInvalidValue;
+    const auto go = [&](auto h) {
+        constexpr int HD = decltype(h)::value;
+        if (mid_dtype == BF16 && out_dtype == BF16) launch_job(SplitKRotateJob<true, uint16_t, HD>(partial, splits, mn, alpha, c, signs, maskbits, out), stream);
+        else if (mid_dtype == BF16) launch_job(SplitKRotateJob<true, float, HD>(partial, splits, mn, alpha, c, signs, maskbits, out), stream);
+        else launch_job(SplitKRotateJob<false, float, HD>(partial, splits, mn, alpha, c, signs, maskbits, out), stream);
+    };
+    if (hd == 32) go(std::integral_constant<int, 32>{});
+    else if (hd == 64) go(std::integral_constant<int, 64>{});
+    else go(std::integral_constant<int, 128>{});
     return hipGetLastError();
 }
 

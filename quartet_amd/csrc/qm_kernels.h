@@ -130,7 +130,7 @@ hipError_t gemm_mxfp4_tn(const uint8_t* a_codes, const uint8_t* a_scales, const 
                          int a_layout, int b_layout, void* workspace, size_t workspace_bytes, hipStream_t stream);
 // the reduction of a product cut into K ranges with that rotation applied to the reduced values (hadamard_bwd.hip)
 hipError_t splitk_reduce_rotated(const float* partial, int splits, int64_t mn, float alpha, int mid_dtype, const uint8_t* maskbits,
-                                 uint32_t sign_word, float c, void* out, int out_dtype, hipStream_t stream);
+                                 int hd, const SignBits& signs, float c, void* out, int out_dtype, hipStream_t stream);
 size_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
 // The product on small and middle-sized tiles (gemm_tile.hip).  Any M; N % 8 == 0; K % 128 == 0, or K % 128 == 64 with
@@ -146,6 +146,7 @@ struct TileProduct {
     void* c;
     const uint8_t* mask;
     int M, N, K;
+    int splits;            // K ranges; more than one: c receives [splits][M][N] fp32 partial sums, unscaled (fp32 c_dtype, no mask)
     int a_tiled, b_tiled;
     float alpha;
     int hd;
@@ -164,7 +165,7 @@ hipError_t gemm_tile(int kind, const TileProduct& g, const TileProduct* second, 
 struct ProductChoice {
     enum Path : int { GENERIC = 0, PERSISTENT = 1, TILE = 2 } path;
     int kind;      // TileKind
-    int splits;    // K ranges of the persistent kernel
+    int splits;    // K ranges (their fp32 partial sums in the workspace, then one ordered reduction)
     bool rotates;
 };
 TileProduct make_product(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes, const uint8_t* b_scales, int64_t M, int64_t N,

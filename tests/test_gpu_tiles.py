@@ -38,7 +38,26 @@ def test_product_on_ragged_extents(oracle, M, N, K):
     assert torch.equal(c16, c32.to(torch.bfloat16))
 
 
-@pytest.mark.parametrize("T,I,O,hd", [(32, 32, 32, 32), (96, 160, 96, 32), (288, 192, 320, 32), (544, 1728, 352, 32), (1056, 640, 1088, 32),
+@pytest.mark.parametrize("M,N,K", [(1, 8, 5376), (33, 72, 4736), (257, 520, 16512), (640, 264, 8256), (1536, 512, 16384)])
+def test_product_cut_into_k_ranges(oracle, M, N, K):
+    """Few tiles and a long contraction: ranges of unequal length, a last range that ends in half a step.  The same sums in
+    another order, each of at most K + ranges fp32 additions (relative error below 1e-5 of the norm); bf16 is the rounding of
+    the fp32 result."""
+    print(f"case ranges {M}x{N}x{K}", flush=True)
+    from quartet_amd import kernels as Kn
+    g = torch.Generator().manual_seed(M + N + K)
+    mk = lambda r: (torch.randint(0, 256, (r, K // 2), generator=g, dtype=torch.uint8),
+                    torch.randint(120, 131, (r, K // 32), generator=g, dtype=torch.uint8))
+    (ac, as_), (bc, bs) = mk(M), mk(N)
+    dev = [t.to("cuda:0") for t in (ac, as_, bc, bs)]
+    c32 = Kn.gemm_mxfp4_tn(*dev, 1.5, torch.float32)
+    c16 = Kn.gemm_mxfp4_tn(*dev, 1.5, torch.bfloat16)
+    want = 1.5 * oracle.gemm_tn(ac.numpy(), as_.numpy(), bc.numpy(), bs.numpy())
+    assert rel(c32.cpu().numpy(), want) < 1e-5
+    assert torch.equal(c16, c32.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("T,I,O,hd", [(32, 32, 32, 32), (4128, 96, 160, 32), (4160, 192, 128, 64), (4224, 128, 256, 128), (96, 160, 96, 32), (288, 192, 320, 32), (544, 1728, 352, 32), (1056, 640, 1088, 32),
                                       (64, 64, 64, 64), (192, 320, 128, 64), (128, 128, 128, 128), (384, 256, 640, 128), (1280, 384, 896, 128)])
 def test_layer_on_padded_operands(oracle, T, I, O, hd):
     """Forward and backward of the production layer against the oracle pipeline (same seeds and signs).  bf16 results: each
