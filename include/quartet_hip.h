@@ -304,6 +304,20 @@ int qm_linear_backward_seeded(const void* e, int e_dtype, int64_t T, int64_t I, 
                               const float* g_matrix, const uint64_t* seed_base, void* stream);
 
 /*
+ * The backward pass of a layer under the error-only scheme (QEW_QEtXFn, backward.py:21-45) behind the same packed forward:
+ * gx = M_x(Q(e) Wq) and gw = M_w(Q(e^T) xq) with Wq, xq the packed quest-coded operands qm_linear_forward left in packed_w
+ * and packed_x with QM_LAYOUT_PADDED, M the masked inverse rotations of their quantizers, products rounded to bf16.  g_mode
+ * QM_ABSMAX_RTN or QM_ABSMAX_SR with seeds[0] for e and seeds[1] for e^T.  gx bf16, gw bf16 or fp32 (the bf16 result
+ * widened).  T, I, O multiples of 32 and of the Hadamard blocks along them.  Same values as multiplying the de-quantized
+ * operands in bf16 with fp32 accumulation, whatever the operands' scales.
+ */
+size_t qm_linear_backward_error_workspace_bytes(int64_t T, int64_t I, int64_t O);
+int qm_linear_backward_error(const void* e, int e_dtype, int64_t T, int64_t I, int64_t O, const void* packed_x, const void* packed_w,
+                             int hd_x, const uint32_t* signs_x, int hd_w, const uint32_t* signs_w, int hd_g,
+                             const uint32_t* signs_g, int g_mode, const uint64_t* seeds, int x_scale_dtype, int w_scale_dtype,
+                             void* workspace, size_t workspace_bytes, void* gx, void* gw, int gw_dtype, void* stream);
+
+/*
  * Producers fused into the activation quantizer.  The tensor the model would hand to a quantized linear is computed
  * group by group inside the quantizer kernel and never written; the result is a packed operand buffer (layout as
  * above) that qm_linear_forward consumes with QM_X_IS_PACKED and qm_linear_backward reads as packed_x.  Hadamard block

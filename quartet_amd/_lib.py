@@ -38,6 +38,8 @@ EXPORTS = (
     "qm_linear_forward",
     "qm_linear_backward",
     "qm_linear_backward_seeded",
+    "qm_linear_backward_error_workspace_bytes",
+    "qm_linear_backward_error",
     "qm_rmsnorm_quantize_mxfp4",
     "qm_swiglu_quantize_mxfp4",
     "qm_rmsnorm_backward_workspace_bytes",
@@ -126,6 +128,10 @@ def lib():
     L.qm_linear_backward.restype = i32
     L.qm_linear_backward.argtypes = [vp, i32, i64, i64, i64, vp, vp, i32, vp, i32, vp, i32, vp, i32, vp, i32, i32, i32, i32, i32,
                                      vp, sz, vp, vp, i32, i32, i32, vp, vp]
+    L.qm_linear_backward_error_workspace_bytes.restype = sz
+    L.qm_linear_backward_error_workspace_bytes.argtypes = [i64, i64, i64]
+    L.qm_linear_backward_error.restype = i32
+    L.qm_linear_backward_error.argtypes = [vp, i32, i64, i64, i64, vp, vp, i32, vp, i32, vp, i32, vp, i32, vp, i32, i32, vp, sz, vp, vp, i32, vp]
     L.qm_linear_backward_seeded.restype = i32
     L.qm_linear_backward_seeded.argtypes = L.qm_linear_backward.argtypes[:-1] + [vp, vp]
     _lib = L
@@ -146,11 +152,11 @@ def host():
 
         import torch  # noqa: F401  (its libraries must be loaded before the extension's)
 
-        from .linear import _gradient_draws
+        from .linear import _error_draws, _gradient_draws
         spec = importlib.util.spec_from_file_location("_quartet_host", HOST_PATH)
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)
-        module.bind(QuartetHipError, _gradient_draws)
+        module.bind(QuartetHipError, _gradient_draws, _error_draws)
         _host = module
     return _host
 

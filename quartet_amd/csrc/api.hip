@@ -384,6 +384,26 @@ WorkLayout work_layout(int64_t T, int64_t I, int64_t O, int mid_dtype) {
     l.total = o;
     return l;
 }
+// the error-only scheme: Q(e), Q(e^T), the packed operands as eight-bit ones, a product before its rotation (one at a time)
+struct ErrorLayout {
+    size_t ec, es, etc, ets, wv, ws, wl, xv, xs, xl, plain, gemm_ws, gemm_ws_bytes, total;
+};
+ErrorLayout error_layout(int64_t T, int64_t I, int64_t O) {
+    ErrorLayout l;
+    size_t o = 0;
+    const auto take = [&](size_t& at, size_t n) { at = o; o += up256(n); };
+    const int64_t Tp = qm::padded_cols(T), Op = qm::padded_cols(O);
+    take(l.ec, code_bytes(T, O)); take(l.es, scale_bytes(T, O));
+    take(l.etc, code_bytes(O, T)); take(l.ets, scale_bytes(O, T));
+    take(l.wv, (size_t)I * Op); take(l.ws, (size_t)I * Op / 32); take(l.wl, (size_t)((I + 127) / 128) * (Op / 128));
+    take(l.xv, (size_t)I * Tp); take(l.xs, (size_t)I * Tp / 32); take(l.xl, (size_t)((I + 127) / 128) * (Tp / 128));
+    take(l.plain, (size_t)(T > O ? T : O) * I * 2);
+    const size_t need_x = qm::gemm_e5m2_workspace_bytes(T, I, Op), need_w = qm::gemm_e5m2_workspace_bytes(O, I, Tp);
+    l.gemm_ws_bytes = need_x > need_w ? need_x : need_w;
+    take(l.gemm_ws, l.gemm_ws_bytes);
+    l.total = o;
+    return l;
+}
 bool tiled_layout(int codes_layout) { return codes_layout != QM_LAYOUT_ROWMAJOR; }
 // the layout the kernels of a single operation are told
 int kernel_layout(int codes_layout) { return tiled_layout(codes_layout) ? QM_LAYOUT_TILED : QM_LAYOUT_ROWMAJOR; }
@@ -464,6 +484,74 @@ int qm_linear_forward(const void* x, int x_dtype, const void* w, int w_dtype, in
     if (!valid_dtype(y_dtype)) return fail(QM_ERR_INVALID, "qm_linear_forward: y_dtype %d", y_dtype);
     return from_hip(qm::gemm_mxfp4_tn(px + lx.c, px + lx.s, pw + lw.c, pw + lw.s, T, O, K, 1.0f, y, y_dtype, kernel_layout(codes_layout), kernel_layout(codes_layout), nullptr, 0, hs),
                     "qm_linear_forward");
+}
+
+size_t qm_linear_backward_error_workspace_bytes(int64_t T, int64_t I, int64_t O) {
+    if (T < 0 || I < 0 || O < 0 || I % 32 || O % 32 || T % 32) return 0;
+    return error_layout(T, I, O).total;
+}
+
+int qm_linear_backward_error(const void* e, int e_dtype, int64_t T, int64_t I, int64_t O, const void* packed_x, const void* packed_w,
+                             int hd_x, const uint32_t* signs_x, int hd_w, const uint32_t* signs_w, int hd_g, const uint32_t* signs_g,
+                             int g_mode, const uint64_t* seeds, int x_scale_dtype, int w_scale_dtype, void* workspace,
+                             size_t workspace_bytes, void* gx, void* gw, int gw_dtype, void* stream) {
+    if (T < 0 || I < 0 || O < 0) return fail(QM_ERR_INVALID, "qm_linear_backward_error: negative extent");
+    if (T == 0 || O == 0 || I == 0) return 0;
+    if (I % 32 || O % 32 || T % 32 || I >= (1 << 23) || O >= (1 << 23) || T >= (1 << 23))
+        return fail(QM_ERR_INVALID, "qm_linear_backward_error: tokens, in_features and out_features must be multiples of 32 below 2^23 (T=%lld I=%lld O=%lld)",
+                    (long long)T, (long long)I, (long long)O);
+    if (g_mode != QM_ABSMAX_RTN && g_mode != QM_ABSMAX_SR) return fail(QM_ERR_INVALID, "qm_linear_backward_error: g_mode %d", g_mode);
+    if (!valid_hd(hd_x) || !valid_hd(hd_w) || !valid_hd(hd_g) || I % hd_x || I % hd_w || T % hd_g || O % hd_g)
+        return fail(QM_ERR_INVALID, "qm_linear_backward_error: extents must be multiples of the Hadamard blocks");
+    if (!valid_dtype(e_dtype) || !valid_dtype(x_scale_dtype) || !valid_dtype(w_scale_dtype) || !valid_dtype(gw_dtype))
+        return fail(QM_ERR_INVALID, "qm_linear_backward_error: dtypes must be QM_BF16/QM_F32");
+    if (!e || !seeds || !packed_x || !packed_w || !gx || !gw || !aligned(e, 16) || !aligned(packed_x, 256) || !aligned(packed_w, 256) ||
+        !aligned(gx, 16) || !aligned(gw, 16))
+        return fail(QM_ERR_INVALID, "qm_linear_backward_error: null or misaligned tensors, seeds or packed operand buffers");
+    const ErrorLayout wl = error_layout(T, I, O);
+    if (!workspace || workspace_bytes < wl.total || !aligned(workspace, 256))
+        return fail(QM_ERR_INVALID, "qm_linear_backward_error: workspace needs %zu bytes, 256-byte aligned", wl.total);
+    const PackedLayout lx = packed_layout(T, I), lw = packed_layout(O, I);
+    const uint8_t* px = static_cast<const uint8_t*>(packed_x);
+    const uint8_t* pw = static_cast<const uint8_t*>(packed_w);
+    uint8_t* k = static_cast<uint8_t*>(workspace);
+    hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
+    int rc = from_hip(qm::quantize_error(e, e_dtype, T, O, hd_g, make_signs(signs_g, hd_g), g_mode, seeds[0], seeds[1], k + wl.ec, k + wl.es, k + wl.etc,
+                                         k + wl.ets, nullptr, hs), "qm_linear_backward_error");
+    if (rc) return rc;
+    const qm::E5m2Args ax{px + lx.c, px + lx.s, T, I, k + wl.xv, k + wl.xs, k + wl.xl};
+    const qm::E5m2Args aw{pw + lw.c, pw + lw.s, O, I, k + wl.wv, k + wl.ws, k + wl.wl};
+    rc = from_hip(qm::expand_e5m2_pair(ax, aw, hs), "qm_linear_backward_error");
+    if (rc) return rc;
+    // value = code * 2^k * fl32(4/3) on the error signal, code * 2^k on the saved operand
+    const float alpha = (float)(1.0 / 0.75);
+    void* gws = wl.gemm_ws_bytes ? k + wl.gemm_ws : nullptr;
+    // one gradient: the product, then the masked inverse rotation of the forward quantizer, in the product's kernel where that is cheaper
+    const auto gradient = [&](size_t ac, size_t as, const qm::E5m2Args& b, int64_t M, void* out, int out_dtype, int hd, const uint32_t* signs,
+                              int scale_dtype, const uint8_t* mask, size_t plain) {
+        qm::TileProduct p = qm::make_product(k + ac, k + as, b.values, b.scales, M, I, qm::padded_cols(b.R), alpha, out, QM_LAYOUT_TILED, QM_LAYOUT_TILED);
+        p.b_e5m2 = 1;
+        p.mask = mask;
+        p.hd = hd;
+        p.signs = make_signs(signs, hd);
+        p.rot_c = qm::hadamard_scale(hd, scale_dtype);
+        const qm::ProductChoice c = qm::choose_product(p, QM_BF16, out_dtype, gws, wl.gemm_ws_bytes);
+        if (c.rotates) return qm::run_product(c, p, QM_BF16, out_dtype, gws, hs);
+        p.mask = nullptr;
+        p.c = k + plain;
+        const hipError_t e1 = qm::run_product(c, p, QM_BF16, QM_BF16, gws, hs);
+        return e1 != hipSuccess ? e1 : qm::masked_hadamard_bwd(p.c, QM_BF16, M, I, hd, scale_dtype, p.signs, mask, out, out_dtype, out_dtype != QM_BF16, hs);
+    };
+    rc = from_hip(gradient(wl.ec, wl.es, aw, T, gx, QM_BF16, hd_x, signs_x, x_scale_dtype, px + lx.m, wl.plain), "qm_linear_backward_error");
+    if (rc) return rc;
+    rc = from_hip(gradient(wl.etc, wl.ets, ax, O, gw, gw_dtype, hd_w, signs_w, w_scale_dtype, pw + lw.m, wl.plain), "qm_linear_backward_error");
+    if (rc) return rc;
+    const auto exact = [&](size_t ac, size_t as, const qm::E5m2Args& b, int64_t M, void* out, int out_dtype, int hd, const uint32_t* signs, int scale_dtype,
+                           const uint8_t* mask) {
+        return qm::E5m2Exact{k + ac, k + as, b, M, alpha, mask, hd, make_signs(signs, hd), qm::hadamard_scale(hd, scale_dtype), out, out_dtype};
+    };
+    return from_hip(qm::e5m2_exact_pair(exact(wl.ec, wl.es, aw, T, gx, QM_BF16, hd_x, signs_x, x_scale_dtype, px + lx.m),
+                                        exact(wl.etc, wl.ets, ax, O, gw, gw_dtype, hd_w, signs_w, w_scale_dtype, pw + lw.m), hs), "qm_linear_backward_error");
 }
 
 int qm_linear_backward(const void* e, int e_dtype, int64_t T, int64_t I, int64_t O, const void* packed_x, const void* packed_w,

@@ -15,6 +15,10 @@
 // contractions, the tile boundary, which the neighbour workgroup on the same CU covers; the smaller tiles are latency-bound
 // and exist to put more workgroups on the chip.  Accumulation order over K is the same in every shape (and in gemm.hip's
 // kernels): results do not depend on the choice.
+//
+// The same kernel multiplies FP4 with an eight-bit (E5M2) B, which is how the error-only scheme contracts over the rows of a
+// packed operand (expand.hip): twice the bytes and twice the matrix cycles of B.  4096^3: 60 us, 8 waves of 128 x 64 on 256 x
+// 256 with the matrix pipe 60 % busy at the clock its power allows, where the FP4 x bf16 kernel (gemm_fp4_bf16.hip) takes 113 us.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -27,16 +31,19 @@ namespace qm {
 
 namespace {
 
-template <int BM_, int BN_, int WM_, int WN_, int STAGES_, int OCC_>
+// E5M2_B: B is eight bits wide (expand.hip), two 1 KiB blocks of 64 contraction indices per 16 columns and K step
+template <int BM_, int BN_, int WM_, int WN_, int STAGES_, int OCC_, bool E5M2_B = false>
 struct TileShape {
+    static constexpr bool kWideB = E5M2_B;
+    static constexpr int kBBlocks = E5M2_B ? 2 : 1;
     static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, STAGES = STAGES_, OCC = OCC_;   // OCC: workgroups per CU
     static constexpr int kWavesN = BN / WN, kWaves = (BM / WM) * kWavesN, kThreads = kWaves * 64;
     static constexpr int TM = WM / 32, TN = WN / 32;
-    static constexpr int kALoads = BM / 16 / kWaves, kBLoads = BN / 16 / kWaves;   // 1 KiB wave-loads per wave and K step
+    static constexpr int kALoads = BM / 16 / kWaves, kBLoads = BN / 16 * kBBlocks / kWaves;   // 1 KiB wave-loads per wave and K step
     static constexpr int kAUnits = (BM + 63) / 64, kUnits = kAUnits + (BN + 63) / 64;   // 64 scale dwords each
     static constexpr int kSLoads = (kUnits + kWaves - 1) / kWaves;
     static constexpr int kLoads = kALoads + kBLoads + kSLoads;   // requests per wave and K step
-    static constexpr int kBOff = BM * kRowBytes, kSAOff = (BM + BN) * kRowBytes, kSBOff = kSAOff + kAUnits * 256;
+    static constexpr int kBOff = BM * kRowBytes, kSAOff = (BM + BN * kBBlocks) * kRowBytes, kSBOff = kSAOff + kAUnits * 256;
     static constexpr int kStageBytes = kSAOff + kUnits * 256;
     static constexpr int kRingBytes = STAGES * kStageBytes;
     static constexpr int kMUnits = BM * BN / 2048, kMLoads = (kMUnits + kWaves - 1) / kWaves;   // mask words of the tile, 64 at a time
@@ -44,11 +51,11 @@ struct TileShape {
     static constexpr int kPitch = BN * 2 + 16;                   // bytes per staged row of the bf16 tile
     static constexpr int kChunks = BN / 8;                       // 16-byte pieces per row
     static constexpr int kRowsPerPass = kThreads / kChunks, kPasses = BM / kRowsPerPass;
-    static_assert(kALoads * 16 * kWaves == BM && kBLoads * 16 * kWaves == BN, "whole wave-loads per wave");
+    static_assert(kALoads * 16 * kWaves == BM && kBLoads * 16 * kWaves == BN * kBBlocks, "whole wave-loads per wave");
     static constexpr int kMaskOff = kMaskEarly ? kRingBytes : (BM * kPitch + 255) / 256 * 256;
-    static constexpr int kSmemBytes = kRingBytes + (kMaskEarly ? kMUnits * 256 : 0);
-    static_assert(kMaskOff + kMUnits * 256 <= kSmemBytes && kSmemBytes * OCC <= 160 * 1024, "LDS of the resident workgroups");
-    static_assert(BM * kPitch <= kRingBytes, "the epilogue stages through the operand ring");
+    static constexpr int kSmemBytes = kMaskOff + kMUnits * 256 > kRingBytes ? kMaskOff + kMUnits * 256 : kRingBytes;
+    static_assert(kSmemBytes * OCC <= 160 * 1024, "LDS of the resident workgroups");
+    static_assert(BM * kPitch <= kMaskOff, "the epilogue stages through the operand ring");
     static_assert(TM == 1 || TM == 2 || TM == 4, "scale dwords of a lane are read as one vector");
     static_assert(TN == 1 || TN == 2, "scale dwords of a lane are read as one vector");
 };
@@ -100,14 +107,17 @@ __device__ __forceinline__ void tile_issue(const TilePlan<S>& p, int stage, int 
 
 template <class S>
 struct TileFrags {
-    uint4 a[S::TM], b[S::TN];
+    uint4 a[S::TM], b[S::TN * S::kBBlocks];
 };
 template <class S>
 __device__ __forceinline__ void tile_read(const uint8_t* __restrict__ stage, int a_off, int b_off, TileFrags<S>& f) {
 #pragma unroll
     for (int i = 0; i < S::TM; ++i) f.a[i] = *reinterpret_cast<const uint4*>(stage + a_off + i * 32 * kRowBytes);
 #pragma unroll
-    for (int j = 0; j < S::TN; ++j) f.b[j] = *reinterpret_cast<const uint4*>(stage + b_off + j * 32 * kRowBytes);
+    for (int j = 0; j < S::TN; ++j)
+#pragma unroll
+        for (int q = 0; q < S::kBBlocks; ++q)
+            f.b[j * S::kBBlocks + q] = *reinterpret_cast<const uint4*>(stage + b_off + q * S::BN * kRowBytes + j * 32 * kRowBytes);
 }
 // SWAP: B's rows (n) are the instruction's first operand, so a lane ends up with quads of consecutive n of one m
 template <class S, int SUB, bool SWAP, bool ZERO>
@@ -118,7 +128,10 @@ __device__ __forceinline__ void tile_mfma(const TileFrags<S>& f, const uint32_t 
         const v8i av = v8i{(int)f.a[i].x, (int)f.a[i].y, (int)f.a[i].z, (int)f.a[i].w, 0, 0, 0, 0};
 #pragma unroll
         for (int j = 0; j < S::TN; ++j) {
-            const v8i bv = v8i{(int)f.b[j].x, (int)f.b[j].y, (int)f.b[j].z, (int)f.b[j].w, 0, 0, 0, 0};
+            // eight-bit operand: a lane holds sixteen bytes of either block of 32 indices, low registers first (FP4: a whole block)
+            const uint4 b0 = f.b[j * S::kBBlocks], b1 = S::kWideB ? f.b[j * S::kBBlocks + S::kBBlocks - 1] : make_uint4(0u, 0u, 0u, 0u);
+            const v8i bv = v8i{(int)b0.x, (int)b0.y, (int)b0.z, (int)b0.w, (int)b1.x, (int)b1.y, (int)b1.z, (int)b1.w};
+            constexpr int kFmtB = S::kWideB ? 1 : 4;   // E5M2, E2M1
             v16f cin;
             if constexpr (ZERO) {
 #pragma unroll
@@ -127,9 +140,9 @@ __device__ __forceinline__ void tile_mfma(const TileFrags<S>& f, const uint32_t 
                 cin = acc[i][j];
             }
             if constexpr (SWAP)
-                acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bv, av, cin, 4, 4, SUB, (int)scb[j], SUB, (int)sca[i]);
+                acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bv, av, cin, kFmtB, 4, SUB, (int)scb[j], SUB, (int)sca[i]);
             else
-                acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(av, bv, cin, 4, 4, SUB, (int)sca[i], SUB, (int)scb[j]);
+                acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(av, bv, cin, 4, kFmtB, SUB, (int)sca[i], SUB, (int)scb[j]);
         }
     }
 }
@@ -158,8 +171,10 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
     const int swz = (lrow >> 2) & 3;
     const int a_off0 = (wm * S::WM + lrow) * kRowBytes + (((2 * half) ^ swz) * 16);
     const int a_off1 = (wm * S::WM + lrow) * kRowBytes + (((2 * half + 1) ^ swz) * 16);
-    const int b_off0 = S::kBOff + (wn * S::WN + lrow) * kRowBytes + (((2 * half) ^ swz) * 16);
-    const int b_off1 = S::kBOff + (wn * S::WN + lrow) * kRowBytes + (((2 * half + 1) ^ swz) * 16);
+    // the 16-byte pieces of B's row for the two halves of a K step: block 2 * half + sub of 32 codes; with eight-bit values bytes
+    // 16 * half of block sub in the first 64 indices and of block 2 + sub in the second
+    const int b_off0 = S::kBOff + (wn * S::WN + lrow) * kRowBytes + (((S::kWideB ? half : 2 * half) ^ swz) * 16);
+    const int b_off1 = S::kBOff + (wn * S::WN + lrow) * kRowBytes + (((S::kWideB ? 2 + half : 2 * half + 1) ^ swz) * 16);
     // scales in LDS: A dword p holds row (p / (32 TM)) * WM + (p % TM) * 32 + (p / TM) % 32, so one read fetches the scale
     // dwords of a lane's TM blocks; B likewise with TN and WN
     const int a_sc_off = S::kSAOff + (wm * 32 + lrow) * (4 * S::TM);
@@ -176,9 +191,9 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
             return tiled ? (uint32_t)((r >> 4) * row16) + (uint32_t)((r & 15) * 64 + pcv * 16) : (uint32_t)(r * code_pitch + pcv * 16);
         };
         plan.kstep_a = g.a_tiled ? 1024 : kRowBytes;
-        plan.kstep_b = g.b_tiled ? 1024 : kRowBytes;
+        plan.kstep_b = g.b_tiled ? 1024 * S::kBBlocks : kRowBytes;
         plan.a = g.a_codes + (int64_t)m0 * code_pitch + (int64_t)k_first * plan.kstep_a;   // m0, n0 are multiples of 16: the same
-        plan.b = g.b_codes + (int64_t)n0 * code_pitch + (int64_t)k_first * plan.kstep_b;   //   expression in both layouts
+        plan.b = g.b_codes + (int64_t)n0 * code_pitch * S::kBBlocks + (int64_t)k_first * plan.kstep_b;   //   expression in both layouts
 #pragma unroll
         for (int j = 0; j < S::kALoads; ++j) {
             const int r = (wave * S::kALoads + j) * 16 + prow;
@@ -186,8 +201,12 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
         }
 #pragma unroll
         for (int j = 0; j < S::kBLoads; ++j) {
-            const int r = (wave * S::kBLoads + j) * 16 + prow;
-            plan.voff_b[j] = row_off(r < last_b ? r : last_b, g.b_tiled);
+            const int u = wave * S::kBLoads + j, r = (u % (S::BN / 16)) * 16 + prow;   // eight-bit B: every column's first 64 indices, then the second
+            const int rr = r < last_b ? r : last_b;
+            if constexpr (S::kWideB)
+                plan.voff_b[j] = (uint32_t)((rr >> 4) * 2 * row16) + (uint32_t)((u / (S::BN / 16)) * 1024 + (rr & 15) * 64 + pcv * 16);
+            else
+                plan.voff_b[j] = row_off(rr, g.b_tiled);
         }
         plan.half_back = (uint32_t)(pcv & 2) * 16u;
         plan.lds_a = (uint32_t)__builtin_amdgcn_readfirstlane((int)(smem_base + wave * S::kALoads * 1024));
@@ -260,7 +279,7 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
         for (int j = 0; j < S::TN; ++j) scb[j] = __builtin_amdgcn_ubfe(sb[j], (uint32_t)sh, 16u);
         tile_read<S>(cur, a_off1, b_off1, f1);
         tile_mfma<S, 0, SWAP, FIRST>(f0, sca, scb, acc);
-        if constexpr (S::TM * S::TN >= S::TM + S::TN) { QM_SCHED_PAIR(0x100, S::TM + S::TN) }
+        if constexpr (S::TM * S::TN >= S::TM + S::TN) { QM_SCHED_PAIR(0x100, S::TM + S::TN * S::kBBlocks) }
         __builtin_amdgcn_sched_barrier(0);
         // younger than the requests of step s + 1: those of the STAGES - 2 steps after it
         __builtin_amdgcn_s_waitcnt(vmcnt_imm((S::STAGES - 2) * S::kLoads));
@@ -273,7 +292,7 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
         settle_scales(sa, sb, s + 1);
         tile_read<S>(nxt, a_off0, b_off0, f0);
         tile_mfma<S, 1, SWAP, false>(f1, sca, scb, acc);
-        if constexpr (S::TM * S::TN >= S::TM + S::TN) { QM_SCHED_PAIR(0x100, S::TM + S::TN) }
+        if constexpr (S::TM * S::TN >= S::TM + S::TN) { QM_SCHED_PAIR(0x100, S::TM + S::TN * S::kBBlocks) }
         __builtin_amdgcn_sched_barrier(0);
         stage = nstage;
     };
@@ -381,12 +400,24 @@ __global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu((S:
     }
 }
 
+// the same with an eight-bit B (one product)
+template <class S, typename OutT>
+__global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu((S::OCC * S::kWaves + 3) / 4))) void gemm_mxfp4_e5m2_tile_kernel(
+    TileProduct g, int tiles) {
+    extern __shared__ uint32_t smem[];
+    const uint32_t smem_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint32_t*)smem;
+    for (int t = (int)blockIdx.x; t < tiles; t += (int)gridDim.x) tile_run<S, OutT>(g, t, smem, smem_base);
+}
+
 template <class S>
 int tiles_of(const TileProduct& p) { return p.M == 0 ? 0 : ((p.M + S::BM - 1) / S::BM) * ((p.N + S::BN - 1) / S::BN) * p.splits; }
 
 template <class S, typename OutT>
 hipError_t launch_tiles(const TileProduct& g, const TileProduct& h, hipStream_t stream) {
-    auto kern = gemm_mxfp4_tn_tile_kernel<S, OutT>;
+    const auto kern = [] {
+        if constexpr (S::kWideB) return gemm_mxfp4_e5m2_tile_kernel<S, OutT>;
+        else return gemm_mxfp4_tn_tile_kernel<S, OutT>;
+    }();
     static std::atomic<bool> lds_allowed[kMaxDevices];
     hipError_t e = allow_dynamic_lds(kern, S::kSmemBytes, lds_allowed);
     if (e != hipSuccess) return e;
@@ -394,7 +425,8 @@ hipError_t launch_tiles(const TileProduct& g, const TileProduct& h, hipStream_t 
     // a grid that is a multiple of 8 so that tile t and t + grid land on the same XCD
     int grid = tiles < S::OCC * device_cus() ? tiles : S::OCC * device_cus();
     if (grid > 8 && grid < tiles) grid -= grid % 8;
-    kern<<<dim3((unsigned)grid), dim3(S::kThreads), S::kSmemBytes, stream>>>(g, h, tg, tiles);
+    if constexpr (S::kWideB) kern<<<dim3((unsigned)grid), dim3(S::kThreads), S::kSmemBytes, stream>>>(g, tiles);
+    else kern<<<dim3((unsigned)grid), dim3(S::kThreads), S::kSmemBytes, stream>>>(g, h, tg, tiles);
     return hipGetLastError();
 }
 
@@ -403,6 +435,12 @@ using Tile128x128 = TileShape<128, 128, 64, 64, 3, 3>;
 using Tile128x64 = TileShape<128, 64, 64, 32, 4, 3>;
 using Tile64x64 = TileShape<64, 64, 32, 32, 4, 4>;
 using Tile64x32 = TileShape<64, 32, 32, 32, 6, 4>;
+// with an eight-bit B.  4096^3 in us: 256x256 in 8 waves of 128 x 64, 3 stages 60; in 4 waves of 128 x 128 66; 256x128 73 to 84;
+// 128x128 with 2 stages three times per CU 74, with 3 stages twice 81
+using Wide256x256 = TileShape<256, 256, 128, 64, 3, 1, true>;
+using Wide128x128 = TileShape<128, 128, 64, 64, 2, 3, true>;
+using Wide128x64 = TileShape<128, 64, 64, 32, 3, 3, true>;
+using Wide64x64 = TileShape<64, 64, 32, 32, 4, 3, true>;
 
 }  // namespace
 
@@ -419,6 +457,14 @@ hipError_t gemm_tile(int shape, const TileProduct& g, const TileProduct* second,
         using S = decltype(s);
         return c_dtype == BF16 ? launch_tiles<S, uint16_t>(g, h, stream) : launch_tiles<S, float>(g, h, stream);
     };
+    if (g.b_e5m2) {
+        switch (shape) {
+            case WIDE_256x256: return go(Wide256x256{});
+            case TILE_128x128: return go(Wide128x128{});
+            case TILE_128x64: return go(Wide128x64{});
+            default: return go(Wide64x64{});
+        }
+    }
     switch (shape) {
         case TILE_256x128: return go(Tile256x128{});
         case TILE_128x128: return go(Tile128x128{});

@@ -25,6 +25,7 @@ using std::optional;
 
 PyObject* g_error_class = nullptr;   // quartet_amd._lib.QuartetHipError
 PyObject* g_draw = nullptr;          // quartet_amd.linear._gradient_draws
+PyObject* g_error_draw = nullptr;    // quartet_amd.linear._error_draws
 
 // ---- errors: raised as Python exceptions, also from the autograd engine's threads --------------------------------
 [[noreturn]] void raise(PyObject* type, const std::string& message) {
@@ -115,6 +116,7 @@ struct Layer : torch::CustomClassHolder {
     int64_t T = 0, I = 0, O = 0;
     int layout = QM_LAYOUT_ROWMAJOR;
     bool seed_base_ok = false;
+    bool error_only = false;   // scheme "Q(E)W_Q(Et)X": the gradient products take the packed operands as they are
     at::ScalarType x_dtype{}, w_dtype{};
     std::vector<int64_t> x_shape;
     explicit Layer(py::handle q) : g_q(q) {}
@@ -254,6 +256,41 @@ Gradients backward_products(const Layer& l, const Tensor& e, const Tensor& packe
     return {gx, gw, sd_x};
 }
 
+// The same for the error-only scheme (backward.py:21-45): Q(e) and Q(e^T) times the packed operands as they are, in bf16
+Gradients error_products(const Layer& l, const Tensor& e, const Tensor& packed_x, const Tensor& packed_w) {
+    const Tensor e2 = rows_of(e, e.size(-1));
+    require_cuda(e2);
+    Signs g_signs;
+    uint64_t seeds[2];
+    bool stochastic;
+    {
+        py::gil_scoped_acquire gil;
+        try {
+            const py::tuple drawn = py::reinterpret_steal<py::object>(PyObject_CallFunctionObjArgs(g_error_draw, l.g_q.p, py::cast(e2).ptr(), nullptr));
+            if (!drawn.ptr()) throw py::error_already_set();
+            g_signs = signs_of(drawn[0]);
+            const py::tuple s = drawn[1];
+            for (int i = 0; i < 2; ++i) seeds[i] = s[i].cast<uint64_t>();
+            stochastic = drawn[2].cast<bool>();
+        } catch (py::error_already_set& err) {
+            err.restore();
+            python_error again;
+            again.persist();
+            throw again;
+        }
+    }
+    const at::ScalarType gw_dtype = l.w_dtype == at::kFloat ? at::kFloat : at::kBFloat16;
+    const int64_t nbytes = (int64_t)qm_linear_backward_error_workspace_bytes(l.T, l.I, l.O);
+    const Tensor work = bytes(nbytes, e2);
+    const Tensor gx = at::empty({l.T, l.I}, e2.options().dtype(at::kBFloat16)), gw = at::empty({l.O, l.I}, e2.options().dtype(gw_dtype));
+    check(qm_linear_backward_error(e2.data_ptr(), dtype_code(e2.scalar_type()), l.T, l.I, l.O, packed_x.data_ptr(), packed_w.data_ptr(), l.a_hd,
+                                   l.a_signs.data(), l.w_hd, l.w_signs.data(), l.g_hd, g_signs.data(), stochastic ? QM_ABSMAX_SR : QM_ABSMAX_RTN,
+                                   seeds, QM_BF16, QM_BF16, work.data_ptr(), (size_t)nbytes, gx.data_ptr(), gw.data_ptr(), dtype_code(gw_dtype),
+                                   stream_of(e2)),
+          "qm_linear_backward_error");
+    return {gx, gw, at::kBFloat16};
+}
+
 void keep_layer(AutogradContext* ctx, const LayerPtr& l) { ctx->saved_data["layer"] = c10::IValue::make_capsule(l); }
 LayerPtr kept_layer(AutogradContext* ctx) { return c10::static_intrusive_pointer_cast<Layer>(ctx->saved_data["layer"].toCapsule()); }
 
@@ -281,7 +318,7 @@ struct LinearFn : Function<LinearFn> {
         const LayerPtr l = kept_layer(ctx);
         const auto saved = ctx->get_saved_variables();
         const c10::OptionalDeviceGuard guard(saved[0].device());
-        const Gradients g = backward_products(*l, grads[0], saved[0], saved[1], false);
+        const Gradients g = l->error_only ? error_products(*l, grads[0], saved[0], saved[1]) : backward_products(*l, grads[0], saved[0], saved[1], false);
         return {g.gx.to(l->x_dtype).view(l->x_shape), g.gw.to(l->w_dtype), Tensor(), Tensor()};
     }
 };
@@ -293,9 +330,10 @@ bool wants_grad(std::initializer_list<const Tensor*> ts) {
 }
 
 py::tuple linear(const Tensor& x, const Tensor& weight, int a_hd, py::handle a_signs, int w_hd, py::handle w_signs, int g_hd, py::handle g_q,
-                 const optional<Tensor>& packed_weight, const optional<Tensor>& x_dense, const optional<Tensor>& w_dense) {
+                 const optional<Tensor>& packed_weight, const optional<Tensor>& x_dense, const optional<Tensor>& w_dense, bool error_only) {
     return from_python([&] {
         const LayerPtr l = make_layer(a_hd, a_signs, w_hd, w_signs, g_hd, g_q, x_dense, w_dense);
+        l->error_only = error_only;
         Tensor packed_w = or_none(packed_weight), packed_x;
         const c10::OptionalDeviceGuard guard(weight.is_cuda() ? std::optional<at::Device>(weight.device()) : std::nullopt);
         const Tensor y = wants_grad({&x, &weight}) ? LinearFn::apply(x, weight, l, &packed_w) : linear_forward(l, x, weight, packed_x, packed_w);
@@ -560,9 +598,10 @@ py::int_ sign_flips(int64_t hd) {
     return py::reinterpret_steal<py::int_>(_PyLong_FromByteArray(raw, sizeof(raw), 1, 0));
 }
 
-void bind(py::object error_class, py::object draw) {
+void bind(py::object error_class, py::object draw, py::object error_draw) {
     g_error_class = error_class.release().ptr();
     g_draw = draw.release().ptr();
+    g_error_draw = error_draw.release().ptr();
 }
 
 }  // namespace

@@ -96,6 +96,39 @@ hipError_t quantize_layer_backward(const void* e, int dtype, int64_t T, int64_t 
                                    uint64_t seed_rows, uint64_t seed_transposed, uint8_t* codes_rows, uint8_t* scales_rows,
                                    uint8_t* codes_transposed, uint8_t* scales_transposed, const RequantArgs& x, const RequantArgs& w,
                                    const uint64_t* seed_base, hipStream_t stream);
+// the two quantizations of e alone
+hipError_t quantize_error(const void* e, int dtype, int64_t T, int64_t O, int hd, const SignBits& signs, int mode, uint64_t seed_rows,
+                          uint64_t seed_transposed, uint8_t* codes_rows, uint8_t* scales_rows, uint8_t* codes_transposed,
+                          uint8_t* scales_transposed, const uint64_t* seed_base, hipStream_t stream);
+// Packed quest-coded tensors [R, C] (padded tiled codes; R and C multiples of 32) as operands of products that contract
+// over R (expand.hip): E5M2 bytes, padded_rows(C) * padded_cols(R) of them, E8M0 scales [C][padded_cols(R) / 32], and one
+// byte per 128 x 128 block, [ceil(C / 128)][padded_cols(R) / 128], nonzero where the block has a value that E5M2 cannot hold
+struct E5m2Args {
+    const uint8_t* codes_in;
+    const uint8_t* scales_in;
+    int64_t R, C;
+    uint8_t* values;
+    uint8_t* scales;
+    uint8_t* lost;
+};
+hipError_t expand_e5m2_pair(const E5m2Args& a, const E5m2Args& b, hipStream_t stream);
+// The columns of a product that such a loss touches, once more and from the packed tensors: c = the masked inverse rotation of
+// bf16(alpha * A B), A [M, K] tiled codes, B the packed [R, C] tensor behind `b`.  Two products in one launch, which ends at
+// once where nothing was lost.
+struct E5m2Exact {
+    const uint8_t* a_codes;
+    const uint8_t* a_scales;
+    E5m2Args b;
+    int64_t M;
+    float alpha;
+    const uint8_t* mask;
+    int hd;
+    SignBits signs;
+    float rot_c;
+    void* c;
+    int out_dtype;
+};
+hipError_t e5m2_exact_pair(const E5m2Exact& a, const E5m2Exact& b, hipStream_t stream);
 hipError_t masked_hadamard_bwd_hd32_pair(const void* ga, int64_t na, int scale_dtype_a, uint32_t sign_a, const uint8_t* mask_a, void* out_a,
                                          const void* gb, int64_t nb, int scale_dtype_b, uint32_t sign_b, const uint8_t* mask_b, void* out_b,
                                          int dtype, int out_dtype_b, hipStream_t stream);
@@ -132,6 +165,7 @@ hipError_t gemm_mxfp4_tn(const uint8_t* a_codes, const uint8_t* a_scales, const 
 hipError_t splitk_reduce_rotated(const float* partial, int splits, int64_t mn, float alpha, int mid_dtype, const uint8_t* maskbits,
                                  int hd, const SignBits& signs, float c, void* out, int out_dtype, hipStream_t stream);
 size_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
+size_t gemm_e5m2_workspace_bytes(int64_t M, int64_t N, int64_t K);   // the same for a product with an eight-bit B
 
 // The product on small and middle-sized tiles (gemm_tile.hip).  Any M; N % 8 == 0; K % 128 == 0, or K % 128 == 64 with
 // row-major operands; c 16-byte aligned.  A tiled operand's last block of 16 rows exists in memory whatever its row count.
@@ -153,8 +187,10 @@ struct TileProduct {
     SignBits signs;
     float rot_c;
     int out_f32;
+    int b_e5m2;            // B holds eight-bit values from expand_e5m2_pair (N % 32 == 0, K % 128 == 0, tiled A)
 };
-enum TileKind : int { TILE_256x128 = 0, TILE_128x128 = 1, TILE_128x64 = 2, TILE_64x64 = 3, TILE_64x32 = 4 };
+// the kinds of an eight-bit B are WIDE_256x256 and 1 .. 3
+enum TileKind : int { TILE_256x128 = 0, WIDE_256x256 = 0, TILE_128x128 = 1, TILE_128x64 = 2, TILE_64x64 = 3, TILE_64x32 = 4 };
 bool gemm_tile_serves(int64_t M, int64_t N, int64_t K, int a_tiled, int b_tiled, const void* c);
 // one product, or two independent ones of the same element type in one grid
 hipError_t gemm_tile(int kind, const TileProduct& g, const TileProduct* second, int c_dtype, hipStream_t stream);

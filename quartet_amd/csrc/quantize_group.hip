@@ -1300,10 +1300,9 @@ hipError_t quantize_layer_forward(const RowmajorArgs& x, const RowmajorArgs* w, 
     return hipGetLastError();
 }
 
-hipError_t quantize_layer_backward(const void* e, int dtype, int64_t T, int64_t O, int hd, const SignBits& signs, int mode,
-                                   uint64_t seed_rows, uint64_t seed_transposed, uint8_t* codes_rows, uint8_t* scales_rows,
-                                   uint8_t* codes_transposed, uint8_t* scales_transposed, const RequantArgs& x, const RequantArgs& w,
-                                   const uint64_t* seed_base, hipStream_t stream) {
+hipError_t quantize_error(const void* e, int dtype, int64_t T, int64_t O, int hd, const SignBits& signs, int mode, uint64_t seed_rows,
+                          uint64_t seed_transposed, uint8_t* codes_rows, uint8_t* scales_rows, uint8_t* codes_transposed,
+                          uint8_t* scales_transposed, const uint64_t* seed_base, hipStream_t stream) {
     const GroupOut orow{reinterpret_cast<uint4*>(codes_rows), scales_rows, nullptr, nullptr};
     with_absmax_mode(mode, [&](auto m) {
         with_hadamard(hd, [&](auto h) {
@@ -1319,6 +1318,21 @@ hipError_t quantize_layer_backward(const void* e, int dtype, int64_t T, int64_t 
                     launch_jobs(stream, jt, jr);
                 });
             });
+        });
+    });
+    return hipGetLastError();
+}
+
+hipError_t quantize_layer_backward(const void* e, int dtype, int64_t T, int64_t O, int hd, const SignBits& signs, int mode,
+                                   uint64_t seed_rows, uint64_t seed_transposed, uint8_t* codes_rows, uint8_t* scales_rows,
+                                   uint8_t* codes_transposed, uint8_t* scales_transposed, const RequantArgs& x, const RequantArgs& w,
+                                   const uint64_t* seed_base, hipStream_t stream) {
+    const hipError_t rc = quantize_error(e, dtype, T, O, hd, signs, mode, seed_rows, seed_transposed, codes_rows, scales_rows, codes_transposed,
+                                         scales_transposed, seed_base, stream);
+    if (rc != hipSuccess) return rc;
+    with_absmax_mode(mode, [&](auto m) {
+        with_hadamard(hd, [&](auto h) {
+            constexpr int M = decltype(m)::value, HD = decltype(h)::value;
             const auto ragged = [](const RequantArgs& a) { return a.R % 128 != 0 || a.C % 128 != 0; };
             with_flag(ragged(x) || ragged(w), [&](auto p) {
                 // a quest-coded operand (post = 1, no de-quantized output): its value type only picks the rounding of hd^-1/2

@@ -5,15 +5,16 @@ Production configuration (main_setup.sh:77-93 of the reference): QuestMXFP4Quant
 activations, AlbertTsengQuantizer on gradients, scheme "Q(E)Q(Wt)t_Q(Et)Q(Xt)t".  For it the layer
 never materialises de-quantized tensors: operands stay packed (E2M1 codes + E8M0 scales + mask
 bits, the tensors notebooks/benchmark_mxfp4.ipynb's CudaGemm saves) and the three products run on
-the block-scaled FP4 MFMA.  Any other mix of quantizers/schemes takes the generic path through the
+the block-scaled FP4 MFMA.  The scheme that quantizes only the error signal ("Q(E)W_Q(Et)X") runs on the same packed
+operands where its products are bf16 ones.  Any other mix of quantizers/schemes takes the generic path through the
 quantizer modules and library GEMMs, as the reference does."""
 import torch
 import torch.nn as nn
 
 from . import _lib
-from .backward import BACKWARD_SCHEMES, EW_EtX_Scheme, QEQWtt_QEtQXtt_Scheme  # noqa: F401
+from .backward import BACKWARD_SCHEMES, EW_EtX_Scheme, QEQWtt_QEtQXtt_Scheme, QEW_QEtX_Scheme  # noqa: F401
 from .quantizers import QUANTIZER_CLASSES, AlbertTsengQuantizer, NoQuantizer, QuestMXFP4Quantizer  # noqa: F401
-from .quantizers.mxfp4 import _fresh_seed
+from .quantizers.mxfp4 import _autocast_bf16, _fresh_seed
 
 
 _SEED_BASE = None
@@ -53,6 +54,14 @@ def _gradient_draws(g_q, seed_base_ok, T, I, O):
     return g_q.sign_bits, seeds, stochastic, g_q._dense, base
 
 
+def _error_draws(g_q, e):
+    """The same for the error-only scheme: no fresh column signs, one seed for e and one for e^T.  Returns (column signs,
+    seeds, stochastic)."""
+    g_q._note_input(e)
+    seeds = (_fresh_seed(), _fresh_seed()) if g_q.stochastic else (0, 0)
+    return g_q.sign_bits, seeds, g_q.stochastic
+
+
 def _cached_weight(x, weight, a_q, w_q, g_q, weight_cache):
     """(cache key, packed Q(W) or None): Q(W) of an unchanged weight (the micro-steps of one accumulation) is quantized
     once and kept by the layer.  The last two entries of the key stand for the code layout, which csrc/host_ext.cpp picks."""
@@ -76,13 +85,15 @@ class QuartetLinearFn:
     backward: re-randomise signs; B1 Q(e); B2 Q(Q(W)^T); B3 GEMM -> grad wrt Q(x);
               B4 Q(e^T); B5 Q(Q(x)^T); B6 GEMM -> grad wrt Q(W);
               B7/B8 masked inverse rotation (straight-through estimators of F1/F2).
+    error_only: the scheme of backward.py:21-45 instead -- no new signs, B1 Q(e), B4 Q(e^T), their products with the packed
+    Q(W) and Q(x) as they are, B7/B8.
     The autograd function itself is native (csrc/host_ext.cpp)."""
 
     @staticmethod
-    def apply(x, weight, a_q, w_q, g_q, weight_cache):
+    def apply(x, weight, a_q, w_q, g_q, weight_cache, error_only=False):
         key, packed_w = _cached_weight(x, weight, a_q, w_q, g_q, weight_cache)
         y, packed_w = _lib.host().linear(x, weight, a_q.hadamard_dim, a_q.sign_bits, w_q.hadamard_dim, w_q.sign_bits, g_q.hadamard_dim, g_q,
-                                         packed_w, _dense(a_q, weight), _dense(w_q, weight))
+                                         packed_w, _dense(a_q, weight), _dense(w_q, weight), error_only)
         if key is not None:
             weight_cache.put(key, packed_w)
         return y
@@ -166,11 +177,36 @@ class QuantizedLinear(nn.Linear):
             return g_q.hadamard_dim == 32 and not any(d % 128 for d in (tokens, self.in_features, self.out_features))
         return True
 
+    def _is_error_only_config(self, x):
+        """The error-only scheme between the same quantizers, with products in bf16 (bf16 autocast, or bf16 tensors throughout)
+        and extents that are multiples of 32 and of the Hadamard blocks."""
+        modules = self._modules
+        a_q, w_q, scheme = modules["activation_quantizer"], modules["weight_quantizer"], modules["backward_scheme"]
+        g_q = scheme.g_quantizer
+        if not (self.use_packed_path and type(scheme) is QEW_QEtX_Scheme and type(a_q) is QuestMXFP4Quantizer
+                and type(w_q) is QuestMXFP4Quantizer and type(g_q) is AlbertTsengQuantizer):
+            return False
+        if a_q.is_dense or w_q.is_dense or g_q.is_dense:
+            return False
+        weight, out = self.weight, (torch.bfloat16, torch.float32)
+        if not (x.is_cuda and weight.is_cuda and x.numel() and x.dtype in out and weight.dtype in out
+                and (x.dtype == weight.dtype == torch.bfloat16 or _autocast_bf16())):
+            return False
+        O, I = weight.shape
+        T = x.numel() // x.shape[-1]
+        return not (x.shape[-1] != I or T % 32 or I % 32 or O % 32 or I % a_q.hadamard_dim or I % w_q.hadamard_dim
+                    or T % g_q.hadamard_dim or O % g_q.hadamard_dim)
+
     def forward(self, x):
         if self._is_production_config(x.numel() // max(x.shape[-1], 1)):
             modules = self._modules
             return QuartetLinearFn.apply(x, self.weight, modules["activation_quantizer"], modules["weight_quantizer"],
                                          modules["backward_scheme"].g_quantizer, self.packed_weight_cache)
+        if self._is_error_only_config(x):
+            a_q, w_q, g_q = self.activation_quantizer, self.weight_quantizer, self.backward_scheme.g_quantizer
+            a_q._note_input(x)
+            w_q._note_input(self.weight)
+            return QuartetLinearFn.apply(x, self.weight, a_q, w_q, g_q, self.packed_weight_cache, True)
         xq = self.activation_quantizer(x)
         wq = self.weight_quantizer(self.weight)
         return self.backward_scheme(xq, wq)

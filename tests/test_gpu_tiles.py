@@ -99,3 +99,66 @@ def test_layer_on_padded_operands(oracle, T, I, O, hd):
     assert rel(y.detach().float().cpu().numpy(), y_ref) <= 3e-3
     assert rel(xd.grad.float().cpu().numpy(), ste(gxq, qx)) <= 5e-3
     assert rel(layer.weight.grad.float().cpu().numpy(), ste(gwq, qw)) <= 5e-3
+
+
+def error_only_layer(q, I, O, hd, dtype):
+    return q.QuantizedLinear(I, O, bias=False, weight_quantizer=q.QuestMXFP4Quantizer(hadamard_dim=hd),
+                             activation_quantizer=q.QuestMXFP4Quantizer(hadamard_dim=hd),
+                             gradient_quantizer=q.AlbertTsengQuantizer(hadamard_dim=hd, stochastic=True),
+                             backward_scheme=q.BACKWARD_SCHEMES["Q(E)W_Q(Et)X"]()).to("cuda:0", dtype)
+
+
+@pytest.mark.parametrize("T,I,O,hd,wide,spread",
+                         [(*case, s) for case in [(32, 32, 32, 32, False), (96, 160, 1056, 32, True), (256, 384, 640, 128, False)] for s in (0, 26, 28, 29, 60)] +
+                         [(544, 1728, 352, 32, False, 0), (4160, 192, 128, 64, True, 28), (4160, 192, 128, 64, True, 29), (1152, 2048, 2176, 32, False, 28)])
+def test_error_only_layer_on_packed_operands(oracle, monkeypatch, T, I, O, hd, wide, spread):
+    """Scheme Q(E)W_Q(Et)X on packed operands, widened to eight bits for its products, against the oracle's de-quantized
+    tensors multiplied in float64.  spread: all but every seventh row of x and of W are scaled by 2^spread, so that the row scales
+    of a block of 32 lie within the eight-bit format (28 octaves) or not.  bf16 results: one rounding of the product and one of the
+    rotation, each of relative size 2^-9, against the oracle's bf16 product rotated exactly."""
+    print(f"case error-only T={T} I={I} O={O} hd={hd} wide={wide} spread={spread}", flush=True)
+    import quartet_amd as q
+    from quartet_amd import kernels as Kn
+    monkeypatch.setattr(Kn, "gemm_mxfp4_bf16_nn", lambda *a, **k: pytest.fail("left the packed path"))
+    scaled = lambda t: torch.where(torch.arange(t.shape[0]).unsqueeze(1) % 7 == 3, t.float(), t.float() * 2.0 ** spread).to(t.dtype)
+    x = scaled(make_input(T, I, torch.bfloat16, seed=1, outlier_frac=0.01))
+    w = scaled(make_input(O, I, torch.bfloat16, seed=2, outlier_frac=0, scale=0.02))
+    idx = np.arange(hd)
+    parity = np.array([[bin(i & j).count("1") & 1 for j in idx] for i in idx])
+    if spread:
+        # an error signal that, rotated along either axis, is nonzero only where the other operand's row is a small one, so that
+        # nothing larger hides what is lost: whole numbers, which neither bf16 nor the rotation rounds
+        pick = torch.Generator().manual_seed(4)
+        s = torch.randint(0, 2, (T, O), generator=pick).double() * 2 - 1
+        s *= (torch.arange(T) % 7 == 3).unsqueeze(1) * (torch.arange(O) % 7 == 3)
+        sign = torch.from_numpy(np.where(parity, -1.0, 1.0))
+        s = (s.view(-1, hd) @ sign).view(T, O)
+        e = ((s.T.reshape(-1, hd) @ sign).view(O, T).T * 2.0 ** -10).to(torch.bfloat16).contiguous()
+    else:
+        e = make_input(T, O, torch.bfloat16, seed=3, outlier_frac=0, scale=1e-3)
+    layer = error_only_layer(q, I, O, hd, torch.float32 if wide else torch.bfloat16)
+    with torch.no_grad():
+        layer.weight.copy_(w.to("cuda:0"))
+    xd = x.to("cuda:0").requires_grad_(True)
+    random.seed(5)
+    with torch.autocast("cuda", torch.bfloat16, enabled=wide):
+        y = layer(xd)
+        y.backward(e.to("cuda:0"))
+    torch.cuda.synchronize()
+    random.seed(5)
+    o, d = oracle, float(oracle.FOUR_THIRDS)
+    qx = o.quantize(to_oracle(x), hd, mode=o.QUEST_RTN, want_mask=True)
+    qw = o.quantize(to_oracle(w.float() if wide else w), hd, mode=o.QUEST_RTN, want_mask=True)
+    qe = o.quantize(to_oracle(e), hd, mode=o.ABSMAX_SR, seed=random.getrandbits(63))
+    qet = o.quantize(to_oracle(e), hd, mode=o.ABSMAX_SR, transposed_in=True, seed=random.getrandbits(63))
+    xv, wv = o.dequantize(qx["codes"], qx["scales"], 1.0).astype(np.float64), o.dequantize(qw["codes"], qw["scales"], 1.0).astype(np.float64)
+    ev, etv = o.dequantize(qe["codes"], qe["scales"], d).astype(np.float64), o.dequantize(qet["codes"], qet["scales"], d).astype(np.float64)
+    c = float(torch.tensor(hd ** -0.5).to(torch.bfloat16))
+    H = np.where(parity, -c, c)
+
+    def rotate(p, mask):
+        keep = np.unpackbits(np.asarray(mask).reshape(p.shape[0], -1), axis=1, bitorder="little")
+        return ((torch.from_numpy(p).to(torch.bfloat16).double().numpy() * keep).reshape(-1, hd) @ H.T).reshape(p.shape)
+    assert rel(y.detach().float().cpu(), xv @ wv.T) < 4e-3
+    assert rel(xd.grad.float().cpu(), rotate(ev @ wv, qx["mask"])) < 4e-3
+    assert rel(layer.weight.grad.float().cpu(), rotate(etv @ xv, qw["mask"])) < 4e-3
