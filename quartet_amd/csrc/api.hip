@@ -482,6 +482,10 @@ int qm_linear_forward(const void* x, int x_dtype, const void* w, int w_dtype, in
     }
     if (rc) return rc;
     if (!valid_dtype(y_dtype)) return fail(QM_ERR_INVALID, "qm_linear_forward: y_dtype %d", y_dtype);
+    if (T <= 64 && O < (1ll << 30) && K < (1ll << 30) && tiled_layout(codes_layout)) {
+        const qm::TileProduct p = qm::make_product(px + lx.c, px + lx.s, pw + lw.c, pw + lw.s, T, O, K, 1.0f, y, QM_LAYOUT_TILED, QM_LAYOUT_TILED);
+        if (qm::gemm_rows_serves(p)) return from_hip(qm::gemm_rows(p, y_dtype, hs), "qm_linear_forward");
+    }
     return from_hip(qm::gemm_mxfp4_tn(px + lx.c, px + lx.s, pw + lw.c, pw + lw.s, T, O, K, 1.0f, y, y_dtype, kernel_layout(codes_layout), kernel_layout(codes_layout), nullptr, 0, hs),
                     "qm_linear_forward");
 }

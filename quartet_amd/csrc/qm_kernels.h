@@ -195,6 +195,11 @@ bool gemm_tile_serves(int64_t M, int64_t N, int64_t K, int a_tiled, int b_tiled,
 // one product, or two independent ones of the same element type in one grid
 hipError_t gemm_tile(int kind, const TileProduct& g, const TileProduct* second, int c_dtype, hipStream_t stream);
 
+// The product of at most 64 rows with a weight, both tiled (gemm_rows.hip): K % 128 == 0, N % 8 == 0, c 16-byte aligned, no mask.
+// Its sums are in another order than the other kernels'.
+bool gemm_rows_serves(const TileProduct& p);
+hipError_t gemm_rows(const TileProduct& p, int c_dtype, hipStream_t stream);
+
 // The kernel a product runs on (gemm.hip).  Products with p.mask set ask for the masked inverse rotation; `rotates` tells
 // whether that kernel applies it (p.c then holds rot_out_dtype elements: c_dtype, or F32 holding the bf16-rounded result)
 // or the caller has to (p.c then holds the plain product in c_dtype).

@@ -57,6 +57,29 @@ def test_product_cut_into_k_ranges(oracle, M, N, K):
     assert torch.equal(c16, c32.to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("T,I,O", [(1, 32, 8), (7, 96, 24), (16, 1152, 40), (9, 8192, 264), (16, 10976, 520),   # up to 16 rows: fewer steps than waves, eight waves
+                                   (17, 416, 4088), (32, 2048, 4104), (32, 2176, 4104),                          # 32 rows: one workgroup per CU, a short K beyond
+                                   (33, 640, 1016), (64, 1664, 4096), (64, 640, 4104), (65, 640, 72)])           # 64 rows, and past every bound
+def test_product_of_few_rows(oracle, T, I, O):
+    """The layer's forward product at the edges of the kernel for few tokens, against the oracle's float64 sums of the same packed
+    operands: fp32 output within K additions (1e-5 of the norm), bf16 output within one rounding of each value (2^-8)."""
+    print(f"case few rows T={T} I={I} O={O}", flush=True)
+    import quartet_amd as q
+    x = make_input(T, I, torch.bfloat16, seed=1, outlier_frac=0.01)
+    w = make_input(O, I, torch.bfloat16, seed=2, outlier_frac=0, scale=0.02)
+    layer = q.QuantizedLinear(I, O, bias=False, weight_quantizer=q.QuestMXFP4Quantizer(), activation_quantizer=q.QuestMXFP4Quantizer(),
+                              gradient_quantizer=q.AlbertTsengQuantizer(), backward_scheme=q.BACKWARD_SCHEMES["Q(E)Q(Wt)t_Q(Et)Q(Xt)t"]())
+    layer = layer.to("cuda:0", torch.bfloat16)
+    with torch.no_grad():
+        layer.weight.copy_(w.to("cuda:0"))
+        y16, y32 = layer(x.to("cuda:0")), layer(x.to("cuda:0").float())
+    o = oracle
+    qx, qf, qw = (o.quantize(to_oracle(t), 32, mode=o.QUEST_RTN) for t in (x, x.float(), w))
+    want, want32 = (o.gemm_tn(a["codes"], a["scales"], qw["codes"], qw["scales"]) for a in (qx, qf))
+    assert rel(y32.cpu().numpy(), want32) < 1e-5
+    assert rel(y16.float().cpu().numpy(), want) < 2 ** -8
+
+
 @pytest.mark.parametrize("T,I,O,hd", [(32, 32, 32, 32), (4128, 96, 160, 32), (4160, 192, 128, 64), (4224, 128, 256, 128), (96, 160, 96, 32), (288, 192, 320, 32), (544, 1728, 352, 32), (1056, 640, 1088, 32),
                                       (64, 64, 64, 64), (192, 320, 128, 64), (128, 128, 128, 128), (384, 256, 640, 128), (1280, 384, 896, 128)])
 def test_layer_on_padded_operands(oracle, T, I, O, hd):
