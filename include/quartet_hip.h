@@ -375,6 +375,17 @@ int qm_rope_split_qkv(const void* qkv, int qkv_dtype, int64_t rows, int64_t seq_
 int qm_rope_merge_qkv_grad(const void* dq, const void* dk, const void* dv, int grad_dtype, int64_t rows, int64_t seq_len,
                            int64_t n_embd, int head_dim, const float* table, void* d_qkv, int out_dtype, void* stream);
 
+/*
+ * Mean cross-entropy of logits [rows, classes] (row-major, logits_dtype) against int64 targets [rows], over the rows whose
+ * target is not ignore_index (F.cross_entropy of src/models/llama.py:254-256): fp32, *loss = mean(log(sum exp(row)) -
+ * row[target]).  No row left: NaN.  A target that is no class makes the loss NaN.
+ *   row_losses  DEVICE scratch, rows floats
+ *   loss        DEVICE pointer to one float
+ * logits aligned to their elements; rows < 2^31.  Two launches, no allocation, sums in a fixed order.
+ */
+int qm_cross_entropy(const void* logits, int logits_dtype, const int64_t* targets, int64_t rows, int64_t classes,
+                     int64_t ignore_index, float* row_losses, float* loss, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -862,4 +862,18 @@ int qm_rope_merge_qkv_grad(const void* dq, const void* dk, const void* dv, int g
                     "qm_rope_merge_qkv_grad");
 }
 
+int qm_cross_entropy(const void* logits, int logits_dtype, const int64_t* targets, int64_t rows, int64_t classes,
+                     int64_t ignore_index, float* row_losses, float* loss, void* stream) {
+    if (!valid_dtype(logits_dtype)) return fail(QM_ERR_INVALID, "qm_cross_entropy: logits_dtype must be QM_BF16/QM_F32");
+    if (rows < 0 || rows >= (1ll << 31) || classes <= 0)
+        return fail(QM_ERR_INVALID, "qm_cross_entropy: need 0 <= rows < 2^31 and classes > 0 (got [%lld, %lld])", (long long)rows, (long long)classes);
+    if (!loss || (rows > 0 && (!logits || !targets || !row_losses)))
+        return fail(QM_ERR_INVALID, "qm_cross_entropy: logits, targets, row_losses and loss must be non-null");
+    if (!aligned(logits, logits_dtype == QM_BF16 ? 2 : 4) || !aligned(targets, 8) || !aligned(row_losses, 4) || !aligned(loss, 4))
+        return fail(QM_ERR_UNALIGNED, "qm_cross_entropy: tensors must be aligned to their elements");
+    return from_hip(qm::cross_entropy_mean(logits, logits_dtype, targets, rows, classes, ignore_index, row_losses, loss,
+                                           reinterpret_cast<hipStream_t>(stream)),
+                    "qm_cross_entropy");
+}
+
 }  // extern "C"

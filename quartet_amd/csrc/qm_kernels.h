@@ -229,6 +229,10 @@ hipError_t gemm_tile_phases(const uint8_t* a_codes, const uint8_t* a_scales, con
 int mfma_only_blocks();
 hipError_t mfma_only(const uint8_t* operands, float* sink, int iters, hipStream_t stream);
 
+// mean cross-entropy over the rows whose target is not `ignore` (loss.hip); losses: scratch, one float per row
+hipError_t cross_entropy_mean(const void* logits, int dtype, const int64_t* targets, int64_t rows, int64_t classes, int64_t ignore,
+                              float* losses, float* loss, hipStream_t stream);
+
 hipError_t masked_hadamard_bwd(const void* g, int g_dtype, int64_t rows, int64_t cols, int hd, int scale_dtype,
                                const SignBits& sb, const uint8_t* maskbits, void* out, int out_dtype,
                                bool round_to_g_dtype, hipStream_t stream);

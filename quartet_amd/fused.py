@@ -11,8 +11,9 @@ Both fall back to the unfused composition (same mathematics, more memory traffic
 production configuration, uses another Hadamard block than 32, or the tensors are not what the kernels take."""
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
-from . import _lib
+from . import _lib, kernels
 from .linear import QuantizedLinear, _cached_weight, _dense
 
 _KERNEL_DTYPES = (torch.float32, torch.bfloat16)
@@ -76,3 +77,17 @@ def swiglu_linear(layer, h12):
         return y
     up, gate = h12.split(h12.shape[-1] // 2, dim=-1)
     return layer(F.silu(up) * gate)
+
+
+def cross_entropy(logits, targets, ignore_index=-1):
+    """F.cross_entropy(logits, targets, ignore_index=ignore_index) of logits [rows, classes].  Where nothing asks for a
+    gradient and the result is an fp32 one (fp32 logits, or bf16 ones under autocast) the logits are read once by a kernel of
+    this package, which keeps log-probabilities in fp32 (the library rounds them to the logits' type)."""
+    plain = (type(logits) is torch.Tensor and logits.is_cuda and not (torch.is_grad_enabled() and logits.requires_grad)
+             and not (torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None
+                      or forward_ad._current_level >= 0))
+    if (plain and (logits.dtype == torch.float32 or (logits.dtype == torch.bfloat16 and torch.is_autocast_enabled("cuda")))
+            and logits.dim() == 2 and logits.shape[1] > 0 and targets.dim() == 1 and targets.dtype == torch.int64
+            and targets.device == logits.device and targets.shape[0] == logits.shape[0]):
+        return kernels.cross_entropy(logits.contiguous(), targets.contiguous(), ignore_index)
+    return F.cross_entropy(logits, targets, ignore_index=ignore_index)

@@ -477,3 +477,18 @@ def linear_backward(e2, packed_x, packed_w, T, I, O, hd_x, signs_x, hd_w, signs_
                                      _ptr(seed_base), _stream())
     _lib.check(rc, "qm_linear_backward")
     return gx, gw
+
+
+def cross_entropy(logits, targets, ignore_index):
+    """Mean cross-entropy of logits [rows, classes] against int64 targets [rows], fp32 scalar (no autograd)."""
+    _require_cuda(logits, targets)
+    assert logits.is_contiguous() and targets.is_contiguous() and targets.dtype == torch.int64
+    rows, classes = logits.shape
+    assert targets.shape == (rows,)
+    scratch = torch.empty(rows + 1, dtype=torch.float32, device=logits.device)
+    loss = scratch.new_empty(())
+    with torch.cuda.device(logits.device):
+        rc = _lib.lib().qm_cross_entropy(_ptr(logits), _dtype_code(logits.dtype), _ptr(targets), rows, classes, ignore_index, _ptr(scratch),
+                                         _ptr(loss), _stream())
+    _lib.check(rc, "qm_cross_entropy")
+    return loss

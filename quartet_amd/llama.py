@@ -9,7 +9,8 @@ linear is a ``QuantizedLinear`` built from registry names; init N(0, init_std) w
 ``init_std / sqrt(2 n_layer)``; cross-entropy over all positions.  The tokenizer the reference attaches
 (tiktoken) is not part of the numerics and is left out.
 
-Everything here except the block linears is stock PyTorch: this module is plumbing around the hot path."""
+Everything here except the block linears and an evaluation's loss is stock PyTorch: this module is plumbing around the hot
+path."""
 import contextlib
 import math
 from dataclasses import dataclass, field
@@ -20,7 +21,7 @@ import torch.nn.functional as F
 from torch.nn.attention import SDPBackend, sdpa_kernel
 
 from .backward import BACKWARD_SCHEMES
-from .fused import rmsnorm_linear, rope_qkv, swiglu_linear
+from .fused import cross_entropy, rmsnorm_linear, rope_qkv, swiglu_linear
 from .linear import QuantizedLinear
 from .quantizers import QUANTIZER_CLASSES
 
@@ -252,7 +253,7 @@ class Llama(nn.Module):
         x = self.transformer.ln_f(x)
         if targets is not None:
             logits = self.lm_head(x)
-            loss = F.cross_entropy(logits.view(-1, logits.size(-1)), targets.view(-1), ignore_index=-1)
+            loss = cross_entropy(logits.view(-1, logits.size(-1)), targets.view(-1), ignore_index=-1)
         else:
             logits = self.lm_head(x[:, [-1], :])
             loss = None

@@ -156,3 +156,37 @@ def test_operator_chain_compiles_fullgraph(ops):
     compiled = torch.compile(fwd, fullgraph=True, backend="aot_eager")
     assert torch.equal(compiled(x, w, h), eager)
     assert torch.equal(compiled(x, w, h), eager)
+
+
+@pytest.mark.parametrize("rows,classes,dtype", [(1, 1, torch.float32), (3, 7, torch.bfloat16), (5, 255, torch.float32), (33, 1025, torch.bfloat16),
+                                                (7, 8192, torch.bfloat16), (4, 8191, torch.float32), (1500, 32000, torch.bfloat16)])
+def test_cross_entropy_against_float64(rows, classes, dtype):
+    """Rows of odd lengths start off the 16-byte boundaries; shorter and longer than one round of requests; more rows than the
+    mean's lanes; ignored rows, -inf entries, a NaN.  A row's sum of exponentials adds classes / 256 + 13 terms in a lane, each
+    within (|x - max| + 2) 2^-23 of its value (|x - max| < 40 for the terms that count): its logarithm errs by at most 5e-6 (1 + classes / 8192), the
+    differences by 2^-23 of the logits (below 64)."""
+    from quartet_amd.fused import cross_entropy
+    g = torch.Generator().manual_seed(rows + classes)
+    logits = (4 * torch.randn(rows, classes, generator=g)).to(dtype)
+    if classes > 7:
+        logits[rows // 2, 1::3] = -float("inf")
+    targets = torch.randint(0, classes, (rows,), generator=g)
+    if classes > 7:
+        targets[rows // 2] = 0
+    if rows > 2:
+        targets[1] = -1
+    want = torch.nn.functional.cross_entropy(logits.double(), targets, ignore_index=-1)
+    x, t = logits.to("cuda:0"), targets.to("cuda:0")
+    with torch.no_grad(), torch.autocast("cuda", torch.bfloat16):
+        got = cross_entropy(x, t)
+        again = cross_entropy(x, t)
+        assert got.dtype == torch.float32 and torch.equal(got, again)
+        assert abs(float(got) - float(want)) < 1e-5 * (1 + classes / 8192) + 64 * 2 ** -23
+        assert torch.isnan(cross_entropy(x, torch.full_like(t, -1)))        # nothing left to average, as the library
+        x[0, classes // 2] = float("nan")
+        t[0] = classes - 1
+        assert torch.isnan(cross_entropy(x, t))
+    # what asks for a gradient, or for a bf16 loss, is the library's as before
+    x = logits.to("cuda:0").requires_grad_(True)
+    assert cross_entropy(x, t).grad_fn is not None
+    assert cross_entropy(x.detach(), t).dtype == dtype
