@@ -375,6 +375,9 @@ int qm_rope_split_qkv(const void* qkv, int qkv_dtype, int64_t rows, int64_t seq_
 int qm_rope_merge_qkv_grad(const void* dq, const void* dk, const void* dv, int grad_dtype, int64_t rows, int64_t seq_len,
                            int64_t n_embd, int head_dim, const float* table, void* d_qkv, int out_dtype, void* stream);
 
+/* Test aid: silu as the SwiGLU producer evaluates it for bf16 tensors, of every bf16 bit pattern: out[65536] */
+int qm_diag_silu_bf16(uint16_t* out, void* stream);
+
 /*
  * Mean cross-entropy of logits [rows, classes] (row-major, logits_dtype) against int64 targets [rows], over the rows whose
  * target is not ignore_index (F.cross_entropy of src/models/llama.py:254-256): fp32, *loss = mean(log(sum exp(row)) -

@@ -862,6 +862,11 @@ int qm_rope_merge_qkv_grad(const void* dq, const void* dk, const void* dv, int g
                     "qm_rope_merge_qkv_grad");
 }
 
+int qm_diag_silu_bf16(uint16_t* out, void* stream) {
+    if (!out) return fail(QM_ERR_INVALID, "qm_diag_silu_bf16: out must be non-null");
+    return from_hip(qm::silu_of_bf16_table(out, reinterpret_cast<hipStream_t>(stream)), "qm_diag_silu_bf16");
+}
+
 int qm_cross_entropy(const void* logits, int logits_dtype, const int64_t* targets, int64_t rows, int64_t classes,
                      int64_t ignore_index, float* row_losses, float* loss, void* stream) {
     if (!valid_dtype(logits_dtype)) return fail(QM_ERR_INVALID, "qm_cross_entropy: logits_dtype must be QM_BF16/QM_F32");

@@ -139,6 +139,8 @@ hipError_t rmsnorm_quantize_hd32(const void* x, int dtype, const void* add, int 
                                  float* factor, bool tiled, hipStream_t stream);
 hipError_t swiglu_quantize_hd32(const void* h12, int dtype, int64_t rows, int64_t hidden, uint32_t sign_word,
                                 uint8_t* codes, uint8_t* scales, uint8_t* maskbits, bool tiled, hipStream_t stream);
+// measurement and test aid: the SwiGLU producer's bf16 silu of all 65536 bit patterns
+hipError_t silu_of_bf16_table(uint16_t* out, hipStream_t stream);
 size_t rmsnorm_backward_workspace_bytes(int64_t rows, int64_t cols);
 hipError_t rmsnorm_backward(const void* gy, int gy_dtype, const void* x, int x_dtype, const float* gain,
                             const float* factor, int64_t rows, int64_t cols, const uint8_t* maskbits, uint32_t sign_word,

@@ -422,3 +422,16 @@ def test_block_with_deferred_residual_sums_matches_the_plain_block(q):
     assert torch.equal(l0, l1)
     for n in g0:
         assert torch.equal(g0[n], g1[n]), n
+
+
+def test_silu_of_every_bf16_value(oracle):
+    """The SwiGLU producer's shortened silu of bf16 tensors: the same bf16 value as the oracle's, for all 65536 inputs."""
+    import ctypes
+    from quartet_amd import _lib
+    out = torch.empty(65536, dtype=torch.int16, device=DEV)
+    _lib.check(_lib.lib().qm_diag_silu_bf16(ctypes.c_void_p(out.data_ptr()), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "qm_diag_silu_bf16")
+    x = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    want = torch.tensor([oracle.silu(float(t)) for t in x]).to(torch.bfloat16)
+    got = out.cpu().view(torch.bfloat16)
+    same = (got.view(torch.int16) == want.view(torch.int16)) | (got.isnan() & want.isnan())
+    assert same.all(), x[~same][:8]
