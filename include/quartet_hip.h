@@ -375,6 +375,16 @@ int qm_rope_split_qkv(const void* qkv, int qkv_dtype, int64_t rows, int64_t seq_
 int qm_rope_merge_qkv_grad(const void* dq, const void* dk, const void* dv, int grad_dtype, int64_t rows, int64_t seq_len,
                            int64_t n_embd, int head_dim, const float* table, void* d_qkv, int out_dtype, void* stream);
 
+/*
+ * The forward pass of a layer for a decoded batch in one launch: y [T, O] = Q(x) Q(W)^T, x [T, I] quantized inside (quest RTN,
+ * Hadamard block 32), packed_w as qm_linear_forward leaves it with QM_LAYOUT_PADDED.  The results are qm_linear_forward's, bit
+ * for bit; the packed x is not kept (no backward pass).  For T <= 16, I % 32 == 0, O % 8 == 0 and few enough groups of x per
+ * CU: qm_linear_decode_serves() tells (1 / 0), QM_ERR_INVALID otherwise.  x and y 16-byte aligned.
+ */
+int qm_linear_decode_serves(int64_t T, int64_t I, int64_t O);
+int qm_linear_decode(const void* x, int x_dtype, int64_t T, int64_t I, int64_t O, const uint32_t* signs_x, const void* packed_w,
+                     size_t packed_w_bytes, void* y, int y_dtype, void* stream);
+
 /* Test aid: silu as the SwiGLU producer evaluates it for bf16 tensors, of every bf16 bit pattern: out[65536] */
 int qm_diag_silu_bf16(uint16_t* out, void* stream);
 

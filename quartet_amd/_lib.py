@@ -47,6 +47,8 @@ EXPORTS = (
     "qm_swiglu_backward",
     "qm_rope_split_qkv",
     "qm_rope_merge_qkv_grad",
+    "qm_linear_decode_serves",
+    "qm_linear_decode",
     "qm_attention_causal",
     "qm_cross_entropy",
     "qm_diag_silu_bf16",
@@ -130,6 +132,10 @@ def lib():
     L.qm_diag_silu_bf16.argtypes = [vp, vp]
     L.qm_attention_causal.restype = i32
     L.qm_attention_causal.argtypes = [vp, vp, vp, vp, i64, i64, i64, i32, vp]
+    L.qm_linear_decode_serves.restype = i32
+    L.qm_linear_decode_serves.argtypes = [i64, i64, i64]
+    L.qm_linear_decode.restype = i32
+    L.qm_linear_decode.argtypes = [vp, i32, i64, i64, i64, vp, vp, ctypes.c_size_t, vp, i32, vp]
     L.qm_cross_entropy.restype = i32
     L.qm_cross_entropy.argtypes = [vp, i32, vp, i64, i64, i64, vp, vp, vp]
     L.qm_rope_merge_qkv_grad.restype = i32

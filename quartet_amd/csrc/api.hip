@@ -490,6 +490,23 @@ int qm_linear_forward(const void* x, int x_dtype, const void* w, int w_dtype, in
                     "qm_linear_forward");
 }
 
+int qm_linear_decode_serves(int64_t T, int64_t I, int64_t O) { return qm::linear_decode_serves(T, I, O) ? 1 : 0; }
+
+int qm_linear_decode(const void* x, int x_dtype, int64_t T, int64_t I, int64_t O, const uint32_t* signs_x, const void* packed_w,
+                     size_t packed_w_bytes, void* y, int y_dtype, void* stream) {
+    if (!valid_dtype(x_dtype) || !valid_dtype(y_dtype)) return fail(QM_ERR_INVALID, "qm_linear_decode: dtypes must be QM_BF16/QM_F32");
+    if (!qm::linear_decode_serves(T, I, O))
+        return fail(QM_ERR_INVALID, "qm_linear_decode: [%lld, %lld] x [%lld] is not served (see qm_linear_decode_serves)", (long long)T, (long long)I, (long long)O);
+    const PackedLayout lw = packed_layout(O, I);
+    if (!x || !aligned(x, 16) || !y || !aligned(y, 16)) return fail(QM_ERR_INVALID, "qm_linear_decode: x and y must be non-null and 16-byte aligned");
+    if (!packed_w || packed_w_bytes < lw.total || !aligned(packed_w, 256))
+        return fail(QM_ERR_INVALID, "qm_linear_decode: the packed weight needs %zu bytes, 256-byte aligned", lw.total);
+    const uint8_t* pw = static_cast<const uint8_t*>(packed_w);
+    return from_hip(qm::linear_decode(x, x_dtype, T, I, O, signs_x ? signs_x[0] : 0u, pw + lw.c, pw + lw.s, y, y_dtype,
+                                      reinterpret_cast<hipStream_t>(stream)),
+                    "qm_linear_decode");
+}
+
 size_t qm_linear_backward_error_workspace_bytes(int64_t T, int64_t I, int64_t O) {
     if (T < 0 || I < 0 || O < 0 || I % 32 || O % 32 || T % 32) return 0;
     return error_layout(T, I, O).total;

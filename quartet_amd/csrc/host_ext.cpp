@@ -305,6 +305,24 @@ Tensor linear_forward(const LayerPtr& l, const Tensor& x, const Tensor& weight, 
     shape.back() = l->O;
     return y.view(shape);
 }
+// A decoded batch against a weight that is already packed: one launch, undefined where that kernel does not serve
+Tensor linear_decode(const Layer& l, const Tensor& x, const Tensor& weight, const Tensor& packed_w) {
+    const int64_t I = weight.size(1), O = weight.size(0);
+    if (x.numel() == 0 || x.numel() > 16 * I || l.a_hd != 32 || l.x_dense.defined() || l.w_dense.defined() || x.size(-1) != I) return {};
+    const int64_t T = x.numel() / I;
+    if (!qm_linear_decode_serves(T, I, O)) return {};
+    require_cuda(x, weight);
+    const Tensor x2 = rows_of(x, I);
+    if (reinterpret_cast<uintptr_t>(x2.data_ptr()) % 16) return {};
+    auto shape = x.sizes().vec();
+    shape.back() = O;
+    const at::ScalarType out_dtype = autocast_bf16() ? at::kBFloat16 : x.scalar_type();
+    Tensor y = at::empty(shape, weight.options().dtype(out_dtype));
+    check(qm_linear_decode(x2.data_ptr(), dtype_code(x2.scalar_type()), T, I, O, l.a_signs.data(), packed_w.data_ptr(), (size_t)packed_w.numel(),
+                           y.data_ptr(), dtype_code(out_dtype), stream_of(x2)),
+          "qm_linear_decode");
+    return y;
+}
 struct LinearFn : Function<LinearFn> {
     static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight, const LayerPtr& l, Tensor* packed_w) {
         Tensor packed_x;
@@ -336,7 +354,10 @@ py::tuple linear(const Tensor& x, const Tensor& weight, int a_hd, py::handle a_s
         l->error_only = error_only;
         Tensor packed_w = or_none(packed_weight), packed_x;
         const c10::OptionalDeviceGuard guard(weight.is_cuda() ? std::optional<at::Device>(weight.device()) : std::nullopt);
-        const Tensor y = wants_grad({&x, &weight}) ? LinearFn::apply(x, weight, l, &packed_w) : linear_forward(l, x, weight, packed_x, packed_w);
+        Tensor y;
+        if (wants_grad({&x, &weight})) y = LinearFn::apply(x, weight, l, &packed_w);
+        else if (packed_w.defined()) y = linear_decode(*l, x, weight, packed_w);
+        if (!y.defined()) y = linear_forward(l, x, weight, packed_x, packed_w);
         return py::make_tuple(y, packed_w);
     });
 }

@@ -202,6 +202,12 @@ hipError_t gemm_tile(int kind, const TileProduct& g, const TileProduct* second, 
 bool gemm_rows_serves(const TileProduct& p);
 hipError_t gemm_rows(const TileProduct& p, int c_dtype, hipStream_t stream);
 
+// The forward pass of a layer for a decoded batch in one launch (gemm_rows.hip): quest RTN of x under Hadamard blocks of 32, times
+// the packed weight (padded tiled codes); x 16-byte, y 8-byte aligned
+bool linear_decode_serves(int64_t T, int64_t I, int64_t O);
+hipError_t linear_decode(const void* x, int x_dtype, int64_t T, int64_t I, int64_t O, uint32_t sign_word, const uint8_t* w_codes,
+                         const uint8_t* w_scales, void* y, int y_dtype, hipStream_t stream);
+
 // The kernel a product runs on (gemm.hip).  Products with p.mask set ask for the masked inverse rotation; `rotates` tells
 // whether that kernel applies it (p.c then holds rot_out_dtype elements: c_dtype, or F32 holding the bf16-rounded result)
 // or the caller has to (p.c then holds the plain product in c_dtype).

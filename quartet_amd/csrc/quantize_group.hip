@@ -33,246 +33,11 @@
 #include "qm_jobs.h"
 #include "qm_kernels.h"
 #include "qm_math.h"
+#include "quantize_group.h"
 
 namespace qm {
 
 namespace {
-
-typedef float v2f __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ void butterfly32(float (&v)[32]) {
-#pragma unroll
-    for (int h = 1; h < 32; h <<= 1) {
-#pragma unroll
-        for (int i = 0; i < 32; ++i) {
-            if (i & h) continue;
-            const float a = v[i], b = v[i + h];
-            v[i] = a + b;
-            v[i + h] = a - b;
-        }
-    }
-}
-
-// pairwise tree: adjacent pairs, then pairs of pairs, ... (the canonical order of the group sums)
-__device__ __forceinline__ float tree_sum32(const float (&p)[32]) {
-    float t[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) t[i] = p[2 * i] + p[2 * i + 1];
-#pragma unroll
-    for (int n = 8; n >= 1; n >>= 1)
-#pragma unroll
-        for (int i = 0; i < n; ++i) t[i] = t[2 * i] + t[2 * i + 1];
-    return t[0];
-}
-
-struct GroupCodes {
-    uint32_t w[4];        // 32 nibbles, element i in bits [4(i%8), +4) of word i/8
-    uint32_t scale_byte;  // E8M0
-    uint32_t keep;        // bit i = |t_i| < 6
-    float deq_scale;      // what a code value is multiplied by in the de-quantized tensor
-};
-
-#define kNegTiny (u2f(0x80000001u))  // -2^-149
-
-// v_cvt_scalef32_sr_pk_fp4_f32 replaces byte SEL of its destination and keeps the other three, but the
-// compiler builtin of this toolchain does not tie the destination to its `old` operand (the untouched bytes
-// come back as whatever the allocated register held), so the instruction is issued directly.
-template <int SEL>
-__device__ __forceinline__ void sr_convert_pair(uint32_t& dst, v2f pair, uint32_t rnd, float scale) {
-    if constexpr (SEL == 0) asm("v_cvt_scalef32_sr_pk_fp4_f32 %0, %1, %2, %3" : "+v"(dst) : "v"(pair), "v"(rnd), "v"(scale));
-    else if constexpr (SEL == 1) asm("v_cvt_scalef32_sr_pk_fp4_f32 %0, %1, %2, %3 op_sel:[0,0,1,0]" : "+v"(dst) : "v"(pair), "v"(rnd), "v"(scale));
-    else if constexpr (SEL == 2) asm("v_cvt_scalef32_sr_pk_fp4_f32 %0, %1, %2, %3 op_sel:[0,0,0,1]" : "+v"(dst) : "v"(pair), "v"(rnd), "v"(scale));
-    else asm("v_cvt_scalef32_sr_pk_fp4_f32 %0, %1, %2, %3 op_sel:[0,0,1,1]" : "+v"(dst) : "v"(pair), "v"(rnd), "v"(scale));
-}
-
-// ties-toward-zero via the round-to-nearest-even convert (see the file comment)
-__device__ __forceinline__ float tie_nudge(float v) {
-    return u2f(__builtin_elementwise_sub_sat(f2u(v), 1u) | 1u);
-}
-
-template <int MODE, bool WANT_MASK>
-__device__ __forceinline__ void quantize_group_regs(const float (&g)[32], uint64_t seed, int64_t group_index,
-                                                    GroupCodes& o) {
-    constexpr bool kQuest = (MODE == QUEST_RTN || MODE == QUEST_SR);
-    constexpr bool kSR = (MODE == ABSMAX_SR || MODE == QUEST_SR);
-    float hw_scale;   // power of two the convert divides by
-    uint32_t thr_bits;  // bit pattern of 6 * scale: |g| < thr  <=>  |t| < 6
-    float t[32];
-    bool all_zero = false;
-    if constexpr (kQuest) {
-        float sq[32];
-#pragma unroll
-        for (int i = 0; i < 32; ++i) sq[i] = g[i] * g[i];
-        const float ms = tree_sum32(sq) * 0.03125f;
-        const float m = tree_sum32(g) * 0.03125f;
-        const float mm = m * m;
-        float var = ms - mm;
-        var = var > 0.0f ? var : 0.0f;
-        const float sd = __builtin_sqrtf(var);
-        const float gs = kQuestG * sd;
-        const float s = gs + 1e-8f;
-        int E = (int)((f2u(s) >> 23) & 0xffu) - 127;
-        E = E > 127 ? 127 : E;
-        o.scale_byte = (uint32_t)(E + 127);
-        hw_scale = pow2i(E);
-        o.deq_scale = hw_scale;
-        thr_bits = f2u(6.0f * hw_scale);
-#pragma unroll
-        for (int i = 0; i < 32; ++i) t[i] = g[i];
-    } else {
-        float a = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 32; ++i) a = fmaxf(a, fabsf(g[i]));
-        all_zero = (a == 0.0f);
-        int k = (int)((f2u(a) >> 23) & 0xffu) - 129;
-        k = k < -127 ? -127 : (k > 127 ? 127 : k);
-        o.scale_byte = (uint32_t)(k + 127);
-        hw_scale = pow2i(k);
-        o.deq_scale = scale_pow2(kFourThirds, k);
-        // |t| < 6 with t = RN(g 2^-k / d): evaluated on the quotient h = RN(g / d) against 6 * 2^k
-        thr_bits = f2u(6.0f * hw_scale);
-        // t = RN(RN(g 2^-k) / d) by definition.  For a group whose maximum is at least 2^-60 this is RN(g / d) scaled by
-        // 2^-k inside the convert: the two-operation quotient is exact for |g| >= 2^-100, and a smaller element lies
-        // below 2^-38 of the scale, so its code is a zero whose sign is the element's own whatever the quotient's last
-        // bit.  A group with a smaller non-zero maximum (where g / d would lose bits to underflow) follows the
-        // definition literally, with a true division, and hands the convert an already scaled value.
-        if (__builtin_expect(a < 0x1p-60f && !all_zero, 0)) {
-#pragma unroll
-            for (int i = 0; i < 32; ++i) t[i] = scale_pow2(g[i], -k) / kFourThirds;
-            hw_scale = 1.0f;
-            thr_bits = f2u(6.0f);
-        } else {
-#pragma unroll
-            for (int i = 0; i < 32; ++i) t[i] = div_four_thirds_fast(g[i]);
-        }
-    }
-    o.keep = 0u;
-    if constexpr (WANT_MASK) {
-        // clip mask, most significant element first so that element 0 lands in bit 0
-        // one compare into the carry flag and one add-with-carry (keep = 2 keep + flag) per element, sixteen
-        // elements per statement (the operand limit of an asm statement)
-        uint32_t keep = 0u;
-        const float thr = u2f(thr_bits);
-#define QM_KEEP_BIT(N) "v_cmp_lt_f32_e64 vcc, |%" #N "|, %17\n\tv_addc_co_u32_e32 %0, vcc, %0, %0, vcc\n\t"
-#define QM_KEEP_16(B)                                                                                               \
-    asm(QM_KEEP_BIT(16) QM_KEEP_BIT(15) QM_KEEP_BIT(14) QM_KEEP_BIT(13) QM_KEEP_BIT(12) QM_KEEP_BIT(11) QM_KEEP_BIT(10) \
-        QM_KEEP_BIT(9) QM_KEEP_BIT(8) QM_KEEP_BIT(7) QM_KEEP_BIT(6) QM_KEEP_BIT(5) QM_KEEP_BIT(4) QM_KEEP_BIT(3)        \
-        QM_KEEP_BIT(2) QM_KEEP_BIT(1)                                                                                   \
-        : "+v"(keep)                                                                                                    \
-        : "v"(t[(B)]), "v"(t[(B) + 1]), "v"(t[(B) + 2]), "v"(t[(B) + 3]), "v"(t[(B) + 4]), "v"(t[(B) + 5]),             \
-          "v"(t[(B) + 6]), "v"(t[(B) + 7]), "v"(t[(B) + 8]), "v"(t[(B) + 9]), "v"(t[(B) + 10]), "v"(t[(B) + 11]),       \
-          "v"(t[(B) + 12]), "v"(t[(B) + 13]), "v"(t[(B) + 14]), "v"(t[(B) + 15]), "v"(thr)                              \
-        : "vcc")
-        QM_KEEP_16(16);
-        QM_KEEP_16(0);
-#undef QM_KEEP_16
-#undef QM_KEEP_BIT
-        o.keep = all_zero ? 0u : keep;
-    }
-
-    // the converts' byte selector must be a literal, hence the macros
-#define QM_RTN_PAIR(B)                                                                                   \
-    w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, tie_nudge(t[wi * 8 + 2 * (B)] + kNegTiny),           \
-                                                 tie_nudge(t[wi * 8 + 2 * (B) + 1] + kNegTiny), hw_scale, (B));
-    // element j of a Philox call (16 elements): its random field is the top 22 bits of word j/4 rotated left by
-    // 8 * (j%4).  The convert reads the field of a pair's first element from bits 31..10 of its random operand and that of
-    // the second from bits 30..9, so the even element's operand is the word rotated by 0 or 16 bits and the odd element's
-    // the word rotated by 7 or 23 (one more bit to the right): one v_alignbit_b32 each, none for a word's first element.
-#define QM_SR_PAIR(B, J0)                                                                                 \
-    {                                                                                                     \
-        const uint32_t pw = ph.w[(J0) >> 2];                                                              \
-        const uint32_t r_even = ((J0) & 3) == 0 ? pw : __builtin_amdgcn_alignbit(pw, pw, 16);             \
-        const uint32_t r_odd = __builtin_amdgcn_alignbit(pw, pw, ((J0) & 3) == 0 ? 25 : 9);               \
-        const v2f pr = {t[wi * 8 + 2 * (B)] + kNegTiny, t[wi * 8 + 2 * (B) + 1] + kNegTiny};              \
-        sr_convert_pair<(B)>(even, pr, r_even, hw_scale);                                                 \
-        sr_convert_pair<(B)>(odd, pr, r_odd, hw_scale);                                                   \
-    }
-    if constexpr (!kSR) {
-#pragma unroll
-        for (int wi = 0; wi < 4; ++wi) {
-            uint32_t w = 0u;
-            QM_RTN_PAIR(0) QM_RTN_PAIR(1) QM_RTN_PAIR(2) QM_RTN_PAIR(3)
-            o.w[wi] = w;
-        }
-    } else {
-        Philox4 ph;
-#pragma unroll
-        for (int wi = 0; wi < 4; ++wi) {
-            // words 0,1 of the call serve the even octet of the pair, words 2,3 the odd one
-            if ((wi & 1) == 0) ph = philox_for_hexadecad(seed, (uint64_t)(group_index * 2 + (wi >> 1)));
-            uint32_t even = 0u, odd = 0u;  // converts driven by the even / odd element's random byte
-            if ((wi & 1) == 0) { QM_SR_PAIR(0, 0) QM_SR_PAIR(1, 2) QM_SR_PAIR(2, 4) QM_SR_PAIR(3, 6) }
-            else { QM_SR_PAIR(0, 8) QM_SR_PAIR(1, 10) QM_SR_PAIR(2, 12) QM_SR_PAIR(3, 14) }
-            o.w[wi] = (even & 0x0f0f0f0fu) | (odd & 0xf0f0f0f0u);
-        }
-    }
-#undef QM_RTN_PAIR
-#undef QM_SR_PAIR
-}
-
-template <typename T>
-__device__ __forceinline__ void load_group(const T* __restrict__ p, float (&v)[32]) {
-    if constexpr (sizeof(T) == 2) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const uint4 raw = reinterpret_cast<const uint4*>(p)[q];
-            const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                v[q * 8 + 2 * i] = u2f(w[i] << 16);
-                v[q * 8 + 2 * i + 1] = u2f(w[i] & 0xffff0000u);
-            }
-        }
-    } else {
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const float4 f = reinterpret_cast<const float4*>(p)[q];
-            v[q * 4] = f.x; v[q * 4 + 1] = f.y; v[q * 4 + 2] = f.z; v[q * 4 + 3] = f.w;
-        }
-    }
-}
-
-template <typename T>
-__device__ __forceinline__ void store_dequant(T* __restrict__ p, const GroupCodes& o) {
-    float v[32];
-#pragma unroll
-    for (int i = 0; i < 32; ++i) {
-        const uint32_t nib = (o.w[i >> 3] >> (4 * (i & 7))) & 15u;
-        const float q = e2m1_value((int)(nib & 7u));
-        v[i] = ((nib & 8u) ? -q : q) * o.deq_scale;
-    }
-    if constexpr (sizeof(T) == 2) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            uint32_t w[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                w[i] = (uint32_t)f32_to_bf16(v[q * 8 + 2 * i]) | ((uint32_t)f32_to_bf16(v[q * 8 + 2 * i + 1]) << 16);
-            reinterpret_cast<uint4*>(p)[q] = make_uint4(w[0], w[1], w[2], w[3]);
-        }
-    } else {
-#pragma unroll
-        for (int q = 0; q < 8; ++q)
-            reinterpret_cast<float4*>(p)[q] = make_float4(v[q * 4], v[q * 4 + 1], v[q * 4 + 2], v[q * 4 + 3]);
-    }
-}
-
-struct GroupOut {
-    uint4* codes;        // [n_groups]
-    uint8_t* scales;     // [n_groups]
-    uint32_t* maskbits;  // [n_groups] or null
-    void* dequant;       // [n_groups * 32] of T or null
-};
-
-// x @ H for one chunk of 32: butterfly, then hd^-1/2 with the column sign folded in (wave-uniform)
-__device__ __forceinline__ void rotate_group(float (&v)[32], float c, uint32_t sign_word, bool rotate = true) {
-    if (rotate) butterfly32(v);  // uniform; without it (c = 1, no signs) the group passes through unchanged
-#pragma unroll
-    for (int j = 0; j < 32; ++j) {
-        const float cj = u2f(f2u(c) ^ (((sign_word >> j) & 1u) << 31));  // wave-uniform: stays in scalar registers
-        v[j] = v[j] * cj;
-    }
-}
 
 // ---- dense 32x32 rotation (rerotate="O32", quantizers/mxfp4.py:61-64 of the reference) on the matrix pipe ----------
 // The reference applies the matrix with tl.dot inside its kernel (mxfp4_triton.py:44-45).  Here each lane owns one

@@ -80,6 +80,37 @@ def test_product_of_few_rows(oracle, T, I, O):
     assert rel(y16.float().cpu().numpy(), want) < 2 ** -8
 
 
+@pytest.mark.parametrize("T,I,O,one_launch", [(1, 32, 8, True), (3, 96, 24, True), (8, 4096, 4096, True), (16, 2048, 520, True), (16, 2080, 520, False), (1, 8160, 264, True),
+                                              (2, 16384, 40, True), (1, 1312, 11008, True), (9, 4096, 4096, False), (17, 64, 64, False)])
+def test_decode_in_one_launch_is_the_same_layer(T, I, O, one_launch):
+    """A few tokens against a packed weight that is kept: quantizer and product in one launch give what the two launches give, bit
+    for bit, at the bounds of that kernel (tokens, groups per CU, padded columns, four and eight waves), for both types of x and y
+    and with column signs."""
+    print(f"case decode T={T} I={I} O={O}", flush=True)
+    import quartet_amd as q
+    from quartet_amd import _lib
+    assert bool(_lib.lib().qm_linear_decode_serves(T, I, O)) == one_launch
+    x = make_input(T, I, torch.bfloat16, seed=1, outlier_frac=0.01).to("cuda:0")
+    w = make_input(O, I, torch.bfloat16, seed=2, outlier_frac=0, scale=0.02)
+    layer = q.QuantizedLinear(I, O, bias=False, weight_quantizer=q.QuestMXFP4Quantizer(), activation_quantizer=q.QuestMXFP4Quantizer(),
+                              gradient_quantizer=q.AlbertTsengQuantizer(), backward_scheme=q.BACKWARD_SCHEMES["Q(E)Q(Wt)t_Q(Et)Q(Xt)t"]())
+    layer = layer.to("cuda:0", torch.bfloat16)
+    with torch.no_grad():
+        layer.weight.copy_(w.to("cuda:0"))
+    for signs in (0, 0x9e3779b9):
+        layer.activation_quantizer.sign_bits = layer.weight_quantizer.sign_bits = signs
+        for xt, amp in ((x, False), (x.float(), False), (x.float(), True)):
+            with torch.no_grad(), torch.autocast("cuda", torch.bfloat16, enabled=amp):
+                q.enable_packed_weight_cache(layer, False)
+                want = layer(xt)
+                q.enable_packed_weight_cache(layer)
+                layer(xt)                       # fills the cache
+                got = layer(xt)
+                assert layer.packed_weight_cache.hits == 1
+                assert got.dtype == want.dtype and got.shape == want.shape and torch.equal(got, want)
+                assert torch.equal(layer(xt[None, :, :])[0], want)
+
+
 @pytest.mark.parametrize("T,I,O,hd", [(32, 32, 32, 32), (4128, 96, 160, 32), (4160, 192, 128, 64), (4224, 128, 256, 128), (96, 160, 96, 32), (288, 192, 320, 32), (544, 1728, 352, 32), (1056, 640, 1088, 32),
                                       (64, 64, 64, 64), (192, 320, 128, 64), (128, 128, 128, 128), (384, 256, 640, 128), (1280, 384, 896, 128)])
 def test_layer_on_padded_operands(oracle, T, I, O, hd):
