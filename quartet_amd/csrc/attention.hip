@@ -2,7 +2,7 @@
 //
 // What bounds it: at 8 x 512 tokens and 5 heads of 128 latency (1.3 GFLOP of unmasked products, 21 MB), at long sequences the
 // matrix pipe and the exponentials.  The library's kernel took 34 us there plus a fill of 4.4 us, this one takes 20 (a chain of
-// eight steps, 1.6 us each); 16 x 2048 x 12 x 128: 620 -> 331 us, 8 x 2048 x 16 x 64: 202 -> 110.
+eight steps, 1.6 us each); 16 x 2048 x 12 x 128: 620 -> 331 us, 8 x 2048 x 16 x 64: 202 -> 110.
 //
 // A workgroup of four waves owns 64 * QB queries of one head, a wave 16 * QB of them; the keys and values of 64 positions at
 // a time go through LDS, the next 64 on their way into registers meanwhile.  Both products have the queries as the
