@@ -1,8 +1,7 @@
 // Causal attention of bf16 heads, forward only: what an evaluated model runs between its attention projections.
 //
 // What bounds it: at 8 x 512 tokens and 5 heads of 128 latency (1.3 GFLOP of unmasked products, 21 MB), at long sequences the
-// matrix pipe and the exponentials.  The library's kernel took 34 us there plus a fill of 4.4 us, this one takes 20 (a chain of
-eight steps, 1.6 us each); 16 x 2048 x 12 x 128: 620 -> 331 us, 8 x 2048 x 16 x 64: 202 -> 110.
+// matrix pipe and the exponentials.  The library's kernel took 34 us there plus a fill of 4.4 us.
 //
 // A workgroup of four waves owns 64 * QB queries of one head, a wave 16 * QB of them; the keys and values of 64 positions at
 // a time go through LDS, the next 64 on their way into registers meanwhile.  Both products have the queries as the
@@ -25,7 +24,6 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 typedef float v2f __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
-typedef uint32_t u4v __attribute__((ext_vector_type(4)));   // arrays of the class uint4 end up in scratch memory
 
 constexpr int kKeys = 64;   // positions per step
 
@@ -43,7 +41,7 @@ __device__ __forceinline__ float across_quarters(float v, F&& f) {
 
 // q, k, v, out: [batch, S, heads, D] contiguous
 template <int D, int QB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void attention_causal_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
+__global__ __launch_bounds__(256) void attention_causal_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
                                                                const uint16_t* __restrict__ v, uint16_t* __restrict__ out, int S, int heads,
                                                                int all_heads, int heads_per_xcd, int q_blocks, float scale_log2e) {
     constexpr int kRows = 64 * QB;                       // queries of the workgroup
@@ -67,26 +65,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
     const int64_t base = (int64_t)(head / heads) * S * pitch + (int64_t)(head % heads) * D;
     const int w0 = q0 + wave * 16 * QB;                  // the wave's first query
 
-    u4v qf[QB][D / 32];
+    uint4 qf[QB][D / 32];
 #pragma unroll
     for (int b = 0; b < QB; ++b) {
         const int row = w0 + b * 16 + col < S ? w0 + b * 16 + col : S - 1;   // a query past the end repeats the last one and is not stored
 #pragma unroll
-        for (int c = 0; c < D / 32; ++c) qf[b][c] = *reinterpret_cast<const u4v*>(q + base + row * pitch + c * 32 + g * 8);
+        for (int c = 0; c < D / 32; ++c) qf[b][c] = *reinterpret_cast<const uint4*>(q + base + row * pitch + c * 32 + g * 8);
     }
-    u4v kr[kKLoads], vr[4];
+    uint4 kr[kKLoads], vr[4];
     const int kg = tid & 15, oct = tid >> 4;             // this lane's unit of V
     const auto request = [&](int k0) {
 #pragma unroll
         for (int j = 0; j < kKLoads; ++j) {
             const int piece = tid + 256 * j, key = k0 + piece / kPieces;
-            kr[j] = *reinterpret_cast<const u4v*>(k + base + (key < S ? key : S - 1) * pitch + piece % kPieces * 8);
+            kr[j] = *reinterpret_cast<const uint4*>(k + base + (key < S ? key : S - 1) * pitch + piece % kPieces * 8);
         }
         if (kVUnits == 256 || tid < kVUnits) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int key = k0 + kg * 4 + i;
-                vr[i] = *reinterpret_cast<const u4v*>(v + base + (key < S ? key : S - 1) * pitch + oct * 8);
+                vr[i] = *reinterpret_cast<const uint4*>(v + base + (key < S ? key : S - 1) * pitch + oct * 8);
             }
         }
     };
@@ -94,14 +92,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
 #pragma unroll
         for (int j = 0; j < kKLoads; ++j) {
             const int piece = tid + 256 * j;
-            *reinterpret_cast<u4v*>(lds_k + piece / kPieces * kKPitch + piece % kPieces * 16) = kr[j];
+            *reinterpret_cast<uint4*>(lds_k + piece / kPieces * kKPitch + piece % kPieces * 16) = kr[j];
         }
         if (kVUnits == 256 || tid < kVUnits) {
+            const uint32_t r[4][4] = {{vr[0].x, vr[0].y, vr[0].z, vr[0].w}, {vr[1].x, vr[1].y, vr[1].z, vr[1].w},
+                                      {vr[2].x, vr[2].y, vr[2].z, vr[2].w}, {vr[3].x, vr[3].y, vr[3].z, vr[3].w}};
 #pragma unroll
             for (int i = 0; i < 4; ++i) {   // d = 8 oct + 2 i and the one after it
                 uint8_t* dst = lds_v + (oct * 8 + 2 * i) * kVPitch + kg * 8;
-                *reinterpret_cast<uint2*>(dst) = make_uint2((vr[0][i] & 0xffffu) | (vr[1][i] << 16), (vr[2][i] & 0xffffu) | (vr[3][i] << 16));
-                *reinterpret_cast<uint2*>(dst + kVPitch) = make_uint2((vr[0][i] >> 16) | (vr[1][i] & 0xffff0000u), (vr[2][i] >> 16) | (vr[3][i] & 0xffff0000u));
+                *reinterpret_cast<uint2*>(dst) = make_uint2((r[0][i] & 0xffffu) | (r[1][i] << 16), (r[2][i] & 0xffffu) | (r[3][i] << 16));
+                *reinterpret_cast<uint2*>(dst + kVPitch) = make_uint2((r[0][i] >> 16) | (r[1][i] & 0xffff0000u), (r[2][i] >> 16) | (r[3][i] & 0xffff0000u));
             }
         }
     };
@@ -130,7 +130,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
             for (int b = 0; b < QB; ++b) s[b][t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int c = 0; c < D / 32; ++c) {
-                const v8bf kf = __builtin_bit_cast(v8bf, *reinterpret_cast<const u4v*>(lds_k + (t * 16 + col) * kKPitch + c * 64 + g * 16));
+                const v8bf kf = __builtin_bit_cast(v8bf, *reinterpret_cast<const uint4*>(lds_k + (t * 16 + col) * kKPitch + c * 64 + g * 16));
 #pragma unroll
                 for (int b = 0; b < QB; ++b)
                     s[b][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, __builtin_bit_cast(v8bf, qf[b][c]), s[b][t], 0, 0, 0);
@@ -139,15 +139,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
         v8bf p[QB][kKeys / 32];
 #pragma unroll
         for (int b = 0; b < QB; ++b) {
-            // a key past the end (read as the last one) lies behind every query that is stored
-            const int reach = w0 + b * 16 + col - k0 - 4 * g;
+            const int query = w0 + b * 16 + col;
             float m = top[b];
 #pragma unroll
             for (int t = 0; t < kKeys / 16; ++t)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const float z = s[b][t][e] * scale_log2e;
-                    s[b][t][e] = t * 16 + e <= reach ? z : -INFINITY;
+                    // a key past the end (read as the last one) lies behind every query that is stored
+                    s[b][t][e] = k0 + t * 16 + 4 * g + e <= query ? z : -INFINITY;
                     m = fmaxf(m, s[b][t][e]);
                 }
             m = across_quarters(m, [](float a, float c) { return fmaxf(a, c); });
@@ -169,10 +169,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
             sum[b] = sum[b] * shrink + part;
 #pragma unroll
             for (int u = 0; u < kKeys / 32; ++u) p[b][u] = as_v8bf(w[2 * u][0], w[2 * u][1], w[2 * u + 1][0], w[2 * u + 1][1]);
-            if (__any(shrink != 1.0f)) {   // later steps seldom raise a maximum
 #pragma unroll
-                for (int d = 0; d < D / 16; ++d) o[b][d] *= shrink;
-            }
+            for (int d = 0; d < D / 16; ++d) o[b][d] *= shrink;
         }
         // contraction slots of a lane: keys 32 u + 4 g .. + 3, then 32 u + 16 + 4 g .. + 3
 #pragma unroll
@@ -219,7 +217,6 @@ bool attention_causal_serves(int64_t batch, int64_t S, int64_t heads, int head_d
 hipError_t attention_causal(const void* q, const void* k, const void* v, void* out, int64_t batch, int64_t S, int64_t heads, int head_dim,
                             hipStream_t stream) {
     if (!attention_causal_serves(batch, S, heads, head_dim)) return hipErrorInvalidValue;
-    // 128 queries per workgroup halve the LDS reads per product; 64 while that would leave CUs idle or with one workgroup each
     const bool wide = batch * heads * ((S + 127) / 128) >= 512;
     if (head_dim == 128) {
         if (wide) launch_attention<128, 2>(q, k, v, out, batch, S, heads, stream);
