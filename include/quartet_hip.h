@@ -389,14 +389,6 @@ int qm_linear_decode(const void* x, int x_dtype, int64_t T, int64_t I, int64_t O
 int qm_diag_silu_bf16(uint16_t* out, void* stream);
 
 /*
- * Causal attention, forward only (F.scaled_dot_product_attention(..., is_causal=True) of src/models/llama.py:146-149):
- * q, k, v, out bf16 [batch, seq_len, heads, head_dim], contiguous, 16-byte aligned, head_dim 64 or 128, softmax scale
- * head_dim^-1/2.  out must not overlap the inputs.
- */
-int qm_attention_causal(const void* q, const void* k, const void* v, void* out, int64_t batch, int64_t seq_len, int64_t heads,
-                        int head_dim, void* stream);
-
-/*
  * Mean cross-entropy of logits [rows, classes] (row-major, logits_dtype) against int64 targets [rows], over the rows whose
  * target is not ignore_index (F.cross_entropy of src/models/llama.py:254-256): fp32, *loss = mean(log(sum exp(row)) -
  * row[target]).  No row left: NaN.  A target that is no class makes the loss NaN.

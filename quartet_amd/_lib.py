@@ -49,7 +49,6 @@ EXPORTS = (
     "qm_rope_merge_qkv_grad",
     "qm_linear_decode_serves",
     "qm_linear_decode",
-    "qm_attention_causal",
     "qm_cross_entropy",
     "qm_diag_silu_bf16",
 )
@@ -130,8 +129,6 @@ def lib():
     L.qm_rope_split_qkv.argtypes = [vp, i32, i64, i64, i64, i32, vp, vp, vp, vp, i32, vp]
     L.qm_diag_silu_bf16.restype = i32
     L.qm_diag_silu_bf16.argtypes = [vp, vp]
-    L.qm_attention_causal.restype = i32
-    L.qm_attention_causal.argtypes = [vp, vp, vp, vp, i64, i64, i64, i32, vp]
     L.qm_linear_decode_serves.restype = i32
     L.qm_linear_decode_serves.argtypes = [i64, i64, i64]
     L.qm_linear_decode.restype = i32

@@ -884,18 +884,6 @@ int qm_diag_silu_bf16(uint16_t* out, void* stream) {
     return from_hip(qm::silu_of_bf16_table(out, reinterpret_cast<hipStream_t>(stream)), "qm_diag_silu_bf16");
 }
 
-int qm_attention_causal(const void* q, const void* k, const void* v, void* out, int64_t batch, int64_t seq_len, int64_t heads, int head_dim,
-                        void* stream) {
-    if (batch < 0 || seq_len < 0 || heads < 0) return fail(QM_ERR_INVALID, "qm_attention_causal: negative extent");
-    if (head_dim != 64 && head_dim != 128) return fail(QM_ERR_INVALID, "qm_attention_causal: head_dim must be 64 or 128 (got %d)", head_dim);
-    if (batch == 0 || seq_len == 0 || heads == 0) return 0;
-    if (!qm::attention_causal_serves(batch, seq_len, heads, head_dim)) return fail(QM_ERR_INVALID, "qm_attention_causal: extents too large");
-    if (!q || !k || !v || !out) return fail(QM_ERR_INVALID, "qm_attention_causal: q, k, v and out must be non-null");
-    if (!aligned(q, 16) || !aligned(k, 16) || !aligned(v, 16) || !aligned(out, 16))
-        return fail(QM_ERR_UNALIGNED, "qm_attention_causal: tensors need 16-byte alignment");
-    return from_hip(qm::attention_causal(q, k, v, out, batch, seq_len, heads, head_dim, reinterpret_cast<hipStream_t>(stream)), "qm_attention_causal");
-}
-
 int qm_cross_entropy(const void* logits, int logits_dtype, const int64_t* targets, int64_t rows, int64_t classes,
                      int64_t ignore_index, float* row_losses, float* loss, void* stream) {
     if (!valid_dtype(logits_dtype)) return fail(QM_ERR_INVALID, "qm_cross_entropy: logits_dtype must be QM_BF16/QM_F32");

@@ -237,10 +237,6 @@ hipError_t gemm_tile_phases(const uint8_t* a_codes, const uint8_t* a_scales, con
 int mfma_only_blocks();
 hipError_t mfma_only(const uint8_t* operands, float* sink, int iters, hipStream_t stream);
 
-// causal attention of bf16 q, k, v [batch, S, heads, head_dim] contiguous into out, likewise (attention.hip); head_dim 64 or 128
-bool attention_causal_serves(int64_t batch, int64_t S, int64_t heads, int head_dim);
-hipError_t attention_causal(const void* q, const void* k, const void* v, void* out, int64_t batch, int64_t S, int64_t heads, int head_dim,
-                            hipStream_t stream);
 // mean cross-entropy over the rows whose target is not `ignore` (loss.hip); losses: scratch, one float per row
 hipError_t cross_entropy_mean(const void* logits, int dtype, const int64_t* targets, int64_t rows, int64_t classes, int64_t ignore,
                               float* losses, float* loss, hipStream_t stream);

@@ -79,27 +79,14 @@ def swiglu_linear(layer, h12):
     return layer(F.silu(up) * gate)
 
 
-def _plain(*tensors):
-    """Ordinary GPU tensors of which nothing asks for a gradient, and no tracer, transform or forward-mode level at work."""
-    return (all(type(t) is torch.Tensor and t.is_cuda and not (torch.is_grad_enabled() and t.requires_grad) for t in tensors)
-            and not (torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None
-                     or forward_ad._current_level >= 0))
-
-
-def causal_attention(q, k, v):
-    """Causal attention of q, k, v [batch, seq_len, heads, head_dim] (the layout rope_qkv returns), or None where the kernel of
-    this package does not serve it: bf16, head_dim 64 or 128, no gradient asked for."""
-    if (_plain(q, k, v) and q.dtype == k.dtype == v.dtype == torch.bfloat16 and q.shape == k.shape == v.shape and q.dim() == 4
-            and q.shape[-1] in (64, 128) and q.numel() > 0 and all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (q, k, v))):
-        return kernels.attention_causal(q, k, v)
-    return None
-
-
 def cross_entropy(logits, targets, ignore_index=-1):
     """F.cross_entropy(logits, targets, ignore_index=ignore_index) of logits [rows, classes].  Where nothing asks for a
     gradient and the result is an fp32 one (fp32 logits, or bf16 ones under autocast) the logits are read once by a kernel of
     this package, which keeps log-probabilities in fp32 (the library rounds them to the logits' type)."""
-    if (_plain(logits) and (logits.dtype == torch.float32 or (logits.dtype == torch.bfloat16 and torch.is_autocast_enabled("cuda")))
+    plain = (type(logits) is torch.Tensor and logits.is_cuda and not (torch.is_grad_enabled() and logits.requires_grad)
+             and not (torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None
+                      or forward_ad._current_level >= 0))
+    if (plain and (logits.dtype == torch.float32 or (logits.dtype == torch.bfloat16 and torch.is_autocast_enabled("cuda")))
             and logits.dim() == 2 and logits.shape[1] > 0 and targets.dim() == 1 and targets.dtype == torch.int64
             and targets.device == logits.device and targets.shape[0] == logits.shape[0]):
         return kernels.cross_entropy(logits.contiguous(), targets.contiguous(), ignore_index)

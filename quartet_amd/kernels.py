@@ -479,19 +479,6 @@ def linear_backward(e2, packed_x, packed_w, T, I, O, hd_x, signs_x, hd_w, signs_
     return gx, gw
 
 
-def attention_causal(q, k, v):
-    """Causal attention of bf16 q, k, v [batch, seq_len, heads, head_dim] (contiguous, head_dim 64 or 128), same shape out (no
-    autograd)."""
-    _require_cuda(q, k, v)
-    assert q.shape == k.shape == v.shape and q.dtype == k.dtype == v.dtype == torch.bfloat16
-    assert q.is_contiguous() and k.is_contiguous() and v.is_contiguous()
-    out = torch.empty_like(q)
-    with torch.cuda.device(q.device):
-        rc = _lib.lib().qm_attention_causal(_ptr(q), _ptr(k), _ptr(v), _ptr(out), *q.shape, _stream())
-    _lib.check(rc, "qm_attention_causal")
-    return out
-
-
 def cross_entropy(logits, targets, ignore_index):
     """Mean cross-entropy of logits [rows, classes] against int64 targets [rows], fp32 scalar (no autograd)."""
     _require_cuda(logits, targets)

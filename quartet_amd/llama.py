@@ -9,7 +9,7 @@ linear is a ``QuantizedLinear`` built from registry names; init N(0, init_std) w
 ``init_std / sqrt(2 n_layer)``; cross-entropy over all positions.  The tokenizer the reference attaches
 (tiktoken) is not part of the numerics and is left out.
 
-Everything here except the block linears and an evaluation's attention and loss is stock PyTorch: this module is plumbing around the hot
+Everything here except the block linears and an evaluation's loss is stock PyTorch: this module is plumbing around the hot
 path."""
 import contextlib
 import math
@@ -21,7 +21,7 @@ import torch.nn.functional as F
 from torch.nn.attention import SDPBackend, sdpa_kernel
 
 from .backward import BACKWARD_SCHEMES
-from .fused import causal_attention, cross_entropy, rmsnorm_linear, rope_qkv, swiglu_linear
+from .fused import cross_entropy, rmsnorm_linear, rope_qkv, swiglu_linear
 from .linear import QuantizedLinear
 from .quantizers import QUANTIZER_CLASSES
 
@@ -50,9 +50,8 @@ class LlamaConfig:
     # not in the reference: RMSNorm and the SwiGLU product are computed inside the activation quantizer of the linear
     # they feed (quartet_amd.fused) instead of being written out; False runs the reference's op-by-op composition
     fuse_producers: bool = True
-    # not in the reference (which leaves the choice to torch's dispatcher): what serves the causal attention.  "auto": where no
-    # gradient is asked for, this package's kernel (bf16 heads of 64 or 128); else of the library's, on a GPU, the
-    # memory-efficient kernels first, then flash, then math --
+    # not in the reference (which leaves the choice to torch's dispatcher): which library kernel serves
+    # F.scaled_dot_product_attention.  "auto": on a GPU, the memory-efficient kernels first, then flash, then math --
     # on MI355X with this PyTorch the memory-efficient pair runs a causal 16 x 12 x 2048 x 128 bf16 layer, forward and
     # backward, in 2.1 ms against the 3.7 ms of the flash pair the dispatcher picks; "default": the dispatcher's order
     sdpa_backend: str = "auto"
@@ -172,18 +171,14 @@ class LlamaAttention(nn.Module):
             q, k, v = qkv.split(self.n_embd, dim=2)
             q, k = apply_rotary(q.view(B, T, self.n_head, hs), k.view(B, T, self.n_head, hs), table)
             v = v.view(B, T, self.n_head, hs)
-        # evaluation: this package's kernel; a training step, dropout, other types and head widths: the library's
-        y = causal_attention(q, k, v) if self.sdpa_backend == "auto" and self.dropout == 0.0 else None
-        if y is None:
-            y = self._library_attention(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2)).transpose(1, 2)
-        out = self.resid_dropout(self.c_proj(y.reshape(B, T, C)))
-        return out if norm is None else (out, x)   # with the fused norm: also x for the residual sum
-
-    def _library_attention(self, q, k, v):
+        q, k, v = q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2)
         if not torch.is_autocast_enabled() and v.dtype != q.dtype:
             v = v.to(q.dtype)
         with _sdpa_choice(self.sdpa_backend, q):
-            return F.scaled_dot_product_attention(q, k, v, attn_mask=None, dropout_p=self.dropout, is_causal=True)
+            y = F.scaled_dot_product_attention(q, k, v, attn_mask=None, dropout_p=self.dropout, is_causal=True)
+        y = y.transpose(1, 2).contiguous().view(B, T, C)
+        out = self.resid_dropout(self.c_proj(y))
+        return out if norm is None else (out, x)   # with the fused norm: also x for the residual sum
 
 
 class LlamaBlock(nn.Module):
