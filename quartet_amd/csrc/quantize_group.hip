@@ -785,7 +785,8 @@ struct RmsNormProducer {
     static constexpr int kOutDtype = F32;  // bf16-or-fp32 normalised value times the fp32 gain is fp32
     static constexpr bool kAdd = !std::is_void<TA>::value;
     using TAdd = typename std::conditional<kAdd, TA, T>::type;
-    static constexpr int kLds = kAdd ? 4 * 512 * 16 : 0;
+    static constexpr bool kStaged = sizeof(T) == 4;
+    static constexpr int kLds = kStaged ? 4 * 512 * 16 : 0;
     const T* x;
     const float* gain;
     float* factor;  // [rows]: 1 / sqrt(mean(x^2) + eps), kept for the backward pass
@@ -793,9 +794,26 @@ struct RmsNormProducer {
     const TAdd* add;
     T* xsum;
 
-    // 8 KiB of LDS per wave of the workgroup: staging of the residual sum on its way out
-    __device__ __forceinline__ static float4* xsum_area() {
-        return reinterpret_cast<float4*>(job_lds) + (threadIdx.x >> 6) * 512;
+    // 8 KiB of LDS per wave, through which fp32 rows and the gain pass on their way to the lanes that own their groups: an
+    // instruction then reads or writes whole 128-byte lines, where a lane's own 128 bytes are eight 16-byte pieces, each
+    // instruction touching 64 lines, which the address unit takes one by one.  Slot 8 l + (q ^ l % 8) holds piece q of lane l's
+    // group: slot-ordered and group-ordered accesses both spread over all banks.  With the residual sum: 4096 x 640 11.2 ->
+    // 9.3 us, 16384 x 1536 53 -> 48, 32768 x 1024 88 -> 70, 16384 x 4096 163 -> 153 (two passes); 512 x 4096 is latency, 11 us
+    // either way.  Requests under per-lane predicates instead of clamped ones: 16384 x 1536 75 us.
+    typedef float v4 __attribute__((ext_vector_type(4)));
+    __device__ __forceinline__ static v4* area() { return reinterpret_cast<v4*>(job_lds) + (threadIdx.x >> 6) * 512; }
+    __device__ __forceinline__ static void settle() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    __device__ __forceinline__ static void read_group(int of_lane, float (&v)[32]) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const v4 t = area()[8 * of_lane + (q ^ (of_lane & 7))];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[4 * q + e] = t[e];
+        }
     }
 
     // The row's factor; `first` leaves with the raw elements of the lane's first group (if it has one).
@@ -804,36 +822,57 @@ struct RmsNormProducer {
     // A lane without a group adds +0, which leaves a sum of squares unchanged.
     // W < 64: the wave holds 64 / W rows of at most W groups each, a row in the W lanes from `seg` on (`lane` counts
     // from there); the partial sums then have W / 16 terms instead of four, the missing ones being the +0 of above.
+    // wave_row: the wave's first row, of `rows`.
     template <int W = 64>
-    __device__ __forceinline__ float prepare(int64_t row, int lane, int groups, int64_t cols, float (&first)[32], int seg = 0) const {
+    __device__ __forceinline__ float prepare(int64_t row, int64_t wave_row, int64_t rows, int lane, int groups, int64_t cols, float (&first)[32],
+                                             int seg) const {
+        // slot 64 i + wlane is piece `piece` of the group of lane 8 i + wlane / 8: group `sub` + 8 i of the row that 8 i / W picks (uniform).
+        // Slots past the row's end are filled from its last group: no branch between the requests.
+        const int wlane = seg + lane, sub = wlane >> 3, piece = (wlane & 7) ^ sub;
+        v4 gains[W / 8];
+        if constexpr (kStaged) {
+#pragma unroll
+            for (int i = 0; i < W / 8; ++i) {
+                const int gg = 8 * i + sub < groups ? 8 * i + sub : groups - 1;
+                gains[i] = *reinterpret_cast<const v4*>(gain + gg * 32 + piece * 4);
+            }
+        }
         float acc = 0.0f;
         for (int base = 0; base < groups; base += 64) {
             const int g = base + lane;
             float s = 0.0f;
+            if constexpr (kStaged) {
+                v4 raw[8];
+                const auto group_of = [&](int i) { return base + 8 * i % W + sub; };
+                const auto row_of = [&](int i) { const int64_t r = wave_row + 8 * i / W; return (r < rows ? r : rows - 1) * cols; };
+                const auto at = [&](int i) { const int gg = group_of(i); return (gg < groups ? gg : groups - 1) * 32 + piece * 4; };
+#pragma unroll
+                for (int i = 0; i < 8; ++i) raw[i] = *reinterpret_cast<const v4*>(x + row_of(i) + at(i));
+                if constexpr (kAdd) {
+                    if constexpr (sizeof(TAdd) == 2) {
+                        typedef uint32_t w2 __attribute__((ext_vector_type(2)));
+                        w2 more[8];
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) more[i] = *reinterpret_cast<const w2*>(add + row_of(i) + at(i));
+#pragma unroll
+                        for (int i = 0; i < 8; ++i)
+                            raw[i] = raw[i] + v4{u2f(more[i][0] << 16), u2f(more[i][0] & 0xffff0000u), u2f(more[i][1] << 16), u2f(more[i][1] & 0xffff0000u)};
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) raw[i] = raw[i] + *reinterpret_cast<const v4*>(add + row_of(i) + at(i));
+                    }
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+                        if (group_of(i) < groups) *reinterpret_cast<v4*>(xsum + row_of(i) + at(i)) = raw[i];
+                }
+#pragma unroll
+                for (int i = 0; i < 8; ++i) area()[64 * i + wlane] = raw[i];
+                settle();
+            }
             if (g < groups) {
                 float v[32];
-                load_group<T>(x + row * cols + g * 32, v);
-                if constexpr (kAdd) {
-                    static_assert(!kAdd || sizeof(T) == 4, "the residual sum is formed in fp32");
-                    float a[32];
-                    load_group<TAdd>(add + row * cols + g * 32, a);
-#pragma unroll
-                    for (int i = 0; i < 32; ++i) v[i] = v[i] + a[i];
-                    if constexpr (W == 64) {
-                        // the sum leaves through LDS so that an instruction stores whole 128-byte lines (a lane's own
-                        // 128 bytes would go out as eight 16-byte pieces of 64 different lines per instruction); slot
-                        // 8 l + (q ^ l % 8) of the wave's area holds piece q of lane l's group: writes and the
-                        // slot-ordered reads both spread over all banks
-                        float4* area = xsum_area();
-#pragma unroll
-                        for (int q = 0; q < 8; ++q)
-                            area[8 * lane + (q ^ (lane & 7))] = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
-                    } else {
-                        float4* dst = reinterpret_cast<float4*>(xsum + row * cols + g * 32);
-#pragma unroll
-                        for (int q = 0; q < 8; ++q) dst[q] = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
-                    }
-                }
+                if constexpr (kStaged) read_group(wlane, v);
+                else load_group<T>(x + row * cols + g * 32, v);
                 if (base == 0) {
 #pragma unroll
                     for (int i = 0; i < 32; ++i) first[i] = v[i];
@@ -842,19 +881,7 @@ struct RmsNormProducer {
                 for (int i = 0; i < 32; ++i) v[i] = v[i] * v[i];
                 s = tree_sum32(v);
             }
-            if constexpr (kAdd && W == 64) {
-                const float4* area = xsum_area();
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const int slot = 64 * i + lane, gl = slot >> 3, piece = (slot & 7) ^ (gl & 7);
-                    if (base + gl < groups)
-                        reinterpret_cast<float4*>(xsum + row * cols + (int64_t)(base + gl) * 32)[piece] = area[slot];
-                }
-                __builtin_amdgcn_wave_barrier();  // the next pass over the row reuses the area
-            }
+            if constexpr (kStaged) settle();   // the next pass over the row, or the gain, reuses the area
 #pragma unroll
             for (int k = 0; k < W / 16; ++k) acc = acc + __shfl(s, seg + (lane & 15) + 16 * k, 64);
         }
@@ -862,11 +889,17 @@ struct RmsNormProducer {
         for (int m = 1; m < 16; m <<= 1) acc = acc + __shfl_xor(acc, m, 64);
         const float f = 1.0f / __builtin_sqrtf(acc / (float)cols + eps);
         if (lane == 0) factor[row] = f;
+        if constexpr (kStaged) {   // the gain of the lanes' first groups, for load()
+#pragma unroll
+            for (int i = 0; i < W / 8; ++i)
+                area()[64 * i + wlane] = gains[i];
+            settle();
+        }
         return f;
     }
     // v holds the group's raw elements on entry when have_raw
     __device__ __forceinline__ void load(int64_t row, int g, int64_t cols, float f, bool have_raw, float (&v)[32]) const {
-        // with a residual sum: the lane reads back what it stored in prepare()
+        // with a residual sum: what the wave stored in prepare()
         if (!have_raw) load_group<T>((kAdd ? xsum : x) + row * cols + g * 32, v);
 #pragma unroll
         for (int i = 0; i < 32; ++i) v[i] = v[i] * f;
@@ -875,7 +908,8 @@ struct RmsNormProducer {
             for (int i = 0; i < 32; i += 2) round_pair_to_bf16(v[i], v[i + 1]);
         }
         float w[32];
-        load_group<float>(gain + g * 32, w);
+        if (kStaged && have_raw) read_group(g, w);
+        else load_group<float>(gain + g * 32, w);
 #pragma unroll
         for (int i = 0; i < 32; ++i) v[i] = v[i] * w[i];
     }
@@ -902,7 +936,7 @@ struct SwiGluProducer {
     const T* h12;  // [rows, 2 cols]: up, then gate
 
     template <int W = 64>
-    __device__ __forceinline__ float prepare(int64_t, int, int, int64_t, float (&)[32], int = 0) const { return 0.0f; }
+    __device__ __forceinline__ float prepare(int64_t, int64_t, int64_t, int, int, int64_t, float (&)[32], int) const { return 0.0f; }
     __device__ __forceinline__ void load(int64_t row, int g, int64_t cols, float, bool, float (&v)[32]) const {
         float gate[32];
         load_group<T>(h12 + row * 2 * cols + g * 32, v);
@@ -942,12 +976,13 @@ struct ProducedRowsJob {
     __device__ __forceinline__ void run(unsigned bid) const {
         const int wlane = threadIdx.x & 63, wave = threadIdx.x >> 6;
         const int lane = wlane & (W - 1), seg = wlane - lane;  // place in the row's segment of the wave
-        int64_t row = ((int64_t)bid * 4 + wave) * (64 / W) + seg / W;
-        if (row - seg / W >= rows) return;  // a whole wave
+        const int64_t wave_row = ((int64_t)bid * 4 + __builtin_amdgcn_readfirstlane(wave)) * (64 / W);
+        int64_t row = wave_row + seg / W;
+        if (wave_row >= rows) return;  // a whole wave
         if (row >= rows) row = rows - 1;    // a segment past the end repeats the last row: same values to the same places
         const int groups = (int)(cols / 32);
         float v[32];
-        const float state = prod.template prepare<W>(row, lane, groups, cols, v, seg);
+        const float state = prod.template prepare<W>(row, wave_row, rows, lane, groups, cols, v, seg);
         // TILED: the row's groups padded to a multiple of four with zero codes and scales; the padding lanes of the last quad
         // are inactive in the loop, so that the scale gather reads zeros from them
         const int groups_p = TILED ? (groups + 3) & ~3 : groups;
