@@ -778,6 +778,13 @@ __device__ __forceinline__ void round_pair_to_bf16(float& a, float& b) {
     b = u2f(w & 0xffff0000u);
 }
 
+// what the lanes of a wave wrote to LDS before is read by its other lanes behind
+__device__ __forceinline__ void wave_settle() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // TA = void: plain.  Otherwise the norm's input is x + add (the residual sum in front of the norm, src/models/llama.py:
 // 170-171), formed here in T's arithmetic and written to xsum, which the rest of the model continues with.
 template <typename T, typename TA = void>
@@ -802,11 +809,6 @@ struct RmsNormProducer {
     // either way.  Requests under per-lane predicates instead of clamped ones: 16384 x 1536 75 us.
     typedef float v4 __attribute__((ext_vector_type(4)));
     __device__ __forceinline__ static v4* area() { return reinterpret_cast<v4*>(job_lds) + (threadIdx.x >> 6) * 512; }
-    __device__ __forceinline__ static void settle() {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
     __device__ __forceinline__ static void read_group(int of_lane, float (&v)[32]) {
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
@@ -867,7 +869,7 @@ struct RmsNormProducer {
                 }
 #pragma unroll
                 for (int i = 0; i < 8; ++i) area()[64 * i + wlane] = raw[i];
-                settle();
+                wave_settle();
             }
             if (g < groups) {
                 float v[32];
@@ -881,7 +883,7 @@ struct RmsNormProducer {
                 for (int i = 0; i < 32; ++i) v[i] = v[i] * v[i];
                 s = tree_sum32(v);
             }
-            if constexpr (kStaged) settle();   // the next pass over the row, or the gain, reuses the area
+            if constexpr (kStaged) wave_settle();   // the next pass over the row, or the gain, reuses the area
 #pragma unroll
             for (int k = 0; k < W / 16; ++k) acc = acc + __shfl(s, seg + (lane & 15) + 16 * k, 64);
         }
@@ -893,10 +895,12 @@ struct RmsNormProducer {
 #pragma unroll
             for (int i = 0; i < W / 8; ++i)
                 area()[64 * i + wlane] = gains[i];
-            settle();
+            wave_settle();
         }
         return f;
     }
+    template <int W>
+    __device__ __forceinline__ void stage(int64_t, int64_t, int, int, int64_t, int) const {}
     // v holds the group's raw elements on entry when have_raw
     __device__ __forceinline__ void load(int64_t row, int g, int64_t cols, float f, bool have_raw, float (&v)[32]) const {
         // with a residual sum: what the wave stored in prepare()
@@ -919,7 +923,7 @@ struct RmsNormProducer {
 // inputs round to the same bf16 value as silu_fixed (tests/test_gpu_fused.py goes through all of them).  A quarter of
 // the denominator keeps its reciprocal a normal number up to 2^128; the last bit on top of it settles the one input
 // (5.9375) whose result lies 2^-24 from a tie.  silu_fixed is some 35 instructions, a polynomial and an IEEE division, and
-// made the producer 92 us at 16384 x 4096 where its bytes take 61; with these six it is 76 (4096 x 1728: 15.2 -> 10.6).
+// made the producer 92 us at 16384 x 4096 where its bytes take 61; with these six it was 76 (4096 x 1728: 15.2 -> 10.6).
 __device__ __forceinline__ float silu_of_bf16(float x) {
     const float e = __builtin_amdgcn_exp2f(x * -1.44269504088896340736f);
     return (x * 0.25f) * __builtin_amdgcn_rcpf(__builtin_fmaf(e, 0.25f, 0x1.000002p-2f));
@@ -932,15 +936,61 @@ __global__ void silu_of_bf16_kernel(uint16_t* __restrict__ out) {
 template <typename T>
 struct SwiGluProducer {
     static constexpr int kOutDtype = sizeof(T) == 2 ? BF16 : F32;
-    static constexpr int kLds = 0;
+    // bf16: whole lines through 8 KiB of LDS per wave, as in the RMSNorm producer; a group is four pieces here, slot
+    // 4 l + (q ^ l / 4 % 4) holds piece q of lane l's group.  16384 x 4096 73 -> 65 us, 32768 x 4096
+    // 141 -> 120; 16384 x 1536 35 either way, up to 4096 x 1728 (11 us) latency
+    static constexpr bool kStaged = sizeof(T) == 2;
+    static constexpr int kLds = kStaged ? 4 * 512 * 16 : 0;
     const T* h12;  // [rows, 2 cols]: up, then gate
 
+    typedef uint32_t v4 __attribute__((ext_vector_type(4)));
+    __device__ __forceinline__ static v4* area() { return reinterpret_cast<v4*>(job_lds) + (threadIdx.x >> 6) * 512; }
     template <int W = 64>
     __device__ __forceinline__ float prepare(int64_t, int64_t, int64_t, int, int, int64_t, float (&)[32], int) const { return 0.0f; }
+    // every lane of the wave: the groups base + lane of its rows
+    template <int W>
+    __device__ __forceinline__ void stage(int64_t wave_row, int64_t rows, int base, int groups, int64_t cols, int wlane) const {
+        if constexpr (kStaged) {
+            const int sub = wlane >> 2, piece = (wlane & 3) ^ ((wlane >> 4) & 3);
+            v4 up[4], gate[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int64_t r = wave_row + 16 * i / W;
+                const int g = base + 16 * i % W + sub;
+                const T* at = h12 + (r < rows ? r : rows - 1) * 2 * cols + (g < groups ? g : groups - 1) * 32 + piece * 8;
+                up[i] = *reinterpret_cast<const v4*>(at);
+                gate[i] = *reinterpret_cast<const v4*>(at + cols);
+            }
+            wave_settle();   // the lanes have read the groups before
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                area()[64 * i + wlane] = up[i];
+                area()[256 + 64 * i + wlane] = gate[i];
+            }
+            wave_settle();
+        }
+    }
+    __device__ __forceinline__ static void read_group(int half, float (&v)[32]) {
+        const int wlane = threadIdx.x & 63;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const v4 t = area()[256 * half + 4 * wlane + (q ^ ((wlane >> 2) & 3))];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[8 * q + 2 * e] = u2f(t[e] << 16);
+                v[8 * q + 2 * e + 1] = u2f(t[e] & 0xffff0000u);
+            }
+        }
+    }
     __device__ __forceinline__ void load(int64_t row, int g, int64_t cols, float, bool, float (&v)[32]) const {
         float gate[32];
-        load_group<T>(h12 + row * 2 * cols + g * 32, v);
-        load_group<T>(h12 + row * 2 * cols + cols + g * 32, gate);
+        if constexpr (kStaged) {
+            read_group(0, v);
+            read_group(1, gate);
+        } else {
+            load_group<T>(h12 + row * 2 * cols + g * 32, v);
+            load_group<T>(h12 + row * 2 * cols + cols + g * 32, gate);
+        }
 #pragma unroll
         for (int i = 0; i < 32; ++i) v[i] = sizeof(T) == 2 ? silu_of_bf16(v[i]) : silu_fixed(v[i]);
         if constexpr (sizeof(T) == 2) {  // a bf16 tensor rounds after each op
@@ -987,7 +1037,10 @@ struct ProducedRowsJob {
         // are inactive in the loop, so that the scale gather reads zeros from them
         const int groups_p = TILED ? (groups + 3) & ~3 : groups;
         const auto tile_slot = [&](int g) { return (row >> 4) * 16 * groups_p + ((g >> 2) * 64 + (int)(row & 15) * 4 + (g & 3)); };
-        for (int g = lane; g < groups; g += W) {
+        for (int base = 0; base < groups; base += W) {
+            const int g = base + lane;
+            prod.template stage<W>(wave_row, rows, base, groups, cols, wlane);
+            if (g >= groups) continue;
             const int64_t gi = row * groups + g;
             const int64_t ci = TILED ? tile_slot(g) : gi;
             prod.load(row, g, cols, state, g == lane, v);
