@@ -15,6 +15,7 @@ from torch.autograd import forward_ad
 
 from . import _lib, kernels
 from .linear import QuantizedLinear, _cached_weight, _dense
+from .one_node import one_node
 
 _KERNEL_DTYPES = (torch.float32, torch.bfloat16)
 
@@ -25,13 +26,38 @@ def _layer_is_fusable(layer, x):
             and layer.weight.dtype in _KERNEL_DTYPES)
 
 
+@one_node
+def _rope(qkv, table, n_head):
+    return _lib.host().rope_qkv(qkv, table, n_head)
+
+
+@one_node
+def _norm_linear(x, add, gain, weight, eps, a_q, w_q, g_q, cache, pass_input):
+    key, packed_w = _cached_weight(x, weight, a_q, w_q, g_q, cache)
+    y, x_next, packed_w = _lib.host().norm_linear(x, add, gain, weight, eps, a_q.sign_bits, w_q.hadamard_dim, w_q.sign_bits, g_q.hadamard_dim, g_q,
+                                                  packed_w, _dense(w_q, weight), pass_input)
+    if key is not None:
+        cache.put(key, packed_w)
+    return (y, x_next) if (pass_input or add is not None) else y
+
+
+@one_node
+def _swiglu_linear(h12, weight, a_q, w_q, g_q, cache):
+    key, packed_w = _cached_weight(h12, weight, a_q, w_q, g_q, cache)
+    y, packed_w = _lib.host().swiglu_linear(h12, weight, a_q.sign_bits, w_q.hadamard_dim, w_q.sign_bits, g_q.hadamard_dim, g_q, packed_w,
+                                            _dense(w_q, weight))
+    if key is not None:
+        cache.put(key, packed_w)
+    return y
+
+
 def rope_qkv(qkv, table, n_head):
     """Split the fused attention projection [B, T, 3C] into q, k, v [B, T, n_head, head_dim] with q and k rotated by the
     (cos, sin) table [T, head_dim/2, 2]."""
     C = qkv.shape[-1] // 3
     hs = C // n_head
     if qkv.is_cuda and qkv.dtype in _KERNEL_DTYPES and hs % 8 == 0 and table.dtype == torch.float32:
-        return _lib.host().rope_qkv(qkv, table.contiguous(), n_head)
+        return _rope(qkv, table.contiguous(), n_head)
     from .llama import apply_rotary
     B, T, _ = qkv.shape
     q, k, v = qkv.split(C, dim=2)
@@ -50,14 +76,8 @@ def rmsnorm_linear(norm, layer, x, pass_input=False, add=None):
         x, add = x + add, None
         pass_input = True
     if fusable:
-        weight, a_q, w_q, g_q = layer.weight, layer.activation_quantizer, layer.weight_quantizer, layer.backward_scheme.g_quantizer
-        cache = layer.packed_weight_cache
-        key, packed_w = _cached_weight(x, weight, a_q, w_q, g_q, cache)
-        y, x_next, packed_w = _lib.host().norm_linear(x, add, norm.weight, weight, norm.eps, a_q.sign_bits, w_q.hadamard_dim, w_q.sign_bits,
-                                                      g_q.hadamard_dim, g_q, packed_w, _dense(w_q, weight), pass_input)
-        if key is not None:
-            cache.put(key, packed_w)
-        return (y, x_next) if (pass_input or add is not None) else y
+        return _norm_linear(x, add, norm.weight, layer.weight, norm.eps, layer.activation_quantizer, layer.weight_quantizer,
+                            layer.backward_scheme.g_quantizer, layer.packed_weight_cache, pass_input)
     if add is not None:
         x = x + add
     y = layer(norm(x))
@@ -67,14 +87,8 @@ def rmsnorm_linear(norm, layer, x, pass_input=False, add=None):
 def swiglu_linear(layer, h12):
     """layer(silu(up) * gate) with (up, gate) the two halves of h12's last dimension."""
     if _layer_is_fusable(layer, h12) and h12.is_cuda and h12.dtype in _KERNEL_DTYPES:
-        weight, a_q, w_q, g_q = layer.weight, layer.activation_quantizer, layer.weight_quantizer, layer.backward_scheme.g_quantizer
-        cache = layer.packed_weight_cache
-        key, packed_w = _cached_weight(h12, weight, a_q, w_q, g_q, cache)
-        y, packed_w = _lib.host().swiglu_linear(h12, weight, a_q.sign_bits, w_q.hadamard_dim, w_q.sign_bits, g_q.hadamard_dim, g_q, packed_w,
-                                                _dense(w_q, weight))
-        if key is not None:
-            cache.put(key, packed_w)
-        return y
+        return _swiglu_linear(h12, layer.weight, layer.activation_quantizer, layer.weight_quantizer, layer.backward_scheme.g_quantizer,
+                              layer.packed_weight_cache)
     up, gate = h12.split(h12.shape[-1] // 2, dim=-1)
     return layer(F.silu(up) * gate)
 

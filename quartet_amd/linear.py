@@ -14,6 +14,7 @@ import torch.nn as nn
 from . import _lib
 from .backward import BACKWARD_SCHEMES, EW_EtX_Scheme, QEQWtt_QEtQXtt_Scheme, QEW_QEtX_Scheme  # noqa: F401
 from .quantizers import QUANTIZER_CLASSES, AlbertTsengQuantizer, NoQuantizer, QuestMXFP4Quantizer  # noqa: F401
+from .one_node import one_node
 from .quantizers.mxfp4 import _autocast_bf16, _fresh_seed
 
 
@@ -90,6 +91,7 @@ class QuartetLinearFn:
     The autograd function itself is native (csrc/host_ext.cpp)."""
 
     @staticmethod
+    @one_node
     def apply(x, weight, a_q, w_q, g_q, weight_cache, error_only=False):
         key, packed_w = _cached_weight(x, weight, a_q, w_q, g_q, weight_cache)
         y, packed_w = _lib.host().linear(x, weight, a_q.hadamard_dim, a_q.sign_bits, w_q.hadamard_dim, w_q.sign_bits, g_q.hadamard_dim, g_q,

@@ -16,6 +16,7 @@ import torch
 
 from .. import _lib
 from .. import kernels as K
+from ..one_node import one_node
 from .base import BaseQuantizer
 
 
@@ -227,9 +228,15 @@ class QuestMXFP4Quantizer(_HadamardQuantizer):
         if self.is_dense:
             return DenseRotationQuantizerFn.apply(x, self.hadamard_matrix, K.QM_QUEST_RTN, True, 1.0)
         # quest-scaled RTN forward with clip mask, masked straight-through backward (mxfp4.py:127-146)
-        return _lib.host().quantizer(x, self.hadamard_dim, self.sign_bits, K.QM_QUEST_RTN, 0, 1.0)
+        return _quest_quantize(x, self.hadamard_dim, self.sign_bits)
 
 
+@one_node
+def _quest_quantize(x, hadamard_dim, sign_bits):
+    return _lib.host().quantizer(x, hadamard_dim, sign_bits, K.QM_QUEST_RTN, 0, 1.0)
+
+
+@one_node
 def _absmax_quantize(x, hadamard_dim, sign_bits, stochastic, post_scale):
     """mxfp4.py:15-34: absmax/(3/4)-scaled RTN or SR forward, unmasked straight-through backward."""
     mode, seed = (K.QM_ABSMAX_SR, _fresh_seed()) if stochastic else (K.QM_ABSMAX_RTN, 0)
