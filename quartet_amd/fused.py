@@ -11,11 +11,10 @@ Both fall back to the unfused composition (same mathematics, more memory traffic
 production configuration, uses another Hadamard block than 32, or the tensors are not what the kernels take."""
 import torch
 import torch.nn.functional as F
-from torch.autograd import forward_ad
 
 from . import _lib, kernels
 from .linear import QuantizedLinear, _cached_weight, _dense
-from .one_node import one_node
+from .one_node import one_node, transformed
 
 _KERNEL_DTYPES = (torch.float32, torch.bfloat16)
 
@@ -98,8 +97,7 @@ def cross_entropy(logits, targets, ignore_index=-1):
     gradient and the result is an fp32 one (fp32 logits, or bf16 ones under autocast) the logits are read once by a kernel of
     this package, which keeps log-probabilities in fp32 (the library rounds them to the logits' type)."""
     plain = (type(logits) is torch.Tensor and logits.is_cuda and not (torch.is_grad_enabled() and logits.requires_grad)
-             and not (torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None
-                      or forward_ad._current_level >= 0))
+             and not (transformed() or torch.compiler.is_compiling()))
     if (plain and (logits.dtype == torch.float32 or (logits.dtype == torch.bfloat16 and torch.is_autocast_enabled("cuda")))
             and logits.dim() == 2 and logits.shape[1] > 0 and targets.dim() == 1 and targets.dtype == torch.int64
             and targets.device == logits.device and targets.shape[0] == logits.shape[0]):

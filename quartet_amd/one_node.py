@@ -4,15 +4,19 @@ The layers' autograd functions are native (csrc/host_ext.cpp): what they allocat
 they launch does not.  ``torch.jit.trace`` would therefore record the allocations and leave the launches out, and a replay
 would return memory nobody wrote.  Under a trace a call goes through a Python autograd function instead, which the
 trace keeps as one node that runs the whole call again: packed weights are looked up, and random numbers drawn, on every
-replay."""
+replay.  The same function answers where a call has no meaning: it has no forward-mode derivative, so a dual tensor raises
+NotImplementedError whether or not anything asks for a gradient (the native call would hand back a tensor without its
+tangent), and no rule for ``torch.func``'s transforms, which raise RuntimeError."""
 import functools
 
 import torch
+from torch._C import _are_functorch_transforms_active, _is_tracing   # 0.15 us a call together; through torch.jit 0.3
+from torch.autograd import forward_ad
 
 
 def transformed():
-    """Whether the calls of this thread are being recorded by a trace."""
-    return torch.jit.is_tracing()
+    """Whether calls are being recorded by a trace, carry forward-mode tangents or run inside a ``torch.func`` transform."""
+    return _is_tracing() or forward_ad._current_level >= 0 or _are_functorch_transforms_active()
 
 
 class _OneNode(torch.autograd.Function):
@@ -47,5 +51,7 @@ def one_node(fn):
     arguments of its own, results a tensor or a tuple."""
     @functools.wraps(fn)
     def call(*args):
-        return _OneNode.apply(fn, *args) if transformed() else fn(*args)
+        if _is_tracing() or forward_ad._current_level >= 0 or _are_functorch_transforms_active():   # transformed(), without its call
+            return _OneNode.apply(fn, *args)
+        return fn(*args)
     return call

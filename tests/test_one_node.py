@@ -4,6 +4,7 @@ import warnings
 
 import pytest
 import torch
+from torch.autograd import forward_ad
 
 import quartet_amd as q
 from quartet_amd import _lib
@@ -60,6 +61,33 @@ def test_a_trace_follows_the_weight(host):
         traced = torch.jit.trace(layer, (x,), check_trace=False)
         layer.weight.mul_(-2.0)
         assert torch.equal(traced(x), layer(x))
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("make", [_layer, q.QuestMXFP4Quantizer, lambda: q.AlbertTsengQuantizer(stochastic=False)])
+def test_tangents_are_refused(host, make, grad):
+    """No forward-mode derivative exists: a dual input or weight raises, also where nothing asks for a gradient; plain
+    tensors go through at a dual level."""
+    module = make()
+    x = torch.randn(8, 64)
+    with forward_ad.dual_level(), torch.set_grad_enabled(grad):
+        with pytest.raises(NotImplementedError):
+            module(forward_ad.make_dual(x, torch.ones_like(x)))
+        if isinstance(module, q.QuantizedLinear):
+            dual = forward_ad.make_dual(module.weight.detach(), torch.ones_like(module.weight))
+            with pytest.raises(NotImplementedError):
+                torch.func.functional_call(module, {"weight": dual}, (x,))
+            module.requires_grad_(False)
+        assert torch.equal(module(x), make()(x))
+
+
+@pytest.mark.parametrize("make", [_layer, q.QuestMXFP4Quantizer])
+def test_function_transforms_are_refused(host, make):
+    module, x = make().requires_grad_(False), torch.randn(4, 8, 64)
+    for transform in (lambda: torch.func.vmap(module)(x), lambda: torch.func.grad(lambda t: module(t).sum())(x[0]),
+                      lambda: torch.func.jvp(module, (x[0],), (x[0],)), lambda: torch.func.vjp(module, x[0])):
+        with pytest.raises(RuntimeError, match="functorch"):
+            transform()
 
 
 @pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning")
