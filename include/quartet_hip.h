@@ -152,9 +152,10 @@ int qm_gemm_mxfp4_bf16_nn(const uint8_t* a_codes, const uint8_t* a_scales, const
 /*
  * qm_gemm_mxfp4_tn for callers that cannot allocate (code under HIP graph capture, serving loops, harnesses that forbid
  * hipMalloc).  It has no counterpart in the reference.  Same arguments and the same results, bit for bit, as
- * qm_gemm_mxfp4_tn offered qm_gemm_workspace_bytes(M, N, K) bytes of workspace; the split-K partial sums live in a
- * device array built into the library (QM_GEMM_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends) instead.
- * A shape whose partial sums need more is rejected with QM_ERR_INVALID.  Nothing in the array has to start at zero
+ * qm_gemm_mxfp4_tn offered QM_GEMM_NOALLOC_SCRATCH_BYTES of workspace; the split-K partial sums live in a device array
+ * built into the library (that many bytes per GPU, held until the process ends) instead.  A product whose cut needs more
+ * runs whole; only one of so few 256 x 256 tiles and so long a K that the ranges filling the CUs do not fit is rejected with
+ * QM_ERR_INVALID (4096 x 1536 x 32768).  Nothing in the array has to start at zero
  * (every partial sum that is read has been written by the same call), but every call on a GPU uses that GPU's one
  * array: calls that overlap on one GPU (two streams, two threads) race.  Allocates nothing, frees nothing --
  * with one proviso about the HIP runtime: the device address of the array is looked up on a device's first use, and

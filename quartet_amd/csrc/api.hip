@@ -266,8 +266,9 @@ int qm_gemm_mxfp4_tn_noalloc(const uint8_t* a_codes, const uint8_t* a_scales, co
     if (M < 0 || N < 0 || K < 0 || K % 32)
         return fail(QM_ERR_INVALID, "qm_gemm_mxfp4_tn_noalloc: need K %% 32 == 0 (M=%lld N=%lld K=%lld)", (long long)M, (long long)N, (long long)K);
     if (M == 0 || N == 0) return 0;
-    // the same cut into K ranges as qm_gemm_mxfp4_tn makes when it is offered qm_gemm_workspace_bytes() of scratch
-    const size_t need = qm::gemm_workspace_bytes(M, N, K);
+    // refused: few tiles and a K so long that the ranges filling the CUs do not fit.  Every other product runs, in the cut that
+    // qm_gemm_mxfp4_tn makes of it where that fits and whole where it does not (2176 x 8192 x 28672: two ranges, 136 MiB).
+    const size_t need = qm::gemm_few_tiles_bytes(M, N, K);
     if (need > kNoAllocScratchBytes)
         return fail(QM_ERR_INVALID, "qm_gemm_mxfp4_tn_noalloc: this shape's split-K partial sums need %zu bytes, the built-in scratch "
                                     "holds %zu (M=%lld N=%lld K=%lld); use qm_gemm_mxfp4_tn with a caller-provided workspace",
@@ -276,7 +277,7 @@ int qm_gemm_mxfp4_tn_noalloc(const uint8_t* a_codes, const uint8_t* a_scales, co
     // library's device image (qm_gemm_noalloc_prepare() does the same ahead of time)
     void* ws = nullptr;
     if (int rc = scratch_of_current_device(&ws)) return rc;
-    return qm_gemm_mxfp4_tn(a_codes, a_scales, b_codes, b_scales, M, N, K, alpha, c, c_dtype, a_layout, b_layout, need ? ws : nullptr, need, stream);
+    return qm_gemm_mxfp4_tn(a_codes, a_scales, b_codes, b_scales, M, N, K, alpha, c, c_dtype, a_layout, b_layout, ws, kNoAllocScratchBytes, stream);
 }
 
 int qm_masked_hadamard_bwd(const void* g, int g_dtype, int64_t rows, int64_t cols, int hadamard_dim, int scale_dtype,

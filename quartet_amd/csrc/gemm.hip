@@ -1062,6 +1062,7 @@ size_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     const bool persistent = persistent_serves(M, N, K, nullptr, nullptr, nullptr), tiles_ok = gemm_tile_serves(M, N, K, 0, 0, nullptr);
     return persistent || tiles_ok ? plan_of_shape(M, N, K, persistent, tiles_ok).scratch_bytes : 0;
 }
+size_t gemm_few_tiles_bytes(int64_t M, int64_t N, int64_t K) { return gemm_supports_tiled(M, N, K) ? scratch_of_few_tiles(M, N, K, device_cus()) : 0; }
 size_t gemm_e5m2_workspace_bytes(int64_t M, int64_t N, int64_t K) { return plan_of_shape(M, N, K, false, true, true).scratch_bytes; }
 
 // The kernel that serves product p.  p.mask: the caller wants the masked inverse rotation applied to the result (mid dtype

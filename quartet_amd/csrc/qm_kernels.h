@@ -167,6 +167,8 @@ hipError_t gemm_mxfp4_tn(const uint8_t* a_codes, const uint8_t* a_scales, const 
 hipError_t splitk_reduce_rotated(const float* partial, int splits, int64_t mn, float alpha, int mid_dtype, const uint8_t* maskbits,
                                  int hd, const SignBits& signs, float c, void* out, int out_dtype, hipStream_t stream);
 size_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
+// the part of it that the ranges filling the persistent kernel's CUs ask for (0: whole tiles already do, or K is short)
+size_t gemm_few_tiles_bytes(int64_t M, int64_t N, int64_t K);
 size_t gemm_e5m2_workspace_bytes(int64_t M, int64_t N, int64_t K);   // the same for a product with an eight-bit B
 
 // The product on small and middle-sized tiles (gemm_tile.hip).  Any M; N % 8 == 0; K % 128 == 0, or K % 128 == 64 with

@@ -122,3 +122,13 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "LIB_PATH", str(tmp_path / "libquartet_hip.so"))
     with pytest.raises(_lib.QuartetHipError, match="no CPU fallback"):
         _lib.lib()
+
+
+@pytest.mark.parametrize("shape", [(2176, 8192, 28672), (2048, 11264, 26624), (1344, 12288, 49152), (512, 512, 512)])
+def test_allocation_free_product_refuses_few_tiles_only(shape):
+    """A cut into K ranges that the built-in scratch cannot hold is not made; it is no reason to refuse the product."""
+    L = _lib.lib()
+    assert L.qm_gemm_mxfp4_tn_noalloc(None, None, None, None, *shape, 1.0, None, 0, 0, 0, None) != 0   # null tensors, or no GPU
+    assert b"built-in scratch" not in L.qm_last_error()
+    assert L.qm_gemm_mxfp4_tn_noalloc(None, None, None, None, 4096, 1536, 32768, 1.0, None, 0, 0, 0, None) == -1
+    assert b"built-in scratch" in L.qm_last_error()

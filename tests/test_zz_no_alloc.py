@@ -72,6 +72,17 @@ def test_noalloc_product_under_graph_capture():
         assert torch.equal(out, want), f"replay {replay}"
 
 
+def test_noalloc_product_runs_whole_where_its_cut_does_not_fit():
+    from quartet_amd import _lib, kernels as K
+    L = _lib.lib()
+    M, N, Kd = 2176, 8192, 28672           # cut into two ranges of 68 MiB each where a workspace is offered
+    assert L.qm_gemm_workspace_bytes(M, N, Kd) > L.qm_gemm_noalloc_scratch_bytes()
+    print(f"case noalloc gemm whole shape={M}x{N}x{Kd}", flush=True)
+    ops = _operands(M, N, Kd, 400, torch.device("cuda:0"))
+    out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda:0")
+    assert torch.equal(K.gemm_mxfp4_tn_noalloc(*ops, 1.0, out), K.gemm_mxfp4_tn(*ops, 1.0, torch.bfloat16, split_k=False))
+
+
 def test_noalloc_product_rejects_what_does_not_fit():
     from quartet_amd import _lib
     L = _lib.lib()
