@@ -208,9 +208,10 @@ int qm_diag_gemm_tile_phases(const uint8_t* a_codes, const uint8_t* a_scales, co
  * bf16 values: a few results in 10^4 differ in the last bf16 bit).
  *   maskbits     [M, N/8] clip-mask bits of the forward quantizer (bit n % 8 of byte n / 8), 4-byte aligned; sign_bits,
  *                scale_dtype as for qm_masked_hadamard_bwd with hadamard_dim 32
- *   Served shapes: those of the persistent kernel without a cut into K ranges -- qm_gemm_fuses_rotation() tells (M, N
- *   multiples of 64 and >= 256, K % 128 == 0 and > 768, scale arrays 16-byte aligned when K % 512 == 0, few enough output
- *   tiles that no workspace would be used); anything else returns QM_ERR_INVALID and the caller makes the two calls.
+ *   Served shapes: qm_gemm_fuses_rotation() tells -- M, N multiples of 64 and >= 256, K % 128 == 0 and > 768, scale arrays
+ *   16-byte aligned when K % 512 == 0, and not so few 256 x 256 tiles with so long a K that ranges of it would fill the CUs.
+ *   Anything else returns QM_ERR_INVALID and the caller makes the two calls.  The product is never cut into K ranges here,
+ *   where qm_gemm_mxfp4_tn may cut it when offered a workspace (and then rounds differently).
  */
 int qm_gemm_fuses_rotation(const uint8_t* a_scales, const uint8_t* b_scales, int64_t M, int64_t N, int64_t K);
 int qm_gemm_mxfp4_tn_rotated(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes, const uint8_t* b_scales,

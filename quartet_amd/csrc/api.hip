@@ -298,9 +298,9 @@ int qm_masked_hadamard_bwd(const void* g, int g_dtype, int64_t rows, int64_t col
 
 int qm_gemm_fuses_rotation(const uint8_t* a_scales, const uint8_t* b_scales, int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 32) return 0;
-    // offered the workspace the plain product would use: a shape it would cut into K ranges is not served
-    const size_t ws = qm::gemm_workspace_bytes(M, N, K);
-    return ws == 0 && qm::gemm_persistent_rotates(a_scales, b_scales, M, N, K) ? 1 : 0;
+    // not where the persistent kernel's few tiles leave CUs idle and K ranges would fill them; whether smaller tiles, or a cut
+    // on them, would be cheaper is the caller's business (qm_linear_backward weighs that by itself)
+    return qm::gemm_few_tiles_bytes(M, N, K) == 0 && qm::gemm_persistent_rotates(a_scales, b_scales, M, N, K) ? 1 : 0;
 }
 
 int qm_gemm_mxfp4_tn_rotated(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes, const uint8_t* b_scales,

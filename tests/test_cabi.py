@@ -132,3 +132,14 @@ def test_allocation_free_product_refuses_few_tiles_only(shape):
     assert b"built-in scratch" not in L.qm_last_error()
     assert L.qm_gemm_mxfp4_tn_noalloc(None, None, None, None, 4096, 1536, 32768, 1.0, None, 0, 0, 0, None) == -1
     assert b"built-in scratch" in L.qm_last_error()
+
+
+def test_rotation_in_the_epilogue_is_offered_for_every_uncut_shape():
+    """Served: the persistent kernel's shapes above K = 768, also where a cut on smaller tiles would be cheaper.  Not served: few
+    tiles whose K ranges would fill the CUs, short contractions, ragged extents."""
+    L = _lib.lib()
+    for shape in [(256, 256, 2560), (256, 256, 1024), (256, 512, 1536), (320, 448, 1920), (2176, 8192, 28672), (8192, 4096, 4096)]:
+        assert L.qm_gemm_fuses_rotation(None, None, *shape) == 1, shape
+    assert L.qm_gemm_workspace_bytes(256, 256, 2560) > 0      # as a plain product it may be cut
+    for shape in [(512, 768, 8192), (4096, 1536, 32768), (256, 256, 768), (250, 256, 1024), (256, 224, 1024), (256, 256, 1088)]:
+        assert L.qm_gemm_fuses_rotation(None, None, *shape) == 0, shape

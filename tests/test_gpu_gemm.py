@@ -230,6 +230,24 @@ def test_product_with_the_inverse_rotation_in_its_epilogue(oracle, K, M, N, K_, 
         assert rel < 4e-3, rel     # the bf16 rounding of the result: 2^-9 relative per element
 
 
+@pytest.mark.parametrize("M,N,K_", [(256, 256, 2560), (320, 448, 3328)])
+def test_rotated_product_where_the_plain_one_may_be_cut(K, M, N, K_):
+    """The same rotation on shapes whose plain product takes a workspace when offered one: against the uncut product."""
+    from quartet_amd import _lib
+    assert _lib.lib().qm_gemm_workspace_bytes(M, N, K_) > 0
+    print(f"case rotated product of a cut shape {M}x{N}x{K_}", flush=True)
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device="cpu").manual_seed(K_)
+    byte = lambda rows, cols, lo=0, hi=256: torch.randint(lo, hi, (rows, cols), generator=g, dtype=torch.uint8).to(dev)
+    ac, bc, as_, bs, keep = byte(M, K_ // 2), byte(N, K_ // 2), byte(M, K_ // 32, 118, 132), byte(N, K_ // 32, 120, 136), byte(M, N // 8)
+    got = K.gemm_mxfp4_tn_rotated(ac, as_, bc, bs, keep, 1.0, torch.float32, 5)
+    plain = K.gemm_mxfp4_tn(ac, as_, bc, bs, 1.0, torch.bfloat16, split_k=False)
+    two = K.masked_hadamard_bwd(plain, 32, torch.float32, 5, keep)
+    assert float((got != two).float().mean()) < 1e-4      # as above: the order of a group's fp32 sum
+    step = two.float().abs() * 2.0 ** -7 + float(plain.float().abs().max()) * 2.0 ** -18
+    assert bool(((got.float() - two.float()).abs() <= step).all())
+
+
 def test_split_k_is_offered_and_reproducible(K):
     from quartet_amd import _lib
     L = _lib.lib()
