@@ -619,7 +619,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     Big4Plan plan;
     plan.lds_codes = (uint32_t)__builtin_amdgcn_readfirstlane((int)(smem_base + wave * 4096));
     plan.lds_scales = (uint32_t)__builtin_amdgcn_readfirstlane((int)(smem_base + kScaleAreaOff + wave * 1024));
-    const int row16 = 16 * code_pitch;   // 16 rows are 8 K bytes in either layout, K >= 512
+    const uint32_t row16 = 16u * (uint32_t)code_pitch;   // 16 rows are 8 K bytes in either layout, 512 <= K < 2^26: 63 rows stay below 2^31
     // the offsets of clamped rows may fall below i * 1024: RAGGED takes them from a base that much further back
     constexpr uint32_t kLoadBias = RAGGED ? 3 * 1024 : 0;
     // source of this lane in wave-load i: row 16 i + lane / 4 of the wave's 64 (at most `last`), swizzled 16-byte column
@@ -627,7 +627,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         const int prow = lane >> 2, pcv = (lane & 3) ^ ((prow >> 2) & 3);
         int r = 16 * i + prow;
         r = r < last ? r : last;
-        const uint32_t off = tiled ? (uint32_t)((r >> 4) * row16 + (r & 15) * 64) : (uint32_t)(r * code_pitch);
+        const uint32_t off = tiled ? (uint32_t)(r >> 4) * row16 + (uint32_t)(r & 15) * 64u : (uint32_t)r * (uint32_t)code_pitch;
         return off + pcv * 16 + kLoadBias - 1024u * i;
     };
     plan.kstep_a = a_tiled ? 1024 : kRowBytes;
@@ -883,7 +883,7 @@ double persistent_cost(int64_t M, int64_t N, int64_t K, int splits, int cus) {
 // addresses.
 bool persistent_serves(int64_t M, int64_t N, int64_t K, const void* a_scales, const void* b_scales, const void* c) {
     const int64_t steps = K / kBK, pad = ((steps + 3) & ~(int64_t)3) - steps;
-    if (N % 64 || M < kBigM || N < kBigN || K % kBK || steps < 4 || pad * 3 > steps || M >= (1 << 30) || N >= (1 << 30) || K >= (1 << 24)) return false;
+    if (N % 64 || M < kBigM || N < kBigN || K % kBK || steps < 4 || pad * 3 > steps || M >= (1 << 30) || N >= (1 << 30) || K >= (1 << 26)) return false;
     if (K % 512 == 0 && ((reinterpret_cast<uintptr_t>(a_scales) | reinterpret_cast<uintptr_t>(b_scales)) & 15)) return false;
     return (reinterpret_cast<uintptr_t>(c) & 15) == 0;
 }

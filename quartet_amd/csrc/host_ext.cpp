@@ -132,16 +132,22 @@ LayerPtr make_layer(int a_hd, py::handle a_signs, int w_hd, py::handle w_signs, 
     return l;
 }
 
+// contractions from here on are not the tile kernels' (csrc/gemm_tile.hip): 32-bit offsets inside a tile.  The packed-weight key
+// of quartet_amd.linear holds which side of it a call's tokens are on.
+constexpr int64_t kLongContraction = 1 << 23;
+
 void set_extents(Layer& l, int64_t T, const Tensor& weight) {
     l.T = T; l.I = weight.size(1); l.O = weight.size(0);
     l.w_dtype = weight.scalar_type();
     // Tiled code bytes (16 rows x 128 elements contiguous, extents padded with zeros).  Row-major where the padding is not
-    // available: rows of y that are not whole 16-byte pieces, and dense forward rotations off the multiples of 128.
+    // available: rows of y that are not whole 16-byte pieces, and dense forward rotations off the multiples of 128; and where
+    // an extent is too long a contraction for the tile kernels and the others too ragged or short for the 256 x 256 one.
     const bool dense = l.x_dense.defined() || l.w_dense.defined();
     const bool classic = l.T % 128 == 0 && l.I % 128 == 0 && l.O % 128 == 0;
-    l.layout = l.O % 8 || (dense && !classic) ? QM_LAYOUT_ROWMAJOR : QM_LAYOUT_PADDED;
+    const bool large = classic && l.T >= 256 && l.I >= 256 && l.O >= 256;
+    l.layout = l.O % 8 || (dense && !classic) || (std::max({l.T, l.I, l.O}) >= kLongContraction && !large) ? QM_LAYOUT_ROWMAJOR : QM_LAYOUT_PADDED;
     // the extents for which a device seed base is promised (set_device_seed_base)
-    l.seed_base_ok = classic && l.T >= 256 && l.I >= 256 && l.O >= 256 && l.a_hd == 32 && l.w_hd == 32 && l.g_hd == 32;
+    l.seed_base_ok = large && l.a_hd == 32 && l.w_hd == 32 && l.g_hd == 32;
 }
 
 Tensor packed_buffer(int64_t rows, int64_t cols, const Tensor& like) { return bytes((int64_t)qm_packed_operand_bytes(rows, cols), like); }
@@ -308,7 +314,7 @@ Tensor linear_forward(const LayerPtr& l, const Tensor& x, const Tensor& weight, 
 // A decoded batch against a weight that is already packed: one launch, undefined where that kernel does not serve
 Tensor linear_decode(const Layer& l, const Tensor& x, const Tensor& weight, const Tensor& packed_w) {
     const int64_t I = weight.size(1), O = weight.size(0);
-    if (x.numel() == 0 || x.numel() > 16 * I || l.a_hd != 32 || l.x_dense.defined() || l.w_dense.defined() || x.size(-1) != I) return {};
+    if (x.numel() == 0 || x.numel() > 16 * I || l.a_hd != 32 || l.x_dense.defined() || l.w_dense.defined() || x.size(-1) != I || O >= kLongContraction) return {};
     const int64_t T = x.numel() / I;
     if (!qm_linear_decode_serves(T, I, O)) return {};
     require_cuda(x, weight);

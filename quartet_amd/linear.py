@@ -65,12 +65,14 @@ def _error_draws(g_q, e):
 
 def _cached_weight(x, weight, a_q, w_q, g_q, weight_cache):
     """(cache key, packed Q(W) or None): Q(W) of an unchanged weight (the micro-steps of one accumulation) is quantized
-    once and kept by the layer.  The last two entries of the key stand for the code layout, which csrc/host_ext.cpp picks."""
+    once and kept by the layer.  The last three entries of the key stand for the code layout, which csrc/host_ext.cpp picks."""
     if weight_cache is None:
         return None, None
     dense = a_q._dense is not None or w_q._dense is not None
-    key = (weight.data_ptr(), weight._version, weight.dtype, weight.shape, w_q.hadamard_dim, w_q.sign_bits,
-           None if w_q._dense is None else w_q._dense_epoch, dense and x.numel() // x.shape[-1] % 128 == 0)
+    shape = weight.shape
+    key = (weight.data_ptr(), weight._version, weight.dtype, shape, w_q.hadamard_dim, w_q.sign_bits,
+           None if w_q._dense is None else w_q._dense_epoch, dense and x.numel() // x.shape[-1] % 128 == 0,
+           x.numel() >= shape[1] << 23)
     return key, weight_cache.get(key)
 
 
@@ -181,7 +183,7 @@ class QuantizedLinear(nn.Linear):
 
     def _is_error_only_config(self, x):
         """The error-only scheme between the same quantizers, with products in bf16 (bf16 autocast, or bf16 tensors throughout)
-        and extents that are multiples of 32 and of the Hadamard blocks."""
+        and extents below 2^23 that are multiples of 32 and of the Hadamard blocks."""
         modules = self._modules
         a_q, w_q, scheme = modules["activation_quantizer"], modules["weight_quantizer"], modules["backward_scheme"]
         g_q = scheme.g_quantizer
@@ -197,7 +199,7 @@ class QuantizedLinear(nn.Linear):
         O, I = weight.shape
         T = x.numel() // x.shape[-1]
         return not (x.shape[-1] != I or T % 32 or I % 32 or O % 32 or I % a_q.hadamard_dim or I % w_q.hadamard_dim
-                    or T % g_q.hadamard_dim or O % g_q.hadamard_dim)
+                    or T % g_q.hadamard_dim or O % g_q.hadamard_dim or max(T, I, O) >= 1 << 23)
 
     def forward(self, x):
         if self._is_production_config(x.numel() // max(x.shape[-1], 1)):
