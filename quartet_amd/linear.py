@@ -103,6 +103,16 @@ class QuartetLinearFn:
         return y
 
 
+_GLOBAL_HOOKS = (nn.modules.module._global_forward_hooks, nn.modules.module._global_forward_pre_hooks, nn.modules.module._global_backward_hooks,
+                 nn.modules.module._global_backward_pre_hooks)
+
+
+def _watched(module):
+    """Whether calling `module` runs more than its class's forward: hooks, or a forward of its own."""
+    return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+                or "forward" in module.__dict__)
+
+
 class PackedWeightCache:
     """The packed Q(W) of a layer's current weight, kept across the micro-steps of one gradient accumulation (the
     weight changes only at the optimizer step, src/optim/base.py:188-207 of the reference).  One entry, replaced --
@@ -191,6 +201,9 @@ class QuantizedLinear(nn.Linear):
                 and type(w_q) is QuestMXFP4Quantizer and type(g_q) is AlbertTsengQuantizer):
             return False
         if a_q.is_dense or w_q.is_dense or g_q.is_dense:
+            return False
+        # this scheme calls its quantizers and itself as modules: where somebody listens, it still does
+        if any(_GLOBAL_HOOKS) or _watched(a_q) or _watched(w_q) or _watched(g_q) or _watched(scheme):
             return False
         weight, out = self.weight, (torch.bfloat16, torch.float32)
         if not (x.is_cuda and weight.is_cuda and x.numel() and x.dtype in out and weight.dtype in out

@@ -653,3 +653,50 @@ def test_error_only_scheme_keeps_the_library_path_for_fp32_products(q, monkeypat
     x = torch.randn(64, 128, device=dev, requires_grad=True)
     layer(x).sum().backward()
     assert torch.isfinite(x.grad).all() and torch.isfinite(layer.weight.grad).all()
+
+
+@pytest.mark.parametrize("kind", ["forward", "pre", "backward", "global", "instance"])
+def test_error_only_scheme_calls_its_modules_where_somebody_listens(q, kind):
+    """Hooks on the quantizers and on the scheme fire, and a forward set on an instance runs, as in the module path; without
+    them the same layer runs on packed operands."""
+    from torch.nn.modules.module import register_module_forward_hook
+    dev = torch.device("cuda:0")
+    torch.manual_seed(3)
+    layer = q.QuantizedLinear(256, 128, bias=False, weight_quantizer=q.QuestMXFP4Quantizer(), activation_quantizer=q.QuestMXFP4Quantizer(),
+                              gradient_quantizer=q.AlbertTsengQuantizer(stochastic=False), backward_scheme=q.BACKWARD_SCHEMES["Q(E)W_Q(Et)X"](),
+                              device=dev, dtype=torch.bfloat16)
+    x, e = torch.randn(96, 256, device=dev, dtype=torch.bfloat16), torch.randn(96, 128, device=dev, dtype=torch.bfloat16)
+    assert layer._is_error_only_config(x)
+    seen = []
+    modules = {"a": layer.activation_quantizer, "w": layer.weight_quantizer, "s": layer.backward_scheme}
+
+    def run():
+        xr = x.clone().requires_grad_(True)
+        layer.weight.grad = None
+        y = layer(xr)
+        y.backward(e)
+        return y.detach(), xr.grad, layer.weight.grad
+    plain = run()
+    handles = []
+    for name, m in modules.items():
+        if kind == "forward":
+            handles.append(m.register_forward_hook(lambda m, i, o, name=name: seen.append(name)))
+        elif kind == "pre":
+            handles.append(m.register_forward_pre_hook(lambda m, i, name=name: seen.append(name)))
+        elif kind == "backward":
+            handles.append(m.register_full_backward_hook(lambda m, gi, go, name=name: seen.append(name)))
+        elif kind == "instance":
+            m.forward = lambda *args, f=m.forward, name=name: (seen.append(name), f(*args))[1]
+    if kind == "global":
+        names = {id(m): name for name, m in modules.items()}
+        handles.append(register_module_forward_hook(lambda m, i, o: seen.append(names[id(m)]) if id(m) in names else None))
+    try:
+        watched = run()
+    finally:
+        for h in handles:
+            h.remove()
+    assert sorted(seen) == ["a", "s", "w"]
+    for a, b in zip(watched, plain):     # operands, products and gradients rounded to bf16 at other places
+        assert float((a.float() - b.float()).norm() / b.float().norm()) < 1e-2
+    if kind != "instance":
+        assert layer._is_error_only_config(x)
