@@ -30,6 +30,7 @@
 #include <type_traits>
 
 #include "gemm_common.h"
+#include "shape_table.h"
 
 namespace qm {
 
@@ -1009,8 +1010,8 @@ bool gemm_supports_tiled(int64_t M, int64_t N, int64_t K) {
            K < (1 << 30);
 }
 
-// The candidates of one shape, worked out once and remembered (per thread, a fixed table: 160 estimates take the host
-// several microseconds)
+// The candidates of one shape, worked out once per thread and remembered (a layer's backward pass asks for two or more shapes
+// several times over; 160 estimates take the host up to several microseconds): up to 256 shapes, 40 KB
 struct ShapePlan {
     int64_t M = -1, N = 0, K = 0;
     int flags = -1;
@@ -1036,11 +1037,7 @@ size_t scratch_of_few_tiles(int64_t M, int64_t N, int64_t K, int cus) {
     }
     return splits > 1 ? (size_t)splits * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
-const ShapePlan& plan_of_shape(int64_t M, int64_t N, int64_t K, bool persistent, bool tiles_ok, bool e5m2 = false) {
-    static thread_local ShapePlan table[64];
-    const int flags = (persistent ? 1 : 0) | (tiles_ok ? 2 : 0) | (e5m2 ? 4 : 0);
-    ShapePlan& e = table[(size_t)(M * 31 + N * 17 + K * 7 + flags) % 64];
-    if (e.M == M && e.N == N && e.K == K && e.flags == flags) return e;
+ShapePlan make_plan(int64_t M, int64_t N, int64_t K, bool persistent, bool tiles_ok, bool e5m2, int flags) {
     const int cus = device_cus();
     ShapePlan p;
     p.M = M; p.N = N; p.K = K; p.flags = flags;
@@ -1054,7 +1051,12 @@ const ShapePlan& plan_of_shape(int64_t M, int64_t N, int64_t K, bool persistent,
     p.cut_bytes = p.cut.cost < best ? (size_t)p.cut.choice.splits * (size_t)M * (size_t)N * sizeof(float) : 0;
     p.scratch_bytes = persistent ? scratch_of_few_tiles(M, N, K, cus) : 0;
     if (p.cut_bytes > p.scratch_bytes) p.scratch_bytes = p.cut_bytes;
-    return e = p;
+    return p;
+}
+const ShapePlan& plan_of_shape(int64_t M, int64_t N, int64_t K, bool persistent, bool tiles_ok, bool e5m2 = false) {
+    static thread_local ShapeTable<ShapePlan, 6> table;
+    const int flags = (persistent ? 1 : 0) | (tiles_ok ? 2 : 0) | (e5m2 ? 4 : 0);
+    return table.find(M, N, K, flags, [&] { return make_plan(M, N, K, persistent, tiles_ok, e5m2, flags); });
 }
 
 // bytes of scratch with which gemm_mxfp4_tn may cut this shape into K ranges (0: it would not)

@@ -31,3 +31,12 @@ def test_qm_math_on_the_host(tmp_path):
             hashes[name] = ((hashes[name] ^ bits) * 1099511628211) & 0xFFFFFFFFFFFFFFFF
     got = re.search(r"exp_hash=([0-9a-f]+) silu_hash=([0-9a-f]+)", run.stdout)
     assert got and int(got.group(1), 16) == hashes["exp"] and int(got.group(2), 16) == hashes["silu"]
+
+
+def test_remembered_shapes_on_the_host(tmp_path):
+    """The table of a product's candidates: extents that are multiples of 64 do not push each other out."""
+    exe = tmp_path / "shape_table_check"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", "-Werror", "-I", os.path.join(ROOT, "quartet_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "shape_table_check.cpp"), "-o", str(exe)], check=True)
+    run = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert run.returncode == 0 and run.stdout.strip().endswith("ok"), run.stdout[-2000:]
