@@ -1125,7 +1125,7 @@ hipError_t run_product(const ProductChoice& c, const TileProduct& p, int c_dtype
             q.c = workspace;
             q.splits = c.splits;
             q.mask = nullptr;
-            e = gemm_tile(c.kind, q, nullptr, F32, stream);
+            e = gemm_tile(c.kind, q, F32, stream);
         } else {
             e = launch_big4<float>(p.a_codes, p.a_scales, p.b_codes, p.b_scales, M, N, K, 1.0f, workspace, p.a_tiled, p.b_tiled, c.splits, cus, stream);
         }
@@ -1146,7 +1146,7 @@ hipError_t run_product(const ProductChoice& c, const TileProduct& p, int c_dtype
         q.splits = 1;
         if (!c.rotates) q.mask = nullptr;
         q.out_f32 = c_dtype == BF16 && rot_out_dtype == F32;
-        return gemm_tile(c.kind, q, nullptr, c_dtype, stream);
+        return gemm_tile(c.kind, q, c_dtype, stream);
     }
     if (c.rotates)
         return launch_big4<uint16_t, true>(p.a_codes, p.a_scales, p.b_codes, p.b_scales, M, N, K, p.alpha, p.c, p.a_tiled, p.b_tiled, 1, cus, stream,

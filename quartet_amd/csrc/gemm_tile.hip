@@ -8,8 +8,7 @@
 // through the ring's LDS and leave as 16-byte pieces of whole rows; on that way a lane holds eight consecutive columns,
 // which is what the masked inverse Hadamard rotation of the layer's backward pass works on: it is applied there (blocks of
 // 32, 64 or 128 along N), with the arithmetic of the stand-alone kernel, bit for bit, and the rotated-basis gradient never
-// travels through memory.  Two independent products of the same element types can share a grid (the two gradient products
-// of a small layer: neither fills the chip alone).
+// travels through memory.
 //
 // What bounds it: at 256 x 128 the LDS reads of the K loop (1.5 x the 256 x 256 kernel's bytes per flop) and, for short
 // contractions, the tile boundary, which the neighbour workgroup on the same CU covers; the smaller tiles are latency-bound
@@ -382,38 +381,26 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
     __syncthreads();  // the staging area is the next tile's ring
 }
 
-// Persistent over the tiles of g, then of h (h.M == 0: none)
 template <class S, typename OutT>
-__global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu((S::OCC * S::kWaves + 3) / 4))) void gemm_mxfp4_tn_tile_kernel(
-    TileProduct g, TileProduct h, int tiles_g, int tiles) {
-    extern __shared__ uint32_t smem[];
-    const uint32_t smem_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint32_t*)smem;
-    for (int t = (int)blockIdx.x; t < tiles; t += (int)gridDim.x) {
-        const bool first = t < tiles_g;   // uniform: every field below is a scalar select
-        TileProduct p;
-#define QM_PICK(f) p.f = first ? g.f : h.f
-        QM_PICK(a_codes); QM_PICK(a_scales); QM_PICK(b_codes); QM_PICK(b_scales); QM_PICK(c); QM_PICK(mask); QM_PICK(M); QM_PICK(N);
-        QM_PICK(K); QM_PICK(splits); QM_PICK(a_tiled); QM_PICK(b_tiled); QM_PICK(alpha); QM_PICK(hd); QM_PICK(signs.w[0]); QM_PICK(signs.w[1]);
-        QM_PICK(signs.w[2]); QM_PICK(signs.w[3]); QM_PICK(rot_c); QM_PICK(out_f32);
-#undef QM_PICK
-        tile_run<S, OutT>(p, first ? t : t - tiles_g, smem, smem_base);
-    }
-}
-
-// the same with an eight-bit B (one product)
-template <class S, typename OutT>
-__global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu((S::OCC * S::kWaves + 3) / 4))) void gemm_mxfp4_e5m2_tile_kernel(
-    TileProduct g, int tiles) {
+__device__ __forceinline__ void run_tiles(const TileProduct& g, int tiles) {   // persistent over the tiles
     extern __shared__ uint32_t smem[];
     const uint32_t smem_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint32_t*)smem;
     for (int t = (int)blockIdx.x; t < tiles; t += (int)gridDim.x) tile_run<S, OutT>(g, t, smem, smem_base);
 }
-
-template <class S>
-int tiles_of(const TileProduct& p) { return p.M == 0 ? 0 : ((p.M + S::BM - 1) / S::BM) * ((p.N + S::BN - 1) / S::BN) * p.splits; }
+template <class S, typename OutT>
+__global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu((S::OCC * S::kWaves + 3) / 4))) void gemm_mxfp4_tn_tile_kernel(
+    TileProduct g, int tiles) {
+    run_tiles<S, OutT>(g, tiles);
+}
+// the same with an eight-bit B
+template <class S, typename OutT>
+__global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu((S::OCC * S::kWaves + 3) / 4))) void gemm_mxfp4_e5m2_tile_kernel(
+    TileProduct g, int tiles) {
+    run_tiles<S, OutT>(g, tiles);
+}
 
 template <class S, typename OutT>
-hipError_t launch_tiles(const TileProduct& g, const TileProduct& h, hipStream_t stream) {
+hipError_t launch_tiles(const TileProduct& g, hipStream_t stream) {
     const auto kern = [] {
         if constexpr (S::kWideB) return gemm_mxfp4_e5m2_tile_kernel<S, OutT>;
         else return gemm_mxfp4_tn_tile_kernel<S, OutT>;
@@ -421,12 +408,11 @@ hipError_t launch_tiles(const TileProduct& g, const TileProduct& h, hipStream_t 
     static std::atomic<bool> lds_allowed[kMaxDevices];
     hipError_t e = allow_dynamic_lds(kern, S::kSmemBytes, lds_allowed);
     if (e != hipSuccess) return e;
-    const int tg = tiles_of<S>(g), tiles = tg + tiles_of<S>(h);
+    const int tiles = ((g.M + S::BM - 1) / S::BM) * ((g.N + S::BN - 1) / S::BN) * g.splits;
     // a grid that is a multiple of 8 so that tile t and t + grid land on the same XCD
     int grid = tiles < S::OCC * device_cus() ? tiles : S::OCC * device_cus();
     if (grid > 8 && grid < tiles) grid -= grid % 8;
-    if constexpr (S::kWideB) kern<<<dim3((unsigned)grid), dim3(S::kThreads), S::kSmemBytes, stream>>>(g, tiles);
-    else kern<<<dim3((unsigned)grid), dim3(S::kThreads), S::kSmemBytes, stream>>>(g, h, tg, tiles);
+    kern<<<dim3((unsigned)grid), dim3(S::kThreads), S::kSmemBytes, stream>>>(g, tiles);
     return hipGetLastError();
 }
 
@@ -450,12 +436,10 @@ bool gemm_tile_serves(int64_t M, int64_t N, int64_t K, int a_tiled, int b_tiled,
            (reinterpret_cast<uintptr_t>(c) & 15) == 0;
 }
 
-hipError_t gemm_tile(int shape, const TileProduct& g, const TileProduct* second, int c_dtype, hipStream_t stream) {
-    TileProduct h{};
-    if (second) h = *second;
+hipError_t gemm_tile(int shape, const TileProduct& g, int c_dtype, hipStream_t stream) {
     const auto go = [&](auto s) {
         using S = decltype(s);
-        return c_dtype == BF16 ? launch_tiles<S, uint16_t>(g, h, stream) : launch_tiles<S, float>(g, h, stream);
+        return c_dtype == BF16 ? launch_tiles<S, uint16_t>(g, stream) : launch_tiles<S, float>(g, stream);
     };
     if (g.b_e5m2) {
         switch (shape) {

@@ -196,8 +196,7 @@ struct TileProduct {
 // the kinds of an eight-bit B are WIDE_256x256 and 1 .. 3
 enum TileKind : int { TILE_256x128 = 0, WIDE_256x256 = 0, TILE_128x128 = 1, TILE_128x64 = 2, TILE_64x64 = 3, TILE_64x32 = 4 };
 bool gemm_tile_serves(int64_t M, int64_t N, int64_t K, int a_tiled, int b_tiled, const void* c);
-// one product, or two independent ones of the same element type in one grid
-hipError_t gemm_tile(int kind, const TileProduct& g, const TileProduct* second, int c_dtype, hipStream_t stream);
+hipError_t gemm_tile(int kind, const TileProduct& g, int c_dtype, hipStream_t stream);
 
 // The product of at most 64 rows with a weight, both tiled (gemm_rows.hip): K % 128 == 0, N % 8 == 0, c 16-byte aligned, no mask.
 // Its sums are in another order than the other kernels'.
