@@ -1,5 +1,6 @@
 """Tensor-level wrappers over the C ABI: allocate outputs with torch, pass raw device pointers and
-the current HIP stream.  PyTorch is only the allocator and stream provider here."""
+the current HIP stream.  PyTorch is only the allocator and stream provider here.  For callers of single operations (the
+operators, packed tensors, tests, measurements); the layers drive the same C entry points from csrc/host_ext.cpp."""
 import ctypes
 
 import torch
@@ -17,10 +18,6 @@ def _dtype_code(dt):
     if dt == torch.float32:
         return QM_F32
     raise TypeError(f"quartet_amd kernels take bfloat16 or float32 tensors, got {dt}")
-
-
-def _torch_dtype(code):
-    return torch.bfloat16 if code == QM_BF16 else torch.float32
 
 
 def _ptr(t):
@@ -304,24 +301,6 @@ def packed_operand_buffer(rows, cols, device):
 QM_W_IS_PACKED, QM_X_IS_PACKED = 1, 2
 
 
-def quantize_dense_into_packed(x2, matrix, tiled):
-    """Quest RTN + clip mask of x2 [rows, cols] under a dense 32 x 32 rotation, written into a fresh packed-operand buffer
-    (what linear_forward fills for a Hadamard rotation): the forward quantizer of a layer whose quantizer holds the matrix
-    of rerotate="O32"."""
-    _require_cuda(x2)
-    assert x2.dim() == 2 and x2.is_contiguous()
-    rows, cols = x2.shape
-    packed = packed_operand_buffer(rows, cols, x2.device)
-    off = (ctypes.c_size_t * 3)()
-    _lib.check(_lib.lib().qm_packed_operand_offsets(rows, cols, off), "qm_packed_operand_offsets")
-    m = _matrix_arg(matrix, x2.device)
-    base = packed.data_ptr()
-    rc = _lib.lib().qm_quantize_mxfp4_dense(_ptr(x2), _dtype_code(x2.dtype), rows, cols, _ptr(m), QM_QUEST_RTN, 0, 0, base + off[0],
-                                            base + off[1], base + off[2], None, _layout(tiled), _stream())
-    _lib.check(rc, "qm_quantize_mxfp4_dense")
-    return packed
-
-
 def linear_forward(x2, w2, hd_x, signs_x, hd_w, signs_w, out_dtype, tiled, packed_w=None, packed_x=None, rows=None):
     """Whole forward pass of a Quartet linear in one foreign call: quantize x [T,I] and w [O,I] (quest RTN + clip
     mask), y = Q(x) Q(w)^T.  Returns (y [T,O], packed_x, packed_w): the byte buffers the backward pass reads.  A
@@ -421,31 +400,6 @@ def swiglu_backward(g, h12, maskbits=None, signs=0, scale_dtype=torch.float32):
                                        _ptr(maskbits), sign_words(signs), _dtype_code(scale_dtype), _ptr(d), _stream())
     _lib.check(rc, "qm_swiglu_backward")
     return d
-
-
-def rope_split_qkv(qkv2, table, n_embd, head_dim, seq_len, out_dtype):
-    """qkv2 [rows, 3 n_embd] -> (q, k, v) [rows, n_embd] of out_dtype, q and k rotated pairwise by table [seq_len, head_dim/2, 2]."""
-    _require_cuda(qkv2, table)
-    assert qkv2.is_contiguous() and table.is_contiguous() and table.dtype == torch.float32
-    assert qkv2.shape[1] == 3 * n_embd and tuple(table.shape) == (seq_len, head_dim // 2, 2)
-    rows = qkv2.shape[0]
-    q, k, v = (torch.empty((rows, n_embd), dtype=out_dtype, device=qkv2.device) for _ in range(3))
-    rc = _lib.lib().qm_rope_split_qkv(_ptr(qkv2), _dtype_code(qkv2.dtype), rows, seq_len, n_embd, head_dim, _ptr(table), _ptr(q),
-                                      _ptr(k), _ptr(v), _dtype_code(out_dtype), _stream())
-    _lib.check(rc, "qm_rope_split_qkv")
-    return q, k, v
-
-
-def rope_merge_qkv_grad(dq, dk, dv, table, n_embd, head_dim, seq_len, out_dtype):
-    """Gradients of rope_split_qkv's outputs, each [rows, n_embd] -> gradient of its input [rows, 3 n_embd] of out_dtype."""
-    _require_cuda(dq, dk, dv, table)
-    assert dq.is_contiguous() and dk.is_contiguous() and dv.is_contiguous() and dq.dtype == dk.dtype == dv.dtype
-    rows = dq.shape[0]
-    d_qkv = torch.empty((rows, 3 * n_embd), dtype=out_dtype, device=dq.device)
-    rc = _lib.lib().qm_rope_merge_qkv_grad(_ptr(dq), _ptr(dk), _ptr(dv), _dtype_code(dq.dtype), rows, seq_len, n_embd, head_dim,
-                                           _ptr(table), _ptr(d_qkv), _dtype_code(out_dtype), _stream())
-    _lib.check(rc, "qm_rope_merge_qkv_grad")
-    return d_qkv
 
 
 def linear_backward(e2, packed_x, packed_w, T, I, O, hd_x, signs_x, hd_w, signs_w, hd_g, signs_g, mode, seeds, x_val_dtype,
