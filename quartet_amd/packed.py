@@ -130,15 +130,24 @@ def pack_absmax(x, hadamard_dim=32, sign_bits=0, stochastic=False, seed=0, tiled
 
 
 def from_operand_buffer(buffer, rows, cols, tiled, quantizer):
-    """The packed tensor inside one of the byte buffers that ``kernels.linear_forward`` returns (views, no copy): what
-    the layer keeps of x or of W for its backward pass.  `quantizer` is the forward quantizer that produced it."""
+    """The packed tensor inside one of the byte buffers that a layer keeps of x or of W (``PackedWeightCache.buffer``, what
+    ``kernels.linear_forward`` returns).  `quantizer` is the forward quantizer that produced it; `tiled` says how the buffer was
+    filled.  A layer fills tiled ones, of any extents (padded to 16 rows and 128 columns), unless out_features is not a
+    multiple of 8, a forward quantizer holds a dense rotation and an extent is not a multiple of 128, or an extent reaches
+    2^23.  Views into the buffer, no copy; of a padded one the codes and scales are row-major copies."""
     off = (ctypes.c_size_t * 3)()
     _lib.check(_lib.lib().qm_packed_operand_offsets(rows, cols, off), "qm_packed_operand_offsets")
 
-    def view(start, width):
+    def view(start, rows, width):
         return buffer[start:start + rows * width].view(rows, width)
-    return PackedTensor(view(off[0], cols // 2), view(off[1], cols // 32), view(off[2], cols // 8), rows, cols,
-                        "tiled" if tiled else "rowmajor", quantizer.hadamard_dim, quantizer.sign_bits, "quest")
+    rows_p, cols_p = -(-rows // 16) * 16, -(-cols // 128) * 128
+    if tiled and (rows_p, cols_p) != (rows, cols):
+        codes = K.untile_codes(view(off[0], rows_p, cols_p // 2))[:rows, :cols // 2].contiguous()
+        scales, tiled = view(off[1], rows, cols_p // 32)[:, :cols // 32].contiguous(), False
+    else:
+        codes, scales = view(off[0], rows, cols // 2), view(off[1], rows, cols // 32)
+    return PackedTensor(codes, scales, view(off[2], rows, cols // 8), rows, cols, "tiled" if tiled else "rowmajor", quantizer.hadamard_dim,
+                        quantizer.sign_bits, "quest")
 
 
 def pack_model_weights(model, tiled=False) -> Dict[str, PackedTensor]:

@@ -68,6 +68,23 @@ def test_views_into_the_operand_buffers(P, T, I, O):
     assert float((y.float() - ref).norm() / ref.norm()) < 5e-3
 
 
+@pytest.mark.parametrize("I,O,hd", [(1728, 640, 32), (128, 72, 32), (256, 384, 64), (64, 100, 32)])
+def test_packed_weight_that_a_layer_keeps(P, I, O, hd):
+    """The buffer in a layer's cache, whatever the extents pad it to, is the weight's own packed tensor."""
+    import quartet_amd as q
+    print(f"case packed weight of a layer {I}x{O} hd={hd}", flush=True)
+    make = lambda: q.QuestMXFP4Quantizer(hadamard_dim=hd)
+    layer = q.QuantizedLinear(I, O, bias=False, weight_quantizer=make(), activation_quantizer=make(),
+                              gradient_quantizer=q.AlbertTsengQuantizer(hadamard_dim=hd), device=DEV, dtype=torch.bfloat16,
+                              backward_scheme=q.BACKWARD_SCHEMES["Q(E)Q(Wt)t_Q(Et)Q(Xt)t"]())
+    q.enable_packed_weight_cache(layer)
+    with torch.no_grad():
+        layer(make_input(33, I, torch.bfloat16, seed=7).to(DEV))
+        got = P.from_operand_buffer(layer.packed_weight_cache.buffer, O, I, O % 8 == 0, layer.weight_quantizer).to_layout("rowmajor")
+        want = P.pack_quest(layer.weight.detach(), hd)
+    assert torch.equal(got.codes, want.codes) and torch.equal(got.scales, want.scales) and torch.equal(got.maskbits, want.maskbits)
+
+
 def test_quantized_checkpoint_of_a_model(P, tmp_path):
     """pack_model_weights -> file -> load: every block linear's packed weight, and the product of a packed activation
     with the reloaded packed weight equals the layer's own forward output."""

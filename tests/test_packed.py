@@ -140,3 +140,27 @@ def test_dequantize_needs_the_gpu():
     p = P.PackedTensor(torch.zeros(4, 16, dtype=torch.uint8), torch.zeros(4, 1, dtype=torch.uint8), None, 4, 32)
     with pytest.raises(QuartetHipError):
         p.dequantize()
+
+
+@pytest.mark.parametrize("rows,cols", [(33, 160), (16, 96), (40, 256), (32, 256)])
+def test_operand_buffer_of_padded_extents(rows, cols):
+    """A buffer filled by hand: 16 x 128 tiles of codes and rows of scales, both of the padded extents, then the mask."""
+    import ctypes
+
+    import quartet_amd as q
+    from quartet_amd import _lib
+    g = torch.Generator().manual_seed(rows)
+    rows_p, cols_p = -(-rows // 16) * 16, -(-cols // 128) * 128
+    codes = torch.randint(0, 256, (rows_p, cols_p // 2), generator=g, dtype=torch.uint8)
+    scales = torch.randint(0, 256, (rows_p, cols_p // 32), generator=g, dtype=torch.uint8)
+    mask = torch.randint(0, 256, (rows, cols // 8), generator=g, dtype=torch.uint8)
+    off = (ctypes.c_size_t * 3)()
+    assert _lib.lib().qm_packed_operand_offsets(rows, cols, off) == 0
+    buffer = torch.zeros(_lib.lib().qm_packed_operand_bytes(rows, cols), dtype=torch.uint8)
+    for r in range(rows_p):
+        for b in range(cols_p // 2):
+            buffer[off[0] + ((r // 16) * (cols_p // 128) + b // 64) * 1024 + r % 16 * 64 + b % 64] = codes[r, b]
+    buffer[off[1]:off[1] + scales.numel()] = scales.flatten()
+    buffer[off[2]:off[2] + mask.numel()] = mask.flatten()
+    t = P.from_operand_buffer(buffer, rows, cols, True, q.QuestMXFP4Quantizer()).to_layout("rowmajor")
+    assert torch.equal(t.codes, codes[:rows, :cols // 2]) and torch.equal(t.scales, scales[:rows, :cols // 32]) and torch.equal(t.maskbits, mask)
