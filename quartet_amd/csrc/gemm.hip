@@ -829,8 +829,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 // ---- which kernel serves a product ----------------------------------------------------------------------------------
 // Estimated durations in microseconds, fitted to 110 shapes of 0.2 to 900 GF (tiled operands; each kernel that serves the
 // shape was timed): mean error 13 %, and the fastest kernel is the one chosen but for 0.3 % of the time on average; with cuts
-// into K ranges (60 shapes, 2 to 16 ranges) but for 1.2 %.  All kernels give the same bits except a cut into K ranges, so
-// nothing but time hangs on the choice.
+// into K ranges (60 shapes, 2 to 16 ranges) but for 1.2 %.  All kernels chosen from here give the same bits except a cut into
+// K ranges, so nothing but time hangs on the choice.  (A layer's forward product of at most 64 tokens may run on gemm_rows.hip
+// instead, before this choice; its sums are in another order.)
 struct KernelCost {
     int bm, bn, per_cu;              // tile, resident workgroups per CU
     double step, shared, boundary;   // one K step of a workgroup alone on its CU; with n of them: n * shared; per tile

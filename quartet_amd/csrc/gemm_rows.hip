@@ -7,7 +7,8 @@
 // whose operands go straight from memory into the registers of v_mfma_scale_f32_16x16x128_f8f6f4, four steps ahead and
 // without a barrier: in the tiled layout one K step of 16 rows is 1 KiB in exactly that instruction's order (lane l: row
 // l % 16, block l / 16 of 32 codes).  The waves' partial sums meet in LDS and are added in wave order, so results are
-// reproducible; they differ from the tile kernels' in the order of the fp32 additions.
+// reproducible; they differ from the tile kernels' in the order of the fp32 additions, which shows where a row's group scales
+// span so many octaves that its sum is not exact in 24 bits (columns of 2^-8 .. 2^8: one bf16 result in 3 * 10^4).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

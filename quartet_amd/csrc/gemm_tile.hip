@@ -12,8 +12,8 @@
 //
 // What bounds it: at 256 x 128 the LDS reads of the K loop (1.5 x the 256 x 256 kernel's bytes per flop) and, for short
 // contractions, the tile boundary, which the neighbour workgroup on the same CU covers; the smaller tiles are latency-bound
-// and exist to put more workgroups on the chip.  Accumulation order over K is the same in every shape (and in gemm.hip's
-// kernels): results do not depend on the choice.
+// and exist to put more workgroups on the chip.  Accumulation order over K is the same in every shape and in gemm.hip's
+// kernels: results depend on the choice only where a product is cut into K ranges.  (gemm_rows.hip's order is its own.)
 //
 // The same kernel multiplies FP4 with an eight-bit (E5M2) B, which is how the error-only scheme contracts over the rows of a
 // packed operand (expand.hip): twice the bytes and twice the matrix cycles of B.  4096^3: 60 us, 8 waves of 128 x 64 on 256 x

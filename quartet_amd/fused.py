@@ -95,7 +95,8 @@ def swiglu_linear(layer, h12):
 def cross_entropy(logits, targets, ignore_index=-1):
     """F.cross_entropy(logits, targets, ignore_index=ignore_index) of logits [rows, classes].  Where nothing asks for a
     gradient and the result is an fp32 one (fp32 logits, or bf16 ones under autocast) the logits are read once by a kernel of
-    this package, which keeps log-probabilities in fp32 (the library rounds them to the logits' type)."""
+    this package, which keeps log-probabilities in fp32 (the library rounds them to the logits' type).  A target that is
+    neither a class nor `ignore_index` is an error of the caller that the device cannot raise: the kernel makes the loss NaN."""
     plain = (type(logits) is torch.Tensor and logits.is_cuda and not (torch.is_grad_enabled() and logits.requires_grad)
              and not (transformed() or torch.compiler.is_compiling()))
     if (plain and (logits.dtype == torch.float32 or (logits.dtype == torch.bfloat16 and torch.is_autocast_enabled("cuda")))

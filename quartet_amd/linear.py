@@ -154,7 +154,15 @@ def invalidate_packed_weights(model):
 
 class QuantizedLinear(nn.Linear):
     """nn.Linear whose forward is scheme(act_q(x), weight_q(W)); the bias parameter, if requested,
-    is never applied -- exactly as in the reference (the scheme calls F.linear(x, w, None))."""
+    is never applied -- exactly as in the reference (the scheme calls F.linear(x, w, None)).
+
+    A call's results can depend on how many tokens it has: on the packed path the product of at most 16 tokens, and of 17
+    to 64 where out_features <= 16 per compute unit (4096) or, up to 32, in_features <= 2048, adds its terms in another
+    order than that of more tokens.  FP4 codes times powers of two add up exactly in fp32 in any order as long as the
+    group scales of a row span few octaves -- no result differed for normal, heavy-tailed and outlier-ridden activations --
+    but with columns whose scales span 2^16 about one bf16 value in 3 * 10^4 rounds differently than the same row's in a
+    larger batch, and behind a further quantizer such a difference can become another FP4 code.  Calls of one token count
+    are reproducible bit for bit, with and without the packed-weight cache."""
 
     def __init__(self, in_features, out_features, weight_quantizer=None, activation_quantizer=None,
                  gradient_quantizer=None, backward_scheme=None, **kwargs):

@@ -201,7 +201,8 @@ class LlamaBlock(nn.Module):
 
 
 class Llama(nn.Module):
-    """Token ids [B, S] -> {"logits", "loss"} (llama.py:177-262)."""
+    """Token ids [B, S] -> {"logits", "loss"} (llama.py:177-262).  An evaluation's loss is NaN where a target is neither a
+    class nor -1 (fused.cross_entropy)."""
 
     def __init__(self, config):
         super().__init__()
