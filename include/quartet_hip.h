@@ -126,8 +126,9 @@ int qm_requantize_transposed_mxfp4_dense(const uint8_t* codes_in, const uint8_t*
  * a_layout / b_layout: layouts of a_codes / b_codes; QM_LAYOUT_TILED needs M and N multiples of 64 and
  * at least 256, and K % 128 == 0 (the shapes the 256x256-tile kernels serve).
  * workspace: optional scratch (NULL, 0 for none).  With qm_gemm_workspace_bytes(M, N, K) > 0 bytes of it, 16-byte
- * aligned, a product with few output tiles and a long K is cut into K ranges whose fp32 partial sums are added in
- * a fixed order (results are reproducible, but differ in rounding from the unsplit product).
+ * aligned, a product whose tiles leave compute units idle for a long K may be cut into K ranges whose fp32 partial sums
+ * are added in a fixed order (results are reproducible, but differ in rounding from the uncut product).  With less it may run
+ * whole.
  */
 size_t qm_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int qm_gemm_mxfp4_tn(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
@@ -268,11 +269,14 @@ int qm_dequantize_mxfp4(const uint8_t* codes, const uint8_t* scales, int64_t R, 
  *                     QM_GW_ROTATED: the same for gw and the weight quantizer (second product, B6; gw_dtype == mid_dtype)
  * codes_layout applies to every packed tensor inside; QM_LAYOUT_TILED needs T, I, O multiples of 128 (forward: T and O
  * multiples of 16, I of 128), QM_LAYOUT_PADDED takes any; both need O % 8 == 0.  T, I, O must be multiples of 32, and of the
- * Hadamard blocks along them, for the backward pass.
+ * Hadamard blocks along them, for the backward pass.  With the tiled layouts a product that contracts over 2^23 or more
+ * indices (T, I or O) runs where the 256 x 256 kernel serves it: the other extents multiples of 64 and >= 256, below 2^26.
+ * With the tiled layouts the forward product of at most 64 tokens may add its terms in another order than that of more
+ * (see qm_linear_decode, which gives the same bits).
  * The forward quantizer's masked inverse rotation is applied by the gradient product that feeds it where the kernel serving
  * the shape can: in the epilogue of the 256 x 256 kernel (bf16 mid_dtype, Hadamard block 32, for gw also gw_dtype ==
  * mid_dtype; see qm_gemm_mxfp4_tn_rotated), in the epilogue of the smaller tile kernels (bf16 mid_dtype, any Hadamard block,
- * any gw_dtype), or in the ordered reduction of a product cut into K ranges (Hadamard block 32, any mid_dtype / gw_dtype);
+ * any gw_dtype), or in the ordered reduction of a product cut into K ranges (any Hadamard block, mid_dtype and gw_dtype);
  * the last two with the arithmetic and roundings of the separate launches.  Elsewhere it is a launch of its own.
  */
 size_t qm_packed_operand_bytes(int64_t rows, int64_t cols);

@@ -46,7 +46,7 @@ qm::SignBits make_signs(const uint32_t* sign_bits, int hd) {
 
 extern "C" {
 
-int qm_version(void) { return 15; }
+int qm_version(void) { return 16; }
 
 const char* qm_last_error(void) { return g_last_error; }
 
