@@ -804,9 +804,10 @@ struct RmsNormProducer {
     // 8 KiB of LDS per wave, through which fp32 rows and the gain pass on their way to the lanes that own their groups: an
     // instruction then reads or writes whole 128-byte lines, where a lane's own 128 bytes are eight 16-byte pieces, each
     // instruction touching 64 lines, which the address unit takes one by one.  Slot 8 l + (q ^ l % 8) holds piece q of lane l's
-    // group: slot-ordered and group-ordered accesses both spread over all banks.  With the residual sum: 4096 x 640 11.2 ->
-    // 9.3 us, 16384 x 1536 53 -> 48, 32768 x 1024 88 -> 70, 16384 x 4096 163 -> 153 (two passes); 512 x 4096 is latency, 11 us
-    // either way.  Requests under per-lane predicates instead of clamped ones: 16384 x 1536 75 us.
+    // group: slot-ordered and group-ordered accesses both spread over all banks.  With the residual sum, inputs cycled through
+    // memory: 4096 x 640 11.7 -> 9.9 us, 16384 x 1536 62 -> 57 (4.7 TB/s; 65 -> 60 inside a layer's step), 32768 x 1024 88 -> 75,
+    // 16384 x 4096 166 -> 156 (two passes); 512 x 4096 is latency, 11 us either way.  Requests under per-lane predicates instead
+    // of clamped ones cost half as much again.
     typedef float v4 __attribute__((ext_vector_type(4)));
     __device__ __forceinline__ static v4* area() { return reinterpret_cast<v4*>(job_lds) + (threadIdx.x >> 6) * 512; }
     __device__ __forceinline__ static void read_group(int of_lane, float (&v)[32]) {
@@ -937,8 +938,9 @@ template <typename T>
 struct SwiGluProducer {
     static constexpr int kOutDtype = sizeof(T) == 2 ? BF16 : F32;
     // bf16: whole lines through 8 KiB of LDS per wave, as in the RMSNorm producer; a group is four pieces here, slot
-    // 4 l + (q ^ l / 4 % 4) holds piece q of lane l's group.  16384 x 4096 73 -> 65 us, 32768 x 4096
-    // 141 -> 120; 16384 x 1536 35 either way, up to 4096 x 1728 (11 us) latency
+    // 4 l + (q ^ l / 4 % 4) holds piece q of lane l's group.  Inputs cycled through memory: 16384 x 4096 73 -> 65 us (4.8 TB/s; 76
+    // inside a layer's step), 32768 x 4096 141 -> 125; 16384 x 1536 33 either way, up to
+    // 4096 x 1728 (11 us) latency
     static constexpr bool kStaged = sizeof(T) == 2;
     static constexpr int kLds = kStaged ? 4 * 512 * 16 : 0;
     const T* h12;  // [rows, 2 cols]: up, then gate
