@@ -608,14 +608,23 @@ def counters_to_json(fetch_dir, write_dir, sq_dir=None):
         copies = [v for k, vs in agg.items() if "copyBuffer" in k for v in vs]
         return copy_bytes / max(copies)
     fu, wu = unit(fetch), unit(write)
-    groups = {"gemm_mxfp4_tn": lambda k: "gemm_mxfp4_tn" in k and "splitk" not in k and "false, true>" not in k,
+
+    def jobs(k):
+        """Names of the jobs that share a job_kernel's grid."""
+        return re.findall(r"qm::(\w+Job)<", k.split("(")[0]) if "qm::job_kernel<" in k else []
+
+    def product(k):
+        """The persistent product's template arguments: element type, stamps, rotation in the epilogue, ragged rows."""
+        m = re.search(r"gemm_mxfp4_tn_big4_kernel<([^>]*)>", k)
+        return m.group(1).split(", ") if m else None
+    groups = {"gemm_mxfp4_tn": lambda k: product(k) is not None and product(k)[2] == "false",
               # the instantiation with the masked inverse rotation in its epilogue (the step's two gradient products)
-              "gemm_mxfp4_tn_rotated": lambda k: "gemm_mxfp4_tn_big4_kernel" in k and "false, true>" in k,
-              "quantize_x_quest_rtn_mask_alone": lambda k: k.startswith("void qm::job_kernel<qm::RowmajorTiledJob") or k.startswith("qm::job_kernel<qm::RowmajorTiledJob"),
-              "forward_quantizer_pair": lambda k: "job_pair_kernel<qm::RowmajorTiledJob" in k,
-              "gradient_quantizer_pair": lambda k: "job_pair_kernel<qm::TransposedJob" in k,
-              "requantizer_pair": lambda k: "job_pair_kernel<qm::RequantJob" in k,
-              "inverse_rotation_pair": lambda k: "job_pair_kernel<qm::HadamardBwdJob" in k}
+              "gemm_mxfp4_tn_rotated": lambda k: product(k) is not None and product(k)[2] == "true",
+              "quantize_x_quest_rtn_mask_alone": lambda k: jobs(k) == ["RowmajorTiledJob"],
+              "forward_quantizer_pair": lambda k: jobs(k) == ["RowmajorTiledJob"] * 2,
+              "gradient_quantizer_pair": lambda k: jobs(k) == ["TransposedJob", "RowmajorTiledJob"],
+              "requantizer_pair": lambda k: jobs(k) == ["RequantJob"] * 2,
+              "inverse_rotation_pair": lambda k: jobs(k) == ["HadamardBwdJob"] * 2}
     out = {}
     for name, match in groups.items():
         f = [v for k, vs in fetch.items() if match(k) for v in vs]
