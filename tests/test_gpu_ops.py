@@ -190,3 +190,15 @@ def test_cross_entropy_against_float64(rows, classes, dtype):
     x = logits.to("cuda:0").requires_grad_(True)
     assert cross_entropy(x, t).grad_fn is not None
     assert cross_entropy(x.detach(), t).dtype == dtype
+
+
+@pytest.mark.parametrize("target", [1024, -2, 2 ** 40, -2 ** 63])
+def test_cross_entropy_of_a_target_that_is_no_class(target):
+    """The kernel reads no logit for it; the loss is NaN, whatever the other rows are."""
+    from quartet_amd.fused import cross_entropy
+    x, t = torch.randn(5, 1024, device="cuda:0"), torch.arange(5, device="cuda:0")
+    with torch.no_grad():
+        assert torch.isfinite(cross_entropy(x, t))
+        t[3] = target
+        assert torch.isnan(cross_entropy(x, t))
+        assert torch.isfinite(cross_entropy(x, t, ignore_index=target))
