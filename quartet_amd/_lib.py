@@ -164,11 +164,13 @@ def host():
 
         import torch  # noqa: F401  (its libraries must be loaded before the extension's)
 
+        from . import one_node
         from .linear import _error_draws, _gradient_draws
         spec = importlib.util.spec_from_file_location("_quartet_host", HOST_PATH)
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)
         module.bind(QuartetHipError, _gradient_draws, _error_draws)
+        one_node.use(module.transformed)
         _host = module
     return _host
 

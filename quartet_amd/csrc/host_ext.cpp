@@ -9,6 +9,8 @@
 // torch's host generator and seeds from the `random` module, in the order e, W^T, e^T, x^T, through one callback.
 #include <torch/extension.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/forward_grad.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
@@ -625,6 +627,14 @@ py::int_ sign_flips(int64_t hd) {
     return py::reinterpret_steal<py::int_>(_PyLong_FromByteArray(raw, sizeof(raw), 1, 0));
 }
 
+// quartet_amd.one_node.transformed() in one call without arguments (0.03 us; every layer call asks)
+PyObject* transformed(PyObject*, PyObject*) {
+    const bool yes = torch::jit::tracer::isTracing() || torch::autograd::ForwardADLevel::try_get_by_idx(0) ||
+                     c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
+    return PyBool_FromLong(yes);
+}
+PyMethodDef transformed_def = {"transformed", transformed, METH_NOARGS, nullptr};
+
 void bind(py::object error_class, py::object draw, py::object error_draw) {
     g_error_class = error_class.release().ptr();
     g_draw = draw.release().ptr();
@@ -641,4 +651,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("rope_qkv", &rope_qkv);
     m.def("quantizer", &quantizer);
     m.def("sign_flips", &sign_flips);
+    m.add_object("transformed", py::reinterpret_steal<py::object>(PyCFunction_New(&transformed_def, nullptr)));
 }

@@ -12,9 +12,9 @@ production configuration, uses another Hadamard block than 32, or the tensors ar
 import torch
 import torch.nn.functional as F
 
-from . import _lib, kernels
+from . import _lib, kernels, one_node
 from .linear import QuantizedLinear, _cached_weight, _dense
-from .one_node import one_node, transformed
+from .one_node import as_one_node
 
 _KERNEL_DTYPES = (torch.float32, torch.bfloat16)
 
@@ -25,12 +25,12 @@ def _layer_is_fusable(layer, x):
             and layer.weight.dtype in _KERNEL_DTYPES)
 
 
-@one_node
+@as_one_node
 def _rope(qkv, table, n_head):
     return _lib.host().rope_qkv(qkv, table, n_head)
 
 
-@one_node
+@as_one_node
 def _norm_linear(x, add, gain, weight, eps, a_q, w_q, g_q, cache, pass_input):
     key, packed_w = _cached_weight(x, weight, a_q, w_q, g_q, cache)
     y, x_next, packed_w = _lib.host().norm_linear(x, add, gain, weight, eps, a_q.sign_bits, w_q.hadamard_dim, w_q.sign_bits, g_q.hadamard_dim, g_q,
@@ -40,7 +40,7 @@ def _norm_linear(x, add, gain, weight, eps, a_q, w_q, g_q, cache, pass_input):
     return (y, x_next) if (pass_input or add is not None) else y
 
 
-@one_node
+@as_one_node
 def _swiglu_linear(h12, weight, a_q, w_q, g_q, cache):
     key, packed_w = _cached_weight(h12, weight, a_q, w_q, g_q, cache)
     y, packed_w = _lib.host().swiglu_linear(h12, weight, a_q.sign_bits, w_q.hadamard_dim, w_q.sign_bits, g_q.hadamard_dim, g_q, packed_w,
@@ -98,7 +98,7 @@ def cross_entropy(logits, targets, ignore_index=-1):
     this package, which keeps log-probabilities in fp32 (the library rounds them to the logits' type).  A target that is
     neither a class nor `ignore_index` is an error of the caller that the device cannot raise: the kernel makes the loss NaN."""
     plain = (type(logits) is torch.Tensor and logits.is_cuda and not (torch.is_grad_enabled() and logits.requires_grad)
-             and not (transformed() or torch.compiler.is_compiling()))
+             and not (one_node.transformed() or torch.compiler.is_compiling()))
     if (plain and (logits.dtype == torch.float32 or (logits.dtype == torch.bfloat16 and torch.is_autocast_enabled("cuda")))
             and logits.dim() == 2 and logits.shape[1] > 0 and targets.dim() == 1 and targets.dtype == torch.int64
             and targets.device == logits.device and targets.shape[0] == logits.shape[0]):

@@ -16,7 +16,7 @@ import torch
 
 from .. import _lib
 from .. import kernels as K
-from ..one_node import one_node
+from ..one_node import as_one_node
 from .base import BaseQuantizer
 
 
@@ -231,12 +231,12 @@ class QuestMXFP4Quantizer(_HadamardQuantizer):
         return _quest_quantize(x, self.hadamard_dim, self.sign_bits)
 
 
-@one_node
+@as_one_node
 def _quest_quantize(x, hadamard_dim, sign_bits):
     return _lib.host().quantizer(x, hadamard_dim, sign_bits, K.QM_QUEST_RTN, 0, 1.0)
 
 
-@one_node
+@as_one_node
 def _absmax_quantize(x, hadamard_dim, sign_bits, stochastic, post_scale):
     """mxfp4.py:15-34: absmax/(3/4)-scaled RTN or SR forward, unmasked straight-through backward."""
     mode, seed = (K.QM_ABSMAX_SR, _fresh_seed()) if stochastic else (K.QM_ABSMAX_RTN, 0)

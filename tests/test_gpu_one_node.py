@@ -50,7 +50,7 @@ def _entry(name):
         return _Call(lambda h: swiglu_linear(layer, h), layer), inputs(512)
     if name == "rope":
         table = rotary_table(32, 64).to(dev)
-        return lambda x: torch.cat([t.flatten() for t in rope_qkv(x.view(1, 64, 192), table, 2)]), inputs(192, torch.float32)
+        return _Call(lambda x: torch.cat([t.flatten() for t in rope_qkv(x.view(1, 64, 192), table, 2)])), inputs(192, torch.float32)
     return (q.QuestMXFP4Quantizer() if name == "quest" else q.AlbertTsengQuantizer(stochastic=True)), inputs(256)
 
 
@@ -62,9 +62,12 @@ def _seeded():
 @pytest.mark.parametrize("grad", [False, True])
 @pytest.mark.parametrize("name", ENTRIES)
 def test_traced_calls_run_their_kernels_on_replay(name, grad):
+    import quartet_amd as q
     call, make = _entry(name)
+    q.enable_packed_weight_cache(call)      # a packed weight from before the trace is in place
     print(f"case trace {name} grad={grad}", flush=True)
     with torch.set_grad_enabled(grad):
+        call(make(1))
         traced = torch.jit.trace(call, (make(1).requires_grad_(grad),), check_trace=False)
         for seed in (2, 3):
             results = []

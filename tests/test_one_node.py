@@ -8,7 +8,7 @@ from torch.autograd import forward_ad
 
 import quartet_amd as q
 from quartet_amd import _lib
-from quartet_amd.one_node import one_node
+from quartet_amd.one_node import as_one_node
 
 
 class _Host:
@@ -52,12 +52,15 @@ def test_a_trace_runs_the_call_again(host, make):
 
 
 @pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning")
-def test_a_trace_follows_the_weight(host):
+@pytest.mark.parametrize("filled", [False, True])
+def test_a_trace_follows_the_weight(host, filled):
     """A replay looks the packed weight up again: nothing of the traced call's weight is kept."""
     layer = _layer()
     q.enable_packed_weight_cache(layer)
     x = torch.randn(8, 64)
     with torch.no_grad():
+        if filled:
+            layer(x)
         traced = torch.jit.trace(layer, (x,), check_trace=False)
         layer.weight.mul_(-2.0)
         assert torch.equal(traced(x), layer(x))
@@ -93,15 +96,16 @@ def test_function_transforms_are_refused(host, make):
 @pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning")
 def test_a_trace_is_differentiable():
     """Two outputs, one of them left out of the loss, an argument that is no tensor, and one without a gradient."""
-    @one_node
+    @as_one_node
     def call(x, add, factor):
         y = x * x * factor + add
         return y, x * 5.0
 
     def net(x, add):
         return call(x, add, 3.0)
-    x, add = torch.randn(4, 6), torch.randn(4, 6)
+    x, add = torch.randn(4, 6).requires_grad_(True), torch.randn(4, 6)
     traced = torch.jit.trace(net, (x, add), check_trace=False)
+    assert not any(node.kind() == "prim::Constant" and node.output().type().kind() == "TensorType" for node in traced.graph.nodes())
     for pick in (0, 1, None):
         a, b = (torch.randn(4, 6, generator=torch.Generator().manual_seed(5)).requires_grad_(True) for _ in range(2))
         for t, f in ((a, traced), (b, net)):
