@@ -585,13 +585,14 @@ struct QuantizerFn : Function<QuantizerFn> {
         if (ctx) {
             if (quest) ctx->save_for_backward({mask});
             ctx->saved_data["shape"] = x.sizes().vec();
-            ctx->saved_data["meta"] = std::vector<int64_t>{rows, cols, a.hd, (int64_t)x.scalar_type(), a.signs.w[0], a.signs.w[1], a.signs.w[2], a.signs.w[3]};
+            ctx->saved_data["meta"] = std::vector<int64_t>{rows, cols, a.hd, (int64_t)x.scalar_type(), a.signs.w[0], a.signs.w[1], a.signs.w[2], a.signs.w[3], quest};
         }
         return deq.view(x.sizes());
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
-        const auto saved = ctx->get_saved_variables();
         const auto m = ctx->saved_data["meta"].toIntVector();
+        // asked for only where something was saved: a graph that keeps no tensor can be gone through again
+        const Tensor mask = m[8] ? ctx->get_saved_variables()[0] : Tensor();
         const at::ScalarType x_dtype = (at::ScalarType)m[3];
         Signs signs;
         for (int i = 0; i < 4; ++i) signs.w[i] = (uint32_t)m[4 + i];
@@ -602,7 +603,7 @@ struct QuantizerFn : Function<QuantizerFn> {
         const at::ScalarType out_dtype = low ? at::kBFloat16 : g.scalar_type();
         Tensor out = at::empty({m[0], m[1]}, g.options().dtype(out_dtype));
         check(qm_masked_hadamard_bwd(g.data_ptr(), dtype_code(g.scalar_type()), m[0], m[1], (int)m[2], dtype_code(low ? at::kBFloat16 : x_dtype),
-                                     signs.data(), saved.empty() ? nullptr : saved[0].data_ptr<uint8_t>(), out.data_ptr(), dtype_code(out_dtype),
+                                     signs.data(), m[8] ? mask.data_ptr<uint8_t>() : nullptr, out.data_ptr(), dtype_code(out_dtype),
                                      stream_of(g)),
               "qm_masked_hadamard_bwd");
         return {out.view(ctx->saved_data["shape"].toIntVector()).to(x_dtype), Tensor()};

@@ -655,6 +655,21 @@ def test_error_only_scheme_keeps_the_library_path_for_fp32_products(q, monkeypat
     assert torch.isfinite(x.grad).all() and torch.isfinite(layer.weight.grad).all()
 
 
+@pytest.mark.parametrize("name", ["AlbertTsengQuantizer", "AlignedAlbertTsengQuantizer", "QuestMXFP4Quantizer"])
+def test_second_backward_of_a_quantizer_module(q, name):
+    """The absmax quantizers keep no tensor for their backward, so it can run again; the clip mask of the other is released."""
+    x = torch.randn(8, 64, device="cuda:0", requires_grad=True)
+    y = q.QUANTIZER_CLASSES[name]()(x)
+    y.backward(torch.ones_like(y))
+    first, x.grad = x.grad, None
+    if name == "QuestMXFP4Quantizer":
+        with pytest.raises(RuntimeError, match="second time"):
+            y.backward(torch.ones_like(y))
+    else:
+        y.backward(torch.ones_like(y))
+        assert torch.equal(x.grad, first)
+
+
 @pytest.mark.parametrize("kind", ["forward", "pre", "backward", "global", "instance"])
 def test_error_only_scheme_calls_its_modules_where_somebody_listens(q, kind):
     """Hooks on the quantizers and on the scheme fire, and a forward set on an instance runs, as in the module path; without
