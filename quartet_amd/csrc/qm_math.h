@@ -72,6 +72,14 @@ QM_HD float div_four_thirds(float g) {
 constexpr float kInvFourThirdsLo = -0x1.8p-26f;
 QM_HD float div_four_thirds_fast(float g) { return __builtin_fmaf(g, 0.75f, g * kInvFourThirdsLo); }
 
+// The strict-threshold rule below on a convert that rounds ties to even: it differs on the ties at 0.75, 1.75 and 3.5 (times a
+// power of two), which that convert rounds up.  Their significands are 1.5 and 1.75, those of the four other ties 1.0 and 1.25.
+// v - v * 3 * 2^-26, rounded once, moves a value with significand s by s * 0.375 units in its last place before rounding: by
+// nothing below s = 4/3 (at s = 1 by one of the half-sized units under it) and by one unit toward zero from s = 4/3 on.  So the
+// three ties end up just below themselves, the value behind each of them on the tie (rounded up, as it should be), and no other
+// value changes sides.  Zeros of either sign come out as +0.
+QM_HD float below_ties(float v) { return __builtin_fmaf(v, -0x1.8p-25f, v); }
+
 // RTN onto the E2M1 magnitudes {0,.5,1,1.5,2,3,4,6}: strict '>' against the seven midpoints,
 // i.e. ties go toward zero and anything above 5 saturates at 6 (mxfp4_triton.py:131-159).
 QM_HD int rtn_code(float A) {
@@ -134,6 +142,14 @@ QM_HD float silu_fixed(float x) { return x / (1.0f + exp_fixed(-x)); }
 struct Philox4 {
     uint32_t w[4];
 };
+// a ^ b ^ c: one instruction on the GPU (the compiler emits two where an operand is wave-uniform)
+QM_HD uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return (uint32_t)__builtin_amdgcn_bitop3_b32((int)a, (int)b, (int)c, 0x96);
+#else
+    return a ^ b ^ c;
+#endif
+}
 template <int ROUNDS>
 QM_HD Philox4 philox4x32(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0, uint32_t k1) {
 #pragma unroll
@@ -141,7 +157,7 @@ QM_HD Philox4 philox4x32(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uin
         // one 32x32->64 multiply each (v_mad_u64_u32 on the GPU)
         const uint64_t p0 = (uint64_t)0xD2511F53u * c0;
         const uint64_t p1 = (uint64_t)0xCD9E8D57u * c2;
-        const uint32_t n0 = (uint32_t)(p1 >> 32) ^ c1 ^ k0, n2 = (uint32_t)(p0 >> 32) ^ c3 ^ k1;
+        const uint32_t n0 = xor3((uint32_t)(p1 >> 32), c1, k0), n2 = xor3((uint32_t)(p0 >> 32), c3, k1);
         c0 = n0; c1 = (uint32_t)p1; c2 = n2; c3 = (uint32_t)p0;
         k0 += 0x9E3779B9u;
         k1 += 0xBB67AE85u;

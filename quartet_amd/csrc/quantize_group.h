@@ -45,8 +45,6 @@ struct GroupCodes {
     float deq_scale;      // what a code value is multiplied by in the de-quantized tensor
 };
 
-#define kNegTiny (u2f(0x80000001u))  // -2^-149
-
 // v_cvt_scalef32_sr_pk_fp4_f32 replaces byte SEL of its destination and keeps the other three, but the
 // compiler builtin of this toolchain does not tie the destination to its `old` operand (the untouched bytes
 // come back as whatever the allocated register held), so the instruction is issued directly.
@@ -58,26 +56,32 @@ __device__ __forceinline__ void sr_convert_pair(uint32_t& dst, v2f pair, uint32_
     else asm("v_cvt_scalef32_sr_pk_fp4_f32 %0, %1, %2, %3 op_sel:[0,0,1,1]" : "+v"(dst) : "v"(pair), "v"(rnd), "v"(scale));
 }
 
-// ties-toward-zero via the round-to-nearest-even convert (see the file comment)
-__device__ __forceinline__ float tie_nudge(float v) {
-    return u2f(__builtin_elementwise_sub_sat(f2u(v), 1u) | 1u);
+// the integer form of below_ties() (the bit pattern b becomes (b - 1) | 1): for groups with infinite statistics, where the
+// fused form would make an infinity a NaN
+__device__ __forceinline__ float below_ties_any(float v) {
+    const float w = v + 0.0f;   // both zeros become +0
+    return u2f(__builtin_elementwise_sub_sat(f2u(w), 1u) | 1u);
 }
 
+// n: the NEGATED rotated group.  The sign rule "negative unless g > 0" makes both zeros negative; on the negated values it reads
+// "positive unless n < 0", and the arithmetic in front of the converts turns zeros of either sign into +0 by itself (x y + z
+// with two exact zeros of opposite sign), so it costs one XOR of the sign bits of eight codes.  Everything else is symmetric.
 template <int MODE, bool WANT_MASK>
-__device__ __forceinline__ void quantize_group_regs(const float (&g)[32], uint64_t seed, int64_t group_index,
+__device__ __forceinline__ void quantize_group_regs(const float (&n)[32], uint64_t seed, int64_t group_index,
                                                     GroupCodes& o) {
     constexpr bool kQuest = (MODE == QUEST_RTN || MODE == QUEST_SR);
     constexpr bool kSR = (MODE == ABSMAX_SR || MODE == QUEST_SR);
     float hw_scale;   // power of two the convert divides by
-    uint32_t thr_bits;  // bit pattern of 6 * scale: |g| < thr  <=>  |t| < 6
+    float thr;        // 6 * scale: |n| < thr  <=>  |t| < 6
     float t[32];
     bool all_zero = false;
+    [[maybe_unused]] bool finite = true;
     if constexpr (kQuest) {
         float sq[32];
 #pragma unroll
-        for (int i = 0; i < 32; ++i) sq[i] = g[i] * g[i];
+        for (int i = 0; i < 32; ++i) sq[i] = n[i] * n[i];
         const float ms = tree_sum32(sq) * 0.03125f;
-        const float m = tree_sum32(g) * 0.03125f;
+        const float m = tree_sum32(n) * 0.03125f;
         const float mm = m * m;
         float var = ms - mm;
         var = var > 0.0f ? var : 0.0f;
@@ -89,13 +93,14 @@ __device__ __forceinline__ void quantize_group_regs(const float (&g)[32], uint64
         o.scale_byte = (uint32_t)(E + 127);
         hw_scale = pow2i(E);
         o.deq_scale = hw_scale;
-        thr_bits = f2u(6.0f * hw_scale);
+        thr = 6.0f * hw_scale;
+        finite = ms < __builtin_inff();
 #pragma unroll
-        for (int i = 0; i < 32; ++i) t[i] = g[i];
+        for (int i = 0; i < 32; ++i) t[i] = n[i];
     } else {
         float a = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 32; ++i) a = fmaxf(a, fabsf(g[i]));
+        for (int i = 0; i < 32; ++i) a = fmaxf(a, fabsf(n[i]));
         all_zero = (a == 0.0f);
         int k = (int)((f2u(a) >> 23) & 0xffu) - 129;
         k = k < -127 ? -127 : (k > 127 ? 127 : k);
@@ -103,7 +108,7 @@ __device__ __forceinline__ void quantize_group_regs(const float (&g)[32], uint64
         hw_scale = pow2i(k);
         o.deq_scale = scale_pow2(kFourThirds, k);
         // |t| < 6 with t = RN(g 2^-k / d): evaluated on the quotient h = RN(g / d) against 6 * 2^k
-        thr_bits = f2u(6.0f * hw_scale);
+        thr = 6.0f * hw_scale;
         // t = RN(RN(g 2^-k) / d) by definition.  For a group whose maximum is at least 2^-60 this is RN(g / d) scaled by
         // 2^-k inside the convert: the two-operation quotient is exact for |g| >= 2^-100, and a smaller element lies
         // below 2^-38 of the scale, so its code is a zero whose sign is the element's own whatever the quotient's last
@@ -111,42 +116,31 @@ __device__ __forceinline__ void quantize_group_regs(const float (&g)[32], uint64
         // definition literally, with a true division, and hands the convert an already scaled value.
         if (__builtin_expect(a < 0x1p-60f && !all_zero, 0)) {
 #pragma unroll
-            for (int i = 0; i < 32; ++i) t[i] = scale_pow2(g[i], -k) / kFourThirds;
+            for (int i = 0; i < 32; ++i) t[i] = scale_pow2(n[i], -k) / kFourThirds + 0.0f;
             hw_scale = 1.0f;
-            thr_bits = f2u(6.0f);
+            thr = 6.0f;
         } else {
 #pragma unroll
-            for (int i = 0; i < 32; ++i) t[i] = div_four_thirds_fast(g[i]);
+            for (int i = 0; i < 32; ++i) t[i] = div_four_thirds_fast(n[i]);   // zeros of either sign: +0
         }
     }
     o.keep = 0u;
     if constexpr (WANT_MASK) {
-        // clip mask, most significant element first so that element 0 lands in bit 0
-        // one compare into the carry flag and one add-with-carry (keep = 2 keep + flag) per element, sixteen
-        // elements per statement (the operand limit of an asm statement)
-        uint32_t keep = 0u;
-        const float thr = u2f(thr_bits);
-#define QM_KEEP_BIT(N) "v_cmp_lt_f32_e64 vcc, |%" #N "|, %17\n\tv_addc_co_u32_e32 %0, vcc, %0, %0, vcc\n\t"
-#define QM_KEEP_16(B)                                                                                               \
-    asm(QM_KEEP_BIT(16) QM_KEEP_BIT(15) QM_KEEP_BIT(14) QM_KEEP_BIT(13) QM_KEEP_BIT(12) QM_KEEP_BIT(11) QM_KEEP_BIT(10) \
-        QM_KEEP_BIT(9) QM_KEEP_BIT(8) QM_KEEP_BIT(7) QM_KEEP_BIT(6) QM_KEEP_BIT(5) QM_KEEP_BIT(4) QM_KEEP_BIT(3)        \
-        QM_KEEP_BIT(2) QM_KEEP_BIT(1)                                                                                   \
-        : "+v"(keep)                                                                                                    \
-        : "v"(t[(B)]), "v"(t[(B) + 1]), "v"(t[(B) + 2]), "v"(t[(B) + 3]), "v"(t[(B) + 4]), "v"(t[(B) + 5]),             \
-          "v"(t[(B) + 6]), "v"(t[(B) + 7]), "v"(t[(B) + 8]), "v"(t[(B) + 9]), "v"(t[(B) + 10]), "v"(t[(B) + 11]),       \
-          "v"(t[(B) + 12]), "v"(t[(B) + 13]), "v"(t[(B) + 14]), "v"(t[(B) + 15]), "v"(thr)                              \
-        : "vcc")
-        QM_KEEP_16(16);
-        QM_KEEP_16(0);
-#undef QM_KEEP_16
-#undef QM_KEEP_BIT
-        o.keep = all_zero ? 0u : keep;
+        // clip mask, most significant element first so that element 0 lands in bit 0: the sign of |t| - 6 scale (never set for
+        // a NaN; |t| = 6 scale gives +0), shifted in by a funnel shift.  The subtraction issues at twice the rate of a compare
+        // and nothing passes through the carry flag: 218 cycles a group against 286 for compare and add-with-carry.  Two
+        // chains of sixteen: the shifts of one depend on each other.
+        uint32_t lo = 0u, hi = 0u;
+#pragma unroll
+        for (int i = 15; i >= 0; --i) {
+            lo = __builtin_amdgcn_alignbit(lo, f2u(fabsf(t[i]) - thr), 31);
+            hi = __builtin_amdgcn_alignbit(hi, f2u(fabsf(t[i + 16]) - thr), 31);
+        }
+        o.keep = all_zero ? 0u : (hi << 16) | lo;
     }
 
     // the converts' byte selector must be a literal, hence the macros
-#define QM_RTN_PAIR(B)                                                                                   \
-    w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, tie_nudge(t[wi * 8 + 2 * (B)] + kNegTiny),           \
-                                                 tie_nudge(t[wi * 8 + 2 * (B) + 1] + kNegTiny), hw_scale, (B));
+#define QM_RTN_PAIR(B) w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, below(t[wi * 8 + 2 * (B)]), below(t[wi * 8 + 2 * (B) + 1]), hw_scale, (B));
     // element j of a Philox call (16 elements): its random field is the top 22 bits of word j/4 rotated left by
     // 8 * (j%4).  The convert reads the field of a pair's first element from bits 31..10 of its random operand and that of
     // the second from bits 30..9, so the even element's operand is the word rotated by 0 or 16 bits and the odd element's
@@ -156,18 +150,26 @@ __device__ __forceinline__ void quantize_group_regs(const float (&g)[32], uint64
         const uint32_t pw = ph.w[(J0) >> 2];                                                              \
         const uint32_t r_even = ((J0) & 3) == 0 ? pw : __builtin_amdgcn_alignbit(pw, pw, 16);             \
         const uint32_t r_odd = __builtin_amdgcn_alignbit(pw, pw, ((J0) & 3) == 0 ? 25 : 9);               \
-        const v2f pr = {t[wi * 8 + 2 * (B)] + kNegTiny, t[wi * 8 + 2 * (B) + 1] + kNegTiny};              \
+        const v2f pr = {t[wi * 8 + 2 * (B)], t[wi * 8 + 2 * (B) + 1]};                                    \
         sr_convert_pair<(B)>(even, pr, r_even, hw_scale);                                                 \
         sr_convert_pair<(B)>(odd, pr, r_odd, hw_scale);                                                   \
     }
     if constexpr (!kSR) {
+        const auto convert = [&](auto below) {
 #pragma unroll
-        for (int wi = 0; wi < 4; ++wi) {
-            uint32_t w = 0u;
-            QM_RTN_PAIR(0) QM_RTN_PAIR(1) QM_RTN_PAIR(2) QM_RTN_PAIR(3)
-            o.w[wi] = w;
-        }
+            for (int wi = 0; wi < 4; ++wi) {
+                uint32_t w = 0u;
+                QM_RTN_PAIR(0) QM_RTN_PAIR(1) QM_RTN_PAIR(2) QM_RTN_PAIR(3)
+                o.w[wi] = w ^ 0x88888888u;
+            }
+        };
+        if (__builtin_expect(finite, 1)) convert([](float v) { return below_ties(v); });
+        else convert([](float v) { return below_ties_any(v); });
     } else {
+        if constexpr (kQuest) {
+#pragma unroll
+            for (int i = 0; i < 32; ++i) t[i] += 0.0f;   // both zeros: +0
+        }
         Philox4 ph;
 #pragma unroll
         for (int wi = 0; wi < 4; ++wi) {
@@ -176,7 +178,8 @@ __device__ __forceinline__ void quantize_group_regs(const float (&g)[32], uint64
             uint32_t even = 0u, odd = 0u;  // converts driven by the even / odd element's random byte
             if ((wi & 1) == 0) { QM_SR_PAIR(0, 0) QM_SR_PAIR(1, 2) QM_SR_PAIR(2, 4) QM_SR_PAIR(3, 6) }
             else { QM_SR_PAIR(0, 8) QM_SR_PAIR(1, 10) QM_SR_PAIR(2, 12) QM_SR_PAIR(3, 14) }
-            o.w[wi] = (even & 0x0f0f0f0fu) | (odd & 0xf0f0f0f0u);
+            // low nibbles from `even`, high ones from `odd`, sign bits back (n is negated)
+            o.w[wi] = (uint32_t)__builtin_amdgcn_bitop3_b32((int)even, (int)odd, 0x0f0f0f0f, 0xe4) ^ 0x88888888u;
         }
     }
 #undef QM_RTN_PAIR
@@ -237,12 +240,12 @@ struct GroupOut {
     void* dequant;       // [n_groups * 32] of T or null
 };
 
-// x @ H for one chunk of 32: butterfly, then hd^-1/2 with the column sign folded in (wave-uniform)
+// -(x @ H) for one chunk of 32 (what quantize_group_regs takes): butterfly, then -hd^-1/2 with the column sign folded in
 __device__ __forceinline__ void rotate_group(float (&v)[32], float c, uint32_t sign_word, bool rotate = true) {
     if (rotate) butterfly32(v);  // uniform; without it (c = 1, no signs) the group passes through unchanged
 #pragma unroll
     for (int j = 0; j < 32; ++j) {
-        const float cj = u2f(f2u(c) ^ (((sign_word >> j) & 1u) << 31));  // wave-uniform: stays in scalar registers
+        const float cj = u2f(f2u(-c) ^ (((sign_word >> j) & 1u) << 31));  // wave-uniform: stays in scalar registers
         v[j] = v[j] * cj;
     }
 }

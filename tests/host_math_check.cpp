@@ -77,6 +77,31 @@ int main() {
     }
     if (rtn_code(1e9f) != 7 || sr_code(7.5f, 0.f) != 7) fail("saturation", 0);
 
+    // below_ties() in front of a convert that rounds ties to even is the strict-threshold rule: every value of the binades that
+    // hold the thresholds, both signs of zero, and in every other binade the values at and next to a threshold's significand
+    {
+        const auto to_even = [](float a) {
+            return (a > 0.25f) + (a >= 0.75f) + (a > 1.25f) + (a >= 1.75f) + (a > 2.5f) + (a >= 3.5f) + (a > 5.0f);
+        };
+        for (uint32_t b = f2u(0.125f); b < f2u(8.0f); ++b) {
+            const float v = u2f(b);
+            if (to_even(below_ties(v)) != rtn_code(v)) fail("below_ties", b);
+            if ((b & 255u) == 0 && f2u(below_ties(-v)) != (f2u(below_ties(v)) | 0x80000000u)) fail("below_ties sign", b);
+        }
+        for (uint32_t e = 30; e < 250; ++e)   // scale 2^(e - 127)
+            for (int m = 0; m < 7; ++m)
+                for (int d = -3; d <= 3; ++d) {
+                    const float mid = 0.5f * (grid[m] + grid[m + 1]), scale = u2f(e << 23);
+                    const float v = u2f(f2u(mid * scale) + (uint32_t)d);
+                    if (to_even(below_ties(v) / scale) != rtn_code(v / scale)) fail("below_ties scaled", f2u(v));
+                }
+        if (f2u(below_ties(0.0f)) != 0u || f2u(below_ties(-0.0f)) != 0u) fail("below_ties of zero", 0);
+        for (uint32_t b = 1; b < 4096; ++b)   // the smallest values keep their sign and do not become zero
+            if (!(below_ties(u2f(b)) > 0.0f) || !(below_ties(u2f(b | 0x80000000u)) < 0.0f)) fail("below_ties of a denormal", b);
+        // the quotient's zeros likewise: positive whatever their sign was
+        if (f2u(div_four_thirds_fast(0.0f)) != 0u || f2u(div_four_thirds_fast(-0.0f)) != 0u) fail("quotient of zero", 0);
+    }
+
     // the uniform of a 22-bit field f turns "u < p" into the carry out of floor(p 2^22) + f: every value of the top 16 bits
     // with the extreme and a few mixed low parts, p on and next to the boundary
     for (uint32_t hi = 0; hi < 65536; ++hi) {
