@@ -66,16 +66,70 @@ __device__ __forceinline__ float below_ties_any(float v) {
 // n: the NEGATED rotated group.  The sign rule "negative unless g > 0" makes both zeros negative; on the negated values it reads
 // "positive unless n < 0", and the arithmetic in front of the converts turns zeros of either sign into +0 by itself (x y + z
 // with two exact zeros of opposite sign), so it costs one XOR of the sign bits of eight codes.  Everything else is symmetric.
+
+// clip mask, most significant element first so that element 0 lands in bit 0: the sign of |t| - 6 scale (never set for a NaN;
+// |t| = 6 scale gives +0), shifted in by a funnel shift.  The subtraction issues at twice the rate of a compare and nothing
+// passes through the carry flag: 218 cycles a group against 286 for compare and add-with-carry.  Two chains of sixteen: the
+// shifts of one depend on each other.
+template <class F>
+__device__ __forceinline__ uint32_t clip_mask(const float (&n)[32], float thr, F&& t_of) {
+    uint32_t lo = 0u, hi = 0u;
+#pragma unroll
+    for (int i = 15; i >= 0; --i) {
+        lo = __builtin_amdgcn_alignbit(lo, f2u(fabsf(t_of(n[i])) - thr), 31);
+        hi = __builtin_amdgcn_alignbit(hi, f2u(fabsf(t_of(n[i + 16])) - thr), 31);
+    }
+    return (hi << 16) | lo;
+}
+// The 32 codes; t_of(n) is the value a convert sees, formed next to it: as an array of its own it would hold 32 more registers.
+template <class F>
+__device__ __forceinline__ void rtn_codes(const float (&n)[32], float hw_scale, F&& t_of, uint32_t (&codes)[4]) {
+    // the converts' byte selector must be a literal, hence the macros
+#define QM_RTN_PAIR(B) w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, t_of(n[wi * 8 + 2 * (B)]), t_of(n[wi * 8 + 2 * (B) + 1]), hw_scale, (B));
+#pragma unroll
+    for (int wi = 0; wi < 4; ++wi) {
+        uint32_t w = 0u;
+        QM_RTN_PAIR(0) QM_RTN_PAIR(1) QM_RTN_PAIR(2) QM_RTN_PAIR(3)
+        codes[wi] = w ^ 0x88888888u;
+    }
+#undef QM_RTN_PAIR
+}
+template <class F>
+__device__ __forceinline__ void sr_codes(const float (&n)[32], float hw_scale, uint64_t seed, int64_t group_index, F&& t_of, uint32_t (&codes)[4]) {
+    // element j of a Philox call (16 elements): its random field is the top 22 bits of word j/4 rotated left by
+    // 8 * (j%4).  The convert reads the field of a pair's first element from bits 31..10 of its random operand and that of
+    // the second from bits 30..9, so the even element's operand is the word rotated by 0 or 16 bits and the odd element's
+    // the word rotated by 7 or 23 (one more bit to the right): one v_alignbit_b32 each, none for a word's first element.
+#define QM_SR_PAIR(B, J0)                                                                                 \
+    {                                                                                                     \
+        const uint32_t pw = ph.w[(J0) >> 2];                                                              \
+        const uint32_t r_even = ((J0) & 3) == 0 ? pw : __builtin_amdgcn_alignbit(pw, pw, 16);             \
+        const uint32_t r_odd = __builtin_amdgcn_alignbit(pw, pw, ((J0) & 3) == 0 ? 25 : 9);               \
+        const v2f pr = {t_of(n[wi * 8 + 2 * (B)]), t_of(n[wi * 8 + 2 * (B) + 1])};                        \
+        sr_convert_pair<(B)>(even, pr, r_even, hw_scale);                                                 \
+        sr_convert_pair<(B)>(odd, pr, r_odd, hw_scale);                                                   \
+    }
+    Philox4 ph;
+#pragma unroll
+    for (int wi = 0; wi < 4; ++wi) {
+        // words 0,1 of the call serve the even octet of the pair, words 2,3 the odd one
+        if ((wi & 1) == 0) ph = philox_for_hexadecad(seed, (uint64_t)(group_index * 2 + (wi >> 1)));
+        uint32_t even, odd;  // converts driven by the even / odd element's random byte; each of their bytes gets written
+        asm("" : "=v"(even), "=v"(odd));
+        if ((wi & 1) == 0) { QM_SR_PAIR(0, 0) QM_SR_PAIR(1, 2) QM_SR_PAIR(2, 4) QM_SR_PAIR(3, 6) }
+        else { QM_SR_PAIR(0, 8) QM_SR_PAIR(1, 10) QM_SR_PAIR(2, 12) QM_SR_PAIR(3, 14) }
+        // low nibbles from `even`, high ones from `odd`, sign bits back (n is negated)
+        codes[wi] = (uint32_t)__builtin_amdgcn_bitop3_b32((int)even, (int)odd, 0x0f0f0f0f, 0xe4) ^ 0x88888888u;
+    }
+#undef QM_SR_PAIR
+}
+
 template <int MODE, bool WANT_MASK>
 __device__ __forceinline__ void quantize_group_regs(const float (&n)[32], uint64_t seed, int64_t group_index,
                                                     GroupCodes& o) {
     constexpr bool kQuest = (MODE == QUEST_RTN || MODE == QUEST_SR);
     constexpr bool kSR = (MODE == ABSMAX_SR || MODE == QUEST_SR);
-    float hw_scale;   // power of two the convert divides by
-    float thr;        // 6 * scale: |n| < thr  <=>  |t| < 6
-    float t[32];
-    bool all_zero = false;
-    [[maybe_unused]] bool finite = true;
+    o.keep = 0u;
     if constexpr (kQuest) {
         float sq[32];
 #pragma unroll
@@ -91,99 +145,36 @@ __device__ __forceinline__ void quantize_group_regs(const float (&n)[32], uint64
         int E = (int)((f2u(s) >> 23) & 0xffu) - 127;
         E = E > 127 ? 127 : E;
         o.scale_byte = (uint32_t)(E + 127);
-        hw_scale = pow2i(E);
+        const float hw_scale = pow2i(E);   // the power of two the convert divides by
         o.deq_scale = hw_scale;
-        thr = 6.0f * hw_scale;
-        finite = ms < __builtin_inff();
-#pragma unroll
-        for (int i = 0; i < 32; ++i) t[i] = n[i];
+        // |n| < 6 * scale  <=>  |t| < 6
+        if constexpr (WANT_MASK) o.keep = clip_mask(n, 6.0f * hw_scale, [](float v) { return v; });
+        if constexpr (kSR) sr_codes(n, hw_scale, seed, group_index, [](float v) { return v + 0.0f; }, o.w);   // both zeros: +0
+        else if (__builtin_expect(ms < __builtin_inff(), 1)) rtn_codes(n, hw_scale, [](float v) { return below_ties(v); }, o.w);
+        else rtn_codes(n, hw_scale, [](float v) { return below_ties_any(v); }, o.w);
     } else {
         float a = 0.0f;
 #pragma unroll
         for (int i = 0; i < 32; ++i) a = fmaxf(a, fabsf(n[i]));
-        all_zero = (a == 0.0f);
+        const bool all_zero = (a == 0.0f);
         int k = (int)((f2u(a) >> 23) & 0xffu) - 129;
         k = k < -127 ? -127 : (k > 127 ? 127 : k);
         o.scale_byte = (uint32_t)(k + 127);
-        hw_scale = pow2i(k);
         o.deq_scale = scale_pow2(kFourThirds, k);
-        // |t| < 6 with t = RN(g 2^-k / d): evaluated on the quotient h = RN(g / d) against 6 * 2^k
-        thr = 6.0f * hw_scale;
+        const auto finish = [&](auto t_of, float hw_scale) {
+            // |t| < 6 with t = RN(g 2^-k / d): evaluated on the quotient h = RN(g / d) against 6 * 2^k
+            if constexpr (WANT_MASK) o.keep = all_zero ? 0u : clip_mask(n, 6.0f * hw_scale, t_of);
+            if constexpr (kSR) sr_codes(n, hw_scale, seed, group_index, t_of, o.w);
+            else rtn_codes(n, hw_scale, [&](float v) { return below_ties(t_of(v)); }, o.w);
+        };
         // t = RN(RN(g 2^-k) / d) by definition.  For a group whose maximum is at least 2^-60 this is RN(g / d) scaled by
         // 2^-k inside the convert: the two-operation quotient is exact for |g| >= 2^-100, and a smaller element lies
         // below 2^-38 of the scale, so its code is a zero whose sign is the element's own whatever the quotient's last
         // bit.  A group with a smaller non-zero maximum (where g / d would lose bits to underflow) follows the
         // definition literally, with a true division, and hands the convert an already scaled value.
-        if (__builtin_expect(a < 0x1p-60f && !all_zero, 0)) {
-#pragma unroll
-            for (int i = 0; i < 32; ++i) t[i] = scale_pow2(n[i], -k) / kFourThirds + 0.0f;
-            hw_scale = 1.0f;
-            thr = 6.0f;
-        } else {
-#pragma unroll
-            for (int i = 0; i < 32; ++i) t[i] = div_four_thirds_fast(n[i]);   // zeros of either sign: +0
-        }
+        if (__builtin_expect(a < 0x1p-60f && !all_zero, 0)) finish([&](float v) { return scale_pow2(v, -k) / kFourThirds + 0.0f; }, 1.0f);
+        else finish([](float v) { return div_four_thirds_fast(v); }, pow2i(k));   // zeros of either sign: +0
     }
-    o.keep = 0u;
-    if constexpr (WANT_MASK) {
-        // clip mask, most significant element first so that element 0 lands in bit 0: the sign of |t| - 6 scale (never set for
-        // a NaN; |t| = 6 scale gives +0), shifted in by a funnel shift.  The subtraction issues at twice the rate of a compare
-        // and nothing passes through the carry flag: 218 cycles a group against 286 for compare and add-with-carry.  Two
-        // chains of sixteen: the shifts of one depend on each other.
-        uint32_t lo = 0u, hi = 0u;
-#pragma unroll
-        for (int i = 15; i >= 0; --i) {
-            lo = __builtin_amdgcn_alignbit(lo, f2u(fabsf(t[i]) - thr), 31);
-            hi = __builtin_amdgcn_alignbit(hi, f2u(fabsf(t[i + 16]) - thr), 31);
-        }
-        o.keep = all_zero ? 0u : (hi << 16) | lo;
-    }
-
-    // the converts' byte selector must be a literal, hence the macros
-#define QM_RTN_PAIR(B) w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, below(t[wi * 8 + 2 * (B)]), below(t[wi * 8 + 2 * (B) + 1]), hw_scale, (B));
-    // element j of a Philox call (16 elements): its random field is the top 22 bits of word j/4 rotated left by
-    // 8 * (j%4).  The convert reads the field of a pair's first element from bits 31..10 of its random operand and that of
-    // the second from bits 30..9, so the even element's operand is the word rotated by 0 or 16 bits and the odd element's
-    // the word rotated by 7 or 23 (one more bit to the right): one v_alignbit_b32 each, none for a word's first element.
-#define QM_SR_PAIR(B, J0)                                                                                 \
-    {                                                                                                     \
-        const uint32_t pw = ph.w[(J0) >> 2];                                                              \
-        const uint32_t r_even = ((J0) & 3) == 0 ? pw : __builtin_amdgcn_alignbit(pw, pw, 16);             \
-        const uint32_t r_odd = __builtin_amdgcn_alignbit(pw, pw, ((J0) & 3) == 0 ? 25 : 9);               \
-        const v2f pr = {t[wi * 8 + 2 * (B)], t[wi * 8 + 2 * (B) + 1]};                                    \
-        sr_convert_pair<(B)>(even, pr, r_even, hw_scale);                                                 \
-        sr_convert_pair<(B)>(odd, pr, r_odd, hw_scale);                                                   \
-    }
-    if constexpr (!kSR) {
-        const auto convert = [&](auto below) {
-#pragma unroll
-            for (int wi = 0; wi < 4; ++wi) {
-                uint32_t w = 0u;
-                QM_RTN_PAIR(0) QM_RTN_PAIR(1) QM_RTN_PAIR(2) QM_RTN_PAIR(3)
-                o.w[wi] = w ^ 0x88888888u;
-            }
-        };
-        if (__builtin_expect(finite, 1)) convert([](float v) { return below_ties(v); });
-        else convert([](float v) { return below_ties_any(v); });
-    } else {
-        if constexpr (kQuest) {
-#pragma unroll
-            for (int i = 0; i < 32; ++i) t[i] += 0.0f;   // both zeros: +0
-        }
-        Philox4 ph;
-#pragma unroll
-        for (int wi = 0; wi < 4; ++wi) {
-            // words 0,1 of the call serve the even octet of the pair, words 2,3 the odd one
-            if ((wi & 1) == 0) ph = philox_for_hexadecad(seed, (uint64_t)(group_index * 2 + (wi >> 1)));
-            uint32_t even = 0u, odd = 0u;  // converts driven by the even / odd element's random byte
-            if ((wi & 1) == 0) { QM_SR_PAIR(0, 0) QM_SR_PAIR(1, 2) QM_SR_PAIR(2, 4) QM_SR_PAIR(3, 6) }
-            else { QM_SR_PAIR(0, 8) QM_SR_PAIR(1, 10) QM_SR_PAIR(2, 12) QM_SR_PAIR(3, 14) }
-            // low nibbles from `even`, high ones from `odd`, sign bits back (n is negated)
-            o.w[wi] = (uint32_t)__builtin_amdgcn_bitop3_b32((int)even, (int)odd, 0x0f0f0f0f, 0xe4) ^ 0x88888888u;
-        }
-    }
-#undef QM_RTN_PAIR
-#undef QM_SR_PAIR
 }
 
 template <typename T>
@@ -240,14 +231,18 @@ struct GroupOut {
     void* dequant;       // [n_groups * 32] of T or null
 };
 
-// -(x @ H) for one chunk of 32 (what quantize_group_regs takes): butterfly, then -hd^-1/2 with the column sign folded in
-__device__ __forceinline__ void rotate_group(float (&v)[32], float c, uint32_t sign_word, bool rotate = true) {
-    if (rotate) butterfly32(v);  // uniform; without it (c = 1, no signs) the group passes through unchanged
+// times -hd^-1/2 with the column sign folded in: the negated group, as quantize_group_regs takes it
+__device__ __forceinline__ void scale_group(float (&v)[32], float c, uint32_t sign_word) {
 #pragma unroll
     for (int j = 0; j < 32; ++j) {
         const float cj = u2f(f2u(-c) ^ (((sign_word >> j) & 1u) << 31));  // wave-uniform: stays in scalar registers
         v[j] = v[j] * cj;
     }
+}
+// -(x @ H) for one chunk of 32
+__device__ __forceinline__ void rotate_group(float (&v)[32], float c, uint32_t sign_word, bool rotate = true) {
+    if (rotate) butterfly32(v);  // uniform; without it (c = 1, no signs) the group passes through unchanged
+    scale_group(v, c, sign_word);
 }
 
 }  // namespace

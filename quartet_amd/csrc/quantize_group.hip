@@ -35,6 +35,7 @@
 
 #include <type_traits>
 
+#include "lds_requests.h"
 #include "qm_jobs.h"
 #include "qm_kernels.h"
 #include "qm_math.h"
@@ -43,6 +44,13 @@
 namespace qm {
 
 namespace {
+
+// what the lanes of a wave wrote to LDS before is read by its other lanes behind
+__device__ __forceinline__ void wave_settle() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 // ---- dense 32x32 rotation (rerotate="O32", quantizers/mxfp4.py:61-64 of the reference) on the matrix pipe ----------
 // The reference applies the matrix with tl.dot inside its kernel (mxfp4_triton.py:44-45).  Here each lane owns one
@@ -489,10 +497,8 @@ struct TransposedJob {
 // 16-byte piece; codes leave through LDS as whole 64-byte row pieces (tiled output: four contiguous 1 KiB tiles per wave).
 constexpr int kRqR = 512, kRqC = 64;
 
-// Hadamard blocks 64 and 128 span row groups 2k, 2k + 1 or all four of the wave's: lane l then handles row group l % 4 of
-// column quad l / 4, so that a block's groups sit in neighbouring lanes (rotate_block).  PADDED: tiled codes of extents that are
-// not multiples of 128, read and completed with the padding of zero codes and scales.
-template <int VAL_DTYPE, int MODE, bool DENSE = false, int HD = 32, bool PADDED = false>
+// (Row-major operands, dense rotations, absmax-coded and de-quantized tensors; a layer's backward pass runs RequantTiledJob.)
+template <int VAL_DTYPE, int MODE, bool DENSE = false>
 struct RequantJob {
     static constexpr int kLds = 4 * kRqC * 4 * 16 + kRqC * 16;
     static constexpr int kWaves = DENSE ? 1 : 3;   // three waves on a SIMD: at 173 registers (two waves) 28 us where three take 24
@@ -502,7 +508,6 @@ struct RequantJob {
     float post;
     Rotation rot;
     uint64_t seed;
-    const uint64_t* seed_base = nullptr;  // device memory, or null: a value the kernel adds to `seed` when it runs
     uint8_t* codes;
     uint8_t* scales;
     void* dequant;
@@ -547,23 +552,13 @@ struct RequantJob {
             dense_rotate(v[0], frag);
             dense_rotate(v[1], frag);
         }
-        if (!active) {
-            if constexpr (PADDED) {
-#pragma unroll
-                for (int gq = 0; gq < 2; ++gq) {
-                    const int cl = 4 * cq + 2 * P + gq;
-                    ocodes[cl * 4 + rg] = make_uint4(0u, 0u, 0u, 0u);
-                    oscales[cl * 16 + wave * 4 + rg] = 0;
-                }
-            }
-            return;
-        }
+        if (!active) return;
 #pragma unroll
         for (int gq = 0; gq < 2; ++gq) {
             const int64_t gi = (ca + 2 * P + gq) * (R / 32) + rbase / 32;
             GroupCodes res;
-            if constexpr (!DENSE) rotate_block<HD>(v[gq], rot);
-            quantize_group_regs<MODE, false>(v[gq], seed_base ? seed + *seed_base : seed, gi, res);
+            if constexpr (!DENSE) rotate_block<32>(v[gq], rot);
+            quantize_group_regs<MODE, false>(v[gq], seed, gi, res);
             if (dequant) store_dequant<T>(reinterpret_cast<T*>(dequant) + gi * 32, res);
             const int cl = 4 * cq + 2 * P + gq;
             ocodes[cl * 4 + rg] = make_uint4(res.w[0], res.w[1], res.w[2], res.w[3]);
@@ -578,9 +573,9 @@ struct RequantJob {
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // tells the compiler it is wave-uniform
         const unsigned bc = bid / grid_r;
         const int64_t r0 = (int64_t)(bid - bc * grid_r) * kRqR, c0 = (int64_t)bc * kRqC;
-        const int64_t in_code_pitch = C / 2, C_p = PADDED ? padded_cols(C) : C, in_scale_pitch = C_p / 32, R_p = PADDED ? padded_cols(R) : R;
+        const int64_t in_code_pitch = C / 2, in_scale_pitch = C / 32;
         const int64_t rw = r0 + wave * 128;          // this wave's first row
-        const int rg = HD == 32 ? lane >> 4 : lane & 3, cq = HD == 32 ? lane & 15 : lane >> 2;   // row group within the wave, column quad
+        const int rg = lane >> 4, cq = lane & 15;   // row group within the wave, column quad
         const int64_t rbase = rw + 32 * rg;
         const int64_t ca = c0 + 4 * cq;              // this lane's first column
         const bool active = rbase < R && ca < C;     // R % 32 == 0 and C % 32 == 0: all of a lane's groups or none
@@ -589,8 +584,8 @@ struct RequantJob {
         if (active) {
             // Uniform row pointers (scalar unit) + the lane's 32-bit byte offset: no per-lane 64-bit address math.
             // Tiled input: rows are 64 bytes apart inside a 16-row block, blocks (C / 128) KiB apart.
-            const int64_t blk = (C_p / 128) * 1024;
-            const uint8_t* cu = tiled_in ? codes_in + tiled_code_offset(rw, c0 / 128, C_p / 128) + (c0 & 127) / 2
+            const int64_t blk = (C / 128) * 1024;
+            const uint8_t* cu = tiled_in ? codes_in + tiled_code_offset(rw, c0 / 128, C / 128) + (c0 & 127) / 2
                                          : codes_in + rw * in_code_pitch + c0 / 2;
             const uint32_t lane_off = (uint32_t)((tiled_in ? 2 * rg * blk : 32 * rg * in_code_pitch) + 2 * cq);
             const int64_t row_step = tiled_in ? 64 : in_code_pitch;                 // next row of a 16-row block
@@ -619,13 +614,13 @@ struct RequantJob {
         column_pair<0>(cw, sc, frag, active, ca, rbase, cq, rg, wave, ocodes, oscales);
         column_pair<1>(cw, sc, frag, active, ca, rbase, cq, rg, wave, ocodes, oscales);
         __syncthreads();
-        const int64_t code_pitch = R / 2, scale_pitch = R_p / 32;
+        const int64_t code_pitch = R / 2, scale_pitch = R / 32;
         // codes: each wave writes its own 64 x 64-byte tile
 #pragma unroll
         for (int it = 0; it < 4; ++it) {
             const int idx = it * 64 + lane, cl = idx >> 2, part = idx & 3;
-            if (c0 + cl < C && rw + part * 32 < R_p) {
-                const int64_t off = tiled_out ? tiled_code_offset(c0 + cl, rw / 128, R_p / 128) + part * 16
+            if (c0 + cl < C && rw + part * 32 < R) {
+                const int64_t off = tiled_out ? tiled_code_offset(c0 + cl, rw / 128, R / 128) + part * 16
                                               : (c0 + cl) * code_pitch + rw / 2 + part * 16;
                 *reinterpret_cast<uint4*>(codes + off) = ocodes[idx];
             }
@@ -638,14 +633,293 @@ struct RequantJob {
                 *reinterpret_cast<uint4*>(dst) = sw;
             } else {
                 const uint32_t w4[4] = {sw.x, sw.y, sw.z, sw.w};
-                if constexpr (PADDED) {   // whole dwords: the row count is padded to 128
+                for (int b = 0; b < 16; ++b)
+                    if (r0 + b * 32 < R) dst[b] = (uint8_t)(w4[b >> 2] >> (8 * (b & 3)));
+            }
+        }
+    }
+};
+
+// ---- the same for a layer's backward pass: tiled quest-coded operands, rotated on the matrix pipe -----------------------
+// One wave owns 128 rows by 64 columns, a workgroup four of them stacked along r, as above.  A wave requests its codes global ->
+// LDS (16-byte pieces) and a scale byte pair per row; the transposing LDS read for 4-bit data hands lane l the 32 codes of column
+// l, k-contiguous, which is how the scaled matrix instruction reads its FP4 operand.  The other operand is the Hadamard matrix
+// with the rows' scales on it: A[j][k] = +-2^(E_k), an eight-bit E5M2 value whose exponent field is the scale byte less a base.
+// So 32 rows x 32 columns are de-quantized, transposed and rotated by one instruction (K = 32 of its 64: columns 32..63 use the
+// other half of A), and two results and sixteen lane-half swaps give every lane the rotated group of its column.
+// Exact: the sums are multiples of half the smallest scale, and while the block's scales span at most ten octaves the instruction
+// adds them without a rounding (2 M random sums of K = 32 and 64 compared with exact ones: none differs up to 10, half of them
+// at 12), so that any order of additions, the butterfly's among them, gives the same fp32 values.  A block with more spread
+// (or scales near the ends of the range) takes rotate_block, its groups in neighbouring lanes, and stores its codes by itself.
+// What bounds it: vector instructions (385 a group, 0.7 us per wave and group of 32 at 2.4 GHz, half of that Philox and the
+// stochastic converts), with six waves on a SIMD to cover the requests; a row group's codes are waited for when they are needed.
+// Both operands of a layer, 8192 x 4096 and 11008 x 4096: 46 us; 16384 x 4096 and 1536 x 4096: 43; 16480 x 1728 and 640 x 1728: 22.
+// The kernel above (544 instructions a group, 64 narrow loads per lane, three waves on a SIMD) took 56, 53 and 26.
+template <int MODE, int HD, bool PADDED>
+struct RequantTiledJob {
+    static constexpr int kRegion = 128 * 32;                                     // a wave's codes, in and out
+    static constexpr int kScalesIn = 4 * kRegion, kScalesOut = kScalesIn + 4 * 256;
+    static constexpr int kLds = kScalesOut + kRqC * 16;
+    static constexpr int kWaves = HD == 32 ? 6 : 4;
+    static constexpr int P = HD / 32;                                            // groups of a Hadamard block
+    const uint8_t* codes_in;
+    const uint8_t* scales_in;
+    int64_t R, C;
+    SignBits signs;
+    Rotation rot;         // of rotate_block
+    uint64_t seed;
+    const uint64_t* seed_base;   // device memory, or null: a value the kernel adds to `seed` when it runs
+    uint8_t* codes;
+    uint8_t* scales;
+    unsigned grid_r, blocks;
+
+    RequantTiledJob(const RequantArgs& a, const SignBits& signs_, const uint64_t* seed_base_)
+        : codes_in(a.codes_in), scales_in(a.scales_in), R(a.R), C(a.C), signs(signs_), rot(make_rotation<HD>(a.val_dtype, signs_)),
+          seed(a.seed), seed_base(seed_base_), codes(a.codes), scales(a.scales), grid_r((unsigned)((a.R + kRqR - 1) / kRqR)),
+          blocks((unsigned)(((a.R + kRqR - 1) / kRqR) * ((a.C + kRqC - 1) / kRqC))) {}
+
+    typedef int v2i __attribute__((ext_vector_type(2)));
+    typedef int v8i __attribute__((ext_vector_type(8)));
+    typedef uint16_t v2u16 __attribute__((ext_vector_type(2)));
+
+    // largest value of either half over the lanes of a half-wave, in every lane of it
+    __device__ __forceinline__ static v2u16 half_wave_max(v2u16 x) {
+        const auto with = [](v2u16 v, int other) { return __builtin_elementwise_max(v, __builtin_bit_cast(v2u16, other)); };
+        x = with(x, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0xB1, 0xf, 0xf, true));    // quad_perm [1,0,3,2]
+        x = with(x, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x4E, 0xf, 0xf, true));    // quad_perm [2,3,0,1]
+        x = with(x, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x141, 0xf, 0xf, true));   // row_half_mirror
+        x = with(x, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x140, 0xf, 0xf, true));   // row_mirror
+        const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, x), __builtin_bit_cast(unsigned, x), false, false);
+        return with(__builtin_bit_cast(v2u16, r[0]), (int)r[1]);
+    }
+
+    // a block of scales with too wide a spread: groups chunk * P .. + P - 1 of the wave's 64 columns
+    __device__ __forceinline__ void wide_spread(int chunk, const uint8_t* region, const uint8_t* scales_lds, uint8_t* scales_out, int lane,
+                                                int64_t rw, int64_t c0, int64_t R_p, uint64_t s) const {
+        const int g = chunk * P + (lane & (P - 1));
+#pragma unroll 1
+        for (int pass = 0; pass < P; ++pass) {
+            const int col = pass * (64 / P) + lane / P;
+            // the group's codes and scale bytes, packed: few registers, for a path that is rarely taken
+            uint32_t w[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        if (r0 + j * 128 < R) *reinterpret_cast<uint32_t*>(dst + 4 * j) = w4[j];
-                } else {
-                    for (int b = 0; b < 16; ++b)
-                        if (r0 + b * 32 < R) dst[b] = (uint8_t)(w4[b >> 2] >> (8 * (b & 3)));
+            for (int i = 0; i < 32; ++i) w[i >> 3] |= ((uint32_t)region[(32 * g + i) * 32 + col / 2] >> (4 * (col & 1)) & 15u) << (4 * (i & 7));
+            const uint4* e = reinterpret_cast<const uint4*>(scales_lds + (col >> 5) * 128 + 32 * g);
+            const uint4 e0 = e[0], e1 = e[1];
+            const uint32_t sc[8] = {e0.x, e0.y, e0.z, e0.w, e1.x, e1.y, e1.z, e1.w};
+            float v[32];
+#define QM_DEQUANT(I)                                                                                                              \
+    v[I] = v2f(__builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w[(I) >> 3], u2f((sc[(I) >> 2] >> (8 * ((I) & 3)) & 0xffu) << 23), ((I) >> 1) & 3)).x;       \
+    v[(I) + 1] = v2f(__builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w[(I) >> 3], u2f((sc[(I) >> 2] >> (8 * (((I) + 1) & 3)) & 0xffu) << 23), ((I) >> 1) & 3)).y;
+            QM_DEQUANT(0) QM_DEQUANT(2) QM_DEQUANT(4) QM_DEQUANT(6) QM_DEQUANT(8) QM_DEQUANT(10) QM_DEQUANT(12) QM_DEQUANT(14)
+            QM_DEQUANT(16) QM_DEQUANT(18) QM_DEQUANT(20) QM_DEQUANT(22) QM_DEQUANT(24) QM_DEQUANT(26) QM_DEQUANT(28) QM_DEQUANT(30)
+#undef QM_DEQUANT
+            rotate_block<HD>(v, rot);
+            GroupCodes res;
+            quantize_group_regs<MODE, false>(v, s, (c0 + col) * (R / 32) + rw / 32 + g, res);
+            if (c0 + col < C)
+                *reinterpret_cast<uint4*>(codes + tiled_code_offset(c0 + col, rw / 128, R_p / 128) + g * 16) = make_uint4(res.w[0], res.w[1], res.w[2], res.w[3]);
+            scales_out[col * 16 + g] = (uint8_t)res.scale_byte;
+        }
+    }
+
+    __device__ __forceinline__ void run(unsigned bid) const {
+        uint8_t* lds = reinterpret_cast<uint8_t*>(job_lds);
+        const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint4*)job_lds;
+        const int tid = threadIdx.x, lane = tid & 63;
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // tells the compiler it is wave-uniform
+        const unsigned bc = bid / grid_r;
+        const int64_t r0 = (int64_t)(bid - bc * grid_r) * kRqR, c0 = (int64_t)bc * kRqC;
+        const int64_t C_p = PADDED ? padded_cols(C) : C, R_p = PADDED ? padded_cols(R) : R;
+        const int64_t rw = r0 + wave * 128;          // this wave's first row
+        uint8_t* region = lds + wave * kRegion;
+        uint8_t* scales_lds = lds + kScalesIn + wave * 256;              // [2 column groups][128 rows]
+        uint8_t* scales_out = lds + kScalesOut + wave * 4;               // [64 columns][16]: this wave's four bytes
+        if (rw < R) {
+            const int rows = (int)(R - rw < 128 ? R - rw : 128);         // a multiple of 32
+            const uint32_t scale_pitch_in = (uint32_t)(C_p / 32);
+            const uint8_t* su = scales_in + rw * scale_pitch_in + c0 / 32;
+            const auto row_of = [&](int r) { return (uint32_t)(!PADDED || r < rows ? r : rows - 1) * scale_pitch_in; };
+            const uint32_t blk = (uint32_t)(C_p / 128) * 1024u;
+            const uint8_t* cu = codes_in + tiled_code_offset(rw, c0 / 128, C_p / 128) + (c0 & 127) / 2;
+            const int last = PADDED ? (int)((padded_rows(R) - rw) / 16) - 1 : 7;
+            const auto rows_at = [&](int i) {   // request i: row group i, a row's 32 bytes in two neighbouring lanes
+                const int b = 2 * i + (lane >> 5);
+                return (uint32_t)(PADDED && b > last ? last : b) * blk + (uint32_t)(((lane >> 1) & 15) * 64 + (lane & 1) * 16);
+            };
+            const uint32_t to = (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds_base + wave * kRegion));
+            // the scale byte pairs of rows lane and 64 + lane (both column groups), then the codes.  One statement, which ends when
+            // the scales are in: left to the compiler, waiting for them would be waiting for everything.
+            uint32_t sa, sb;
+            asm volatile("global_load_ushort %0, %2, %4\n\tglobal_load_ushort %1, %3, %4\n\t"
+                         "s_mov_b32 m0, %9\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %5, %13\n\t"
+                         "s_mov_b32 m0, %10\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %6, %13\n\t"
+                         "s_mov_b32 m0, %11\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %7, %13\n\t"
+                         "s_mov_b32 m0, %12\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %8, %13\n\t"
+                         "s_setprio 0\n\ts_waitcnt vmcnt(4)"
+                         : "=&v"(sa), "=&v"(sb)
+                         : "v"(row_of(lane)), "v"(row_of(64 + lane)), "s"(su), "v"(rows_at(0)), "v"(rows_at(1)), "v"(rows_at(2)), "v"(rows_at(3)), "s"(to),
+                           "s"(to + 1024u), "s"(to + 2048u), "s"(to + 3072u), "s"(cu)
+                         : "memory");
+            if (PADDED && c0 + 32 >= C) {   // C % 64 == 32: the second column group is padding
+                sa = (sa & 0xffu) * 0x101u;
+                sb = (sb & 0xffu) * 0x101u;
+            }
+            const uint64_t s = seed_base ? seed + *seed_base : seed;
+            scales_lds[lane] = (uint8_t)sa;
+            scales_lds[128 + lane] = (uint8_t)(sa >> 8);
+            scales_lds[64 + lane] = (uint8_t)sb;
+            scales_lds[192 + lane] = (uint8_t)(sb >> 8);
+            // extremes of the scales of each row group and column group (low half: columns 0..31)
+            const auto halves = [](uint32_t b) { return __builtin_bit_cast(v2u16, (b & 0xffu) | (b & 0xff00u) << 8); };
+            const v2u16 full = {255, 255};
+            const v2u16 hi_a = half_wave_max(halves(sa)), hi_b = half_wave_max(halves(sb));
+            const v2u16 lo_a = half_wave_max(full - halves(sa)), lo_b = half_wave_max(full - halves(sb));
+            uint32_t smin[2] = {0u, 0u};   // per column group: byte c = smallest scale of chunk c (the row groups of a Hadamard block)
+            uint32_t fast = 0u;            // chunks whose scales are close enough together
+#pragma unroll
+            for (int c = 0; c < 4 / P; ++c) {
+                bool ok = true;
+#pragma unroll
+                for (int cg = 0; cg < 2; ++cg) {
+                    uint32_t top = 0u, bottom = 0u;   // largest scale, largest 255 - scale
+#pragma unroll
+                    for (int g = c * P; g < c * P + P; ++g) {
+                        const uint32_t h = (uint32_t)__builtin_amdgcn_readlane(__builtin_bit_cast(int, g < 2 ? hi_a : hi_b), 32 * (g & 1)) >> (16 * cg) & 0xffu;
+                        const uint32_t l = (uint32_t)__builtin_amdgcn_readlane(__builtin_bit_cast(int, g < 2 ? lo_a : lo_b), 32 * (g & 1)) >> (16 * cg) & 0xffu;
+                        top = h > top ? h : top;
+                        bottom = l > bottom ? l : bottom;
+                    }
+                    const uint32_t low = 255u - bottom;
+                    smin[cg] |= low << (8 * c);
+                    ok = ok && top - low <= 10u && low >= 32u && top <= 240u;
                 }
+                fast |= (ok ? 1u : 0u) << c;
+            }
+            wave_settle();
+            // results: piece g of column l at slot l ^ 2 g of the KiB that held row group g's codes
+            uint4* stage = reinterpret_cast<uint4*>(region);
+            const auto rotate_chunk = [&](int c, int lane) {
+                // the signs of A's bytes: lane (j, half h) holds S[j][16 h + 4 d + q] in byte q of dword d
+                uint32_t hs[4];
+                {
+                    const uint32_t j = (uint32_t)lane;
+                    const uint32_t all = 0x80808080u;
+                    const uint32_t quad = (j & 1u) << 15 | (j & 2u) << 22 | ((j ^ (j >> 1)) & 1u) << 31;
+                    const uint32_t t = quad ^ ((j & 16u) && (j & 32u) ? all : 0u);
+                    hs[0] = t;
+                    hs[1] = t ^ ((j & 4u) ? all : 0u);
+                    hs[2] = t ^ ((j & 8u) ? all : 0u);
+                    hs[3] = hs[1] ^ ((j & 8u) ? all : 0u);
+                }
+                const uint32_t low[2] = {smin[0] >> (8 * c) & 0xffu, smin[1] >> (8 * c) & 0xffu};
+                v2i b[P][2];
+                uint32_t ex[P][2][4];
+#pragma unroll
+                for (int kb = 0; kb < P; ++kb) {
+                    const int g = c * P + kb;
+#pragma unroll
+                    for (int q = 0; q < 2; ++q)
+                        b[kb][q] = __builtin_amdgcn_ds_read_tr4_b64_v2i32(
+                            (__attribute__((address_space(3))) v2i*)(uintptr_t)(lds_base + wave * kRegion + (32 * g + 16 * q + (lane & 15)) * 32 + (lane >> 4) * 8));
+#pragma unroll
+                    for (int cg = 0; cg < 2; ++cg) {
+                        const uint4 e = *reinterpret_cast<const uint4*>(scales_lds + cg * 128 + 32 * g + 16 * (lane >> 5));
+                        const uint32_t w[4] = {e.x, e.y, e.z, e.w};
+                        // exponent fields 1 .. 11 of E5M2 bytes: no byte carries into the next
+                        const uint32_t base = (low[cg] - 1u) * 0x04040404u;
+#pragma unroll
+                        for (int d = 0; d < 4; ++d) ex[kb][cg][d] = (w[d] << 2) - base;
+                    }
+                }
+#pragma unroll 1
+                for (int ob = 0; ob < P; ++ob) {
+                    v16f d0, d1;
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) d0[e] = d1[e] = 0.0f;
+#pragma unroll
+                    for (int kb = 0; kb < P; ++kb) {
+                        const uint32_t flip = (__builtin_popcount((unsigned)(ob & kb)) & 1) ? 0x80808080u : 0u;
+                        const v8i codes_k = v8i{b[kb][0].x, b[kb][0].y, b[kb][1].x, b[kb][1].y, 0, 0, 0, 0};
+                        const auto a = [&](int cg, int d) { return (int)xor3(ex[kb][cg][d], hs[d], flip); };
+                        // scale bytes: A's values are 2^(field - 15) = 2^(S - low - 14); codes carry none (127)
+                        int z[4];   // zeros that do not hold registers from one iteration to the next
+                        asm volatile("v_mov_b32 %0, 0\n\tv_mov_b32 %1, 0\n\tv_mov_b32 %2, 0\n\tv_mov_b32 %3, 0" : "=v"(z[0]), "=v"(z[1]), "=v"(z[2]), "=v"(z[3]));
+                        d0 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(v8i{a(0, 0), a(0, 1), a(0, 2), a(0, 3), z[0], z[1], z[2], z[3]}, codes_k, d0, 1, 4, 0,
+                                                                             (int)(low[0] + 14u), 0, 127);
+                        d1 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(v8i{z[0], z[1], z[2], z[3], a(1, 0), a(1, 1), a(1, 2), a(1, 3)}, codes_k, d1, 1, 4, 0,
+                                                                             (int)(low[1] + 14u), 0, 127);
+                    }
+                    // element e of a lane's result is row j = 8 (e / 4) + 4 (lane / 32) + e % 4 of column lane % 32 (+ 32 for d1)
+                    float v[32];
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        const auto r = __builtin_amdgcn_permlane32_swap(f2u(d0[e]), f2u(d1[e]), false, false);
+                        v[8 * (e / 4) + (e % 4)] = u2f(r[0]);
+                        v[8 * (e / 4) + 4 + (e % 4)] = u2f(r[1]);
+                    }
+                    scale_group(v, rot.c, ob == 0 ? signs.w[0] : ob == 1 ? signs.w[1] : ob == 2 ? signs.w[2] : signs.w[3]);
+                    const int g = c * P + ob;
+                    GroupCodes res;
+                    quantize_group_regs<MODE, false>(v, s, (c0 * (R / 32) + rw / 32 + g) + (uint32_t)(lane * (int)(R / 32)), res);
+                    stage[64 * g + (lane ^ (2 * g))] = make_uint4(res.w[0], res.w[1], res.w[2], res.w[3]);
+                    scales_out[lane * 16 + g] = (uint8_t)res.scale_byte;
+                }
+            };
+            uint32_t staged = 0u;   // row groups whose codes pass through LDS: all but those of wide_spread
+#pragma unroll 1
+            for (int c = 0; c < 4 / P; ++c) {
+                // an opaque copy: what is worked out from it stays inside the loop instead of holding registers across it
+                int lane = (int)threadIdx.x & 63;
+                asm volatile("" : "+v"(lane));
+                // row group i is the wave's i-th request of codes: this chunk's are in once at most the later groups' are pending
+                // (a store may be among the pending ones: the wait is then longer, not shorter)
+                if (c == 0) __builtin_amdgcn_s_waitcnt(vmcnt_imm(4 - P));
+                else if (P == 1 && c == 1) __builtin_amdgcn_s_waitcnt(vmcnt_imm(2));
+                wave_settle();
+                const bool inside = !PADDED || 32 * c * P < rows;   // otherwise padding: zero codes and scales
+                if (inside && !(fast >> c & 1u)) {
+                    wide_spread(c, region, scales_lds, scales_out, lane, rw, c0, R_p, s);
+                } else if (!inside) {
+                    staged |= ((1u << P) - 1u) << (c * P);
+#pragma unroll
+                    for (int g = c * P; g < c * P + P; ++g) {
+                        stage[64 * g + (lane ^ (2 * g))] = make_uint4(0u, 0u, 0u, 0u);
+                        scales_out[lane * 16 + g] = 0;
+                    }
+                } else {
+                    staged |= ((1u << P) - 1u) << (c * P);
+                    rotate_chunk(c, lane);
+                }
+                // two row groups' codes leave together, 32 bytes per column (all requests have been waited for by then)
+                if (P > 1 || (c & 1)) {
+                    if (c == (P == 1 ? 1 : 0)) __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+                    wave_settle();
+#pragma unroll
+                    for (int h = 0; h < (P == 4 ? 2 : 1); ++h) {
+                        const int pair = P == 4 ? h : P == 2 ? c : c >> 1;
+#pragma unroll
+                        for (int it = 0; it < 2; ++it) {
+                            const int idx = it * 64 + lane, cl = idx >> 1, g = 2 * pair + (idx & 1);
+                            if (c0 + cl < C && (staged >> g & 1u))
+                                *reinterpret_cast<uint4*>(codes + tiled_code_offset(c0 + cl, rw / 128, R_p / 128) + g * 16) = stage[64 * g + (cl ^ (2 * g))];
+                        }
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        // scales: one column's 16 bytes (the workgroup's 512 rows) per thread
+        if (tid < kRqC && c0 + tid < C) {
+            const uint4 sw = *reinterpret_cast<const uint4*>(lds + kScalesOut + tid * 16);
+            uint8_t* dst = scales + (c0 + tid) * (R_p / 32) + r0 / 32;
+            if (r0 + kRqR <= R && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
+                *reinterpret_cast<uint4*>(dst) = sw;
+            } else {   // whole dwords: the row count is padded to 128
+                const uint32_t w4[4] = {sw.x, sw.y, sw.z, sw.w};
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (r0 + j * 128 < R) *reinterpret_cast<uint32_t*>(dst + 4 * j) = w4[j];
             }
         }
     }
@@ -781,13 +1055,6 @@ __device__ __forceinline__ void round_pair_to_bf16(float& a, float& b) {
     const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{a, b}, v2bf16));
     a = u2f(w << 16);
     b = u2f(w & 0xffff0000u);
-}
-
-// what the lanes of a wave wrote to LDS before is read by its other lanes behind
-__device__ __forceinline__ void wave_settle() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // TA = void: plain.  Otherwise the norm's input is x + add (the residual sum in front of the norm, src/models/llama.py:
@@ -1215,14 +1482,7 @@ hipError_t quantize_layer_backward(const void* e, int dtype, int64_t T, int64_t 
             constexpr int M = decltype(m)::value, HD = decltype(h)::value;
             const auto ragged = [](const RequantArgs& a) { return a.R % 128 != 0 || a.C % 128 != 0; };
             with_flag(ragged(x) || ragged(w), [&](auto p) {
-                // a quest-coded operand (post = 1, no de-quantized output): its value type only picks the rounding of hd^-1/2
-                const auto requant = [&](const RequantArgs& a) {
-                    return RequantJob<BF16, M, false, HD, decltype(p)::value>(a.codes_in, a.scales_in, a.R, a.C, 1.0f, make_rotation<HD>(a.val_dtype, signs),
-                                                                              a.seed, a.codes, a.scales, nullptr, true, true);
-                };
-                auto jx = requant(x), jw = requant(w);
-                jx.seed_base = jw.seed_base = seed_base;
-                launch_jobs(stream, jx, jw);
+                launch_jobs(stream, RequantTiledJob<M, HD, decltype(p)::value>(x, signs, seed_base), RequantTiledJob<M, HD, decltype(p)::value>(w, signs, seed_base));
             });
         });
     });
