@@ -538,8 +538,8 @@ int qm_linear_backward_error(const void* e, int e_dtype, int64_t T, int64_t I, i
     const uint8_t* pw = static_cast<const uint8_t*>(packed_w);
     uint8_t* k = static_cast<uint8_t*>(workspace);
     hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
-    int rc = from_hip(qm::quantize_error(e, e_dtype, T, O, hd_g, make_signs(signs_g, hd_g), g_mode, seeds[0], seeds[1], k + wl.ec, k + wl.es, k + wl.etc,
-                                         k + wl.ets, nullptr, hs), "qm_linear_backward_error");
+    const qm::ErrorArgs ae{e, e_dtype, T, O, seeds[0], seeds[1], k + wl.ec, k + wl.es, k + wl.etc, k + wl.ets};
+    int rc = from_hip(qm::quantize_error(ae, hd_g, make_signs(signs_g, hd_g), g_mode, nullptr, hs), "qm_linear_backward_error");
     if (rc) return rc;
     const qm::E5m2Args ax{px + lx.c, px + lx.s, T, I, k + wl.xv, k + wl.xs, k + wl.xl};
     const qm::E5m2Args aw{pw + lw.c, pw + lw.s, O, I, k + wl.wv, k + wl.ws, k + wl.wl};
@@ -711,8 +711,8 @@ int qm_linear_backward_seeded(const void* e, int e_dtype, int64_t T, int64_t I, 
             return fail(QM_ERR_INVALID, "qm_linear_backward: null, misaligned or ill-typed tensors, or extents that are not multiples of the Hadamard blocks");
         const qm::RequantArgs rw{pw + lw.c, pw + lw.s, O, I, w_val_dtype, seeds[1], k + wl.wtc, k + wl.wts};
         const qm::RequantArgs rx{px + lx.c, px + lx.s, T, I, x_val_dtype, seeds[3], k + wl.xtc, k + wl.xts};
-        rc = from_hip(qm::quantize_layer_backward(e, e_dtype, T, O, hd_g, make_signs(signs_g, hd_g), g_mode, seeds[0], seeds[2], k + wl.ec, k + wl.es,
-                                                  k + wl.etc, k + wl.ets, rx, rw, seed_base, hs), "qm_linear_backward");
+        const qm::ErrorArgs ae{e, e_dtype, T, O, seeds[0], seeds[2], k + wl.ec, k + wl.es, k + wl.etc, k + wl.ets};
+        rc = from_hip(qm::quantize_layer_backward(ae, hd_g, make_signs(signs_g, hd_g), g_mode, rx, rw, seed_base, hs), "qm_linear_backward");
         if (rc) return rc;
         rc = product_gx();
         if (rc) return rc;

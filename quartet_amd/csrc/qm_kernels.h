@@ -90,16 +90,22 @@ struct RequantArgs {
 };
 // forward quantizers (quest RTN + clip mask) of x and, unless w is null, of the weight
 hipError_t quantize_layer_forward(const RowmajorArgs& x, const RowmajorArgs* w, int hd, hipStream_t stream);
-// backward: absmax quantizer of e [T, O] along its rows and of its transpose along T, and the transposed, re-quantized
-// packed x and W.  seed_base: null, or device memory holding a value the kernels add to every seed when they run.
-hipError_t quantize_layer_backward(const void* e, int dtype, int64_t T, int64_t O, int hd, const SignBits& signs, int mode,
-                                   uint64_t seed_rows, uint64_t seed_transposed, uint8_t* codes_rows, uint8_t* scales_rows,
-                                   uint8_t* codes_transposed, uint8_t* scales_transposed, const RequantArgs& x, const RequantArgs& w,
+struct ErrorArgs {        // e [T, O], quantized along its rows and, transposed, along T
+    const void* e;
+    int dtype;
+    int64_t T, O;
+    uint64_t seed_rows, seed_transposed;
+    uint8_t* codes_rows;
+    uint8_t* scales_rows;
+    uint8_t* codes_transposed;
+    uint8_t* scales_transposed;
+};
+// backward: absmax quantizer of e along its rows and of its transpose, and the transposed, re-quantized packed x and W, in one
+// grid.  seed_base: null, or device memory holding a value the kernels add to every seed when they run.
+hipError_t quantize_layer_backward(const ErrorArgs& e, int hd, const SignBits& signs, int mode, const RequantArgs& x, const RequantArgs& w,
                                    const uint64_t* seed_base, hipStream_t stream);
 // the two quantizations of e alone
-hipError_t quantize_error(const void* e, int dtype, int64_t T, int64_t O, int hd, const SignBits& signs, int mode, uint64_t seed_rows,
-                          uint64_t seed_transposed, uint8_t* codes_rows, uint8_t* scales_rows, uint8_t* codes_transposed,
-                          uint8_t* scales_transposed, const uint64_t* seed_base, hipStream_t stream);
+hipError_t quantize_error(const ErrorArgs& e, int hd, const SignBits& signs, int mode, const uint64_t* seed_base, hipStream_t stream);
 // Packed quest-coded tensors [R, C] (padded tiled codes; R and C multiples of 32) as operands of products that contract
 // over R (expand.hip): E5M2 bytes, padded_rows(C) * padded_cols(R) of them, E8M0 scales [C][padded_cols(R) / 32], and one
 // byte per 128 x 128 block, [ceil(C / 128)][padded_cols(R) / 128], nonzero where the block has a value that E5M2 cannot hold

@@ -1447,46 +1447,44 @@ hipError_t quantize_layer_forward(const RowmajorArgs& x, const RowmajorArgs* w, 
     return hipGetLastError();
 }
 
-hipError_t quantize_error(const void* e, int dtype, int64_t T, int64_t O, int hd, const SignBits& signs, int mode, uint64_t seed_rows,
-                          uint64_t seed_transposed, uint8_t* codes_rows, uint8_t* scales_rows, uint8_t* codes_transposed,
-                          uint8_t* scales_transposed, const uint64_t* seed_base, hipStream_t stream) {
-    const GroupOut orow{reinterpret_cast<uint4*>(codes_rows), scales_rows, nullptr, nullptr};
+namespace {
+// the two quantizations of e as jobs (with `more` jobs' instantiations for the same mode, Hadamard block and raggedness in one grid)
+template <typename F>
+hipError_t with_error_jobs(const ErrorArgs& a, int hd, const SignBits& signs, int mode, const uint64_t* seed_base, bool ragged, F&& f) {
+    const GroupOut orow{reinterpret_cast<uint4*>(a.codes_rows), a.scales_rows, nullptr, nullptr};
     with_absmax_mode(mode, [&](auto m) {
         with_hadamard(hd, [&](auto h) {
             constexpr int M = decltype(m)::value, HD = decltype(h)::value;
-            with_elem_type(dtype, [&](auto t) {
-                with_flag(T % 128 != 0 || O % 128 != 0, [&](auto p) {
+            with_elem_type(a.dtype, [&](auto t) {
+                with_flag(ragged, [&](auto p) {
                     using T_ = decltype(t);
                     constexpr bool PADDED = decltype(p)::value;
-                    const Rotation rot = make_rotation<HD>(dtype, signs);
-                    TransposedJob<T_, M, false, HD, PADDED> jt(e, T, O, rot, seed_transposed, codes_transposed, scales_transposed, nullptr, true);
-                    RowmajorTiledJob<T_, M, false, HD, PADDED> jr(e, T, O, rot, seed_rows, orow);
+                    const Rotation rot = make_rotation<HD>(a.dtype, signs);
+                    TransposedJob<T_, M, false, HD, PADDED> jt(a.e, a.T, a.O, rot, a.seed_transposed, a.codes_transposed, a.scales_transposed, nullptr, true);
+                    RowmajorTiledJob<T_, M, false, HD, PADDED> jr(a.e, a.T, a.O, rot, a.seed_rows, orow);
                     jt.seed_base = jr.seed_base = seed_base;
-                    launch_jobs(stream, jt, jr);
+                    f(jt, jr, m, h, p);
                 });
             });
         });
     });
     return hipGetLastError();
 }
+bool ragged_extents(int64_t a, int64_t b) { return a % 128 != 0 || b % 128 != 0; }
+}  // namespace
 
-hipError_t quantize_layer_backward(const void* e, int dtype, int64_t T, int64_t O, int hd, const SignBits& signs, int mode,
-                                   uint64_t seed_rows, uint64_t seed_transposed, uint8_t* codes_rows, uint8_t* scales_rows,
-                                   uint8_t* codes_transposed, uint8_t* scales_transposed, const RequantArgs& x, const RequantArgs& w,
+hipError_t quantize_error(const ErrorArgs& e, int hd, const SignBits& signs, int mode, const uint64_t* seed_base, hipStream_t stream) {
+    return with_error_jobs(e, hd, signs, mode, seed_base, ragged_extents(e.T, e.O),
+                           [&](const auto& jt, const auto& jr, auto, auto, auto) { launch_jobs(stream, jt, jr); });
+}
+
+hipError_t quantize_layer_backward(const ErrorArgs& e, int hd, const SignBits& signs, int mode, const RequantArgs& x, const RequantArgs& w,
                                    const uint64_t* seed_base, hipStream_t stream) {
-    const hipError_t rc = quantize_error(e, dtype, T, O, hd, signs, mode, seed_rows, seed_transposed, codes_rows, scales_rows, codes_transposed,
-                                         scales_transposed, seed_base, stream);
-    if (rc != hipSuccess) return rc;
-    with_absmax_mode(mode, [&](auto m) {
-        with_hadamard(hd, [&](auto h) {
-            constexpr int M = decltype(m)::value, HD = decltype(h)::value;
-            const auto ragged = [](const RequantArgs& a) { return a.R % 128 != 0 || a.C % 128 != 0; };
-            with_flag(ragged(x) || ragged(w), [&](auto p) {
-                launch_jobs(stream, RequantTiledJob<M, HD, decltype(p)::value>(x, signs, seed_base), RequantTiledJob<M, HD, decltype(p)::value>(w, signs, seed_base));
-            });
-        });
+    return with_error_jobs(e, hd, signs, mode, seed_base, ragged_extents(e.T, e.O) || ragged_extents(x.R, x.C) || ragged_extents(w.R, w.C),
+                           [&](const auto& jt, const auto& jr, auto m, auto h, auto p) {
+        using Requant = RequantTiledJob<decltype(m)::value, decltype(h)::value, decltype(p)::value>;
+        launch_jobs(stream, jt, jr, Requant(x, signs, seed_base), Requant(w, signs, seed_base));
     });
-    return hipGetLastError();
 }
 
 }  // namespace qm
