@@ -827,30 +827,36 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 }
 
 // ---- which kernel serves a product ----------------------------------------------------------------------------------
-// Estimated durations in microseconds, fitted to 110 shapes of 0.2 to 900 GF (tiled operands; each kernel that serves the
-// shape was timed): mean error 13 %, and the fastest kernel is the one chosen but for 0.3 % of the time on average; with cuts
-// into K ranges (60 shapes, 2 to 16 ranges) but for 1.2 %.  All kernels chosen from here give the same bits except a cut into
-// K ranges, so nothing but time hangs on the choice.  (A layer's forward product of at most 64 tokens may run on gemm_rows.hip
-// instead, before this choice; its sums are in another order.)
+// Estimated durations in microseconds, fitted to 70 shapes of 0.2 to 740 GF with tiled operands: every kernel that serves the
+// shape and cuts into 2 to 4 K ranges, each launch between two 8192 x 4096 x 4096 products (alone and back to back the kernels run at
+// another clock and in another order of speed): mean error 6 %, and the choice costs 0.3 % more than the fastest on average.
+// All kernels chosen from here give the same bits except a cut into K ranges, so nothing but time hangs on the choice.  (A
+// layer's forward product of at most 64 tokens may run on gemm_rows.hip instead, before this choice; its sums are in another
+// order.)
 struct KernelCost {
     int bm, bn, per_cu;              // tile, resident workgroups per CU
     double step, shared, boundary;   // one K step of a workgroup alone on its CU; with n of them: n * shared; per tile
-    double rotate[3];                // what the rotation (blocks of 32, 64, 128) adds to a round of per_cu tiles; 0: not served
+    double rotate[3], more[3];       // what the rotation (blocks of 32, 64, 128) adds to the first round of per_cu tiles and to each further one
 };
-constexpr KernelCost kTileCosts[] = {{256, 128, 2, 0.726, 0.648, 2.4, {5.6, 8.5, 9.6}},
-                                     {128, 128, 3, 0.198, 0.373, 1.5, {2.7, 4.4, 5.0}},
-                                     {128, 64, 3, 0.170, 0.277, 0.9, {1.5, 2.1, 0.0}},
-                                     {64, 64, 4, 0.129, 0.207, 0.63, {0.8, 1.1, 0.0}},
-                                     {64, 32, 4, 0.176, 0.139, 0.71, {0.7, 0.0, 0.0}}};
+constexpr KernelCost kTileCosts[] = {{256, 128, 2, 0.461, 0.488, 5.6, {10.0, 12.0, 14.0}, {10.0, 12.0, 14.0}},
+                                     {128, 128, 3, 0.155, 0.294, 1.71, {6.0, 7.5, 9.0}, {1.5, 3.8, 5.0}},
+                                     {128, 64, 3, 0.172, 0.204, 0.99, {2.4, 3.6, 0.0}, {0.8, 2.2, 0.0}},
+                                     {64, 64, 4, 0.152, 0.129, 0.72, {1.0, 1.5, 0.0}, {0.8, 1.4, 0.0}},
+                                     {64, 32, 4, 0.099, 0.091, 0.71, {0.7, 0.0, 0.0}, {0.7, 0.0, 0.0}}};
+// 256 x 128 tiles over fewer than kShortTallSteps K steps, which request their scales step by step
+constexpr KernelCost kShortTall = {256, 128, 2, 0.60, 0.68, 2.5, {10.0, 12.0, 14.0}, {10.0, 12.0, 14.0}};
 // with an eight-bit B (70 shapes, cuts included: mean error 9 %, 2.9 % from the fastest choice on average)
-constexpr KernelCost kWideTileCosts[] = {{256, 256, 1, 1.068, 1.068, 8.0, {9.0, 10.9, 12.3}},
-                                         {128, 128, 3, 0.203, 0.560, 1.1, {3.7, 4.6, 5.7}},
-                                         {128, 64, 3, 0.246, 0.393, 0.42, {1.4, 2.0, 0.0}},
-                                         {64, 64, 3, 0.196, 0.297, 0.60, {0.7, 1.0, 0.0}}};
-const KernelCost* tile_costs(bool e5m2) { return e5m2 ? kWideTileCosts : kTileCosts; }
+constexpr KernelCost kWideTileCosts[] = {{256, 256, 1, 1.068, 1.068, 8.0, {9.0, 10.9, 12.3}, {9.0, 10.9, 12.3}},
+                                         {128, 128, 3, 0.203, 0.560, 1.1, {6.0, 7.5, 9.0}, {1.5, 3.8, 5.0}},
+                                         {128, 64, 3, 0.246, 0.393, 0.42, {2.4, 3.6, 0.0}, {0.8, 2.2, 0.0}},
+                                         {64, 64, 3, 0.196, 0.297, 0.60, {1.0, 1.5, 0.0}, {0.8, 1.4, 0.0}}};
+const KernelCost& tile_costs(bool e5m2, int kind, int64_t K, int splits) {
+    if (!e5m2 && kind == TILE_256x128 && K / kBK / splits < kShortTallSteps) return kShortTall;
+    return (e5m2 ? kWideTileCosts : kTileCosts)[kind];
+}
 int last_tile_kind(bool e5m2) { return e5m2 ? TILE_64x64 : TILE_64x32; }
-constexpr double kLaunch = 2.3, kPersistentStep = 0.88, kPersistentBoundary = 3.7, kPersistentRotate = 3.5;
-constexpr double kMemory = 3.2e6, kRotateMemory = 6.6e6;   // bytes per us of the reduction and of a rotation pass of its own
+constexpr double kLaunch = 3.0, kPersistentStep = 0.675, kPersistentBoundary = 5.5, kPersistentRotate = 3.9;
+constexpr double kMemory = 5.5e6, kRotateMemory = 5.2e6;   // bytes per us of the reduction and of a rotation pass of its own
 
 double ranges_cost(int64_t M, int64_t N, int splits) {   // writing, reading and reducing the partial sums of a cut product
     return splits == 1 ? 0.0 : kLaunch + (4.0 * splits + 2.0) * (double)M * (double)N / kMemory;
@@ -865,10 +871,11 @@ double tile_cost(const KernelCost& k, int64_t M, int64_t N, int64_t K, int split
     return kLaunch + full * round(k.per_cu) + (rest ? round((rest + cus - 1) / cus) : 0.0) + ranges_cost(M, N, splits);
 }
 // the masked inverse rotation in the epilogue of a tile kernel, and as a kernel of its own
-double tile_rotate_cost(const KernelCost& k, int64_t M, int64_t N, int hd, int cus) {
+double tile_rotate_cost(const KernelCost& k, int64_t M, int64_t N, int hd, int out_bytes, int cus) {
     const int64_t tiles = ((M + k.bm - 1) / k.bm) * ((N + k.bn - 1) / k.bn);
     const double rounds = (double)((tiles + cus - 1) / cus) / k.per_cu;
-    return k.rotate[hd == 32 ? 0 : hd == 64 ? 1 : 2] * (rounds > 1.0 ? rounds : 1.0);
+    const int h = hd == 32 ? 0 : hd == 64 ? 1 : 2;
+    return k.rotate[h] + (rounds > 1.0 ? (rounds - 1.0) * k.more[h] : 0.0) + (double)M * (double)N * (out_bytes - 2) / kRotateMemory;
 }
 double separate_rotate_cost(int64_t M, int64_t N, int in_bytes, int out_bytes) {
     return kLaunch + 0.5 + (double)M * (double)N * (in_bytes + out_bytes) / kRotateMemory;
@@ -909,7 +916,7 @@ Cut cheapest_cut(int64_t M, int64_t N, int64_t K, bool persistent, bool tiles_ok
         if (persistent && K % 512 == 0 && (K / 512) % sp == 0 && K / 512 / sp >= 2)
             consider(ProductChoice::PERSISTENT, 0, sp, persistent_cost(M, N, K, sp, cus));
         if (tiles_ok)
-            for (int kind = TILE_256x128; kind <= TILE_64x64; ++kind) consider(ProductChoice::TILE, kind, sp, tile_cost(tile_costs(e5m2)[kind], M, N, K, sp, cus));
+            for (int kind = TILE_256x128; kind <= TILE_64x64; ++kind) consider(ProductChoice::TILE, kind, sp, tile_cost(tile_costs(e5m2, kind, K, sp), M, N, K, sp, cus));
     }
     return best;
 }
@@ -1023,8 +1030,13 @@ struct ShapePlan {
     size_t cut_bytes = 0;       // scratch of the cut, 0 if it would not be made
     size_t scratch_bytes = 0;   // what a caller is asked to provide: at least cut_bytes
 };
-// Few tiles of the persistent kernel and a long K: callers hold room for the ranges that would fill its CUs, whether or not
-// a cut on smaller tiles, or none, turns out cheaper
+// Few tiles and a long K: callers hold room for the ranges that would fill the CUs, whether or not a cut turns out cheaper than
+// the whole product (it mostly does from 64 K steps on).  Ranges of the persistent kernel; where that one has none, four ranges of
+// 128 x 128 tiles, if those are an eighth of the CUs at most.
+size_t scratch_of_few_small_tiles(int64_t M, int64_t N, int64_t K, int cus) {
+    const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
+    return tiles * 8 <= cus && K >= 16 * kBK ? (size_t)4 * (size_t)M * (size_t)N * sizeof(float) : 0;
+}
 size_t scratch_of_few_tiles(int64_t M, int64_t N, int64_t K, int cus) {
     const int64_t tiles = ((M + kBigM - 1) / kBigM) * ((N + kBigN - 1) / kBigN), nblk = K / 512;
     if (K % 512 || tiles * 4 >= cus * 3 || nblk < 4) return 0;
@@ -1047,12 +1059,13 @@ ShapePlan make_plan(int64_t M, int64_t N, int64_t K, bool persistent, bool tiles
     double best = 1e30;
     if (persistent) best = p.persistent = persistent_cost(M, N, K, 1, cus);
     for (int kind = TILE_256x128; kind <= last_tile_kind(e5m2); ++kind) {
-        p.tile[kind] = tiles_ok ? tile_cost(tile_costs(e5m2)[kind], M, N, K, 1, cus) : 1e30;
+        p.tile[kind] = tiles_ok ? tile_cost(tile_costs(e5m2, kind, K, 1), M, N, K, 1, cus) : 1e30;
         best = p.tile[kind] < best ? p.tile[kind] : best;
     }
     p.cut = cheapest_cut(M, N, K, persistent, tiles_ok, e5m2, cus);
     p.cut_bytes = p.cut.cost < best ? (size_t)p.cut.choice.splits * (size_t)M * (size_t)N * sizeof(float) : 0;
     p.scratch_bytes = persistent ? scratch_of_few_tiles(M, N, K, cus) : 0;
+    if (tiles_ok && !e5m2 && !p.scratch_bytes) p.scratch_bytes = scratch_of_few_small_tiles(M, N, K, cus);
     if (p.cut_bytes > p.scratch_bytes) p.scratch_bytes = p.cut_bytes;
     return p;
 }
@@ -1104,8 +1117,8 @@ ProductChoice choose_product(const TileProduct& p, int c_dtype, int rot_out_dtyp
         consider({ProductChoice::PERSISTENT, 0, 1, false}, plan.persistent + separate);
     }
     for (int kind = TILE_256x128; tiles_ok && kind <= last_tile_kind(e5m2); ++kind) {
-        const KernelCost& k = tile_costs(e5m2)[kind];
-        if (rotate && bf16 && k.bn >= p.hd) consider({ProductChoice::TILE, kind, 1, true}, plan.tile[kind] + tile_rotate_cost(k, M, N, p.hd, cus));
+        const KernelCost& k = tile_costs(e5m2, kind, K, 1);
+        if (rotate && bf16 && k.bn >= p.hd) consider({ProductChoice::TILE, kind, 1, true}, plan.tile[kind] + tile_rotate_cost(k, M, N, p.hd, rot_out_dtype == BF16 ? 2 : 4, cus));
         consider({ProductChoice::TILE, kind, 1, false}, plan.tile[kind] + separate);
     }
     return best;

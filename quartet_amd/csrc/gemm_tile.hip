@@ -3,7 +3,7 @@
 //
 // One design, five tile shapes.  A workgroup of W waves owns a BM x BN tile, each wave WM x WN of it in 32 x 32 blocks of
 // v_mfma_scale_f32_32x32x64_f8f6f4.  Operands go global -> LDS directly (16 bytes per lane, XOR-swizzled 16-byte slots)
-// into a ring of STAGES K steps of 128, scales as one dword per row and step; one barrier per step.  Rows past the end of a
+// into a ring of STAGES K steps of 128, scales beside them in blocks of four steps; one barrier per step.  Rows past the end of a
 // matrix are requested as its last row (their products are dropped), so no request leaves the operands.  bf16 results pass
 // through the ring's LDS and leave as 16-byte pieces of whole rows; on that way a lane holds eight consecutive columns,
 // which is what the masked inverse Hadamard rotation of the layer's backward pass works on: it is applied there (blocks of
@@ -16,8 +16,9 @@
 // kernels: results depend on the choice only where a product is cut into K ranges.  (gemm_rows.hip's order is its own.)
 //
 // The same kernel multiplies FP4 with an eight-bit (E5M2) B, which is how the error-only scheme contracts over the rows of a
-// packed operand (expand.hip): twice the bytes and twice the matrix cycles of B.  4096^3: 60 us, 8 waves of 128 x 64 on 256 x
-// 256 with the matrix pipe 60 % busy at the clock its power allows, where the FP4 x bf16 kernel (gemm_fp4_bf16.hip) takes 113 us.
+// packed operand (expand.hip): twice the bytes and twice the matrix cycles of B.  4096^3 among the other kernels of a training
+// step: 74 us (76 with scales step by step), 8 waves of 128 x 64 on 256 x 256 with the matrix pipe over 60 % busy at the clock its
+// power allows, where the FP4 x bf16 kernel (gemm_fp4_bf16.hip) takes 113 us and more.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -30,23 +31,33 @@ namespace qm {
 
 namespace {
 
-// E5M2_B: B is eight bits wide (expand.hip), two 1 KiB blocks of 64 contraction indices per 16 columns and K step
-template <int BM_, int BN_, int WM_, int WN_, int STAGES_, int OCC_, bool E5M2_B = false>
+// E5M2_B: B is eight bits wide (expand.hip), two 1 KiB blocks of 64 contraction indices per 16 columns and K step.
+// BLOCKS: scales travel in blocks of four K steps, 16 bytes per row and request, into an area of their own, from where every wave
+// takes its rows' into registers (K >= 512 and 4-byte aligned scale rows).  Otherwise one dword per row and K step, in the ring:
+// every dword lies in another line, and those requests are two thirds of all.  4608 x 1536 x 8192 55 -> 40 us,
+// 2048 x 4096 x 4096 32 -> 25, 512 x 11008 x 4096 27 -> 22; without any scale requests (wrong results) 37, 22 and 19.
+template <int BM_, int BN_, int WM_, int WN_, int STAGES_, int OCC_, bool E5M2_B = false, bool BLOCKS_ = true>
 struct TileShape {
+    using Narrow = TileShape<BM_, BN_, WM_, WN_, STAGES_, OCC_, E5M2_B, false>;
+    static constexpr bool kBlocks = BLOCKS_;
     static constexpr bool kWideB = E5M2_B;
     static constexpr int kBBlocks = E5M2_B ? 2 : 1;
     static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, STAGES = STAGES_, OCC = OCC_;   // OCC: workgroups per CU
     static constexpr int kWavesN = BN / WN, kWaves = (BM / WM) * kWavesN, kThreads = kWaves * 64;
     static constexpr int TM = WM / 32, TN = WN / 32;
     static constexpr int kALoads = BM / 16 / kWaves, kBLoads = BN / 16 * kBBlocks / kWaves;   // 1 KiB wave-loads per wave and K step
-    static constexpr int kAUnits = (BM + 63) / 64, kUnits = kAUnits + (BN + 63) / 64;   // 64 scale dwords each
+    static constexpr int kAUnits = (BM + 63) / 64, kUnits = kAUnits + (BN + 63) / 64;   // requests of 64 rows' scales each
     static constexpr int kSLoads = (kUnits + kWaves - 1) / kWaves;
-    static constexpr int kLoads = kALoads + kBLoads + kSLoads;   // requests per wave and K step
-    static constexpr int kBOff = BM * kRowBytes, kSAOff = (BM + BN * kBBlocks) * kRowBytes, kSBOff = kSAOff + kAUnits * 256;
-    static constexpr int kStageBytes = kSAOff + kUnits * 256;
-    static constexpr int kRingBytes = STAGES * kStageBytes;
+    static constexpr int kLoads = kALoads + kBLoads + (kBlocks ? 0 : kSLoads);   // requests per wave and K step
+    static constexpr int kUnitBytes = kBlocks ? 1024 : 256;
+    // scales: in the stage (BLOCKS: behind the ring)
+    static constexpr int kBOff = BM * kRowBytes, kCodeBytes = (BM + BN * kBBlocks) * kRowBytes;
+    static constexpr int kStageBytes = kCodeBytes + (kBlocks ? 0 : kUnits * kUnitBytes);
+    static constexpr int kSAOff = kBlocks ? STAGES * kStageBytes : kCodeBytes, kSBOff = kSAOff + kAUnits * kUnitBytes;
+    static constexpr int kRingBytes = STAGES * kStageBytes + (kBlocks ? kUnits * kUnitBytes : 0);
     static constexpr int kMUnits = BM * BN / 2048, kMLoads = (kMUnits + kWaves - 1) / kWaves;   // mask words of the tile, 64 at a time
-    static constexpr bool kMaskEarly = BM < 256;                 // 256 x 128: no room beside the ring for two workgroups per CU
+    // ahead of the operands where there is room beside the ring for OCC workgroups per CU
+    static constexpr bool kMaskEarly = BM < 256 && (kRingBytes + kMUnits * 256) * OCC <= 160 * 1024;
     static constexpr int kPitch = BN * 2 + 16;                   // bytes per staged row of the bf16 tile
     static constexpr int kChunks = BN / 8;                       // 16-byte pieces per row
     static constexpr int kRowsPerPass = kThreads / kChunks, kPasses = BM / kRowsPerPass;
@@ -101,7 +112,36 @@ __device__ __forceinline__ void tile_issue(const TilePlan<S>& p, int stage, int 
     for (int j = 0; j < S::kBLoads; ++j) load_lds_b128_s(b, p.voff_b[j] - back, p.lds_b + off + j * 1024);
     const int sback = half ? 2 : 0;
 #pragma unroll
-    for (int u = 0; u < S::kSLoads; ++u) load_lds_b32_s(p.s[u] + ks * 4 - sback, p.voff_s[u], p.lds_s[u] + off);
+    for (int u = 0; u < S::kSLoads; ++u)
+        if constexpr (!S::kBlocks) load_lds_b32_s(p.s[u] + ks * 4 - sback, p.voff_s[u], p.lds_s[u] + off);
+}
+// BLOCKS: the 16 bytes of every row from K step ks on
+template <class S>
+__device__ __forceinline__ void tile_issue_scales(const TilePlan<S>& p, int ks) {
+#pragma unroll
+    for (int u = 0; u < S::kSLoads; ++u) load_lds_b128_s(p.s[u] + ks * 4, p.voff_s[u], p.lds_s[u]);
+}
+// the scale dwords of a lane's rows for four K steps
+template <class S>
+struct TileScales {
+    uint4 a[S::TM], b[S::TN];
+};
+template <class S>
+__device__ __forceinline__ void tile_read_scales(const uint8_t* __restrict__ smem, int a_off, int b_off, TileScales<S>& r) {
+#pragma unroll
+    for (int i = 0; i < S::TM; ++i) r.a[i] = *reinterpret_cast<const uint4*>(smem + a_off + i * 32 * 16);
+#pragma unroll
+    for (int j = 0; j < S::TN; ++j) r.b[j] = *reinterpret_cast<const uint4*>(smem + b_off + j * 32 * 16);
+}
+template <int Q>
+__device__ __forceinline__ uint32_t dword_of(const uint4& v) {
+    return Q == 0 ? v.x : Q == 1 ? v.y : Q == 2 ? v.z : v.w;
+}
+// the dwords from `by` on first (uniform)
+__device__ __forceinline__ uint4 rotate_dwords(uint4 v, int by) {
+    if (by & 1) v = make_uint4(v.y, v.z, v.w, v.x);
+    if (by & 2) v = make_uint4(v.z, v.w, v.x, v.y);
+    return v;
 }
 
 template <class S>
@@ -176,8 +216,9 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
     const int b_off1 = S::kBOff + (wn * S::WN + lrow) * kRowBytes + (((S::kWideB ? 2 + half : 2 * half + 1) ^ swz) * 16);
     // scales in LDS: A dword p holds row (p / (32 TM)) * WM + (p % TM) * 32 + (p / TM) % 32, so one read fetches the scale
     // dwords of a lane's TM blocks; B likewise with TN and WN
-    const int a_sc_off = S::kSAOff + (wm * 32 + lrow) * (4 * S::TM);
-    const int b_sc_off = S::kSBOff + (wn * 32 + lrow) * (4 * S::TN);
+    // (BLOCKS: 16 bytes per row, in the rows' order)
+    const int a_sc_off = S::kSAOff + (S::kBlocks ? (wm * S::WM + lrow) * 16 : (wm * 32 + lrow) * (4 * S::TM));
+    const int b_sc_off = S::kSBOff + (S::kBlocks ? (wn * S::WN + lrow) * 16 : (wn * 32 + lrow) * (4 * S::TN));
     const int sh = 16 * half;
 
     TilePlan<S> plan;
@@ -186,9 +227,9 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
         const int pcv = (lane & 3) ^ ((prow >> 2) & 3);
         const int64_t row16 = (int64_t)16 * code_pitch;
         const int last_a = (g.a_tiled ? (M + 15) & ~15 : M) - 1 - m0, last_b = (g.b_tiled ? (N + 15) & ~15 : N) - 1 - n0;
-        const auto row_off = [&](int r, int tiled) {
-            return tiled ? (uint32_t)((r >> 4) * row16) + (uint32_t)((r & 15) * 64 + pcv * 16) : (uint32_t)(r * code_pitch + pcv * 16);
-        };
+        // 16 rows are row16 bytes in either layout
+        const uint32_t row_a = g.a_tiled ? 64u : (uint32_t)code_pitch, row_b = g.b_tiled ? 64u : (uint32_t)code_pitch;
+        const auto row_off = [&](int r, uint32_t row_bytes) { return (uint32_t)(r >> 4) * (uint32_t)row16 + (uint32_t)(r & 15) * row_bytes + pcv * 16; };
         plan.kstep_a = g.a_tiled ? 1024 : kRowBytes;
         plan.kstep_b = g.b_tiled ? 1024 * S::kBBlocks : kRowBytes;
         plan.a = g.a_codes + (int64_t)m0 * code_pitch + (int64_t)k_first * plan.kstep_a;   // m0, n0 are multiples of 16: the same
@@ -196,7 +237,7 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
 #pragma unroll
         for (int j = 0; j < S::kALoads; ++j) {
             const int r = (wave * S::kALoads + j) * 16 + prow;
-            plan.voff_a[j] = row_off(r < last_a ? r : last_a, g.a_tiled);
+            plan.voff_a[j] = row_off(r < last_a ? r : last_a, row_a);
         }
 #pragma unroll
         for (int j = 0; j < S::kBLoads; ++j) {
@@ -205,7 +246,7 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
             if constexpr (S::kWideB)
                 plan.voff_b[j] = (uint32_t)((rr >> 4) * 2 * row16) + (uint32_t)((u / (S::BN / 16)) * 1024 + (rr & 15) * 64 + pcv * 16);
             else
-                plan.voff_b[j] = row_off(rr, g.b_tiled);
+                plan.voff_b[j] = row_off(rr, row_b);
         }
         plan.half_back = (uint32_t)(pcv & 2) * 16u;
         plan.lds_a = (uint32_t)__builtin_amdgcn_readfirstlane((int)(smem_base + wave * S::kALoads * 1024));
@@ -217,13 +258,13 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
             const int unit = (wave + u * S::kWaves) % S::kUnits;
             const bool is_a = unit < S::kAUnits;
             const int p = (is_a ? unit : unit - S::kAUnits) * 64 + lane;
-            const int ra = (p / (32 * S::TM)) * S::WM + (p % S::TM) * 32 + (p / S::TM) % 32;
-            const int rb = (p / (32 * S::TN)) * S::WN + (p % S::TN) * 32 + (p / S::TN) % 32;
+            const int ra = S::kBlocks ? p : (p / (32 * S::TM)) * S::WM + (p % S::TM) * 32 + (p / S::TM) % 32;
+            const int rb = S::kBlocks ? p : (p / (32 * S::TN)) * S::WN + (p % S::TN) * 32 + (p / S::TN) % 32;
             const int la = M - 1 - m0, lb = N - 1 - n0;
             const int r = is_a ? (ra < la ? ra : la) : (rb < lb ? rb : lb);
             plan.s[u] = (is_a ? g.a_scales + (int64_t)m0 * groups : g.b_scales + (int64_t)n0 * groups) + k_first * 4;
             plan.voff_s[u] = (uint32_t)(r * groups);
-            plan.lds_s[u] = (uint32_t)__builtin_amdgcn_readfirstlane((int)(smem_base + S::kSAOff + unit * 256));
+            plan.lds_s[u] = (uint32_t)__builtin_amdgcn_readfirstlane((int)(smem_base + S::kSAOff + unit * S::kUnitBytes));
         }
     }
     // The rotation's mask words of the tile, [BM][BN / 32] in LDS: with room beside the ring they are requested ahead of
@@ -252,51 +293,125 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
 #pragma unroll
         for (int j = 0; j < S::TN; ++j) b[j] >>= down;
     };
-#pragma unroll
-    for (int s = 0; s < S::STAGES; ++s) issue(s, s < nk ? s : nk - 1);
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm((S::STAGES - 1) * S::kLoads));  // step 0 is in; later ones may be pending
-    __syncthreads();
     TileFrags<S> f0, f1;
-    uint32_t sa[S::TM], sb[S::TN];
-    read_dwords<S::TM>(smem_bytes + a_sc_off, sa);
-    read_dwords<S::TN>(smem_bytes + b_sc_off, sb);
-    settle_scales(sa, sb, 0);
-    tile_read<S>(smem_bytes, a_off0, b_off0, f0);
-
     v16f acc[S::TM][S::TN];
     int stage = 0;
-    // one K step: `stage` is the ring slot it consumes and then refills with step s + STAGES
-    auto step = [&](auto first_tag, int s) {
-        constexpr bool FIRST = decltype(first_tag)::value;
-        const int nstage = stage == S::STAGES - 1 ? 0 : stage + 1;
-        const uint8_t* cur = smem_bytes + stage * S::kStageBytes;
-        const uint8_t* nxt = smem_bytes + nstage * S::kStageBytes;
-        uint32_t sca[S::TM], scb[S::TN];
+    if constexpr (S::kBlocks) {
+        // blocks of four K steps; the last block of an nk that is no multiple of four requests the row's final 16 bytes, whose
+        // first dwords the block before has used
+        const auto block_at = [&](int ks) { return ks + 4 <= nk ? ks : nk - 4; };
+        tile_issue_scales<S>(plan, 0);
 #pragma unroll
-        for (int i = 0; i < S::TM; ++i) sca[i] = __builtin_amdgcn_ubfe(sa[i], (uint32_t)sh, 16u);
-#pragma unroll
-        for (int j = 0; j < S::TN; ++j) scb[j] = __builtin_amdgcn_ubfe(sb[j], (uint32_t)sh, 16u);
-        tile_read<S>(cur, a_off1, b_off1, f1);
-        tile_mfma<S, 0, SWAP, FIRST>(f0, sca, scb, acc);
-        if constexpr (S::TM * S::TN >= S::TM + S::TN) { QM_SCHED_PAIR(0x100, S::TM + S::TN * S::kBBlocks) }
-        __builtin_amdgcn_sched_barrier(0);
-        // younger than the requests of step s + 1: those of the STAGES - 2 steps after it
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm((S::STAGES - 2) * S::kLoads));
+        for (int s = 0; s < S::STAGES; ++s) issue(s, s < nk ? s : nk - 1);
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm((S::STAGES - 1) * S::kLoads));  // the scales and step 0 are in; later ones may be pending
         __syncthreads();
-        __builtin_amdgcn_sched_barrier(0);
-        // past the end: a repeat nobody reads keeps the counts of outstanding requests uniform
-        issue(stage, s + S::STAGES < nk ? s + S::STAGES : nk - 1);
-        read_dwords<S::TM>(nxt + a_sc_off, sa);
-        read_dwords<S::TN>(nxt + b_sc_off, sb);
-        settle_scales(sa, sb, s + 1);
-        tile_read<S>(nxt, a_off0, b_off0, f0);
-        tile_mfma<S, 1, SWAP, false>(f1, sca, scb, acc);
-        if constexpr (S::TM * S::TN >= S::TM + S::TN) { QM_SCHED_PAIR(0x100, S::TM + S::TN * S::kBBlocks) }
-        __builtin_amdgcn_sched_barrier(0);
-        stage = nstage;
-    };
-    step(std::true_type{}, 0);
-    for (int ks = 1; ks < nk; ++ks) step(std::false_type{}, ks);
+        TileScales<S> sc;
+        tile_read_scales<S>(smem_bytes, a_sc_off, b_sc_off, sc);
+        tile_read<S>(smem_bytes, a_off0, b_off0, f0);
+        // one K step, dword Q of its block's scales: `stage` is the ring slot it consumes and then refills with step s + STAGES
+        auto step = [&](auto first_tag, auto q_tag, int s) {
+            constexpr bool FIRST = decltype(first_tag)::value;
+            constexpr int Q = decltype(q_tag)::value;
+            const int nstage = stage == S::STAGES - 1 ? 0 : stage + 1;
+            const uint8_t* cur = smem_bytes + stage * S::kStageBytes;
+            const uint8_t* nxt = smem_bytes + nstage * S::kStageBytes;
+            uint32_t sca[S::TM], scb[S::TN];
+#pragma unroll
+            for (int i = 0; i < S::TM; ++i) sca[i] = __builtin_amdgcn_ubfe(dword_of<Q>(sc.a[i]), (uint32_t)sh, 16u);
+#pragma unroll
+            for (int j = 0; j < S::TN; ++j) scb[j] = __builtin_amdgcn_ubfe(dword_of<Q>(sc.b[j]), (uint32_t)sh, 16u);
+            tile_read<S>(cur, a_off1, b_off1, f1);
+            tile_mfma<S, 0, SWAP, FIRST>(f0, sca, scb, acc);
+            if constexpr (S::TM * S::TN >= S::TM + S::TN) { QM_SCHED_PAIR(0x100, S::TM + S::TN * S::kBBlocks) }
+            __builtin_amdgcn_sched_barrier(0);
+            // younger than the requests of step s + 1: those of the STAGES - 2 steps after it, and the scales requested in this
+            // block's first step where that is one of them; the next block's scales, which the block's last step reads, are younger
+            // than all but the requests of two steps
+            constexpr int kPending = (S::STAGES - 2) * S::kLoads + (Q >= 1 && Q <= S::STAGES - 1 ? S::kSLoads : 0);
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm(Q == 3 && kPending > 2 * S::kLoads ? 2 * S::kLoads : kPending));
+            __syncthreads();
+            __builtin_amdgcn_sched_barrier(0);
+            // past the end: a repeat nobody reads keeps the counts of outstanding requests uniform
+            issue(stage, s + S::STAGES < nk ? s + S::STAGES : nk - 1);
+            if constexpr (Q == 0) tile_issue_scales<S>(plan, block_at(s + 4));   // every wave has taken this block's scales
+            if constexpr (Q == 3) tile_read_scales<S>(smem_bytes, a_sc_off, b_sc_off, sc);
+            tile_read<S>(nxt, a_off0, b_off0, f0);
+            tile_mfma<S, 1, SWAP, false>(f1, sca, scb, acc);
+            if constexpr (S::TM * S::TN >= S::TM + S::TN) { QM_SCHED_PAIR(0x100, S::TM + S::TN * S::kBBlocks) }
+            __builtin_amdgcn_sched_barrier(0);
+            stage = nstage;
+        };
+        using Q0 = std::integral_constant<int, 0>;
+        using Q1 = std::integral_constant<int, 1>;
+        using Q2 = std::integral_constant<int, 2>;
+        using Q3 = std::integral_constant<int, 3>;
+        // (four bodies with a way out behind each, instead of a first block, a loop and a tail, are slower: 42 us for 40 at
+        // 4608 x 1536 x 8192, 83 for 71 with the eight-bit B of 4096^3)
+        const auto rest_of_block = [&](int ks) {
+            step(std::false_type{}, Q1{}, ks + 1);
+            step(std::false_type{}, Q2{}, ks + 2);
+            step(std::false_type{}, Q3{}, ks + 3);
+        };
+        step(std::true_type{}, Q0{}, 0);
+        rest_of_block(0);
+        int ks = 4;
+        for (; ks + 4 <= nk; ks += 4) {
+            step(std::false_type{}, Q0{}, ks);
+            rest_of_block(ks);
+        }
+        if (const int left = nk - ks; left > 0) {   // the short block's dwords are the last ones of its 16 bytes
+#pragma unroll
+            for (int i = 0; i < S::TM; ++i) sc.a[i] = rotate_dwords(sc.a[i], 4 - left);
+#pragma unroll
+            for (int j = 0; j < S::TN; ++j) sc.b[j] = rotate_dwords(sc.b[j], 4 - left);
+            step(std::false_type{}, Q0{}, ks);
+            if (left > 1) step(std::false_type{}, Q1{}, ks + 1);
+            if (left > 2) step(std::false_type{}, Q2{}, ks + 2);
+        }
+    } else {
+#pragma unroll
+        for (int s = 0; s < S::STAGES; ++s) issue(s, s < nk ? s : nk - 1);
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm((S::STAGES - 1) * S::kLoads));  // step 0 is in; later ones may be pending
+        __syncthreads();
+        uint32_t sa[S::TM], sb[S::TN];
+        read_dwords<S::TM>(smem_bytes + a_sc_off, sa);
+        read_dwords<S::TN>(smem_bytes + b_sc_off, sb);
+        settle_scales(sa, sb, 0);
+        tile_read<S>(smem_bytes, a_off0, b_off0, f0);
+
+        // one K step: `stage` is the ring slot it consumes and then refills with step s + STAGES
+        auto step = [&](auto first_tag, int s) {
+            constexpr bool FIRST = decltype(first_tag)::value;
+            const int nstage = stage == S::STAGES - 1 ? 0 : stage + 1;
+            const uint8_t* cur = smem_bytes + stage * S::kStageBytes;
+            const uint8_t* nxt = smem_bytes + nstage * S::kStageBytes;
+            uint32_t sca[S::TM], scb[S::TN];
+#pragma unroll
+            for (int i = 0; i < S::TM; ++i) sca[i] = __builtin_amdgcn_ubfe(sa[i], (uint32_t)sh, 16u);
+#pragma unroll
+            for (int j = 0; j < S::TN; ++j) scb[j] = __builtin_amdgcn_ubfe(sb[j], (uint32_t)sh, 16u);
+            tile_read<S>(cur, a_off1, b_off1, f1);
+            tile_mfma<S, 0, SWAP, FIRST>(f0, sca, scb, acc);
+            if constexpr (S::TM * S::TN >= S::TM + S::TN) { QM_SCHED_PAIR(0x100, S::TM + S::TN * S::kBBlocks) }
+            __builtin_amdgcn_sched_barrier(0);
+            // younger than the requests of step s + 1: those of the STAGES - 2 steps after it
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm((S::STAGES - 2) * S::kLoads));
+            __syncthreads();
+            __builtin_amdgcn_sched_barrier(0);
+            // past the end: a repeat nobody reads keeps the counts of outstanding requests uniform
+            issue(stage, s + S::STAGES < nk ? s + S::STAGES : nk - 1);
+            read_dwords<S::TM>(nxt + a_sc_off, sa);
+            read_dwords<S::TN>(nxt + b_sc_off, sb);
+            settle_scales(sa, sb, s + 1);
+            tile_read<S>(nxt, a_off0, b_off0, f0);
+            tile_mfma<S, 1, SWAP, false>(f1, sca, scb, acc);
+            if constexpr (S::TM * S::TN >= S::TM + S::TN) { QM_SCHED_PAIR(0x100, S::TM + S::TN * S::kBBlocks) }
+            __builtin_amdgcn_sched_barrier(0);
+            stage = nstage;
+        };
+        step(std::true_type{}, 0);
+        for (int ks = 1; ks < nk; ++ks) step(std::false_type{}, ks);
+    }
     // every request has landed and every wave has read its last fragments: the ring becomes the staging area
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
     __syncthreads();
@@ -421,7 +536,7 @@ using Tile128x128 = TileShape<128, 128, 64, 64, 3, 3>;
 using Tile128x64 = TileShape<128, 64, 64, 32, 4, 3>;
 using Tile64x64 = TileShape<64, 64, 32, 32, 4, 4>;
 using Tile64x32 = TileShape<64, 32, 32, 32, 6, 4>;
-// with an eight-bit B.  4096^3 in us: 256x256 in 8 waves of 128 x 64, 3 stages 60; in 4 waves of 128 x 128 66; 256x128 73 to 84;
+// with an eight-bit B.  4096^3 alone in us, scales step by step: 256x256 in 8 waves of 128 x 64, 3 stages 60; in 4 waves of 128 x 128 66; 256x128 73 to 84;
 // 128x128 with 2 stages three times per CU 74, with 3 stages twice 81
 using Wide256x256 = TileShape<256, 256, 128, 64, 3, 1, true>;
 using Wide128x128 = TileShape<128, 128, 64, 64, 2, 3, true>;
@@ -437,9 +552,19 @@ bool gemm_tile_serves(int64_t M, int64_t N, int64_t K, int a_tiled, int b_tiled,
 }
 
 hipError_t gemm_tile(int shape, const TileProduct& g, int c_dtype, hipStream_t stream) {
-    const auto go = [&](auto s) {
+    // blocks of scales: every K range has at least four steps, all whole, and scale rows start at multiples of four bytes
+    const bool blocks = g.K % kBK == 0 && g.K / kBK / g.splits >= 4 &&
+                        ((reinterpret_cast<uintptr_t>(g.a_scales) | reinterpret_cast<uintptr_t>(g.b_scales)) & 3) == 0;
+    const auto run = [&](auto s) {
         using S = decltype(s);
         return c_dtype == BF16 ? launch_tiles<S, uint16_t>(g, stream) : launch_tiles<S, float>(g, stream);
+    };
+    // 256 x 128 over fewer than eight steps: its two blocks of 384 rows are more in front of the first step than they save behind it
+    // (4096 x 3456 x 640 in an evaluated model 14 us, 16 with blocks)
+    const auto go = [&](auto s) {
+        using S = decltype(s);
+        const bool few = !S::kWideB && S::BM == 256 && g.K / kBK / g.splits < kShortTallSteps;
+        return blocks && !few ? run(s) : run(typename S::Narrow{});
     };
     if (g.b_e5m2) {
         switch (shape) {

@@ -200,6 +200,7 @@ struct TileProduct {
     int b_e5m2;            // B holds eight-bit values from expand_e5m2_pair (N % 32 == 0, K % 128 == 0, tiled A)
 };
 // the kinds of an eight-bit B are WIDE_256x256 and 1 .. 3
+constexpr int kShortTallSteps = 8;   // see gemm_tile()
 enum TileKind : int { TILE_256x128 = 0, WIDE_256x256 = 0, TILE_128x128 = 1, TILE_128x64 = 2, TILE_64x64 = 3, TILE_64x32 = 4 };
 bool gemm_tile_serves(int64_t M, int64_t N, int64_t K, int a_tiled, int b_tiled, const void* c);
 hipError_t gemm_tile(int kind, const TileProduct& g, int c_dtype, hipStream_t stream);

@@ -150,6 +150,30 @@ def test_gemm_tiled_operands_match_rowmajor(K, M, N, K_, a_tiled, b_tiled):
     assert torch.equal(got16, want.to(torch.bfloat16))
 
 
+# The tile kernels request scales in blocks of four K steps of 128 (from four steps on; 256 x 128 tiles from eight on): three to
+# eleven steps are every length of the last block with and without a whole one in front, on tiles of 64 x 32, 64 x 64, 128 x 64
+# and 128 x 128 (row-major and tiled); 256 x 128 tiles serve the last shape.  Scales differ from row to row and from block to
+# block; every partial sum is a multiple of 1/4 of at most 27 * 128 * 36 * 16 < 2^21, so fp32 holds it exactly.
+@pytest.mark.parametrize("M,N,tiled,steps",
+                         [(*mnt, s) for mnt in [(200, 136, False), (1000, 520, False), (1000, 1032, False), (4352, 4160, True), (4360, 4104, False)]
+                          for s in range(3, 12)] + [(3000, 4104, False, s) for s in (3, 4, 5, 6, 24, 25, 26, 27)])
+def test_tile_kernels_scale_blocks(K, M, N, tiled, steps):
+    print(f"case scale blocks {M}x{N} steps={steps} tiled={tiled}", flush=True)
+    dev, K_ = torch.device("cuda:0"), steps * 128
+    g = torch.Generator(device="cpu").manual_seed(M + N * 3 + steps)
+    ac = torch.randint(0, 256, (M, K_ // 2), generator=g, dtype=torch.uint8).to(dev)
+    bc = torch.randint(0, 256, (N, K_ // 2), generator=g, dtype=torch.uint8).to(dev)
+    as_ = torch.randint(127, 130, (M, K_ // 32), generator=g, dtype=torch.uint8).to(dev)
+    bs = torch.randint(127, 130, (N, K_ // 32), generator=g, dtype=torch.uint8).to(dev)
+    want = _torch_dequant(ac, as_) @ _torch_dequant(bc, bs).T
+    a_in, b_in = (K.tile_codes(ac), K.tile_codes(bc)) if tiled else (ac, bc)
+    got = K.gemm_mxfp4_tn(a_in, as_, b_in, bs, alpha=1.0, out_dtype=torch.float32, a_tiled=tiled, b_tiled=tiled)
+    got16 = K.gemm_mxfp4_tn(a_in, as_, b_in, bs, alpha=1.0, out_dtype=torch.bfloat16, a_tiled=tiled, b_tiled=tiled)
+    torch.cuda.synchronize()
+    assert torch.equal(got.double(), want)
+    assert torch.equal(got16, got.to(torch.bfloat16))
+
+
 @pytest.mark.parametrize("tiled", [False, True])
 def test_gemm_scale_arrays_off_16_byte_alignment(K, tiled):
     """K % 512 == 0 with scale arrays that are 4-byte but not 16-byte aligned: the persistent kernel's 16-byte scale

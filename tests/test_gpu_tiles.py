@@ -216,3 +216,9 @@ def test_error_only_layer_on_packed_operands(oracle, monkeypatch, T, I, O, hd, w
     assert rel(y.detach().float().cpu(), xv @ wv.T) < 4e-3
     assert rel(xd.grad.float().cpu(), rotate(ev @ wv, qx["mask"])) < 4e-3
     assert rel(layer.weight.grad.float().cpu(), rotate(etv @ xv, qw["mask"])) < 4e-3
+
+
+# contractions of 4, 6, 7, 8, 10, 11 and 12 steps of 128: the lengths of the last block of scales that the cases above leave out
+@pytest.mark.parametrize("T,I,O", [(512, 192, 768), (896, 256, 1024), (1280, 320, 1408), (1536, 2048, 896)])
+def test_error_only_layer_on_whole_steps(oracle, monkeypatch, T, I, O):
+    test_error_only_layer_on_packed_operands(oracle, monkeypatch, T, I, O, 32, True, 0)
