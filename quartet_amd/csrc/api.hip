@@ -387,7 +387,7 @@ WorkLayout work_layout(int64_t T, int64_t I, int64_t O, int mid_dtype) {
 }
 // the error-only scheme: Q(e), Q(e^T), the packed operands as eight-bit ones, a product before its rotation (one at a time)
 struct ErrorLayout {
-    size_t ec, es, etc, ets, wv, ws, wl, xv, xs, xl, plain, gemm_ws, gemm_ws_bytes, total;
+    size_t ec, es, etc, ets, wv, ws, wl, wf, xv, xs, xl, xf, plain, gemm_ws, gemm_ws_bytes, total;
 };
 ErrorLayout error_layout(int64_t T, int64_t I, int64_t O) {
     ErrorLayout l;
@@ -396,8 +396,8 @@ ErrorLayout error_layout(int64_t T, int64_t I, int64_t O) {
     const int64_t Tp = qm::padded_cols(T), Op = qm::padded_cols(O);
     take(l.ec, code_bytes(T, O)); take(l.es, scale_bytes(T, O));
     take(l.etc, code_bytes(O, T)); take(l.ets, scale_bytes(O, T));
-    take(l.wv, (size_t)I * Op); take(l.ws, (size_t)I * Op / 32); take(l.wl, (size_t)((I + 127) / 128) * (Op / 128));
-    take(l.xv, (size_t)I * Tp); take(l.xs, (size_t)I * Tp / 32); take(l.xl, (size_t)((I + 127) / 128) * (Tp / 128));
+    take(l.wv, (size_t)I * Op); take(l.ws, (size_t)I * Op / 32); take(l.wl, (size_t)((I + 127) / 128) * (Op / 128)); take(l.wf, (size_t)qm::six_bit_flags(O, I));
+    take(l.xv, (size_t)I * Tp); take(l.xs, (size_t)I * Tp / 32); take(l.xl, (size_t)((I + 127) / 128) * (Tp / 128)); take(l.xf, (size_t)qm::six_bit_flags(T, I));
     take(l.plain, (size_t)(T > O ? T : O) * I * 2);
     const size_t need_x = qm::gemm_e5m2_workspace_bytes(T, I, Op), need_w = qm::gemm_e5m2_workspace_bytes(O, I, Tp);
     l.gemm_ws_bytes = need_x > need_w ? need_x : need_w;
@@ -539,10 +539,10 @@ int qm_linear_backward_error(const void* e, int e_dtype, int64_t T, int64_t I, i
     uint8_t* k = static_cast<uint8_t*>(workspace);
     hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
     const qm::ErrorArgs ae{e, e_dtype, T, O, seeds[0], seeds[1], k + wl.ec, k + wl.es, k + wl.etc, k + wl.ets};
-    int rc = from_hip(qm::quantize_error(ae, hd_g, make_signs(signs_g, hd_g), g_mode, nullptr, hs), "qm_linear_backward_error");
+    const qm::E5m2Args ax{px + lx.c, px + lx.s, T, I, k + wl.xv, k + wl.xs, k + wl.xl, qm::six_bits_serve(qm::padded_cols(T)) ? k + wl.xf : nullptr};
+    const qm::E5m2Args aw{pw + lw.c, pw + lw.s, O, I, k + wl.wv, k + wl.ws, k + wl.wl, qm::six_bits_serve(qm::padded_cols(O)) ? k + wl.wf : nullptr};
+    int rc = from_hip(qm::quantize_error(ae, hd_g, make_signs(signs_g, hd_g), g_mode, ax, aw, hs), "qm_linear_backward_error");
     if (rc) return rc;
-    const qm::E5m2Args ax{px + lx.c, px + lx.s, T, I, k + wl.xv, k + wl.xs, k + wl.xl};
-    const qm::E5m2Args aw{pw + lw.c, pw + lw.s, O, I, k + wl.wv, k + wl.ws, k + wl.wl};
     rc = from_hip(qm::expand_e5m2_pair(ax, aw, hs), "qm_linear_backward_error");
     if (rc) return rc;
     // value = code * 2^k * fl32(4/3) on the error signal, code * 2^k on the saved operand
@@ -553,6 +553,7 @@ int qm_linear_backward_error(const void* e, int e_dtype, int64_t T, int64_t I, i
                               int scale_dtype, const uint8_t* mask, size_t plain) {
         qm::TileProduct p = qm::make_product(k + ac, k + as, b.values, b.scales, M, I, qm::padded_cols(b.R), alpha, out, QM_LAYOUT_TILED, QM_LAYOUT_TILED);
         p.b_e5m2 = 1;
+        p.b_wide = b.wide;
         p.mask = mask;
         p.hd = hd;
         p.signs = make_signs(signs, hd);

@@ -1,19 +1,27 @@
 // Packed MXFP4 [R, C] as the K x N operand of a product that contracts over its rows (the error-only scheme's Q(e) W and
 // Q(e^T) x, backward.py:21-45).  The matrix instruction scales 32 consecutive contraction indices of a column together, but the
 // tensor's E8M0 scales belong to 32 consecutive columns of a row, so codes cannot be multiplied as they are.  They can be
-// widened: within a block of 32 rows and 32 columns every value is a code times a power of two, which E5M2 (two mantissa
-// bits where E2M1 has one, 31 octaves from its smallest subnormal up) holds exactly as long as the row scales of the block lie
-// within 28 octaves of the largest.  Output: E5M2 bytes [C][R padded to 128] in blocks of 16 columns x 64 rows (1 KiB, what one
-// wave requests into LDS), one E8M0 byte per column and 32 rows.  A block of 128 x 128 that holds a value outside the range
-// says so in `lost`, and the columns it touches are computed once more from the packed tensors (ExactJob): results never
-// depend on the spread of the scales.
+// widened: within a block of 32 rows and 32 columns every value is a code times a power of two, which six bits (E3M2: two
+// mantissa bits where E2M1 has one) hold exactly as long as the row scales of the block lie within 5 octaves of the largest, and
+// eight bits (E5M2) within 28.  The matrix instruction takes six bits at the rate of four, eight at half of it, and the bytes
+// count too: the product of 4096^3 runs 58 us with six and 76 with eight.  The format is chosen per block of 512 rows (four K
+// steps) and 256 columns, by its scales alone (expand_formats.h); rows of zeros count for no range.  Rows of activations with
+// outliers of three degrees of freedom stay within 5 octaves but for a block in a hundred or less.
 //
-// Bound by memory: half a byte read and one byte written per element.  A thread takes four consecutive rows and 16 columns;
+// Output: slots of 2 KiB per 16 columns and 128 rows.  Eight bits: 16 columns x 64 rows (1 KiB, what one wave requests into
+// LDS), twice.  Six bits: of every column's 24 bytes per 32 rows the first sixteen, [column][32 rows]; the last eight of
+// 32 columns, [32 rows][column], lie in the second half of the even slot.  One E8M0 byte per column and 32 rows.  A block of 128
+// x 128 that holds a value outside the range says so in `lost`, and the columns it touches are computed once more from the packed
+// tensors (ExactJob): results never depend on the spread of the scales.
+//
+// Bound by memory: half a byte read and three quarters (or one) written per element; 14.6 us for 4096 x 4096 twice (12.9 in eight
+// bits only: packing six bits and the look at the format cost more than the bytes saved).  A thread takes four consecutive rows and 16 columns;
 // v_perm_b32 looks four codes at a time up in an eight-byte table of the row's E5M2 magnitudes, eight more turn 4 x 4 bytes
 // round, and the transposed dwords meet in LDS.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "expand_formats.h"
 #include "qm_jobs.h"
 #include "qm_kernels.h"
 #include "qm_math.h"
@@ -24,9 +32,9 @@ namespace {
 
 constexpr int kTile = 128;                       // rows and columns per workgroup
 constexpr int kColPitch = 128, kGroupPad = 32;   // LDS: 128 bytes per column, 16 columns padded by 32 bytes (banks)
-constexpr int kTop = 13;                         // the largest code, 6 = 1.5 * 2^2, times 2^13 is E5M2's largest 1.5 * 2^15
+constexpr int kTop = 13, kBias = 15;             // E5M2: the largest code, 6 = 1.5 * 2^2, times 2^13 is the largest value used, 1.5 * 2^15
 
-// the E5M2 magnitude bytes of the codes 0 .. 7 times 2^(x - 15), x >= 0; x < 0: zeros
+// the E5M2 or E3M2 magnitude bits of the codes 0 .. 7 times 2^(x - bias), x >= 0; x < 0: zeros
 __device__ __forceinline__ void magnitude_table(int x, uint32_t& lo, uint32_t& hi) {
     // x >= 2: code 1 (0.5) has the exponent field x - 1, codes 2, 3 (1, 1.5) x, 4, 5 x + 1, 6, 7 x + 2; odd codes mantissa 10
     const uint32_t e = 4u * (uint32_t)x;
@@ -63,7 +71,9 @@ struct ExpandJob {
             if (r < R) codes[i] = *reinterpret_cast<const uint2*>(a.codes_in + tiled_code_offset(r + i, bc, csteps) + g * 8);
         }
         job_requests_issued();
+        const bool six = a.wide && a.wide[(int64_t)(bc / 2) * ((ksteps + 3) / 4) + br / 4] == 0;
         __syncthreads();
+        const int top_octaves = six ? kTop6 : kTop, bias = six ? kBias6 : kBias, even_sign = six ? 2 : 4, odd_sign = six ? 2 : 0;
         // per 32 rows the largest scale of each column group: a wave's quads lie in one block of 32 rows
         uint32_t top = 0;
 #pragma unroll
@@ -73,20 +83,20 @@ struct ExpandJob {
         }
         top = max(top, (uint32_t)__shfl_xor((int)top, 16, 64));
         top = max(top, (uint32_t)__shfl_xor((int)top, 32, 64));
-        const int block_scale = top == 255u ? 255 : (int)top - ((int)top < kTop ? (int)top : kTop);
+        const int block_scale = top == 255u ? 255 : (int)top - ((int)top < top_octaves ? (int)top : top_octaves);
         bool lost = false;
         uint32_t even[4][2], odd[4][2];   // row i: bytes of columns 8 h + 0, 2, 4, 6 and 8 h + 1, 3, 5, 7
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int x = 15 + (int)((row_scales[4 * quad + i] >> (8 * (g >> 1))) & 0xffu) - block_scale;
+            const int x = bias + (int)((row_scales[4 * quad + i] >> (8 * (g >> 1))) & 0xffu) - block_scale;
             uint32_t lo, hi;
             magnitude_table(x, lo, hi);
             lost |= x < 0 && top != 255u && ((codes[i].x | codes[i].y) & 0x77777777u);   // a NaN scale: the block is NaN as it is
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const uint32_t w = h ? codes[i].y : codes[i].x;
-                even[i][h] = __builtin_amdgcn_perm(hi, lo, w & 0x07070707u) | ((w & 0x08080808u) << 4);
-                odd[i][h] = __builtin_amdgcn_perm(hi, lo, (w >> 4) & 0x07070707u) | (w & 0x80808080u);
+                even[i][h] = __builtin_amdgcn_perm(hi, lo, w & 0x07070707u) | ((w & 0x08080808u) << even_sign);
+                odd[i][h] = __builtin_amdgcn_perm(hi, lo, (w >> 4) & 0x07070707u) | ((w & 0x80808080u) >> odd_sign);
             }
         }
         // 4 rows x 4 columns of bytes turned round: dword = the four rows of one column
@@ -109,10 +119,25 @@ struct ExpandJob {
         uint8_t* group_scales = reinterpret_cast<uint8_t*>(row_scales);   // everyone has read the row scales
         if (lane < 8 && !(lane & 1)) group_scales[(lane >> 1) * 4 + wave] = (uint8_t)block_scale;
         __syncthreads();
-        // values: blocks of 16 columns x 64 rows, 1 KiB each; a wave writes one at a time
         job_stores_next();
+        const int col = lane >> 2, rows32 = lane & 3;
 #pragma unroll
-        for (int it = 0; it < 4; ++it) {
+        for (int it = 0; it < 2 && six; ++it) {   // 16 columns, 32 rows of one to a lane: 24 bytes, sixteen of them and eight apart
+            const int cg = it * 4 + wave;
+            if (c0 + cg * 16 < C) {
+                const uint4* src = reinterpret_cast<const uint4*>(turned + cg * (16 * kColPitch + kGroupPad) + col * kColPitch + rows32 * 32);
+                const uint4 v0 = src[0], v1 = src[1];
+                const auto pack = [](uint32_t v) { return __builtin_amdgcn_udot4(v, 0x4001u, 0u, false) | (__builtin_amdgcn_udot4(v, 0x40010000u, 0u, false) << 12); };
+                const uint32_t w0 = pack(v0.x), w1 = pack(v0.y), w2 = pack(v0.z), w3 = pack(v0.w), w4 = pack(v1.x), w5 = pack(v1.y), w6 = pack(v1.z), w7 = pack(v1.w);
+                uint8_t* panel = a.values + (((int64_t)(c0 / 16 + cg) * ksteps + br) << 11);
+                *reinterpret_cast<uint4*>(panel + lane * 16) = make_uint4(w0 | (w1 << 24), (w1 >> 8) | (w2 << 16), (w2 >> 16) | (w3 << 8), w4 | (w5 << 24));
+                uint8_t* pair = a.values + (((int64_t)((c0 / 16 + cg) & ~1) * ksteps + br) << 11);
+                *reinterpret_cast<uint2*>(pair + 1024 + rows32 * 256 + ((cg & 1) * 16 + col) * 8) = make_uint2((w5 >> 8) | (w6 << 16), (w6 >> 16) | (w7 << 8));
+            }
+        }
+        // eight bits: blocks of 16 columns x 64 rows, 1 KiB each; a wave writes one at a time
+#pragma unroll
+        for (int it = 0; it < 4 && !six; ++it) {
             const int block = it * 4 + wave, cg = block >> 1, half = block & 1;   // 16 blocks of the workgroup
             if (c0 + cg * 16 < C) {
                 const uint4 v = *reinterpret_cast<const uint4*>(turned + cg * (16 * kColPitch + kGroupPad) + (lane >> 2) * kColPitch + half * 64 + (lane & 3) * 16);

@@ -845,11 +845,11 @@ constexpr KernelCost kTileCosts[] = {{256, 128, 2, 0.461, 0.488, 5.6, {10.0, 12.
                                      {64, 32, 4, 0.099, 0.091, 0.71, {0.7, 0.0, 0.0}, {0.7, 0.0, 0.0}}};
 // 256 x 128 tiles over fewer than kShortTallSteps K steps, which request their scales step by step
 constexpr KernelCost kShortTall = {256, 128, 2, 0.60, 0.68, 2.5, {10.0, 12.0, 14.0}, {10.0, 12.0, 14.0}};
-// with an eight-bit B (70 shapes, cuts included: mean error 9 %, 2.9 % from the fastest choice on average)
-constexpr KernelCost kWideTileCosts[] = {{256, 256, 1, 1.068, 1.068, 8.0, {9.0, 10.9, 12.3}, {9.0, 10.9, 12.3}},
-                                         {128, 128, 3, 0.203, 0.560, 1.1, {6.0, 7.5, 9.0}, {1.5, 3.8, 5.0}},
-                                         {128, 64, 3, 0.246, 0.393, 0.42, {2.4, 3.6, 0.0}, {0.8, 2.2, 0.0}},
-                                         {64, 64, 3, 0.196, 0.297, 0.60, {1.0, 1.5, 0.0}, {0.8, 1.4, 0.0}}};
+// with a B of six or eight bits (expand.hip; six bits in 14 shapes of 512 x 640 x 2048 to 4096^3, rotation included)
+constexpr KernelCost kWideTileCosts[] = {{256, 256, 1, 1.14, 1.14, 4.0, {9.0, 10.9, 12.3}, {10.0, 11.0, 12.3}},
+                                         {128, 128, 3, 0.45, 0.33, 3.0, {7.0, 8.0, 9.0}, {2.0, 3.8, 5.0}},
+                                         {128, 64, 3, 0.31, 0.24, 1.0, {2.4, 3.6, 0.0}, {0.8, 2.2, 0.0}},
+                                         {64, 64, 3, 0.21, 0.18, 0.60, {1.0, 1.5, 0.0}, {0.8, 1.4, 0.0}}};
 const KernelCost& tile_costs(bool e5m2, int kind, int64_t K, int splits) {
     if (!e5m2 && kind == TILE_256x128 && K / kBK / splits < kShortTallSteps) return kShortTall;
     return (e5m2 ? kWideTileCosts : kTileCosts)[kind];

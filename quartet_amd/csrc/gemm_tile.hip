@@ -15,10 +15,10 @@
 // and exist to put more workgroups on the chip.  Accumulation order over K is the same in every shape and in gemm.hip's
 // kernels: results depend on the choice only where a product is cut into K ranges.  (gemm_rows.hip's order is its own.)
 //
-// The same kernel multiplies FP4 with an eight-bit (E5M2) B, which is how the error-only scheme contracts over the rows of a
-// packed operand (expand.hip): twice the bytes and twice the matrix cycles of B.  4096^3 among the other kernels of a training
-// step: 74 us (76 with scales step by step), 8 waves of 128 x 64 on 256 x 256 with the matrix pipe over 60 % busy at the clock its
-// power allows, where the FP4 x bf16 kernel (gemm_fp4_bf16.hip) takes 113 us and more.
+// The same kernel multiplies FP4 with a B of six (E3M2) or eight (E5M2) bits, which is how the error-only scheme contracts over
+// the rows of a packed operand (expand.hip): 1.5 times the bytes of B at FP4's matrix rate, or twice the bytes at half of it.  4096^3
+// among the other kernels of a training step, 8 waves of 128 x 64 on 256 x 256: 58 us in six bits, 74 in eight, where the FP4 x
+// bf16 kernel (gemm_fp4_bf16.hip) takes 113 us and more.  4 waves of 128 x 128 read a third fewer bytes from LDS and take 67.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -36,16 +36,19 @@ namespace {
 // takes its rows' into registers (K >= 512 and 4-byte aligned scale rows).  Otherwise one dword per row and K step, in the ring:
 // every dword lies in another line, and those requests are two thirds of all.  4608 x 1536 x 8192 55 -> 40 us,
 // 2048 x 4096 x 4096 32 -> 25, 512 x 11008 x 4096 27 -> 22; without any scale requests (wrong results) 37, 22 and 19.
-template <int BM_, int BN_, int WM_, int WN_, int STAGES_, int OCC_, bool E5M2_B = false, bool BLOCKS_ = true>
+template <int BM_, int BN_, int WM_, int WN_, int STAGES_, int OCC_, bool E5M2_B = false, bool BLOCKS_ = true, bool MIXED_ = false>
 struct TileShape {
     using Narrow = TileShape<BM_, BN_, WM_, WN_, STAGES_, OCC_, E5M2_B, false>;
+    using Mixed = TileShape<BM_, BN_, WM_, WN_, STAGES_, OCC_, true, true, true>;
     static constexpr bool kBlocks = BLOCKS_;
     static constexpr bool kWideB = E5M2_B;
+    static constexpr bool kMixed = MIXED_;   // blocks of four K steps and 256 columns of B in six or eight bits each
     static constexpr int kBBlocks = E5M2_B ? 2 : 1;
     static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, STAGES = STAGES_, OCC = OCC_;   // OCC: workgroups per CU
     static constexpr int kWavesN = BN / WN, kWaves = (BM / WM) * kWavesN, kThreads = kWaves * 64;
     static constexpr int TM = WM / 32, TN = WN / 32;
     static constexpr int kALoads = BM / 16 / kWaves, kBLoads = BN / 16 * kBBlocks / kWaves;   // 1 KiB wave-loads per wave and K step
+    static constexpr int kUnits6 = BN / 16 + BN / 32, kBLoads6 = (kUnits6 + kWaves - 1) / kWaves;   // six-bit B
     static constexpr int kAUnits = (BM + 63) / 64, kUnits = kAUnits + (BN + 63) / 64;   // requests of 64 rows' scales each
     static constexpr int kSLoads = (kUnits + kWaves - 1) / kWaves;
     static constexpr int kLoads = kALoads + kBLoads + (kBlocks ? 0 : kSLoads);   // requests per wave and K step
@@ -54,7 +57,8 @@ struct TileShape {
     static constexpr int kBOff = BM * kRowBytes, kCodeBytes = (BM + BN * kBBlocks) * kRowBytes;
     static constexpr int kStageBytes = kCodeBytes + (kBlocks ? 0 : kUnits * kUnitBytes);
     static constexpr int kSAOff = kBlocks ? STAGES * kStageBytes : kCodeBytes, kSBOff = kSAOff + kAUnits * kUnitBytes;
-    static constexpr int kRingBytes = STAGES * kStageBytes + (kBlocks ? kUnits * kUnitBytes : 0);
+    static constexpr int kFlagOff = STAGES * kStageBytes + (kBlocks ? kUnits * kUnitBytes : 0);
+    static constexpr int kRingBytes = kFlagOff + (kMixed ? kMaxSixBlocks / 8 : 0);
     static constexpr int kMUnits = BM * BN / 2048, kMLoads = (kMUnits + kWaves - 1) / kWaves;   // mask words of the tile, 64 at a time
     // ahead of the operands where there is room beside the ring for OCC workgroups per CU
     static constexpr bool kMaskEarly = BM < 256 && (kRingBytes + kMUnits * 256) * OCC <= 160 * 1024;
@@ -144,6 +148,37 @@ __device__ __forceinline__ uint4 rotate_dwords(uint4 v, int by) {
     return v;
 }
 
+// The blocks of four K steps from `first` up to `end` whose format flag is `want`, in ascending order.  flags: one bit per block,
+// in LDS; every wave walks them alike.
+struct BlockWalk {
+    const uint64_t* flags;
+    uint64_t word;
+    int base, end;
+    uint32_t invert;
+    __device__ __forceinline__ uint64_t load(int at) const {
+        const uint2 v = *reinterpret_cast<const uint2*>(flags + (at >> 6));
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)v.x), hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)v.y);
+        return ((uint64_t)(hi ^ invert) << 32) | (lo ^ invert);
+    }
+    __device__ __forceinline__ BlockWalk(const uint8_t* f, int first, int last, bool want)
+        : flags(reinterpret_cast<const uint64_t*>(f)), base(first & ~63), end(last), invert(want ? 0u : ~0u) {
+        word = load(base) & (~0ull << (first & 63));
+    }
+    __device__ __forceinline__ int next() {   // `end` behind the last one, and from then on
+        while (!word) {
+            if (base + 64 >= end) return end;
+            base += 64;
+            word = load(base);
+        }
+        const int b = base + __builtin_ctzll(word);
+        word &= word - 1;
+        return b < end ? b : end;
+    }
+};
+
+// `count` of them (uniform), zeros behind
+__device__ __forceinline__ uint4 first_dwords(uint4 v, int count) { return make_uint4(v.x, count > 1 ? v.y : 0u, count > 2 ? v.z : 0u, 0u); }
+
 template <class S>
 struct TileFrags {
     uint4 a[S::TM], b[S::TN * S::kBBlocks];
@@ -159,18 +194,17 @@ __device__ __forceinline__ void tile_read(const uint8_t* __restrict__ stage, int
             f.b[j * S::kBBlocks + q] = *reinterpret_cast<const uint4*>(stage + b_off + q * S::BN * kRowBytes + j * 32 * kRowBytes);
 }
 // SWAP: B's rows (n) are the instruction's first operand, so a lane ends up with quads of consecutive n of one m
-template <class S, int SUB, bool SWAP, bool ZERO>
-__device__ __forceinline__ void tile_mfma(const TileFrags<S>& f, const uint32_t (&sca)[S::TM], const uint32_t (&scb)[S::TN],
-                                          v16f (&acc)[S::TM][S::TN]) {
-#pragma unroll
-    for (int i = 0; i < S::TM; ++i) {
+template <class S, int SUB, bool SWAP, bool ZERO, bool SIX = false>
+__device__ __forceinline__ void tile_mfma_row(int i, const TileFrags<S>& f, const uint32_t (&sca)[S::TM], const uint32_t (&scb)[S::TN],
+                                              v16f (&acc)[S::TM][S::TN]) {
+    {
         const v8i av = v8i{(int)f.a[i].x, (int)f.a[i].y, (int)f.a[i].z, (int)f.a[i].w, 0, 0, 0, 0};
 #pragma unroll
         for (int j = 0; j < S::TN; ++j) {
             // eight-bit operand: a lane holds sixteen bytes of either block of 32 indices, low registers first (FP4: a whole block)
             const uint4 b0 = f.b[j * S::kBBlocks], b1 = S::kWideB ? f.b[j * S::kBBlocks + S::kBBlocks - 1] : make_uint4(0u, 0u, 0u, 0u);
             const v8i bv = v8i{(int)b0.x, (int)b0.y, (int)b0.z, (int)b0.w, (int)b1.x, (int)b1.y, (int)b1.z, (int)b1.w};
-            constexpr int kFmtB = S::kWideB ? 1 : 4;   // E5M2, E2M1
+            constexpr int kFmtB = SIX ? 3 : S::kWideB ? 1 : 4;   // E3M2 (24 of the 32 bytes count), E5M2, E2M1
             v16f cin;
             if constexpr (ZERO) {
 #pragma unroll
@@ -184,6 +218,13 @@ __device__ __forceinline__ void tile_mfma(const TileFrags<S>& f, const uint32_t 
                 acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(av, bv, cin, 4, kFmtB, SUB, (int)sca[i], SUB, (int)scb[j]);
         }
     }
+}
+
+template <class S, int SUB, bool SWAP, bool ZERO, bool SIX = false>
+__device__ __forceinline__ void tile_mfma(const TileFrags<S>& f, const uint32_t (&sca)[S::TM], const uint32_t (&scb)[S::TN],
+                                          v16f (&acc)[S::TM][S::TN]) {
+#pragma unroll
+    for (int i = 0; i < S::TM; ++i) tile_mfma_row<S, SUB, SWAP, ZERO, SIX>(i, f, sca, scb, acc);
 }
 
 template <class S, typename OutT>
@@ -201,7 +242,7 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
     // instantiation only), stores its partial sums, unscaled, into slab r of c = [splits][M][N]
     const int tiles = tiles_m * tiles_n, range = t / tiles;
     const int nk_all = (K + kBK - 1) / kBK;
-    const int k_first = range * nk_all / g.splits, nk = (range + 1) * nk_all / g.splits - k_first;
+    const int k_first = S::kMixed ? 0 : range * nk_all / g.splits, nk = (range + 1) * nk_all / g.splits - k_first;
     const int half_step = (K % kBK) && range == g.splits - 1 ? nk - 1 : -1;  // the K step that covers only 64 indices (K % 128 == 64), or none
     int tm, tn;
     tile_of_block<(S::BM >= 256 ? 4 : 8)>(t - range * tiles, tiles_m, tiles_n, tm, tn);
@@ -296,7 +337,141 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
     TileFrags<S> f0, f1;
     v16f acc[S::TM][S::TN];
     int stage = 0;
-    if constexpr (S::kBlocks) {
+    if constexpr (S::kMixed) {
+        // B's blocks of four K steps in six bits, then those in eight: two passes of the same loop, each over its blocks, so that a
+        // block costs what its format does (all in eight bits: as without this; every second one: half way).  The short last block
+        // of a K that is no multiple of four steps is filled up with muted ones: a tail of its own, as below, makes the compiler
+        // keep the accumulators in memory.
+        const int blocks_all = (nk_all + 3) / 4, b_end = (range + 1) * blocks_all / g.splits;
+        const uint8_t* flags = g.b_wide + (int64_t)(n0 / kWideStrip) * blocks_all;
+        for (int base = wave * 64; base < blocks_all; base += S::kThreads) {
+            const uint64_t bits = __builtin_amdgcn_ballot_w64(base + lane < blocks_all && flags[base + lane < blocks_all ? base + lane : 0] != 0);
+            if (lane == 0) *reinterpret_cast<uint2*>(smem_bytes + S::kFlagOff + base / 8) = make_uint2((uint32_t)bits, (uint32_t)(bits >> 32));
+        }
+#pragma unroll
+        for (int i = 0; i < S::TM; ++i)
+#pragma unroll
+            for (int j = 0; j < S::TN; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+        __syncthreads();
+        const auto phase = [&](auto six_tag) {
+            constexpr bool SIX = decltype(six_tag)::value;
+            constexpr int kB = SIX ? S::kBLoads6 : S::kBLoads, kLoads = S::kALoads + kB;
+            BlockWalk walk(smem_bytes + S::kFlagOff, range * blocks_all / g.splits, b_end, !SIX);
+            int block = walk.next();
+            if (block == b_end) return;
+            uint32_t voff_b[kB], lds_b[kB];
+#pragma unroll
+            for (int j = 0; j < kB; ++j) {
+                // six bits: every column's 16 bytes of a block of 32 indices, then, by 32 columns, its 8 bytes
+                const int u = SIX ? (wave * kB + j) % S::kUnits6 : wave * kB + j, pair = u - S::BN / 16;
+                if (SIX && pair >= 0) {
+                    const int last_pair = (N - 1 - n0) >> 5;
+                    voff_b[j] = (uint32_t)(pair < last_pair ? pair : last_pair) * (uint32_t)(32 * K) + 1024u + lane * 16;
+                } else {
+                    const int r = (u % (S::BN / 16)) * 16 + (lane >> 2), rr = r < N - 1 - n0 ? r : N - 1 - n0;
+                    voff_b[j] = (uint32_t)(rr >> 4) * (uint32_t)(16 * K) + (uint32_t)((u / (S::BN / 16)) * 1024 + (rr & 15) * 64 + ((lane & 3) ^ ((lane >> 4) & 3)) * 16);
+                }
+                lds_b[j] = (uint32_t)__builtin_amdgcn_readfirstlane((int)(smem_base + S::kBOff + u * 1024));
+            }
+            const auto issue_one = [&](int slot, int ks, int l) {
+                ks = ks < nk_all ? ks : nk_all - 1;
+                const uint32_t off = (uint32_t)slot * S::kStageBytes;
+                if (l < S::kALoads) load_lds_b128_s(plan.a + (int64_t)ks * plan.kstep_a, plan.voff_a[l], plan.lds_a + off + l * 1024);
+                else load_lds_b128_s(plan.b + (int64_t)ks * plan.kstep_b, voff_b[l - S::kALoads], lds_b[l - S::kALoads] + off);
+            };
+            const auto issue = [&](int slot, int ks) {
+#pragma unroll
+                for (int l = 0; l < kLoads; ++l) issue_one(slot, ks, l);
+            };
+            const auto scales_at = [&](int b) { return 4 * b + 4 <= nk_all ? 4 * b : nk_all - 4; };   // the last block: its row's final 16 bytes
+            const auto read_row = [&](const uint8_t* slot, int sub, TileFrags<S>& f, int i) {
+                f.a[i] = *reinterpret_cast<const uint4*>(slot + (sub ? a_off1 : a_off0) + i * 32 * kRowBytes);
+                if (const int j = i; j < S::TN) {
+                    if constexpr (SIX) {
+                        const int piece = 2 * half + sub;
+                        f.b[2 * j] = *reinterpret_cast<const uint4*>(slot + S::kBOff + (wn * S::WN + j * 32 + lrow) * kRowBytes + ((piece ^ swz) * 16));
+                        const uint2 v = *reinterpret_cast<const uint2*>(slot + S::kBOff + S::BN * kRowBytes + (wn * (S::WN / 32) + j) * 1024 + piece * 256 + lrow * 8);
+                        f.b[2 * j + 1] = make_uint4(v.x, v.y, 0u, 0u);
+                    } else {
+                        f.b[2 * j] = *reinterpret_cast<const uint4*>(slot + (sub ? b_off1 : b_off0) + j * 32 * kRowBytes);
+                        f.b[2 * j + 1] = *reinterpret_cast<const uint4*>(slot + (sub ? b_off1 : b_off0) + S::BN * kRowBytes + j * 32 * kRowBytes);
+                    }
+                }
+            };
+            const auto read = [&](const uint8_t* slot, int sub, TileFrags<S>& f) {
+#pragma unroll
+                for (int i = 0; i < S::TM; ++i) read_row(slot, sub, f, i);
+            };
+            int stage = 0;
+            tile_issue_scales<S>(plan, scales_at(block));
+#pragma unroll
+            for (int s = 0; s < S::STAGES; ++s) issue(s, 4 * block + s);
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm((S::STAGES - 1) * kLoads));
+            __syncthreads();
+            TileScales<S> sc;
+            tile_read_scales<S>(smem_bytes, a_sc_off, b_sc_off, sc);
+            read(smem_bytes, 0, f0);
+            int next = block;
+            // one K step, as below; the requests of a block's last steps are the first ones of the block that follows it here.
+            // Requests, reads and products dealt out by 32 rows, where they otherwise stand between the barrier and the first
+            // product: 59.2 -> 58.3 us at 4096^3.
+            auto step = [&](auto q_tag) {
+                constexpr int Q = decltype(q_tag)::value;
+                const int nstage = stage == S::STAGES - 1 ? 0 : stage + 1;
+                const uint8_t* cur = smem_bytes + stage * S::kStageBytes;
+                const uint8_t* nxt = smem_bytes + nstage * S::kStageBytes;
+                uint32_t sca[S::TM], scb[S::TN];
+#pragma unroll
+                for (int i = 0; i < S::TM; ++i) sca[i] = __builtin_amdgcn_ubfe(dword_of<Q>(sc.a[i]), (uint32_t)sh, 16u);
+#pragma unroll
+                for (int j = 0; j < S::TN; ++j) scb[j] = __builtin_amdgcn_ubfe(dword_of<Q>(sc.b[j]), (uint32_t)sh, 16u);
+                read(cur, 1, f1);
+                tile_mfma<S, 0, SWAP, false, SIX>(f0, sca, scb, acc);
+                if constexpr (S::TM * S::TN >= S::TM + S::TN) { QM_SCHED_PAIR(0x100, S::TM + S::TN * 2) }
+                __builtin_amdgcn_sched_barrier(0);
+                constexpr int kPending = (S::STAGES - 2) * kLoads + (Q >= 1 && Q <= S::STAGES - 1 ? S::kSLoads : 0);
+                __builtin_amdgcn_s_waitcnt(vmcnt_imm(Q == 3 && kPending > 2 * kLoads ? 2 * kLoads : kPending));
+                __syncthreads();
+                __builtin_amdgcn_sched_barrier(0);
+                const int ks = Q + S::STAGES < 4 ? 4 * block + Q + S::STAGES : 4 * next + Q + S::STAGES - 4;
+                if constexpr (Q == 3) tile_read_scales<S>(smem_bytes, a_sc_off, b_sc_off, sc);
+#pragma unroll
+                for (int i = 0; i < S::TM; ++i) {   // a request or two, the reads, the products of every 32 rows
+#pragma unroll
+                    for (int l = i * kLoads / S::TM; l < (i + 1) * kLoads / S::TM; ++l) issue_one(stage, ks, l);
+                    if (Q == 0 && i == S::TM - 1) tile_issue_scales<S>(plan, scales_at(next));
+                    read_row(nxt, 0, f0, i);
+                    tile_mfma_row<S, 1, SWAP, false, SIX>(i, f1, sca, scb, acc);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                stage = nstage;
+            };
+            for (bool more = true; more;) {
+                // K no multiple of four steps: the last block's dwords are the last ones of its 16 bytes, and the steps that it
+                // lacks repeat its last one with scales of 2^-127 on both sides, whose products vanish
+                if (const int left = nk_all - 4 * block; left < 4) {
+#pragma unroll
+                    for (int i = 0; i < S::TM; ++i) sc.a[i] = first_dwords(rotate_dwords(sc.a[i], 4 - left), left);
+#pragma unroll
+                    for (int j = 0; j < S::TN; ++j) sc.b[j] = first_dwords(rotate_dwords(sc.b[j], 4 - left), left);
+                }
+                next = walk.next();
+                more = next < b_end;
+                next = more ? next : block;
+                step(std::integral_constant<int, 0>{});
+                step(std::integral_constant<int, 1>{});
+                step(std::integral_constant<int, 2>{});
+                step(std::integral_constant<int, 3>{});
+                block = next;
+            }
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+            __syncthreads();
+        };
+        phase(std::true_type{});
+        phase(std::false_type{});
+    } else if constexpr (S::kBlocks) {
         // blocks of four K steps; the last block of an nk that is no multiple of four requests the row's final 16 bytes, whose
         // first dwords the block before has used
         const auto block_at = [&](int ks) { return ks + 4 <= nk ? ks : nk - 4; };
@@ -564,6 +739,8 @@ hipError_t gemm_tile(int shape, const TileProduct& g, int c_dtype, hipStream_t s
     const auto go = [&](auto s) {
         using S = decltype(s);
         const bool few = !S::kWideB && S::BM == 256 && g.K / kBK / g.splits < kShortTallSteps;
+        if constexpr (S::kWideB)
+            if (g.b_wide) return run(typename S::Mixed{});
         return blocks && !few ? run(s) : run(typename S::Narrow{});
     };
     if (g.b_e5m2) {

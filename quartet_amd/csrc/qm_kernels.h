@@ -104,11 +104,9 @@ struct ErrorArgs {        // e [T, O], quantized along its rows and, transposed,
 // grid.  seed_base: null, or device memory holding a value the kernels add to every seed when they run.
 hipError_t quantize_layer_backward(const ErrorArgs& e, int hd, const SignBits& signs, int mode, const RequantArgs& x, const RequantArgs& w,
                                    const uint64_t* seed_base, hipStream_t stream);
-// the two quantizations of e alone
-hipError_t quantize_error(const ErrorArgs& e, int hd, const SignBits& signs, int mode, const uint64_t* seed_base, hipStream_t stream);
 // Packed quest-coded tensors [R, C] (padded tiled codes; R and C multiples of 32) as operands of products that contract
-// over R (expand.hip): E5M2 bytes, padded_rows(C) * padded_cols(R) of them, E8M0 scales [C][padded_cols(R) / 32], and one
-// byte per 128 x 128 block, [ceil(C / 128)][padded_cols(R) / 128], nonzero where the block has a value that E5M2 cannot hold
+// over R (expand.hip): E3M2 or E5M2 values in padded_rows(C) * padded_cols(R) bytes, E8M0 scales [C][padded_cols(R) / 32], and
+// one byte per 128 x 128 block, [ceil(C / 128)][padded_cols(R) / 128], nonzero where the block has a value that its format cannot hold
 struct E5m2Args {
     const uint8_t* codes_in;
     const uint8_t* scales_in;
@@ -116,7 +114,18 @@ struct E5m2Args {
     uint8_t* values;
     uint8_t* scales;
     uint8_t* lost;
+    uint8_t* wide;   // [ceil(C / kWideStrip)][blocks of four K steps]: nonzero where the block is in eight bits; null: all of it is
 };
+constexpr int kWideStrip = 256, kMaxSixBlocks = 2048;
+// Contractions that may be in six bits: whole blocks of four steps, of which padding is an eighth at most, and flags that fit
+// beside the ring
+inline bool six_bits_serve(int64_t K) {
+    const int64_t steps = K / 128, blocks = (steps + 3) / 4;
+    return steps >= 4 && (4 * blocks - steps) * 8 <= steps && blocks <= kMaxSixBlocks;
+}
+inline int64_t six_bit_flags(int64_t R, int64_t C) { return (C + kWideStrip - 1) / kWideStrip * (((R + 127) / 128 + 3) / 4); }
+// both quantizations of the error signal, and the formats of the operands that their products take (E5m2Args::wide)
+hipError_t quantize_error(const ErrorArgs& e, int hd, const SignBits& signs, int mode, const E5m2Args& x, const E5m2Args& w, hipStream_t stream);
 hipError_t expand_e5m2_pair(const E5m2Args& a, const E5m2Args& b, hipStream_t stream);
 // The columns of a product that such a loss touches, once more and from the packed tensors: c = the masked inverse rotation of
 // bf16(alpha * A B), A [M, K] tiled codes, B the packed [R, C] tensor behind `b`.  Two products in one launch, which ends at
@@ -197,7 +206,8 @@ struct TileProduct {
     SignBits signs;
     float rot_c;
     int out_f32;
-    int b_e5m2;            // B holds eight-bit values from expand_e5m2_pair (N % 32 == 0, K % 128 == 0, tiled A)
+    int b_e5m2;            // B holds values from expand_e5m2_pair (N % 32 == 0, K % 128 == 0, tiled A)
+    const uint8_t* b_wide; // its formats (E5m2Args::wide), or null: eight bits everywhere
 };
 // the kinds of an eight-bit B are WIDE_256x256 and 1 .. 3
 constexpr int kShortTallSteps = 8;   // see gemm_tile()

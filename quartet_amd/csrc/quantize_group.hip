@@ -35,6 +35,7 @@
 
 #include <type_traits>
 
+#include "expand_formats.h"
 #include "lds_requests.h"
 #include "qm_jobs.h"
 #include "qm_kernels.h"
@@ -1473,9 +1474,9 @@ hipError_t with_error_jobs(const ErrorArgs& a, int hd, const SignBits& signs, in
 bool ragged_extents(int64_t a, int64_t b) { return a % 128 != 0 || b % 128 != 0; }
 }  // namespace
 
-hipError_t quantize_error(const ErrorArgs& e, int hd, const SignBits& signs, int mode, const uint64_t* seed_base, hipStream_t stream) {
-    return with_error_jobs(e, hd, signs, mode, seed_base, ragged_extents(e.T, e.O),
-                           [&](const auto& jt, const auto& jr, auto, auto, auto) { launch_jobs(stream, jt, jr); });
+hipError_t quantize_error(const ErrorArgs& e, int hd, const SignBits& signs, int mode, const E5m2Args& x, const E5m2Args& w, hipStream_t stream) {
+    return with_error_jobs(e, hd, signs, mode, nullptr, ragged_extents(e.T, e.O),
+                           [&](const auto& jt, const auto& jr, auto, auto, auto) { launch_jobs(stream, SpanJob(x), SpanJob(w), jt, jr); });
 }
 
 hipError_t quantize_layer_backward(const ErrorArgs& e, int hd, const SignBits& signs, int mode, const RequantArgs& x, const RequantArgs& w,

@@ -218,7 +218,50 @@ def test_error_only_layer_on_packed_operands(oracle, monkeypatch, T, I, O, hd, w
     assert rel(layer.weight.grad.float().cpu(), rotate(etv @ xv, qw["mask"])) < 4e-3
 
 
-# contractions of 4, 6, 7, 8, 10, 11 and 12 steps of 128: the lengths of the last block of scales that the cases above leave out
-@pytest.mark.parametrize("T,I,O", [(512, 192, 768), (896, 256, 1024), (1280, 320, 1408), (1536, 2048, 896)])
-def test_error_only_layer_on_whole_steps(oracle, monkeypatch, T, I, O):
-    test_error_only_layer_on_packed_operands(oracle, monkeypatch, T, I, O, 32, True, 0)
+# contractions of 4, 6, 7, 8, 10, 11, 12 and 33 steps of 128: whole and short last blocks of four steps.  From 4, 8, 11, 12, ... steps
+# on, blocks of 512 rows and 256 columns whose row scales lie within five octaves are widened to six bits, others to eight.
+@pytest.mark.parametrize("T,I,O,spread", [(512, 192, 768, 0), (896, 256, 1024, 0), (1280, 320, 1408, 0), (1536, 2048, 896, 0)] +
+                         [(*case, s) for case in [(512, 320, 512), (1536, 96, 1408), (4224, 544, 640)] for s in (4, 5, 6, 12)])
+def test_error_only_layer_on_whole_steps(oracle, monkeypatch, T, I, O, spread):
+    test_error_only_layer_on_packed_operands(oracle, monkeypatch, T, I, O, 32, True, spread)
+
+
+@pytest.mark.parametrize("T,I,O", [(4224, 544, 1408), (2048, 2048, 4096)])
+def test_error_only_layer_with_both_widths_in_one_product(oracle, T, I, O):
+    """Outliers in single blocks of 512 rows and 256 columns, the last block among them, zero rows (which count for no range) and
+    rows as small as a zero group's scale: every column group of 32 against float64, with the tolerance of the test above."""
+    print(f"case error-only widths T={T} I={I} O={O}", flush=True)
+    import quartet_amd as q
+    x = make_input(T, I, torch.bfloat16, seed=1, outlier_frac=0).float()
+    w = make_input(O, I, torch.bfloat16, seed=2, outlier_frac=0, scale=0.02).float()
+    x[600:640, 256:300] *= 2.0 ** 7
+    x[T - 20:, :32] *= 2.0 ** 9
+    x[1030:1040] = 0.0
+    x[1100:1110, 64:96] *= 2.0 ** -24
+    x[1600:1610, I - 32:] *= 2.0 ** -28
+    w[O - 3, 300:320] *= 2.0 ** 8
+    x, w = x.to(torch.bfloat16), w.to(torch.bfloat16)
+    e = make_input(T, O, torch.bfloat16, seed=3, outlier_frac=0, scale=1e-3)
+    layer = error_only_layer(q, I, O, 32, torch.bfloat16)
+    with torch.no_grad():
+        layer.weight.copy_(w.to("cuda:0"))
+    xd = x.to("cuda:0").requires_grad_(True)
+    random.seed(5)
+    layer(xd).backward(e.to("cuda:0"))
+    torch.cuda.synchronize()
+    random.seed(5)
+    o, d = oracle, float(oracle.FOUR_THIRDS)
+    qx, qw = (o.quantize(to_oracle(t), 32, mode=o.QUEST_RTN, want_mask=True) for t in (x, w))
+    qe = o.quantize(to_oracle(e), 32, mode=o.ABSMAX_SR, seed=random.getrandbits(63))
+    qet = o.quantize(to_oracle(e), 32, mode=o.ABSMAX_SR, transposed_in=True, seed=random.getrandbits(63))
+    on_gpu = lambda t, scale: torch.from_numpy(o.dequantize(t["codes"], t["scales"], scale)).to("cuda:0").double()
+    parity = torch.tensor([[bin(i & j).count("1") & 1 for j in range(32)] for i in range(32)], device="cuda:0")
+    H = torch.where(parity == 1, -1.0, 1.0).double() * float(torch.tensor(32 ** -0.5).to(torch.bfloat16))
+
+    def groups(p, mask):   # the bf16 product, masked and rotated, as groups of 32 columns
+        keep = torch.from_numpy(np.unpackbits(np.asarray(mask).reshape(p.shape[0], -1), axis=1, bitorder="little")).to("cuda:0")
+        return (p.to(torch.bfloat16).double() * keep).view(p.shape[0], -1, 32) @ H
+    for got, want in [(xd.grad, groups(on_gpu(qe, d) @ on_gpu(qw, 1.0), qx["mask"])),
+                      (layer.weight.grad, groups(on_gpu(qet, d) @ on_gpu(qx, 1.0), qw["mask"]))]:
+        err = (got.double().view(want.shape) - want).square().sum((0, 2)).sqrt() / want.square().sum((0, 2)).sqrt()
+        assert float(err.max()) < 4e-3, float(err.max())
