@@ -29,8 +29,10 @@ constexpr int kRowsDepth = 4;   // K steps requested ahead of the products
 template <int TM, int WAVES, typename OutT>
 __device__ __forceinline__ void add_waves(v4f (&partial)[WAVES][TM][64], const v4f (&acc)[TM], int wave, int lane, int n0, int M, int N, float alpha,
                                           OutT* __restrict__ c) {
+    if (wave < WAVES) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i) partial[wave][i][lane] = acc[i];
+        for (int i = 0; i < TM; ++i) partial[wave][i][lane] = acc[i];
+    }
     __syncthreads();
     for (int t = (int)threadIdx.x; t < TM * 64; t += WAVES * 64) {
         const int i = t >> 6, l = t & 63, m = i * 16 + (l & 15), n = n0 + 4 * (l >> 4);
@@ -122,9 +124,12 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_mxfp4_tn_rows_kernel(const ui
 // The same with the forward quantizer of x (Hadamard block 32, quest RTN) in front of the product, in every workgroup: the
 // decoded batch is so small that quantizing it 256 times over costs no more time than doing it once in a launch of its own,
 // and a layer call is one launch.  The codes lie in LDS as [K step][row][64 bytes], the scales as one byte per group; the
-// weight's first eight K steps are on their way meanwhile.  Bit-identical to the two launches.
+// weight's first eight K steps are on their way meanwhile.  Up to sixteen waves quantize, a group to a lane where that is enough
+// for all; WAVES of them multiply.  With WAVES alone, 8 x 4096 x 4096 took its 1024 groups four to a lane, one after the other, each
+// with its own wait for memory: 9.1 us, now 7.0.  Bit-identical to the two launches.
+constexpr int kDecodeThreads = 1024;
 template <int WAVES, typename T, typename OutT>
-__global__ __launch_bounds__(WAVES * 64) void linear_decode_kernel(const T* __restrict__ x, float rot_c, uint32_t sign_word,
+__global__ __launch_bounds__(kDecodeThreads) void linear_decode_kernel(const T* __restrict__ x, float rot_c, uint32_t sign_word,
                                                                     const uint8_t* __restrict__ b_codes, const uint8_t* __restrict__ b_scales, int M, int N,
                                                                     int I, int K, OutT* __restrict__ c) {
     __shared__ v4f partial[WAVES][1][64];
@@ -133,7 +138,8 @@ __global__ __launch_bounds__(WAVES * 64) void linear_decode_kernel(const T* __re
     const int row = lane & 15, block = lane >> 4, shift = 8 * block;
     const int nk = K / kBK, groups = K / 32, real_groups = I / 32;
     const int n0 = (int)blockIdx.x * 16;
-    const int first = wave * nk / WAVES, end = (wave + 1) * nk / WAVES;
+    const bool multiplies = wave < WAVES;
+    const int first = multiplies ? wave * nk / WAVES : 0, end = multiplies ? (wave + 1) * nk / WAVES : 0;
     uint8_t* const x_scales = reinterpret_cast<uint8_t*>(x_codes + M * groups);
 
     const int b_row = n0 + row < N ? n0 + row : N - 1;
@@ -156,7 +162,7 @@ __global__ __launch_bounds__(WAVES * 64) void linear_decode_kernel(const T* __re
         request(f0, first);
         request(f1, first + kRowsDepth);
     }
-    for (int i = (int)threadIdx.x; i < M * groups; i += WAVES * 64) {
+    for (int i = (int)threadIdx.x; i < M * groups; i += (int)blockDim.x) {
         const int r = i / groups, g = i - r * groups, at = ((g >> 2) * M + r) * 4 + (g & 3);
         GroupCodes o{};   // columns past the end: zero codes and scales
         if (g < real_groups) {
@@ -226,8 +232,8 @@ hipError_t gemm_rows(const TileProduct& p, int c_dtype, hipStream_t stream) {
 }
 
 // One launch instead of two while a CU's share of quantizing is no more than 1024 groups, four per lane (about 5 us, what the
-// quantizer's own launch takes): 8x4096x4096 9.0 us against 4.2 + 4.2 and 1x4096x11008 7.2 against 4.4 + 5.6, where a call's
-// host time, which is what bounds both, falls from 12.5 to 10.3 us
+// quantizer's own launch takes): 8x4096x4096 7.0 us against 4.2 + 4.2 and 1x4096x11008 7.2 against 4.4 + 5.6, where a call's
+// host time, which is what bounds both, falls from 12.5 to 10.3 us (and from 8.9 to 7.2 with fewer attribute look-ups)
 bool linear_decode_serves(int64_t T, int64_t I, int64_t O) {
     if (!(T > 0 && T <= 16 && I > 0 && I % 32 == 0 && I < (1 << 20) && O >= 8 && O % 8 == 0 && O < (1 << 24))) return false;
     const int64_t per_cu = ((O + 15) / 16 + device_cus() - 1) / device_cus();
@@ -243,7 +249,9 @@ hipError_t linear_decode(const void* x, int x_dtype, int64_t T, int64_t I, int64
     const dim3 grid((unsigned)((O + 15) / 16));
     const auto go = [&](auto waves, auto tx, auto ty) {   // as many waves as gemm_rows() takes: the same sums in the same order
         constexpr int W = decltype(waves)::value;
-        linear_decode_kernel<W, decltype(tx), decltype(ty)><<<grid, dim3(W * 64), lds, stream>>>(
+        const int64_t lanes = (T * (K / 32) + 63) / 64 * 64;
+        const unsigned threads = (unsigned)(lanes < W * 64 ? W * 64 : lanes < kDecodeThreads ? lanes : kDecodeThreads);
+        linear_decode_kernel<W, decltype(tx), decltype(ty)><<<grid, dim3(threads), lds, stream>>>(
             static_cast<const decltype(tx)*>(x), c, sign_word, w_codes, w_scales, (int)T, (int)O, (int)I, K, static_cast<decltype(ty)*>(y));
     };
     const auto typed = [&](auto waves) {
