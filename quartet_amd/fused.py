@@ -19,10 +19,13 @@ from .one_node import as_one_node
 _KERNEL_DTYPES = (torch.float32, torch.bfloat16)
 
 
-def _layer_is_fusable(layer, x):
-    return (isinstance(layer, QuantizedLinear) and layer._is_production_config(x.numel() // max(x.shape[-1], 1)) and layer.weight.is_cuda
-            and layer.activation_quantizer.hadamard_dim == 32 and not layer.activation_quantizer.is_dense
-            and layer.weight.dtype in _KERNEL_DTYPES)
+def _fusable_parts(layer, x):
+    """(weight, activation, weight and gradient quantizer) of a layer whose input a kernel here may produce, else None."""
+    parts = layer._production_parts(x) if isinstance(layer, QuantizedLinear) else None
+    if parts is None:
+        return None
+    weight, a_q = parts[:2]
+    return parts if weight.is_cuda and a_q.hadamard_dim == 32 and a_q._dense is None and weight.dtype in _KERNEL_DTYPES else None
 
 
 @as_one_node
@@ -69,14 +72,14 @@ def rmsnorm_linear(norm, layer, x, pass_input=False, add=None):
     `pass_input` returns (layer(norm(x)), x): use the second value for the residual sum around the norm, so that the sum
     of x's two gradients happens inside the RMSNorm backward kernel.  With `add` returns (layer(norm(x + add)), x + add):
     the residual sum in front of the norm is formed inside the quantizer kernel."""
-    fusable = (_layer_is_fusable(layer, x) and x.is_cuda and x.dtype in _KERNEL_DTYPES and norm.weight.dtype == torch.float32
-               and x.shape[-1] <= 8192)
+    gain, parts = norm.weight, _fusable_parts(layer, x)
+    fusable = parts is not None and x.is_cuda and x.dtype in _KERNEL_DTYPES and gain.dtype == torch.float32 and x.shape[-1] <= 8192
     if fusable and add is not None and not (x.dtype == torch.float32 and add.dtype in _KERNEL_DTYPES and add.shape == x.shape):
         x, add = x + add, None
         pass_input = True
     if fusable:
-        return _norm_linear(x, add, norm.weight, layer.weight, norm.eps, layer.activation_quantizer, layer.weight_quantizer,
-                            layer.backward_scheme.g_quantizer, layer.packed_weight_cache, pass_input)
+        weight, *quantizers = parts
+        return _norm_linear(x, add, gain, weight, norm.eps, *quantizers, layer.packed_weight_cache, pass_input)
     if add is not None:
         x = x + add
     y = layer(norm(x))
@@ -85,9 +88,9 @@ def rmsnorm_linear(norm, layer, x, pass_input=False, add=None):
 
 def swiglu_linear(layer, h12):
     """layer(silu(up) * gate) with (up, gate) the two halves of h12's last dimension."""
-    if _layer_is_fusable(layer, h12) and h12.is_cuda and h12.dtype in _KERNEL_DTYPES:
-        return _swiglu_linear(h12, layer.weight, layer.activation_quantizer, layer.weight_quantizer, layer.backward_scheme.g_quantizer,
-                              layer.packed_weight_cache)
+    parts = _fusable_parts(layer, h12)
+    if parts is not None and h12.is_cuda and h12.dtype in _KERNEL_DTYPES:
+        return _swiglu_linear(h12, *parts, layer.packed_weight_cache)
     up, gate = h12.split(h12.shape[-1] // 2, dim=-1)
     return layer(F.silu(up) * gate)
 
