@@ -113,8 +113,8 @@ def test_decode_in_one_launch_is_the_same_layer(T, I, O, one_launch):
 
 # groups between the multiplying waves' lanes and sixteen waves' (320, 432, 1020 of them), behind four and eight multiplying waves
 @pytest.mark.parametrize("T,I,O", [(5, 2048, 264), (9, 1536, 40), (15, 2176, 520), (2, 9216, 24)])
-def test_decode_with_quantizing_waves_beside_the_multiplying_ones(oracle, T, I, O):
-    test_decode_in_one_launch_is_the_same_layer(oracle, T, I, O, True)
+def test_decode_with_quantizing_waves_beside_the_multiplying_ones(T, I, O):
+    test_decode_in_one_launch_is_the_same_layer(T, I, O, True)
 
 
 @pytest.mark.parametrize("T,I,O,hd", [(32, 32, 32, 32), (4128, 96, 160, 32), (4160, 192, 128, 64), (4224, 128, 256, 128), (96, 160, 96, 32), (288, 192, 320, 32), (544, 1728, 352, 32), (1056, 640, 1088, 32),
