@@ -855,7 +855,7 @@ const KernelCost& tile_costs(bool e5m2, int kind, int64_t K, int splits) {
     return (e5m2 ? kWideTileCosts : kTileCosts)[kind];
 }
 int last_tile_kind(bool e5m2) { return e5m2 ? TILE_64x64 : TILE_64x32; }
-constexpr double kLaunch = 3.0, kPersistentStep = 0.675, kPersistentBoundary = 5.5, kPersistentRotate = 3.9;
+constexpr double kLaunch = 3.0, kPersistentStep = 0.675, kPersistentBoundary = 5.5, kPersistentMuted = 1.6, kPersistentRotate = 3.9;
 constexpr double kMemory = 5.5e6, kRotateMemory = 5.2e6;   // bytes per us of the reduction and of a rotation pass of its own
 
 double ranges_cost(int64_t M, int64_t N, int splits) {   // writing, reading and reducing the partial sums of a cut product
@@ -883,14 +883,16 @@ double separate_rotate_cost(int64_t M, int64_t N, int in_bytes, int out_bytes) {
 double persistent_cost(int64_t M, int64_t N, int64_t K, int splits, int cus) {
     const int64_t items = ((M + kBigM - 1) / kBigM) * ((N + kBigN - 1) / kBigN) * splits;
     const int64_t steps = (K / kBK / splits + 3) & ~(int64_t)3;
-    return kLaunch + (double)((items + cus - 1) / cus) * (steps * kPersistentStep + kPersistentBoundary) + ranges_cost(M, N, splits);
+    const double boundary = kPersistentBoundary + (K % 512 ? kPersistentMuted : 0.0);
+    return kLaunch + (double)((items + cus - 1) / cus) * (steps * kPersistentStep + boundary) + ranges_cost(M, N, splits);
 }
 
 // The persistent kernel: M any, N a multiple of 64, at least one tile; it walks K in blocks of four steps: K % 512 == 0
 // directly (scale rows are then 16-byte aligned like their base), other multiples of 128 with up to three muted steps in
-// the last block; their 16-byte scale requests start at 4-byte aligned addresses.  Muted steps cost what others do, and the
-// estimate counts them.  (Passing over the products of a muted step instead, by a branch, makes the
-// compiler keep a second set of accumulators, in memory.)
+// the last block; their 16-byte scale requests start at 4-byte aligned addresses.  Muted steps cost what others do, and their
+// tile 1.6 us more at its boundary, and the estimate counts them (16480 x 1728 x 640 with the rotation: 33 us, 28 on 128 x 128
+// tiles).  (Passing over the products of a muted step instead, by a branch, makes the compiler keep a second set of
+// accumulators, in memory.)
 bool persistent_serves(int64_t M, int64_t N, int64_t K, const void* a_scales, const void* b_scales, const void* c) {
     const int64_t steps = K / kBK;
     if (N % 64 || M < kBigM || N < kBigN || K % kBK || steps < 4 || M >= (1 << 30) || N >= (1 << 30) || K >= (1 << 26)) return false;
