@@ -642,9 +642,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     const int wave_u = wave;
     int load_tm, load_tn, load_split;  // work item the load stream is in
     auto plan_tile = [&](int item) {
-        const int t = item / splits;
-        load_split = item - t * splits;
-        tile_of_block(t, tiles_m, tiles_n, load_tm, load_tn);
+        const int r = xcd_run(item, total_items);
+        load_split = r / total;
+        tile_of_run(r - load_split * total, tiles_m, tiles_n, load_tm, load_tn);
         // N, and but for RAGGED M, is a multiple of 64: a wave's 64-row share of a panel is inside the matrix or outside it as a
         // whole; an outside share reads the matrix's last 64 rows instead (its products are dropped by the epilogue).
         // RAGGED: A's rows past the end read the last row (of the last block of 16 in a tiled operand).

@@ -57,15 +57,16 @@ __device__ __forceinline__ void store_tile(const v16f& t, float alpha, OutT* __r
     }
 }
 
-// Tile order: workgroup ids are dealt round-robin to the 8 XCDs by the hardware; give each XCD a
-// contiguous run of tiles in an order that walks groups of GM tile rows column by column, so the tiles that
-// share an L2 also share A and B panels.
-// GM: tile rows per group (about a thousand matrix rows).
+// Item order: workgroup ids are dealt round-robin to the 8 XCDs by the hardware; give each XCD a contiguous run of items, of any
+// number of them, K ranges of a product being runs of tiles one after the other.
+__device__ __forceinline__ int xcd_run(int id, int total) {
+    const int xcd = id & 7, rest = total & 7;
+    return xcd * (total >> 3) + (xcd < rest ? xcd : rest) + (id >> 3);
+}
+// Tile order: groups of GM tile rows (about a thousand matrix rows), column by column, so that the tiles of a run, which share an
+// L2, also share A and B panels.
 template <int GM = 4>
-__device__ __forceinline__ void tile_of_block(int bid, int tiles_m, int tiles_n, int& tm, int& tn) {
-    const int total = tiles_m * tiles_n;
-    int t = bid;
-    if ((total & 7) == 0) t = (bid & 7) * (total >> 3) + (bid >> 3);
+__device__ __forceinline__ void tile_of_run(int t, int tiles_m, int tiles_n, int& tm, int& tn) {
     const int per_group = GM * tiles_n;
     const int group = t / per_group;
     const int first_m = group * GM;

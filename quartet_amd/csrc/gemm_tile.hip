@@ -240,12 +240,12 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
     const int code_pitch = K / 2, groups = K / 32;
     // a work item is (tile, K range): range r covers steps [r * all / splits, (r + 1) * all / splits) and, with splits > 1 (fp32
     // instantiation only), stores its partial sums, unscaled, into slab r of c = [splits][M][N]
-    const int tiles = tiles_m * tiles_n, range = t / tiles;
+    const int tiles = tiles_m * tiles_n, item = xcd_run(t, tiles * g.splits), range = item / tiles;
     const int nk_all = (K + kBK - 1) / kBK;
     const int k_first = S::kMixed ? 0 : range * nk_all / g.splits, nk = (range + 1) * nk_all / g.splits - k_first;
     const int half_step = (K % kBK) && range == g.splits - 1 ? nk - 1 : -1;  // the K step that covers only 64 indices (K % 128 == 64), or none
     int tm, tn;
-    tile_of_block<(S::BM >= 256 ? 4 : 8)>(t - range * tiles, tiles_m, tiles_n, tm, tn);
+    tile_of_run<(S::BM >= 256 ? 4 : 8)>(item - range * tiles, tiles_m, tiles_n, tm, tn);
     const int m0 = tm * S::BM, n0 = tn * S::BN;
 
     const int swz = (lrow >> 2) & 3;
