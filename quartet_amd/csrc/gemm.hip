@@ -856,7 +856,7 @@ const KernelCost& tile_costs(bool e5m2, int kind, int64_t K, int splits) {
 }
 int last_tile_kind(bool e5m2) { return e5m2 ? TILE_64x64 : TILE_64x32; }
 constexpr double kLaunch = 3.0, kPersistentStep = 0.675, kPersistentBoundary = 5.5, kPersistentMuted = 1.6, kPersistentRotate = 3.9;
-constexpr double kMemory = 5.5e6, kRotateMemory = 5.2e6;   // bytes per us of the reduction and of a rotation pass of its own
+constexpr double kMemory = 5.5e6, kRotateMemory = 5.2e6, kWideStores = 1.0e7;   // bytes per us of the reduction, of a rotation pass of its own, of what fp32 results add
 
 double ranges_cost(int64_t M, int64_t N, int splits) {   // writing, reading and reducing the partial sums of a cut product
     return splits == 1 ? 0.0 : kLaunch + (4.0 * splits + 2.0) * (double)M * (double)N / kMemory;
@@ -875,7 +875,7 @@ double tile_rotate_cost(const KernelCost& k, int64_t M, int64_t N, int hd, int o
     const int64_t tiles = ((M + k.bm - 1) / k.bm) * ((N + k.bn - 1) / k.bn);
     const double rounds = (double)((tiles + cus - 1) / cus) / k.per_cu;
     const int h = hd == 32 ? 0 : hd == 64 ? 1 : 2;
-    return k.rotate[h] + (rounds > 1.0 ? (rounds - 1.0) * k.more[h] : 0.0) + (double)M * (double)N * (out_bytes - 2) / kRotateMemory;
+    return k.rotate[h] + (rounds > 1.0 ? (rounds - 1.0) * k.more[h] : 0.0) + (double)M * (double)N * (out_bytes - 2) / kWideStores;
 }
 double separate_rotate_cost(int64_t M, int64_t N, int in_bytes, int out_bytes) {
     return kLaunch + 0.5 + (double)M * (double)N * (in_bytes + out_bytes) / kRotateMemory;

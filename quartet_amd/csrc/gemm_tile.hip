@@ -621,10 +621,10 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
                     __builtin_nontemporal_store(u4v{v.x, v.y, v.z, v.w}, reinterpret_cast<u4v*>(out + (int64_t)r * S::kRowsPerPass * N));
             }
         } else {
-            // A loop per block size, not unrolled: a tile runs this code once or twice per launch, and what bounds it then is
+            // A loop per block size and type, not unrolled: a tile runs this code once or twice per launch, and what bounds it then is
             // fetching instructions.  Unrolled with the choice of the block size inside, 256 x 256 tiles took 8 us longer
             // (4096^3, 59.8 -> 51.8), 128 x 128 ones 2 to 3 (8192 x 2048 x 2048, 46.9 -> 43.2); unrolled twice is no faster.
-            const auto rotate_rows = [&](auto hd_tag) {
+            const auto rotate_rows = [&](auto hd_tag, auto f32_tag) {
                 constexpr int HD = decltype(hd_tag)::value;
                 if constexpr (S::BN >= HD) {
 #pragma unroll 1
@@ -645,22 +645,32 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
 #pragma unroll
                         for (int i = 0; i < 4; ++i)
                             o[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{v[2 * i] * g.rot_c, v[2 * i + 1] * g.rot_c}, v2bf));
-                        if (col_ok && row < M) {
-                            const int64_t at = (int64_t)row * N + out_col;
-                            if (!g.out_f32) {
-                                __builtin_nontemporal_store(u4v{o[0], o[1], o[2], o[3]}, reinterpret_cast<u4v*>(reinterpret_cast<uint16_t*>(g.c) + at));
-                            } else {   // the bf16-rounded result, widened
-                                f4v* dst = reinterpret_cast<f4v*>(reinterpret_cast<float*>(g.c) + at);
-                                __builtin_nontemporal_store(f4v{u2f(o[0] << 16), u2f(o[0] & 0xffff0000u), u2f(o[1] << 16), u2f(o[1] & 0xffff0000u)}, dst);
-                                __builtin_nontemporal_store(f4v{u2f(o[2] << 16), u2f(o[2] & 0xffff0000u), u2f(o[3] << 16), u2f(o[3] & 0xffff0000u)}, dst + 1);
+                        if constexpr (!decltype(f32_tag)::value) {
+                            if (col_ok && row < M)
+                                __builtin_nontemporal_store(u4v{o[0], o[1], o[2], o[3]}, reinterpret_cast<u4v*>(reinterpret_cast<uint16_t*>(g.c) + (int64_t)row * N + out_col));
+                        } else {
+                            // The bf16-rounded result, widened.  A lane's 32 bytes would be every other 16 bytes of two stores, so the
+                            // values go back to where they were and the wave stores its rows four values a lane, whole lines: a step
+                            // with 8192 x 6656 weights and 448 tokens takes 193 us, 255 with half lines as non-temporal stores, 207 as
+                            // others; 4096 x 11008 and 2048 tokens 293, 329 and 306.
+                            *reinterpret_cast<uint4*>(smem_bytes + line * S::kPitch + chunk * 16) = make_uint4(o[0], o[1], o[2], o[3]);
+                            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                            for (int h = 0; h < 2; ++h) {
+                                const int at = h * 256 + lane * 4, col = at % S::BN, wline = r * S::kRowsPerPass + wave * (64 / S::kChunks) + at / S::BN;
+                                const uint2 q = *reinterpret_cast<const uint2*>(smem_bytes + wline * S::kPitch + col * 2);
+                                if (n0 + col < N && m0 + wline < M)
+                                    __builtin_nontemporal_store(f4v{u2f(q.x << 16), u2f(q.x & 0xffff0000u), u2f(q.y << 16), u2f(q.y & 0xffff0000u)},
+                                                                reinterpret_cast<f4v*>(reinterpret_cast<float*>(g.c) + (int64_t)(m0 + wline) * N + n0 + col));
                             }
                         }
                     }
                 }
             };
-            if (g.hd == 32) rotate_rows(std::integral_constant<int, 32>{});
-            else if (g.hd == 64) rotate_rows(std::integral_constant<int, 64>{});
-            else rotate_rows(std::integral_constant<int, 128>{});
+            const auto rotate = [&](auto hd_tag) { g.out_f32 ? rotate_rows(hd_tag, std::true_type{}) : rotate_rows(hd_tag, std::false_type{}); };
+            if (g.hd == 32) rotate(std::integral_constant<int, 32>{});
+            else if (g.hd == 64) rotate(std::integral_constant<int, 64>{});
+            else rotate(std::integral_constant<int, 128>{});
         }
     } else {
         float* c = reinterpret_cast<float*>(g.c) + (int64_t)range * M * N;
