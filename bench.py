@@ -622,8 +622,7 @@ def counters_to_json(fetch_dir, write_dir, sq_dir=None):
               "gemm_mxfp4_tn_rotated": lambda k: product(k) is not None and product(k)[2] == "true",
               "quantize_x_quest_rtn_mask_alone": lambda k: jobs(k) == ["RowmajorTiledJob"],
               "forward_quantizer_pair": lambda k: jobs(k) == ["RowmajorTiledJob"] * 2,
-              "gradient_quantizer_pair": lambda k: jobs(k) == ["TransposedJob", "RowmajorTiledJob"],
-              "requantizer_pair": lambda k: jobs(k) == ["RequantJob"] * 2,
+              "backward_quantizers": lambda k: jobs(k) == ["TransposedJob", "RowmajorTiledJob"] + ["RequantTiledJob"] * 2,
               "inverse_rotation_pair": lambda k: jobs(k) == ["HadamardBwdJob"] * 2}
     out = {}
     for name, match in groups.items():
