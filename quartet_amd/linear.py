@@ -216,7 +216,8 @@ class QuantizedLinear(nn.Linear):
         plain = a_q._dense is None and w_q._dense is None and g_q._dense is None and g_q.rerotate != "O32"
         if not plain and not self._is_production_config(x.numel() // max(x.shape[-1], 1)):
             return None
-        weight = self._parameters.get("weight")
+        # a subclass (a parametrization makes one) or the instance itself may have a weight of its own in front of the parameter
+        weight = self._parameters.get("weight") if type(self) is QuantizedLinear and "weight" not in self.__dict__ else None
         return self.weight if weight is None else weight, a_q, w_q, g_q
 
     def _is_error_only_config(self, x):

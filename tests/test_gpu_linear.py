@@ -715,3 +715,33 @@ def test_error_only_scheme_calls_its_modules_where_somebody_listens(q, kind):
         assert float((a.float() - b.float()).norm() / b.float().norm()) < 1e-2
     if kind != "instance":
         assert layer._is_error_only_config(x)
+
+
+@pytest.mark.parametrize("where", ["parametrization", "property", "instance"])
+def test_layer_takes_the_weight_that_its_attribute_names(q, where):
+    """A weight in front of the parameter -- a parametrization's, a subclass's, the instance's own -- is the one that counts."""
+    print(f"case weight attribute {where}", flush=True)
+    torch.manual_seed(3)
+    make = lambda cls: cls(64, 96, bias=False, weight_quantizer=q.QuestMXFP4Quantizer(), activation_quantizer=q.QuestMXFP4Quantizer(),
+                           gradient_quantizer=q.AlbertTsengQuantizer(),
+                           backward_scheme=q.BACKWARD_SCHEMES["Q(E)Q(Wt)t_Q(Et)Q(Xt)t"]()).to("cuda:0", torch.bfloat16)
+    x = torch.randn(128, 64, device="cuda:0", dtype=torch.bfloat16)
+
+    class Negated(q.QuantizedLinear):
+        weight = property(lambda self: -self._parameters["weight"])
+    layer = make(q.QuantizedLinear)
+    with torch.no_grad():
+        want = layer(x)
+        if where == "property":
+            other = make(q.QuantizedLinear)
+            other.load_state_dict(layer.state_dict())
+            other.__class__ = Negated
+            layer = other
+        elif where == "instance":
+            layer.__dict__["weight"] = -layer.weight
+        else:
+            class Negate(torch.nn.Module):
+                def forward(self, w):
+                    return -w
+            torch.nn.utils.parametrize.register_parametrization(layer, "weight", Negate())
+        assert torch.equal(layer(x), -want)
