@@ -72,8 +72,10 @@ def rmsnorm_linear(norm, layer, x, pass_input=False, add=None):
     `pass_input` returns (layer(norm(x)), x): use the second value for the residual sum around the norm, so that the sum
     of x's two gradients happens inside the RMSNorm backward kernel.  With `add` returns (layer(norm(x + add)), x + add):
     the residual sum in front of the norm is formed inside the quantizer kernel."""
-    gain, parts = norm.weight, _fusable_parts(layer, x)
-    fusable = parts is not None and x.is_cuda and x.dtype in _KERNEL_DTYPES and gain.dtype == torch.float32 and x.shape[-1] <= 8192
+    parts = _fusable_parts(layer, x)
+    fusable = parts is not None and x.is_cuda and x.dtype in _KERNEL_DTYPES
+    gain = norm.weight if fusable else None   # in front of any other layer `norm` need not have one
+    fusable = fusable and gain.dtype == torch.float32 and x.shape[-1] <= 8192
     if fusable and add is not None and not (x.dtype == torch.float32 and add.dtype in _KERNEL_DTYPES and add.shape == x.shape):
         x, add = x + add, None
         pass_input = True

@@ -149,3 +149,20 @@ def test_sdpa_backend_choice_is_validated_and_inert_on_cpu():
     assert isinstance(_sdpa_choice("default", q), contextlib.nullcontext)
     with pytest.raises(ValueError):
         _sdpa_choice("flash", q)
+
+
+@pytest.mark.parametrize("kind", ["nn.Linear", "no quantizers", "production, on the CPU"])
+def test_rmsnorm_linear_takes_any_norm_in_front_of_an_unfused_layer(kind):
+    """Only a fused call needs the norm's gain: elsewhere `norm` is whatever can be called."""
+    from quartet_amd import quantizers as Q
+    from quartet_amd.backward import QEQWtt_QEtQXtt_Scheme
+    from quartet_amd.fused import rmsnorm_linear
+    layer = {"nn.Linear": lambda: nn.Linear(64, 32, bias=False), "no quantizers": lambda: QuantizedLinear(64, 32, bias=False),
+             "production, on the CPU": lambda: QuantizedLinear(64, 32, Q.QuestMXFP4Quantizer(), Q.QuestMXFP4Quantizer(),
+                                                               Q.AlbertTsengQuantizer(), QEQWtt_QEtQXtt_Scheme(), bias=False)}[kind]()
+    if kind.startswith("production"):
+        layer.forward = lambda t: torch.nn.functional.linear(t, layer.weight)   # the layer's own kernels need a GPU
+    x = torch.randn(8, 64)
+    assert torch.equal(rmsnorm_linear(nn.Identity(), layer, x), layer(x))
+    y, total = rmsnorm_linear(lambda t: 2 * t, layer, x, add=x)
+    assert torch.equal(total, x + x) and torch.equal(y, layer(2 * (x + x)))
