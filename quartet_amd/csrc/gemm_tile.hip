@@ -227,7 +227,10 @@ __device__ __forceinline__ void tile_mfma(const TileFrags<S>& f, const uint32_t 
     for (int i = 0; i < S::TM; ++i) tile_mfma_row<S, SUB, SWAP, ZERO, SIX>(i, f, sca, scb, acc);
 }
 
-template <class S, typename OutT>
+// ROT: the masked inverse rotation in the epilogue (bf16 results of the product).  A template argument: with both epilogues in one
+// kernel the plain product holds the rotation's lane constants too, 16 to 38 registers, and 128 x 128 and 256 x 128 tiles kept some
+// in memory: an inference call of 1000 x 1536 x 8192 15.0 us and an evaluated 30 M model's pass 993, 14.5 and 973 without.
+template <class S, typename OutT, bool ROT>
 __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* smem, uint32_t smem_base) {
     constexpr bool SWAP = sizeof(OutT) == 2;
     uint8_t* smem_bytes = reinterpret_cast<uint8_t*>(smem);
@@ -323,7 +326,7 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
                            (uint32_t)__builtin_amdgcn_readfirstlane((int)(smem_base + at + unit * 256)));
         }
     };
-    if (SWAP && S::kMaskEarly && g.mask) issue_mask(S::kMaskOff);
+    if constexpr (ROT && S::kMaskEarly) issue_mask(S::kMaskOff);
 
     const auto issue = [&](int stage, int ks) { tile_issue<S>(plan, stage, ks, ks == half_step); };
     // the scale dwords of a half step arrive two bytes early (see tile_issue).  Without a branch: a K step is one basic block.
@@ -591,7 +594,7 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
     __syncthreads();
     const float alpha = g.splits > 1 ? 1.0f : g.alpha;
-    if (SWAP && !S::kMaskEarly && g.mask) issue_mask(S::kMaskOff);
+    if constexpr (ROT && !S::kMaskEarly) issue_mask(S::kMaskOff);
     if constexpr (SWAP) {
 #pragma unroll
         for (int i = 0; i < S::TM; ++i)
@@ -605,14 +608,14 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
                     *reinterpret_cast<uint2*>(smem_bytes + (wm * S::WM + i * 32 + lrow) * S::kPitch + (wn * S::WN + j * 32 + 8 * b + 4 * half) * 2) =
                         make_uint2(__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1));
                 }
-        if constexpr (!S::kMaskEarly) __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+        if constexpr (ROT && !S::kMaskEarly) __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
         __syncthreads();
         const int chunk = tid % S::kChunks, rsub = tid / S::kChunks;
         const int out_col = n0 + chunk * 8;
         typedef uint32_t u4v __attribute__((ext_vector_type(4)));
         typedef float f4v __attribute__((ext_vector_type(4)));
         const bool col_ok = out_col < N;   // N is a multiple of 8
-        if (!g.mask) {
+        if constexpr (!ROT) {
             uint16_t* out = reinterpret_cast<uint16_t*>(g.c) + (int64_t)(m0 + rsub) * N + out_col;
 #pragma unroll
             for (int r = 0; r < S::kPasses; ++r) {
@@ -690,29 +693,29 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
     __syncthreads();  // the staging area is the next tile's ring
 }
 
-template <class S, typename OutT>
+template <class S, typename OutT, bool ROT>
 __device__ __forceinline__ void run_tiles(const TileProduct& g, int tiles) {   // persistent over the tiles
     extern __shared__ uint32_t smem[];
     const uint32_t smem_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint32_t*)smem;
-    for (int t = (int)blockIdx.x; t < tiles; t += (int)gridDim.x) tile_run<S, OutT>(g, t, smem, smem_base);
+    for (int t = (int)blockIdx.x; t < tiles; t += (int)gridDim.x) tile_run<S, OutT, ROT>(g, t, smem, smem_base);
 }
-template <class S, typename OutT>
+template <class S, typename OutT, bool ROT>
 __global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu((S::OCC * S::kWaves + 3) / 4))) void gemm_mxfp4_tn_tile_kernel(
     TileProduct g, int tiles) {
-    run_tiles<S, OutT>(g, tiles);
+    run_tiles<S, OutT, ROT>(g, tiles);
 }
 // the same with an eight-bit B
-template <class S, typename OutT>
+template <class S, typename OutT, bool ROT>
 __global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu((S::OCC * S::kWaves + 3) / 4))) void gemm_mxfp4_e5m2_tile_kernel(
     TileProduct g, int tiles) {
-    run_tiles<S, OutT>(g, tiles);
+    run_tiles<S, OutT, ROT>(g, tiles);
 }
 
-template <class S, typename OutT>
+template <class S, typename OutT, bool ROT = false>
 hipError_t launch_tiles(const TileProduct& g, hipStream_t stream) {
     const auto kern = [] {
-        if constexpr (S::kWideB) return gemm_mxfp4_e5m2_tile_kernel<S, OutT>;
-        else return gemm_mxfp4_tn_tile_kernel<S, OutT>;
+        if constexpr (S::kWideB) return gemm_mxfp4_e5m2_tile_kernel<S, OutT, ROT>;
+        else return gemm_mxfp4_tn_tile_kernel<S, OutT, ROT>;
     }();
     static std::atomic<bool> lds_allowed[kMaxDevices];
     hipError_t e = allow_dynamic_lds(kern, S::kSmemBytes, lds_allowed);
@@ -751,7 +754,8 @@ hipError_t gemm_tile(int shape, const TileProduct& g, int c_dtype, hipStream_t s
                         ((reinterpret_cast<uintptr_t>(g.a_scales) | reinterpret_cast<uintptr_t>(g.b_scales)) & 3) == 0;
     const auto run = [&](auto s) {
         using S = decltype(s);
-        return c_dtype == BF16 ? launch_tiles<S, uint16_t>(g, stream) : launch_tiles<S, float>(g, stream);
+        if (c_dtype != BF16) return launch_tiles<S, float>(g, stream);
+        return g.mask ? launch_tiles<S, uint16_t, true>(g, stream) : launch_tiles<S, uint16_t>(g, stream);
     };
     // 256 x 128 over fewer than eight steps: its two blocks of 384 rows are more in front of the first step than they save behind it
     // (4096 x 3456 x 640 in an evaluated model 14 us, 16 with blocks)

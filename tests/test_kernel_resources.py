@@ -1,0 +1,40 @@
+"""What the kernels of the built library were compiled to need, from the metadata of its code objects."""
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+
+from quartet_amd import _lib
+
+LLVM = "/opt/rocm/llvm/bin"
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    """{demangled name: (vector registers, bytes of scratch per lane)}"""
+    tools = [shutil.which(t, path=f"{LLVM}:{os.environ['PATH']}") for t in ("llvm-objdump", "llvm-readelf", "c++filt")]
+    if not os.path.exists(_lib.LIB_PATH) or not all(tools):
+        pytest.skip("needs the built library, ROCm's LLVM tools and c++filt")
+    where = tmp_path_factory.mktemp("objects")
+    lib = shutil.copy(_lib.LIB_PATH, where)
+    subprocess.run([tools[0], "--offloading", lib], cwd=where, check=True, capture_output=True)
+    found = {}
+    for f in sorted(os.listdir(where)):
+        if f.endswith("gfx950"):
+            notes = subprocess.run([tools[1], "--notes", os.path.join(where, f)], check=True, capture_output=True, text=True).stdout
+            for k in notes.split("  - .agpr_count:")[1:]:
+                get = lambda key: re.search(rf"^    \.{key}:\s+(\S+)", k, re.M).group(1)
+                found[get("name")] = (int(get("vgpr_count")), int(get("private_segment_fixed_size")))
+    names = subprocess.run([tools[2]], input="\n".join(found), check=True, capture_output=True, text=True).stdout.split("\n")
+    return dict(zip(names, found.values()))
+
+
+def test_products_without_a_rotation_keep_nothing_in_memory(kernels):
+    """A tile runs 5 to 30 K steps: what its prologue spills is not paid back.  The last template argument is the rotation."""
+    tiles = {n: v for n, v in kernels.items() if "tile_kernel<" in n}
+    plain = {n: v for n, v in tiles.items() if "true>(qm::TileProduct" not in n}
+    persistent = {n: v for n, v in kernels.items() if "gemm_mxfp4_tn_big4_kernel" in n}
+    assert plain and persistent
+    assert {n: v for n, v in {**plain, **persistent}.items() if v[1]} == {}
