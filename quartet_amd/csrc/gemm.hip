@@ -1031,13 +1031,8 @@ struct ShapePlan {
     size_t cut_bytes = 0;       // scratch of the cut, 0 if it would not be made
     size_t scratch_bytes = 0;   // what a caller is asked to provide: at least cut_bytes
 };
-// Few tiles and a long K: callers hold room for the ranges that would fill the CUs, whether or not a cut turns out cheaper than
-// the whole product (it mostly does from 64 K steps on).  Ranges of the persistent kernel; where that one has none, four ranges of
-// 128 x 128 tiles, if those are an eighth of the CUs at most.
-size_t scratch_of_few_small_tiles(int64_t M, int64_t N, int64_t K, int cus) {
-    const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
-    return tiles * 8 <= cus && K >= 16 * kBK ? (size_t)4 * (size_t)M * (size_t)N * sizeof(float) : 0;
-}
+// Few tiles of the persistent kernel and a long K: callers hold room for its ranges that would fill the CUs, whether or not a cut
+// turns out cheaper than the whole product (it mostly does from 64 K steps on).
 size_t scratch_of_few_tiles(int64_t M, int64_t N, int64_t K, int cus) {
     const int64_t tiles = ((M + kBigM - 1) / kBigM) * ((N + kBigN - 1) / kBigN), nblk = K / 512;
     if (K % 512 || tiles * 4 >= cus * 3 || nblk < 4) return 0;
@@ -1066,7 +1061,6 @@ ShapePlan make_plan(int64_t M, int64_t N, int64_t K, bool persistent, bool tiles
     p.cut = cheapest_cut(M, N, K, persistent, tiles_ok, e5m2, cus);
     p.cut_bytes = p.cut.cost < best ? (size_t)p.cut.choice.splits * (size_t)M * (size_t)N * sizeof(float) : 0;
     p.scratch_bytes = persistent ? scratch_of_few_tiles(M, N, K, cus) : 0;
-    if (tiles_ok && !e5m2 && !p.scratch_bytes) p.scratch_bytes = scratch_of_few_small_tiles(M, N, K, cus);
     if (p.cut_bytes > p.scratch_bytes) p.scratch_bytes = p.cut_bytes;
     return p;
 }
@@ -1076,7 +1070,8 @@ const ShapePlan& plan_of_shape(int64_t M, int64_t N, int64_t K, bool persistent,
     return table.find(M, N, K, flags, [&] { return make_plan(M, N, K, persistent, tiles_ok, e5m2, flags); });
 }
 
-// bytes of scratch with which gemm_mxfp4_tn may cut this shape into K ranges (0: it would not)
+// bytes of scratch with which gemm_mxfp4_tn makes every cut into K ranges that it would make of this shape (0: it would make none;
+// scratch_of_few_tiles asks for some that may go unused)
 size_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     const bool persistent = persistent_serves(M, N, K, nullptr, nullptr, nullptr), tiles_ok = gemm_tile_serves(M, N, K, 0, 0, nullptr);
     return persistent || tiles_ok ? plan_of_shape(M, N, K, persistent, tiles_ok).scratch_bytes : 0;

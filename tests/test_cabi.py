@@ -134,12 +134,18 @@ def test_allocation_free_product_refuses_few_tiles_only(shape):
     assert b"built-in scratch" in L.qm_last_error()
 
 
+@pytest.mark.parametrize("shape", [(256, 256, 2560), (320, 448, 3328), (256, 512, 2560), (128, 128, 2048), (448, 384, 2176)])
+def test_scratch_is_asked_for_by_products_that_may_be_cut(shape):
+    """16 to 26 K steps of a few small tiles run whole, so nothing is asked for."""
+    assert _lib.lib().qm_gemm_workspace_bytes(*shape) == 0
+
+
 def test_rotation_in_the_epilogue_is_offered_for_every_uncut_shape():
     """Served: the persistent kernel's shapes above K = 768, also where a cut on smaller tiles would be cheaper.  Not served: few
     tiles whose K ranges would fill the CUs, short contractions, ragged extents."""
     L = _lib.lib()
     for shape in [(256, 256, 2560), (256, 256, 1024), (256, 512, 1536), (320, 448, 1920), (2176, 8192, 28672), (8192, 4096, 4096)]:
         assert L.qm_gemm_fuses_rotation(None, None, *shape) == 1, shape
-    assert L.qm_gemm_workspace_bytes(256, 256, 2560) > 0      # as a plain product it may be cut
+    assert L.qm_gemm_workspace_bytes(256, 256, 6400) > 0 and L.qm_gemm_fuses_rotation(None, None, 256, 256, 6400) == 1   # cut as a plain product
     for shape in [(512, 768, 8192), (4096, 1536, 32768), (256, 256, 768), (250, 256, 1024), (256, 224, 1024), (256, 256, 1088)]:
         assert L.qm_gemm_fuses_rotation(None, None, *shape) == 0, shape

@@ -254,11 +254,11 @@ def test_product_with_the_inverse_rotation_in_its_epilogue(oracle, K, M, N, K_, 
         assert rel < 4e-3, rel     # the bf16 rounding of the result: 2^-9 relative per element
 
 
-@pytest.mark.parametrize("M,N,K_", [(256, 256, 2560), (320, 448, 3328)])
-def test_rotated_product_where_the_plain_one_may_be_cut(K, M, N, K_):
-    """The same rotation on shapes whose plain product takes a workspace when offered one: against the uncut product."""
+@pytest.mark.parametrize("M,N,K_,cut", [(256, 256, 2560, False), (320, 448, 3328, False), (256, 256, 6400, True), (320, 448, 7296, True)])
+def test_rotated_product_where_the_plain_one_may_be_cut(K, M, N, K_, cut):
+    """The same rotation on shapes whose plain product is (or nearly is) cut when offered a workspace: against the uncut product."""
     from quartet_amd import _lib
-    assert _lib.lib().qm_gemm_workspace_bytes(M, N, K_) > 0
+    assert (_lib.lib().qm_gemm_workspace_bytes(M, N, K_) > 0) == cut
     print(f"case rotated product of a cut shape {M}x{N}x{K_}", flush=True)
     dev = torch.device("cuda:0")
     g = torch.Generator(device="cpu").manual_seed(K_)
@@ -266,6 +266,9 @@ def test_rotated_product_where_the_plain_one_may_be_cut(K, M, N, K_):
     ac, bc, as_, bs, keep = byte(M, K_ // 2), byte(N, K_ // 2), byte(M, K_ // 32, 118, 132), byte(N, K_ // 32, 120, 136), byte(M, N // 8)
     got = K.gemm_mxfp4_tn_rotated(ac, as_, bc, bs, keep, 1.0, torch.float32, 5)
     plain = K.gemm_mxfp4_tn(ac, as_, bc, bs, 1.0, torch.bfloat16, split_k=False)
+    # sums in another order round differently in fp32: the product in ranges shows itself
+    in_fp32 = [K.gemm_mxfp4_tn(ac, as_, bc, bs, 1.0, torch.float32, split_k=s) for s in (True, False)]
+    assert torch.equal(*in_fp32) != cut
     two = K.masked_hadamard_bwd(plain, 32, torch.float32, 5, keep)
     assert float((got != two).float().mean()) < 1e-4      # as above: the order of a group's fp32 sum
     step = two.float().abs() * 2.0 ** -7 + float(plain.float().abs().max()) * 2.0 ** -18
