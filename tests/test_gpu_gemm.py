@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-from tests.util import make_input, to_oracle
+from tests.util import make_input, product_is_cut, to_oracle
 
 pytestmark = pytest.mark.gpu
 REL_FRO_TOL = 1e-3
@@ -95,7 +95,7 @@ def _torch_dequant(codes, scales):
                                     # K a multiple of 128 that the persistent kernel pads to whole blocks of four steps with
                                     # zero-scale steps: three, two and one real steps in the last block; one tile and many
                                     (512, 768, 1920), (4352, 4608, 3840), (320, 256, 3712), (768, 512, 2944), (4608, 4352, 1920),
-                                    # few output tiles, long K: cut into K ranges (split-K) when scratch is offered
+                                    # few output tiles, long K: cut into K ranges (split-K) when scratch is offered, but for the third
                                     (512, 256, 8192), (320, 640, 16384), (1920, 640, 4096),
                                     # K % 128 == 64 (row-major operands): a final half step on the 256x128 kernel; one tile,
                                     # tiles over the edge, one and a half K steps, the 30 M Llama's hidden width
@@ -258,7 +258,7 @@ def test_product_with_the_inverse_rotation_in_its_epilogue(oracle, K, M, N, K_, 
 def test_rotated_product_where_the_plain_one_may_be_cut(K, M, N, K_, cut):
     """The same rotation on shapes whose plain product is (or nearly is) cut when offered a workspace: against the uncut product."""
     from quartet_amd import _lib
-    assert (_lib.lib().qm_gemm_workspace_bytes(M, N, K_) > 0) == cut
+    assert (_lib.lib().qm_gemm_workspace_bytes(M, N, K_) > 0) == product_is_cut(M, N, K_) == cut
     print(f"case rotated product of a cut shape {M}x{N}x{K_}", flush=True)
     dev = torch.device("cuda:0")
     g = torch.Generator(device="cpu").manual_seed(K_)
@@ -266,9 +266,6 @@ def test_rotated_product_where_the_plain_one_may_be_cut(K, M, N, K_, cut):
     ac, bc, as_, bs, keep = byte(M, K_ // 2), byte(N, K_ // 2), byte(M, K_ // 32, 118, 132), byte(N, K_ // 32, 120, 136), byte(M, N // 8)
     got = K.gemm_mxfp4_tn_rotated(ac, as_, bc, bs, keep, 1.0, torch.float32, 5)
     plain = K.gemm_mxfp4_tn(ac, as_, bc, bs, 1.0, torch.bfloat16, split_k=False)
-    # sums in another order round differently in fp32: the product in ranges shows itself
-    in_fp32 = [K.gemm_mxfp4_tn(ac, as_, bc, bs, 1.0, torch.float32, split_k=s) for s in (True, False)]
-    assert torch.equal(*in_fp32) != cut
     two = K.masked_hadamard_bwd(plain, 32, torch.float32, 5, keep)
     assert float((got != two).float().mean()) < 1e-4      # as above: the order of a group's fp32 sum
     step = two.float().abs() * 2.0 ** -7 + float(plain.float().abs().max()) * 2.0 ** -18

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 import torch
 
-from tests.util import make_input, to_oracle
+from tests.util import make_input, product_is_cut, to_oracle
 
 pytestmark = pytest.mark.gpu
 
@@ -488,15 +488,15 @@ def test_weight_gradient_widened_in_the_kernel(q, T, I, O):
 
 @pytest.mark.parametrize("mid_dtype,gw_dtype", [(torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32),
                                                 (torch.float32, torch.float32)])
-def test_backward_with_products_cut_into_k_ranges(q, mid_dtype, gw_dtype):
-    """Few output tiles and a long contraction: both gradient products are cut into K ranges, and the ordered reduction of
-    the ranges applies the masked inverse rotation in the same pass.  Bit for bit what the kernels give one by one
-    (quantizers, re-quantizers, the products with their plain reduction, the inverse rotation as a kernel of its own)."""
-    print(f"case backward with split products mid={mid_dtype} gw={gw_dtype}", flush=True)
+@pytest.mark.parametrize("T,I,O,gx_cut,gw_cut", [(4096, 512, 2048, False, False), (8192, 256, 512, False, True), (9216, 512, 9216, True, True)])
+def test_backward_with_products_cut_into_k_ranges(q, mid_dtype, gw_dtype, T, I, O, gx_cut, gw_cut):
+    """Few output tiles and a long contraction: gradient products are cut into K ranges (of the tile kernels at I = 256, of the
+    persistent one at 9216), and the ordered reduction of the ranges applies the masked inverse rotation in the same pass.  Bit for bit
+    what the kernels give one by one (quantizers, re-quantizers, the products with their plain reduction, the inverse rotation as a
+    kernel of its own), also where scratch is offered and neither product is cut."""
+    print(f"case backward with split products {T}x{I}x{O} mid={mid_dtype} gw={gw_dtype}", flush=True)
     from quartet_amd import kernels as K
-    from quartet_amd import _lib
-    T, I, O = 4096, 512, 2048
-    assert _lib.lib().qm_gemm_workspace_bytes(T, I, O) > 0 and _lib.lib().qm_gemm_workspace_bytes(O, I, T) > 0
+    assert product_is_cut(T, I, O) == gx_cut and product_is_cut(O, I, T) == gw_cut
     dev = "cuda:0"
     x = make_input(T, I, mid_dtype, seed=21).to(dev)
     w = make_input(O, I, mid_dtype, seed=22, scale=0.02).to(dev)

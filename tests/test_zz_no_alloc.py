@@ -4,6 +4,8 @@ arguments are rejected."""
 import pytest
 import torch
 
+from tests.util import product_is_cut
+
 pytestmark = pytest.mark.gpu
 
 
@@ -20,11 +22,12 @@ def test_noalloc_product_matches_the_allocating_entry_point(out_dtype):
     dev = torch.device("cuda:0")
     L = _lib.lib()
     # both shapes are cut into K ranges (few tiles, long K), the second needs less scratch than the first
-    shapes = [(512, 768, 8192), (256, 512, 4096)]
+    shapes = [(512, 512, 16384), (256, 256, 8192)]
     assert L.qm_gemm_workspace_bytes(*shapes[0]) > L.qm_gemm_workspace_bytes(*shapes[1]) > 0
     for call, (M, N, Kd) in enumerate(shapes):
         print(f"case noalloc gemm call={call} shape={M}x{N}x{Kd} {out_dtype}", flush=True)
         ac, as_, bc, bs = _operands(M, N, Kd, 100 + call, dev)
+        assert product_is_cut(M, N, Kd)
         want = K.gemm_mxfp4_tn(ac, as_, bc, bs, 16.0 / 9.0, out_dtype)     # allocates its split-K workspace
         out = torch.full((M, N), float("nan"), dtype=out_dtype, device=dev)
         K.gemm_noalloc_prepare()      # the one step that may load the library's device image; a no-op from then on
@@ -47,10 +50,10 @@ def test_noalloc_product_matches_the_allocating_entry_point(out_dtype):
 def test_noalloc_product_under_graph_capture():
     """A split-K product captured into a HIP graph through the allocation-free entry point: every replay, with eager work
     and synchronisations in between, gives the bits of the eager allocating call on the operands then in place."""
-    from quartet_amd import _lib, kernels as K
+    from quartet_amd import kernels as K
     dev = torch.device("cuda:0")
-    M, N, Kd = 512, 768, 8192
-    assert _lib.lib().qm_gemm_workspace_bytes(M, N, Kd) > 0
+    M, N, Kd = 512, 256, 8192
+    assert product_is_cut(M, N, Kd)
     ac, as_, bc, bs = _operands(M, N, Kd, 300, dev)
     out = torch.zeros((M, N), dtype=torch.bfloat16, device=dev)
     K.gemm_noalloc_prepare()
@@ -75,7 +78,7 @@ def test_noalloc_product_under_graph_capture():
 def test_noalloc_product_runs_whole_where_its_cut_does_not_fit():
     from quartet_amd import _lib, kernels as K
     L = _lib.lib()
-    M, N, Kd = 2176, 8192, 28672           # cut into two ranges of 68 MiB each where a workspace is offered
+    M, N, Kd = 2176, 8192, 28672           # cut into four ranges of 68 MiB each where a workspace is offered
     assert L.qm_gemm_workspace_bytes(M, N, Kd) > L.qm_gemm_noalloc_scratch_bytes()
     print(f"case noalloc gemm whole shape={M}x{N}x{Kd}", flush=True)
     ops = _operands(M, N, Kd, 400, torch.device("cuda:0"))

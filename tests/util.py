@@ -34,3 +34,14 @@ def make_input(rows, cols, dtype, seed, outlier_frac=1e-3, scale=1.0, zero_rows=
     if zero_rows:
         x[:zero_rows] = 0
     return x.to(dtype)
+
+
+def product_is_cut(M, N, K):
+    """Whether the library cuts the FP4 product into K ranges where it is offered scratch: over scales that spread, sums in another
+    order than the whole product's round differently in fp32."""
+    from quartet_amd import kernels
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    part = lambda rows, cols, lo, hi: torch.randint(lo, hi, (rows, cols), generator=g, dtype=torch.uint8, device="cuda")
+    operands = (part(M, K // 2, 0, 256), part(M, K // 32, 112, 136), part(N, K // 2, 0, 256), part(N, K // 32, 112, 136))
+    ranges, whole = (kernels.gemm_mxfp4_tn(*operands, 1.0, torch.float32, split_k=s) for s in (True, False))
+    return not torch.equal(ranges, whole)
