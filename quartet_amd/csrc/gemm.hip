@@ -15,8 +15,8 @@
 // instruction needs.
 //
 // Kernels, picked by choose_product() at the end of the file:
-//   gemm_mxfp4_tn_big4_kernel  any M >= 256, N a multiple of 64 and >= 256, K a multiple of 128 whose last block of four K steps
-//                              repeats (muted) up to three steps.
+//   gemm_mxfp4_tn_big4_kernel  any M >= 256, N a multiple of 64 and >= 256, K a multiple of 128 but not 640, whose last block of four
+//                              K steps repeats (muted) up to three steps.
 //                              Persistent, 256x256 macro tile, 4 waves x 128x128, operands global -> LDS directly into a
 //                              4-stage ring, scales in blocks of four K steps, row-major or tiled code bytes, optional split-K.
 //   gemm_tile.hip              tiles from 256x128 down to 64x32 for everything too small or too short for that one.
@@ -889,13 +889,14 @@ double persistent_cost(int64_t M, int64_t N, int64_t K, int splits, int cus) {
 
 // The persistent kernel: M any, N a multiple of 64, at least one tile; it walks K in blocks of four steps: K % 512 == 0
 // directly (scale rows are then 16-byte aligned like their base), other multiples of 128 with up to three muted steps in
-// the last block; their 16-byte scale requests start at 4-byte aligned addresses.  Muted steps cost what others do, and their
+// the last block; their 16-byte scale requests start at 4-byte aligned addresses.  Not five steps: with three of eight muted the
+// tile kernels are cheaper for every M and N, with the rotation and without.  Muted steps cost what others do, and their
 // tile 1.6 us more at its boundary, and the estimate counts them (16480 x 1728 x 640 with the rotation: 33 us, 28 on 128 x 128
 // tiles).  (Passing over the products of a muted step instead, by a branch, makes the compiler keep a second set of
 // accumulators, in memory.)
 bool persistent_serves(int64_t M, int64_t N, int64_t K, const void* a_scales, const void* b_scales, const void* c) {
     const int64_t steps = K / kBK;
-    if (N % 64 || M < kBigM || N < kBigN || K % kBK || steps < 4 || M >= (1 << 30) || N >= (1 << 30) || K >= (1 << 26)) return false;
+    if (N % 64 || M < kBigM || N < kBigN || K % kBK || steps < 4 || steps == 5 || M >= (1 << 30) || N >= (1 << 30) || K >= (1 << 26)) return false;
     if (K % 512 == 0 && ((reinterpret_cast<uintptr_t>(a_scales) | reinterpret_cast<uintptr_t>(b_scales)) & 15)) return false;
     return (reinterpret_cast<uintptr_t>(c) & 15) == 0;
 }
