@@ -19,7 +19,7 @@ constexpr int kZeroGroup = 100;          // the scale byte of an all-zero group 
 // One workgroup per block of 512 rows and 256 columns: are the scales of 32 rows of a column group too far apart somewhere?
 struct SpanJob {
     static constexpr int kLds = 16 * (32 * 8 + 8);
-    static constexpr int kWaves = 8;
+    static constexpr int kWaves = 1;
     E5m2Args a;
     unsigned grid_r, blocks;
     explicit SpanJob(const E5m2Args& args)

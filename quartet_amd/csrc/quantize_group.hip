@@ -651,17 +651,21 @@ struct RequantJob {
 // Exact: the sums are multiples of half the smallest scale, and while the block's scales span at most ten octaves the instruction
 // adds them without a rounding (2 M random sums of K = 32 and 64 compared with exact ones: none differs up to 10, half of them
 // at 12), so that any order of additions, the butterfly's among them, gives the same fp32 values.  A block with more spread
-// (or scales near the ends of the range) takes rotate_block, its groups in neighbouring lanes, and stores its codes by itself.
+// (or scales near the ends of the range) takes rotate_block, its groups in neighbouring lanes, and stores its codes by itself: a row of
+// zeros (scale 2^-27) sends its 32 rows there.  With 5 % of the tokens zero a step of 16480 x 1728 x 640 takes 135 us for 129, of
+// 8192 x 4096 x 4096 296 for 293; the kernel above made them 157 and 301 with and without zeros.
 // What bounds it: vector instructions (385 a group, 0.7 us per wave and group of 32 at 2.4 GHz, half of that Philox and the
-// stochastic converts), with six waves on a SIMD to cover the requests; a row group's codes are waited for when they are needed.
-// Both operands of a layer, 8192 x 4096 and 11008 x 4096: 46 us; 16384 x 4096 and 1536 x 4096: 43; 16480 x 1728 and 640 x 1728: 22.
-// The kernel above (544 instructions a group, 64 narrow loads per lane, three waves on a SIMD) took 56, 53 and 26.
+// stochastic converts); a row group's codes are waited for when they are needed.  It runs in one grid with the quantizers of the
+// error signal, compiled to 128 registers (four waves on a SIMD), 132 with padded extents and 140 and 160 with blocks of 64 and 128
+// (three).  Both operands of a layer in a grid of their own, which fit six waves, 8192 x 4096 and 11008 x 4096: 46 us; 16384 x 4096 and
+// 1536 x 4096: 43; 16480 x 1728 and 640 x 1728: 22.  The kernel above (544 instructions a group, 64 narrow loads per lane, three waves on a
+// SIMD) took 56, 53 and 26.  The four jobs of 8192 x 4096 x 4096 in one grid take 68 us, in two 71.
 template <int MODE, int HD, bool PADDED>
 struct RequantTiledJob {
     static constexpr int kRegion = 128 * 32;                                     // a wave's codes, in and out
     static constexpr int kScalesIn = 4 * kRegion, kScalesOut = kScalesIn + 4 * 256;
     static constexpr int kLds = kScalesOut + kRqC * 16;
-    static constexpr int kWaves = HD == 32 ? 6 : 4;
+    static constexpr int kWaves = 1;
     static constexpr int P = HD / 32;                                            // groups of a Hadamard block
     const uint8_t* codes_in;
     const uint8_t* scales_in;
