@@ -65,7 +65,8 @@ __device__ __forceinline__ float below_ties_any(float v) {
 
 // n: the NEGATED rotated group.  The sign rule "negative unless g > 0" makes both zeros negative; on the negated values it reads
 // "positive unless n < 0", and the arithmetic in front of the converts turns zeros of either sign into +0 by itself (x y + z
-// with two exact zeros of opposite sign), so it costs one XOR of the sign bits of eight codes.  Everything else is symmetric.
+// with two exact zeros of opposite sign), so it costs one XOR of the sign bits of eight codes.  Everything else is symmetric but for
+// NaNs, which keep their sign where numbers are negated: their codes are the largest magnitude (the converts') of either sign.
 
 // clip mask, most significant element first so that element 0 lands in bit 0: the sign of |t| - 6 scale (never set for a NaN;
 // |t| = 6 scale gives +0), shifted in by a funnel shift.  The subtraction issues at twice the rate of a compare and nothing

@@ -411,3 +411,41 @@ def test_dense_rotation_with_the_hadamard_matrix_is_close_to_the_butterfly(oracl
     b = K.quantize_mxfp4_dense(x.to(dev), Hd.to(dev), K.QM_QUEST_RTN, want_mask=True)
     assert torch.equal(a[1], b[1])
     assert float((a[0] != b[0]).float().mean()) < 0.01
+
+
+@pytest.mark.parametrize("hd,transposed", [(1, False)] + [(hd, t) for hd in (32, 64, 128) for t in (False, True)])   # 1: rotated already
+@pytest.mark.parametrize("mode", list(MODES))
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_groups_that_are_not_finite(oracle, K, dtype, mode, hd, transposed):
+    """One value per Hadamard block that is infinite, not a number or so large that its square is not finite.  Quest groups with
+    infinities and overflowing statistics and absmax groups of large values follow the definition bit for bit.  A NaN becomes the
+    largest magnitude, of either sign (from the hardware's converts), or a negative zero (the definition's, where codes are compared
+    out), and is clipped; its group's scale is the definition's.  (What an absmax group with an infinity or
+    a NaN holds is not defined.)  No group touches another."""
+    print(f"case not finite mode={mode} hd={hd} dtype={dtype} transposed={transposed}", flush=True)
+    rows, cols, quest = 48, 512, mode.startswith("quest")
+    values = [float("inf"), -float("inf"), 1e19, -1e30, 3e38, float("nan"), -float("nan")]
+    x = make_input(rows, cols, dtype, seed=hd + MODES[mode], outlier_frac=0)
+    for r in range(2, rows):
+        for block in range(0, cols, 128):
+            x[r, block + (5 * r + block // 128) % 128] = values[r % 7]
+    given = x.t().contiguous() if transposed else x
+    codes, scales, mask, _ = K.quantize_mxfp4(given.to("cuda:0"), hd, None, MODES[mode], transposed, None, 99, want_mask=quest and not transposed)
+    torch.cuda.synchronize()
+    ref = oracle.quantize(to_oracle(given), hd, mode=MODES[mode], transposed_in=transposed, seed=99, want_mask=True)
+    nibbles = lambda c: np.stack([c & 15, c >> 4], -1).reshape(rows, cols // 32, 32)
+    got, want = nibbles(codes.cpu().numpy()), nibbles(ref["codes"])
+    got_scales = scales.cpu().numpy()
+    # the value that a group sees: its block's, wherever that lies
+    width = max(hd, 32)
+    blocks = x.float().view(rows, cols // width, width)
+    spread = lambda flag: flag.any(-1).repeat_interleave(width // 32, 1).numpy()
+    infinite, nan = spread(blocks.isinf()), spread(blocks.isnan())
+    defined = ~nan & (quest or ~infinite)
+    assert defined.any() and nan.any() and np.array_equal(got_scales[defined], ref["scales"][defined]) and np.array_equal(got[defined], want[defined])
+    if mask is not None:
+        assert np.array_equal(mask.cpu().numpy(), ref["mask"])
+    if quest:
+        elements = x.float().view(rows, cols // 32, 32).isnan().numpy() if hd == 1 else np.repeat(nan[..., None], 32, -1)
+        assert np.array_equal(got_scales[nan], ref["scales"][nan]) and bool(((got[elements] & 7 == 7) | (got[elements] == 8)).all())
+        assert np.array_equal(got[~elements], want[~elements])
