@@ -227,9 +227,9 @@ __device__ __forceinline__ void tile_mfma(const TileFrags<S>& f, const uint32_t 
     for (int i = 0; i < S::TM; ++i) tile_mfma_row<S, SUB, SWAP, ZERO, SIX>(i, f, sca, scb, acc);
 }
 
-// ROT: the masked inverse rotation in the epilogue (bf16 results of the product).  A template argument: with both epilogues in one
-// kernel the plain product holds the rotation's lane constants too, 16 to 38 registers, and 128 x 128 and 256 x 128 tiles kept some
-// in memory: an inference call of 1000 x 1536 x 8192 15.0 us and an evaluated 30 M model's pass 993, 14.5 and 973 without.
+// ROT: the masked inverse rotation in the epilogue (bf16 results of the product).  A template argument: a plain product that carries
+// the rotation's code behind a branch is slower with the same registers (an inference call of 1000 x 1536 x 8192 15.8 us, 15.5
+// without; an evaluated 30 M model's pass 1000 and 992).
 template <class S, typename OutT, bool ROT>
 __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* smem, uint32_t smem_base) {
     constexpr bool SWAP = sizeof(OutT) == 2;
@@ -610,7 +610,11 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
                 }
         if constexpr (ROT && !S::kMaskEarly) __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
         __syncthreads();
-        const int chunk = tid % S::kChunks, rsub = tid / S::kChunks;
+        // an opaque copy: what is worked out from it (the rotation's signs, addresses) otherwise holds 16 to 38 registers from ahead of
+        // the loop over tiles on, through every K step, and up to 200 bytes a lane of scratch (an error-only step of 4096^3 187 us, now 183)
+        int id = tid;
+        if constexpr (ROT) asm volatile("" : "+v"(id));
+        const int chunk = id % S::kChunks, rsub = id / S::kChunks;
         const int out_col = n0 + chunk * 8;
         typedef uint32_t u4v __attribute__((ext_vector_type(4)));
         typedef float f4v __attribute__((ext_vector_type(4)));
@@ -660,7 +664,7 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
                             __builtin_amdgcn_wave_barrier();
 #pragma unroll
                             for (int h = 0; h < 2; ++h) {
-                                const int at = h * 256 + lane * 4, col = at % S::BN, wline = r * S::kRowsPerPass + wave * (64 / S::kChunks) + at / S::BN;
+                                const int at = h * 256 + (id & 63) * 4, col = at % S::BN, wline = r * S::kRowsPerPass + wave * (64 / S::kChunks) + at / S::BN;
                                 const uint2 q = *reinterpret_cast<const uint2*>(smem_bytes + wline * S::kPitch + col * 2);
                                 if (n0 + col < N && m0 + wline < M)
                                     __builtin_nontemporal_store(f4v{u2f(q.x << 16), u2f(q.x & 0xffff0000u), u2f(q.y << 16), u2f(q.y & 0xffff0000u)},
