@@ -4,7 +4,7 @@
 // widened: within a block of 32 rows and 32 columns every value is a code times a power of two, which six bits (E3M2: two
 // mantissa bits where E2M1 has one) hold exactly as long as the row scales of the block lie within 5 octaves of the largest, and
 // eight bits (E5M2) within 28.  The matrix instruction takes six bits at the rate of four, eight at half of it, and the bytes
-// count too: the product of 4096^3 runs 58 us with six and 76 with eight.  The format is chosen per block of 512 rows (four K
+// count too: the product of 4096^3 with its rotation runs 50 us with six and 63 with eight.  The format is chosen per block of 512 rows (four K
 // steps) and 256 columns, by its scales alone (expand_formats.h); rows of zeros count for no range.  Rows of activations with
 // outliers of three degrees of freedom stay within 5 octaves but for a block in a hundred or less.
 //
@@ -14,8 +14,9 @@
 // x 128 that holds a value outside the range says so in `lost`, and the columns it touches are computed once more from the packed
 // tensors (ExactJob): results never depend on the spread of the scales.
 //
-// Bound by memory: half a byte read and three quarters (or one) written per element; 14.6 us for 4096 x 4096 twice (12.9 in eight
-// bits only: packing six bits and the look at the format cost more than the bytes saved).  A thread takes four consecutive rows and 16 columns;
+// Bound by memory: half a byte read and three quarters (or one) written per element; 14.3 us for 4096 x 4096 twice in either format
+// (12.9 where only eight bits exist: packing six bits and the look at the format cost more than the bytes saved).  A thread takes
+// four consecutive rows and 16 columns;
 // v_perm_b32 looks four codes at a time up in an eight-byte table of the row's E5M2 magnitudes, eight more turn 4 x 4 bytes
 // round, and the transposed dwords meet in LDS.
 #include <hip/hip_runtime.h>

@@ -17,8 +17,9 @@
 //
 // The same kernel multiplies FP4 with a B of six (E3M2) or eight (E5M2) bits, which is how the error-only scheme contracts over
 // the rows of a packed operand (expand.hip): 1.5 times the bytes of B at FP4's matrix rate, or twice the bytes at half of it.  4096^3
-// among the other kernels of a training step, 8 waves of 128 x 64 on 256 x 256: 58 us in six bits, 74 in eight, where the FP4 x
-// bf16 kernel (gemm_fp4_bf16.hip) takes 113 us and more.  4 waves of 128 x 128 read a third fewer bytes from LDS and take 67.
+// among the other kernels of a training step, 8 waves of 128 x 64 on 256 x 256, rotation included: 50 us in six bits, 63 in eight,
+// where the FP4 x bf16 kernel (gemm_fp4_bf16.hip) takes 113 us and more.  4 waves of 128 x 128 read a third fewer bytes from LDS and
+// took 67 where these took 58 (with the rotation as it was then, see rotate_rows).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -419,7 +420,7 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
             int next = block;
             // one K step, as below; the requests of a block's last steps are the first ones of the block that follows it here.
             // Requests, reads and products dealt out by 32 rows, where they otherwise stand between the barrier and the first
-            // product: 59.2 -> 58.3 us at 4096^3.
+            // product: 59.2 -> 58.3 us at 4096^3 (with the rotation as it was then, see rotate_rows).
             auto step = [&](auto q_tag) {
                 constexpr int Q = decltype(q_tag)::value;
                 const int nstage = stage == S::STAGES - 1 ? 0 : stage + 1;

@@ -652,8 +652,9 @@ struct RequantJob {
 // adds them without a rounding (2 M random sums of K = 32 and 64 compared with exact ones: none differs up to 10, half of them
 // at 12), so that any order of additions, the butterfly's among them, gives the same fp32 values.  A block with more spread
 // (or scales near the ends of the range) takes rotate_block, its groups in neighbouring lanes, and stores its codes by itself: a row of
-// zeros (scale 2^-27) sends its 32 rows there.  With 5 % of the tokens zero a step of 16480 x 1728 x 640 takes 135 us for 129, of
-// 8192 x 4096 x 4096 296 for 293; the kernel above made them 157 and 301 with and without zeros.
+// zeros (scale 2^-27) among others sends its Hadamard block of rows there.  Steps with 5 % of the tokens zero, in us (none zero; on the
+// kernel above, either way): 16480 x 1728 x 640 131 (124; 152), 8192 x 4096 x 4096 294 (289; 298), with blocks of 64 333 (327; 338), of
+// 128 337 (330; 345), 16512 x 1792 x 640 with blocks of 128 140 (133; 171).  Zero rows together, as padding behind the tokens, cost nothing.
 // What bounds it: vector instructions (385 a group, 0.7 us per wave and group of 32 at 2.4 GHz, half of that Philox and the
 // stochastic converts); a row group's codes are waited for when they are needed.  It runs in one grid with the quantizers of the
 // error signal, compiled to 128 registers (four waves on a SIMD), 132 with padded extents and 140 and 160 with blocks of 64 and 128
