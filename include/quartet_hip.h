@@ -278,11 +278,15 @@ int qm_dequantize_mxfp4(const uint8_t* codes, const uint8_t* scales, int64_t R, 
  * mid_dtype; see qm_gemm_mxfp4_tn_rotated), in the epilogue of the smaller tile kernels (bf16 mid_dtype, any Hadamard block,
  * any gw_dtype), or in the ordered reduction of a product cut into K ranges (any Hadamard block, mid_dtype and gw_dtype);
  * the last two with the arithmetic and roundings of the separate launches.  Elsewhere it is a launch of its own.
+ * Where both gradient products (bf16 mid_dtype, padded or tiled layout, Hadamard blocks 32) run fastest in one launch of the 256 x 256
+ * kernel, they do: with its epilogue for gx and for gw, of either gw_dtype, and without K ranges.
+ * qm_linear_backward_in_one_launch tells (1 / 0).
  */
 size_t qm_packed_operand_bytes(int64_t rows, int64_t cols);
 /* offsets: HOST array of three (codes, scales, mask bits); returns 0, or QM_ERR_INVALID unless cols % 32 == 0 */
 int qm_packed_operand_offsets(int64_t rows, int64_t cols, size_t* offsets);
 size_t qm_linear_backward_workspace_bytes(int64_t T, int64_t I, int64_t O, int mid_dtype);
+int qm_linear_backward_in_one_launch(int64_t T, int64_t I, int64_t O, int hd_x, int hd_w, int gw_dtype, int rotated_flags);
 int qm_linear_forward(const void* x, int x_dtype, const void* w, int w_dtype, int64_t T, int64_t I, int64_t O,
                       int hd_x, const uint32_t* signs_x, int hd_w, const uint32_t* signs_w, void* packed_x,
                       size_t packed_x_bytes, void* packed_w, size_t packed_w_bytes, int packed_flags, void* y,

@@ -413,6 +413,42 @@ bool seed_base_served(int codes_layout, int64_t T, int64_t I, int64_t O, int hd_
     return tiled_layout(codes_layout) && hd_a == 32 && hd_b == 32 && hd_c == 32 && T % 128 == 0 && I % 128 == 0 &&
            O % 128 == 0;
 }
+extern "C++" {
+// A gradient product of the backward pass and the kernel that serves it by itself: with the masked inverse rotation of the forward
+// quantizer (into final_dst) where that kernel applies it, otherwise without (into plain.c)
+struct GradProduct {
+    qm::TileProduct p;
+    qm::ProductChoice choice;
+    int out_dtype;
+    // what a launch of both products would do: this one with the rotation wherever it is wanted
+    qm::TileProduct whole;
+    qm::ProductChoice whole_choice;   // its estimate counts a rotation pass of its own
+    int whole_dtype;                  // -1: not to be had
+};
+GradProduct plan_gradient(const qm::TileProduct& plain, void* final_dst, bool want_rotation, int hd, int mid_dtype, int final_dtype, const uint8_t* mask,
+                          const uint32_t* signs, int scale_dtype, void* ws, size_t ws_bytes) {
+    GradProduct g{plain, {}, mid_dtype, plain, {}, want_rotation ? -1 : mid_dtype};
+    if (want_rotation && final_dst && aligned(final_dst, 16) && valid_dtype(scale_dtype) && valid_hd(hd) && plain.N % hd == 0) {
+        qm::TileProduct r = plain;
+        r.c = final_dst;
+        r.mask = mask;
+        r.hd = hd;
+        r.signs = make_signs(signs, hd);
+        r.rot_c = qm::hadamard_scale(hd, scale_dtype);
+        const qm::ProductChoice c = qm::choose_product(r, mid_dtype, final_dtype, ws, ws_bytes);
+        if (c.rotates) return GradProduct{r, c, final_dtype, r, c, final_dtype};
+        g.whole = r;
+        g.whole_choice = c;
+        g.whole_dtype = final_dtype;
+    }
+    g.choice = qm::choose_product(plain, mid_dtype, mid_dtype, ws, ws_bytes);
+    if (!want_rotation) g.whole_choice = g.choice;
+    return g;
+}
+bool one_launch(const GradProduct& x, const GradProduct& w, int mid_dtype) {
+    return x.whole_dtype >= 0 && w.whole_dtype >= 0 && qm::pair_pays(x.whole, x.whole_choice, x.whole_dtype, w.whole, w.whole_choice, w.whole_dtype, mid_dtype);
+}
+}
 }  // namespace
 
 size_t qm_packed_operand_bytes(int64_t rows, int64_t cols) {
@@ -432,6 +468,19 @@ int qm_packed_operand_offsets(int64_t rows, int64_t cols, size_t* offsets) {
 size_t qm_linear_backward_workspace_bytes(int64_t T, int64_t I, int64_t O, int mid_dtype) {
     if (T < 0 || I < 0 || O < 0 || I % 32 || O % 32 || T % 32 || !valid_dtype(mid_dtype)) return 0;
     return work_layout(T, I, O, mid_dtype).total;
+}
+
+int qm_linear_backward_in_one_launch(int64_t T, int64_t I, int64_t O, int hd_x, int hd_w, int gw_dtype, int rotated_flags) {
+    if (T <= 0 || I <= 0 || O <= 0 || I % 32 || O % 32 || T % 32 || !valid_hd(hd_x) || !valid_hd(hd_w) || !valid_dtype(gw_dtype)) return 0;
+    if (T >= (1ll << 31) || I >= (1ll << 31) || O >= (1ll << 31)) return 0;
+    // nothing is read: stand-ins with the alignment that qm_linear_backward asks for
+    uint8_t* at = reinterpret_cast<uint8_t*>((uintptr_t)256);
+    const size_t ws = work_layout(T, I, O, QM_BF16).gemm_ws_bytes;
+    const auto plan = [&](int64_t M, int64_t K, bool rotate, int hd, int out) {
+        return plan_gradient(qm::make_product(at, at, at, at, M, I, qm::padded_cols(K), 1.0f, at, QM_LAYOUT_TILED, QM_LAYOUT_TILED), at, rotate, hd, QM_BF16, out, at,
+                             nullptr, QM_BF16, ws ? at : nullptr, ws);
+    };
+    return one_launch(plan(T, O, !(rotated_flags & QM_GX_ROTATED), hd_x, QM_BF16), plan(O, T, !(rotated_flags & QM_GW_ROTATED), hd_w, gw_dtype), QM_BF16) ? 1 : 0;
 }
 
 int qm_linear_forward(const void* x, int x_dtype, const void* w, int w_dtype, int64_t T, int64_t I, int64_t O, int hd_x,
@@ -649,26 +698,11 @@ int qm_linear_backward_seeded(const void* e, int e_dtype, int64_t T, int64_t I, 
     if (codes_layout == QM_LAYOUT_TILED && (T % 128 || I % 128 || O % 128))
         return fail(QM_ERR_INVALID, "qm_linear_backward: QM_LAYOUT_TILED needs T, I, O multiples of 128 (QM_LAYOUT_PADDED takes any multiples of 32)");
     const int64_t Kx = tiled ? qm::padded_cols(O) : O, Kw = tiled ? qm::padded_cols(T) : T;
-    struct GradProduct {
-        qm::TileProduct p;
-        qm::ProductChoice choice;
-        int out_dtype;
-    };
     const auto plan_product = [&](size_t ac, size_t as, size_t bc, size_t bs, int64_t M, int64_t N, int64_t K, void* plain_dst, void* final_dst,
                                   bool want_rotation, int hd, int final_dtype, const uint8_t* mask, const uint32_t* signs, int scale_dtype) {
-        GradProduct g{qm::make_product(k + ac, k + as, k + bc, k + bs, M, N, K, alpha, plain_dst, kernel_layout(codes_layout), kernel_layout(codes_layout)), {}, mid_dtype};
-        if (want_rotation && final_dst && aligned(final_dst, 16) && valid_dtype(scale_dtype) && valid_hd(hd) && N % hd == 0) {
-            qm::TileProduct r = g.p;
-            r.c = final_dst;
-            r.mask = mask;
-            r.hd = hd;
-            r.signs = make_signs(signs, hd);
-            r.rot_c = qm::hadamard_scale(hd, scale_dtype);
-            const qm::ProductChoice c = qm::choose_product(r, mid_dtype, final_dtype, gws, wl.gemm_ws_bytes);
-            if (c.rotates) return GradProduct{r, c, final_dtype};
-        }
-        g.choice = qm::choose_product(g.p, mid_dtype, mid_dtype, gws, wl.gemm_ws_bytes);
-        return g;
+        const int kl = kernel_layout(codes_layout);
+        return plan_gradient(qm::make_product(k + ac, k + as, k + bc, k + bs, M, N, K, alpha, plain_dst, kl, kl), final_dst, want_rotation, hd, mid_dtype, final_dtype,
+                             mask, signs, scale_dtype, gws, wl.gemm_ws_bytes);
     };
     const GradProduct gx_plan = plan_product(wl.ec, wl.es, wl.wtc, wl.wts, T, I, Kx, gx_product, gx, !gx_rotated, hd_x, mid_dtype, px + lx.m, signs_x, x_scale_dtype);
     const GradProduct gw_plan = plan_product(wl.etc, wl.ets, wl.xtc, wl.xts, O, I, Kw, gw_product, gw, !gw_rotated, hd_w, gw_dtype, pw + lw.m, signs_w, w_scale_dtype);
@@ -715,6 +749,8 @@ int qm_linear_backward_seeded(const void* e, int e_dtype, int64_t T, int64_t I, 
         const qm::ErrorArgs ae{e, e_dtype, T, O, seeds[0], seeds[2], k + wl.ec, k + wl.es, k + wl.etc, k + wl.ets};
         rc = from_hip(qm::quantize_layer_backward(ae, hd_g, make_signs(signs_g, hd_g), g_mode, rx, rw, seed_base, hs), "qm_linear_backward");
         if (rc) return rc;
+        if (one_launch(gx_plan, gw_plan, mid_dtype))
+            return from_hip(qm::run_pair(gx_plan.whole, gx_plan.whole_dtype, gw_plan.whole, gw_plan.whole_dtype, hs), "qm_linear_backward");
         rc = product_gx();
         if (rc) return rc;
         rc = product_gw();

@@ -421,12 +421,16 @@ struct RotEpilogue {
 };
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-template <bool ROT = false, bool RAGGED = false>
-__device__ __forceinline__ void big4_epilogue_bf16(v16f (&acc)[4][4], float alpha, uint16_t* __restrict__ c, int64_t m0,
+// WIDE: the rotated, bf16-rounded result leaves widened to fp32 (the weight gradient of an fp32 weight), 32 columns at a time through
+// the same 4 KiB, whole 128-byte lines out.
+template <bool ROT = false, bool RAGGED = false, bool WIDE = false>
+__device__ __forceinline__ void big4_epilogue_bf16(v16f (&acc)[4][4], float alpha, void* __restrict__ c, int64_t m0,
                                                    int64_t n0, int64_t N, int wm, int wn, int wave, int lane_in,
                                                    uint8_t* smem_bytes, int rows_valid, int cols_valid,
                                                    [[maybe_unused]] const RotEpilogue& rot, [[maybe_unused]] const u32x4 (&keep)[4],
                                                    [[maybe_unused]] bool keep_shifted) {
+    static_assert(ROT || !WIDE, "plain fp32 results have an epilogue of their own");
+    constexpr int kOut = WIDE ? 4 : 2;   // bytes per result
     // The opaque copy keeps the address arithmetic below inside the (rarely executed) epilogue instead of being
     // hoisted out of the K loop, where it would hold dozens of registers across the MFMA schedule.
     // the lane index straight from the hardware, so that no copy of it has to stay alive through the K loop
@@ -439,8 +443,20 @@ __device__ __forceinline__ void big4_epilogue_bf16(v16f (&acc)[4][4], float alph
     uint8_t* wr = region + lrow * 128 + half * 8;
     const int wsw = (lrow & 7) * 16;
     const uint8_t* rd = region + rsub * 128 + ((chunk ^ rsub) * 16);  // rows rsub + 8k share rsub's swizzle
-    const int64_t pitch8 = N * 16;                                   // eight rows of bf16
-    uint8_t* out = reinterpret_cast<uint8_t*>(c + (m0 + wm * 128 + rsub) * N + n0 + wn * 128) + chunk * 16;
+    const int64_t pitch8 = N * 8 * kOut;                             // eight rows
+    uint8_t* out = static_cast<uint8_t*>(c) + ((m0 + wm * 128 + rsub) * N + n0 + wn * 128) * kOut + chunk * 16;
+    // rows [32 i, 32 i + 32) of the wave's tile, the 128 bytes of each that the stage holds, from byte `col` of its columns on
+    const auto put_rows = [&](int i, int col) {
+#pragma unroll
+        for (int r8 = 0; r8 < 4; ++r8)
+            if (!RAGGED || i * 32 + r8 * 8 + rsub < rows_valid) {
+                const uint4 v = *reinterpret_cast<const uint4*>(rd + r8 * 1024);
+                // streaming store: the tile is not read again by this kernel, and keeping it out of the L2 leaves the
+                // operand panels there (measured: -1.3 % on the product alone, -3 % on the whole layer step)
+                typedef uint32_t u4v __attribute__((ext_vector_type(4)));
+                __builtin_nontemporal_store(u4v{v.x, v.y, v.z, v.w}, reinterpret_cast<u4v*>(out + r8 * pitch8 + col));
+            }
+    };
     // ROT: `keep[i]` holds the four mask words of the lane's row in block row i (one per 32 x 32 block: its group of 32 n),
     // requested at the tile's first K step.  The +-1 matrix: lane (n' = lane % 32, half h) holds, for instruction q,
     // S[n'][n] sign[n] at n = 8 (2 q + rho) + 4 h + e
@@ -525,10 +541,18 @@ __device__ __forceinline__ void big4_epilogue_bf16(v16f (&acc)[4][4], float alph
                             float q[4];
 #pragma unroll
                             for (int e = 0; e < 4; ++e) q[e] = decltype(scaled)::value ? r[jj][4 * b + e] * rot.c : r[jj][4 * b + e];
-                            const v2bf p0 = __builtin_convertvector(v2f{q[0], q[1]}, v2bf);
-                            const v2bf p1 = __builtin_convertvector(v2f{q[2], q[3]}, v2bf);
-                            *reinterpret_cast<uint2*>(wr + (((jj * 4 + b) * 16) ^ wsw)) =
-                                make_uint2(__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1));
+                            const uint32_t p0 = __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{q[0], q[1]}, v2bf));
+                            const uint32_t p1 = __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{q[2], q[3]}, v2bf));
+                            if constexpr (WIDE)
+                                *reinterpret_cast<uint4*>(region + lrow * 128 + (((2 * b + half) * 16) ^ wsw)) =
+                                    make_uint4(p0 << 16, p0 & 0xffff0000u, p1 << 16, p1 & 0xffff0000u);
+                            else
+                                *reinterpret_cast<uint2*>(wr + (((jj * 4 + b) * 16) ^ wsw)) = make_uint2(p0, p1);
+                        }
+                        if constexpr (WIDE) {   // N is a multiple of 64: both blocks of the pass are inside
+                            __builtin_amdgcn_wave_barrier();
+                            put_rows(i, (2 * jp + jj) * 128);
+                            __builtin_amdgcn_wave_barrier();
                         }
                     }
                 };
@@ -536,16 +560,7 @@ __device__ __forceinline__ void big4_epilogue_bf16(v16f (&acc)[4][4], float alph
                 else emit(std::true_type{});
             }
             // the region is private to the wave; LDS operations of one wave complete in order
-            const auto put = [&](int r8) {
-                const uint4 v = *reinterpret_cast<const uint4*>(rd + r8 * 1024);
-                // streaming store: the tile is not read again by this kernel, and keeping it out of the L2 leaves the
-                // operand panels there (measured: -1.3 % on the product alone, -3 % on the whole layer step)
-                typedef uint32_t u4v __attribute__((ext_vector_type(4)));
-                __builtin_nontemporal_store(u4v{v.x, v.y, v.z, v.w}, reinterpret_cast<u4v*>(out + r8 * pitch8 + jp * 128));
-            };
-#pragma unroll
-            for (int r8 = 0; r8 < 4; ++r8)
-                if (!RAGGED || i * 32 + r8 * 8 + rsub < rows_valid) put(r8);
+            if constexpr (!WIDE) put_rows(i, jp * 128);
             // keeps the passes apart: a scheduler that reads many passes' accumulators into vector registers ahead of time
             // pushes the K loop's live values out to scratch memory, and their reloads wait for every operand load in flight
             __builtin_amdgcn_sched_barrier(0);
@@ -565,17 +580,40 @@ __device__ __forceinline__ unsigned long long shader_clock() {
     return t;
 }
 
+// Two products in one grid: the gradients of a layer, gx = Q(e) Q(W^T)^T [T x I, over O] and gw = Q(e^T) Q(x^T)^T [O x I, over T].  They
+// share nothing but N; the one with more K steps comes first and is "the long one".  Launched one after the other each ends in a
+// round of tiles that fills part of the chip, or is cut into K ranges whose partial sums travel through memory; together the tiles
+// of one fill the gaps of the other.  Every XCD has a contiguous run of either product's tiles, its W = grid / 8 workgroups take the
+// long ones in turn, then `rounds` short ones each, and those that had one long tile fewer take the short ones that are left:
+// the host picks `rounds` so that all end together.  What bounds it is what bounds the kernel with one product (the power limit: 3.4 to
+// 4.1 PFLOP/s); figures at pair_pays().
+struct Big4Other {   // the short product; the long one is the kernel's first arguments
+    const uint8_t* a_codes;
+    const uint8_t* a_scales;
+    const uint8_t* b_codes;
+    const uint8_t* b_scales;
+    void* c;
+    RotEpilogue rot;
+    int M, K;
+    int rounds;
+    int kind, long_kind;   // Big4Result of the short and of the long product
+};
+struct Big4NoOther {};
+enum Big4Result : int { BIG4_PLAIN = 1, BIG4_ROTATED = 2, BIG4_WIDE = 4 };   // bf16, with the rotation, with it and widened to fp32
+
 // Persistent: the grid is one workgroup per CU (or fewer); each workgroup walks tiles bid, bid + grid, ... as one
 // flat stream of K steps.  The loads that refill a freed ring stage simply continue into the next tile, so the
 // pipeline never drains between tiles and the epilogue runs while the next tile's first four stages arrive.
 // RAGGED: M is not a multiple of 64 (an instantiation of its own: the row tests cost the others 2 to 8 % in registers).
-template <typename OutT, bool STAMP = false, bool ROT = false, bool RAGGED = false>
+// PAIR: two products (Big4Other), tiled operands; the sum of the kinds of result that they have.
+template <typename OutT, bool STAMP = false, bool ROT = false, bool RAGGED = false, int PAIR = 0>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_mxfp4_tn_big4_kernel(
     const uint8_t* __restrict__ a_codes, const uint8_t* __restrict__ a_scales, const uint8_t* __restrict__ b_codes,
     const uint8_t* __restrict__ b_scales, int M, int N, int K, float alpha, OutT* __restrict__ c, int a_tiled,
     int b_tiled, int splits, int late, [[maybe_unused]] unsigned long long* __restrict__ stamps,
-    [[maybe_unused]] RotEpilogue rot = RotEpilogue{}) {
+    [[maybe_unused]] RotEpilogue rot = RotEpilogue{}, [[maybe_unused]] std::conditional_t<PAIR != 0, Big4Other, Big4NoOther> other = {}) {
     static_assert(!ROT || sizeof(OutT) == 2, "the fused inverse rotation is part of the bf16 epilogue");
+    static_assert(!PAIR || (ROT && !STAMP && (PAIR & (BIG4_ROTATED | BIG4_WIDE))), "a pair without any rotation holds mask words that nothing reads");
     extern __shared__ uint32_t smem[];
     uint8_t* smem_bytes = reinterpret_cast<uint8_t*>(smem);
     const uint32_t smem_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint32_t*)smem;
@@ -624,11 +662,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     // the offsets of clamped rows may fall below i * 1024: RAGGED takes them from a base that much further back
     constexpr uint32_t kLoadBias = RAGGED ? 3 * 1024 : 0;
     // source of this lane in wave-load i: row 16 i + lane / 4 of the wave's 64 (at most `last`), swizzled 16-byte column
-    const auto lane_source = [&](int i, int last, int tiled) {
+    const auto lane_source = [&](int i, int last, int tiled, uint32_t rows16, int pitch) {
         const int prow = lane >> 2, pcv = (lane & 3) ^ ((prow >> 2) & 3);
         int r = 16 * i + prow;
         r = r < last ? r : last;
-        const uint32_t off = tiled ? (uint32_t)(r >> 4) * row16 + (uint32_t)(r & 15) * 64u : (uint32_t)r * (uint32_t)code_pitch;
+        const uint32_t off = tiled ? (uint32_t)(r >> 4) * rows16 + (uint32_t)(r & 15) * 64u : (uint32_t)r * (uint32_t)pitch;
         return off + pcv * 16 + kLoadBias - 1024u * i;
     };
     plan.kstep_a = a_tiled ? 1024 : kRowBytes;
@@ -636,32 +674,70 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     plan.lane_scales_a = plan.lane_scales_b = (uint32_t)(lane * groups);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        plan.voff_a[i] = lane_source(i, 63, a_tiled);
-        plan.voff_b[i] = lane_source(i, 63, b_tiled);
+        plan.voff_a[i] = lane_source(i, 63, a_tiled, row16, code_pitch);
+        plan.voff_b[i] = lane_source(i, 63, b_tiled, row16, code_pitch);
     }
     const int wave_u = wave;
     int load_tm, load_tn, load_split;  // work item the load stream is in
+    [[maybe_unused]] bool load_short = false;
+    // the panels of the tile at (load_tm, load_tn) of a product
+    const auto plan_panels = [&](const uint8_t* ac, const uint8_t* as, const uint8_t* bc, const uint8_t* bs, int rows, int pitch, int64_t k0) {
+        // N, and but for RAGGED M, is a multiple of 64: a wave's 64-row share of a panel is inside the matrix or outside it as a
+        // whole; an outside share reads the matrix's last 64 rows instead (its products are dropped by the epilogue).
+        // RAGGED: A's rows past the end read the last row (of the last block of 16 in a tiled operand).
+        const int g = pitch / 16;
+        int64_t m0 = (int64_t)load_tm * kBigM + wave_u * 64, n0 = (int64_t)load_tn * kBigN + wave_u * 64;
+        m0 = m0 < rows ? m0 : RAGGED ? (int64_t)((rows - 1) & ~63) : (int64_t)rows - 64;
+        n0 = n0 < N ? n0 : (int64_t)N - 64;
+        plan.a = ac + m0 * pitch + k0 * plan.kstep_a - kLoadBias;
+        plan.b = bc + n0 * pitch + k0 * plan.kstep_b - kLoadBias;
+        if constexpr (RAGGED || PAIR) {   // otherwise the lane offsets never change
+            const int last = RAGGED ? rows - 1 - (int)m0 : 63, last_code = a_tiled ? last | 15 : last;
+            const uint32_t rows16 = 16u * (uint32_t)pitch;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                plan.voff_a[i] = lane_source(i, last_code, a_tiled, rows16, pitch);
+                if constexpr (PAIR) plan.voff_b[i] = lane_source(i, 63, b_tiled, rows16, pitch);
+            }
+            plan.lane_scales_a = (uint32_t)((lane < last ? lane : last) * g);
+            if constexpr (PAIR) plan.lane_scales_b = (uint32_t)(lane * g);
+        }
+        plan.sa = as + m0 * g + k0 * 4;
+        plan.sb = bs + n0 * g + k0 * 4;
+    };
+    // PAIR: the next of this workgroup's tiles, the `taken`-th; false behind the last one
+    [[maybe_unused]] int taken = 0;
+    const auto next_of_pair = [&]() -> bool {
+        if constexpr (PAIR != 0) {
+            const int W = (int)gridDim.x >> 3, j = (int)blockIdx.x >> 3, xcd = (int)blockIdx.x & 7, back = 7 - xcd;
+            const int short_tiles = (other.M + kBigM - 1) / kBigM * tiles_n;
+            const int longs = (total >> 3) + (xcd < (total & 7) ? 1 : 0), shorts = (short_tiles >> 3) + (back < (short_tiles & 7) ? 1 : 0);
+            const int heavy = longs % W;   // workgroups with a long tile more than the others
+            int at = j + W * taken;
+            load_short = at >= longs;
+            if (load_short) {
+                const int r = taken - longs / W - (j < heavy ? 1 : 0);
+                if (r >= other.rounds && heavy && j < heavy) return false;
+                at = r < other.rounds || !heavy ? j + W * r : W * other.rounds + (j - heavy) + (W - heavy) * (r - other.rounds);
+                if (at >= shorts) return false;
+                // the short product's extra tiles go to the XCDs that have none of the long one's
+                at += back * (short_tiles >> 3) + (back < (short_tiles & 7) ? back : short_tiles & 7);
+                tile_of_run(at, (other.M + kBigM - 1) / kBigM, tiles_n, load_tm, load_tn);
+            } else {
+                at += xcd * (total >> 3) + (xcd < (total & 7) ? xcd : total & 7);
+                tile_of_run(at, tiles_m, tiles_n, load_tm, load_tn);
+            }
+            ++taken;
+            if (load_short) plan_panels(other.a_codes, other.a_scales, other.b_codes, other.b_scales, other.M, other.K / 2, 0);
+            else plan_panels(a_codes, a_scales, b_codes, b_scales, M, code_pitch, 0);
+        }
+        return true;
+    };
     auto plan_tile = [&](int item) {
         const int r = xcd_run(item, total_items);
         load_split = r / total;
         tile_of_run(r - load_split * total, tiles_m, tiles_n, load_tm, load_tn);
-        // N, and but for RAGGED M, is a multiple of 64: a wave's 64-row share of a panel is inside the matrix or outside it as a
-        // whole; an outside share reads the matrix's last 64 rows instead (its products are dropped by the epilogue).
-        // RAGGED: A's rows past the end read the last row (of the last block of 16 in a tiled operand).
-        int64_t m0 = (int64_t)load_tm * kBigM + wave_u * 64, n0 = (int64_t)load_tn * kBigN + wave_u * 64;
-        m0 = m0 < M ? m0 : RAGGED ? (int64_t)((M - 1) & ~63) : (int64_t)M - 64;
-        n0 = n0 < N ? n0 : (int64_t)N - 64;
-        const int64_t k0 = (int64_t)load_split * nk_real;  // first K step of the item
-        plan.a = a_codes + m0 * code_pitch + k0 * plan.kstep_a - kLoadBias;
-        plan.b = b_codes + n0 * code_pitch + k0 * plan.kstep_b - kLoadBias;
-        if constexpr (RAGGED) {   // otherwise the lane offsets never change
-            const int last = M - 1 - (int)m0, last_code = a_tiled ? last | 15 : last;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) plan.voff_a[i] = lane_source(i, last_code, a_tiled);
-            plan.lane_scales_a = (uint32_t)((lane < last ? lane : last) * groups);
-        }
-        plan.sa = a_scales + m0 * groups + k0 * 4;
-        plan.sb = b_scales + n0 * groups + k0 * 4;
+        plan_panels(a_codes, a_scales, b_codes, b_scales, M, code_pitch, (int64_t)load_split * nk_real);   // from the item's first K step
     };
 
     // Short contractions: every other group of eight workgroups (one per XCD) starts `late` x 1024 cycles late -- about the
@@ -671,7 +747,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     // 32768 x 1536 x 1536: 53-57 us in step, 45-46 us out of step; with the late start always the latter).
     if (((int)blockIdx.x >> 3) & 1)
         for (int i = 0; i < late; ++i) __builtin_amdgcn_s_sleep(16);
-    plan_tile((int)blockIdx.x);
+    if constexpr (PAIR != 0) {
+        if (!next_of_pair()) return;
+    } else {
+        plan_tile((int)blockIdx.x);
+    }
     big4_issue_scales(plan, 0, 0);  // K >= 512: the first block is a whole one
     big4_issue_codes(plan, 0, 0);
     big4_issue_codes(plan, 1, 1);
@@ -687,11 +767,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 
     int par = 0;
     stamp();
-    for (int t = (int)blockIdx.x; t < total_items; t += stride) {
+    [[maybe_unused]] bool more = true;
+    for (int t = (int)blockIdx.x; PAIR ? more : t < total_items; t += stride) {
         v16f acc[4][4];
         const int64_t m0 = (int64_t)load_tm * kBigM, n0 = (int64_t)load_tn * kBigN;  // the load stream is still in item t
-        const int cur_split = load_split;
-        const int rows_valid = (int)(M - m0) - wm * 128, cols_valid = (int)(N - n0) - wn * 128;
+        const int cur_split = PAIR ? 0 : load_split;
+        int rows = M, steps_real = nk_real;   // of the product that the tile belongs to
+        int result = ROT ? BIG4_ROTATED : BIG4_PLAIN;
+        [[maybe_unused]] RotEpilogue turn = rot;
+        void* dst = c;
+        if constexpr (PAIR != 0) {
+            result = other.long_kind;
+            if (load_short) {
+                rows = other.M;
+                steps_real = other.K / kBK;
+                result = other.kind;
+                turn = other.rot;
+                dst = other.c;
+            }
+        }
+        const int steps = PAIR ? (steps_real + 3) & ~3 : nk, muted_steps = PAIR ? steps - steps_real : muted;
+        const int rows_valid = (int)(rows - m0) - wm * 128, cols_valid = (int)(N - n0) - wn * 128;
         // One block of four K steps.  The load stream is four K steps ahead and rolls over into the next tile;
         // after the last tile it re-requests the current steps (never consumed), which keeps the outstanding-load
         // counts uniform.  FIRST: the tile's first products overwrite the accumulators instead of adding to them.
@@ -704,15 +800,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         [[maybe_unused]] u32x4 keep[4];
         [[maybe_unused]] bool keep_shifted = false;
         if constexpr (ROT) {
-            const int64_t mask_pitch = N / 8;
+            // a plain product of a pair has no mask: its requests, which the counts of pending ones include, read 16 bytes of A
+            const int64_t mask_pitch = PAIR && result == BIG4_PLAIN ? 0 : N / 8;
             int64_t ncol = n0 + wn * 128;
             keep_shifted = ncol + 128 > N;   // wave-uniform; N >= 256
             ncol = keep_shifted ? (int64_t)N - 128 : ncol;
+            if (PAIR && result == BIG4_PLAIN) ncol = 0;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 int64_t mrow = m0 + wm * 128 + i * 32 + lrow;
-                mrow = mrow < M ? mrow : (int64_t)M - 1;
-                const uint8_t* src = rot.mask + mrow * mask_pitch + ncol / 8;
+                mrow = mrow < rows ? mrow : (int64_t)rows - 1;
+                const uint8_t* src = turn.mask + mrow * mask_pitch + ncol / 8;
                 asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(keep[i]) : "v"(src) : "memory");
             }
         }
@@ -721,16 +819,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             // the four mask-word requests are younger than the stages the first block's steps 0..2 wait for
             constexpr int EX = (FIRST && ROT) ? 4 : 0;
             int lks = ks + 4;
-            if (lks == nk) {
-                if (t + stride < total_items) {
+            if (lks == steps) {
+                if constexpr (PAIR != 0) {
+                    more = next_of_pair();
+                    lks = more ? 0 : ks;
+                } else if (t + stride < total_items) {
                     plan_tile(t + stride);
                     lks = 0;
                 } else {
                     lks = ks;
                 }
             }
-            const int lbase = lks + 4 <= nk_real ? lks : nk_real - 4;    // a short last block: the row's final four steps
-            const int first_live = ks + 4 > nk_real ? muted : 0;         // this block's steps below it are muted
+            const int lbase = lks + 4 <= steps_real ? lks : steps_real - 4;    // a short last block: the row's final four steps (a next tile's first: 0)
+            const int first_live = ks + 4 > steps_real ? muted_steps : 0;      // this block's steps below it are muted
             const auto sw = [&](int q) { return q < first_live ? 0 : 16; };
             big4_step<0, sizeof(OutT) == 2, FIRST, EX>(plan, smem_bytes, lbase, lbase * 4, sw(0), par, a_off0, a_off1, b_off0, b_off1, a_sc_off, b_sc_off, sh, st, acc);
             big4_step<1, sizeof(OutT) == 2, false, EX>(plan, smem_bytes, lbase + 1, 0, sw(1), par, a_off0, a_off1, b_off0, b_off1, a_sc_off, b_sc_off, sh, st, acc);
@@ -739,13 +840,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             par ^= 1;
         };
         block4(0, std::true_type{});
-        for (int ks = 4; ks < nk; ks += 4) block4(ks, std::false_type{});
+        for (int ks = 4; ks < steps; ks += 4) block4(ks, std::false_type{});
         stamp();
-        if constexpr (sizeof(OutT) == 2) {
-            big4_epilogue_bf16<ROT, RAGGED>(acc, alpha, reinterpret_cast<uint16_t*>(c), m0, n0, N, wm, wn, wave, lane, smem_bytes,
-                                    rows_valid, cols_valid, rot, keep, keep_shifted);
+        if constexpr (PAIR != 0) {
+            const auto leave = [&](auto rotated, auto wide) {
+                big4_epilogue_bf16<decltype(rotated)::value, RAGGED, decltype(wide)::value>(acc, alpha, dst, m0, n0, N, wm, wn, wave, lane, smem_bytes,
+                                                                                            rows_valid, cols_valid, turn, keep, keep_shifted);
+            };
+            if ((PAIR & BIG4_PLAIN) && result == BIG4_PLAIN) {
+                // a use of the words that the tile requested, so that their registers stay theirs until they have arrived
+#pragma unroll
+                for (int i = 0; i < 4; ++i) asm volatile("" ::"v"(keep[i]));
+                leave(std::false_type{}, std::false_type{});
+            } else if ((PAIR & BIG4_WIDE) && ((PAIR & BIG4_ROTATED) == 0 || result == BIG4_WIDE)) leave(std::true_type{}, std::true_type{});
+            else leave(std::true_type{}, std::false_type{});
+        } else if constexpr (sizeof(OutT) == 2) {
+            big4_epilogue_bf16<ROT, RAGGED>(acc, alpha, dst, m0, n0, N, wm, wn, wave, lane, smem_bytes, rows_valid, cols_valid, turn, keep, keep_shifted);
         } else {
-            OutT* dst = splits > 1 ? c + (int64_t)cur_split * M * N : c;
+            OutT* slab = splits > 1 ? c + (int64_t)cur_split * M * N : c;
             const float a_eff = splits > 1 ? 1.0f : alpha;
             acc_settle();
 #pragma unroll
@@ -754,7 +866,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
                 for (int j = 0; j < 4; ++j)
                     if (i * 32 < rows_valid && j * 32 < cols_valid) {
                         const int64_t row0 = m0 + wm * 128 + i * 32, col = n0 + wn * 128 + j * 32 + lrow;
-                        store_tile<OutT, true>(acc[i][j], a_eff, dst, row0, col, N, half, RAGGED ? rows_valid - i * 32 : 32);
+                        store_tile<OutT, true>(acc[i][j], a_eff, slab, row0, col, N, half, RAGGED ? rows_valid - i * 32 : 32);
                     }
         }
         stamp();
@@ -942,7 +1054,7 @@ hipError_t launch_big4_as(const uint8_t* a_codes, const uint8_t* a_scales, const
     if (g > 8 && g < items) g -= g % 8;
     dim3 grid((unsigned)g), block(256);
     kern<<<grid, block, kBig4SmemBytes, stream>>>(a_codes, a_scales, b_codes, b_scales, (int)M, (int)N, (int)K, alpha,
-                                                  reinterpret_cast<OutT*>(c), a_tiled, b_tiled, splits, big4_late_start(K, splits), nullptr, rot);
+                                                  reinterpret_cast<OutT*>(c), a_tiled, b_tiled, splits, big4_late_start(K, splits), nullptr, rot, Big4NoOther{});
     return hipGetLastError();
 }
 template <typename OutT, bool ROT = false>
@@ -1003,7 +1115,7 @@ hipError_t gemm_tile_phases(const uint8_t* a_codes, const uint8_t* a_scales, con
     kern<<<dim3((unsigned)g), dim3(256), kBig4SmemBytes, stream>>>(a_codes, a_scales, b_codes, b_scales, (int)M, (int)N, (int)K, alpha,
                                                                   reinterpret_cast<uint16_t*>(c), a_layout == LAYOUT_TILED,
                                                                   b_layout == LAYOUT_TILED, 1, big4_late_start(K, 1), stamps,
-                                                                  RotEpilogue{rot_mask, 0u, hadamard_scale(32, BF16)});
+                                                                  RotEpilogue{rot_mask, 0u, hadamard_scale(32, BF16)}, Big4NoOther{});
     *grid_out = (int)g;
     return hipGetLastError();
 }
@@ -1096,6 +1208,7 @@ ProductChoice choose_product(const TileProduct& p, int c_dtype, int rot_out_dtyp
     if (plan.cut_bytes && workspace && plan.cut_bytes <= workspace_bytes && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0) {
         ProductChoice c = plan.cut.choice;
         c.rotates = rotate;
+        c.cost = plan.cut.cost;
         return c;
     }
     const double separate = rotate ? separate_rotate_cost(M, N, c_dtype == BF16 ? 2 : 4, rot_out_dtype == BF16 ? 2 : 4) : 0.0;
@@ -1105,6 +1218,7 @@ ProductChoice choose_product(const TileProduct& p, int c_dtype, int rot_out_dtyp
         if (cost < best_cost) {
             best_cost = cost;
             best = c;
+            best.cost = cost;
         }
     };
     const bool bf16 = c_dtype == BF16;
@@ -1167,6 +1281,86 @@ hipError_t run_product(const ProductChoice& c, const TileProduct& p, int c_dtype
     if (c_dtype == BF16)
         return launch_big4<uint16_t>(p.a_codes, p.a_scales, p.b_codes, p.b_scales, M, N, K, p.alpha, p.c, p.a_tiled, p.b_tiled, 1, cus, stream);
     return launch_big4<float>(p.a_codes, p.a_scales, p.b_codes, p.b_scales, M, N, K, p.alpha, p.c, p.a_tiled, p.b_tiled, 1, cus, stream);
+}
+
+// ---- the two gradient products of a layer in one launch --------------------------------------------------------------
+namespace {
+int64_t big_tiles(const TileProduct& p) { return (int64_t)((p.M + kBigM - 1) / kBigM) * ((p.N + kBigN - 1) / kBigN); }
+int pair_grid(int64_t tiles, int cus) { return (int)(tiles < cus ? tiles : cus) & ~7; }   // as many workgroups on every XCD
+double pair_tile_cost(int64_t K) { return ((K / kBK + 3) & ~(int64_t)3) * kPersistentStep + kPersistentBoundary + (K % 512 ? kPersistentMuted : 0.0); }
+// when the last workgroup of the fullest XCD ends, and how many short tiles every workgroup takes first (see Big4Other)
+double pair_makespan(const TileProduct& lng, const TileProduct& sht, int cus, int* rounds) {
+    const int64_t tl = big_tiles(lng), ts = big_tiles(sht), W = pair_grid(tl + ts, cus) / 8, L = (tl + 7) / 8, S = (ts + 7) / 8, heavy = L % W;
+    const double cl = pair_tile_cost(lng.K), cs = pair_tile_cost(sht.K);
+    double best = 1e30;
+    for (int64_t b = 0; b <= (S + W - 1) / W; ++b) {
+        const int64_t left = S - W * b > 0 ? S - W * b : 0;
+        const double all = (double)(L / W) * cl + b * cs, with = heavy ? all + cl : 0.0, without = all + (double)((left + W - heavy - 1) / (W - heavy)) * cs;
+        const double end = with > without ? with : without;
+        if (end < best) {
+            best = end;
+            *rounds = (int)b;
+        }
+    }
+    return best;
+}
+template <int PAIR, bool RAGGED>
+hipError_t launch_pair_as(const TileProduct& lng, const Big4Other& other, const RotEpilogue& rot, int late, int grid, hipStream_t stream) {
+    auto kern = gemm_mxfp4_tn_big4_kernel<uint16_t, false, true, RAGGED, PAIR>;
+    static std::atomic<bool> lds_allowed[kMaxDevices];
+    const hipError_t e = allow_dynamic_lds(kern, kBig4SmemBytes, lds_allowed);
+    if (e != hipSuccess) return e;
+    kern<<<dim3((unsigned)grid), dim3(256), kBig4SmemBytes, stream>>>(lng.a_codes, lng.a_scales, lng.b_codes, lng.b_scales, lng.M, lng.N, lng.K, lng.alpha,
+                                                                      static_cast<uint16_t*>(lng.c), 1, 1, 1, late, nullptr, rot, other);
+    return hipGetLastError();
+}
+}  // namespace
+
+// Served: both products by the persistent kernel, tiled, with at least one tile per CU between them (fewer leave CUs idle, which
+// smaller tiles and K ranges do not); bf16 results, plain or with the rotation over blocks of 32, one of them with it, and only
+// rotated ones widened.  Worth it where the estimate of the one launch is clearly below the sum of the two products' own.  Timed
+// against two launches, whole training steps: 52 shapes from 0.62 to 0.94 of that sum are 0.99 to 1.19 times as fast (mean 1.05; 4096 x
+// 2048 x 4096 116 us, now 104; 16384 x 1536 x 4608 behind its norm 471 -> 453; 16384 x 4096 x 1536 behind SwiGLU 457 -> 431; 8192 x 4096^2
+// 291 -> 287), what is gained being the idle part of each product's last round, or writing and reading partial sums; none lies
+// between 0.94 and 1, where the estimates (6 % off on average) no longer tell.
+constexpr double kPairMargin = 0.95;
+bool pair_pays(const TileProduct& x, const ProductChoice& cx, int x_out, const TileProduct& w, const ProductChoice& cw, int w_out, int c_dtype) {
+    if (c_dtype != BF16 || x.N != w.N || x.alpha != w.alpha || x.b_e5m2 || w.b_e5m2) return false;
+    const auto serves = [](const TileProduct& p, int out) {
+        return p.a_tiled && p.b_tiled && (p.mask ? p.hd == 32 : out == BF16) && persistent_serves(p.M, p.N, p.K, p.a_scales, p.b_scales, p.c);
+    };
+    if (!serves(x, x_out) || !serves(w, w_out) || (!x.mask && !w.mask)) return false;
+    const int cus = device_cus();
+    if (cus < 8 || big_tiles(x) + big_tiles(w) < cus) return false;
+    int rounds;
+    const bool x_long = x.K > w.K;
+    double cost = kLaunch + pair_makespan(x_long ? x : w, x_long ? w : x, cus, &rounds) + kPersistentRotate;
+    if (x.mask && x_out != BF16) cost += (double)x.M * x.N * 2 / kWideStores;
+    if (w.mask && w_out != BF16) cost += (double)w.M * w.N * 2 / kWideStores;
+    return cost < kPairMargin * (cx.cost + cw.cost);
+}
+hipError_t run_pair(const TileProduct& x, int x_out, const TileProduct& w, int w_out, hipStream_t stream) {
+    const bool x_long = x.K > w.K;
+    const TileProduct &lng = x_long ? x : w, &sht = x_long ? w : x;
+    const int cus = device_cus();
+    const auto kind = [](const TileProduct& p, int out) { return !p.mask ? BIG4_PLAIN : out == BF16 ? BIG4_ROTATED : BIG4_WIDE; };
+    // a plain product's mask requests, which nothing reads, go to its A
+    const auto rot = [](const TileProduct& p) { return RotEpilogue{p.mask ? p.mask : p.a_codes, p.signs.w[0], p.rot_c}; };
+    Big4Other o{sht.a_codes, sht.a_scales, sht.b_codes, sht.b_scales, sht.c, rot(sht), sht.M, sht.K, 0,
+                kind(sht, x_long ? w_out : x_out), kind(lng, x_long ? x_out : w_out)};
+    pair_makespan(lng, sht, cus, &o.rounds);
+    const int late = big4_late_start(sht.K, 1), grid = pair_grid(big_tiles(x) + big_tiles(w), cus);
+    const auto go = [&](auto pair) {
+        constexpr int P = decltype(pair)::value;
+        return x.M % 64 || w.M % 64 ? launch_pair_as<P, true>(lng, o, rot(lng), late, grid, stream) : launch_pair_as<P, false>(lng, o, rot(lng), late, grid, stream);
+    };
+    switch (o.kind | o.long_kind) {
+        case BIG4_ROTATED: return go(std::integral_constant<int, BIG4_ROTATED>{});
+        case BIG4_ROTATED | BIG4_WIDE: return go(std::integral_constant<int, BIG4_ROTATED | BIG4_WIDE>{});
+        case BIG4_PLAIN | BIG4_ROTATED: return go(std::integral_constant<int, BIG4_PLAIN | BIG4_ROTATED>{});
+        case BIG4_PLAIN | BIG4_WIDE: return go(std::integral_constant<int, BIG4_PLAIN | BIG4_WIDE>{});
+        default: return hipErrorInvalidValue;
+    }
 }
 
 TileProduct make_product(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes, const uint8_t* b_scales, int64_t M, int64_t N,

@@ -234,11 +234,16 @@ struct ProductChoice {
     int kind;      // TileKind
     int splits;    // K ranges (their fp32 partial sums in the workspace, then one ordered reduction)
     bool rotates;
+    double cost = 0.0;   // the estimate, in microseconds, a rotation in a pass of its own included
 };
 TileProduct make_product(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes, const uint8_t* b_scales, int64_t M, int64_t N,
                          int64_t K, float alpha, void* c, int a_layout, int b_layout);
 ProductChoice choose_product(const TileProduct& p, int c_dtype, int rot_out_dtype, const void* workspace, size_t workspace_bytes);
 hipError_t run_product(const ProductChoice& c, const TileProduct& p, int c_dtype, int rot_out_dtype, void* workspace, hipStream_t stream);
+// The gradient products x and w of a layer in one launch of the persistent kernel: whether it serves them and is expected to be
+// faster than running them as cx and cw say; p.mask and *_out as in choose_product.  The results are those of the persistent kernel.
+bool pair_pays(const TileProduct& x, const ProductChoice& cx, int x_out, const TileProduct& w, const ProductChoice& cw, int w_out, int c_dtype);
+hipError_t run_pair(const TileProduct& x, int x_out, const TileProduct& w, int w_out, hipStream_t stream);
 // the rotation in the persistent kernel's bf16 epilogue (Hadamard block 32)
 bool gemm_persistent_rotates(const uint8_t* a_scales, const uint8_t* b_scales, int64_t M, int64_t N, int64_t K);
 hipError_t gemm_persistent_rotated(TileProduct p, hipStream_t stream);
