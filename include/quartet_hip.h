@@ -274,13 +274,13 @@ int qm_dequantize_mxfp4(const uint8_t* codes, const uint8_t* scales, int64_t R, 
  * With the tiled layouts the forward product of at most 64 tokens may add its terms in another order than that of more
  * (see qm_linear_decode, which gives the same bits).
  * The forward quantizer's masked inverse rotation is applied by the gradient product that feeds it where the kernel serving
- * the shape can: in the epilogue of the 256 x 256 kernel (bf16 mid_dtype, Hadamard block 32, for gw also gw_dtype ==
- * mid_dtype; see qm_gemm_mxfp4_tn_rotated), in the epilogue of the smaller tile kernels (bf16 mid_dtype, any Hadamard block,
+ * the shape can: in the epilogue of the 256 x 256 kernel (bf16 mid_dtype, column signs that
+ * repeat every 32, for gw alone also gw_dtype == mid_dtype; see qm_gemm_mxfp4_tn_rotated), in the epilogue of the smaller tile kernels (bf16 mid_dtype, any Hadamard block,
  * any gw_dtype), or in the ordered reduction of a product cut into K ranges (any Hadamard block, mid_dtype and gw_dtype);
  * the last two with the arithmetic and roundings of the separate launches.  Elsewhere it is a launch of its own.
- * Where both gradient products (bf16 mid_dtype, padded or tiled layout, Hadamard blocks 32) run fastest in one launch of the 256 x 256
+ * Where both gradient products (bf16 mid_dtype, padded or tiled layout, the same Hadamard block) run fastest in one launch of the 256 x 256
  * kernel, they do: with its epilogue for gx and for gw, of either gw_dtype, and without K ranges.
- * qm_linear_backward_in_one_launch tells (1 / 0).
+ * qm_linear_backward_in_one_launch tells (1 / 0; of forward quantizers without column signs).
  */
 size_t qm_packed_operand_bytes(int64_t rows, int64_t cols);
 /* offsets: HOST array of three (codes, scales, mask bits); returns 0, or QM_ERR_INVALID unless cols % 32 == 0 */

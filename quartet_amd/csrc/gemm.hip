@@ -408,22 +408,25 @@ __device__ __forceinline__ void big4_step(const Big4Plan& plan, uint8_t* smem_by
 // columns per wave through a private 4 KiB LDS stage outside the operand ring, so the next tile's operands
 // keep streaming in underneath; 16-byte chunks are XOR-swizzled by row so that writes and reads spread over
 // all banks.
-// ROT: the masked inverse Hadamard rotation of the layer's backward pass (groups of 32 along n) applied to the tile before it
+// ROT (a Hadamard block, 32, 64 or 128; 0: none): the masked inverse Hadamard rotation of the layer's backward pass applied to the tile before it
 // is stored: out[m][n'] = c * sum_n (bf16(alpha * acc[m][n]) * keep[m][n]) * S[n'][n] * sign[n], S the 32 x 32 Sylvester
 // matrix.  With the operand roles swapped a lane holds 16 of a group's 32 n for one m, which is the layout the bf16
 // matrix instruction reads its second operand in (k along the registers, column = lane % 32); its first operand is the
 // +-1 matrix, rebuilt per tile from the sign word.  The sums are fp32 sums of bf16 values in the instruction's order
 // (the stand-alone kernel adds them as a butterfly), the factor c and the final rounding are the same.
+// Blocks of 64 and 128 are sums and differences of those of 32 in the lane's own registers: 32 or 128 vector additions a pass, which
+// makes this kernel serve what 128 x 128 tiles with lane exchanges did.  us per training step, hd 128: 8192 x 4096^2 335 -> 306,
+// 8192 x 1536 x 4608 with an fp32 weight 204 -> 192, 6912 x 7168 x 3968 477 -> 440; hd 64: 8192 x 4096^2 332 -> 302.
 struct RotEpilogue {
     const uint8_t* mask;  // [M][N / 8] clip-mask bits, bit n % 8 of byte n / 8
-    uint32_t signs;       // bit n: column n of the Hadamard block negated
+    uint32_t signs;       // bit n: column n of every 32 of the Hadamard block negated
     float c;              // 32^-1/2, rounded to the scale dtype
 };
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // WIDE: the rotated, bf16-rounded result leaves widened to fp32 (the weight gradient of an fp32 weight), 32 columns at a time through
 // the same 4 KiB, whole 128-byte lines out.
-template <bool ROT = false, bool RAGGED = false, bool WIDE = false>
+template <int ROT = 0, bool RAGGED = false, bool WIDE = false>
 __device__ __forceinline__ void big4_epilogue_bf16(v16f (&acc)[4][4], float alpha, void* __restrict__ c, int64_t m0,
                                                    int64_t n0, int64_t N, int wm, int wn, int wave, int lane_in,
                                                    uint8_t* smem_bytes, int rows_valid, int cols_valid,
@@ -431,6 +434,7 @@ __device__ __forceinline__ void big4_epilogue_bf16(v16f (&acc)[4][4], float alph
                                                    [[maybe_unused]] bool keep_shifted) {
     static_assert(ROT || !WIDE, "plain fp32 results have an epilogue of their own");
     constexpr int kOut = WIDE ? 4 : 2;   // bytes per result
+    constexpr int kSide = ROT == 128 ? 4 : 2;   // blocks of 32 columns per pass
     // The opaque copy keeps the address arithmetic below inside the (rarely executed) epilogue instead of being
     // hoisted out of the K loop, where it would hold dozens of registers across the MFMA schedule.
     // the lane index straight from the hardware, so that no copy of it has to stay alive through the K loop
@@ -487,8 +491,8 @@ __device__ __forceinline__ void big4_epilogue_bf16(v16f (&acc)[4][4], float alph
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
 #pragma unroll
-        for (int jp = 0; jp < 2; ++jp) {
-            if (i * 32 >= rows_valid || jp * 64 >= cols_valid) continue;  // uniform: this pass lies outside the matrix
+        for (int jp = 0; jp < 4 / kSide; ++jp) {
+            if (i * 32 >= rows_valid || jp * kSide * 32 >= cols_valid) continue;  // uniform: this pass lies outside the matrix
             if constexpr (!ROT) {
 #pragma unroll
                 for (int jj = 0; jj < 2; ++jj) {
@@ -502,18 +506,19 @@ __device__ __forceinline__ void big4_epilogue_bf16(v16f (&acc)[4][4], float alph
                             make_uint2(__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1));
                     }
                 }
+                put_rows(i, jp * 128);
             } else {
                 // Both blocks of the pass go through the matrix pipe before either result is read: the second block's
                 // conversion and masking run while the first block's instructions are in flight (the opaque copies below
                 // keep the read-out of the results behind both blocks' matrix instructions).  Per tile 15.9 k -> 14.7 k cycles.
-                v16f r[2];
+                v16f r[kSide];
 #pragma unroll
-                for (int jj = 0; jj < 2; ++jj) {
-                    const v16f& t = acc[i][2 * jp + jj];
+                for (int jj = 0; jj < kSide; ++jj) {
+                    const v16f& t = acc[i][kSide * jp + jj];
                     // the block rounded to bf16 and masked: register pair 2 b + k holds n = 8 b + 4 half + 2 k, + 1
                     // the block's mask word: word j of the row's four, or word j + 2 where the wave requested the row's last
                     // 16 bytes (its columns hang over the edge of N; blocks 2 and 3 are then outside and skipped)
-                    const uint32_t kword = keep_shifted ? keep[i][(2 * jp + jj + 2) & 3] : keep[i][2 * jp + jj];
+                    const uint32_t kword = keep_shifted ? keep[i][(kSide * jp + jj + 2) & 3] : keep[i][kSide * jp + jj];
                     const uint32_t kw = kword >> (4 * half);
                     uint32_t pk[8];
 #pragma unroll
@@ -532,10 +537,27 @@ __device__ __forceinline__ void big4_epilogue_bf16(v16f (&acc)[4][4], float alph
                     z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(hmat[0], __builtin_bit_cast(v8bf, u32x4{pk[0], pk[1], pk[2], pk[3]}), z, 0, 0, 0);
                     r[jj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(hmat[1], __builtin_bit_cast(v8bf, u32x4{pk[4], pk[5], pk[6], pk[7]}), z, 0, 0, 0);
                 }
+                if constexpr (ROT > 32) {
+                    // the block of 64 or 128 is Sylvester's matrix of order 2 or 4 over these of order 32: sums and differences
+#pragma unroll
+                    for (int jj = 0; jj < kSide; ++jj) asm volatile("" : "+v"(r[jj]));
+#pragma unroll
+                    for (int st = 1; st < ROT / 32; st *= 2)
+#pragma unroll
+                        for (int jj = 0; jj < kSide; ++jj)
+                            if (!(jj & st)) {
+#pragma unroll
+                                for (int e = 0; e < 16; ++e) {
+                                    const float u = r[jj][e], v = r[jj + st][e];
+                                    r[jj][e] = u + v;
+                                    r[jj + st][e] = u - v;
+                                }
+                            }
+                }
                 const auto emit = [&](auto scaled) {
 #pragma unroll
-                    for (int jj = 0; jj < 2; ++jj) {
-                        asm volatile("" : "+v"(r[jj]));
+                    for (int jj = 0; jj < kSide; ++jj) {
+                        if constexpr (ROT == 32) asm volatile("" : "+v"(r[jj]));
 #pragma unroll
                         for (int b = 0; b < 4; ++b) {
                             float q[4];
@@ -547,20 +569,21 @@ __device__ __forceinline__ void big4_epilogue_bf16(v16f (&acc)[4][4], float alph
                                 *reinterpret_cast<uint4*>(region + lrow * 128 + (((2 * b + half) * 16) ^ wsw)) =
                                     make_uint4(p0 << 16, p0 & 0xffff0000u, p1 << 16, p1 & 0xffff0000u);
                             else
-                                *reinterpret_cast<uint2*>(wr + (((jj * 4 + b) * 16) ^ wsw)) = make_uint2(p0, p1);
+                                *reinterpret_cast<uint2*>(wr + ((((jj & 1) * 4 + b) * 16) ^ wsw)) = make_uint2(p0, p1);
                         }
+                        // the region is private to the wave; LDS operations of one wave complete in order
                         if constexpr (WIDE) {   // N is a multiple of 64: both blocks of the pass are inside
                             __builtin_amdgcn_wave_barrier();
-                            put_rows(i, (2 * jp + jj) * 128);
+                            put_rows(i, (kSide * jp + jj) * 128);
                             __builtin_amdgcn_wave_barrier();
+                        } else if (jj & 1) {
+                            put_rows(i, (kSide * jp + jj) / 2 * 128);
                         }
                     }
                 };
                 if (c_in_matrix) emit(std::false_type{});
                 else emit(std::true_type{});
             }
-            // the region is private to the wave; LDS operations of one wave complete in order
-            if constexpr (!WIDE) put_rows(i, jp * 128);
             // keeps the passes apart: a scheduler that reads many passes' accumulators into vector registers ahead of time
             // pushes the K loop's live values out to scratch memory, and their reloads wait for every operand load in flight
             __builtin_amdgcn_sched_barrier(0);
@@ -606,7 +629,7 @@ enum Big4Result : int { BIG4_PLAIN = 1, BIG4_ROTATED = 2, BIG4_WIDE = 4 };   // 
 // pipeline never drains between tiles and the epilogue runs while the next tile's first four stages arrive.
 // RAGGED: M is not a multiple of 64 (an instantiation of its own: the row tests cost the others 2 to 8 % in registers).
 // PAIR: two products (Big4Other), tiled operands; the sum of the kinds of result that they have.
-template <typename OutT, bool STAMP = false, bool ROT = false, bool RAGGED = false, int PAIR = 0>
+template <typename OutT, bool STAMP = false, int ROT = 0, bool RAGGED = false, int PAIR = 0>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_mxfp4_tn_big4_kernel(
     const uint8_t* __restrict__ a_codes, const uint8_t* __restrict__ a_scales, const uint8_t* __restrict__ b_codes,
     const uint8_t* __restrict__ b_scales, int M, int N, int K, float alpha, OutT* __restrict__ c, int a_tiled,
@@ -844,7 +867,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         stamp();
         if constexpr (PAIR != 0) {
             const auto leave = [&](auto rotated, auto wide) {
-                big4_epilogue_bf16<decltype(rotated)::value, RAGGED, decltype(wide)::value>(acc, alpha, dst, m0, n0, N, wm, wn, wave, lane, smem_bytes,
+                big4_epilogue_bf16<decltype(rotated)::value ? ROT : 0, RAGGED, decltype(wide)::value>(acc, alpha, dst, m0, n0, N, wm, wn, wave, lane, smem_bytes,
                                                                                             rows_valid, cols_valid, turn, keep, keep_shifted);
             };
             if ((PAIR & BIG4_PLAIN) && result == BIG4_PLAIN) {
@@ -967,7 +990,8 @@ const KernelCost& tile_costs(bool e5m2, int kind, int64_t K, int splits) {
     return (e5m2 ? kWideTileCosts : kTileCosts)[kind];
 }
 int last_tile_kind(bool e5m2) { return e5m2 ? TILE_64x64 : TILE_64x32; }
-constexpr double kLaunch = 3.0, kPersistentStep = 0.675, kPersistentBoundary = 5.5, kPersistentMuted = 1.6, kPersistentRotate = 3.9;
+constexpr double kLaunch = 3.0, kPersistentStep = 0.675, kPersistentBoundary = 5.5, kPersistentMuted = 1.6;
+double persistent_rotate_cost(int hd) { return hd == 32 ? 3.9 : hd == 64 ? 4.5 : 5.0; }
 constexpr double kMemory = 5.5e6, kRotateMemory = 5.2e6, kWideStores = 1.0e7;   // bytes per us of the reduction, of a rotation pass of its own, of what fp32 results add
 
 double ranges_cost(int64_t M, int64_t N, int splits) {   // writing, reading and reducing the partial sums of a cut product
@@ -1013,6 +1037,14 @@ bool persistent_serves(int64_t M, int64_t N, int64_t K, const void* a_scales, co
     return (reinterpret_cast<uintptr_t>(c) & 15) == 0;
 }
 
+// The rotation in the persistent kernel's epilogue: column signs that are the same in every 32 of a block of 64 or 128 (none, in a
+// layer whose forward quantizers are not re-randomized)
+bool persistent_rotates(const TileProduct& p) {
+    for (int j = 1; j < p.hd / 32; ++j)
+        if (p.signs.w[j] != p.signs.w[0]) return false;
+    return p.N % p.hd == 0;
+}
+
 // The cheapest cut of a product into K ranges (splits == 1: none is possible): each range keeps at least four K steps, on the
 // persistent kernel whole blocks of four steps and at least two of them.  Few tiles and a long K leave CUs idle: 640 x 1728 x
 // 16512 took 49 us whole and 32 us in three ranges of 128 x 128 tiles, 1536 x 4096 x 16384 110 us and 71 us in two ranges.
@@ -1039,7 +1071,7 @@ Cut cheapest_cut(int64_t M, int64_t N, int64_t K, bool persistent, bool tiles_ok
 // item, where the tile boundary is a third or more of a tile; longer ones neither gain nor lose (within 0.7 %)
 int big4_late_start(int64_t K, int splits) { return K / kBK / splits <= 16 ? 6 : 0; }
 
-template <typename OutT, bool ROT, bool RAGGED>
+template <typename OutT, int ROT, bool RAGGED>
 hipError_t launch_big4_as(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
                           const uint8_t* b_scales, int64_t M, int64_t N, int64_t K, float alpha, void* c, int a_tiled,
                           int b_tiled, int splits, int cus, hipStream_t stream, const RotEpilogue& rot) {
@@ -1057,7 +1089,7 @@ hipError_t launch_big4_as(const uint8_t* a_codes, const uint8_t* a_scales, const
                                                   reinterpret_cast<OutT*>(c), a_tiled, b_tiled, splits, big4_late_start(K, splits), nullptr, rot, Big4NoOther{});
     return hipGetLastError();
 }
-template <typename OutT, bool ROT = false>
+template <typename OutT, int ROT = 0>
 hipError_t launch_big4(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
                        const uint8_t* b_scales, int64_t M, int64_t N, int64_t K, float alpha, void* c, int a_tiled,
                        int b_tiled, int splits, int cus, hipStream_t stream, const RotEpilogue& rot = RotEpilogue{}) {
@@ -1104,7 +1136,7 @@ hipError_t gemm_tile_phases(const uint8_t* a_codes, const uint8_t* a_scales, con
     if (!gemm_supports_tiled(M, N, K) || K % 512 || ((reinterpret_cast<uintptr_t>(a_scales) | reinterpret_cast<uintptr_t>(b_scales)) & 15))
         return hipErrorInvalidValue;
     // rot_mask: the instantiation whose epilogue carries the masked inverse rotation (no sign flips, bf16 scale)
-    auto kern = rot_mask ? gemm_mxfp4_tn_big4_kernel<uint16_t, true, true> : gemm_mxfp4_tn_big4_kernel<uint16_t, true, false>;
+    auto kern = rot_mask ? gemm_mxfp4_tn_big4_kernel<uint16_t, true, 32> : gemm_mxfp4_tn_big4_kernel<uint16_t, true, 0>;
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kBig4SmemBytes);
     if (e != hipSuccess) return e;
     const int64_t items = ((M + kBigM - 1) / kBigM) * ((N + kBigN - 1) / kBigN);
@@ -1224,7 +1256,7 @@ ProductChoice choose_product(const TileProduct& p, int c_dtype, int rot_out_dtyp
     const bool bf16 = c_dtype == BF16;
     const int cus = device_cus();
     if (persistent) {
-        if (rotate && bf16 && rot_out_dtype == BF16 && p.hd == 32) consider({ProductChoice::PERSISTENT, 0, 1, true}, plan.persistent + kPersistentRotate);
+        if (rotate && bf16 && rot_out_dtype == BF16 && persistent_rotates(p)) consider({ProductChoice::PERSISTENT, 0, 1, true}, plan.persistent + persistent_rotate_cost(p.hd));
         consider({ProductChoice::PERSISTENT, 0, 1, false}, plan.persistent + separate);
     }
     for (int kind = TILE_256x128; tiles_ok && kind <= last_tile_kind(e5m2); ++kind) {
@@ -1275,9 +1307,13 @@ hipError_t run_product(const ProductChoice& c, const TileProduct& p, int c_dtype
         q.out_f32 = c_dtype == BF16 && rot_out_dtype == F32;
         return gemm_tile(c.kind, q, c_dtype, stream);
     }
-    if (c.rotates)
-        return launch_big4<uint16_t, true>(p.a_codes, p.a_scales, p.b_codes, p.b_scales, M, N, K, p.alpha, p.c, p.a_tiled, p.b_tiled, 1, cus, stream,
-                                           RotEpilogue{p.mask, p.signs.w[0], p.rot_c});
+    if (c.rotates) {
+        const auto rotated = [&](auto hd) {
+            return launch_big4<uint16_t, decltype(hd)::value>(p.a_codes, p.a_scales, p.b_codes, p.b_scales, M, N, K, p.alpha, p.c, p.a_tiled, p.b_tiled, 1, cus, stream,
+                                                              RotEpilogue{p.mask, p.signs.w[0], p.rot_c});
+        };
+        return p.hd == 32 ? rotated(std::integral_constant<int, 32>{}) : p.hd == 64 ? rotated(std::integral_constant<int, 64>{}) : rotated(std::integral_constant<int, 128>{});
+    }
     if (c_dtype == BF16)
         return launch_big4<uint16_t>(p.a_codes, p.a_scales, p.b_codes, p.b_scales, M, N, K, p.alpha, p.c, p.a_tiled, p.b_tiled, 1, cus, stream);
     return launch_big4<float>(p.a_codes, p.a_scales, p.b_codes, p.b_scales, M, N, K, p.alpha, p.c, p.a_tiled, p.b_tiled, 1, cus, stream);
@@ -1304,9 +1340,9 @@ double pair_makespan(const TileProduct& lng, const TileProduct& sht, int cus, in
     }
     return best;
 }
-template <int PAIR, bool RAGGED>
+template <int PAIR, int ROT, bool RAGGED>
 hipError_t launch_pair_as(const TileProduct& lng, const Big4Other& other, const RotEpilogue& rot, int late, int grid, hipStream_t stream) {
-    auto kern = gemm_mxfp4_tn_big4_kernel<uint16_t, false, true, RAGGED, PAIR>;
+    auto kern = gemm_mxfp4_tn_big4_kernel<uint16_t, false, ROT, RAGGED, PAIR>;
     static std::atomic<bool> lds_allowed[kMaxDevices];
     const hipError_t e = allow_dynamic_lds(kern, kBig4SmemBytes, lds_allowed);
     if (e != hipSuccess) return e;
@@ -1317,8 +1353,8 @@ hipError_t launch_pair_as(const TileProduct& lng, const Big4Other& other, const 
 }  // namespace
 
 // Served: both products by the persistent kernel, tiled, with at least one tile per CU between them (fewer leave CUs idle, which
-// smaller tiles and K ranges do not); bf16 results, plain or with the rotation over blocks of 32, one of them with it, and only
-// rotated ones widened.  Worth it where the estimate of the one launch is clearly below the sum of the two products' own.  Timed
+// smaller tiles and K ranges do not); bf16 results, plain or with the rotation (both over the same block; beside a
+// plain one over 32), one of them with it, and only rotated ones widened.  Worth it where the estimate of the one launch is clearly below the sum of the two products' own.  Timed
 // against two launches, whole training steps: 52 shapes from 0.62 to 0.94 of that sum are 0.99 to 1.19 times as fast (mean 1.05; 4096 x
 // 2048 x 4096 116 us, now 104; 16384 x 1536 x 4608 behind its norm 471 -> 453; 16384 x 4096 x 1536 behind SwiGLU 457 -> 431; 8192 x 4096^2
 // 291 -> 287), what is gained being the idle part of each product's last round, or writing and reading partial sums; none lies
@@ -1327,14 +1363,16 @@ constexpr double kPairMargin = 0.95;
 bool pair_pays(const TileProduct& x, const ProductChoice& cx, int x_out, const TileProduct& w, const ProductChoice& cw, int w_out, int c_dtype) {
     if (c_dtype != BF16 || x.N != w.N || x.alpha != w.alpha || x.b_e5m2 || w.b_e5m2) return false;
     const auto serves = [](const TileProduct& p, int out) {
-        return p.a_tiled && p.b_tiled && (p.mask ? p.hd == 32 : out == BF16) && persistent_serves(p.M, p.N, p.K, p.a_scales, p.b_scales, p.c);
+        return p.a_tiled && p.b_tiled && (p.mask ? persistent_rotates(p) : out == BF16) && persistent_serves(p.M, p.N, p.K, p.a_scales, p.b_scales, p.c);
     };
     if (!serves(x, x_out) || !serves(w, w_out) || (!x.mask && !w.mask)) return false;
+    const int hd = x.mask ? x.hd : w.hd;
+    if (x.mask && w.mask ? x.hd != w.hd : hd != 32) return false;
     const int cus = device_cus();
     if (cus < 8 || big_tiles(x) + big_tiles(w) < cus) return false;
     int rounds;
     const bool x_long = x.K > w.K;
-    double cost = kLaunch + pair_makespan(x_long ? x : w, x_long ? w : x, cus, &rounds) + kPersistentRotate;
+    double cost = kLaunch + pair_makespan(x_long ? x : w, x_long ? w : x, cus, &rounds) + persistent_rotate_cost(hd);
     if (x.mask && x_out != BF16) cost += (double)x.M * x.N * 2 / kWideStores;
     if (w.mask && w_out != BF16) cost += (double)w.M * w.N * 2 / kWideStores;
     return cost < kPairMargin * (cx.cost + cw.cost);
@@ -1350,9 +1388,17 @@ hipError_t run_pair(const TileProduct& x, int x_out, const TileProduct& w, int w
                 kind(sht, x_long ? w_out : x_out), kind(lng, x_long ? x_out : w_out)};
     pair_makespan(lng, sht, cus, &o.rounds);
     const int late = big4_late_start(sht.K, 1), grid = pair_grid(big_tiles(x) + big_tiles(w), cus);
+    const auto go_rotated = [&](auto pair, auto hd) {
+        constexpr int P = decltype(pair)::value, R = decltype(hd)::value;
+        return x.M % 64 || w.M % 64 ? launch_pair_as<P, R, true>(lng, o, rot(lng), late, grid, stream) : launch_pair_as<P, R, false>(lng, o, rot(lng), late, grid, stream);
+    };
+    const int hd = x.mask ? x.hd : w.hd;
     const auto go = [&](auto pair) {
-        constexpr int P = decltype(pair)::value;
-        return x.M % 64 || w.M % 64 ? launch_pair_as<P, true>(lng, o, rot(lng), late, grid, stream) : launch_pair_as<P, false>(lng, o, rot(lng), late, grid, stream);
+        if constexpr ((decltype(pair)::value & BIG4_PLAIN) == 0) {   // a plain one comes with blocks of 32
+            if (hd == 64) return go_rotated(pair, std::integral_constant<int, 64>{});
+            if (hd == 128) return go_rotated(pair, std::integral_constant<int, 128>{});
+        }
+        return go_rotated(pair, std::integral_constant<int, 32>{});
     };
     switch (o.kind | o.long_kind) {
         case BIG4_ROTATED: return go(std::integral_constant<int, BIG4_ROTATED>{});
