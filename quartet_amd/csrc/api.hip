@@ -445,8 +445,9 @@ GradProduct plan_gradient(const qm::TileProduct& plain, void* final_dst, bool wa
     if (!want_rotation) g.whole_choice = g.choice;
     return g;
 }
-bool one_launch(const GradProduct& x, const GradProduct& w, int mid_dtype) {
-    return x.whole_dtype >= 0 && w.whole_dtype >= 0 && qm::pair_pays(x.whole, x.whole_choice, x.whole_dtype, w.whole, w.whole_choice, w.whole_dtype, mid_dtype);
+qm::PairChoice plan_pair(const GradProduct& x, const GradProduct& w, int mid_dtype) {
+    if (x.whole_dtype < 0 || w.whole_dtype < 0) return {qm::PairChoice::SEPARATE, 0, 0};
+    return qm::choose_pair(x.whole, x.whole_choice, x.whole_dtype, w.whole, w.whole_choice, w.whole_dtype, mid_dtype);
 }
 }
 }  // namespace
@@ -480,7 +481,7 @@ int qm_linear_backward_in_one_launch(int64_t T, int64_t I, int64_t O, int hd_x, 
         return plan_gradient(qm::make_product(at, at, at, at, M, I, qm::padded_cols(K), 1.0f, at, QM_LAYOUT_TILED, QM_LAYOUT_TILED), at, rotate, hd, QM_BF16, out, at,
                              nullptr, QM_BF16, ws ? at : nullptr, ws);
     };
-    return one_launch(plan(T, O, !(rotated_flags & QM_GX_ROTATED), hd_x, QM_BF16), plan(O, T, !(rotated_flags & QM_GW_ROTATED), hd_w, gw_dtype), QM_BF16) ? 1 : 0;
+    return (int)plan_pair(plan(T, O, !(rotated_flags & QM_GX_ROTATED), hd_x, QM_BF16), plan(O, T, !(rotated_flags & QM_GW_ROTATED), hd_w, gw_dtype), QM_BF16).path;
 }
 
 int qm_linear_forward(const void* x, int x_dtype, const void* w, int w_dtype, int64_t T, int64_t I, int64_t O, int hd_x,
@@ -749,8 +750,8 @@ int qm_linear_backward_seeded(const void* e, int e_dtype, int64_t T, int64_t I, 
         const qm::ErrorArgs ae{e, e_dtype, T, O, seeds[0], seeds[2], k + wl.ec, k + wl.es, k + wl.etc, k + wl.ets};
         rc = from_hip(qm::quantize_layer_backward(ae, hd_g, make_signs(signs_g, hd_g), g_mode, rx, rw, seed_base, hs), "qm_linear_backward");
         if (rc) return rc;
-        if (one_launch(gx_plan, gw_plan, mid_dtype))
-            return from_hip(qm::run_pair(gx_plan.whole, gx_plan.whole_dtype, gw_plan.whole, gw_plan.whole_dtype, hs), "qm_linear_backward");
+        if (const qm::PairChoice pair = plan_pair(gx_plan, gw_plan, mid_dtype); pair.path != qm::PairChoice::SEPARATE)
+            return from_hip(qm::run_pair(pair, gx_plan.whole, gx_plan.whole_dtype, gw_plan.whole, gw_plan.whole_dtype, hs), "qm_linear_backward");
         rc = product_gx();
         if (rc) return rc;
         rc = product_gw();

@@ -1358,27 +1358,79 @@ hipError_t launch_pair_as(const TileProduct& lng, const Big4Other& other, const 
 // against two launches, whole training steps: 52 shapes from 0.62 to 0.94 of that sum are 0.99 to 1.19 times as fast (mean 1.05; 4096 x
 // 2048 x 4096 116 us, now 104; 16384 x 1536 x 4608 behind its norm 471 -> 453; 16384 x 4096 x 1536 behind SwiGLU 457 -> 431; 8192 x 4096^2
 // 291 -> 287), what is gained being the idle part of each product's last round, or writing and reading partial sums; none lies
-// between 0.94 and 1, where the estimates (6 % off on average) no longer tell.
-constexpr double kPairMargin = 0.95;
-bool pair_pays(const TileProduct& x, const ProductChoice& cx, int x_out, const TileProduct& w, const ProductChoice& cw, int w_out, int c_dtype) {
-    if (c_dtype != BF16 || x.N != w.N || x.alpha != w.alpha || x.b_e5m2 || w.b_e5m2) return false;
+// between 0.94 and 1, near which the estimates (6 % off on average) no longer tell.
+constexpr double kPairMargin = 0.97;
+double persistent_pair_cost(const TileProduct& x, int x_out, const TileProduct& w, int w_out, int cus) {
     const auto serves = [](const TileProduct& p, int out) {
         return p.a_tiled && p.b_tiled && (p.mask ? persistent_rotates(p) : out == BF16) && persistent_serves(p.M, p.N, p.K, p.a_scales, p.b_scales, p.c);
     };
-    if (!serves(x, x_out) || !serves(w, w_out) || (!x.mask && !w.mask)) return false;
+    if (!serves(x, x_out) || !serves(w, w_out)) return 1e30;
     const int hd = x.mask ? x.hd : w.hd;
-    if (x.mask && w.mask ? x.hd != w.hd : hd != 32) return false;
-    const int cus = device_cus();
-    if (cus < 8 || big_tiles(x) + big_tiles(w) < cus) return false;
+    if (x.mask && w.mask ? x.hd != w.hd : hd != 32) return 1e30;
+    if (cus < 8 || big_tiles(x) + big_tiles(w) < cus) return 1e30;
     int rounds;
     const bool x_long = x.K > w.K;
     double cost = kLaunch + pair_makespan(x_long ? x : w, x_long ? w : x, cus, &rounds) + persistent_rotate_cost(hd);
     if (x.mask && x_out != BF16) cost += (double)x.M * x.N * 2 / kWideStores;
     if (w.mask && w_out != BF16) cost += (double)w.M * w.N * 2 / kWideStores;
-    return cost < kPairMargin * (cx.cost + cw.cost);
+    return cost;
 }
-hipError_t run_pair(const TileProduct& x, int x_out, const TileProduct& w, int w_out, hipStream_t stream) {
+// What a tile costs its CU among others of a pair, in us: a K step, the boundary, the rotation; and a K step of a tile whose CU has
+// others beside it, and when they are done; its half of the launch, first fill and drain.  Fitted to 20 shapes from 512 x 640 x 1920 to 32768 x 1536 x 1536.
+struct PairTile {
+    int kind, bm;   // as many columns as rows
+    double step, boundary, rotate, beside, after, launch;
+};
+constexpr PairTile kPairTiles[] = {{TILE_128x128, 128, 0.26, 0.99, 0.63, 0.37, 0.25, 3.5}, {TILE_64x64, 64, 0.129, 0.36, 0.19, 0.30, 0.14, 2.0}};
+constexpr double kTilePairMargin = 0.9;   // on 60 other shapes: at worst 0.995 times as fast, GPU time of the backward pass 0.92 of two launches' on average
+// Tiles go to the CUs as they become free, the longer contraction's first: every CU its share of those, then the others to even it
+// out.  A tile of very many steps is still running when the others are done.
+double tile_pair_cost(const TileProduct& x, int x_out, const PairTile& kx, const TileProduct& w, int w_out, const PairTile& kw, int cus) {
+    const auto tiles = [](const TileProduct& p, const PairTile& k) { return (int64_t)((p.M + k.bm - 1) / k.bm) * ((p.N + k.bm - 1) / k.bm); };
+    const auto tile = [](const TileProduct& p, const PairTile& k) { return p.K / kBK * k.step + k.boundary + (p.mask ? k.rotate : 0.0); };
     const bool x_long = x.K > w.K;
+    const TileProduct &lng = x_long ? x : w, &sht = x_long ? w : x;
+    const PairTile &kl = x_long ? kx : kw, &ks = x_long ? kw : kx;
+    const int64_t tl = tiles(lng, kl), ts = tiles(sht, ks);
+    const double cl = tile(lng, kl), cs = tile(sht, ks), mean = (tl * cl + ts * cs) / cus;
+    const double most_long = (double)((tl + cus - 1) / cus) * cl;
+    // the CUs with most of the long ones, and whole short ones up to the mean on the others
+    const double even = mean + (ts > 0 ? 0.5 * cs : 0.0);
+    double all = most_long > even ? most_long : even;
+    if (tl % cus == 0) all = (double)(tl / cus) * cl + (double)((ts + cus - 1) / cus) * cs;
+    const double left = lng.K / kBK - all / kl.beside;
+    double cost = kx.launch + kw.launch + all + (left > 0.0 ? left * kl.after : 0.0);
+    if (x.mask && x_out != BF16) cost += (double)x.M * x.N * 2 / kWideStores;
+    if (w.mask && w_out != BF16) cost += (double)w.M * w.N * 2 / kWideStores;
+    return cost;
+}
+PairChoice choose_pair(const TileProduct& x, const ProductChoice& cx, int x_out, const TileProduct& w, const ProductChoice& cw, int w_out, int c_dtype) {
+    PairChoice best{PairChoice::SEPARATE, 0, 0};
+    if (c_dtype != BF16 || x.N != w.N || x.alpha != w.alpha || x.b_e5m2 || w.b_e5m2 || (!x.mask && !w.mask)) return best;
+    const int cus = device_cus();
+    const double apart = cx.cost + cw.cost, one = persistent_pair_cost(x, x_out, w, w_out, cus);
+    double cost = 1e30;
+    if (one < kPairMargin * apart) {
+        cost = 1.1 * one;   // it is the more hopeful one of the two estimates
+        best = {PairChoice::PERSISTENT, 0, 0};
+    }
+    for (const PairTile& kx : kPairTiles)
+        for (const PairTile& kw : kPairTiles)
+            if (x.K > w.K ? gemm_tile_pair_serves(x, kx.kind, w, kw.kind) : gemm_tile_pair_serves(w, kw.kind, x, kx.kind)) {
+                const double c = tile_pair_cost(x, x_out, kx, w, w_out, kw, cus);
+                if (c < kTilePairMargin * apart && c < cost) {
+                    cost = c;
+                    best = {PairChoice::TILE, kx.kind, kw.kind};
+                }
+            }
+    return best;
+}
+hipError_t run_pair(const PairChoice& c, const TileProduct& x, int x_out, const TileProduct& w, int w_out, hipStream_t stream) {
+    const bool x_long = x.K > w.K;
+    if (c.path == PairChoice::TILE)
+        return x_long ? gemm_tile_pair(x, c.kind_x, x_out != BF16, w, c.kind_w, w_out != BF16, stream)
+                      : gemm_tile_pair(w, c.kind_w, w_out != BF16, x, c.kind_x, x_out != BF16, stream);
+    if (c.path != PairChoice::PERSISTENT) return hipErrorInvalidValue;
     const TileProduct &lng = x_long ? x : w, &sht = x_long ? w : x;
     const int cus = device_cus();
     const auto kind = [](const TileProduct& p, int out) { return !p.mask ? BIG4_PLAIN : out == BF16 ? BIG4_ROTATED : BIG4_WIDE; };

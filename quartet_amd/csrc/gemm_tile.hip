@@ -733,6 +733,36 @@ hipError_t launch_tiles(const TileProduct& g, hipStream_t stream) {
     return hipGetLastError();
 }
 
+// Both gradient products of a layer in one grid, A's tiles first (the longer contraction's: they are on their way while B's pass
+// through the chip).  Launched one after the other, each product ends in tiles that leave most of the chip idle, and a weight gradient
+// of few tiles and many tokens is cut into K ranges whose partial sums travel through memory; here its whole tiles run beside the
+// input gradient's.  us of a layer's backward pass on the GPU, two launches against one: 512 x 640 x 1920 25 -> 21, 2048^3 44 -> 37, 1824 x
+// 2048 x 1408 39 -> 34, 16480 x 1728 x 640 (64 x 64 tiles of the weight gradient) 93 -> 87, 16384 x 1536 x 1536 124 -> 106, 13312 x 8704 x 640
+// 220 -> 195.  What bounds it: as each product by itself, and for the last tiles of a long contraction its serial chain (0.25 us a step).
+// Workgroups are dealt out by the hardware as CUs become free, which evens the two out.  B's tiles begin at a multiple of eight, so that both keep their runs of tiles to an XCD (xcd_run).
+template <class SA, bool ROT_A, class SB, bool ROT_B>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SA::OCC < SB::OCC ? SA::OCC : SB::OCC))) void gemm_mxfp4_tn_pair_kernel(
+    TileProduct a, TileProduct b, int tiles_a, int tiles_b) {
+    static_assert(SA::kThreads == 256 && SB::kThreads == 256, "one size of workgroup");
+    extern __shared__ uint32_t smem[];
+    const uint32_t smem_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint32_t*)smem;
+    const int t = (int)blockIdx.x, first_b = (tiles_a + 7) & ~7;
+    if (t < tiles_a) tile_run<SA, uint16_t, ROT_A>(a, t, smem, smem_base);
+    else if (t >= first_b && t - first_b < tiles_b) tile_run<SB, uint16_t, ROT_B>(b, t - first_b, smem, smem_base);
+}
+template <class SA, bool ROT_A, class SB, bool ROT_B>
+hipError_t launch_pair(const TileProduct& a, const TileProduct& b, hipStream_t stream) {
+    const auto kern = gemm_mxfp4_tn_pair_kernel<SA, ROT_A, SB, ROT_B>;
+    constexpr int kLds = SA::kSmemBytes > SB::kSmemBytes ? SA::kSmemBytes : SB::kSmemBytes;
+    static std::atomic<bool> lds_allowed[kMaxDevices];
+    const hipError_t e = allow_dynamic_lds(kern, kLds, lds_allowed);
+    if (e != hipSuccess) return e;
+    const auto tiles = [](const TileProduct& g, int bm, int bn) { return ((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); };
+    const int ta = tiles(a, SA::BM, SA::BN), tb = tiles(b, SB::BM, SB::BN);
+    kern<<<dim3((unsigned)(((ta + 7) & ~7) + tb)), dim3(256), kLds, stream>>>(a, b, ta, tb);
+    return hipGetLastError();
+}
+
 using Tile256x128 = TileShape<256, 128, 128, 64, 3, 2>;
 using Tile128x128 = TileShape<128, 128, 64, 64, 3, 3>;
 using Tile128x64 = TileShape<128, 64, 64, 32, 4, 3>;
@@ -751,6 +781,30 @@ bool gemm_tile_serves(int64_t M, int64_t N, int64_t K, int a_tiled, int b_tiled,
     const bool k_ok = K % kBK == 0 || (K % kBK == 64 && K >= 192 && !a_tiled && !b_tiled);
     return M > 0 && N >= 8 && N % 8 == 0 && K > 0 && k_ok && M < (1 << 30) && N < (1 << 30) && K < (1 << 23) &&
            (reinterpret_cast<uintptr_t>(c) & 15) == 0;
+}
+
+// a: the longer contraction; tiles of 128 x 128 or 64 x 64 either; scales in blocks (see gemm_tile), at least one of them rotated
+bool gemm_tile_pair_serves(const TileProduct& a, int shape_a, const TileProduct& b, int shape_b) {
+    const auto serves = [](const TileProduct& g, int shape) {
+        return (shape == TILE_128x128 || shape == TILE_64x64) && !g.b_e5m2 && gemm_tile_serves(g.M, g.N, g.K, g.a_tiled, g.b_tiled, g.c) && g.K % kBK == 0 &&
+               g.K / kBK >= 4 && ((reinterpret_cast<uintptr_t>(g.a_scales) | reinterpret_cast<uintptr_t>(g.b_scales)) & 3) == 0 &&
+               (!g.mask || (g.hd <= (shape == TILE_64x64 ? 64 : 128) && g.N % g.hd == 0));
+    };
+    return (a.mask || b.mask) && serves(a, shape_a) && serves(b, shape_b);
+}
+hipError_t gemm_tile_pair(TileProduct a, int shape_a, bool a_f32, TileProduct b, int shape_b, bool b_f32, hipStream_t stream) {
+    if (!gemm_tile_pair_serves(a, shape_a, b, shape_b)) return hipErrorInvalidValue;
+    a.splits = b.splits = 1;
+    a.out_f32 = a_f32;
+    b.out_f32 = b_f32;
+    const auto rotations = [&](auto sa, auto sb) {
+        using SA = decltype(sa);
+        using SB = decltype(sb);
+        if (!a.mask) return launch_pair<SA, false, SB, true>(a, b, stream);
+        return b.mask ? launch_pair<SA, true, SB, true>(a, b, stream) : launch_pair<SA, true, SB, false>(a, b, stream);
+    };
+    if (shape_a == TILE_64x64) return shape_b == TILE_64x64 ? rotations(Tile64x64{}, Tile64x64{}) : rotations(Tile64x64{}, Tile128x128{});
+    return shape_b == TILE_64x64 ? rotations(Tile128x128{}, Tile64x64{}) : rotations(Tile128x128{}, Tile128x128{});
 }
 
 hipError_t gemm_tile(int shape, const TileProduct& g, int c_dtype, hipStream_t stream) {

@@ -214,6 +214,9 @@ constexpr int kShortTallSteps = 8;   // see gemm_tile()
 enum TileKind : int { TILE_256x128 = 0, WIDE_256x256 = 0, TILE_128x128 = 1, TILE_128x64 = 2, TILE_64x64 = 3, TILE_64x32 = 4 };
 bool gemm_tile_serves(int64_t M, int64_t N, int64_t K, int a_tiled, int b_tiled, const void* c);
 hipError_t gemm_tile(int kind, const TileProduct& g, int c_dtype, hipStream_t stream);
+// two products (bf16 results, or with a mask and *_f32 widened ones) in one grid; TileKinds 128x128 and 64x64
+bool gemm_tile_pair_serves(const TileProduct& a, int kind_a, const TileProduct& b, int kind_b);
+hipError_t gemm_tile_pair(TileProduct a, int kind_a, bool a_f32, TileProduct b, int kind_b, bool b_f32, hipStream_t stream);
 
 // The product of at most 64 rows with a weight, both tiled (gemm_rows.hip): K % 128 == 0, N % 8 == 0, c 16-byte aligned, no mask.
 // Its sums are in another order than the other kernels'.
@@ -240,10 +243,14 @@ TileProduct make_product(const uint8_t* a_codes, const uint8_t* a_scales, const 
                          int64_t K, float alpha, void* c, int a_layout, int b_layout);
 ProductChoice choose_product(const TileProduct& p, int c_dtype, int rot_out_dtype, const void* workspace, size_t workspace_bytes);
 hipError_t run_product(const ProductChoice& c, const TileProduct& p, int c_dtype, int rot_out_dtype, void* workspace, hipStream_t stream);
-// The gradient products x and w of a layer in one launch of the persistent kernel: whether it serves them and is expected to be
-// faster than running them as cx and cw say; p.mask and *_out as in choose_product.  The results are those of the persistent kernel.
-bool pair_pays(const TileProduct& x, const ProductChoice& cx, int x_out, const TileProduct& w, const ProductChoice& cw, int w_out, int c_dtype);
-hipError_t run_pair(const TileProduct& x, int x_out, const TileProduct& w, int w_out, hipStream_t stream);
+// The gradient products x and w of a layer in one launch: of which kernel, if that is expected to be faster than running them as cx
+// and cw say; p.mask and *_out as in choose_product.  The results are those of the kernel without K ranges.
+struct PairChoice {
+    enum Path : int { SEPARATE = 0, PERSISTENT = 1, TILE = 2 } path;
+    int kind_x, kind_w;   // TileKinds
+};
+PairChoice choose_pair(const TileProduct& x, const ProductChoice& cx, int x_out, const TileProduct& w, const ProductChoice& cw, int w_out, int c_dtype);
+hipError_t run_pair(const PairChoice& c, const TileProduct& x, int x_out, const TileProduct& w, int w_out, hipStream_t stream);
 // the rotation in the persistent kernel's bf16 epilogue (Hadamard block 32)
 bool gemm_persistent_rotates(const uint8_t* a_scales, const uint8_t* b_scales, int64_t M, int64_t N, int64_t K);
 hipError_t gemm_persistent_rotated(TileProduct p, hipStream_t stream);

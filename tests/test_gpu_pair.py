@@ -2,6 +2,7 @@
 import pytest
 import torch
 
+from tests.test_kernel_resources import kernels  # noqa: F401  (a fixture)
 from tests.util import make_input
 
 pytestmark = pytest.mark.gpu
@@ -12,31 +13,46 @@ ALPHA = float(torch.tensor(4.0 / 3.0, dtype=torch.float32) ** 2)
 
 # K steps in whole blocks of four and not (muted ones), either product the long one, as many K steps; tiles over the edges of M and N by
 # multiples of 64 and 32 rows; numbers of tiles that the XCDs and their workgroups share evenly and not, fewer long tiles than workgroups
-@pytest.mark.parametrize("T,I,O", [(4096, 2048, 4096), (5888, 4800, 1536), (4128, 4096, 4128), (1696, 2816, 7680), (6624, 4608, 1024), (3456, 3712, 1280),
-                                   (2112, 3392, 4896)])
+@pytest.mark.parametrize("T,I,O", [(4096, 2048, 4096), (5888, 4800, 1536), (3168, 1984, 4800), (2944, 5440, 2080), (2016, 5312, 4096), (6144, 3072, 3072)])
 @pytest.mark.parametrize("gx_rotated,gw_dtype", [(False, torch.bfloat16), (False, torch.float32), (True, torch.bfloat16), (True, torch.float32)])
 def test_gradients_in_one_launch(monkeypatch, T, I, O, gx_rotated, gw_dtype):
-    check_gradients(monkeypatch, T, I, O, 32, gx_rotated, gw_dtype, True, 0x5A5A5A5A, 0x0F0F1234)
+    check_gradients(monkeypatch, T, I, O, 32, gx_rotated, gw_dtype, 1, 0x5A5A5A5A, 0x0F0F1234)
 
 
-# blocks of 64 and 128 in the epilogue of one launch and of two (16384 x 2048 x 2048: the input gradient by itself, the weight gradient
-# cut), with column signs that repeat every 32 and with others, which that epilogue does not take
-@pytest.mark.parametrize("T,I,O,hd,paired", [(4096, 2048, 4096, 128, True), (4160, 2112, 4096, 64, True), (2048, 4096, 4224, 128, True), (16384, 2048, 2048, 64, False)])
+# blocks of 64 and 128 in the epilogue of one launch and (14464 x 576 x 1024) of two, with column signs that repeat every 32 and with others, which that epilogue does not take
+@pytest.mark.parametrize("T,I,O,hd,path", [(2560, 2560, 5248, 128, 1), (2560, 3584, 5728, 128, 1), (1216, 4608, 4352, 64, 1), (3168, 1984, 4800, 64, 1), (14464, 576, 1024, 64, 0)])
 @pytest.mark.parametrize("gw_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("repeat", [True, False])
-def test_wider_blocks(monkeypatch, T, I, O, hd, paired, gw_dtype, repeat):
+def test_wider_blocks(monkeypatch, T, I, O, hd, path, gw_dtype, repeat):
+    if not repeat and path == 1:   # the smaller tiles', or two launches
+        path = None
     signs = [sum((s if repeat else s * 3 ** j & 0xFFFFFFFF) << 32 * j for j in range(hd // 32)) for s in (0x5A5A5A5A, 0x0F0F1234)]
-    check_gradients(monkeypatch, T, I, O, hd, False, gw_dtype, paired, *signs)
+    check_gradients(monkeypatch, T, I, O, hd, False, gw_dtype, path, *signs)
 
 
-def check_gradients(monkeypatch, T, I, O, hd, gx_rotated, gw_dtype, paired, sx, sw):
+# the smaller tiles: either product the long one, four K steps and many, 128 x 128 and 64 x 64 of either product (paths as chosen now),
+# ragged rows and columns, as many tiles as there are CUs and a handful; Hadamard blocks of every width
+@pytest.mark.parametrize("T,I,O,hd", [(512, 640, 1920, 32), (1792, 1152, 2560, 32), (640, 4096, 8192, 32), (1888, 1664, 3584, 32), (4128, 1088, 4128, 32), (1024, 1056, 1536, 32),
+                                      (8192, 512, 2048, 64), (2304, 1408, 2048, 64), (2304, 768, 3200, 128), (480, 2048, 8832, 32), (9216, 512, 9216, 32)])
+@pytest.mark.parametrize("gw_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("gx_rotated", [False, True])
+def test_gradients_in_one_launch_of_small_tiles(monkeypatch, T, I, O, hd, gx_rotated, gw_dtype):
+    if gx_rotated and hd != 32:
+        pytest.skip("rotated gradients are those of blocks of 32")
+    signs = [sum((s * 3 ** j & 0xFFFFFFFF) << 32 * j for j in range(hd // 32)) for s in (0x5A5A5A5A, 0x0F0F1234)]
+    check_gradients(monkeypatch, T, I, O, hd, gx_rotated, gw_dtype, 2, *signs)
+
+
+def check_gradients(monkeypatch, T, I, O, hd, gx_rotated, gw_dtype, path, sx, sw):
     """Both kernels round the fp32 sums of the same K order to bf16, mask them and rotate them in fp32; the rotation's sums of 32 to 128
     values are in another order than the stand-alone kernel's (2^-24 of a group's norm apart), which turns a bf16 rounding now and
     then: at most one result in 10^4, by one step of 2^-8 of its value or, where a group cancels, 2^-20 of the group.  Without a
-    rotation (gx_rotated) the bits are the same, and so are a wide gradient's and a bf16 one's."""
+    rotation (gx_rotated) the bits are the same, and so are a wide gradient's and a bf16 one's; and all of them on the smaller tiles (path
+    2), whose rotation is the stand-alone kernel's."""
     print(f"case pair {T}x{I}x{O} hd={hd} gx_rotated={gx_rotated} gw={gw_dtype}", flush=True)
     from quartet_amd import _lib, kernels as K
-    assert _lib.lib().qm_linear_backward_in_one_launch(T, I, O, hd, hd, int(gw_dtype == torch.float32), int(gx_rotated)) == paired
+    if path is not None:
+        assert _lib.lib().qm_linear_backward_in_one_launch(T, I, O, hd, hd, int(gw_dtype == torch.float32), int(gx_rotated)) == path
     monkeypatch.setattr(K, "_layout", lambda tiled: QM_LAYOUT_PADDED if tiled == "padded" else K.QM_LAYOUT_TILED if tiled else K.QM_LAYOUT_ROWMAJOR)
     dev, bf16 = "cuda:0", torch.bfloat16
     x = make_input(T, I, bf16, seed=21).to(dev)
@@ -63,6 +79,8 @@ def check_gradients(monkeypatch, T, I, O, hd, gx_rotated, gw_dtype, paired, sx, 
         assert torch.equal(gx, gxq)
     for got, product, signs, mask in [(gw, gwq, sw, wm)] + ([] if gx_rotated else [(gx, gxq, sx, xm)]):
         want = K.masked_hadamard_bwd(product, hd, bf16, signs, mask)
+        if path == 2:
+            assert torch.equal(got.float(), want.float())
         far = (got.float() - want.float()).abs()
         group = product.float().view(-1, hd).norm(dim=1).repeat_interleave(hd).view(want.shape)
         assert int((far > 0).sum()) <= want.numel() * 1e-4
@@ -70,12 +88,19 @@ def check_gradients(monkeypatch, T, I, O, hd, gx_rotated, gw_dtype, paired, sx, 
 
 
 def test_which_gradients_share_a_launch():
-    """Fewer tiles than CUs, other Hadamard blocks, extents that the kernel does not serve: two launches, as before."""
+    """Two launches (0), one of the 256 x 256 kernel (1), one of smaller tiles (2)."""
     from quartet_amd import _lib
     pairs = _lib.lib().qm_linear_backward_in_one_launch
     assert pairs(4096, 2048, 4096, 32, 32, _lib.QM_BF16, 0) == 1
-    assert pairs(9216, 512, 9216, 32, 32, _lib.QM_BF16, 0) == 0      # 144 tiles
-    assert pairs(4096, 2080, 4096, 32, 32, _lib.QM_BF16, 0) == 0     # in_features not a multiple of 64
+    assert pairs(4096, 2080, 4096, 32, 32, _lib.QM_BF16, 0) == 2     # in_features not a multiple of 64
+    assert pairs(1024, 1024, 256, 32, 32, _lib.QM_BF16, 0) == 0      # two K steps
     assert pairs(4096, 2048, 4096, 32, 32, _lib.QM_F32, 3) == 0      # no rotation at all
     assert pairs(0, 2048, 4096, 32, 32, _lib.QM_BF16, 0) == 0 and pairs(4096, 2048, 4100, 32, 32, _lib.QM_BF16, 0) == 0
     assert pairs(4096, 2048, 4096, 48, 32, _lib.QM_BF16, 0) == 0 and pairs(4096, 2048, 4096, 32, 32, 7, 0) == 0
+
+
+def test_pairs_keep_nothing_in_memory(kernels):
+    """No kernel with two products spills: a tile runs 4 to 30 K steps."""
+    pairs = {n: v for n, v in kernels.items() if "pair_kernel<" in n or ("big4_kernel" in n and not n.split("(unsigned char const*")[0].endswith(", 0>"))}
+    assert len(pairs) >= 20
+    assert {n: v for n, v in pairs.items() if v[1]} == {}
