@@ -77,6 +77,14 @@ int qm_quantize_mxfp4(const void* x, int x_dtype, int64_t rows, int64_t cols, in
                       void* dequant, int codes_layout, void* stream);
 
 /*
+ * qm_quantize_mxfp4 where only the values are wanted, as the quantizer modules return them (quantizers/mxfp4.py:17-28,
+ * 129-140): row-major x, in-kernel random numbers, hadamard_dim 32, 64 or 128, no codes and scales.  dequant (required) and
+ * maskbits (or NULL) as there, the same bits.  x and dequant 16-byte, maskbits 4-byte aligned.
+ */
+int qm_pseudo_quantize_mxfp4(const void* x, int x_dtype, int64_t rows, int64_t cols, int hadamard_dim, const uint32_t* sign_bits,
+                             int mode, uint64_t seed, uint8_t* maskbits, void* dequant, void* stream);
+
+/*
  * De-quantize a packed [R, C] tensor, transpose it, rotate and re-quantize along R:
  * outputs codes_out [C, R/2], scales_out [C, R/32].  Replaces
  * `g_quantizer(wq.T.contiguous())` / `g_quantizer(xq.T.contiguous())`

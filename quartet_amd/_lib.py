@@ -49,6 +49,7 @@ EXPORTS = (
     "qm_rope_merge_qkv_grad",
     "qm_linear_decode_serves",
     "qm_linear_backward_in_one_launch",
+    "qm_pseudo_quantize_mxfp4",
     "qm_linear_decode",
     "qm_cross_entropy",
     "qm_diag_silu_bf16",
@@ -134,6 +135,8 @@ def lib():
     L.qm_linear_decode_serves.argtypes = [i64, i64, i64]
     L.qm_linear_backward_in_one_launch.restype = i32
     L.qm_linear_backward_in_one_launch.argtypes = [i64, i64, i64, i32, i32, i32, i32]
+    L.qm_pseudo_quantize_mxfp4.restype = i32
+    L.qm_pseudo_quantize_mxfp4.argtypes = [vp, i32, i64, i64, i32, vp, i32, u64, vp, vp, vp]
     L.qm_linear_decode.restype = i32
     L.qm_linear_decode.argtypes = [vp, i32, i64, i64, i64, vp, vp, ctypes.c_size_t, vp, i32, vp]
     L.qm_cross_entropy.restype = i32

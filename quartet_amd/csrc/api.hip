@@ -81,6 +81,22 @@ int qm_quantize_mxfp4(const void* x, int x_dtype, int64_t rows, int64_t cols, in
                     "qm_quantize_mxfp4");
 }
 
+int qm_pseudo_quantize_mxfp4(const void* x, int x_dtype, int64_t rows, int64_t cols, int hadamard_dim, const uint32_t* sign_bits, int mode,
+                             uint64_t seed, uint8_t* maskbits, void* dequant, void* stream) {
+    if (!valid_dtype(x_dtype)) return fail(QM_ERR_INVALID, "qm_pseudo_quantize_mxfp4: x_dtype %d is not QM_BF16/QM_F32", x_dtype);
+    if (!valid_hd(hadamard_dim)) return fail(QM_ERR_INVALID, "qm_pseudo_quantize_mxfp4: hadamard_dim %d not in {32,64,128}", hadamard_dim);
+    if (!valid_mode(mode)) return fail(QM_ERR_INVALID, "qm_pseudo_quantize_mxfp4: unknown mode %d", mode);
+    if (rows < 0 || cols < 0) return fail(QM_ERR_INVALID, "qm_pseudo_quantize_mxfp4: negative shape [%lld, %lld]", (long long)rows, (long long)cols);
+    if (cols % hadamard_dim) return fail(QM_ERR_INVALID, "qm_pseudo_quantize_mxfp4: cols %lld not a multiple of hadamard_dim %d", (long long)cols, hadamard_dim);
+    if (rows == 0 || cols == 0) return 0;
+    if (!x || !dequant) return fail(QM_ERR_INVALID, "qm_pseudo_quantize_mxfp4: x and dequant must be non-null");
+    if (!aligned(x, 16) || !aligned(dequant, 16) || !aligned(maskbits, 4))
+        return fail(QM_ERR_UNALIGNED, "qm_pseudo_quantize_mxfp4: x and dequant need 16-byte, maskbits 4-byte alignment");
+    return from_hip(qm::quantize_values(x, x_dtype, rows, cols, hadamard_dim, make_signs(sign_bits, hadamard_dim), mode, seed, maskbits, dequant,
+                                        reinterpret_cast<hipStream_t>(stream)),
+                    "qm_pseudo_quantize_mxfp4");
+}
+
 int qm_requantize_transposed_mxfp4(const uint8_t* codes_in, const uint8_t* scales_in, int64_t R, int64_t C, float post,
                                    int val_dtype, int hadamard_dim, const uint32_t* sign_bits, int mode,
                                    const float* u, uint64_t seed, uint8_t* codes_out, uint8_t* scales_out,

@@ -574,13 +574,11 @@ struct QuantizerFn : Function<QuantizerFn> {
         const Tensor x2 = chunk_rows(x, a.hd);
         const int64_t rows = x2.size(0), cols = x2.size(1);
         const bool quest = a.mode == QM_QUEST_RTN || a.mode == QM_QUEST_SR;
-        const Tensor codes = bytes(rows * cols / 2, x2), scales = bytes(rows * cols / 32, x2);
         Tensor mask, deq = at::empty({rows, cols}, x2.options());
         if (quest) mask = bytes(rows * cols / 8, x2);
-        check(qm_quantize_mxfp4(x2.data_ptr(), dtype_code(x2.scalar_type()), rows, cols, a.hd, a.signs.data(), a.mode, 0, nullptr, a.seed,
-                                codes.data_ptr<uint8_t>(), scales.data_ptr<uint8_t>(), quest ? mask.data_ptr<uint8_t>() : nullptr, deq.data_ptr(),
-                                QM_LAYOUT_ROWMAJOR, stream_of(x2)),
-              "qm_quantize_mxfp4");
+        check(qm_pseudo_quantize_mxfp4(x2.data_ptr(), dtype_code(x2.scalar_type()), rows, cols, a.hd, a.signs.data(), a.mode, a.seed,
+                                       quest ? mask.data_ptr<uint8_t>() : nullptr, deq.data_ptr(), stream_of(x2)),
+              "qm_pseudo_quantize_mxfp4");
         if (a.post != 1.0) deq.mul_(a.post);
         if (ctx) {
             if (quest) ctx->save_for_backward({mask});

@@ -28,6 +28,9 @@ __host__ __device__ inline int64_t tiled_code_offset(int64_t r, int64_t kb, int6
 hipError_t quantize_mxfp4(const void* x, int dtype, int64_t rows, int64_t cols, int hd, const SignBits& sb, int mode,
                           bool transposed_in, const float* u, uint64_t seed, uint8_t* codes, uint8_t* scales,
                           uint8_t* maskbits, void* dequant, int codes_layout, hipStream_t stream);
+// its de-quantized values and clip mask (or null) alone: row-major x, in-kernel random numbers, hd 32, 64 or 128
+hipError_t quantize_values(const void* x, int dtype, int64_t rows, int64_t cols, int hd, const SignBits& sb, int mode, uint64_t seed, uint8_t* maskbits,
+                           void* values, hipStream_t stream);
 // whether quantize_mxfp4 / requantize_transposed_mxfp4 can emit (read) tiled codes for these arguments
 bool quantize_supports_tiled(int64_t rows, int64_t cols, int hd, int mode, bool transposed_in, const float* u,
                              const uint8_t* maskbits);

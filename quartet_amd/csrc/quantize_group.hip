@@ -364,6 +364,78 @@ void launch_rowmajor_wide(int mode, const void* x, int64_t n, float c, const Sig
     }
 }
 
+// ---- only the values: what the quantizer modules return -------------------------------------------------------------
+// One group per lane, flat over the tensor, no codes and scales written.  A wave's 64 groups are contiguous, and pass through LDS both
+// ways: an instruction then moves a contiguous KiB, where a lane's own group is four (fp32: eight) 16-byte pieces 64 (128) bytes
+// from its neighbour's.  Slot kPieces l + (q ^ swizzle) holds piece q of lane l's group: slot-ordered and group-ordered accesses both
+// spread over all banks.  The last wave of a tensor, if it is not whole, takes its groups lane by lane.
+// What bounds it: HBM.  16384 x 4096 bf16 with mask, blocks of 64: 75 us with codes and scales, every value taken apart by hand; 62
+// without the former and by hardware converts; 47 (5.9 TB/s) with whole lines.  With the straight-through backward behind it 117 -> 95.5,
+// blocks of 32 113 -> 95, stochastic absmax 115 -> 93; 32768 x 8192 446 -> 370.
+template <typename T, int MODE, bool WANT_MASK, int HD>
+__global__ __launch_bounds__(256) void quantize_values_kernel(const T* __restrict__ x, int64_t n_groups, Rotation rot, uint64_t seed,
+                                                              uint32_t* __restrict__ maskbits, T* __restrict__ values) {
+    constexpr int kPieces = 2 * (int)sizeof(T);   // 16-byte pieces per group
+    job_starts();
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int64_t first = (int64_t)blockIdx.x * 256 + wave * 64, gi = first + lane;
+    const bool whole = first + 64 <= n_groups;   // uniform
+    if (gi >= n_groups) return;  // n_groups is a multiple of HD/32: the lanes of a chunk leave together
+    uint4* area = job_lds + wave * 64 * kPieces;
+    const auto swizzle = [](int l) { return sizeof(T) == 2 ? (l >> 2) & 3 : l & 7; };
+    // slot 64 i + lane: piece lane % kPieces, swizzled, of group 64 i / kPieces + lane / kPieces
+    const auto piece_of_slot = [&](int i) {
+        const int group = (64 * i + lane) / kPieces;
+        return group * kPieces + ((lane % kPieces) ^ swizzle(group));
+    };
+    float v[32];
+    if (whole) {
+        const uint4* src = reinterpret_cast<const uint4*>(x + first * 32);
+        uint4 raw[kPieces];
+#pragma unroll
+        for (int i = 0; i < kPieces; ++i) raw[i] = src[piece_of_slot(i)];
+        job_requests_issued();
+#pragma unroll
+        for (int i = 0; i < kPieces; ++i) area[64 * i + lane] = raw[i];
+        wave_settle();
+#pragma unroll
+        for (int q = 0; q < kPieces; ++q) {
+            const uint4 t = area[kPieces * lane + (q ^ swizzle(lane))];
+            const uint32_t w[4] = {t.x, t.y, t.z, t.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if constexpr (sizeof(T) == 2) {
+                    v[q * 8 + 2 * i] = u2f(w[i] << 16);
+                    v[q * 8 + 2 * i + 1] = u2f(w[i] & 0xffff0000u);
+                } else {
+                    v[q * 4 + i] = u2f(w[i]);
+                }
+            }
+        }
+    } else {
+        load_group<T>(x + gi * 32, v);
+    }
+    rotate_block<HD>(v, rot);
+    GroupCodes o;
+    quantize_group_regs<MODE, WANT_MASK>(v, seed, gi, o);
+    uint4 out[kPieces];
+    group_values<T>(o, out);
+    job_stores_next();
+    if constexpr (WANT_MASK) maskbits[gi] = o.keep;
+    if (whole) {
+        wave_settle();
+#pragma unroll
+        for (int q = 0; q < kPieces; ++q) area[kPieces * lane + (q ^ swizzle(lane))] = out[q];
+        wave_settle();
+        uint4* dst = reinterpret_cast<uint4*>(values + first * 32);
+#pragma unroll
+        for (int i = 0; i < kPieces; ++i) dst[piece_of_slot(i)] = area[64 * i + lane];
+    } else {
+#pragma unroll
+        for (int q = 0; q < kPieces; ++q) reinterpret_cast<uint4*>(values + gi * 32)[q] = out[q];
+    }
+}
+
 // ---- transposed input: x is [P, Q] row-major, output is the [Q, P] tensor quantized along P ----------
 // A workgroup owns a strip of 256 bytes of columns (128 bf16 / 64 fp32) by 128 rows; wave w owns p-group w.
 // A lane reads its column (bf16: two adjacent columns per 32-bit load) at 32 successive rows straight from
@@ -1406,9 +1478,18 @@ hipError_t swiglu_quantize_hd32(const void* h12, int dtype, int64_t rows, int64_
     return hipGetLastError();
 }
 
-// ---- the quantizer launches of one layer ------------------------------------------------------------------------
+// ---- the quantizer launches of one layer, and of a quantizer module -----------------------------------------------
 
 namespace {
+template <typename F>
+void with_mode(int mode, F&& f) {
+    switch (mode) {
+        case QUEST_RTN: return f(std::integral_constant<int, QUEST_RTN>{});
+        case ABSMAX_RTN: return f(std::integral_constant<int, ABSMAX_RTN>{});
+        case ABSMAX_SR: return f(std::integral_constant<int, ABSMAX_SR>{});
+        default: return f(std::integral_constant<int, QUEST_SR>{});
+    }
+}
 template <typename F>
 void with_elem_type(int dtype, F&& f) {
     if (dtype == BF16) f(uint16_t{});
@@ -1431,6 +1512,24 @@ void with_hadamard(int hd, F&& f) {
     else f(std::integral_constant<int, 128>{});
 }
 }  // namespace
+
+hipError_t quantize_values(const void* x, int dtype, int64_t rows, int64_t cols, int hd, const SignBits& sb, int mode, uint64_t seed, uint8_t* maskbits,
+                           void* values, hipStream_t stream) {
+    const int64_t n_groups = rows * cols / 32;
+    with_elem_type(dtype, [&](auto t) {
+        using T = decltype(t);
+        with_mode(mode, [&](auto m) {
+            with_flag(maskbits != nullptr, [&](auto k) {
+                with_hadamard(hd, [&](auto h) {
+                    constexpr int HD = decltype(h)::value;
+                    quantize_values_kernel<T, decltype(m)::value, decltype(k)::value, HD><<<dim3((unsigned)((n_groups + 255) / 256)), dim3(256), 256 * 32 * sizeof(T), stream>>>(
+                        reinterpret_cast<const T*>(x), n_groups, make_rotation<HD>(dtype, sb), seed, reinterpret_cast<uint32_t*>(maskbits), reinterpret_cast<T*>(values));
+                });
+            });
+        });
+    });
+    return hipGetLastError();
+}
 
 hipError_t quantize_layer_forward(const RowmajorArgs& x, const RowmajorArgs* w, int hd, hipStream_t stream) {
     const auto out_of = [](const RowmajorArgs& a) {
