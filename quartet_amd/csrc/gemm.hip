@@ -426,7 +426,7 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // WIDE: the rotated, bf16-rounded result leaves widened to fp32 (the weight gradient of an fp32 weight), 32 columns at a time through
 // the same 4 KiB, whole 128-byte lines out.
-template <int ROT = 0, bool RAGGED = false, bool WIDE = false>
+template <int ROT = 0, bool RAGGED = false, bool WIDE = false, bool UNIT = false>
 __device__ __forceinline__ void big4_epilogue_bf16(v16f (&acc)[4][4], float alpha, void* __restrict__ c, int64_t m0,
                                                    int64_t n0, int64_t N, int wm, int wn, int wave, int lane_in,
                                                    uint8_t* smem_bytes, int rows_valid, int cols_valid,
@@ -500,8 +500,8 @@ __device__ __forceinline__ void big4_epilogue_bf16(v16f (&acc)[4][4], float alph
                     for (int b = 0; b < 4; ++b) {
                         const v16f& t = acc[i][2 * jp + jj];
                         const float t0 = acc_read(t[4 * b]), t1 = acc_read(t[4 * b + 1]), t2 = acc_read(t[4 * b + 2]), t3 = acc_read(t[4 * b + 3]);
-                        const v2bf p0 = __builtin_convertvector(v2f{t0 * alpha, t1 * alpha}, v2bf);
-                        const v2bf p1 = __builtin_convertvector(v2f{t2 * alpha, t3 * alpha}, v2bf);
+                        const v2bf p0 = __builtin_convertvector(UNIT ? v2f{t0, t1} : v2f{t0 * alpha, t1 * alpha}, v2bf);
+                        const v2bf p1 = __builtin_convertvector(UNIT ? v2f{t2, t3} : v2f{t2 * alpha, t3 * alpha}, v2bf);
                         *reinterpret_cast<uint2*>(wr + (((jj * 4 + b) * 16) ^ wsw)) =
                             make_uint2(__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1));
                     }
@@ -628,8 +628,11 @@ enum Big4Result : int { BIG4_PLAIN = 1, BIG4_ROTATED = 2, BIG4_WIDE = 4 };   // 
 // flat stream of K steps.  The loads that refill a freed ring stage simply continue into the next tile, so the
 // pipeline never drains between tiles and the epilogue runs while the next tile's first four stages arrive.
 // RAGGED: M is not a multiple of 64 (an instantiation of its own: the row tests cost the others 2 to 8 % in registers).
+// UNIT: alpha is 1 (a layer's forward product, bf16 result): 256 multiplications less among the epilogue's ~770 vector instructions a
+// tile, which nothing overlaps.  Whole inference calls: 16384 x 1536 x 8192 125.8 -> 123.0 us, 16384 x 1536 x 4608 80.6 -> 79.3, 8192 x 4096 x
+// 11008 194.2 -> 192.8; 8192 x 4096 x 4096 the same.
 // PAIR: two products (Big4Other), tiled operands; the sum of the kinds of result that they have.
-template <typename OutT, bool STAMP = false, int ROT = 0, bool RAGGED = false, int PAIR = 0>
+template <typename OutT, bool STAMP = false, int ROT = 0, bool RAGGED = false, int PAIR = 0, bool UNIT = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_mxfp4_tn_big4_kernel(
     const uint8_t* __restrict__ a_codes, const uint8_t* __restrict__ a_scales, const uint8_t* __restrict__ b_codes,
     const uint8_t* __restrict__ b_scales, int M, int N, int K, float alpha, OutT* __restrict__ c, int a_tiled,
@@ -878,7 +881,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             } else if ((PAIR & BIG4_WIDE) && ((PAIR & BIG4_ROTATED) == 0 || result == BIG4_WIDE)) leave(std::true_type{}, std::true_type{});
             else leave(std::true_type{}, std::false_type{});
         } else if constexpr (sizeof(OutT) == 2) {
-            big4_epilogue_bf16<ROT, RAGGED>(acc, alpha, dst, m0, n0, N, wm, wn, wave, lane, smem_bytes, rows_valid, cols_valid, turn, keep, keep_shifted);
+            big4_epilogue_bf16<ROT, RAGGED, false, UNIT>(acc, alpha, dst, m0, n0, N, wm, wn, wave, lane, smem_bytes, rows_valid, cols_valid, turn, keep, keep_shifted);
         } else {
             OutT* slab = splits > 1 ? c + (int64_t)cur_split * M * N : c;
             const float a_eff = splits > 1 ? 1.0f : alpha;
@@ -1071,11 +1074,11 @@ Cut cheapest_cut(int64_t M, int64_t N, int64_t K, bool persistent, bool tiles_ok
 // item, where the tile boundary is a third or more of a tile; longer ones neither gain nor lose (within 0.7 %)
 int big4_late_start(int64_t K, int splits) { return K / kBK / splits <= 16 ? 6 : 0; }
 
-template <typename OutT, int ROT, bool RAGGED>
+template <typename OutT, int ROT, bool RAGGED, bool UNIT = false>
 hipError_t launch_big4_as(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
                           const uint8_t* b_scales, int64_t M, int64_t N, int64_t K, float alpha, void* c, int a_tiled,
                           int b_tiled, int splits, int cus, hipStream_t stream, const RotEpilogue& rot) {
-    auto kern = gemm_mxfp4_tn_big4_kernel<OutT, false, ROT, RAGGED>;
+    auto kern = gemm_mxfp4_tn_big4_kernel<OutT, false, ROT, RAGGED, 0, UNIT>;
     static std::atomic<bool> lds_allowed[kMaxDevices];
     hipError_t e = allow_dynamic_lds(kern, kBig4SmemBytes, lds_allowed);
     if (e != hipSuccess) return e;
@@ -1093,6 +1096,10 @@ template <typename OutT, int ROT = 0>
 hipError_t launch_big4(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes,
                        const uint8_t* b_scales, int64_t M, int64_t N, int64_t K, float alpha, void* c, int a_tiled,
                        int b_tiled, int splits, int cus, hipStream_t stream, const RotEpilogue& rot = RotEpilogue{}) {
+    if constexpr (sizeof(OutT) == 2 && ROT == 0)
+        if (alpha == 1.0f)
+            return M % 64 ? launch_big4_as<OutT, 0, true, true>(a_codes, a_scales, b_codes, b_scales, M, N, K, alpha, c, a_tiled, b_tiled, splits, cus, stream, rot)
+                          : launch_big4_as<OutT, 0, false, true>(a_codes, a_scales, b_codes, b_scales, M, N, K, alpha, c, a_tiled, b_tiled, splits, cus, stream, rot);
     if (M % 64)
         return launch_big4_as<OutT, ROT, true>(a_codes, a_scales, b_codes, b_scales, M, N, K, alpha, c, a_tiled, b_tiled, splits, cus, stream, rot);
     return launch_big4_as<OutT, ROT, false>(a_codes, a_scales, b_codes, b_scales, M, N, K, alpha, c, a_tiled, b_tiled, splits, cus, stream, rot);
