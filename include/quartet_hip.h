@@ -403,6 +403,22 @@ int qm_linear_decode_serves(int64_t T, int64_t I, int64_t O);
 int qm_linear_decode(const void* x, int x_dtype, int64_t T, int64_t I, int64_t O, const uint32_t* signs_x, const void* packed_w,
                      size_t packed_w_bytes, void* y, int y_dtype, void* stream);
 
+/*
+ * Forward products of an evaluated model (nothing is kept for a backward pass) whose bf16 result feeds one kernel: the product's own
+ * epilogue goes on with it and the result never travels through memory; the same bits as the separate launches.  packed_x [T, I]
+ * and packed_w are operands in QM_LAYOUT_PADDED, T > 64, I % 32 == 0.
+ * qm_linear_swiglu_quantize: packed_w [2 hidden, I] = (up, gate) (src/models/llama.py:113-114); packed receives the codes and scales of
+ *   qm_swiglu_quantize_mxfp4 of the bf16 product, without its clip mask.  hidden % 32 == 0.
+ * qm_linear_rope: packed_w [3 n_embd, I]; q, k, v [T, n_embd] bf16 as qm_rope_split_qkv gives them.  head_dim % 8 == 0.
+ * The *_serves functions tell where they run and are expected to be faster (1 / 0).
+ */
+int qm_linear_swiglu_serves(int64_t T, int64_t I, int64_t hidden);
+int qm_linear_swiglu_quantize(const void* packed_x, size_t packed_x_bytes, const void* packed_w, size_t packed_w_bytes, int64_t T,
+                              int64_t I, int64_t hidden, const uint32_t* sign_bits, void* packed, size_t packed_bytes, void* stream);
+int qm_linear_rope_serves(int64_t T, int64_t I, int64_t n_embd, int head_dim);
+int qm_linear_rope(const void* packed_x, size_t packed_x_bytes, const void* packed_w, size_t packed_w_bytes, int64_t T, int64_t I,
+                   int64_t n_embd, int head_dim, int64_t seq_len, const float* table, void* q, void* k, void* v, void* stream);
+
 /* Test aid: silu as the SwiGLU producer evaluates it for bf16 tensors, of every bf16 bit pattern: out[65536] */
 int qm_diag_silu_bf16(uint16_t* out, void* stream);
 

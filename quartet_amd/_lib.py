@@ -50,6 +50,10 @@ EXPORTS = (
     "qm_linear_decode_serves",
     "qm_linear_backward_in_one_launch",
     "qm_pseudo_quantize_mxfp4",
+    "qm_linear_swiglu_serves",
+    "qm_linear_swiglu_quantize",
+    "qm_linear_rope_serves",
+    "qm_linear_rope",
     "qm_linear_decode",
     "qm_cross_entropy",
     "qm_diag_silu_bf16",
@@ -137,6 +141,14 @@ def lib():
     L.qm_linear_backward_in_one_launch.argtypes = [i64, i64, i64, i32, i32, i32, i32]
     L.qm_pseudo_quantize_mxfp4.restype = i32
     L.qm_pseudo_quantize_mxfp4.argtypes = [vp, i32, i64, i64, i32, vp, i32, u64, vp, vp, vp]
+    L.qm_linear_swiglu_serves.restype = i32
+    L.qm_linear_swiglu_serves.argtypes = [i64, i64, i64]
+    L.qm_linear_swiglu_quantize.restype = i32
+    L.qm_linear_swiglu_quantize.argtypes = [vp, ctypes.c_size_t, vp, ctypes.c_size_t, i64, i64, i64, vp, vp, ctypes.c_size_t, vp]
+    L.qm_linear_rope_serves.restype = i32
+    L.qm_linear_rope_serves.argtypes = [i64, i64, i64, i32]
+    L.qm_linear_rope.restype = i32
+    L.qm_linear_rope.argtypes = [vp, ctypes.c_size_t, vp, ctypes.c_size_t, i64, i64, i64, i32, i64, vp, vp, vp, vp, vp]
     L.qm_linear_decode.restype = i32
     L.qm_linear_decode.argtypes = [vp, i32, i64, i64, i64, vp, vp, ctypes.c_size_t, vp, i32, vp]
     L.qm_cross_entropy.restype = i32

@@ -557,6 +557,69 @@ int qm_linear_forward(const void* x, int x_dtype, const void* w, int w_dtype, in
                     "qm_linear_forward");
 }
 
+namespace {
+// a product of an evaluated model on packed operands in the padded layout, of the extents that those kernels take
+bool after_product(int64_t T, int64_t I, int64_t N, const uint8_t* px, const uint8_t* pw, void* c, qm::TileProduct* p) {
+    // up to 64 tokens the layers add their terms in another order (gemm_rows.hip)
+    if (T <= 64 || I <= 0 || N <= 0 || I % 32 || N % 8 || T >= (1 << 30) || I >= (1 << 23) || N >= (1 << 30)) return false;
+    const PackedLayout lx = packed_layout(T, I), lw = packed_layout(N, I);
+    *p = qm::make_product(px + lx.c, px + lx.s, pw + lw.c, pw + lw.s, T, N, qm::padded_cols(I), 1.0f, c, QM_LAYOUT_TILED, QM_LAYOUT_TILED);
+    return qm::gemm_tile_after_serves(*p);
+}
+uint8_t* stand_in() { return reinterpret_cast<uint8_t*>((uintptr_t)256); }   // for questions in which nothing is read
+}  // namespace
+
+int qm_linear_swiglu_serves(int64_t T, int64_t I, int64_t hidden) {
+    qm::TileProduct p;
+    if (hidden <= 0 || hidden % 32 || hidden >= (1 << 23) || !after_product(T, I, 2 * hidden, stand_in(), stand_in(), stand_in(), &p)) return 0;
+    return qm::product_after_pays(p, 0.6, 3.5 + (double)T * hidden * 4.66 / 4.8e6) ? 1 : 0;
+}
+
+int qm_linear_swiglu_quantize(const void* packed_x, size_t packed_x_bytes, const void* packed_w, size_t packed_w_bytes, int64_t T, int64_t I,
+                              int64_t hidden, const uint32_t* sign_bits, void* packed, size_t packed_bytes, void* stream) {
+    qm::TileProduct p;
+    uint8_t* out = static_cast<uint8_t*>(packed);
+    if (hidden <= 0 || hidden % 32 || hidden >= (1 << 23) ||
+        !after_product(T, I, 2 * hidden, static_cast<const uint8_t*>(packed_x), static_cast<const uint8_t*>(packed_w), out, &p))
+        return fail(QM_ERR_INVALID, "qm_linear_swiglu_quantize: [%lld, %lld] x [2 x %lld] is not served (see qm_linear_swiglu_serves)", (long long)T, (long long)I,
+                    (long long)hidden);
+    const PackedLayout l = packed_layout(T, hidden);
+    if (!packed_x || packed_x_bytes < packed_layout(T, I).total || !aligned(packed_x, 256) || !packed_w || packed_w_bytes < packed_layout(2 * hidden, I).total ||
+        !aligned(packed_w, 256) || !packed || packed_bytes < l.total || !aligned(packed, 256))
+        return fail(QM_ERR_INVALID, "qm_linear_swiglu_quantize: packed operand buffers too small, null or not 256-byte aligned");
+    qm::TileAfter after{};
+    p.c = out + l.c;
+    after.scales = out + l.s;
+    after.sign_word = sign_bits ? sign_bits[0] : 0u;
+    after.c = qm::hadamard_scale(32, QM_BF16);
+    return from_hip(qm::gemm_tile_swiglu(p, after, reinterpret_cast<hipStream_t>(stream)), "qm_linear_swiglu_quantize");
+}
+
+int qm_linear_rope_serves(int64_t T, int64_t I, int64_t n_embd, int head_dim) {
+    qm::TileProduct p;
+    if (n_embd <= 0 || n_embd > (1 << 24) || head_dim <= 0 || head_dim % 8 || n_embd % head_dim ||
+        !after_product(T, I, 3 * n_embd, stand_in(), stand_in(), stand_in(), &p))
+        return 0;
+    return qm::product_after_pays(p, 0.3, 3.0 + (double)T * n_embd * 12.0 / 5.0e6) ? 1 : 0;
+}
+
+int qm_linear_rope(const void* packed_x, size_t packed_x_bytes, const void* packed_w, size_t packed_w_bytes, int64_t T, int64_t I, int64_t n_embd,
+                   int head_dim, int64_t seq_len, const float* table, void* q, void* k, void* v, void* stream) {
+    qm::TileProduct p;
+    if (n_embd <= 0 || n_embd > (1 << 24) || head_dim <= 0 || head_dim % 8 || n_embd % head_dim || seq_len <= 0 || seq_len > (1 << 30) ||
+        !after_product(T, I, 3 * n_embd, static_cast<const uint8_t*>(packed_x), static_cast<const uint8_t*>(packed_w), q, &p))
+        return fail(QM_ERR_INVALID, "qm_linear_rope: [%lld, %lld] x [3 x %lld], head_dim %d is not served (see qm_linear_rope_serves)", (long long)T, (long long)I,
+                    (long long)n_embd, head_dim);
+    if (!packed_x || packed_x_bytes < packed_layout(T, I).total || !aligned(packed_x, 256) || !packed_w || packed_w_bytes < packed_layout(3 * n_embd, I).total ||
+        !aligned(packed_w, 256) || !table || !q || !k || !v || !aligned(table, 16) || !aligned(q, 16) || !aligned(k, 16) || !aligned(v, 16))
+        return fail(QM_ERR_INVALID, "qm_linear_rope: packed operand buffers too small, null or not 256-byte aligned, or tensors not 16-byte aligned");
+    qm::TileAfter after{};
+    after.q = q; after.k = k; after.v = v;
+    after.table = table;
+    after.seq_len = (int)seq_len; after.width = (int)n_embd; after.head_dim = head_dim;
+    return from_hip(qm::gemm_tile_rope(p, after, reinterpret_cast<hipStream_t>(stream)), "qm_linear_rope");
+}
+
 int qm_linear_decode_serves(int64_t T, int64_t I, int64_t O) { return qm::linear_decode_serves(T, I, O) ? 1 : 0; }
 
 int qm_linear_decode(const void* x, int x_dtype, int64_t T, int64_t I, int64_t O, const uint32_t* signs_x, const void* packed_w,

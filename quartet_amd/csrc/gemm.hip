@@ -1472,6 +1472,15 @@ hipError_t run_pair(const PairChoice& c, const TileProduct& x, int x_out, const 
     }
 }
 
+// Whether a product on 128 x 128 tiles whose epilogue goes on with what is made of it (`end` us a tile and CU) is expected to beat the
+// fastest kernel of the product alone and a pass of its own over its result (us)
+bool product_after_pays(const TileProduct& p, double end, double pass) {
+    const int cus = device_cus();
+    const KernelCost& k = tile_costs(false, TILE_128x128, p.K, 1);
+    const double tiles = (double)((p.M + 127) / 128) * ((p.N + 127) / 128);
+    return tile_cost(k, p.M, p.N, p.K, 1, cus) + end * tiles / cus < choose_product(p, BF16, BF16, nullptr, 0).cost + pass;
+}
+
 TileProduct make_product(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes, const uint8_t* b_scales, int64_t M, int64_t N,
                          int64_t K, float alpha, void* c, int a_layout, int b_layout) {
     TileProduct p{};

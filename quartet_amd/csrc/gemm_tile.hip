@@ -27,6 +27,7 @@
 
 #include "gemm_common.h"
 #include "hadamard_octet.h"
+#include "quantize_group.h"
 
 namespace qm {
 
@@ -231,8 +232,15 @@ __device__ __forceinline__ void tile_mfma(const TileFrags<S>& f, const uint32_t 
 // ROT: the masked inverse rotation in the epilogue (bf16 results of the product).  A template argument: a plain product that carries
 // the rotation's code behind a branch is slower with the same registers (an inference call of 1000 x 1536 x 8192 15.8 us, 15.5
 // without; an evaluated 30 M model's pass 1000 and 992).
-template <class S, typename OutT, bool ROT>
-__device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* smem, uint32_t smem_base) {
+// Evaluated 30 M model, 4096 tokens: 4096 x 3456 x 640 with SwiGLU and quantizer in its end 16.1 us (256 x 128 tiles 17.7), 12.7 and 12.5 as two
+// launches; 4096 x 1920 x 640 with the rotary split 12.3 us, 16.4 as two; a pass of the model 1004 -> 924.  What bounds them: the 1400
+// vector instructions of a group's quantizer, three waves to a SIMD, and a second round of few tiles.
+// AFTER: what becomes of a plain bf16 result in an evaluated model, instead of being stored (TileAfter): nothing else, the SwiGLU of its two
+// halves quantized for the next layer, or its split into q, k and v with the rotary embedding.
+enum TileEnd : int { END_STORE = 0, END_SWIGLU = 1, END_ROPE = 2 };
+template <class S, typename OutT, bool ROT, int AFTER = END_STORE>
+__device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* smem, uint32_t smem_base, [[maybe_unused]] const TileAfter& after = TileAfter{}) {
+    static_assert(AFTER == END_STORE || (sizeof(OutT) == 2 && !ROT && !S::kWideB), "ends of plain bf16 products");
     constexpr bool SWAP = sizeof(OutT) == 2;
     uint8_t* smem_bytes = reinterpret_cast<uint8_t*>(smem);
     const int tid = threadIdx.x, lane = tid & 63;
@@ -240,7 +248,9 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
     const int wm = wave / S::kWavesN, wn = wave % S::kWavesN;
     const int lrow = lane & 31, half = lane >> 5;
     const int M = g.M, N = g.N, K = g.K;
-    const int tiles_m = (M + S::BM - 1) / S::BM, tiles_n = (N + S::BN - 1) / S::BN;
+    // SwiGLU: half of a tile's columns are of the one half of B's rows, half the same columns of the other; with the next layer's padding
+    const int hidden = N / 2, hidden_groups = hidden / 32, hidden_padded = (hidden_groups + 3) & ~3;
+    const int tiles_m = (M + S::BM - 1) / S::BM, tiles_n = AFTER == END_SWIGLU ? (hidden_padded * 64 + S::BN - 1) / S::BN : (N + S::BN - 1) / S::BN;
     const int code_pitch = K / 2, groups = K / 32;
     // a work item is (tile, K range): range r covers steps [r * all / splits, (r + 1) * all / splits) and, with splits > 1 (fp32
     // instantiation only), stores its partial sums, unscaled, into slab r of c = [splits][M][N]
@@ -251,6 +261,23 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
     int tm, tn;
     tile_of_run<(S::BM >= 256 ? 4 : 8)>(item - range * tiles, tiles_m, tiles_n, tm, tn);
     const int m0 = tm * S::BM, n0 = tn * S::BN;
+    const int h0 = tn * (S::BN / 2);
+    // the packed operand's place of group gh of a row, in 16-byte pieces
+    const auto packed_slot = [&](int row, int gh) { return (int64_t)(row >> 4) * 16 * hidden_padded + ((gh >> 2) * 64 + (row & 15) * 4 + (gh & 3)); };
+    if constexpr (AFTER == END_SWIGLU)
+        if (h0 >= hidden) {   // a tile of padding: zero codes and scales
+            for (int u = tid; u < S::BM * (S::BN / 64); u += S::kThreads) {
+                const int row = m0 + u / (S::BN / 64), gh = h0 / 32 + u % (S::BN / 64);
+                if (row >= M || gh >= hidden_padded) continue;
+                reinterpret_cast<uint4*>(g.c)[packed_slot(row, gh)] = make_uint4(0u, 0u, 0u, 0u);
+                after.scales[(int64_t)row * hidden_padded + gh] = 0;
+            }
+            return;
+        }
+    const auto source_of = [&](int r) {   // B's row behind column r of the tile
+        const int h = h0 + r % (S::BN / 2) < hidden ? h0 + r % (S::BN / 2) : hidden - 1;
+        return r < S::BN / 2 ? h : hidden + h;
+    };
 
     const int swz = (lrow >> 2) & 3;
     const int a_off0 = (wm * S::WM + lrow) * kRowBytes + (((2 * half) ^ swz) * 16);
@@ -278,7 +305,7 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
         plan.kstep_a = g.a_tiled ? 1024 : kRowBytes;
         plan.kstep_b = g.b_tiled ? 1024 * S::kBBlocks : kRowBytes;
         plan.a = g.a_codes + (int64_t)m0 * code_pitch + (int64_t)k_first * plan.kstep_a;   // m0, n0 are multiples of 16: the same
-        plan.b = g.b_codes + (int64_t)n0 * code_pitch * S::kBBlocks + (int64_t)k_first * plan.kstep_b;   //   expression in both layouts
+        plan.b = g.b_codes + (AFTER == END_SWIGLU ? 0 : (int64_t)n0 * code_pitch * S::kBBlocks) + (int64_t)k_first * plan.kstep_b;   //   expression in both layouts
 #pragma unroll
         for (int j = 0; j < S::kALoads; ++j) {
             const int r = (wave * S::kALoads + j) * 16 + prow;
@@ -291,7 +318,7 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
             if constexpr (S::kWideB)
                 plan.voff_b[j] = (uint32_t)((rr >> 4) * 2 * row16) + (uint32_t)((u / (S::BN / 16)) * 1024 + (rr & 15) * 64 + pcv * 16);
             else
-                plan.voff_b[j] = row_off(rr, row_b);
+                plan.voff_b[j] = row_off(AFTER == END_SWIGLU ? source_of(r) : rr, row_b);
         }
         plan.half_back = (uint32_t)(pcv & 2) * 16u;
         plan.lds_a = (uint32_t)__builtin_amdgcn_readfirstlane((int)(smem_base + wave * S::kALoads * 1024));
@@ -306,8 +333,8 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
             const int ra = S::kBlocks ? p : (p / (32 * S::TM)) * S::WM + (p % S::TM) * 32 + (p / S::TM) % 32;
             const int rb = S::kBlocks ? p : (p / (32 * S::TN)) * S::WN + (p % S::TN) * 32 + (p / S::TN) % 32;
             const int la = M - 1 - m0, lb = N - 1 - n0;
-            const int r = is_a ? (ra < la ? ra : la) : (rb < lb ? rb : lb);
-            plan.s[u] = (is_a ? g.a_scales + (int64_t)m0 * groups : g.b_scales + (int64_t)n0 * groups) + k_first * 4;
+            const int r = is_a ? (ra < la ? ra : la) : AFTER == END_SWIGLU ? source_of(rb) : (rb < lb ? rb : lb);
+            plan.s[u] = (is_a ? g.a_scales + (int64_t)m0 * groups : g.b_scales + (AFTER == END_SWIGLU ? 0 : (int64_t)n0 * groups)) + k_first * 4;
             plan.voff_s[u] = (uint32_t)(r * groups);
             plan.lds_s[u] = (uint32_t)__builtin_amdgcn_readfirstlane((int)(smem_base + S::kSAOff + unit * S::kUnitBytes));
         }
@@ -620,7 +647,70 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
         typedef uint32_t u4v __attribute__((ext_vector_type(4)));
         typedef float f4v __attribute__((ext_vector_type(4)));
         const bool col_ok = out_col < N;   // N is a multiple of 8
-        if constexpr (!ROT) {
+        if constexpr (AFTER == END_SWIGLU) {
+            // A lane per row and group: the arithmetic of the producer (SwiGluProducer) and the quantizer on the bf16 values that would
+            // have been stored, the same bits; no clip mask, which only a backward pass reads.
+            constexpr int kSide = S::BN / 64;   // groups of the next operand per row of the tile
+#pragma unroll 1
+            for (int u = id; u < S::BM * kSide; u += S::kThreads) {
+                const int line = u / kSide, row = m0 + line, side = u % kSide, gh = h0 / 32 + side;
+                const auto read_group = [&](int at, float (&v)[32]) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const uint4 raw = *reinterpret_cast<const uint4*>(smem_bytes + line * S::kPitch + at + q * 16);
+                        const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            v[8 * q + 2 * e] = u2f(w[e] << 16);
+                            v[8 * q + 2 * e + 1] = u2f(w[e] & 0xffff0000u);
+                        }
+                    }
+                };
+                float v[32], gate[32];
+                read_group(side * 64, v);
+                read_group(S::BN + side * 64, gate);
+                swiglu_group_bf16(v, gate);
+                rotate_group(v, after.c, after.sign_word);
+                GroupCodes o;
+                quantize_group_regs<QUEST_RTN, false>(v, 0, 0, o);
+                if (row >= M || gh >= hidden_padded) continue;
+                const bool real = gh < hidden_groups;
+                reinterpret_cast<uint4*>(g.c)[packed_slot(row, gh)] = real ? make_uint4(o.w[0], o.w[1], o.w[2], o.w[3]) : make_uint4(0u, 0u, 0u, 0u);
+                after.scales[(int64_t)row * hidden_padded + gh] = real ? (uint8_t)o.scale_byte : 0;
+            }
+        } else if constexpr (AFTER == END_ROPE) {
+            // (q, k, v) by thirds of the columns, pairs of q and k rotated in fp32: the arithmetic of rope_qkv_kernel on the bf16 values that
+            // would have been stored, the same bits
+            const int part = out_col / after.width, c = out_col - part * after.width, pair = (c % after.head_dim) >> 1;
+            uint16_t* dst = static_cast<uint16_t*>(part == 0 ? after.q : part == 1 ? after.k : after.v);
+            constexpr int kAtOnce = S::kPasses < 4 ? S::kPasses : 4;   // passes whose table entries are on their way together
+            int pos = (m0 + rsub) % after.seq_len;
+#pragma unroll 1
+            for (int r0 = 0; r0 < S::kPasses; r0 += kAtOnce) {
+                float4 t[kAtOnce][2];
+#pragma unroll
+                for (int i = 0; i < kAtOnce; ++i) {
+                    if (part < 2) {   // rows past the end have positions, too
+                        const float4* cs = reinterpret_cast<const float4*>(after.table + ((int64_t)pos * (after.head_dim / 2) + pair) * 2);
+                        t[i][0] = cs[0];
+                        t[i][1] = cs[1];
+                    }
+                    for (pos += S::kRowsPerPass; pos >= after.seq_len;) pos -= after.seq_len;
+                }
+#pragma unroll
+                for (int i = 0; i < kAtOnce; ++i) {
+                    const int line = (r0 + i) * S::kRowsPerPass + rsub, row = m0 + line;
+                    uint4 v = *reinterpret_cast<const uint4*>(smem_bytes + line * S::kPitch + chunk * 16);
+                    const auto turn = [](uint32_t w, float co, float si) {
+                        const float a = u2f(w << 16), b = u2f(w & 0xffff0000u);
+                        return __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{a * co - b * si, a * si + b * co}, v2bf));
+                    };
+                    if (part < 2)
+                        v = make_uint4(turn(v.x, t[i][0].x, t[i][0].y), turn(v.y, t[i][0].z, t[i][0].w), turn(v.z, t[i][1].x, t[i][1].y), turn(v.w, t[i][1].z, t[i][1].w));
+                    if (col_ok && row < M) *reinterpret_cast<uint4*>(dst + (int64_t)row * after.width + c) = v;
+                }
+            }
+        } else if constexpr (!ROT) {
             uint16_t* out = reinterpret_cast<uint16_t*>(g.c) + (int64_t)(m0 + rsub) * N + out_col;
 #pragma unroll
             for (int r = 0; r < S::kPasses; ++r) {
@@ -763,6 +853,29 @@ hipError_t launch_pair(const TileProduct& a, const TileProduct& b, hipStream_t s
     return hipGetLastError();
 }
 
+// a plain product with one of those ends
+template <class S, int AFTER>
+__global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu((S::OCC * S::kWaves + 3) / 4))) void gemm_mxfp4_tn_after_kernel(
+    TileProduct g, TileAfter after, int tiles) {
+    extern __shared__ uint32_t smem[];
+    const uint32_t smem_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint32_t*)smem;
+    for (int t = (int)blockIdx.x; t < tiles; t += (int)gridDim.x) tile_run<S, uint16_t, false, AFTER>(g, t, smem, smem_base, after);
+}
+template <class S, int AFTER>
+hipError_t launch_after(TileProduct g, const TileAfter& after, hipStream_t stream) {
+    const auto kern = gemm_mxfp4_tn_after_kernel<S, AFTER>;
+    static std::atomic<bool> lds_allowed[kMaxDevices];
+    const hipError_t e = allow_dynamic_lds(kern, S::kSmemBytes, lds_allowed);
+    if (e != hipSuccess) return e;
+    g.splits = 1;
+    const int cols = AFTER == END_SWIGLU ? (int)padded_cols(g.N / 2) * 2 : g.N;
+    const int tiles = ((g.M + S::BM - 1) / S::BM) * ((cols + S::BN - 1) / S::BN);
+    int grid = tiles < S::OCC * device_cus() ? tiles : S::OCC * device_cus();
+    if (grid > 8 && grid < tiles) grid -= grid % 8;
+    kern<<<dim3((unsigned)grid), dim3(S::kThreads), S::kSmemBytes, stream>>>(g, after, tiles);
+    return hipGetLastError();
+}
+
 using Tile256x128 = TileShape<256, 128, 128, 64, 3, 2>;
 using Tile128x128 = TileShape<128, 128, 64, 64, 3, 3>;
 using Tile128x64 = TileShape<128, 64, 64, 32, 4, 3>;
@@ -805,6 +918,20 @@ hipError_t gemm_tile_pair(TileProduct a, int shape_a, bool a_f32, TileProduct b,
     };
     if (shape_a == TILE_64x64) return shape_b == TILE_64x64 ? rotations(Tile64x64{}, Tile64x64{}) : rotations(Tile64x64{}, Tile128x128{});
     return shape_b == TILE_64x64 ? rotations(Tile128x128{}, Tile64x64{}) : rotations(Tile128x128{}, Tile128x128{});
+}
+
+// tiled operands of either end: whole K steps, dwords of scales, offsets into all of B in 32 bits
+bool gemm_tile_after_serves(const TileProduct& g) {
+    return g.a_tiled && g.b_tiled && !g.b_e5m2 && !g.mask && gemm_tile_serves(g.M, g.N, g.K, 1, 1, g.c) && g.K % kBK == 0 && (int64_t)g.N * (g.K / 2) < (1ll << 31) &&
+           ((reinterpret_cast<uintptr_t>(g.a_scales) | reinterpret_cast<uintptr_t>(g.b_scales)) & 3) == 0;
+}
+hipError_t gemm_tile_swiglu(const TileProduct& g, const TileAfter& after, hipStream_t stream) {
+    if (!gemm_tile_after_serves(g) || g.N % 64) return hipErrorInvalidValue;
+    return g.K / kBK >= 4 ? launch_after<Tile128x128, END_SWIGLU>(g, after, stream) : launch_after<Tile128x128::Narrow, END_SWIGLU>(g, after, stream);
+}
+hipError_t gemm_tile_rope(const TileProduct& g, const TileAfter& after, hipStream_t stream) {
+    if (!gemm_tile_after_serves(g) || g.N != 3 * after.width || after.width % after.head_dim || after.head_dim % 8) return hipErrorInvalidValue;
+    return g.K / kBK >= 4 ? launch_after<Tile128x128, END_ROPE>(g, after, stream) : launch_after<Tile128x128::Narrow, END_ROPE>(g, after, stream);
 }
 
 hipError_t gemm_tile(int shape, const TileProduct& g, int c_dtype, hipStream_t stream) {

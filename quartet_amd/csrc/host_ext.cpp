@@ -379,6 +379,18 @@ struct NormArgs {
     bool has_add, pass_input;
     Tensor* packed_w;
 };
+// Q(rmsnorm(x2 [+ add2]) * gain) as the layer's packed operand; x2 becomes the sum
+Tensor normed_into_packed(const Layer& l, Tensor& x2, const Tensor& add2, const Tensor& gain, double eps, Tensor& factor) {
+    Tensor packed_x = packed_buffer(l.T, l.I, x2), x_sum;
+    factor = at::empty({l.T}, x2.options().dtype(at::kFloat));
+    if (add2.defined()) x_sum = at::empty_like(x2);
+    check(qm_rmsnorm_quantize_mxfp4(x2.data_ptr(), dtype_code(x2.scalar_type()), ptr(add2), add2.defined() ? dtype_code(add2.scalar_type()) : 0,
+                                    add2.defined() ? x_sum.data_ptr() : nullptr, gain.data_ptr<float>(), (float)eps, l.T, l.I, l.a_signs.data(),
+                                    packed_x.data_ptr(), (size_t)packed_x.numel(), factor.data_ptr<float>(), l.layout, stream_of(x2)),
+          "qm_rmsnorm_quantize_mxfp4");
+    if (add2.defined()) x2 = x_sum;
+    return packed_x;
+}
 struct NormLinearFn : Function<NormLinearFn> {
     static variable_list forward(AutogradContext* ctx, const Tensor& x, const optional<Tensor>& add_in, const Tensor& gain,
                                  const Tensor& weight, const LayerPtr& l, const NormArgs& args) {
@@ -389,17 +401,8 @@ struct NormLinearFn : Function<NormLinearFn> {
         set_extents(*l, x2.size(0), weight);
         l->x_dtype = at::kFloat;   // the normalised tensor times the fp32 gain is an fp32 tensor
         const Tensor gain_c = gain.contiguous();
-        Tensor packed_x = packed_buffer(l->T, I, x2), factor = at::empty({l->T}, x2.options().dtype(at::kFloat)), add2, x_sum;
-        if (args.has_add) {
-            add2 = rows_of(add, I);
-            x_sum = at::empty_like(x2);
-        }
-        check(qm_rmsnorm_quantize_mxfp4(x2.data_ptr(), dtype_code(x2.scalar_type()), ptr(add2), args.has_add ? dtype_code(add2.scalar_type()) : 0,
-                                        args.has_add ? x_sum.data_ptr() : nullptr, gain_c.data_ptr<float>(), (float)args.eps, l->T, I,
-                                        l->a_signs.data(), packed_x.data_ptr(), (size_t)packed_x.numel(), factor.data_ptr<float>(), l->layout,
-                                        stream_of(x2)),
-              "qm_rmsnorm_quantize_mxfp4");
-        if (args.has_add) x2 = x_sum;
+        Tensor factor;
+        Tensor packed_x = normed_into_packed(*l, x2, args.has_add ? rows_of(add, I) : Tensor(), gain_c, args.eps, factor);
         Tensor y = forward_products(*l, Tensor(), weight, autocast_bf16() ? at::kBFloat16 : at::kFloat, packed_x, *args.packed_w);
         if (ctx) {
             ctx->set_materialize_grads(false);
@@ -555,6 +558,61 @@ py::tuple rope_qkv(const Tensor& qkv, const Tensor& table, int64_t n_head) {
     });
 }
 
+// ---- evaluated models: layers behind an RMSNorm whose bf16 result feeds one kernel, which runs in the product's epilogue ------------
+// Nothing is kept for a backward pass.  Packed weights are given; where a kernel does not serve, None comes back and nothing was launched.
+py::object norm_swiglu_linear(const Tensor& x, const optional<Tensor>& add, const Tensor& gain, double eps, const Tensor& w12, const Tensor& packed_w12,
+                              py::handle a_signs12, const Tensor& w, const Tensor& packed_w, py::handle a_signs, int w_hd, py::handle w_signs) {
+    return from_python([&]() -> py::object {
+        const int64_t I = w12.size(1), hidden = w.size(1);
+        const LayerPtr l = make_layer(32, a_signs12, 32, py::none(), 32, py::none(), std::nullopt, std::nullopt);
+        const LayerPtr next = make_layer(32, a_signs, w_hd, w_signs, 32, py::none(), std::nullopt, std::nullopt);
+        const Tensor add_t = or_none(add);
+        require_cuda(x, gain, w12, w, add_t);
+        const c10::OptionalDeviceGuard guard(w12.device());
+        const int64_t T = x.numel() / I;
+        if (!qm_linear_swiglu_serves(T, I, hidden)) return py::none();
+        set_extents(*l, T, w12);
+        set_extents(*next, T, w);
+        if (l->layout != QM_LAYOUT_PADDED || next->layout != QM_LAYOUT_PADDED || l->O != 2 * hidden) return py::none();
+        Tensor x2 = rows_of(x, I), factor;
+        Tensor packed_x = normed_into_packed(*l, x2, add_t.defined() ? rows_of(add_t, I) : Tensor(), gain.contiguous(), eps, factor);
+        Tensor packed_h = packed_buffer(T, hidden, x2), packed = packed_w;
+        check(qm_linear_swiglu_quantize(packed_x.data_ptr(), (size_t)packed_x.numel(), packed_w12.data_ptr(), (size_t)packed_w12.numel(), T, I, hidden,
+                                        next->a_signs.data(), packed_h.data_ptr(), (size_t)packed_h.numel(), stream_of(x2)),
+              "qm_linear_swiglu_quantize");
+        const Tensor y = forward_products(*next, Tensor(), w, at::kBFloat16, packed_h, packed);
+        auto shape = x.sizes().vec();
+        shape.back() = next->O;
+        return py::make_tuple(y.view(shape), add_t.defined() ? x2.view(x.sizes()) : x);
+    });
+}
+py::object norm_rope_linear(const Tensor& x, const optional<Tensor>& add, const Tensor& gain, double eps, const Tensor& weight, const Tensor& packed_w,
+                            py::handle a_signs, const Tensor& table, int64_t n_head) {
+    return from_python([&]() -> py::object {
+        const int64_t I = weight.size(1), C = weight.size(0) / 3, hs = C / n_head;
+        const LayerPtr l = make_layer(32, a_signs, 32, py::none(), 32, py::none(), std::nullopt, std::nullopt);
+        const Tensor add_t = or_none(add);
+        require_cuda(x, gain, weight, table, add_t);
+        const c10::OptionalDeviceGuard guard(weight.device());
+        const int64_t T = x.numel() / I;
+        if (x.dim() != 3 || weight.size(0) != 3 * C || !qm_linear_rope_serves(T, I, C, (int)hs)) return py::none();
+        const int64_t B = x.size(0), S = x.size(1);
+        if (table.dim() != 3 || table.size(0) != S || table.size(1) != hs / 2 || table.size(2) != 2 || !table.is_contiguous() ||
+            reinterpret_cast<uintptr_t>(table.data_ptr()) % 16)
+            return py::none();
+        set_extents(*l, T, weight);
+        if (l->layout != QM_LAYOUT_PADDED) return py::none();
+        Tensor x2 = rows_of(x, I), factor;
+        Tensor packed_x = normed_into_packed(*l, x2, add_t.defined() ? rows_of(add_t, I) : Tensor(), gain.contiguous(), eps, factor);
+        Tensor out[3];
+        for (Tensor& t : out) t = at::empty({B, S, n_head, hs}, x2.options().dtype(at::kBFloat16));
+        check(qm_linear_rope(packed_x.data_ptr(), (size_t)packed_x.numel(), packed_w.data_ptr(), (size_t)packed_w.numel(), T, I, C, (int)hs, S,
+                             table.data_ptr<float>(), out[0].data_ptr(), out[1].data_ptr(), out[2].data_ptr(), stream_of(x2)),
+              "qm_linear_rope");
+        return py::make_tuple(out[0], out[1], out[2], add_t.defined() ? x2.view(x.sizes()) : x);
+    });
+}
+
 // ---- quantizer modules: pseudo-quantized tensor forward, straight-through backward (quantizers/mxfp4.py:15-34,127-146)
 struct QuantizerArgs {
     int hd, mode;
@@ -648,6 +706,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("norm_linear", &norm_linear);
     m.def("swiglu_linear", &swiglu_linear);
     m.def("rope_qkv", &rope_qkv);
+    m.def("norm_swiglu_linear", &norm_swiglu_linear);
+    m.def("norm_rope_linear", &norm_rope_linear);
     m.def("quantizer", &quantizer);
     m.def("sign_flips", &sign_flips);
     m.add_object("transformed", py::reinterpret_steal<py::object>(PyCFunction_New(&transformed_def, nullptr)));

@@ -212,6 +212,21 @@ struct TileProduct {
     int b_e5m2;            // B holds values from expand_e5m2_pair (N % 32 == 0, K % 128 == 0, tiled A)
     const uint8_t* b_wide; // its formats (E5m2Args::wide), or null: eight bits everywhere
 };
+// What a product in an evaluated model is for (gemm_tile.hip).  SwiGLU: B's rows are (up, gate), c receives the tiled codes of
+// Q(silu(up) * gate), quest RTN over Hadamard blocks of 32, [M, N / 2] padded, scales its scale bytes; no clip mask.  RoPE: N is 3 width, c is not used.
+struct TileAfter {
+    uint8_t* scales;
+    uint32_t sign_word;
+    float c;
+    void* q;
+    void* k;
+    void* v;
+    const float* table;   // [seq_len, head_dim / 2, 2]
+    int seq_len, width, head_dim;
+};
+bool gemm_tile_after_serves(const TileProduct& g);
+hipError_t gemm_tile_swiglu(const TileProduct& g, const TileAfter& after, hipStream_t stream);
+hipError_t gemm_tile_rope(const TileProduct& g, const TileAfter& after, hipStream_t stream);
 // the kinds of an eight-bit B are WIDE_256x256 and 1 .. 3
 constexpr int kShortTallSteps = 8;   // see gemm_tile()
 enum TileKind : int { TILE_256x128 = 0, WIDE_256x256 = 0, TILE_128x128 = 1, TILE_128x64 = 2, TILE_64x64 = 3, TILE_64x32 = 4 };
@@ -245,6 +260,7 @@ struct ProductChoice {
 TileProduct make_product(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* b_codes, const uint8_t* b_scales, int64_t M, int64_t N,
                          int64_t K, float alpha, void* c, int a_layout, int b_layout);
 ProductChoice choose_product(const TileProduct& p, int c_dtype, int rot_out_dtype, const void* workspace, size_t workspace_bytes);
+bool product_after_pays(const TileProduct& p, double end, double pass);   // see TileAfter
 hipError_t run_product(const ProductChoice& c, const TileProduct& p, int c_dtype, int rot_out_dtype, void* workspace, hipStream_t stream);
 // The gradient products x and w of a layer in one launch: of which kernel, if that is expected to be faster than running them as cx
 // and cw say; p.mask and *_out as in choose_product.  The results are those of the kernel without K ranges.

@@ -260,6 +260,35 @@ __device__ __forceinline__ void rotate_group(float (&v)[32], float c, uint32_t s
     scale_group(v, c, sign_word);
 }
 
+typedef __bf16 v2bf16 __attribute__((ext_vector_type(2)));
+// round to bf16 and back (round to nearest even, v_cvt_pk_bf16_f32)
+__device__ __forceinline__ void round_pair_to_bf16(float& a, float& b) {
+    const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{a, b}, v2bf16));
+    a = u2f(w << 16);
+    b = u2f(w & 0xffff0000u);
+}
+
+// silu of a bf16 value, to be rounded to bf16: the hardware's exponential and reciprocal, which for every one of the 65536
+// inputs round to the same bf16 value as silu_fixed (tests/test_gpu_fused.py goes through all of them).  A quarter of
+// the denominator keeps its reciprocal a normal number up to 2^128; the last bit on top of it settles the one input
+// (5.9375) whose result lies 2^-24 from a tie.  silu_fixed is some 35 instructions, a polynomial and an IEEE division, and
+// made the producer 92 us at 16384 x 4096 where its bytes take 61; with these six it was 76 (4096 x 1728: 15.2 -> 10.6).
+__device__ __forceinline__ float silu_of_bf16(float x) {
+    const float e = __builtin_amdgcn_exp2f(x * -1.44269504088896340736f);
+    return (x * 0.25f) * __builtin_amdgcn_rcpf(__builtin_fmaf(e, 0.25f, 0x1.000002p-2f));
+}
+// silu(up) * gate of a group in bf16, rounded after each operation as bf16 tensors are; the product in `up`
+__device__ __forceinline__ void swiglu_group_bf16(float (&up)[32], const float (&gate)[32]) {
+#pragma unroll
+    for (int i = 0; i < 32; ++i) up[i] = silu_of_bf16(up[i]);
+#pragma unroll
+    for (int i = 0; i < 32; i += 2) round_pair_to_bf16(up[i], up[i + 1]);
+#pragma unroll
+    for (int i = 0; i < 32; ++i) up[i] = up[i] * gate[i];
+#pragma unroll
+    for (int i = 0; i < 32; i += 2) round_pair_to_bf16(up[i], up[i + 1]);
+}
+
 }  // namespace
 
 }  // namespace qm

@@ -1127,14 +1127,6 @@ hipError_t requantize_transposed_dense(const uint8_t* codes_in, const uint8_t* s
 
 namespace {
 
-typedef __bf16 v2bf16 __attribute__((ext_vector_type(2)));
-// round to bf16 and back (round to nearest even, v_cvt_pk_bf16_f32)
-__device__ __forceinline__ void round_pair_to_bf16(float& a, float& b) {
-    const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{a, b}, v2bf16));
-    a = u2f(w << 16);
-    b = u2f(w & 0xffff0000u);
-}
-
 // TA = void: plain.  Otherwise the norm's input is x + add (the residual sum in front of the norm, src/models/llama.py:
 // 170-171), formed here in T's arithmetic and written to xsum, which the rest of the model continues with.
 template <typename T, typename TA = void>
@@ -1270,15 +1262,6 @@ struct RmsNormProducer {
     }
 };
 
-// silu of a bf16 value, to be rounded to bf16: the hardware's exponential and reciprocal, which for every one of the 65536
-// inputs round to the same bf16 value as silu_fixed (tests/test_gpu_fused.py goes through all of them).  A quarter of
-// the denominator keeps its reciprocal a normal number up to 2^128; the last bit on top of it settles the one input
-// (5.9375) whose result lies 2^-24 from a tie.  silu_fixed is some 35 instructions, a polynomial and an IEEE division, and
-// made the producer 92 us at 16384 x 4096 where its bytes take 61; with these six it was 76 (4096 x 1728: 15.2 -> 10.6).
-__device__ __forceinline__ float silu_of_bf16(float x) {
-    const float e = __builtin_amdgcn_exp2f(x * -1.44269504088896340736f);
-    return (x * 0.25f) * __builtin_amdgcn_rcpf(__builtin_fmaf(e, 0.25f, 0x1.000002p-2f));
-}
 __global__ void silu_of_bf16_kernel(uint16_t* __restrict__ out) {
     const uint32_t x = blockIdx.x * 256 + threadIdx.x;
     out[x] = f32_to_bf16(silu_of_bf16(u2f(x << 16)));
@@ -1343,17 +1326,11 @@ struct SwiGluProducer {
             load_group<T>(h12 + row * 2 * cols + g * 32, v);
             load_group<T>(h12 + row * 2 * cols + cols + g * 32, gate);
         }
-#pragma unroll
-        for (int i = 0; i < 32; ++i) v[i] = sizeof(T) == 2 ? silu_of_bf16(v[i]) : silu_fixed(v[i]);
-        if constexpr (sizeof(T) == 2) {  // a bf16 tensor rounds after each op
-#pragma unroll
-            for (int i = 0; i < 32; i += 2) round_pair_to_bf16(v[i], v[i + 1]);
-        }
-#pragma unroll
-        for (int i = 0; i < 32; ++i) v[i] = v[i] * gate[i];
         if constexpr (sizeof(T) == 2) {
+            swiglu_group_bf16(v, gate);
+        } else {
 #pragma unroll
-            for (int i = 0; i < 32; i += 2) round_pair_to_bf16(v[i], v[i + 1]);
+            for (int i = 0; i < 32; ++i) v[i] = silu_fixed(v[i]) * gate[i];
         }
     }
 };

@@ -97,6 +97,77 @@ def swiglu_linear(layer, h12):
     return layer(F.silu(up) * gate)
 
 
+def _evaluated(norm, layers, x, add):
+    """[(weight, its packed form, activation and weight quantizer)] of the layers behind an RMSNorm where nothing asks for a gradient, the
+    products are bf16 ones under autocast, and every weight's packed form is kept and up to date; else None."""
+    if not (x.is_cuda and torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16) or one_node.transformed() or torch.compiler.is_compiling():
+        return None
+    gain = getattr(norm, "weight", None)
+    tensors = [x, gain] if add is None else [x, gain, add]
+    if not (isinstance(gain, torch.Tensor) and gain.dtype == torch.float32 and x.dtype in _KERNEL_DTYPES and 0 < x.shape[-1] <= 8192 and 0 < x.numel() < 1 << 27):
+        return None
+    if add is not None and not (x.dtype == torch.float32 and add.dtype in _KERNEL_DTYPES and add.shape == x.shape):
+        return None
+    if any(t.device != x.device for t in tensors):
+        return None
+    found = []
+    for layer in layers:
+        parts = _fusable_parts(layer, x)
+        if parts is None or layer.packed_weight_cache is None or parts[0].device != x.device:
+            return None
+        weight, a_q, w_q, g_q = parts
+        if w_q._dense is not None:
+            return None
+        key, _ = _cached_weight(x, weight, a_q, w_q, g_q, _KEY_ONLY)
+        if layer.packed_weight_cache.key != key:
+            return None
+        found.append((weight, layer.packed_weight_cache, a_q, w_q))
+        tensors.append(weight)
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+        return None
+    return found
+
+
+class _KeyOnly:
+    @staticmethod
+    def get(key):
+        return None
+
+
+_KEY_ONLY = _KeyOnly()
+
+
+def rmsnorm_swiglu_linear(norm, w12, c_proj, x, add=None):
+    """(c_proj(silu(up) * gate), x [+ add]) with (up, gate) = w12(norm(x [+ add])): ``rmsnorm_linear`` and ``swiglu_linear``.  In an
+    evaluation under bf16 autocast with packed weights kept, w12's product goes on to the SwiGLU and the quantizer in its epilogue and
+    its result is never written; the same bits."""
+    parts = _evaluated(norm, (w12, c_proj), x, add)
+    if parts is not None and w12.out_features == 2 * c_proj.in_features:
+        (w, cache, a_q, _), (w2, cache2, a_q2, w_q2) = parts
+        out = _lib.host().norm_swiglu_linear(x, add, norm.weight, norm.eps, w, cache.buffer, a_q.sign_bits, w2, cache2.buffer, a_q2.sign_bits, w_q2.hadamard_dim,
+                                             w_q2.sign_bits)
+        if out is not None:
+            cache.hits += 1
+            cache2.hits += 1
+            return out
+    h12, x = rmsnorm_linear(norm, w12, x, pass_input=True, add=add)
+    return swiglu_linear(c_proj, h12), x
+
+
+def rmsnorm_rope_linear(norm, c_attn, x, table, n_head, add=None):
+    """(q, k, v, x [+ add]): ``rmsnorm_linear`` and ``rope_qkv``, in an evaluation as ``rmsnorm_swiglu_linear`` with the split and the rotary
+    embedding in c_attn's epilogue."""
+    parts = _evaluated(norm, (c_attn,), x, add)
+    if parts is not None and table.dtype == torch.float32 and c_attn.out_features % (3 * n_head) == 0:
+        (w, cache, a_q, _), = parts
+        out = _lib.host().norm_rope_linear(x, add, norm.weight, norm.eps, w, cache.buffer, a_q.sign_bits, table, n_head)
+        if out is not None:
+            cache.hits += 1
+            return out
+    qkv, x = rmsnorm_linear(norm, c_attn, x, pass_input=True, add=add)
+    return (*rope_qkv(qkv, table, n_head), x)
+
+
 def cross_entropy(logits, targets, ignore_index=-1):
     """F.cross_entropy(logits, targets, ignore_index=ignore_index) of logits [rows, classes].  Where nothing asks for a
     gradient and the result is an fp32 one (fp32 logits, or bf16 ones under autocast) the logits are read once by a kernel of

@@ -21,7 +21,7 @@ import torch.nn.functional as F
 from torch.nn.attention import SDPBackend, sdpa_kernel
 
 from .backward import BACKWARD_SCHEMES
-from .fused import cross_entropy, rmsnorm_linear, rope_qkv, swiglu_linear
+from .fused import cross_entropy, rmsnorm_rope_linear, rmsnorm_swiglu_linear
 from .linear import QuantizedLinear
 from .quantizers import QUANTIZER_CLASSES
 
@@ -133,8 +133,7 @@ class LlamaMLP(nn.Module):
         """`norm`: the block's RMSNorm, applied to x (+ `add`, the attention branch's output) here, fused into w12's
         quantizer, instead of by the caller."""
         if norm is not None:   # returns (mlp output, x + add for the residual sum)
-            h12, x = rmsnorm_linear(norm, self.w12, x, pass_input=True, add=add)
-            return swiglu_linear(self.c_proj, h12), x
+            return rmsnorm_swiglu_linear(norm, self.w12, self.c_proj, x, add=add)
         up, gate = self.w12(x).split(self.hidden_dim, dim=-1)
         return self.c_proj(F.silu(up) * gate)
 
@@ -161,14 +160,10 @@ class LlamaAttention(nn.Module):
     def forward(self, x, table, norm=None, add=None):
         B, T, C = x.shape
         hs = C // self.n_head
-        if norm is None:
-            qkv = self.c_attn(x)
+        if norm is not None:   # the fused path: split, rotate and convert in one kernel, or in the projection's
+            q, k, v, x = rmsnorm_rope_linear(norm, self.c_attn, x, table, self.n_head, add=add)
         else:
-            qkv, x = rmsnorm_linear(norm, self.c_attn, x, pass_input=True, add=add)
-        if norm is not None:   # the fused path: split, rotate and convert in one kernel
-            q, k, v = rope_qkv(qkv, table, self.n_head)
-        else:
-            q, k, v = qkv.split(self.n_embd, dim=2)
+            q, k, v = self.c_attn(x).split(self.n_embd, dim=2)
             q, k = apply_rotary(q.view(B, T, self.n_head, hs), k.view(B, T, self.n_head, hs), table)
             v = v.view(B, T, self.n_head, hs)
         q, k, v = q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2)

@@ -1,0 +1,118 @@
+"""Products of an evaluated model whose epilogue goes on with their result."""
+import ctypes
+
+import pytest
+import torch
+
+from tests.util import make_input
+
+pytestmark = pytest.mark.gpu
+BF16, LAYOUT_PADDED = torch.bfloat16, 2
+
+
+def packed(K, monkeypatch, x, w):
+    """The padded operands of a layer, as its forward pass leaves them, and its bf16 result."""
+    monkeypatch.setattr(K, "_layout", lambda tiled: LAYOUT_PADDED)
+    y, px, pw = K.linear_forward(x, w, 32, 0x5A5A5A5A, 32, 0x0F0F1234, BF16, True)
+    return y, px, pw
+
+
+def codes_and_scales(K, buffer, rows, cols):
+    off = (ctypes.c_size_t * 3)()
+    from quartet_amd import _lib
+    assert _lib.lib().qm_packed_operand_offsets(rows, cols, off) == 0
+    padded = (cols + 127) // 128 * 128
+    tiles = buffer[off[0]: off[0] + (rows + 15) // 16 * 16 * padded // 2].view((rows + 15) // 16, padded // 128, 16, 64)
+    codes = tiles.permute(0, 2, 1, 3).reshape(-1, padded // 2)[:rows]
+    return codes, buffer[off[1]: off[1] + rows * padded // 32].view(rows, padded // 32)
+
+
+# one tile and several, ragged rows, an odd and an even number of groups, whole tiles of padding behind the columns, fewer K steps than four
+@pytest.mark.parametrize("T,I,hidden", [(65, 96, 32), (127, 640, 96), (129, 512, 1696), (384, 544, 1728), (1000, 640, 160), (513, 1536, 4096)])
+@pytest.mark.parametrize("signs", [None, 0x9E3779B9])
+def test_swiglu_and_quantizer_in_the_product(monkeypatch, T, I, hidden, signs):
+    """Codes and scales, padding included, bit for bit those of the product, then the producer."""
+    print(f"case product with SwiGLU {T}x{I}x2*{hidden}", flush=True)
+    from quartet_amd import _lib, kernels as K
+    x = make_input(T, I, BF16, seed=1, outlier_frac=0.01).to("cuda:0")
+    w = make_input(2 * hidden, I, BF16, seed=2, outlier_frac=0, scale=0.05).to("cuda:0")
+    h12, px, pw = packed(K, monkeypatch, x, w)
+    want = codes_and_scales(K, K.swiglu_quantize(h12, signs, True), T, hidden)
+    out = K.packed_operand_buffer(T, hidden, x.device).fill_(0xA5)
+    rc = _lib.lib().qm_linear_swiglu_quantize(px.data_ptr(), px.numel(), pw.data_ptr(), pw.numel(), T, I, hidden, K.sign_words(signs), out.data_ptr(), out.numel(), None)
+    _lib.check(rc, "qm_linear_swiglu_quantize")
+    for got, ref in zip(codes_and_scales(K, out, T, hidden), want):
+        assert torch.equal(got, ref)
+
+
+# sequences shorter and longer than a pass over a tile's rows, of one token, rows over the tile's edge; heads narrower than a tile and wider
+@pytest.mark.parametrize("B,S,I,heads,hs", [(8, 512, 640, 5, 128), (3, 43, 96, 3, 8), (130, 1, 160, 2, 64), (5, 17, 512, 1, 136), (9, 15, 256, 4, 72)])
+def test_rotary_split_in_the_product(monkeypatch, B, S, I, heads, hs):
+    print(f"case product with rotary split {B}x{S}x{I} heads={heads}x{hs}", flush=True)
+    from quartet_amd import _lib, kernels as K
+    from quartet_amd.llama import rotary_table
+    T, C = B * S, heads * hs
+    x = make_input(T, I, BF16, seed=1, outlier_frac=0.01).to("cuda:0")
+    w = make_input(3 * C, I, BF16, seed=2, outlier_frac=0, scale=0.05).to("cuda:0")
+    table = rotary_table(hs, S).to("cuda:0").contiguous()
+    qkv, px, pw = packed(K, monkeypatch, x, w)
+    want = [torch.empty(T, C, dtype=BF16, device="cuda:0") for _ in range(3)]
+    got = [torch.full_like(t, float("nan")) for t in want]
+    L = _lib.lib()
+    _lib.check(L.qm_rope_split_qkv(qkv.data_ptr(), 0, T, S, C, hs, table.data_ptr(), *[t.data_ptr() for t in want], 0, None), "qm_rope_split_qkv")
+    rc = L.qm_linear_rope(px.data_ptr(), px.numel(), pw.data_ptr(), pw.numel(), T, I, C, hs, S, table.data_ptr(), *[t.data_ptr() for t in got], None)
+    _lib.check(rc, "qm_linear_rope")
+    for g, r in zip(got, want):
+        assert torch.equal(g, r)
+
+
+def test_what_those_products_refuse():
+    from quartet_amd import _lib
+    L = _lib.lib()
+    b = torch.empty(1 << 22, dtype=torch.uint8, device="cuda:0")
+    p, n = b.data_ptr(), b.numel()
+    swiglu = lambda T=128, I=128, hidden=64, px=p, size=n, out=p: L.qm_linear_swiglu_quantize(px, size, p, n, T, I, hidden, None, out, n, None)
+    assert swiglu(T=64) == -1 and swiglu(I=100) == -1 and swiglu(hidden=48) == -1 and swiglu(px=None) == -1 and swiglu(size=64) == -1 and swiglu(out=p + 16) == -1
+    rope = lambda T=128, I=128, C=64, hs=8, S=16, q=p, table=p: L.qm_linear_rope(p, n, p, n, T, I, C, hs, S, table, q, p, p, None)
+    assert rope(T=64) == -1 and rope(hs=12) == -1 and rope(C=60, hs=8) == -1 and rope(S=0) == -1 and rope(q=None) == -1 and rope(table=p + 4) == -1
+    assert L.qm_linear_swiglu_serves(64, 640, 1728) == 0 and L.qm_linear_rope_serves(4096, 640, 640, 12) == 0
+
+
+@pytest.mark.parametrize("add_dtype", [None, BF16, torch.float32])
+def test_an_evaluated_model_is_the_same_model(add_dtype):
+    """With packed weights kept, without (two launches instead of one), and the residual sum: the same bits; and gradients go on asking
+    for the path that keeps what they need."""
+    import quartet_amd as q
+    from quartet_amd.fused import rmsnorm_rope_linear, rmsnorm_swiglu_linear
+    from quartet_amd.llama import Llama, llama_30m, rotary_table
+    torch.manual_seed(3)
+    with torch.device("cuda"):
+        model = Llama(llama_30m(n_layer=1, sequence_length=128)).eval()
+    block = model.transformer.h[0]
+    x = make_input(288, 640, torch.float32, seed=5).view(3, 96, 640).to("cuda:0")
+    add = None if add_dtype is None else make_input(288, 640, add_dtype, seed=6).view(3, 96, 640).to("cuda:0")
+    table = rotary_table(128, 96).to("cuda:0")
+
+    def run():
+        with torch.no_grad(), torch.autocast("cuda", dtype=BF16):
+            return (*rmsnorm_swiglu_linear(block.ln_2, block.mlp.w12, block.mlp.c_proj, x, add=add),
+                    *rmsnorm_rope_linear(block.ln_1, block.attn.c_attn, x, table, 5, add=add))
+    want = run()
+    q.enable_packed_weight_cache(model)
+    run()                                   # quantizes the weights
+    got = run()
+    assert all(m.packed_weight_cache.hits == 1 for m in (block.mlp.w12, block.mlp.c_proj, block.attn.c_attn))
+    for g, r in zip(got, want):
+        assert g.dtype == r.dtype and g.shape == r.shape and torch.equal(g, r)
+    with torch.no_grad():
+        block.mlp.w12.weight.mul_(2.0)      # a kept form that is out of date is not used
+        changed = run()[0]
+        q.enable_packed_weight_cache(model, False)
+    assert torch.equal(changed, run()[0]) and not torch.equal(changed, want[0])
+    xg = x.clone().requires_grad_(True)
+    q.enable_packed_weight_cache(model)
+    for _ in range(2):
+        with torch.autocast("cuda", dtype=BF16):
+            y, _ = rmsnorm_swiglu_linear(block.ln_2, block.mlp.w12, block.mlp.c_proj, xg, add=add)
+        y.float().sum().backward()
+    assert torch.isfinite(xg.grad).all() and block.mlp.w12.weight.grad is not None
