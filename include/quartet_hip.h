@@ -419,6 +419,14 @@ int qm_linear_rope_serves(int64_t T, int64_t I, int64_t n_embd, int head_dim);
 int qm_linear_rope(const void* packed_x, size_t packed_x_bytes, const void* packed_w, size_t packed_w_bytes, int64_t T, int64_t I,
                    int64_t n_embd, int head_dim, int64_t seq_len, const float* table, void* q, void* k, void* v, void* stream);
 
+/*
+ * RMSNorm in front of an unquantized layer (src/models/llama.py:64-75; the model's last one) with the residual sum before it:
+ * out [rows, cols] of out_dtype = (x + add) / sqrt(mean((x + add)^2) + eps) * gain, in fp32.  x fp32, add NULL, bf16 or fp32, gain fp32
+ * [cols]; cols % 4 == 0, cols <= 4096; 16-byte aligned.
+ */
+int qm_rmsnorm(const float* x, const void* add, int add_dtype, const float* gain, float eps, int64_t rows, int64_t cols, void* out,
+               int out_dtype, void* stream);
+
 /* Test aid: silu as the SwiGLU producer evaluates it for bf16 tensors, of every bf16 bit pattern: out[65536] */
 int qm_diag_silu_bf16(uint16_t* out, void* stream);
 

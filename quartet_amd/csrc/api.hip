@@ -997,6 +997,16 @@ int qm_rope_merge_qkv_grad(const void* dq, const void* dk, const void* dv, int g
                     "qm_rope_merge_qkv_grad");
 }
 
+int qm_rmsnorm(const float* x, const void* add, int add_dtype, const float* gain, float eps, int64_t rows, int64_t cols, void* out, int out_dtype, void* stream) {
+    if (!valid_dtype(out_dtype) || (add && !valid_dtype(add_dtype))) return fail(QM_ERR_INVALID, "qm_rmsnorm: dtypes must be QM_BF16/QM_F32");
+    if (rows < 0 || rows >= (1ll << 32) || cols <= 0 || cols % 4 || cols > 4096)
+        return fail(QM_ERR_INVALID, "qm_rmsnorm: need 0 <= rows < 2^32 and cols a multiple of 4 in [4, 4096] (got [%lld, %lld])", (long long)rows, (long long)cols);
+    if (rows == 0) return 0;
+    if (!x || !gain || !out) return fail(QM_ERR_INVALID, "qm_rmsnorm: x, gain and out must be non-null");
+    if (!aligned(x, 16) || !aligned(add, 16) || !aligned(gain, 16) || !aligned(out, 16)) return fail(QM_ERR_UNALIGNED, "qm_rmsnorm: tensors need 16-byte alignment");
+    return from_hip(qm::rmsnorm_rows(x, add, add_dtype, gain, eps, rows, cols, out, out_dtype, reinterpret_cast<hipStream_t>(stream)), "qm_rmsnorm");
+}
+
 int qm_diag_silu_bf16(uint16_t* out, void* stream) {
     if (!out) return fail(QM_ERR_INVALID, "qm_diag_silu_bf16: out must be non-null");
     return from_hip(qm::silu_of_bf16_table(out, reinterpret_cast<hipStream_t>(stream)), "qm_diag_silu_bf16");

@@ -286,6 +286,10 @@ hipError_t gemm_tile_phases(const uint8_t* a_codes, const uint8_t* a_scales, con
 int mfma_only_blocks();
 hipError_t mfma_only(const uint8_t* operands, float* sink, int iters, hipStream_t stream);
 
+// RMSNorm of (x + add) (norm.hip): fp32 x, add null, bf16 or fp32, out bf16 or fp32; cols % 4 == 0, cols <= 4096
+hipError_t rmsnorm_rows(const float* x, const void* add, int add_dtype, const float* gain, float eps, int64_t rows, int64_t cols, void* out, int out_dtype,
+                        hipStream_t stream);
+
 // mean cross-entropy over the rows whose target is not `ignore` (loss.hip); losses: scratch, one float per row
 hipError_t cross_entropy_mean(const void* logits, int dtype, const int64_t* targets, int64_t rows, int64_t classes, int64_t ignore,
                               float* losses, float* loss, hipStream_t stream);

@@ -13,7 +13,7 @@ import torch
 import torch.nn.functional as F
 
 from . import _lib, kernels, one_node
-from .linear import QuantizedLinear, _cached_weight, _dense
+from .linear import _GLOBAL_HOOKS, QuantizedLinear, _cached_weight, _dense, _watched
 from .one_node import as_one_node
 
 _KERNEL_DTYPES = (torch.float32, torch.bfloat16)
@@ -166,6 +166,26 @@ def rmsnorm_rope_linear(norm, c_attn, x, table, n_head, add=None):
             return out
     qkv, x = rmsnorm_linear(norm, c_attn, x, pass_input=True, add=add)
     return (*rope_qkv(qkv, table, n_head), x)
+
+
+def rmsnorm(norm, x, add=None):
+    """norm(x [+ add]) in front of a plain linear layer.  In an evaluation under bf16 autocast in one pass, rounded to the bf16 that autocast
+    hands the layer."""
+    plain = (type(x) is torch.Tensor and x.is_cuda and x.dtype == torch.float32 and torch.is_autocast_enabled("cuda")
+             and torch.get_autocast_dtype("cuda") == torch.bfloat16 and not (one_node.transformed() or torch.compiler.is_compiling()))
+    if plain:
+        from .llama import RMSNorm
+        plain = type(norm) is RMSNorm and not (any(_GLOBAL_HOOKS) or _watched(norm))
+    if plain:
+        gain, cols = norm.weight, x.shape[-1]
+        watched = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, add, gain))
+        if (not watched and gain.dtype == torch.float32 and gain.shape == (cols,) and gain.device == x.device and 0 < cols <= 4096
+                and cols % 4 == 0 and 0 < x.numel() < 1 << 31
+                and (add is None or (add.dtype in _KERNEL_DTYPES and add.shape == x.shape and add.device == x.device))):
+            rows = [t if t is None else t.reshape(-1, cols).contiguous() for t in (x, add)]
+            if not any(t is not None and t.data_ptr() % 16 for t in (*rows, gain)):
+                return kernels.rmsnorm(rows[0], gain.contiguous(), norm.eps, rows[1], torch.bfloat16).view(x.shape)
+    return norm(x if add is None else x + add)
 
 
 def cross_entropy(logits, targets, ignore_index=-1):

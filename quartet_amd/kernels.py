@@ -349,6 +349,19 @@ def rmsnorm_quantize(x2, gain, eps, signs, tiled, add=None):
     return (packed, factor) if add is None else (packed, factor, x_sum)
 
 
+def rmsnorm(x2, gain, eps, add=None, out_dtype=torch.float32):
+    """rmsnorm(x2 [+ add]) * gain of fp32 x2 [rows, cols] in out_dtype."""
+    _require_cuda(x2, gain, add)
+    assert x2.is_contiguous() and x2.dtype == torch.float32 and gain.is_contiguous() and gain.dtype == torch.float32 and gain.shape == (x2.shape[1],)
+    assert add is None or (add.is_contiguous() and add.shape == x2.shape)
+    out = torch.empty(x2.shape, dtype=out_dtype, device=x2.device)
+    with torch.cuda.device(x2.device):
+        rc = _lib.lib().qm_rmsnorm(_ptr(x2), _ptr(add), _dtype_code(add.dtype) if add is not None else 0, _ptr(gain), float(eps), x2.shape[0],
+                                   x2.shape[1], _ptr(out), _dtype_code(out_dtype), _stream())
+    _lib.check(rc, "qm_rmsnorm")
+    return out
+
+
 def swiglu_quantize(h12, signs, tiled):
     """Q(silu(up) * gate) of h12 [rows, 2 hidden] = (up, gate) without writing the product: packed operand buffer."""
     _require_cuda(h12)

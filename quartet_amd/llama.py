@@ -21,7 +21,7 @@ import torch.nn.functional as F
 from torch.nn.attention import SDPBackend, sdpa_kernel
 
 from .backward import BACKWARD_SCHEMES
-from .fused import cross_entropy, rmsnorm_rope_linear, rmsnorm_swiglu_linear
+from .fused import cross_entropy, rmsnorm, rmsnorm_rope_linear, rmsnorm_swiglu_linear
 from .linear import QuantizedLinear
 from .quantizers import QUANTIZER_CLASSES
 
@@ -244,9 +244,7 @@ class Llama(nn.Module):
             else:
                 x = block(x if pending is None else x + pending, table)
                 pending = None
-        if pending is not None:
-            x = x + pending
-        x = self.transformer.ln_f(x)
+        x = rmsnorm(self.transformer.ln_f, x, pending)
         if targets is not None:
             logits = self.lm_head(x)
             loss = cross_entropy(logits.view(-1, logits.size(-1)), targets.view(-1), ignore_index=-1)

@@ -1,6 +1,7 @@
-"""Products of an evaluated model whose epilogue goes on with their result."""
+"""Products of an evaluated model whose epilogue goes on with their result, and its last norm."""
 import ctypes
 
+import numpy as np
 import pytest
 import torch
 
@@ -116,3 +117,40 @@ def test_an_evaluated_model_is_the_same_model(add_dtype):
             y, _ = rmsnorm_swiglu_linear(block.ln_2, block.mlp.w12, block.mlp.c_proj, xg, add=add)
         y.float().sum().backward()
     assert torch.isfinite(xg.grad).all() and block.mlp.w12.weight.grad is not None
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 4), (5, 640), (4, 768), (7, 772), (3, 1536), (9, 1540), (2, 4096)])
+@pytest.mark.parametrize("add_dtype", [None, BF16, torch.float32])
+@pytest.mark.parametrize("out_dtype", [BF16, torch.float32])
+def test_last_norm(rows, cols, add_dtype, out_dtype):
+    """Against float64: the fp32 sum of at most 16 + 6 additions in a row, a root, a quotient and three products: 2^-24 each, 25 of them;
+    bf16 results one rounding to eight significant bits more, 2^-8."""
+    from quartet_amd import kernels as K
+    x = make_input(rows, cols, torch.float32, seed=rows + cols)
+    add = None if add_dtype is None else make_input(rows, cols, add_dtype, seed=3)
+    gain = 1 + 0.1 * torch.randn(cols, generator=torch.Generator().manual_seed(1))
+    s = (x if add is None else x + add.float()).double()
+    want = s / torch.sqrt((s * s).mean(-1, keepdim=True) + 1e-5) * gain.double()
+    got = K.rmsnorm(x.to("cuda:0"), gain.to("cuda:0"), 1e-5, None if add is None else add.to("cuda:0"), out_dtype).cpu()
+    assert got.dtype == out_dtype
+    err = ((got.double() - want).abs() / want.abs().clamp_min(1e-30)).numpy()
+    assert np.all(err <= 25 * 2.0 ** -24 + (2.0 ** -8 if out_dtype == BF16 else 0.0))
+
+
+def test_last_norm_of_a_model_takes_the_module_where_somebody_listens_or_asks_for_gradients():
+    from quartet_amd.fused import rmsnorm
+    from quartet_amd.llama import RMSNorm
+    norm = RMSNorm(640).to("cuda:0")
+    x = torch.randn(2, 70, 640, device="cuda:0")
+    with torch.autocast("cuda", dtype=BF16):
+        with torch.no_grad():
+            one = rmsnorm(norm, x)
+            assert one.dtype == BF16 and float((one.float() - norm(x)).abs().max()) < 2.0 ** -6
+            seen = []
+            handle = norm.register_forward_hook(lambda *a: seen.append(1))
+            assert torch.equal(rmsnorm(norm, x), norm(x)) and len(seen) == 2
+            handle.remove()
+        y = rmsnorm(norm, x)
+        assert y.dtype == torch.float32 and y.requires_grad
+    with torch.no_grad():
+        assert torch.equal(rmsnorm(norm, x, x), norm(x + x))
