@@ -330,6 +330,8 @@ int qm_linear_backward_seeded(const void* e, int e_dtype, int64_t T, int64_t I, 
  * operands in bf16 with fp32 accumulation, whatever the operands' scales.
  */
 size_t qm_linear_backward_error_workspace_bytes(int64_t T, int64_t I, int64_t O);
+/* whether its two products run in one launch (1 / 0; forward quantizers with the same Hadamard block and signs) */
+int qm_linear_backward_error_in_one_launch(int64_t T, int64_t I, int64_t O, int hd, int gw_dtype);
 int qm_linear_backward_error(const void* e, int e_dtype, int64_t T, int64_t I, int64_t O, const void* packed_x, const void* packed_w,
                              int hd_x, const uint32_t* signs_x, int hd_w, const uint32_t* signs_w, int hd_g,
                              const uint32_t* signs_g, int g_mode, const uint64_t* seeds, int x_scale_dtype, int w_scale_dtype,

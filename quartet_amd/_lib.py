@@ -55,6 +55,7 @@ EXPORTS = (
     "qm_linear_rope_serves",
     "qm_linear_rope",
     "qm_rmsnorm",
+    "qm_linear_backward_error_in_one_launch",
     "qm_linear_decode",
     "qm_cross_entropy",
     "qm_diag_silu_bf16",
@@ -152,6 +153,8 @@ def lib():
     L.qm_linear_rope.argtypes = [vp, ctypes.c_size_t, vp, ctypes.c_size_t, i64, i64, i64, i32, i64, vp, vp, vp, vp, vp]
     L.qm_rmsnorm.restype = i32
     L.qm_rmsnorm.argtypes = [vp, vp, i32, vp, f32, i64, i64, vp, i32, vp]
+    L.qm_linear_backward_error_in_one_launch.restype = i32
+    L.qm_linear_backward_error_in_one_launch.argtypes = [i64, i64, i64, i32, i32]
     L.qm_linear_decode.restype = i32
     L.qm_linear_decode.argtypes = [vp, i32, i64, i64, i64, vp, vp, ctypes.c_size_t, vp, i32, vp]
     L.qm_cross_entropy.restype = i32

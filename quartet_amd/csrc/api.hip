@@ -430,6 +430,12 @@ bool seed_base_served(int codes_layout, int64_t T, int64_t I, int64_t O, int hd_
            O % 128 == 0;
 }
 extern "C++" {
+// Both products of the error-only scheme on whole 256 x 256 tiles: one grid for them.  us per step, two launches against one: 4096^3 174 -> 169.6,
+// 2048 x 8192 x 4096 218.8 -> 215; what is gained is one start and one last wave of tiles.
+bool wide_pair(const qm::TileProduct& x, const qm::ProductChoice& cx, const qm::TileProduct& w, const qm::ProductChoice& cw) {
+    const auto whole = [](const qm::ProductChoice& c) { return c.path == qm::ProductChoice::TILE && c.kind == qm::WIDE_256x256 && c.splits == 1 && c.rotates; };
+    return whole(cx) && whole(cw) && qm::gemm_wide_pair_serves(x, w);
+}
 // A gradient product of the backward pass and the kernel that serves it by itself: with the masked inverse rotation of the forward
 // quantizer (into final_dst) where that kernel applies it, otherwise without (into plain.c)
 struct GradProduct {
@@ -642,6 +648,22 @@ size_t qm_linear_backward_error_workspace_bytes(int64_t T, int64_t I, int64_t O)
     return error_layout(T, I, O).total;
 }
 
+int qm_linear_backward_error_in_one_launch(int64_t T, int64_t I, int64_t O, int hd, int gw_dtype) {
+    if (T <= 0 || I <= 0 || O <= 0 || I % 32 || O % 32 || T % 32 || I >= (1 << 23) || O >= (1 << 23) || T >= (1 << 23) || !valid_hd(hd) || I % hd || !valid_dtype(gw_dtype)) return 0;
+    uint8_t* at = reinterpret_cast<uint8_t*>((uintptr_t)256);   // nothing is read
+    const size_t ws = error_layout(T, I, O).gemm_ws_bytes;
+    const auto product = [&](int64_t M, int64_t R) {
+        qm::TileProduct p = qm::make_product(at, at, at, at, M, I, qm::padded_cols(R), 1.0f, at, QM_LAYOUT_TILED, QM_LAYOUT_TILED);
+        p.b_e5m2 = 1;
+        p.b_wide = qm::six_bits_serve(qm::padded_cols(R)) ? at : nullptr;
+        p.mask = at;
+        p.hd = hd;
+        return p;
+    };
+    const qm::TileProduct x = product(T, O), w = product(O, T);
+    return wide_pair(x, qm::choose_product(x, QM_BF16, QM_BF16, ws ? at : nullptr, ws), w, qm::choose_product(w, QM_BF16, gw_dtype, ws ? at : nullptr, ws)) ? 1 : 0;
+}
+
 int qm_linear_backward_error(const void* e, int e_dtype, int64_t T, int64_t I, int64_t O, const void* packed_x, const void* packed_w,
                              int hd_x, const uint32_t* signs_x, int hd_w, const uint32_t* signs_w, int hd_g, const uint32_t* signs_g,
                              int g_mode, const uint64_t* seeds, int x_scale_dtype, int w_scale_dtype, void* workspace,
@@ -678,8 +700,7 @@ int qm_linear_backward_error(const void* e, int e_dtype, int64_t T, int64_t I, i
     const float alpha = (float)(1.0 / 0.75);
     void* gws = wl.gemm_ws_bytes ? k + wl.gemm_ws : nullptr;
     // one gradient: the product, then the masked inverse rotation of the forward quantizer, in the product's kernel where that is cheaper
-    const auto gradient = [&](size_t ac, size_t as, const qm::E5m2Args& b, int64_t M, void* out, int out_dtype, int hd, const uint32_t* signs,
-                              int scale_dtype, const uint8_t* mask, size_t plain) {
+    const auto product_of = [&](size_t ac, size_t as, const qm::E5m2Args& b, int64_t M, void* out, int hd, const uint32_t* signs, int scale_dtype, const uint8_t* mask) {
         qm::TileProduct p = qm::make_product(k + ac, k + as, b.values, b.scales, M, I, qm::padded_cols(b.R), alpha, out, QM_LAYOUT_TILED, QM_LAYOUT_TILED);
         p.b_e5m2 = 1;
         p.b_wide = b.wide;
@@ -687,17 +708,29 @@ int qm_linear_backward_error(const void* e, int e_dtype, int64_t T, int64_t I, i
         p.hd = hd;
         p.signs = make_signs(signs, hd);
         p.rot_c = qm::hadamard_scale(hd, scale_dtype);
-        const qm::ProductChoice c = qm::choose_product(p, QM_BF16, out_dtype, gws, wl.gemm_ws_bytes);
-        if (c.rotates) return qm::run_product(c, p, QM_BF16, out_dtype, gws, hs);
-        p.mask = nullptr;
-        p.c = k + plain;
-        const hipError_t e1 = qm::run_product(c, p, QM_BF16, QM_BF16, gws, hs);
-        return e1 != hipSuccess ? e1 : qm::masked_hadamard_bwd(p.c, QM_BF16, M, I, hd, scale_dtype, p.signs, mask, out, out_dtype, out_dtype != QM_BF16, hs);
+        return p;
     };
-    rc = from_hip(gradient(wl.ec, wl.es, aw, T, gx, QM_BF16, hd_x, signs_x, x_scale_dtype, px + lx.m, wl.plain), "qm_linear_backward_error");
-    if (rc) return rc;
-    rc = from_hip(gradient(wl.etc, wl.ets, ax, O, gw, gw_dtype, hd_w, signs_w, w_scale_dtype, pw + lw.m, wl.plain), "qm_linear_backward_error");
-    if (rc) return rc;
+    const auto gradient = [&](qm::TileProduct p, const qm::ProductChoice& c, int out_dtype, int scale_dtype) {
+        if (c.rotates) return qm::run_product(c, p, QM_BF16, out_dtype, gws, hs);
+        void* out = p.c;
+        const uint8_t* mask = p.mask;
+        p.mask = nullptr;
+        p.c = k + wl.plain;
+        const hipError_t e1 = qm::run_product(c, p, QM_BF16, QM_BF16, gws, hs);
+        return e1 != hipSuccess ? e1 : qm::masked_hadamard_bwd(p.c, QM_BF16, p.M, I, p.hd, scale_dtype, p.signs, mask, out, out_dtype, out_dtype != QM_BF16, hs);
+    };
+    const qm::TileProduct gxp = product_of(wl.ec, wl.es, aw, T, gx, hd_x, signs_x, x_scale_dtype, px + lx.m);
+    const qm::TileProduct gwp = product_of(wl.etc, wl.ets, ax, O, gw, hd_w, signs_w, w_scale_dtype, pw + lw.m);
+    const qm::ProductChoice cx = qm::choose_product(gxp, QM_BF16, QM_BF16, gws, wl.gemm_ws_bytes), cw = qm::choose_product(gwp, QM_BF16, gw_dtype, gws, wl.gemm_ws_bytes);
+    if (wide_pair(gxp, cx, gwp, cw)) {
+        rc = from_hip(O > T ? qm::gemm_wide_pair(gxp, false, gwp, gw_dtype != QM_BF16, hs) : qm::gemm_wide_pair(gwp, gw_dtype != QM_BF16, gxp, false, hs), "qm_linear_backward_error");
+        if (rc) return rc;
+    } else {
+        rc = from_hip(gradient(gxp, cx, QM_BF16, x_scale_dtype), "qm_linear_backward_error");
+        if (rc) return rc;
+        rc = from_hip(gradient(gwp, cw, gw_dtype, w_scale_dtype), "qm_linear_backward_error");
+        if (rc) return rc;
+    }
     const auto exact = [&](size_t ac, size_t as, const qm::E5m2Args& b, int64_t M, void* out, int out_dtype, int hd, const uint32_t* signs, int scale_dtype,
                            const uint8_t* mask) {
         return qm::E5m2Exact{k + ac, k + as, b, M, alpha, mask, hd, make_signs(signs, hd), qm::hadamard_scale(hd, scale_dtype), out, out_dtype};

@@ -806,6 +806,30 @@ __global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu((S:
     run_tiles<S, OutT, ROT>(g, tiles);
 }
 
+// Both gradient products of the error-only scheme in one grid, on tiles of one shape, with the rotation: a workgroup begins a tile of the
+// second while others still hold one of the first, where two launches wait for the last of them.
+template <class S>
+__global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu((S::OCC * S::kWaves + 3) / 4))) void gemm_mxfp4_e5m2_pair_kernel(
+    TileProduct a, TileProduct b, int tiles_a, int tiles_b) {
+    extern __shared__ uint32_t smem[];
+    const uint32_t smem_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint32_t*)smem;
+    const int first_b = (tiles_a + 7) & ~7, t = (int)blockIdx.x;
+    if (t >= tiles_a && (t < first_b || t - first_b >= tiles_b)) return;
+    const bool second = t >= first_b;
+    TileProduct g = a;   // uniform
+    g.a_codes = second ? b.a_codes : a.a_codes;
+    g.a_scales = second ? b.a_scales : a.a_scales;
+    g.b_codes = second ? b.b_codes : a.b_codes;
+    g.b_scales = second ? b.b_scales : a.b_scales;
+    g.c = second ? b.c : a.c;
+    g.mask = second ? b.mask : a.mask;
+    g.M = second ? b.M : a.M;
+    g.K = second ? b.K : a.K;
+    g.rot_c = second ? b.rot_c : a.rot_c;
+    g.out_f32 = second ? b.out_f32 : a.out_f32;
+    g.b_wide = second ? b.b_wide : a.b_wide;
+    tile_run<S, uint16_t, true>(g, second ? t - first_b : t, smem, smem_base);
+}
 template <class S, typename OutT, bool ROT = false>
 hipError_t launch_tiles(const TileProduct& g, hipStream_t stream) {
     const auto kern = [] {
@@ -894,6 +918,31 @@ bool gemm_tile_serves(int64_t M, int64_t N, int64_t K, int a_tiled, int b_tiled,
     const bool k_ok = K % kBK == 0 || (K % kBK == 64 && K >= 192 && !a_tiled && !b_tiled);
     return M > 0 && N >= 8 && N % 8 == 0 && K > 0 && k_ok && M < (1 << 30) && N < (1 << 30) && K < (1 << 23) &&
            (reinterpret_cast<uintptr_t>(c) & 15) == 0;
+}
+
+// of the same N, alpha, Hadamard block and signs, on 256 x 256 tiles with formats chosen per block
+bool gemm_wide_pair_serves(const TileProduct& a, const TileProduct& b) {
+    const auto serves = [](const TileProduct& g) {
+        return g.b_e5m2 && g.b_wide && g.mask && gemm_tile_serves(g.M, g.N, g.K, g.a_tiled, g.b_tiled, g.c) && g.K / kBK >= 4;
+    };
+    for (int w = 0; w < 4; ++w)
+        if (a.signs.w[w] != b.signs.w[w]) return false;
+    return serves(a) && serves(b) && a.N == b.N && a.alpha == b.alpha && a.hd == b.hd;
+}
+hipError_t gemm_wide_pair(TileProduct a, bool a_f32, TileProduct b, bool b_f32, hipStream_t stream) {
+    using S = Wide256x256::Mixed;
+    if (!gemm_wide_pair_serves(a, b)) return hipErrorInvalidValue;
+    a.splits = b.splits = 1;
+    a.out_f32 = a_f32;
+    b.out_f32 = b_f32;
+    const auto kern = gemm_mxfp4_e5m2_pair_kernel<S>;
+    static std::atomic<bool> lds_allowed[kMaxDevices];
+    const hipError_t e = allow_dynamic_lds(kern, S::kSmemBytes, lds_allowed);
+    if (e != hipSuccess) return e;
+    const auto tiles = [](const TileProduct& g) { return ((g.M + S::BM - 1) / S::BM) * ((g.N + S::BN - 1) / S::BN); };
+    const int ta = tiles(a), tb = tiles(b);
+    kern<<<dim3((unsigned)(((ta + 7) & ~7) + tb)), dim3(S::kThreads), S::kSmemBytes, stream>>>(a, b, ta, tb);
+    return hipGetLastError();
 }
 
 // a: the longer contraction; tiles of 128 x 128 or 64 x 64 either; scales in blocks (see gemm_tile), at least one of them rotated

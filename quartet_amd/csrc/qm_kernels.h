@@ -235,6 +235,9 @@ hipError_t gemm_tile(int kind, const TileProduct& g, int c_dtype, hipStream_t st
 // two products (bf16 results, or with a mask and *_f32 widened ones) in one grid; TileKinds 128x128 and 64x64
 bool gemm_tile_pair_serves(const TileProduct& a, int kind_a, const TileProduct& b, int kind_b);
 hipError_t gemm_tile_pair(TileProduct a, int kind_a, bool a_f32, TileProduct b, int kind_b, bool b_f32, hipStream_t stream);
+// the gradient products of the error-only scheme in one grid (both WIDE_256x256, rotated, without K ranges)
+bool gemm_wide_pair_serves(const TileProduct& a, const TileProduct& b);
+hipError_t gemm_wide_pair(TileProduct a, bool a_f32, TileProduct b, bool b_f32, hipStream_t stream);
 
 // The product of at most 64 rows with a weight, both tiled (gemm_rows.hip): K % 128 == 0, N % 8 == 0, c 16-byte aligned, no mask.
 // Its sums are in another order than the other kernels'.

@@ -106,3 +106,12 @@ def test_pairs_keep_nothing_in_memory(kernels):
     pairs = {n: v for n, v in kernels.items() if "pair_kernel<" in n or re.search(r"big4_kernel<.*, [1-9], (true|false)>\(", n)}
     assert len(pairs) >= 20
     assert {n: v for n, v in pairs.items() if v[1]} == {}
+
+
+@pytest.mark.parametrize("T,I,O", [(4064, 4000, 3872), (3360, 3936, 3840)])
+def test_error_only_gradients_in_one_launch(oracle, T, I, O):
+    """Tiles over every edge, either product with more of them, both widths of the widened operands: against float64, as two launches are."""
+    from quartet_amd import _lib
+    from tests.test_gpu_tiles import test_error_only_layer_with_both_widths_in_one_product as against_float64
+    assert _lib.lib().qm_linear_backward_error_in_one_launch(T, I, O, 32, _lib.QM_BF16) == 1
+    against_float64(oracle, T, I, O)
