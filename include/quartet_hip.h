@@ -371,6 +371,15 @@ int qm_rmsnorm_quantize_mxfp4(const void* x, int x_dtype, const void* add, int a
                               void* packed, size_t packed_bytes, float* factor, int codes_layout, void* stream);
 int qm_swiglu_quantize_mxfp4(const void* h12, int dtype, int64_t rows, int64_t hidden, const uint32_t* sign_bits,
                              void* packed, size_t packed_bytes, int codes_layout, void* stream);
+/* The same, and in the same grid the forward quantizer of the layer's fp32 weight w [out_features, cols] (Hadamard block 32), which
+ * qm_linear_forward then takes with QM_W_IS_PACKED: QM_LAYOUT_PADDED, an fp32 x with a bf16 summand or none; a bf16 h12. */
+int qm_rmsnorm_quantize_with_weight_mxfp4(const void* x, int x_dtype, const void* add, int add_dtype, void* x_sum, const float* gain,
+                                          float eps, int64_t rows, int64_t cols, const uint32_t* sign_bits, void* packed,
+                                          size_t packed_bytes, float* factor, const float* w, int64_t out_features,
+                                          const uint32_t* signs_w, void* packed_w, size_t packed_w_bytes, void* stream);
+int qm_swiglu_quantize_with_weight_mxfp4(const void* h12, int dtype, int64_t rows, int64_t hidden, const uint32_t* sign_bits,
+                                         void* packed, size_t packed_bytes, const float* w, int64_t out_features,
+                                         const uint32_t* signs_w, void* packed_w, size_t packed_w_bytes, void* stream);
 size_t qm_rmsnorm_backward_workspace_bytes(int64_t rows, int64_t cols);
 int qm_rmsnorm_backward(const void* gy, int gy_dtype, const void* x, int x_dtype, const float* gain,
                         const float* factor, int64_t rows, int64_t cols, const uint8_t* maskbits,

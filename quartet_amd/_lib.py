@@ -55,6 +55,8 @@ EXPORTS = (
     "qm_linear_rope_serves",
     "qm_linear_rope",
     "qm_rmsnorm",
+    "qm_rmsnorm_quantize_with_weight_mxfp4",
+    "qm_swiglu_quantize_with_weight_mxfp4",
     "qm_linear_backward_error_in_one_launch",
     "qm_linear_decode",
     "qm_cross_entropy",
@@ -155,6 +157,10 @@ def lib():
     L.qm_rmsnorm.argtypes = [vp, vp, i32, vp, f32, i64, i64, vp, i32, vp]
     L.qm_linear_backward_error_in_one_launch.restype = i32
     L.qm_linear_backward_error_in_one_launch.argtypes = [i64, i64, i64, i32, i32]
+    L.qm_rmsnorm_quantize_with_weight_mxfp4.restype = i32
+    L.qm_rmsnorm_quantize_with_weight_mxfp4.argtypes = [vp, i32, vp, i32, vp, vp, f32, i64, i64, vp, vp, ctypes.c_size_t, vp, vp, i64, vp, vp, ctypes.c_size_t, vp]
+    L.qm_swiglu_quantize_with_weight_mxfp4.restype = i32
+    L.qm_swiglu_quantize_with_weight_mxfp4.argtypes = [vp, i32, i64, i64, vp, vp, ctypes.c_size_t, vp, i64, vp, vp, ctypes.c_size_t, vp]
     L.qm_linear_decode.restype = i32
     L.qm_linear_decode.argtypes = [vp, i32, i64, i64, i64, vp, vp, ctypes.c_size_t, vp, i32, vp]
     L.qm_cross_entropy.restype = i32

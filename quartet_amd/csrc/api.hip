@@ -903,9 +903,9 @@ int qm_linear_backward_seeded(const void* e, int e_dtype, int64_t T, int64_t I, 
     return gw_fused ? 0 : rotate_gw();
 }
 
-int qm_rmsnorm_quantize_mxfp4(const void* x, int x_dtype, const void* add, int add_dtype, void* x_sum, const float* gain, float eps,
+static int rmsnorm_quantize(const void* x, int x_dtype, const void* add, int add_dtype, void* x_sum, const float* gain, float eps,
                               int64_t rows, int64_t cols, const uint32_t* sign_bits, void* packed, size_t packed_bytes,
-                              float* factor, int codes_layout, void* stream) {
+                              float* factor, int codes_layout, const qm::RowmajorArgs* weight, void* stream) {
     if (!valid_layer_layout(codes_layout)) return fail(QM_ERR_INVALID, "qm_rmsnorm_quantize_mxfp4: unknown codes_layout %d", codes_layout);
     if (!valid_dtype(x_dtype)) return fail(QM_ERR_INVALID, "qm_rmsnorm_quantize_mxfp4: x_dtype %d is not QM_BF16/QM_F32", x_dtype);
     if (rows < 0 || cols <= 0 || cols % 32)
@@ -924,12 +924,12 @@ int qm_rmsnorm_quantize_mxfp4(const void* x, int x_dtype, const void* add, int a
         return fail(QM_ERR_INVALID, "qm_rmsnorm_quantize_mxfp4: a residual summand needs an fp32 x, a valid add_dtype and x_sum");
     uint8_t* p = static_cast<uint8_t*>(packed);
     return from_hip(qm::rmsnorm_quantize_hd32(x, x_dtype, add, add_dtype, x_sum, gain, eps, rows, cols, sign_bits ? sign_bits[0] : 0u, p + l.c, p + l.s,
-                                              p + l.m, factor, tiled_layout(codes_layout), reinterpret_cast<hipStream_t>(stream)),
+                                              p + l.m, factor, tiled_layout(codes_layout), weight, reinterpret_cast<hipStream_t>(stream)),
                     "qm_rmsnorm_quantize_mxfp4");
 }
 
-int qm_swiglu_quantize_mxfp4(const void* h12, int dtype, int64_t rows, int64_t hidden, const uint32_t* sign_bits, void* packed,
-                             size_t packed_bytes, int codes_layout, void* stream) {
+static int swiglu_quantize(const void* h12, int dtype, int64_t rows, int64_t hidden, const uint32_t* sign_bits, void* packed,
+                             size_t packed_bytes, int codes_layout, const qm::RowmajorArgs* weight, void* stream) {
     if (!valid_layer_layout(codes_layout)) return fail(QM_ERR_INVALID, "qm_swiglu_quantize_mxfp4: unknown codes_layout %d", codes_layout);
     if (!valid_dtype(dtype)) return fail(QM_ERR_INVALID, "qm_swiglu_quantize_mxfp4: dtype %d is not QM_BF16/QM_F32", dtype);
     if (rows < 0 || hidden <= 0 || hidden % 32)
@@ -946,8 +946,51 @@ int qm_swiglu_quantize_mxfp4(const void* h12, int dtype, int64_t rows, int64_t h
         return fail(QM_ERR_UNALIGNED, "qm_swiglu_quantize_mxfp4: h12 needs 16-byte, packed 256-byte alignment");
     uint8_t* p = static_cast<uint8_t*>(packed);
     return from_hip(qm::swiglu_quantize_hd32(h12, dtype, rows, hidden, sign_bits ? sign_bits[0] : 0u, p + l.c, p + l.s, p + l.m,
-                                             tiled_layout(codes_layout), reinterpret_cast<hipStream_t>(stream)),
+                                             tiled_layout(codes_layout), weight, reinterpret_cast<hipStream_t>(stream)),
                     "qm_swiglu_quantize_mxfp4");
+}
+
+int qm_rmsnorm_quantize_mxfp4(const void* x, int x_dtype, const void* add, int add_dtype, void* x_sum, const float* gain, float eps,
+                              int64_t rows, int64_t cols, const uint32_t* sign_bits, void* packed, size_t packed_bytes,
+                              float* factor, int codes_layout, void* stream) {
+    return rmsnorm_quantize(x, x_dtype, add, add_dtype, x_sum, gain, eps, rows, cols, sign_bits, packed, packed_bytes, factor, codes_layout, nullptr, stream);
+}
+int qm_swiglu_quantize_mxfp4(const void* h12, int dtype, int64_t rows, int64_t hidden, const uint32_t* sign_bits, void* packed,
+                             size_t packed_bytes, int codes_layout, void* stream) {
+    return swiglu_quantize(h12, dtype, rows, hidden, sign_bits, packed, packed_bytes, codes_layout, nullptr, stream);
+}
+
+namespace {
+// the weight that a producer's grid takes along: fp32 [out_features, cols], QM_LAYOUT_PADDED
+int weight_args(const char* who, const void* w, int64_t out_features, int64_t cols, const uint32_t* signs_w, void* packed_w, size_t packed_w_bytes,
+                qm::RowmajorArgs* a) {
+    if (out_features <= 0 || out_features >= (1ll << 31) - 16 || cols <= 0 || cols % 32)
+        return fail(QM_ERR_INVALID, "%s: need a weight [out_features, %lld]", who, (long long)cols);
+    const PackedLayout l = packed_layout(out_features, cols);
+    if (!w || !aligned(w, 16) || !packed_w || packed_w_bytes < l.total || !aligned(packed_w, 256))
+        return fail(QM_ERR_INVALID, "%s: w must be non-null and 16-byte aligned, packed_w hold %zu bytes, 256-byte aligned", who, l.total);
+    uint8_t* p = static_cast<uint8_t*>(packed_w);
+    *a = qm::RowmajorArgs{w, QM_F32, out_features, cols, make_signs(signs_w, 32), p + l.c, p + l.s, p + l.m};
+    return 0;
+}
+}  // namespace
+
+int qm_rmsnorm_quantize_with_weight_mxfp4(const void* x, int x_dtype, const void* add, int add_dtype, void* x_sum, const float* gain, float eps,
+                                          int64_t rows, int64_t cols, const uint32_t* sign_bits, void* packed, size_t packed_bytes, float* factor,
+                                          const float* w, int64_t out_features, const uint32_t* signs_w, void* packed_w, size_t packed_w_bytes, void* stream) {
+    if (x_dtype != QM_F32 || (add && add_dtype != QM_BF16) || rows <= 0)
+        return fail(QM_ERR_INVALID, "qm_rmsnorm_quantize_with_weight_mxfp4: needs rows, an fp32 x and a bf16 summand or none");
+    qm::RowmajorArgs a;
+    if (int rc = weight_args("qm_rmsnorm_quantize_with_weight_mxfp4", w, out_features, cols, signs_w, packed_w, packed_w_bytes, &a)) return rc;
+    return rmsnorm_quantize(x, x_dtype, add, add_dtype, x_sum, gain, eps, rows, cols, sign_bits, packed, packed_bytes, factor, QM_LAYOUT_PADDED, &a, stream);
+}
+int qm_swiglu_quantize_with_weight_mxfp4(const void* h12, int dtype, int64_t rows, int64_t hidden, const uint32_t* sign_bits, void* packed,
+                                         size_t packed_bytes, const float* w, int64_t out_features, const uint32_t* signs_w, void* packed_w,
+                                         size_t packed_w_bytes, void* stream) {
+    if (dtype != QM_BF16 || rows <= 0) return fail(QM_ERR_INVALID, "qm_swiglu_quantize_with_weight_mxfp4: needs rows of a bf16 h12");
+    qm::RowmajorArgs a;
+    if (int rc = weight_args("qm_swiglu_quantize_with_weight_mxfp4", w, out_features, hidden, signs_w, packed_w, packed_w_bytes, &a)) return rc;
+    return swiglu_quantize(h12, dtype, rows, hidden, sign_bits, packed, packed_bytes, QM_LAYOUT_PADDED, &a, stream);
 }
 
 size_t qm_rmsnorm_backward_workspace_bytes(int64_t rows, int64_t cols) {

@@ -200,6 +200,12 @@ Tensor forward_products(const Layer& l, const Tensor& x2, const Tensor& weight, 
     return y;
 }
 
+// Whether a producer's grid quantizes the layer's weight along: it is not packed yet, fp32, aligned, under a Hadamard block of 32
+bool takes_weight(const Layer& l, const Tensor& weight, const Tensor* packed_w) {
+    return packed_w && !packed_w->defined() && l.T > 0 && l.layout == QM_LAYOUT_PADDED && l.w_hd == 32 && !l.w_dense.defined() && weight.scalar_type() == at::kFloat &&
+           weight.is_contiguous() && reinterpret_cast<uintptr_t>(weight.data_ptr()) % 16 == 0;
+}
+
 // Straight-through backward of a forward quantizer with a dense rotation: (g * clip mask) @ matrix^T per group of 32, in
 // g's dtype like the module path's product.
 Tensor dense_rotation_backward(const Tensor& g, const Tensor& maskbits, const Tensor& dense, at::ScalarType x_dtype, at::ScalarType scale_dtype) {
@@ -380,14 +386,24 @@ struct NormArgs {
     Tensor* packed_w;
 };
 // Q(rmsnorm(x2 [+ add2]) * gain) as the layer's packed operand; x2 becomes the sum
-Tensor normed_into_packed(const Layer& l, Tensor& x2, const Tensor& add2, const Tensor& gain, double eps, Tensor& factor) {
+// packed_w: where the layer's weight goes along, undefined on entry (see takes_weight)
+Tensor normed_into_packed(const Layer& l, Tensor& x2, const Tensor& add2, const Tensor& gain, double eps, Tensor& factor, const Tensor& weight = Tensor(),
+                          Tensor* packed_w = nullptr) {
     Tensor packed_x = packed_buffer(l.T, l.I, x2), x_sum;
     factor = at::empty({l.T}, x2.options().dtype(at::kFloat));
     if (add2.defined()) x_sum = at::empty_like(x2);
-    check(qm_rmsnorm_quantize_mxfp4(x2.data_ptr(), dtype_code(x2.scalar_type()), ptr(add2), add2.defined() ? dtype_code(add2.scalar_type()) : 0,
-                                    add2.defined() ? x_sum.data_ptr() : nullptr, gain.data_ptr<float>(), (float)eps, l.T, l.I, l.a_signs.data(),
-                                    packed_x.data_ptr(), (size_t)packed_x.numel(), factor.data_ptr<float>(), l.layout, stream_of(x2)),
-          "qm_rmsnorm_quantize_mxfp4");
+    if (takes_weight(l, weight, packed_w) && x2.scalar_type() == at::kFloat && (!add2.defined() || add2.scalar_type() == at::kBFloat16)) {
+        *packed_w = packed_buffer(l.O, l.I, weight);
+        check(qm_rmsnorm_quantize_with_weight_mxfp4(x2.data_ptr(), QM_F32, ptr(add2), QM_BF16, add2.defined() ? x_sum.data_ptr() : nullptr, gain.data_ptr<float>(),
+                                                    (float)eps, l.T, l.I, l.a_signs.data(), packed_x.data_ptr(), (size_t)packed_x.numel(), factor.data_ptr<float>(),
+                                                    weight.data_ptr<float>(), l.O, l.w_signs.data(), packed_w->data_ptr(), (size_t)packed_w->numel(), stream_of(x2)),
+              "qm_rmsnorm_quantize_with_weight_mxfp4");
+    } else {
+        check(qm_rmsnorm_quantize_mxfp4(x2.data_ptr(), dtype_code(x2.scalar_type()), ptr(add2), add2.defined() ? dtype_code(add2.scalar_type()) : 0,
+                                        add2.defined() ? x_sum.data_ptr() : nullptr, gain.data_ptr<float>(), (float)eps, l.T, l.I, l.a_signs.data(),
+                                        packed_x.data_ptr(), (size_t)packed_x.numel(), factor.data_ptr<float>(), l.layout, stream_of(x2)),
+              "qm_rmsnorm_quantize_mxfp4");
+    }
     if (add2.defined()) x2 = x_sum;
     return packed_x;
 }
@@ -402,7 +418,7 @@ struct NormLinearFn : Function<NormLinearFn> {
         l->x_dtype = at::kFloat;   // the normalised tensor times the fp32 gain is an fp32 tensor
         const Tensor gain_c = gain.contiguous();
         Tensor factor;
-        Tensor packed_x = normed_into_packed(*l, x2, args.has_add ? rows_of(add, I) : Tensor(), gain_c, args.eps, factor);
+        Tensor packed_x = normed_into_packed(*l, x2, args.has_add ? rows_of(add, I) : Tensor(), gain_c, args.eps, factor, weight, args.packed_w);
         Tensor y = forward_products(*l, Tensor(), weight, autocast_bf16() ? at::kBFloat16 : at::kFloat, packed_x, *args.packed_w);
         if (ctx) {
             ctx->set_materialize_grads(false);
@@ -469,9 +485,17 @@ struct SwigluLinearFn : Function<SwigluLinearFn> {
         set_extents(*l, h2.size(0), weight);
         l->x_dtype = h12.scalar_type();
         Tensor packed_x = packed_buffer(l->T, I, h2);
-        check(qm_swiglu_quantize_mxfp4(h2.data_ptr(), dtype_code(h2.scalar_type()), l->T, I, l->a_signs.data(), packed_x.data_ptr(),
-                                       (size_t)packed_x.numel(), l->layout, stream_of(h2)),
-              "qm_swiglu_quantize_mxfp4");
+        if (takes_weight(*l, weight, packed_w) && h2.scalar_type() == at::kBFloat16) {
+            *packed_w = packed_buffer(l->O, I, weight);
+            check(qm_swiglu_quantize_with_weight_mxfp4(h2.data_ptr(), QM_BF16, l->T, I, l->a_signs.data(), packed_x.data_ptr(), (size_t)packed_x.numel(),
+                                                       weight.data_ptr<float>(), l->O, l->w_signs.data(), packed_w->data_ptr(), (size_t)packed_w->numel(),
+                                                       stream_of(h2)),
+                  "qm_swiglu_quantize_with_weight_mxfp4");
+        } else {
+            check(qm_swiglu_quantize_mxfp4(h2.data_ptr(), dtype_code(h2.scalar_type()), l->T, I, l->a_signs.data(), packed_x.data_ptr(),
+                                           (size_t)packed_x.numel(), l->layout, stream_of(h2)),
+                  "qm_swiglu_quantize_mxfp4");
+        }
         const Tensor y = forward_products(*l, Tensor(), weight, autocast_bf16() ? at::kBFloat16 : h12.scalar_type(), packed_x, *packed_w);
         if (ctx) {
             ctx->save_for_backward({h2, packed_x, *packed_w});

@@ -154,9 +154,12 @@ hipError_t masked_hadamard_bwd_hd32_pair(const void* ga, int64_t na, int scale_d
 // Producers fused into the forward quantizer (Hadamard block 32, quest RTN, clip mask) and their backward passes
 hipError_t rmsnorm_quantize_hd32(const void* x, int dtype, const void* add, int add_dtype, void* xsum, const float* gain, float eps,
                                  int64_t rows, int64_t cols, uint32_t sign_word, uint8_t* codes, uint8_t* scales, uint8_t* maskbits,
-                                 float* factor, bool tiled, hipStream_t stream);
+                                 float* factor, bool tiled, const RowmajorArgs* weight, hipStream_t stream);
 hipError_t swiglu_quantize_hd32(const void* h12, int dtype, int64_t rows, int64_t hidden, uint32_t sign_word,
-                                uint8_t* codes, uint8_t* scales, uint8_t* maskbits, bool tiled, hipStream_t stream);
+                                uint8_t* codes, uint8_t* scales, uint8_t* maskbits, bool tiled, const RowmajorArgs* weight, hipStream_t stream);
+// weight: null, or the layer's weight (Hadamard block 32), quantized in the same grid; for tiled codes of these dtypes
+bool producer_takes_weight(int dtype, int add_dtype, int w_dtype);   // no summand: BF16
+bool swiglu_takes_weight(int dtype, int w_dtype);
 // measurement and test aid: the SwiGLU producer's bf16 silu of all 65536 bit patterns
 hipError_t silu_of_bf16_table(uint16_t* out, hipStream_t stream);
 size_t rmsnorm_backward_workspace_bytes(int64_t rows, int64_t cols);

@@ -1134,6 +1134,7 @@ struct RmsNormProducer {
     static constexpr int kOutDtype = F32;  // bf16-or-fp32 normalised value times the fp32 gain is fp32
     static constexpr bool kAdd = !std::is_void<TA>::value;
     using TAdd = typename std::conditional<kAdd, TA, T>::type;
+    static constexpr bool kWithWeight = sizeof(T) == 4 && (!kAdd || sizeof(TAdd) == 2);
     static constexpr bool kStaged = sizeof(T) == 4;
     static constexpr int kLds = kStaged ? 4 * 512 * 16 : 0;
     const T* x;
@@ -1274,7 +1275,7 @@ struct SwiGluProducer {
     // 4 l + (q ^ l / 4 % 4) holds piece q of lane l's group.  Inputs cycled through memory: 16384 x 4096 73 -> 65 us (4.8 TB/s; 76
     // inside a layer's step), 32768 x 4096 141 -> 125; 16384 x 1536 33 either way, up to
     // 4096 x 1728 (11 us) latency
-    static constexpr bool kStaged = sizeof(T) == 2;
+    static constexpr bool kStaged = sizeof(T) == 2, kWithWeight = sizeof(T) == 2;
     static constexpr int kLds = kStaged ? 4 * 512 * 16 : 0;
     const T* h12;  // [rows, 2 cols]: up, then gate
 
@@ -1392,46 +1393,63 @@ struct ProducedRowsJob {
     }
 };
 
+// The quantizer of the layer's weight rides in the same grid, behind the rows, where the launch is one of a training step under
+// autocast: fp32 weights, tiled codes of any extents.  By itself it is a launch of a few microseconds that mostly starts and ends
+// (1536 x 4096: 9.6 us, 4608 x 1536 11).  us per training step with the two launches and with one: 16384 x 1536 x 4608 behind its norm 449 ->
+// 443.5, 16384 x 4096 x 1536 behind SwiGLU 431 -> 424.5, 1024 x 4096 x 8192 201.7 -> 198.4.
+using WeightJob = RowmajorTiledJob<float, QUEST_RTN, true, 32, true>;
+WeightJob weight_job(const RowmajorArgs& w) {
+    return WeightJob(w.x, w.rows, w.cols, make_rotation<32>(w.dtype, w.signs), 0,
+                     GroupOut{reinterpret_cast<uint4*>(w.codes), w.scales, reinterpret_cast<uint32_t*>(w.maskbits), nullptr});
+}
+
 template <typename P, int W>
-void launch_produced_w(const P& prod, int64_t rows, int64_t cols, uint32_t sign_word, const GroupOut& out, bool tiled,
+void launch_produced_w(const P& prod, int64_t rows, int64_t cols, uint32_t sign_word, const GroupOut& out, bool tiled, const RowmajorArgs* weight,
                        hipStream_t stream) {
-    if (tiled) launch_job(ProducedRowsJob<P, true, W>(prod, rows, cols, sign_word, out), stream);
+    const ProducedRowsJob<P, true, W> job(prod, rows, cols, sign_word, out);
+    if constexpr (P::kWithWeight)
+        if (weight) return launch_jobs(stream, job, weight_job(*weight));
+    if (tiled) launch_job(job, stream);
     else launch_job(ProducedRowsJob<P, false, W>(prod, rows, cols, sign_word, out), stream);
 }
 
 template <typename P>
 void launch_produced(const P& prod, int64_t rows, int64_t cols, uint32_t sign_word, uint8_t* codes, uint8_t* scales,
-                     uint8_t* maskbits, bool tiled, hipStream_t stream) {
+                     uint8_t* maskbits, bool tiled, const RowmajorArgs* weight, hipStream_t stream) {
     const GroupOut out{reinterpret_cast<uint4*>(codes), scales, reinterpret_cast<uint32_t*>(maskbits), nullptr};
-    if (cols <= 16 * 32) launch_produced_w<P, 16>(prod, rows, cols, sign_word, out, tiled, stream);
-    else if (cols <= 32 * 32) launch_produced_w<P, 32>(prod, rows, cols, sign_word, out, tiled, stream);
-    else launch_produced_w<P, 64>(prod, rows, cols, sign_word, out, tiled, stream);
+    if (cols <= 16 * 32) launch_produced_w<P, 16>(prod, rows, cols, sign_word, out, tiled, weight, stream);
+    else if (cols <= 32 * 32) launch_produced_w<P, 32>(prod, rows, cols, sign_word, out, tiled, weight, stream);
+    else launch_produced_w<P, 64>(prod, rows, cols, sign_word, out, tiled, weight, stream);
 }
 
 }  // namespace
+
+bool producer_takes_weight(int dtype, int add_dtype, int w_dtype) { return dtype == F32 && add_dtype == BF16 && w_dtype == F32; }
+bool swiglu_takes_weight(int dtype, int w_dtype) { return dtype == BF16 && w_dtype == F32; }
 
 // Q(rmsnorm(x) * gain): Hadamard block 32, quest RTN, clip mask; factor [rows] receives 1 / sqrt(mean(x^2) + eps).
 // add != null (x fp32 only): the norm's input is x + add, also written to xsum [rows, cols] fp32.
 hipError_t rmsnorm_quantize_hd32(const void* x, int dtype, const void* add, int add_dtype, void* xsum, const float* gain, float eps,
                                  int64_t rows, int64_t cols, uint32_t sign_word, uint8_t* codes, uint8_t* scales, uint8_t* maskbits,
-                                 float* factor, bool tiled, hipStream_t stream) {
+                                 float* factor, bool tiled, const RowmajorArgs* weight, hipStream_t stream) {
     if (rows == 0) return hipSuccess;
+    if (weight && !(tiled && producer_takes_weight(dtype, add ? add_dtype : BF16, weight->dtype))) return hipErrorInvalidValue;
     if (add) {
         if (dtype != F32) return hipErrorInvalidValue;
         const float* xp = reinterpret_cast<const float*>(x);
         float* sp = reinterpret_cast<float*>(xsum);
         if (add_dtype == BF16)
             launch_produced(RmsNormProducer<float, uint16_t>{xp, gain, factor, eps, reinterpret_cast<const uint16_t*>(add), sp}, rows,
-                            cols, sign_word, codes, scales, maskbits, tiled, stream);
+                            cols, sign_word, codes, scales, maskbits, tiled, weight, stream);
         else
             launch_produced(RmsNormProducer<float, float>{xp, gain, factor, eps, reinterpret_cast<const float*>(add), sp}, rows, cols,
-                            sign_word, codes, scales, maskbits, tiled, stream);
+                            sign_word, codes, scales, maskbits, tiled, weight, stream);
     } else if (dtype == BF16) {
         launch_produced(RmsNormProducer<uint16_t>{reinterpret_cast<const uint16_t*>(x), gain, factor, eps, nullptr, nullptr}, rows,
-                        cols, sign_word, codes, scales, maskbits, tiled, stream);
+                        cols, sign_word, codes, scales, maskbits, tiled, weight, stream);
     } else {
         launch_produced(RmsNormProducer<float>{reinterpret_cast<const float*>(x), gain, factor, eps, nullptr, nullptr}, rows, cols,
-                        sign_word, codes, scales, maskbits, tiled, stream);
+                        sign_word, codes, scales, maskbits, tiled, weight, stream);
     }
     return hipGetLastError();
 }
@@ -1444,14 +1462,15 @@ hipError_t silu_of_bf16_table(uint16_t* out, hipStream_t stream) {
 
 // Q(silu(up) * gate) of h12 [rows, 2 hidden] = (up, gate): Hadamard block 32, quest RTN, clip mask
 hipError_t swiglu_quantize_hd32(const void* h12, int dtype, int64_t rows, int64_t hidden, uint32_t sign_word,
-                                uint8_t* codes, uint8_t* scales, uint8_t* maskbits, bool tiled, hipStream_t stream) {
+                                uint8_t* codes, uint8_t* scales, uint8_t* maskbits, bool tiled, const RowmajorArgs* weight, hipStream_t stream) {
     if (rows == 0) return hipSuccess;
+    if (weight && !(tiled && swiglu_takes_weight(dtype, weight->dtype))) return hipErrorInvalidValue;
     if (dtype == BF16)
         launch_produced(SwiGluProducer<uint16_t>{reinterpret_cast<const uint16_t*>(h12)}, rows, hidden, sign_word, codes,
-                        scales, maskbits, tiled, stream);
+                        scales, maskbits, tiled, weight, stream);
     else
         launch_produced(SwiGluProducer<float>{reinterpret_cast<const float*>(h12)}, rows, hidden, sign_word, codes, scales,
-                        maskbits, tiled, stream);
+                        maskbits, tiled, weight, stream);
     return hipGetLastError();
 }
 
