@@ -594,7 +594,7 @@ py::object norm_swiglu_linear(const Tensor& x, const optional<Tensor>& add, cons
         require_cuda(x, gain, w12, w, add_t);
         const c10::OptionalDeviceGuard guard(w12.device());
         const int64_t T = x.numel() / I;
-        if (!qm_linear_swiglu_serves(T, I, hidden)) return py::none();
+        if (x.size(-1) != I || gain.numel() != I || !qm_linear_swiglu_serves(T, I, hidden)) return py::none();
         set_extents(*l, T, w12);
         set_extents(*next, T, w);
         if (l->layout != QM_LAYOUT_PADDED || next->layout != QM_LAYOUT_PADDED || l->O != 2 * hidden) return py::none();
@@ -619,7 +619,7 @@ py::object norm_rope_linear(const Tensor& x, const optional<Tensor>& add, const 
         require_cuda(x, gain, weight, table, add_t);
         const c10::OptionalDeviceGuard guard(weight.device());
         const int64_t T = x.numel() / I;
-        if (x.dim() != 3 || weight.size(0) != 3 * C || !qm_linear_rope_serves(T, I, C, (int)hs)) return py::none();
+        if (x.dim() != 3 || x.size(2) != I || gain.numel() != I || weight.size(0) != 3 * C || !qm_linear_rope_serves(T, I, C, (int)hs)) return py::none();
         const int64_t B = x.size(0), S = x.size(1);
         if (table.dim() != 3 || table.size(0) != S || table.size(1) != hs / 2 || table.size(2) != 2 || !table.is_contiguous() ||
             reinterpret_cast<uintptr_t>(table.data_ptr()) % 16)

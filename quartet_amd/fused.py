@@ -168,10 +168,10 @@ def rmsnorm_rope_linear(norm, c_attn, x, table, n_head, add=None):
     return (*rope_qkv(qkv, table, n_head), x)
 
 
-def rmsnorm(norm, x, add=None):
-    """norm(x [+ add]) in front of a plain linear layer.  In an evaluation under bf16 autocast in one pass, rounded to the bf16 that autocast
-    hands the layer."""
-    plain = (type(x) is torch.Tensor and x.is_cuda and x.dtype == torch.float32 and torch.is_autocast_enabled("cuda")
+def rmsnorm(norm, layer, x, add=None):
+    """norm(x [+ add]) in front of `layer`.  Where that is a plain nn.Linear, in an evaluation under bf16 autocast in one pass, rounded to the
+    bf16 that autocast hands the layer."""
+    plain = (type(layer) is torch.nn.Linear and not _watched(layer) and type(x) is torch.Tensor and x.is_cuda and x.dtype == torch.float32 and torch.is_autocast_enabled("cuda")
              and torch.get_autocast_dtype("cuda") == torch.bfloat16 and not (one_node.transformed() or torch.compiler.is_compiling()))
     if plain:
         from .llama import RMSNorm
@@ -181,7 +181,7 @@ def rmsnorm(norm, x, add=None):
         watched = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, add, gain))
         if (not watched and gain.dtype == torch.float32 and gain.shape == (cols,) and gain.device == x.device and 0 < cols <= 4096
                 and cols % 4 == 0 and 0 < x.numel() < 1 << 31
-                and (add is None or (add.dtype in _KERNEL_DTYPES and add.shape == x.shape and add.device == x.device))):
+                and (add is None or (type(add) is torch.Tensor and add.dtype in _KERNEL_DTYPES and add.shape == x.shape and add.device == x.device))):
             rows = [t if t is None else t.reshape(-1, cols).contiguous() for t in (x, add)]
             if not any(t is not None and t.data_ptr() % 16 for t in (*rows, gain)):
                 return kernels.rmsnorm(rows[0], gain.contiguous(), norm.eps, rows[1], torch.bfloat16).view(x.shape)

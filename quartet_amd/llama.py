@@ -244,7 +244,7 @@ class Llama(nn.Module):
             else:
                 x = block(x if pending is None else x + pending, table)
                 pending = None
-        x = rmsnorm(self.transformer.ln_f, x, pending)
+        x = rmsnorm(self.transformer.ln_f, self.lm_head, x, pending)
         if targets is not None:
             logits = self.lm_head(x)
             loss = cross_entropy(logits.view(-1, logits.size(-1)), targets.view(-1), ignore_index=-1)

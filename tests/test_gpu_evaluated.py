@@ -140,17 +140,44 @@ def test_last_norm(rows, cols, add_dtype, out_dtype):
 def test_last_norm_of_a_model_takes_the_module_where_somebody_listens_or_asks_for_gradients():
     from quartet_amd.fused import rmsnorm
     from quartet_amd.llama import RMSNorm
-    norm = RMSNorm(640).to("cuda:0")
+    class Head(torch.nn.Linear):
+        pass
+    norm, head = RMSNorm(640).to("cuda:0"), torch.nn.Linear(640, 8, bias=False).to("cuda:0")
     x = torch.randn(2, 70, 640, device="cuda:0")
     with torch.autocast("cuda", dtype=BF16):
         with torch.no_grad():
-            one = rmsnorm(norm, x)
+            one = rmsnorm(norm, head, x)
             assert one.dtype == BF16 and float((one.float() - norm(x)).abs().max()) < 2.0 ** -6
             seen = []
             handle = norm.register_forward_hook(lambda *a: seen.append(1))
-            assert torch.equal(rmsnorm(norm, x), norm(x)) and len(seen) == 2
+            assert torch.equal(rmsnorm(norm, head, x), norm(x)) and len(seen) == 2
             handle.remove()
-        y = rmsnorm(norm, x)
+            # another head, or one that somebody watches, sees the norm's own result
+            assert rmsnorm(norm, Head(640, 8, device="cuda:0"), x).dtype == torch.float32
+            handle = head.register_forward_pre_hook(lambda *a: None)
+            assert torch.equal(rmsnorm(norm, head, x), norm(x))
+            handle.remove()
+        y = rmsnorm(norm, head, x)
         assert y.dtype == torch.float32 and y.requires_grad
     with torch.no_grad():
-        assert torch.equal(rmsnorm(norm, x, x), norm(x + x))
+        assert torch.equal(rmsnorm(norm, head, x, x), norm(x + x))
+
+
+def test_rows_that_are_not_the_layer_s_are_refused_as_without_packed_weights():
+    """An input of twice the layer's width is as many rows again: nothing may be launched for them on results of half the size."""
+    import quartet_amd as q
+    from quartet_amd.fused import rmsnorm_rope_linear, rmsnorm_swiglu_linear
+    from quartet_amd.llama import LlamaBlock, RMSNorm, llama_30m, rotary_table
+    with torch.device("cuda"):
+        block, wide = LlamaBlock(llama_30m(n_layer=1)).eval(), RMSNorm(1280)
+    q.enable_packed_weight_cache(block)
+    table = rotary_table(128, 96).to("cuda:0")
+    with torch.no_grad(), torch.autocast("cuda", dtype=BF16):
+        x = torch.randn(3, 96, 640, device="cuda:0")
+        rmsnorm_rope_linear(block.ln_1, block.attn.c_attn, x, table, 5)
+        rmsnorm_swiglu_linear(block.ln_2, block.mlp.w12, block.mlp.c_proj, x)
+        for norm in (block.ln_1, wide):
+            with pytest.raises(RuntimeError):
+                rmsnorm_rope_linear(norm, block.attn.c_attn, torch.randn(3, 96, 1280, device="cuda:0"), table, 5)
+            with pytest.raises(RuntimeError):
+                rmsnorm_swiglu_linear(norm, block.mlp.w12, block.mlp.c_proj, torch.randn(3, 96, 1280, device="cuda:0"))
