@@ -36,16 +36,17 @@ __device__ __forceinline__ void run_job(unsigned bid, const A& a, const Rest&...
     }
 }
 
-constexpr int least(int a) { return a; }
+// J::kWaves: resident waves per SIMD the job is to be compiled for (1: the fewest it can do with, 0: what the launch's other jobs
+// want), for the job of a launch that wants fewest
 template <typename... Ts>
-constexpr int least(int a, Ts... rest) {
-    const int r = least(rest...);
-    return a < r ? a : r;
+constexpr int wanted_waves(Ts... waves) {
+    int least = 0;
+    ((least = waves && (!least || waves < least) ? waves : least), ...);
+    return least ? least : 1;
 }
 
-// J::kWaves: resident waves per SIMD the job is to be compiled for (1: no wish), for the job of a launch that wants fewest
 template <class... Jobs>
-__global__ __launch_bounds__(256, least(Jobs::kWaves...)) void job_kernel(Jobs... jobs) {
+__global__ __launch_bounds__(256, wanted_waves(Jobs::kWaves...)) void job_kernel(Jobs... jobs) {
     job_starts();
     run_job(blockIdx.x, jobs...);
 }

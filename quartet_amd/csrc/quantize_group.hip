@@ -246,6 +246,13 @@ void launch_rowmajor_dense(int mode, const void* x, int64_t rows, int64_t cols, 
     }
 }
 
+// Waves on a SIMD that the grid of the backward pass's four quantizers (not the error signal's by themselves) is compiled for: as many as fit without scratch memory.  Left
+// alone the compiler took 128 to 160 registers (three waves, four for whole tiles of blocks of 32) where 96 do for blocks of 32 and 107
+// and 127 for blocks of 64 and 128; six waves would spill.  The other waves' arithmetic hides one's requests.  us of the grid, before
+// and now: 1824 x 1408 x 2048 18.8 -> 14.5, 20000 x 704 x 704 33.8 -> 30.2, blocks of 64 8192 x 4096 x 4096 83.7 -> 76.3; per step
+// 8192 x 4096 x 4096 285 -> 280, 8192 x 4096 x 11008 693 -> 685, blocks of 128 8192 x 1536 x 4608 194 -> 191.
+constexpr int backward_waves(int hd) { return hd == 32 ? 5 : 4; }
+
 // Tiled code layout ([rows/16][cols/128][16 rows][64 bytes]).  Workgroup b owns block b / chunks of 16 rows and run
 // b % chunks of 512 columns (four code tiles); wave w owns rows 4w..4w+3 of the block, lane l its row l / 16 and
 // group l % 16 of the run: the wave reads four contiguous KiB (bf16) and writes, per tile, four rows' 64-byte pieces
@@ -255,7 +262,7 @@ void launch_rowmajor_dense(int mode, const void* x, int64_t rows, int64_t cols, 
 template <typename T, int MODE, bool WANT_MASK, int HD = 32, bool PADDED = false>
 struct RowmajorTiledJob {
     static constexpr int kLds = 0;
-    static constexpr int kWaves = 1;
+    static constexpr int kWaves = MODE == QUEST_RTN ? 8 : 0;   // forward: 62 registers; with padded extents 70 without the bound
     const T* x;
     int rows, groups, groups_p, chunks;   // groups of 32 per row: of the tensor, of its padded code tiles
     Rotation rot;
@@ -455,7 +462,7 @@ constexpr int kTrP = 128;
 template <typename T, int MODE, bool DENSE = false, int HD = 32, bool PADDED = false>
 struct TransposedJob {
     static constexpr int kLds = TrTile<T>::kQ * (4 * 16 + 4);
-    static constexpr int kWaves = 1;
+    static constexpr int kWaves = 0;
     const T* x;
     int64_t P, Q;
     Rotation rot;
@@ -729,8 +736,7 @@ struct RequantJob {
 // 128 337 (330; 345), 16512 x 1792 x 640 with blocks of 128 140 (133; 171).  Zero rows together, as padding behind the tokens, cost nothing.
 // What bounds it: vector instructions (385 a group, 0.7 us per wave and group of 32 at 2.4 GHz, half of that Philox and the
 // stochastic converts); a row group's codes are waited for when they are needed.  It runs in one grid with the quantizers of the
-// error signal, compiled to 128 registers (four waves on a SIMD), 132 with padded extents and 140 and 160 with blocks of 64 and 128
-// (three).  Both operands of a layer in a grid of their own, which fit six waves, 8192 x 4096 and 11008 x 4096: 46 us; 16384 x 4096 and
+// error signal (backward_waves).  Both operands of a layer in a grid of their own, 8192 x 4096 and 11008 x 4096: 46 us; 16384 x 4096 and
 // 1536 x 4096: 43; 16480 x 1728 and 640 x 1728: 22.  The kernel above (544 instructions a group, 64 narrow loads per lane, three waves on a
 // SIMD) took 56, 53 and 26.  The four jobs of 8192 x 4096 x 4096 in one grid take 68 us, in two 71.
 template <int MODE, int HD, bool PADDED>
@@ -738,7 +744,7 @@ struct RequantTiledJob {
     static constexpr int kRegion = 128 * 32;                                     // a wave's codes, in and out
     static constexpr int kScalesIn = 4 * kRegion, kScalesOut = kScalesIn + 4 * 256;
     static constexpr int kLds = kScalesOut + kRqC * 16;
-    static constexpr int kWaves = 1;
+    static constexpr int kWaves = backward_waves(HD);
     static constexpr int P = HD / 32;                                            // groups of a Hadamard block
     const uint8_t* codes_in;
     const uint8_t* scales_in;

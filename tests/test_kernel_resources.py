@@ -47,3 +47,12 @@ def test_a_rotation_in_the_epilogue_holds_no_registers_through_the_product(kerne
     for n, registers in rotating.items():
         plain = tiles[n.replace("true>(qm::TileProduct", "false>(qm::TileProduct")]
         assert registers <= plain + 4, (n, registers, plain)
+
+
+def test_backward_quantizers_fit_their_waves_without_scratch(kernels):
+    """The grid of the four quantizers of a backward pass: 512 registers a lane shared by five waves, four for wider blocks."""
+    grids = {n: v for n, v in kernels.items() if "job_kernel<" in n and "TransposedJob<" in n and "RequantTiledJob<" in n}
+    assert len(grids) >= 12
+    for n, (registers, scratch) in grids.items():
+        block = int(re.search(r"RequantTiledJob<\d+, (\d+),", n).group(1))
+        assert scratch == 0 and registers <= (96 if block == 32 else 128), (n, registers, scratch)
