@@ -7,8 +7,11 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "qm_kernels.h"
 #include "qm_math.h"
+#include "streaming.h"
 
 namespace qm {
 
@@ -60,7 +63,8 @@ __device__ __forceinline__ float widen(uint16_t x) { return u2f((uint32_t)x << 1
 __device__ __forceinline__ float widen(float x) { return x; }
 
 // losses[row] = log(sum exp(logits[row])) - logits[row][target], 0 for an ignored row; a target that is no class: NaN
-template <typename T>
+// STREAM: requests past the caches.  4096 x 32000 bf16 57 -> 48.5 us (5.4 TB/s), 600 x 32000 13.0 -> 13.3
+template <typename T, bool STREAM>
 __global__ __launch_bounds__(kLossThreads) void cross_entropy_rows_kernel(const T* __restrict__ logits, const int64_t* __restrict__ targets,
                                                                           int64_t classes, int64_t ignore, float* __restrict__ losses) {
     constexpr int kPer = 16 / sizeof(T), kAhead = 4;
@@ -82,7 +86,7 @@ __global__ __launch_bounds__(kLossThreads) void cross_entropy_rows_kernel(const 
     for (; i + (kAhead - 1) * kLossThreads < pieces; i += kAhead * kLossThreads) {
         uint4 raw[kAhead];
 #pragma unroll
-        for (int j = 0; j < kAhead; ++j) raw[j] = p[i + j * kLossThreads];
+        for (int j = 0; j < kAhead; ++j) raw[j] = STREAM ? stream_load(p + i + j * kLossThreads) : p[i + j * kLossThreads];
         float v[kAhead * kPer];
 #pragma unroll
         for (int j = 0; j < kAhead; ++j) {
@@ -147,13 +151,17 @@ __global__ __launch_bounds__(1024) void cross_entropy_mean_kernel(const float* _
 
 hipError_t cross_entropy_mean(const void* logits, int dtype, const int64_t* targets, int64_t rows, int64_t classes, int64_t ignore,
                               float* losses, float* loss, hipStream_t stream) {
+    const auto go = [&](const auto* x, auto past) {
+        using T = std::remove_const_t<std::remove_pointer_t<decltype(x)>>;
+        cross_entropy_rows_kernel<T, decltype(past)::value><<<dim3((unsigned)rows), dim3(kLossThreads), 0, stream>>>(x, targets, classes, ignore, losses);
+    };
+    const auto by_size = [&](const auto* x) {
+        if (rows * classes * (int64_t)sizeof(*x) >= kPastTheCaches) go(x, std::true_type{});
+        else go(x, std::false_type{});
+    };
     if (rows > 0) {
-        if (dtype == BF16)
-            cross_entropy_rows_kernel<uint16_t><<<dim3((unsigned)rows), dim3(kLossThreads), 0, stream>>>(static_cast<const uint16_t*>(logits), targets,
-                                                                                                         classes, ignore, losses);
-        else
-            cross_entropy_rows_kernel<float><<<dim3((unsigned)rows), dim3(kLossThreads), 0, stream>>>(static_cast<const float*>(logits), targets, classes,
-                                                                                                      ignore, losses);
+        if (dtype == BF16) by_size(static_cast<const uint16_t*>(logits));
+        else by_size(static_cast<const float*>(logits));
     }
     cross_entropy_mean_kernel<<<dim3(1), dim3(1024), 0, stream>>>(losses, targets, rows, ignore, loss);
     return hipGetLastError();

@@ -4,8 +4,11 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "qm_kernels.h"
 #include "qm_math.h"
+#include "streaming.h"
 
 namespace qm {
 
@@ -14,23 +17,34 @@ namespace {
 typedef float v2f __attribute__((ext_vector_type(2)));
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 
-template <typename T>
+// STREAM: past the caches (streaming.h)
+template <bool STREAM = false, typename V>
+__device__ __forceinline__ V load_vector(const V* p) {
+    if constexpr (STREAM) return stream_load(p);
+    else return *p;
+}
+template <bool STREAM = false, typename V>
+__device__ __forceinline__ void store_vector(V* p, const V& v) {
+    if constexpr (STREAM) stream_store(p, v);
+    else *p = v;
+}
+template <bool STREAM = false, typename T>
 __device__ __forceinline__ float4 load4(const T* p) {
     if constexpr (sizeof(T) == 2) {
-        const uint2 raw = *reinterpret_cast<const uint2*>(p);
+        const uint2 raw = load_vector<STREAM>(reinterpret_cast<const uint2*>(p));
         return make_float4(u2f(raw.x << 16), u2f(raw.x & 0xffff0000u), u2f(raw.y << 16), u2f(raw.y & 0xffff0000u));
     } else {
-        return *reinterpret_cast<const float4*>(p);
+        return load_vector<STREAM>(reinterpret_cast<const float4*>(p));
     }
 }
-template <typename T>
+template <bool STREAM = false, typename T>
 __device__ __forceinline__ void store4(T* p, float4 v) {
     if constexpr (sizeof(T) == 2) {
         const uint32_t lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{v.x, v.y}, v2bf));
         const uint32_t hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{v.z, v.w}, v2bf));
-        *reinterpret_cast<uint2*>(p) = make_uint2(lo, hi);
+        store_vector<STREAM>(reinterpret_cast<uint2*>(p), make_uint2(lo, hi));
     } else {
-        *reinterpret_cast<float4*>(p) = v;
+        store_vector<STREAM>(reinterpret_cast<float4*>(p), v);
     }
 }
 
@@ -100,7 +114,7 @@ inline int rows_per_block(int64_t rows) { return (int)((rows + 1023) / 1024 > 0 
 //   dx_i = f g_i gy_i - x_i f^3 / cols * sum_j gy_j g_j x_j,      dgain_i = sum_rows gy_i x_i f.
 // A workgroup walks rpb rows, RB at a time; thread t owns columns 4 (t + 256 k) .. +3 of each, keeps the rows in registers
 // between the reduction and the update, and adds its columns' gain-gradient terms over the rows: one partial row per workgroup.
-template <typename TG, typename TX, int NK, int RB>
+template <typename TG, typename TX, int NK, int RB, bool STREAM>
 __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const TG* __restrict__ gy, const TX* __restrict__ x,
                                                           const float* __restrict__ gain, const float* __restrict__ factor,
                                                           int64_t rows, int cols, int rpb, InverseRotation rot,
@@ -129,9 +143,9 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const TG* __restrict__
             for (int k = 0; k < NK; ++k) {
                 const int col = (k * 256 + (int)threadIdx.x) * 4;
                 if (col < cols) {  // cols % 32 == 0: the eight lanes of a group of 32 are in or out together
-                    gk[j][k] = load4(gy + r * cols + col);
+                    gk[j][k] = load4<STREAM>(gy + r * cols + col);
                     if (rot.maskbits) gk[j][k] = inverse_rotate_quad<sizeof(TG) == 2>(gk[j][k], rot, r * cols + col);
-                    xk[j][k] = load4(x + r * cols + col);
+                    xk[j][k] = load4<STREAM>(x + r * cols + col);
                 }
             }
         }
@@ -175,11 +189,11 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const TG* __restrict__
                             const uint32_t hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{d.z, d.w}, v2bf));
                             d = make_float4(u2f(lo << 16), u2f(lo & 0xffff0000u), u2f(hi << 16), u2f(hi & 0xffff0000u));
                         }
-                        const float4 sk = load4(skip + (rb + j) * cols + col);
+                        const float4 sk = load4<STREAM>(skip + (rb + j) * cols + col);
                         d = make_float4(d.x + sk.x, d.y + sk.y, d.z + sk.z, d.w + sk.w);
                     }
-                    store4(dx + (rb + j) * cols + col, d);
-                    if (dx_bf16) store4(dx_bf16 + (rb + j) * cols + col, d);  // the gradient of a bf16 summand of x
+                    store4<STREAM>(dx + (rb + j) * cols + col, d);
+                    if (dx_bf16) store4<STREAM>(dx_bf16 + (rb + j) * cols + col, d);  // the gradient of a bf16 summand of x
                 }
             }
         }
@@ -369,7 +383,7 @@ __global__ __launch_bounds__(256) void swiglu_bwd_kernel(const TG* __restrict__ 
 template <typename T>
 __device__ __forceinline__ void load8(const T* p, float (&v)[8]) {
     if constexpr (sizeof(T) == 2) {
-        const uint4 raw = *reinterpret_cast<const uint4*>(p);
+        const uint4 raw = stream_load(reinterpret_cast<const uint4*>(p));
         const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -377,7 +391,7 @@ __device__ __forceinline__ void load8(const T* p, float (&v)[8]) {
             v[2 * i + 1] = u2f(w[i] & 0xffff0000u);
         }
     } else {
-        const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4);
+        const float4 a = stream_load(reinterpret_cast<const float4*>(p)), b = stream_load(reinterpret_cast<const float4*>(p + 4));
         v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
         v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
     }
@@ -388,10 +402,10 @@ __device__ __forceinline__ void store8(T* p, const float (&v)[8]) {
         uint32_t w[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) w[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{v[2 * i], v[2 * i + 1]}, v2bf));
-        *reinterpret_cast<uint4*>(p) = make_uint4(w[0], w[1], w[2], w[3]);
+        stream_store(reinterpret_cast<uint4*>(p), make_uint4(w[0], w[1], w[2], w[3]));
     } else {
-        *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
-        *reinterpret_cast<float4*>(p + 4) = make_float4(v[4], v[5], v[6], v[7]);
+        stream_store(reinterpret_cast<float4*>(p), make_float4(v[0], v[1], v[2], v[3]));
+        stream_store(reinterpret_cast<float4*>(p + 4), make_float4(v[4], v[5], v[6], v[7]));
     }
 }
 template <bool ROUND_BF16>
@@ -436,7 +450,9 @@ __device__ __forceinline__ void inverse_rotate_oct(float (&v)[8], const InverseR
 }
 
 // hidden % 8 == 0: the same arithmetic per element as swiglu_bwd_kernel, half as many memory instructions per element
-// (used when the gradient arrives rotated: there the mask byte per quad of the other kernel is what it saves)
+// (used when the gradient arrives rotated: there the mask byte per quad of the other kernel is what it saves).  Past the caches both
+// ways: a step of 16384 x 4096 x 1536 417.9 -> 405 us (the next launch no longer waits for this one's lines to be written back),
+// by itself 2048 x 1728 10.7 -> 9.3, 4096 x 1728 16.4 -> 14.7, 16384 x 4096 115 either way.
 template <typename TG, typename TH>
 __global__ __launch_bounds__(256) void swiglu_bwd_oct_kernel(const TG* __restrict__ g, const TH* __restrict__ h12,
                                                              int64_t rows, int64_t hidden, InverseRotation rot,
@@ -472,6 +488,12 @@ int64_t rmsnorm_bwd_blocks(int64_t rows, int64_t cols) {
     return (rows + rows_per_block(rows) - 1) / rows_per_block(rows);
 }
 
+// The cooperative kernel's tensors (up to 16 bytes an element) past the caches: dirty lines of a large result are written back during the
+// next launch.  us of a layer's step with a bf16 summand, through the caches and past them: 4096 x 2048 111.6 -> 107.9, 16384 x 2048
+// 339 -> 325, 6144 x 4096 262 -> 256.5, 8192 x 4096 338 -> 328; but 1024 x 3072 69.2 -> 74.7, 2048 x 2048 70.2 -> 75.3: there the step
+// lives in the cache.  (Not in rmsnorm_bwd_rows_kernel: 16384 x 1536 80 us, 89 past them.)
+inline bool past_the_caches(int64_t rows, int64_t cols) { return rows * cols * 16 >= kPastTheCaches; }
+
 template <typename TG, typename TX>
 void launch_rmsnorm_bwd(const void* gy, const void* x, const float* gain, const float* factor, int64_t rows, int cols,
                         const InverseRotation& rot, const void* skip, void* dx, void* dx_bf16, float* partial,
@@ -485,9 +507,19 @@ void launch_rmsnorm_bwd(const void* gy, const void* x, const float* gain, const 
     uint16_t* dxb = reinterpret_cast<uint16_t*>(dx_bf16);
     if (cols <= 768) rmsnorm_bwd_rows_kernel<TG, TX, 3><<<grid, block, 0, stream>>>(g, xp, gain, factor, rows, cols, rot, sk, dxp, dxb, partial);
     else if (rows_kernel_serves(cols)) rmsnorm_bwd_rows_kernel<TG, TX, 6><<<grid, block, 0, stream>>>(g, xp, gain, factor, rows, cols, rot, sk, dxp, dxb, partial);
-    else if (cols <= 2048) rmsnorm_bwd_kernel<TG, TX, 2, 4><<<grid, block, 0, stream>>>(g, xp, gain, factor, rows, cols, rpb, rot, sk, dxp, reinterpret_cast<uint16_t*>(dx_bf16), partial);
-    else if (cols <= 4096) rmsnorm_bwd_kernel<TG, TX, 4, 2><<<grid, block, 0, stream>>>(g, xp, gain, factor, rows, cols, rpb, rot, sk, dxp, reinterpret_cast<uint16_t*>(dx_bf16), partial);
-    else rmsnorm_bwd_kernel<TG, TX, 8, 1><<<grid, block, 0, stream>>>(g, xp, gain, factor, rows, cols, rpb, rot, sk, dxp, reinterpret_cast<uint16_t*>(dx_bf16), partial);
+    else {
+        const auto go = [&](auto nk, auto rb, auto stream_) {
+            rmsnorm_bwd_kernel<TG, TX, decltype(nk)::value, decltype(rb)::value, decltype(stream_)::value>
+                <<<grid, block, 0, stream>>>(g, xp, gain, factor, rows, cols, rpb, rot, sk, dxp, dxb, partial);
+        };
+        const auto by_cols = [&](auto stream_) {
+            if (cols <= 2048) go(std::integral_constant<int, 2>{}, std::integral_constant<int, 4>{}, stream_);
+            else if (cols <= 4096) go(std::integral_constant<int, 4>{}, std::integral_constant<int, 2>{}, stream_);
+            else go(std::integral_constant<int, 8>{}, std::integral_constant<int, 1>{}, stream_);
+        };
+        if (past_the_caches(rows, cols)) by_cols(std::true_type{});
+        else by_cols(std::false_type{});
+    }
 }
 
 }  // namespace

@@ -40,6 +40,7 @@
 #include "qm_jobs.h"
 #include "qm_kernels.h"
 #include "qm_math.h"
+#include "streaming.h"
 #include "quantize_group.h"
 
 namespace qm {
@@ -377,8 +378,8 @@ void launch_rowmajor_wide(int mode, const void* x, int64_t n, float c, const Sig
 // from its neighbour's.  Slot kPieces l + (q ^ swizzle) holds piece q of lane l's group: slot-ordered and group-ordered accesses both
 // spread over all banks.  The last wave of a tensor, if it is not whole, takes its groups lane by lane.
 // What bounds it: HBM.  16384 x 4096 bf16 with mask, blocks of 64: 75 us with codes and scales, every value taken apart by hand; 62
-// without the former and by hardware converts; 47 (5.9 TB/s) with whole lines.  With the straight-through backward behind it 117 -> 95.5,
-// blocks of 32 113 -> 95, stochastic absmax 115 -> 93; 32768 x 8192 446 -> 370.
+// without the former and by hardware converts; 48 with whole lines, 46.3 (6.0 TB/s) with loads and stores past
+// the caches (57 with the stores alone; 6000 x 2048 10.9 -> 10.4).  With the straight-through backward behind it 117 -> 91.
 template <typename T, int MODE, bool WANT_MASK, int HD>
 __global__ __launch_bounds__(256) void quantize_values_kernel(const T* __restrict__ x, int64_t n_groups, Rotation rot, uint64_t seed,
                                                               uint32_t* __restrict__ maskbits, T* __restrict__ values) {
@@ -400,7 +401,7 @@ __global__ __launch_bounds__(256) void quantize_values_kernel(const T* __restric
         const uint4* src = reinterpret_cast<const uint4*>(x + first * 32);
         uint4 raw[kPieces];
 #pragma unroll
-        for (int i = 0; i < kPieces; ++i) raw[i] = src[piece_of_slot(i)];
+        for (int i = 0; i < kPieces; ++i) raw[i] = stream_load(src + piece_of_slot(i));
         job_requests_issued();
 #pragma unroll
         for (int i = 0; i < kPieces; ++i) area[64 * i + lane] = raw[i];
@@ -436,7 +437,7 @@ __global__ __launch_bounds__(256) void quantize_values_kernel(const T* __restric
         wave_settle();
         uint4* dst = reinterpret_cast<uint4*>(values + first * 32);
 #pragma unroll
-        for (int i = 0; i < kPieces; ++i) dst[piece_of_slot(i)] = area[64 * i + lane];
+        for (int i = 0; i < kPieces; ++i) stream_store(dst + piece_of_slot(i), area[64 * i + lane]);
     } else {
 #pragma unroll
         for (int q = 0; q < kPieces; ++q) reinterpret_cast<uint4*>(values + gi * 32)[q] = out[q];

@@ -1,0 +1,57 @@
+"""Kernels that take tensors of 96 MiB and more past the caches: whole calls above that size against the same rows in calls below it."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+BF16, F32 = torch.bfloat16, torch.float32
+
+
+def parts(t, n=2):
+    return [p.contiguous() for p in t.chunk(n)]
+
+
+# the cooperative kernel's three widths (two, four and eight vectors a lane), a width that leaves lanes idle
+@pytest.mark.parametrize("rows,cols", [(3074, 2048), (3001, 2112), (1537, 4096), (770, 8192)])
+@pytest.mark.parametrize("dtype", [BF16, F32])
+def test_rmsnorm_backward(rows, cols, dtype):
+    """Rows do not depend on each other: the same bits.  The gain's gradient: fp32 sums of 1024 or fewer rows a partial sum, then of as many
+    partial sums, in another order: 2^-24 of the absolute terms for each of at most 2048 additions, 40 of them at random signs."""
+    print(f"case rmsnorm backward {rows}x{cols} {dtype}", flush=True)
+    from quartet_amd import kernels as K
+    assert rows * cols * 16 >= 96 << 20 > (rows + 1) // 2 * cols * 16
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    new = lambda *s, dt=F32: torch.randn(*s, generator=gen, device="cuda").to(dt)
+    x, gy, skip, gain = new(rows, cols, dt=dtype), new(rows, cols, dt=BF16), new(rows, cols, dt=dtype), 1 + 0.1 * new(cols)
+    factor = (x.float().square().mean(-1) + 1e-5).rsqrt()
+    mask = torch.randint(0, 256, (rows, cols // 8), generator=gen, device="cuda", dtype=torch.uint8)
+    run = lambda x, gy, skip, factor, mask: K.rmsnorm_backward(gy, x, gain, factor, mask, 0x5A5A1234, BF16, skip=skip, want_bf16_copy=True)
+    whole, halves = run(x, gy, skip, factor, mask), [run(*p) for p in zip(*map(parts, (x, gy, skip, factor, mask)))]
+    assert torch.equal(whole[0], torch.cat([h[0] for h in halves])) and torch.equal(whole[2], torch.cat([h[2] for h in halves]))
+    unmasked = K.masked_hadamard_bwd(gy, 32, BF16, 0x5A5A1234, mask, F32)
+    scale = (unmasked.double() * x.double() * factor.double()[:, None]).abs().sum(0)
+    assert ((whole[1] - sum(h[1] for h in halves)).double().abs() <= 40 * 2.0 ** -24 * scale + 1e-30).all()
+
+
+@pytest.mark.parametrize("rows,cols,hd,dtype", [(12289, 4096, 32, BF16), (6145, 4096, 64, F32), (24577, 2048, 128, BF16)])
+def test_inverse_rotation(rows, cols, hd, dtype):
+    print(f"case inverse rotation {rows}x{cols} hd={hd} {dtype}", flush=True)
+    from quartet_amd import kernels as K
+    g = torch.randn(rows, cols, generator=torch.Generator(device="cuda").manual_seed(hd), device="cuda").to(dtype)
+    mask = torch.randint(0, 256, (rows, cols // 8), device="cuda", dtype=torch.uint8)
+    assert g.numel() * g.element_size() >= 96 << 20
+    run = lambda g, m: K.masked_hadamard_bwd(g, hd, BF16, 0x0F1E2D3C, m)
+    assert torch.equal(run(g, mask), torch.cat([run(*p) for p in zip(parts(g), parts(mask))]))
+
+
+@pytest.mark.parametrize("rows,classes,dtype", [(1573, 32000, BF16), (787, 32003, F32), (1600, 31999, BF16)])
+def test_loss(rows, classes, dtype):
+    """The mean of two halves' means: at most 16 + 10 + 2 fp32 additions of positive losses and a division, twice: 64 roundings."""
+    print(f"case loss {rows}x{classes} {dtype}", flush=True)
+    from quartet_amd import kernels as K
+    gen = torch.Generator(device="cuda").manual_seed(classes)
+    logits = torch.randn(rows, classes, generator=gen, device="cuda").to(dtype)
+    targets = torch.randint(0, classes, (rows,), generator=gen, device="cuda")
+    assert logits.numel() * logits.element_size() >= 96 << 20
+    whole = float(K.cross_entropy(logits, targets, -1))
+    halves = sum(float(K.cross_entropy(a, b, -1)) * len(b) for a, b in zip(parts(logits), parts(targets))) / rows
+    assert abs(whole - halves) <= 64 * 2.0 ** -24 * abs(halves)
