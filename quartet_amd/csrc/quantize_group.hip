@@ -1158,7 +1158,12 @@ struct RmsNormProducer {
     // memory: 4096 x 640 11.7 -> 9.9 us, 16384 x 1536 62 -> 57 (4.7 TB/s; 65 -> 60 inside a layer's step), 32768 x 1024 88 -> 75,
     // 16384 x 4096 166 -> 156 (two passes); 512 x 4096 is latency, 11 us either way.  Requests under per-lane predicates instead
     // of clamped ones cost half as much again.
+    // 121 to 126 registers with a bf16 summand, four waves on a SIMD: the pieces' offsets are one register each, and the gain is requested
+    // when the row has left its own registers (with addresses per tensor and the gain asked for at the start: 133 and 160, three waves).
+    // us inside a layer's step: 32768 x 1024 75.0 -> 65.7, 20000 x 704 36.0 -> 32.2, 16384 x 1536 with the weight 62.0 -> 59.7; latency, the
+    // same either way, at 2048 x 2048 14.4 and 4096 x 640 10.
     typedef float v4 __attribute__((ext_vector_type(4)));
+    typedef uint32_t w2 __attribute__((ext_vector_type(2)));
     __device__ __forceinline__ static v4* area() { return reinterpret_cast<v4*>(job_lds) + (threadIdx.x >> 6) * 512; }
     __device__ __forceinline__ static void read_group(int of_lane, float (&v)[32]) {
 #pragma unroll
@@ -1182,14 +1187,6 @@ struct RmsNormProducer {
         // slot 64 i + wlane is piece `piece` of the group of lane 8 i + wlane / 8: group `sub` + 8 i of the row that 8 i / W picks (uniform).
         // Slots past the row's end are filled from its last group: no branch between the requests.
         const int wlane = seg + lane, sub = wlane >> 3, piece = (wlane & 7) ^ sub;
-        v4 gains[W / 8];
-        if constexpr (kStaged) {
-#pragma unroll
-            for (int i = 0; i < W / 8; ++i) {
-                const int gg = 8 * i + sub < groups ? 8 * i + sub : groups - 1;
-                gains[i] = *reinterpret_cast<const v4*>(gain + gg * 32 + piece * 4);
-            }
-        }
         float acc = 0.0f;
         for (int base = 0; base < groups; base += 64) {
             const int g = base + lane;
@@ -1198,25 +1195,30 @@ struct RmsNormProducer {
                 v4 raw[8];
                 const auto group_of = [&](int i) { return base + 8 * i % W + sub; };
                 const auto row_of = [&](int i) { const int64_t r = wave_row + 8 * i / W; return (r < rows ? r : rows - 1) * cols; };
-                const auto at = [&](int i) { const int gg = group_of(i); return (gg < groups ? gg : groups - 1) * 32 + piece * 4; };
+                // the lane's element as a 32-bit offset from its row's (uniform) start: one register a slot instead of an address per tensor
+                const auto at = [&](int i) { const int gg = group_of(i); return (uint32_t)((gg < groups ? gg : groups - 1) * 32 + piece * 4); };
+                const auto piece_at = [&](auto* t, int i) {   // of four elements
+                    using V = std::conditional_t<sizeof(*t) == 4, v4, w2>;
+                    using B = std::conditional_t<std::is_const_v<std::remove_pointer_t<decltype(t)>>, const char, char>;
+                    return reinterpret_cast<std::conditional_t<std::is_const_v<B>, const V, V>*>(reinterpret_cast<B*>(t + row_of(i)) + at(i) * (uint32_t)sizeof(*t));
+                };
 #pragma unroll
-                for (int i = 0; i < 8; ++i) raw[i] = *reinterpret_cast<const v4*>(x + row_of(i) + at(i));
+                for (int i = 0; i < 8; ++i) raw[i] = *piece_at(x, i);
                 if constexpr (kAdd) {
                     if constexpr (sizeof(TAdd) == 2) {
-                        typedef uint32_t w2 __attribute__((ext_vector_type(2)));
                         w2 more[8];
 #pragma unroll
-                        for (int i = 0; i < 8; ++i) more[i] = *reinterpret_cast<const w2*>(add + row_of(i) + at(i));
+                        for (int i = 0; i < 8; ++i) more[i] = *piece_at(add, i);
 #pragma unroll
                         for (int i = 0; i < 8; ++i)
                             raw[i] = raw[i] + v4{u2f(more[i][0] << 16), u2f(more[i][0] & 0xffff0000u), u2f(more[i][1] << 16), u2f(more[i][1] & 0xffff0000u)};
                     } else {
 #pragma unroll
-                        for (int i = 0; i < 8; ++i) raw[i] = raw[i] + *reinterpret_cast<const v4*>(add + row_of(i) + at(i));
+                        for (int i = 0; i < 8; ++i) raw[i] = raw[i] + *piece_at(add, i);
                     }
 #pragma unroll
                     for (int i = 0; i < 8; ++i)
-                        if (group_of(i) < groups) *reinterpret_cast<v4*>(xsum + row_of(i) + at(i)) = raw[i];
+                        if (group_of(i) < groups) *piece_at(xsum, i) = raw[i];
                 }
 #pragma unroll
                 for (int i = 0; i < 8; ++i) area()[64 * i + wlane] = raw[i];
@@ -1237,6 +1239,14 @@ struct RmsNormProducer {
             if constexpr (kStaged) wave_settle();   // the next pass over the row, or the gain, reuses the area
 #pragma unroll
             for (int k = 0; k < W / 16; ++k) acc = acc + __shfl(s, seg + (lane & 15) + 16 * k, 64);
+        }
+        v4 gains[W / 8];
+        if constexpr (kStaged) {   // not before: 32 registers that the row needs
+#pragma unroll
+            for (int i = 0; i < W / 8; ++i) {
+                const int gg = 8 * i + sub < groups ? 8 * i + sub : groups - 1;
+                gains[i] = *reinterpret_cast<const v4*>(gain + gg * 32 + piece * 4);
+            }
         }
 #pragma unroll
         for (int m = 1; m < 16; m <<= 1) acc = acc + __shfl_xor(acc, m, 64);

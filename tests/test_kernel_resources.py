@@ -56,3 +56,11 @@ def test_backward_quantizers_fit_their_waves_without_scratch(kernels):
     for n, (registers, scratch) in grids.items():
         block = int(re.search(r"RequantTiledJob<\d+, (\d+),", n).group(1))
         assert scratch == 0 and registers <= (96 if block == 32 else 128), (n, registers, scratch)
+
+
+def test_norm_producers_fit_four_waves_without_scratch(kernels):
+    """The RMSNorm in front of a quantizer, fp32 rows with a bf16 residual summand, as the model calls it."""
+    found = {n: v for n, v in kernels.items() if "RmsNormProducer<float, unsigned short>, true" in n}
+    assert len(found) >= 6
+    for n, (registers, scratch) in found.items():
+        assert scratch == 0 and registers <= 128, (n, registers, scratch)
