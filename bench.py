@@ -614,12 +614,13 @@ def counters_to_json(fetch_dir, write_dir, sq_dir=None):
         return re.findall(r"qm::(\w+Job)<", k.split("(")[0]) if "qm::job_kernel<" in k else []
 
     def product(k):
-        """The persistent product's template arguments: element type, stamps, rotation in the epilogue, ragged rows."""
+        """The persistent product's template arguments: element type, stamps, Hadamard block of the rotation in the epilogue (0: none), ragged
+        rows, which of two products in one grid are widened or rotated (0: one product), alpha of one."""
         m = re.search(r"gemm_mxfp4_tn_big4_kernel<([^>]*)>", k)
         return m.group(1).split(", ") if m else None
-    groups = {"gemm_mxfp4_tn": lambda k: product(k) is not None and product(k)[2] == "false",
-              # the instantiation with the masked inverse rotation in its epilogue (the step's two gradient products)
-              "gemm_mxfp4_tn_rotated": lambda k: product(k) is not None and product(k)[2] == "true",
+    groups = {"gemm_mxfp4_tn": lambda k: product(k) is not None and product(k)[2] == "0",
+              # the instantiation with the masked inverse rotation in its epilogue (the step's two gradient products, in one grid)
+              "gemm_mxfp4_tn_rotated": lambda k: product(k) is not None and product(k)[2] != "0",
               "quantize_x_quest_rtn_mask_alone": lambda k: jobs(k) == ["RowmajorTiledJob"],
               "forward_quantizer_pair": lambda k: jobs(k) == ["RowmajorTiledJob"] * 2,
               "backward_quantizers": lambda k: jobs(k) == ["TransposedJob", "RowmajorTiledJob"] + ["RequantTiledJob"] * 2,
@@ -630,6 +631,8 @@ def counters_to_json(fetch_dir, write_dir, sq_dir=None):
         w = [v for k, vs in write.items() if match(k) for v in vs]
         if f and w:
             out[name] = {"fetch_bytes": round(sum(f) / len(f) * fu), "write_bytes": round(sum(w) / len(w) * wu), "dispatches": len(f)}
+            if name == "gemm_mxfp4_tn_rotated" and all(product(k)[4] != "0" for k in fetch if match(k)):
+                out[name]["products"] = 2   # in one launch
             vi = [v for k, vs in valu.items() if match(k) for v in vs]
             wv = [v for k, vs in waves.items() if match(k) for v in vs]
             if vi and wv:
@@ -972,7 +975,8 @@ def main():
         traffic, source = _traffic_entry(prof, "gemm_mxfp4_tn")
         if fused and traffic is not None:
             t_rot, _ = _traffic_entry(prof, "gemm_mxfp4_tn_rotated")
-            if t_rot is not None:   # per launch, as the step runs them: one plain product, two with the rotation (these also read mask bits)
+            if t_rot is not None:   # per product, as the step runs them: one plain, two with the rotation (these also read mask bits)
+                t_rot /= prof["kernels"]["gemm_mxfp4_tn_rotated"].get("products", 1)
                 source = {**source, "plain_product_bytes": traffic, "rotated_product_bytes": t_rot}
                 traffic = round((traffic + 2.0 * t_rot) / 3.0, 1)
         what = "mean of the step's three products, timed inside the step"
