@@ -286,8 +286,10 @@ int qm_dequantize_mxfp4(const uint8_t* codes, const uint8_t* scales, int64_t R, 
  * repeat every 32, for gw alone also gw_dtype == mid_dtype; see qm_gemm_mxfp4_tn_rotated), in the epilogue of the smaller tile kernels (bf16 mid_dtype, any Hadamard block,
  * any gw_dtype), or in the ordered reduction of a product cut into K ranges (any Hadamard block, mid_dtype and gw_dtype);
  * the last two with the arithmetic and roundings of the separate launches.  Elsewhere it is a launch of its own.
- * Where both gradient products (bf16 mid_dtype, padded or tiled layout, the same Hadamard block) run fastest in one launch, they
+ * Where both gradient products (bf16 mid_dtype, padded or tiled layout, no g_matrix) run fastest in one launch, they
  * do: of the 256 x 256 kernel, with its epilogue for gx and for gw, of either gw_dtype, or of the smaller tiles; without K ranges.
+ * That is decided for all forms of a layer's call alike: gw has the same bits with QM_GX_ROTATED and without, and is summed in K
+ * ranges with either gw_dtype or neither.
  * qm_linear_backward_in_one_launch tells (1, 2; 0: they do not; of forward quantizers without column signs).
  */
 size_t qm_packed_operand_bytes(int64_t rows, int64_t cols);

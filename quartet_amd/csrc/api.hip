@@ -436,40 +436,48 @@ bool wide_pair(const qm::TileProduct& x, const qm::ProductChoice& cx, const qm::
     const auto whole = [](const qm::ProductChoice& c) { return c.path == qm::ProductChoice::TILE && c.kind == qm::WIDE_256x256 && c.splits == 1 && c.rotates; };
     return whole(cx) && whole(cw) && qm::gemm_wide_pair_serves(x, w);
 }
-// A gradient product of the backward pass and the kernel that serves it by itself: with the masked inverse rotation of the forward
-// quantizer (into final_dst) where that kernel applies it, otherwise without (into plain.c)
+// The masked inverse rotation of the forward quantizer in a gradient product, into dst
+qm::TileProduct with_rotation(qm::TileProduct p, void* dst, int hd, const uint8_t* mask, const uint32_t* signs, int scale_dtype) {
+    p.c = dst;
+    p.mask = mask;
+    p.hd = hd;
+    p.signs = make_signs(signs, hd);
+    p.rot_c = qm::hadamard_scale(hd, scale_dtype);
+    return p;
+}
+// A gradient product of the backward pass and the kernel that serves it by itself: with that rotation where that kernel applies it,
+// otherwise without (into plain.c)
 struct GradProduct {
     qm::TileProduct p;
     qm::ProductChoice choice;
     int out_dtype;
-    // what a launch of both products would do: this one with the rotation wherever it is wanted
-    qm::TileProduct whole;
-    qm::ProductChoice whole_choice;   // its estimate counts a rotation pass of its own
-    int whole_dtype;                  // -1: not to be had
 };
 GradProduct plan_gradient(const qm::TileProduct& plain, void* final_dst, bool want_rotation, int hd, int mid_dtype, int final_dtype, const uint8_t* mask,
                           const uint32_t* signs, int scale_dtype, void* ws, size_t ws_bytes) {
-    GradProduct g{plain, {}, mid_dtype, plain, {}, want_rotation ? -1 : mid_dtype};
     if (want_rotation && final_dst && aligned(final_dst, 16) && valid_dtype(scale_dtype) && valid_hd(hd) && plain.N % hd == 0) {
-        qm::TileProduct r = plain;
-        r.c = final_dst;
-        r.mask = mask;
-        r.hd = hd;
-        r.signs = make_signs(signs, hd);
-        r.rot_c = qm::hadamard_scale(hd, scale_dtype);
+        const qm::TileProduct r = with_rotation(plain, final_dst, hd, mask, signs, scale_dtype);
         const qm::ProductChoice c = qm::choose_product(r, mid_dtype, final_dtype, ws, ws_bytes);
-        if (c.rotates) return GradProduct{r, c, final_dtype, r, c, final_dtype};
-        g.whole = r;
-        g.whole_choice = c;
-        g.whole_dtype = final_dtype;
+        if (c.rotates) return {r, c, final_dtype};
     }
-    g.choice = qm::choose_product(plain, mid_dtype, mid_dtype, ws, ws_bytes);
-    if (!want_rotation) g.whole_choice = g.choice;
-    return g;
+    return {plain, qm::choose_product(plain, mid_dtype, mid_dtype, ws, ws_bytes), mid_dtype};
 }
-qm::PairChoice plan_pair(const GradProduct& x, const GradProduct& w, int mid_dtype) {
-    if (x.whole_dtype < 0 || w.whole_dtype < 0) return {qm::PairChoice::SEPARATE, 0, 0};
-    return qm::choose_pair(x.whole, x.whole_choice, x.whole_dtype, w.whole, w.whole_choice, w.whole_dtype, mid_dtype);
+// How the two gradient products of a layer on tiled operands share a launch, of bf16 results.  One launch adds a whole contraction up
+// in one chain, launched apart a product may be cut into K ranges, which rounds differently: so a layer's gradients must not change with
+// the form of its call (gx left rotated for the fused kernel behind it, an fp32 or a bf16 weight).  It is decided from what all forms have in
+// common, the extents, the Hadamard blocks and the kind of column signs, with the figures of the form that rotates both into bf16; the
+// weight gradient's type counts where neither product would be cut, whose sums are then the same either way.  The other forms' own estimates are up to
+// 0.05 higher, still below two launches'.
+qm::PairChoice gradient_pair(int64_t T, int64_t I, int64_t O, int hd_x, int hd_w, const uint32_t* signs_x, const uint32_t* signs_w, int gw_dtype) {
+    uint8_t* at = reinterpret_cast<uint8_t*>((uintptr_t)256);   // nothing is read: stand-ins with the alignment that a layer's tensors have
+    const size_t ws_bytes = work_layout(T, I, O, QM_BF16).gemm_ws_bytes;
+    const auto product = [&](int64_t M, int64_t K, int hd, const uint32_t* signs) {
+        return with_rotation(qm::make_product(at, at, at, at, M, I, qm::padded_cols(K), 1.0f, at, QM_LAYOUT_TILED, QM_LAYOUT_TILED), at, hd, at, signs, QM_BF16);
+    };
+    const auto choose = [&](const qm::TileProduct& p, int out) { return qm::choose_product(p, QM_BF16, out, ws_bytes ? at : nullptr, ws_bytes); };
+    const qm::TileProduct x = product(T, O, hd_x, signs_x), w = product(O, T, hd_w, signs_w);
+    const qm::ProductChoice cx = choose(x, QM_BF16), cw = choose(w, QM_BF16);
+    if (gw_dtype != QM_BF16 && cx.splits == 1 && cw.splits == 1) return qm::choose_pair(x, cx, QM_BF16, w, choose(w, gw_dtype), gw_dtype);
+    return qm::choose_pair(x, cx, QM_BF16, w, cw, QM_BF16);
 }
 }
 }  // namespace
@@ -496,14 +504,15 @@ size_t qm_linear_backward_workspace_bytes(int64_t T, int64_t I, int64_t O, int m
 int qm_linear_backward_in_one_launch(int64_t T, int64_t I, int64_t O, int hd_x, int hd_w, int gw_dtype, int rotated_flags) {
     if (T <= 0 || I <= 0 || O <= 0 || I % 32 || O % 32 || T % 32 || !valid_hd(hd_x) || !valid_hd(hd_w) || !valid_dtype(gw_dtype)) return 0;
     if (T >= (1ll << 31) || I >= (1ll << 31) || O >= (1ll << 31)) return 0;
-    // nothing is read: stand-ins with the alignment that qm_linear_backward asks for
-    uint8_t* at = reinterpret_cast<uint8_t*>((uintptr_t)256);
-    const size_t ws = work_layout(T, I, O, QM_BF16).gemm_ws_bytes;
-    const auto plan = [&](int64_t M, int64_t K, bool rotate, int hd, int out) {
-        return plan_gradient(qm::make_product(at, at, at, at, M, I, qm::padded_cols(K), 1.0f, at, QM_LAYOUT_TILED, QM_LAYOUT_TILED), at, rotate, hd, QM_BF16, out, at,
-                             nullptr, QM_BF16, ws ? at : nullptr, ws);
+    if (I % hd_x || I % hd_w) return 0;
+    const qm::PairChoice pair = gradient_pair(T, I, O, hd_x, hd_w, nullptr, nullptr, gw_dtype);
+    uint8_t* at = reinterpret_cast<uint8_t*>((uintptr_t)256);   // nothing is read
+    const auto product = [&](int64_t M, int64_t K, bool rotate, int hd) {
+        const qm::TileProduct p = qm::make_product(at, at, at, at, M, I, qm::padded_cols(K), 1.0f, at, QM_LAYOUT_TILED, QM_LAYOUT_TILED);
+        return rotate ? with_rotation(p, at, hd, at, nullptr, QM_BF16) : p;
     };
-    return (int)plan_pair(plan(T, O, !(rotated_flags & QM_GX_ROTATED), hd_x, QM_BF16), plan(O, T, !(rotated_flags & QM_GW_ROTATED), hd_w, gw_dtype), QM_BF16).path;
+    const qm::TileProduct x = product(T, O, !(rotated_flags & QM_GX_ROTATED), hd_x), w = product(O, T, !(rotated_flags & QM_GW_ROTATED), hd_w);
+    return qm::pair_serves(pair, x, QM_BF16, w, gw_dtype) ? (int)pair.path : 0;
 }
 
 int qm_linear_forward(const void* x, int x_dtype, const void* w, int w_dtype, int64_t T, int64_t I, int64_t O, int hd_x,
@@ -811,14 +820,25 @@ int qm_linear_backward_seeded(const void* e, int e_dtype, int64_t T, int64_t I, 
     if (codes_layout == QM_LAYOUT_TILED && (T % 128 || I % 128 || O % 128))
         return fail(QM_ERR_INVALID, "qm_linear_backward: QM_LAYOUT_TILED needs T, I, O multiples of 128 (QM_LAYOUT_PADDED takes any multiples of 32)");
     const int64_t Kx = tiled ? qm::padded_cols(O) : O, Kw = tiled ? qm::padded_cols(T) : T;
-    const auto plan_product = [&](size_t ac, size_t as, size_t bc, size_t bs, int64_t M, int64_t N, int64_t K, void* plain_dst, void* final_dst,
-                                  bool want_rotation, int hd, int final_dtype, const uint8_t* mask, const uint32_t* signs, int scale_dtype) {
-        const int kl = kernel_layout(codes_layout);
-        return plan_gradient(qm::make_product(k + ac, k + as, k + bc, k + bs, M, N, K, alpha, plain_dst, kl, kl), final_dst, want_rotation, hd, mid_dtype, final_dtype,
-                             mask, signs, scale_dtype, gws, wl.gemm_ws_bytes);
+    const int kl = kernel_layout(codes_layout);
+    const bool blocks_ok = valid_hd(hd_x) && valid_hd(hd_w) && I % hd_x == 0 && I % hd_w == 0 && valid_dtype(x_scale_dtype) && valid_dtype(w_scale_dtype);
+    const qm::PairChoice pair = tiled && !g_matrix && mid_dtype == QM_BF16 && blocks_ok ? gradient_pair(T, I, O, hd_x, hd_w, signs_x, signs_w, gw_dtype)
+                                                                                        : qm::PairChoice{qm::PairChoice::SEPARATE, 0, 0};
+    const qm::TileProduct gx_plain = qm::make_product(k + wl.ec, k + wl.es, k + wl.wtc, k + wl.wts, T, I, Kx, alpha, gx_product, kl, kl);
+    const qm::TileProduct gw_plain = qm::make_product(k + wl.etc, k + wl.ets, k + wl.xtc, k + wl.xts, O, I, Kw, alpha, gw_product, kl, kl);
+    qm::TileProduct gx_whole = gx_plain, gw_whole = gw_plain;
+    if (pair.path != qm::PairChoice::SEPARATE) {
+        if (!gx_rotated) gx_whole = with_rotation(gx_plain, gx, hd_x, px + lx.m, signs_x, x_scale_dtype);
+        if (!gw_rotated) gw_whole = with_rotation(gw_plain, gw, hd_w, pw + lw.m, signs_w, w_scale_dtype);
+    }
+    const bool together = qm::pair_serves(pair, gx_whole, mid_dtype, gw_whole, gw_dtype);
+    // a call whose form that launch does not take (no rotation at all) runs two, without K ranges like the others of its layer
+    void* cuts = pair.path == qm::PairChoice::SEPARATE ? gws : nullptr;
+    const auto plan = [&](const qm::TileProduct& plain, void* dst, bool rotated, int hd, int dtype, const uint8_t* mask, const uint32_t* signs, int scale_dtype) {
+        return together ? GradProduct{} : plan_gradient(plain, dst, !rotated, hd, mid_dtype, dtype, mask, signs, scale_dtype, cuts, wl.gemm_ws_bytes);
     };
-    const GradProduct gx_plan = plan_product(wl.ec, wl.es, wl.wtc, wl.wts, T, I, Kx, gx_product, gx, !gx_rotated, hd_x, mid_dtype, px + lx.m, signs_x, x_scale_dtype);
-    const GradProduct gw_plan = plan_product(wl.etc, wl.ets, wl.xtc, wl.xts, O, I, Kw, gw_product, gw, !gw_rotated, hd_w, gw_dtype, pw + lw.m, signs_w, w_scale_dtype);
+    const GradProduct gx_plan = plan(gx_plain, gx, gx_rotated, hd_x, mid_dtype, px + lx.m, signs_x, x_scale_dtype);
+    const GradProduct gw_plan = plan(gw_plain, gw, gw_rotated, hd_w, gw_dtype, pw + lw.m, signs_w, w_scale_dtype);
     const bool gx_fused = gx_plan.choice.rotates, gw_fused = gw_plan.choice.rotates;
     const auto run = [&](const GradProduct& g) {
         return from_hip(qm::run_product(g.choice, g.p, mid_dtype, g.out_dtype, gws, hs), "qm_linear_backward");
@@ -826,7 +846,6 @@ int qm_linear_backward_seeded(const void* e, int e_dtype, int64_t T, int64_t I, 
     const auto product_gx = [&]() { return run(gx_plan); };
     const auto product_gw = [&]() { return run(gw_plan); };
     if (g_matrix) {
-        const int kl = kernel_layout(codes_layout);
         // a dense rotation in the gradient quantizer (rerotate="O32"): the same eight steps on the dense-rotation kernels
         if (hd_g != 32 || T % 128 || I % 128 || O % 128)
             return fail(QM_ERR_INVALID, "qm_linear_backward: a dense gradient rotation needs hd_g == 32 and T, I, O multiples of 128 "
@@ -862,8 +881,7 @@ int qm_linear_backward_seeded(const void* e, int e_dtype, int64_t T, int64_t I, 
         const qm::ErrorArgs ae{e, e_dtype, T, O, seeds[0], seeds[2], k + wl.ec, k + wl.es, k + wl.etc, k + wl.ets};
         rc = from_hip(qm::quantize_layer_backward(ae, hd_g, make_signs(signs_g, hd_g), g_mode, rx, rw, seed_base, hs), "qm_linear_backward");
         if (rc) return rc;
-        if (const qm::PairChoice pair = plan_pair(gx_plan, gw_plan, mid_dtype); pair.path != qm::PairChoice::SEPARATE)
-            return from_hip(qm::run_pair(pair, gx_plan.whole, gx_plan.whole_dtype, gw_plan.whole, gw_plan.whole_dtype, hs), "qm_linear_backward");
+        if (together) return from_hip(qm::run_pair(pair, gx_whole, mid_dtype, gw_whole, gw_dtype, hs), "qm_linear_backward");
         rc = product_gx();
         if (rc) return rc;
         rc = product_gw();

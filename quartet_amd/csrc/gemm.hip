@@ -1247,7 +1247,7 @@ ProductChoice choose_product(const TileProduct& p, int c_dtype, int rot_out_dtyp
     if (!persistent && !tiles_ok) return {ProductChoice::GENERIC, 0, 1, false};
     const ShapePlan& plan = plan_of_shape(M, N, K, persistent, tiles_ok, e5m2);
     // a cut into K ranges rounds differently: whether to make it is decided on the product alone, so that a product and the
-    // same product with the rotation agree
+    // same product with the rotation agree (a layer's two gradients may share a launch instead, without cuts: see gradient_pair)
     if (plan.cut_bytes && workspace && plan.cut_bytes <= workspace_bytes && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0) {
         ProductChoice c = plan.cut.choice;
         c.rotates = rotate;
@@ -1371,17 +1371,17 @@ hipError_t launch_pair_as(const TileProduct& lng, const Big4Other& other, const 
 // 291 -> 287), what is gained being the idle part of each product's last round, or writing and reading partial sums; none lies
 // between 0.94 and 1, near which the estimates (6 % off on average) no longer tell.
 constexpr double kPairMargin = 0.97;
-double persistent_pair_cost(const TileProduct& x, int x_out, const TileProduct& w, int w_out, int cus) {
+bool persistent_pair_serves(const TileProduct& x, int x_out, const TileProduct& w, int w_out) {
     const auto serves = [](const TileProduct& p, int out) {
         return p.a_tiled && p.b_tiled && (p.mask ? persistent_rotates(p) : out == BF16) && persistent_serves(p.M, p.N, p.K, p.a_scales, p.b_scales, p.c);
     };
-    if (!serves(x, x_out) || !serves(w, w_out)) return 1e30;
-    const int hd = x.mask ? x.hd : w.hd;
-    if (x.mask && w.mask ? x.hd != w.hd : hd != 32) return 1e30;
-    if (cus < 8 || big_tiles(x) + big_tiles(w) < cus) return 1e30;
+    const int hd = x.mask ? x.hd : w.hd, cus = device_cus();
+    return serves(x, x_out) && serves(w, w_out) && (x.mask && w.mask ? x.hd == w.hd : hd == 32) && cus >= 8 && big_tiles(x) + big_tiles(w) >= cus;
+}
+double persistent_pair_cost(const TileProduct& x, int x_out, const TileProduct& w, int w_out, int cus) {
     int rounds;
     const bool x_long = x.K > w.K;
-    double cost = kLaunch + pair_makespan(x_long ? x : w, x_long ? w : x, cus, &rounds) + persistent_rotate_cost(hd);
+    double cost = kLaunch + pair_makespan(x_long ? x : w, x_long ? w : x, cus, &rounds) + persistent_rotate_cost(x.mask ? x.hd : w.hd);
     if (x.mask && x_out != BF16) cost += (double)x.M * x.N * 2 / kWideStores;
     if (w.mask && w_out != BF16) cost += (double)w.M * w.N * 2 / kWideStores;
     return cost;
@@ -1415,11 +1415,16 @@ double tile_pair_cost(const TileProduct& x, int x_out, const PairTile& kx, const
     if (w.mask && w_out != BF16) cost += (double)w.M * w.N * 2 / kWideStores;
     return cost;
 }
-PairChoice choose_pair(const TileProduct& x, const ProductChoice& cx, int x_out, const TileProduct& w, const ProductChoice& cw, int w_out, int c_dtype) {
+bool pair_serves(const PairChoice& c, const TileProduct& x, int x_out, const TileProduct& w, int w_out) {
+    if (c.path == PairChoice::SEPARATE || x.N != w.N || x.alpha != w.alpha || x.b_e5m2 || w.b_e5m2 || (!x.mask && !w.mask)) return false;
+    if (c.path == PairChoice::PERSISTENT) return persistent_pair_serves(x, x_out, w, w_out);
+    return x.K > w.K ? gemm_tile_pair_serves(x, c.kind_x, w, c.kind_w) : gemm_tile_pair_serves(w, c.kind_w, x, c.kind_x);
+}
+PairChoice choose_pair(const TileProduct& x, const ProductChoice& cx, int x_out, const TileProduct& w, const ProductChoice& cw, int w_out) {
     PairChoice best{PairChoice::SEPARATE, 0, 0};
-    if (c_dtype != BF16 || x.N != w.N || x.alpha != w.alpha || x.b_e5m2 || w.b_e5m2 || (!x.mask && !w.mask)) return best;
     const int cus = device_cus();
-    const double apart = cx.cost + cw.cost, one = persistent_pair_cost(x, x_out, w, w_out, cus);
+    const double apart = cx.cost + cw.cost;
+    const double one = pair_serves({PairChoice::PERSISTENT, 0, 0}, x, x_out, w, w_out) ? persistent_pair_cost(x, x_out, w, w_out, cus) : 1e30;
     double cost = 1e30;
     if (one < kPairMargin * apart) {
         cost = 1.1 * one;   // it is the more hopeful one of the two estimates
@@ -1427,7 +1432,7 @@ PairChoice choose_pair(const TileProduct& x, const ProductChoice& cx, int x_out,
     }
     for (const PairTile& kx : kPairTiles)
         for (const PairTile& kw : kPairTiles)
-            if (x.K > w.K ? gemm_tile_pair_serves(x, kx.kind, w, kw.kind) : gemm_tile_pair_serves(w, kw.kind, x, kx.kind)) {
+            if (pair_serves({PairChoice::TILE, kx.kind, kw.kind}, x, x_out, w, w_out)) {
                 const double c = tile_pair_cost(x, x_out, kx, w, w_out, kw, cus);
                 if (c < kTilePairMargin * apart && c < cost) {
                     cost = c;

@@ -274,7 +274,9 @@ struct PairChoice {
     enum Path : int { SEPARATE = 0, PERSISTENT = 1, TILE = 2 } path;
     int kind_x, kind_w;   // TileKinds
 };
-PairChoice choose_pair(const TileProduct& x, const ProductChoice& cx, int x_out, const TileProduct& w, const ProductChoice& cw, int w_out, int c_dtype);
+PairChoice choose_pair(const TileProduct& x, const ProductChoice& cx, int x_out, const TileProduct& w, const ProductChoice& cw, int w_out);
+// whether that launch takes these products: one of them with its rotation at least
+bool pair_serves(const PairChoice& c, const TileProduct& x, int x_out, const TileProduct& w, int w_out);
 hipError_t run_pair(const PairChoice& c, const TileProduct& x, int x_out, const TileProduct& w, int w_out, hipStream_t stream);
 // the rotation in the persistent kernel's bf16 epilogue (Hadamard block 32)
 bool gemm_persistent_rotates(const uint8_t* a_scales, const uint8_t* b_scales, int64_t M, int64_t N, int64_t K);

@@ -89,6 +89,28 @@ def check_gradients(monkeypatch, T, I, O, hd, gx_rotated, gw_dtype, path, sx, sw
         assert bool((far <= 2.0 ** -7 * want.float().abs() + 2.0 ** -20 * group).all())
 
 
+# a weight gradient that launched by itself is cut into K ranges (whether it is, and by which kernel, is near the line of the choice),
+# one that is not, one that two launches serve
+@pytest.mark.parametrize("T,I,O", [(32768, 640, 3456), (16480, 1728, 640), (4096, 2048, 4608), (16384, 5504, 512)])
+def test_a_fused_layer_has_the_unfused_ones_weight_gradient(monkeypatch, T, I, O):
+    """Bit for bit, whether the input gradient is rotated back by its product or left rotated for the kernel behind it."""
+    print(f"case weight gradient of fused and unfused {T}x{I}x{O}", flush=True)
+    from quartet_amd import kernels as K
+    monkeypatch.setattr(K, "_layout", lambda tiled: QM_LAYOUT_PADDED)
+    dev, bf16 = "cuda:0", torch.bfloat16
+    x = make_input(T, I, bf16, seed=21).to(dev)
+    w = make_input(O, I, bf16, seed=22, scale=0.02).to(dev)
+    e = make_input(T, O, bf16, seed=23, scale=1e-2, outlier_frac=0).to(dev)
+    _, px, pw = K.linear_forward(x, w, 32, 0x5A5A5A5A, 32, 0x0F0F1234, bf16, True)
+    grads = {}
+    for rotated in (False, True):
+        for dtype in (bf16, torch.float32):
+            grads[rotated, dtype] = K.linear_backward(e, px, pw, T, I, O, 32, 0x5A5A5A5A, 32, 0x0F0F1234, 32, 0x13572468, K.QM_ABSMAX_SR, [11, 12, 13, 14],
+                                                      bf16, bf16, bf16, bf16, bf16, True, gx_rotated=rotated, gw_dtype=dtype)[1]
+    for dtype in (bf16, torch.float32):
+        assert torch.equal(grads[False, dtype], grads[True, dtype])
+
+
 def test_which_gradients_share_a_launch():
     """Two launches (0), one of the 256 x 256 kernel (1), one of smaller tiles (2)."""
     from quartet_amd import _lib
