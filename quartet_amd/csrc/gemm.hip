@@ -1364,19 +1364,31 @@ hipError_t launch_pair_as(const TileProduct& lng, const Big4Other& other, const 
 }  // namespace
 
 // Served: both products by the persistent kernel, tiled, with at least one tile per CU between them (fewer leave CUs idle, which
-// smaller tiles and K ranges do not); bf16 results, plain or with the rotation (both over the same block; beside a
-// plain one over 32), one of them with it, and only rotated ones widened.  Worth it where the estimate of the one launch is clearly below the sum of the two products' own.  Timed
-// against two launches, whole training steps: 52 shapes from 0.62 to 0.94 of that sum are 0.99 to 1.19 times as fast (mean 1.05; 4096 x
-// 2048 x 4096 116 us, now 104; 16384 x 1536 x 4608 behind its norm 471 -> 453; 16384 x 4096 x 1536 behind SwiGLU 457 -> 431; 8192 x 4096^2
-// 291 -> 287), what is gained being the idle part of each product's last round, or writing and reading partial sums; none lies
-// between 0.94 and 1, near which the estimates (6 % off on average) no longer tell.
-constexpr double kPairMargin = 0.97;
+// smaller tiles and K ranges do not) and eight K steps a tile (with four the larger product is bound by its stores, 541 MB of them in
+// 24576 x 11008 x 512, which long tiles beside it leave to fewer CUs: 666 us, 632 in two launches); bf16 results, plain or with the rotation
+// (both over the same block; beside a plain one over 32), one of them with it, and only rotated ones widened.  What is gained is the idle part
+// of each product's last round, or writing and reading partial sums.  Worth it where the estimate of the one launch is below this part
+// of the sum of the two products' own; whole training steps, two launches against one:
+//   both on this kernel apart, too: one estimate on both sides.  8192 x 4096^2 (0.94) 294 -> 289, 16384 x 4096^2 and 4096 x 8192^2 (0.97)
+//   545 -> 541 and 518 -> 517; of ten shapes from 0.94 to 0.98 one is slower, by 1.2 %.
+constexpr double kPairLike = 0.97;
+//   one of them cut into K ranges: 16384 x 1728 x 4096 (0.90) 333 -> 311, 32768 x 2048 x 3072 (0.91) 509 -> 502, 24576 x 1152 x 4608 (0.93)
+//   410 -> 400; from 0.936 to 0.956 as many are slower (24576 x 6144 x 1152 with an fp32 weight 533 -> 553) as are faster (24576 x 1920 x 3456 437 -> 414).
+constexpr double kPairCut = 0.935;
+//   one of them whole on the tile kernels: 16480 x 3456 x 2048 (0.80) 342 -> 307, 12288 x 7168 x 1152 (0.87) 315 -> 300; 8192 x 7168 x 1152
+//   (0.89) is even (219 -> 221 on one card, 221 -> 217 on another), 4096 x 2048 x 5504 (0.90) 141.5 -> 143.5, 4096 x 4096 x 4608 (0.94) 203 -> 213.
+constexpr double kPairUnlike = 0.89;
+double pair_margin(const ProductChoice& cx, const ProductChoice& cw) {
+    if (cx.splits > 1 || cw.splits > 1) return kPairCut;
+    return cx.path == ProductChoice::PERSISTENT && cw.path == ProductChoice::PERSISTENT ? kPairLike : kPairUnlike;
+}
 bool persistent_pair_serves(const TileProduct& x, int x_out, const TileProduct& w, int w_out) {
     const auto serves = [](const TileProduct& p, int out) {
         return p.a_tiled && p.b_tiled && (p.mask ? persistent_rotates(p) : out == BF16) && persistent_serves(p.M, p.N, p.K, p.a_scales, p.b_scales, p.c);
     };
     const int hd = x.mask ? x.hd : w.hd, cus = device_cus();
-    return serves(x, x_out) && serves(w, w_out) && (x.mask && w.mask ? x.hd == w.hd : hd == 32) && cus >= 8 && big_tiles(x) + big_tiles(w) >= cus;
+    return serves(x, x_out) && serves(w, w_out) && (x.mask && w.mask ? x.hd == w.hd : hd == 32) && cus >= 8 && big_tiles(x) + big_tiles(w) >= cus &&
+           x.K >= 8 * kBK && w.K >= 8 * kBK;
 }
 double persistent_pair_cost(const TileProduct& x, int x_out, const TileProduct& w, int w_out, int cus) {
     int rounds;
@@ -1387,13 +1399,19 @@ double persistent_pair_cost(const TileProduct& x, int x_out, const TileProduct& 
     return cost;
 }
 // What a tile costs its CU among others of a pair, in us: a K step, the boundary, the rotation; and a K step of a tile whose CU has
-// others beside it, and when they are done; its half of the launch, first fill and drain.  Fitted to 20 shapes from 512 x 640 x 1920 to 32768 x 1536 x 1536.
+// others beside it, of up to 12 steps (in their boundaries for a third of their time and more) and of more, and when they are done; its
+// half of the launch, first fill and drain.  Fitted to 20 shapes from 512 x 640 x 1920 to 32768 x 1536 x 1536; the fifth figure to weight gradients of
+// 192 and 256 steps beside tiles of 27 and 32: 32768 x 640 x 3456 and 24576 x 640 x 4096, which take 332 and 368 us a step in two launches
+// (the gradient in three K ranges), 338 and 374 in one.
 struct PairTile {
     int kind, bm;   // as many columns as rows
-    double step, boundary, rotate, beside, after, launch;
+    double step, boundary, rotate, beside, beside_long, after, launch;
 };
-constexpr PairTile kPairTiles[] = {{TILE_128x128, 128, 0.26, 0.99, 0.63, 0.37, 0.25, 3.5}, {TILE_64x64, 64, 0.129, 0.36, 0.19, 0.30, 0.14, 2.0}};
-constexpr double kTilePairMargin = 0.9;   // on 60 other shapes: at worst 0.995 times as fast, GPU time of the backward pass 0.92 of two launches' on average
+constexpr int kShortPairSteps = 12;
+constexpr PairTile kPairTiles[] = {{TILE_128x128, 128, 0.26, 0.99, 0.63, 0.37, 0.45, 0.25, 3.5}, {TILE_64x64, 64, 0.129, 0.36, 0.19, 0.30, 0.30, 0.14, 2.0}};
+// 60 other shapes: GPU time of the backward pass 0.92 of two launches' on average.  19 more from 0.80 to 0.90: whole steps 1.02 to 1.14 times as
+// fast (16480 x 1728 x 640 122 -> 114.5, 24576 x 4608 x 640 324 -> 296); where gx is left rotated for the kernel behind it, 0.99 to 1.09
+constexpr double kTilePairMargin = 0.9;
 // Tiles go to the CUs as they become free, the longer contraction's first: every CU its share of those, then the others to even it
 // out.  A tile of very many steps is still running when the others are done.
 double tile_pair_cost(const TileProduct& x, int x_out, const PairTile& kx, const TileProduct& w, int w_out, const PairTile& kw, int cus) {
@@ -1409,7 +1427,7 @@ double tile_pair_cost(const TileProduct& x, int x_out, const PairTile& kx, const
     const double even = mean + (ts > 0 ? 0.5 * cs : 0.0);
     double all = most_long > even ? most_long : even;
     if (tl % cus == 0) all = (double)(tl / cus) * cl + (double)((ts + cus - 1) / cus) * cs;
-    const double left = lng.K / kBK - all / kl.beside;
+    const double left = lng.K / kBK - all / (sht.K / kBK <= kShortPairSteps ? kl.beside : kl.beside_long);
     double cost = kx.launch + kw.launch + all + (left > 0.0 ? left * kl.after : 0.0);
     if (x.mask && x_out != BF16) cost += (double)x.M * x.N * 2 / kWideStores;
     if (w.mask && w_out != BF16) cost += (double)w.M * w.N * 2 / kWideStores;
@@ -1426,7 +1444,7 @@ PairChoice choose_pair(const TileProduct& x, const ProductChoice& cx, int x_out,
     const double apart = cx.cost + cw.cost;
     const double one = pair_serves({PairChoice::PERSISTENT, 0, 0}, x, x_out, w, w_out) ? persistent_pair_cost(x, x_out, w, w_out, cus) : 1e30;
     double cost = 1e30;
-    if (one < kPairMargin * apart) {
+    if (one < pair_margin(cx, cw) * apart) {
         cost = 1.1 * one;   // it is the more hopeful one of the two estimates
         best = {PairChoice::PERSISTENT, 0, 0};
     }
