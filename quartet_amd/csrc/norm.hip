@@ -68,9 +68,15 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const float* __restri
 // cols % 4 == 0, cols <= 4096; x, gain, out (fp32) and an fp32 summand 16-byte, bf16 ones 8-byte aligned
 hipError_t rmsnorm_rows(const float* x, const void* add, int add_dtype, const float* gain, float eps, int64_t rows, int64_t cols, void* out, int out_dtype,
                         hipStream_t stream) {
-    const dim3 grid((unsigned)((rows + 3) / 4)), block(256);
+    constexpr int64_t kRows = 1 << 25;   // of a launch: a grid has fewer than 2^32 threads, 64 a row
     const auto go = [&](auto nv, const auto* a, auto* o) {
-        rmsnorm_rows_kernel<decltype(nv)::value><<<grid, block, 0, stream>>>(x, a, gain, eps, rows, (int)cols, o);
+        for (int64_t r = 0; r < rows; r += kRows) {
+            using A = std::remove_const_t<std::remove_pointer_t<decltype(a)>>;
+            const A* ar = nullptr;
+            if constexpr (!std::is_void<A>::value) ar = a + r * cols;
+            const int64_t n = rows - r < kRows ? rows - r : kRows;
+            rmsnorm_rows_kernel<decltype(nv)::value><<<dim3((unsigned)((n + 3) / 4)), dim3(256), 0, stream>>>(x + r * cols, ar, gain, eps, n, (int)cols, o + r * cols);
+        }
     };
     const auto by_out = [&](auto nv, const auto* a) {
         if (out_dtype == BF16) go(nv, a, static_cast<uint16_t*>(out));

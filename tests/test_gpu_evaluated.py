@@ -137,6 +137,20 @@ def test_last_norm(rows, cols, add_dtype, out_dtype):
     assert np.all(err <= 25 * 2.0 ** -24 + (2.0 ** -8 if out_dtype == BF16 else 0.0))
 
 
+def test_last_norm_of_more_rows_than_a_grid_holds():
+    """64 threads a row and fewer than 2^32 threads in a launch: every row past 2^25 and 2^26 is what it is by itself."""
+    from quartet_amd import kernels as K
+    rows = (1 << 26) + 5
+    print(f"case last norm of {rows} rows", flush=True)
+    x = torch.randn(rows, 4, device="cuda:0", generator=torch.Generator("cuda:0").manual_seed(2))
+    add = torch.randn(rows, 4, device="cuda:0", generator=torch.Generator("cuda:0").manual_seed(3)).to(BF16)
+    gain = torch.tensor([0.5, 1.0, 1.5, 2.0], device="cuda:0")
+    got = K.rmsnorm(x, gain, 1e-5, add, BF16)
+    for at in (0, (1 << 25) - 4, 1 << 25, (1 << 26) - 4, 1 << 26):
+        part = slice(at, at + 9)
+        assert torch.equal(got[part], K.rmsnorm(x[part].contiguous(), gain, 1e-5, add[part].contiguous(), BF16))
+
+
 def test_last_norm_of_a_model_takes_the_module_where_somebody_listens_or_asks_for_gradients():
     from quartet_amd.fused import rmsnorm
     from quartet_amd.llama import RMSNorm
