@@ -153,7 +153,10 @@ hipError_t cross_entropy_mean(const void* logits, int dtype, const int64_t* targ
                               float* losses, float* loss, hipStream_t stream) {
     const auto go = [&](const auto* x, auto past) {
         using T = std::remove_const_t<std::remove_pointer_t<decltype(x)>>;
-        cross_entropy_rows_kernel<T, decltype(past)::value><<<dim3((unsigned)rows), dim3(kLossThreads), 0, stream>>>(x, targets, classes, ignore, losses);
+        constexpr int64_t kRows = 1 << 23;   // of a launch: a grid has fewer than 2^32 threads
+        for (int64_t r = 0; r < rows; r += kRows)
+            cross_entropy_rows_kernel<T, decltype(past)::value><<<dim3((unsigned)(rows - r < kRows ? rows - r : kRows)), dim3(kLossThreads), 0, stream>>>(
+                x + r * classes, targets + r, classes, ignore, losses + r);
     };
     const auto by_size = [&](const auto* x) {
         if (rows * classes * (int64_t)sizeof(*x) >= kPastTheCaches) go(x, std::true_type{});

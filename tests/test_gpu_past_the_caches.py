@@ -55,3 +55,26 @@ def test_loss(rows, classes, dtype):
     whole = float(K.cross_entropy(logits, targets, -1))
     halves = sum(float(K.cross_entropy(a, b, -1)) * len(b) for a, b in zip(parts(logits), parts(targets))) / rows
     assert abs(whole - halves) <= 64 * 2.0 ** -24 * abs(halves)
+
+
+def test_loss_of_more_rows_than_a_grid_holds():
+    """256 threads a row and fewer than 2^32 threads in a launch: the rows' losses past 2^23 and 2^24 are those of the rows by themselves."""
+    from quartet_amd import _lib
+    rows, classes = (1 << 24) + 3, 5
+    print(f"case loss of {rows} rows", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    logits = torch.randn(rows, classes, generator=gen, device="cuda").to(BF16)
+    targets = torch.randint(0, classes, (rows,), generator=gen, device="cuda")
+
+    def run(at, n):
+        losses, loss = torch.full((n,), -1.0, device="cuda"), torch.empty((), device="cuda")
+        part, t = logits[at:at + n], targets[at:at + n]   # the same addresses
+        rc = _lib.lib().qm_cross_entropy(part.data_ptr(), _lib.QM_BF16, t.data_ptr(), n, classes, -1, losses.data_ptr(), loss.data_ptr(), None)
+        _lib.check(rc, "qm_cross_entropy")
+        torch.cuda.synchronize()
+        return losses, float(loss)
+    losses, mean = run(0, rows)
+    for at in (0, (1 << 23) - 4, 1 << 23, (1 << 24) - 4):
+        assert torch.equal(losses[at:at + 7], run(at, 7)[0])
+    assert bool((losses > 0).all())
+    assert abs(mean - float(losses.double().mean())) <= ((rows >> 10) + 12) * 2.0 ** -24 * mean
