@@ -378,11 +378,18 @@ void launch_rowmajor_wide(int mode, const void* x, int64_t n, float c, const Sig
 // from its neighbour's.  Slot kPieces l + (q ^ swizzle) holds piece q of lane l's group: slot-ordered and group-ordered accesses both
 // spread over all banks.  The last wave of a tensor, if it is not whole, takes its groups lane by lane.
 // What bounds it: HBM.  16384 x 4096 bf16 with mask, blocks of 64: 75 us with codes and scales, every value taken apart by hand; 62
-// without the former and by hardware converts; 48 with whole lines, 46.3 (6.0 TB/s) with loads and stores past
-// the caches (57 with the stores alone; 6000 x 2048 10.9 -> 10.4).  With the straight-through backward behind it 117 -> 91.
+// without the former and by hardware converts; 48 with whole lines.
+// past_in, past_out: loads and stores past the caches, by size: the values are what the next launch reads.  us in bf16 with a product
+// by 1024 columns behind it, an elementwise reader, and the straight-through backward alone, which leaves the values unread;
+// neither, loads, both:
+//   8192 x 4096 (64 MiB)    77.2 79.2 84.5    42.3 43.2 46.6    60 58 60
+//   16384 x 4096 (128 MiB) 129.3 130.3 137.2   84.0 82.0 86.7    101.5 87.9 90.3
+//   24576 x 4096 (192 MiB) 220.9 212.0 220.9    140.4 126.3 136.5    149.6 135.2 130.4
+//   32768 x 4096 (256 MiB) 267.3 261.7 268.0   184.8 186.5 183.4    197.3 177.4 174.3
+//   32768 x 8192 (512 MiB) 537.7 534.3 518.4   365.8 370.0 357.8    380.0 360.6 354.0
 template <typename T, int MODE, bool WANT_MASK, int HD>
 __global__ __launch_bounds__(256) void quantize_values_kernel(const T* __restrict__ x, int64_t n_groups, Rotation rot, uint64_t seed,
-                                                              uint32_t* __restrict__ maskbits, T* __restrict__ values) {
+                                                              uint32_t* __restrict__ maskbits, T* __restrict__ values, bool past_in, bool past_out) {
     constexpr int kPieces = 2 * (int)sizeof(T);   // 16-byte pieces per group
     job_starts();
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -400,8 +407,13 @@ __global__ __launch_bounds__(256) void quantize_values_kernel(const T* __restric
     if (whole) {
         const uint4* src = reinterpret_cast<const uint4*>(x + first * 32);
         uint4 raw[kPieces];
+        if (past_in) {
 #pragma unroll
-        for (int i = 0; i < kPieces; ++i) raw[i] = stream_load(src + piece_of_slot(i));
+            for (int i = 0; i < kPieces; ++i) raw[i] = stream_load(src + piece_of_slot(i));
+        } else {
+#pragma unroll
+            for (int i = 0; i < kPieces; ++i) raw[i] = src[piece_of_slot(i)];
+        }
         job_requests_issued();
 #pragma unroll
         for (int i = 0; i < kPieces; ++i) area[64 * i + lane] = raw[i];
@@ -436,8 +448,13 @@ __global__ __launch_bounds__(256) void quantize_values_kernel(const T* __restric
         for (int q = 0; q < kPieces; ++q) area[kPieces * lane + (q ^ swizzle(lane))] = out[q];
         wave_settle();
         uint4* dst = reinterpret_cast<uint4*>(values + first * 32);
+        if (past_out) {
 #pragma unroll
-        for (int i = 0; i < kPieces; ++i) stream_store(dst + piece_of_slot(i), area[64 * i + lane]);
+            for (int i = 0; i < kPieces; ++i) stream_store(dst + piece_of_slot(i), area[64 * i + lane]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < kPieces; ++i) dst[piece_of_slot(i)] = area[64 * i + lane];
+        }
     } else {
 #pragma unroll
         for (int q = 0; q < kPieces; ++q) reinterpret_cast<uint4*>(values + gi * 32)[q] = out[q];
@@ -1531,12 +1548,14 @@ hipError_t quantize_values(const void* x, int dtype, int64_t rows, int64_t cols,
     const int64_t n_groups = rows * cols / 32;
     with_elem_type(dtype, [&](auto t) {
         using T = decltype(t);
+        const int64_t bytes = rows * cols * (int64_t)sizeof(T);
         with_mode(mode, [&](auto m) {
             with_flag(maskbits != nullptr, [&](auto k) {
                 with_hadamard(hd, [&](auto h) {
                     constexpr int HD = decltype(h)::value;
                     quantize_values_kernel<T, decltype(m)::value, decltype(k)::value, HD><<<dim3((unsigned)((n_groups + 255) / 256)), dim3(256), 256 * 32 * sizeof(T), stream>>>(
-                        reinterpret_cast<const T*>(x), n_groups, make_rotation<HD>(dtype, sb), seed, reinterpret_cast<uint32_t*>(maskbits), reinterpret_cast<T*>(values));
+                        reinterpret_cast<const T*>(x), n_groups, make_rotation<HD>(dtype, sb), seed, reinterpret_cast<uint32_t*>(maskbits), reinterpret_cast<T*>(values),
+                        bytes >= kPastTheCaches, bytes >= kMoreThanTheCaches);
                 });
             });
         });

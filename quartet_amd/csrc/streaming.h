@@ -1,14 +1,16 @@
-// Loads and stores of values that no launch soon after reads: they pass through the caches without displacing what others keep there.
-// Whether that pays is measured kernel by kernel (each says so beside its accesses).
+// Loads and stores past the caches: they displace nothing that others keep there, and what they store is not there for a reader.
+// Whether that pays, and from which size on, is measured kernel by kernel (each says so beside its accesses).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 namespace qm {
 
-// Most of what the memory-side cache holds (256 MB).  Kernels that gain only on tensors which do not stay there take these accesses
-// from here on.
+// A tensor of this size and a result as large are most of what the memory-side cache holds (256 MB).  Kernels that gain only on tensors
+// which do not stay there take these accesses from here on.
 constexpr int64_t kPastTheCaches = 96ll << 20;
+// A result from here on cannot be there as a whole when the next launch reads it.
+constexpr int64_t kMoreThanTheCaches = 256ll << 20;
 
 template <typename V>
 __device__ __forceinline__ V stream_load(const V* p) {

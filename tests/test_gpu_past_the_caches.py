@@ -43,6 +43,27 @@ def test_inverse_rotation(rows, cols, hd, dtype):
     assert torch.equal(run(g, mask), torch.cat([run(*p) for p in zip(parts(g), parts(mask))]))
 
 
+# past 96 MiB (loads) and past 256 MiB (stores, too), a last wave that is not whole
+@pytest.mark.parametrize("rows,cols,hd,dtype", [(12297, 4096, 32, BF16), (6145, 4160, 64, F32), (24577, 2048, 128, BF16), (32769, 4096, 64, BF16), (16385, 4224, 32, F32)])
+@pytest.mark.parametrize("mode", ["QUEST_RTN", "ABSMAX_RTN"])
+def test_quantizer_values(rows, cols, hd, dtype, mode):
+    print(f"case quantizer values {rows}x{cols} hd={hd} {dtype} {mode}", flush=True)
+    from quartet_amd import _lib, kernels as K
+    x = torch.randn(rows, cols, generator=torch.Generator(device="cuda").manual_seed(hd), device="cuda").to(dtype)
+    assert x.numel() * x.element_size() >= 96 << 20
+    quest = mode == "QUEST_RTN"
+
+    def run(x):
+        values, mask = torch.empty_like(x), torch.zeros(x.shape[0], cols // 8, dtype=torch.uint8, device="cuda")
+        rc = _lib.lib().qm_pseudo_quantize_mxfp4(x.data_ptr(), _lib.QM_BF16 if dtype == BF16 else _lib.QM_F32, *x.shape, hd, K.sign_words(0x0F1E2D3C), getattr(K, "QM_" + mode), 0,
+                                                 mask.data_ptr() if quest else None, values.data_ptr(), None)
+        _lib.check(rc, "qm_pseudo_quantize_mxfp4")
+        return values, mask
+    whole, halves = run(x), [run(p) for p in parts(x, 3)]
+    for got, want in zip(whole, zip(*halves)):
+        assert torch.equal(got, torch.cat(want))
+
+
 @pytest.mark.parametrize("rows,classes,dtype", [(1573, 32000, BF16), (787, 32003, F32), (1600, 31999, BF16)])
 def test_loss(rows, classes, dtype):
     """The mean of two halves' means: at most 16 + 10 + 2 fp32 additions of positive losses and a division, twice: 64 roundings."""
