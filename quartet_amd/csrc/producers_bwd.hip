@@ -488,11 +488,15 @@ int64_t rmsnorm_bwd_blocks(int64_t rows, int64_t cols) {
     return (rows + rows_per_block(rows) - 1) / rows_per_block(rows);
 }
 
-// The cooperative kernel's tensors (up to 16 bytes an element) past the caches: dirty lines of a large result are written back during the
-// next launch.  us of a layer's step with a bf16 summand, through the caches and past them: 4096 x 2048 111.6 -> 107.9, 16384 x 2048
-// 339 -> 325, 6144 x 4096 262 -> 256.5, 8192 x 4096 338 -> 328; but 1024 x 3072 69.2 -> 74.7, 2048 x 2048 70.2 -> 75.3: there the step
-// lives in the cache.  (Not in rmsnorm_bwd_rows_kernel: 16384 x 1536 80 us, 89 past them.)
-inline bool past_the_caches(int64_t rows, int64_t cols) { return rows * cols * 16 >= kPastTheCaches; }
+// The cooperative kernel's tensors past the caches, counted as they are: dirty lines of a large result are written back during the next
+// launch.  us of a layer's step with a bf16 summand of an fp32 x (16 bytes an element), through the caches and past them: 4096 x 2048 111.6
+// -> 107.9, 16384 x 2048 339 -> 325, 6144 x 4096 262 -> 256.5, 8192 x 4096 338 -> 328; but 1024 x 3072 69.2 -> 74.7, 2048 x 2048 70.2 -> 75.3: there
+// the step lives in the cache.  A bf16 x by itself (6 bytes): 2048 x 4096 (48 MiB) 255 -> 257, 3072
+// x 4096 (72) 333 -> 337, 4096 x 4096 (96) 400 -> 392, 8192 x 2048 (96) 357 -> 343.  (Not in rmsnorm_bwd_rows_kernel: 16384 x 1536 80 us, 89 past them.)
+template <typename TG, typename TX>
+bool past_the_caches(int64_t rows, int64_t cols, bool skip, bool bf16_copy) {
+    return rows * cols * (int64_t)(sizeof(TG) + (skip ? 3 : 2) * sizeof(TX) + (bf16_copy ? 2 : 0)) >= kPastTheCaches;
+}
 
 template <typename TG, typename TX>
 void launch_rmsnorm_bwd(const void* gy, const void* x, const float* gain, const float* factor, int64_t rows, int cols,
@@ -517,7 +521,7 @@ void launch_rmsnorm_bwd(const void* gy, const void* x, const float* gain, const 
             else if (cols <= 4096) go(std::integral_constant<int, 4>{}, std::integral_constant<int, 2>{}, stream_);
             else go(std::integral_constant<int, 8>{}, std::integral_constant<int, 1>{}, stream_);
         };
-        if (past_the_caches(rows, cols)) by_cols(std::true_type{});
+        if (past_the_caches<TG, TX>(rows, cols, skip != nullptr, dx_bf16 != nullptr)) by_cols(std::true_type{});
         else by_cols(std::false_type{});
     }
 }

@@ -32,6 +32,25 @@ def test_rmsnorm_backward(rows, cols, dtype):
     assert ((whole[1] - sum(h[1] for h in halves)).double().abs() <= 40 * 2.0 ** -24 * scale + 1e-30).all()
 
 
+# of a bf16 x, by itself (6 bytes an element) and with a skip gradient and a copy (10)
+@pytest.mark.parametrize("rows,cols,extra", [(8193, 2048, False), (4098, 4096, False), (4917, 2048, True), (1230, 8192, True)])
+def test_rmsnorm_backward_of_bf16(rows, cols, extra):
+    """Rows do not depend on each other: the same bits."""
+    print(f"case rmsnorm backward of bf16 {rows}x{cols} {extra}", flush=True)
+    from quartet_amd import kernels as K
+    per = 10 if extra else 6
+    assert rows * cols * per >= 96 << 20 > (rows + 1) // 2 * cols * per
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    x, gy, skip = (torch.randn(rows, cols, generator=gen, device="cuda").to(BF16) for _ in range(3))
+    gain = 1 + 0.1 * torch.randn(cols, generator=gen, device="cuda")
+    factor = (x.float().square().mean(-1) + 1e-5).rsqrt()
+    mask = torch.randint(0, 256, (rows, cols // 8), generator=gen, device="cuda", dtype=torch.uint8)
+    run = lambda x, gy, skip, factor, mask: K.rmsnorm_backward(gy, x, gain, factor, mask, 0x5A5A1234, BF16, skip=skip if extra else None, want_bf16_copy=extra)
+    whole, halves = run(x, gy, skip, factor, mask), [run(*p) for p in zip(*map(parts, (x, gy, skip, factor, mask)))]
+    for i in (0, 2) if extra else (0,):
+        assert torch.equal(whole[i], torch.cat([h[i] for h in halves]))
+
+
 @pytest.mark.parametrize("rows,cols,hd,dtype", [(12289, 4096, 32, BF16), (6145, 4096, 64, F32), (24577, 2048, 128, BF16)])
 def test_inverse_rotation(rows, cols, hd, dtype):
     print(f"case inverse rotation {rows}x{cols} hd={hd} {dtype}", flush=True)
