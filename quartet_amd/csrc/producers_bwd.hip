@@ -452,7 +452,9 @@ __device__ __forceinline__ void inverse_rotate_oct(float (&v)[8], const InverseR
 // hidden % 8 == 0: the same arithmetic per element as swiglu_bwd_kernel, half as many memory instructions per element
 // (used when the gradient arrives rotated: there the mask byte per quad of the other kernel is what it saves).  Past the caches both
 // ways: a step of 16384 x 4096 x 1536 417.9 -> 405 us (the next launch no longer waits for this one's lines to be written back),
-// by itself 2048 x 1728 10.7 -> 9.3, 4096 x 1728 16.4 -> 14.7, 16384 x 4096 115 either way.
+// by itself 2048 x 1728 10.7 -> 9.3, 4096 x 1728 16.4 -> 14.7, 16384 x 4096 115 either way.  No threshold: training steps of a whole MLP, in which
+// the backward quantizers of the layer in front read the result at once, are the same either way (2048 tokens x 1536 x 4096 264, 4096
+// 420, 8192 677, 16384 1188; 16384 x 640 x 1728 490), the reader being bound by its vector instructions.
 template <typename TG, typename TH>
 __global__ __launch_bounds__(256) void swiglu_bwd_oct_kernel(const TG* __restrict__ g, const TH* __restrict__ h12,
                                                              int64_t rows, int64_t hidden, InverseRotation rot,
