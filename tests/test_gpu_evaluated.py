@@ -119,6 +119,30 @@ def test_an_evaluated_model_is_the_same_model(add_dtype):
     assert torch.isfinite(xg.grad).all() and block.mlp.w12.weight.grad is not None
 
 
+def test_an_evaluated_attention_of_many_tokens_is_the_same():
+    """Enough tokens for the rotary split to ride along: the bits of the two launches."""
+    import quartet_amd as q
+    from quartet_amd import _lib
+    from quartet_amd.fused import rmsnorm_rope_linear
+    from quartet_amd.llama import Llama, llama_30m, rotary_table
+    torch.manual_seed(3)
+    with torch.device("cuda"):
+        block = Llama(llama_30m(n_layer=1, sequence_length=512)).eval().transformer.h[0]
+    x = make_input(1100, 640, torch.float32, seed=5).view(5, 220, 640).to("cuda:0")
+    add = make_input(1100, 640, BF16, seed=6).view(5, 220, 640).to("cuda:0")
+    table = rotary_table(128, 220).to("cuda:0")
+    assert _lib.lib().qm_linear_rope_serves(1100, 640, 640, 128) == 1
+
+    def run():
+        with torch.no_grad(), torch.autocast("cuda", dtype=BF16):
+            return rmsnorm_rope_linear(block.ln_1, block.attn.c_attn, x, table, 5, add=add)
+    want = run()
+    q.enable_packed_weight_cache(block)
+    run()                                   # quantizes the weight
+    for g, r in zip(run(), want):
+        assert g.dtype == r.dtype and g.shape == r.shape and torch.equal(g, r)
+
+
 @pytest.mark.parametrize("rows,cols", [(1, 4), (5, 640), (4, 768), (7, 772), (3, 1536), (9, 1540), (2, 4096)])
 @pytest.mark.parametrize("add_dtype", [None, BF16, torch.float32])
 @pytest.mark.parametrize("out_dtype", [BF16, torch.float32])
