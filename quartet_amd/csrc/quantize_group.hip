@@ -387,6 +387,7 @@ void launch_rowmajor_wide(int mode, const void* x, int64_t n, float c, const Sig
 //   24576 x 4096 (192 MiB) 220.9 212.0 220.9    140.4 126.3 136.5    149.6 135.2 130.4
 //   32768 x 4096 (256 MiB) 267.3 261.7 268.0   184.8 186.5 183.4    197.3 177.4 174.3
 //   32768 x 8192 (512 MiB) 537.7 534.3 518.4   365.8 370.0 357.8    380.0 360.6 354.0
+// WANT_MASK: maskbits or null; the quest modes always work it out, as the quantizer modules want it, the absmax modes where it is asked for
 template <typename T, int MODE, bool WANT_MASK, int HD>
 __global__ __launch_bounds__(256) void quantize_values_kernel(const T* __restrict__ x, int64_t n_groups, Rotation rot, uint64_t seed,
                                                               uint32_t* __restrict__ maskbits, T* __restrict__ values, bool past_in, bool past_out) {
@@ -441,7 +442,7 @@ __global__ __launch_bounds__(256) void quantize_values_kernel(const T* __restric
     uint4 out[kPieces];
     group_values<T>(o, out);
     job_stores_next();
-    if constexpr (WANT_MASK) maskbits[gi] = o.keep;
+    if (WANT_MASK && maskbits) maskbits[gi] = o.keep;
     if (whole) {
         wave_settle();
 #pragma unroll
@@ -1550,14 +1551,17 @@ hipError_t quantize_values(const void* x, int dtype, int64_t rows, int64_t cols,
         using T = decltype(t);
         const int64_t bytes = rows * cols * (int64_t)sizeof(T);
         with_mode(mode, [&](auto m) {
-            with_flag(maskbits != nullptr, [&](auto k) {
+            constexpr int MODE = decltype(m)::value;
+            const auto go = [&](auto k) {
                 with_hadamard(hd, [&](auto h) {
                     constexpr int HD = decltype(h)::value;
-                    quantize_values_kernel<T, decltype(m)::value, decltype(k)::value, HD><<<dim3((unsigned)((n_groups + 255) / 256)), dim3(256), 256 * 32 * sizeof(T), stream>>>(
+                    quantize_values_kernel<T, MODE, decltype(k)::value, HD><<<dim3((unsigned)((n_groups + 255) / 256)), dim3(256), 256 * 32 * sizeof(T), stream>>>(
                         reinterpret_cast<const T*>(x), n_groups, make_rotation<HD>(dtype, sb), seed, reinterpret_cast<uint32_t*>(maskbits), reinterpret_cast<T*>(values),
                         bytes >= kPastTheCaches, bytes >= kMoreThanTheCaches);
                 });
-            });
+            };
+            if constexpr (MODE == QUEST_RTN || MODE == QUEST_SR) go(std::true_type{});
+            else with_flag(maskbits != nullptr, go);
         });
     });
     return hipGetLastError();

@@ -41,6 +41,25 @@ def test_values_are_those_of_the_codes(oracle, rows, cols, hd, dtype, mode):
         assert np.array_equal(mask.cpu().numpy(), ref["mask"].reshape(-1))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("hd", [32, 128])
+@pytest.mark.parametrize("mode", ["QUEST_RTN", "ABSMAX_RTN", "ABSMAX_SR", "QUEST_SR"])
+def test_the_mask_may_be_left_out_or_asked_for(mode, hd, dtype):
+    """Either way the values and masks of the quantizer that writes codes, too."""
+    from quartet_amd import _lib, kernels as K
+    print(f"case values with and without mask hd={hd} {dtype} {mode}", flush=True)
+    rows, cols, code = 37, 1152, getattr(K, "QM_" + mode)
+    x = make_input(rows, cols, dtype, seed=hd, outlier_frac=0.01).to("cuda:0")
+    _, _, want_mask, want = K.quantize_mxfp4(x, hd, 0x5A5A1234, code, seed=77, want_mask=True, want_dequant=True)
+    for with_mask in (False, True):
+        values, mask = torch.full_like(x, float("nan")), torch.zeros(rows * cols // 8, dtype=torch.uint8, device="cuda:0")
+        rc = _lib.lib().qm_pseudo_quantize_mxfp4(x.data_ptr(), _lib.QM_BF16 if dtype == torch.bfloat16 else _lib.QM_F32, rows, cols, hd, K.sign_words(0x5A5A1234), code, 77,
+                                                 mask.data_ptr() if with_mask else None, values.data_ptr(), None)
+        _lib.check(rc, "qm_pseudo_quantize_mxfp4")
+        assert torch.equal(values, want.view(values.shape))
+        assert torch.equal(mask, want_mask.view(-1)) if with_mask else not mask.any()
+
+
 def test_values_of_nothing_and_of_misaligned_tensors():
     from quartet_amd import _lib, kernels as K
     L = _lib.lib()
