@@ -137,3 +137,79 @@ def test_error_only_gradients_in_one_launch(oracle, T, I, O):
     from tests.test_gpu_tiles import test_error_only_layer_with_both_widths_in_one_product as against_float64
     assert _lib.lib().qm_linear_backward_error_in_one_launch(T, I, O, 32, _lib.QM_BF16) == 1
     against_float64(oracle, T, I, O)
+
+
+# a weight gradient of fp32 weights (widened in the kernel) and of bf16 ones, as the first product of the grid (more tokens than out-features) and as
+# the second, every Hadamard block; tiles over the edges
+@pytest.mark.parametrize("T,I,O", [(4096, 3840, 3968), (3968, 3840, 4096)])
+@pytest.mark.parametrize("hd,wide", [(32, True), (64, False), (64, True), (128, False), (128, True)])
+def test_error_only_gradients_of_every_form_in_one_launch(oracle, T, I, O, hd, wide):
+    """Against float64 on the oracle's tensors, every row: a rounding of the product to bf16 (2^-9), whose fp32 sum may lie on the other side of
+    a tie, and one of the rotation."""
+    import random
+
+    import numpy as np
+
+    import quartet_amd as q
+    from quartet_amd import _lib
+    from tests.test_gpu_tiles import error_only_layer
+    from tests.util import to_oracle
+    print(f"case error-only pair {T}x{I}x{O} hd={hd} wide={wide}", flush=True)
+    assert _lib.lib().qm_linear_backward_error_in_one_launch(T, I, O, hd, _lib.QM_F32 if wide else _lib.QM_BF16) == 1
+    x = make_input(T, I, torch.bfloat16, seed=1, outlier_frac=0.01)
+    w = make_input(O, I, torch.bfloat16, seed=2, outlier_frac=0, scale=0.02)
+    e = make_input(T, O, torch.bfloat16, seed=3, outlier_frac=0, scale=1e-3)
+    layer = error_only_layer(q, I, O, hd, torch.float32 if wide else torch.bfloat16)
+    with torch.no_grad():
+        layer.weight.copy_(w.to("cuda:0"))
+    xd = x.to("cuda:0").requires_grad_(True)
+    random.seed(5)
+    with torch.autocast("cuda", torch.bfloat16, enabled=wide):
+        layer(xd).backward(e.to("cuda:0"))
+    assert xd.grad.dtype == torch.bfloat16 and layer.weight.grad.dtype == (torch.float32 if wide else torch.bfloat16)
+    random.seed(5)
+    o, d = oracle, float(oracle.FOUR_THIRDS)
+    qx = o.quantize(to_oracle(x), hd, mode=o.QUEST_RTN, want_mask=True)
+    qw = o.quantize(to_oracle(w.float() if wide else w), hd, mode=o.QUEST_RTN, want_mask=True)
+    qe = o.quantize(to_oracle(e), hd, mode=o.ABSMAX_SR, seed=random.getrandbits(63))
+    qet = o.quantize(to_oracle(e), hd, mode=o.ABSMAX_SR, transposed_in=True, seed=random.getrandbits(63))
+    on_gpu = lambda t, scale: torch.from_numpy(o.dequantize(t["codes"], t["scales"], scale)).to("cuda:0").double()
+    parity = torch.tensor([[bin(i & j).count("1") & 1 for j in range(hd)] for i in range(hd)], device="cuda:0")
+    H = torch.where(parity == 1, -1.0, 1.0).double() * float(torch.tensor(hd ** -0.5).to(torch.bfloat16))
+
+    def rotated(p, mask):
+        keep = torch.from_numpy(np.unpackbits(np.asarray(mask).reshape(p.shape[0], -1), axis=1, bitorder="little")).to("cuda:0")
+        return ((p.to(torch.bfloat16).double() * keep).view(-1, hd) @ H).view(p.shape)
+    for got, want in [(xd.grad, rotated(on_gpu(qe, d) @ on_gpu(qw, 1.0), qx["mask"])), (layer.weight.grad, rotated(on_gpu(qet, d) @ on_gpu(qx, 1.0), qw["mask"]))]:
+        err = (got.double() - want).norm(dim=1) / want.norm(dim=1)
+        assert float(err.max()) < 4e-3, float(err.max())
+
+
+# forward quantizers over different Hadamard blocks: the smaller tiles rotate either product by its own
+@pytest.mark.parametrize("T,I,O", [(512, 640, 1920), (1888, 1664, 3584), (2048, 2048, 1536)])
+@pytest.mark.parametrize("hd_x,hd_w,gx_rotated", [(32, 64, False), (32, 128, False), (64, 32, False), (128, 64, False), (32, 64, True)])
+@pytest.mark.parametrize("gw_dtype", [torch.bfloat16, torch.float32])
+def test_different_blocks_in_one_launch(monkeypatch, T, I, O, hd_x, hd_w, gx_rotated, gw_dtype):
+    """Bit for bit the products and the stand-alone rotations."""
+    print(f"case pair of blocks {T}x{I}x{O} hd={hd_x}, {hd_w} gx_rotated={gx_rotated} gw={gw_dtype}", flush=True)
+    from quartet_amd import _lib, kernels as K
+    assert _lib.lib().qm_linear_backward_in_one_launch(T, I, O, hd_x, hd_w, int(gw_dtype == torch.float32), int(gx_rotated)) == 2
+    monkeypatch.setattr(K, "_layout", lambda tiled: QM_LAYOUT_PADDED if tiled == "padded" else K.QM_LAYOUT_TILED if tiled else K.QM_LAYOUT_ROWMAJOR)
+    dev, bf16 = "cuda:0", torch.bfloat16
+    x = make_input(T, I, bf16, seed=21).to(dev)
+    w = make_input(O, I, bf16, seed=22, scale=0.02).to(dev)
+    e = make_input(T, O, bf16, seed=23, scale=1e-2, outlier_frac=0).to(dev)
+    sx, sw, sg, seeds = 0x5A5A5A5A, 0x0F0F1234, 0x13572468, [11, 12, 13, 14]
+    _, px, pw = K.linear_forward(x, w, hd_x, sx, hd_w, sw, bf16, "padded")
+    gx, gw = K.linear_backward(e, px, pw, T, I, O, hd_x, sx, hd_w, sw, 32, sg, K.QM_ABSMAX_SR, seeds, bf16, bf16, bf16, bf16, bf16,
+                               "padded", gx_rotated=gx_rotated, gw_dtype=gw_dtype)
+    xc, xs, xm, _ = K.quantize_mxfp4(x, hd_x, sx, K.QM_QUEST_RTN, want_mask=True)
+    wc, ws, wm, _ = K.quantize_mxfp4(w, hd_w, sw, K.QM_QUEST_RTN, want_mask=True)
+    ec, es, _, _ = K.quantize_mxfp4(e, 32, sg, K.QM_ABSMAX_SR, seed=seeds[0])
+    wtc, wts, _ = K.requantize_transposed_mxfp4(wc, ws, 1.0, bf16, 32, sg, K.QM_ABSMAX_SR, seed=seeds[1])
+    etc, ets, _, _ = K.quantize_mxfp4(e, 32, sg, K.QM_ABSMAX_SR, transposed_in=True, seed=seeds[2])
+    xtc, xts, _ = K.requantize_transposed_mxfp4(xc, xs, 1.0, bf16, 32, sg, K.QM_ABSMAX_SR, seed=seeds[3])
+    gxq = K.gemm_mxfp4_tn(ec, es, wtc, wts, ALPHA, bf16, split_k=False)
+    gwq = K.gemm_mxfp4_tn(etc, ets, xtc, xts, ALPHA, bf16, split_k=False)
+    assert torch.equal(gx, gxq if gx_rotated else K.masked_hadamard_bwd(gxq, hd_x, bf16, sx, xm))
+    assert torch.equal(gw.float(), K.masked_hadamard_bwd(gwq, hd_w, bf16, sw, wm).float())
