@@ -9,6 +9,7 @@
 #include "../../include/quartet_hip.h"
 #include "qm_kernels.h"
 #include "qm_math.h"
+#include "shape_table.h"
 
 namespace {
 
@@ -467,7 +468,7 @@ GradProduct plan_gradient(const qm::TileProduct& plain, void* final_dst, bool wa
 // common, the extents, the Hadamard blocks and the kind of column signs, with the figures of the form that rotates both into bf16; the
 // weight gradient's type counts where neither product would be cut, whose sums are then the same either way.  With gx left rotated the estimate is
 // up to 0.07 nearer to two launches', and 40 such steps that share a launch are 0.96 to 1.09 times as fast for it, all but two 0.99 and more.
-qm::PairChoice gradient_pair(int64_t T, int64_t I, int64_t O, int hd_x, int hd_w, const uint32_t* signs_x, const uint32_t* signs_w, int gw_dtype) {
+qm::PairChoice choose_gradient_pair(int64_t T, int64_t I, int64_t O, int hd_x, int hd_w, const uint32_t* signs_x, const uint32_t* signs_w, int gw_dtype) {
     uint8_t* at = reinterpret_cast<uint8_t*>((uintptr_t)256);   // nothing is read: stand-ins with the alignment that a layer's tensors have
     const size_t ws_bytes = work_layout(T, I, O, QM_BF16).gemm_ws_bytes;
     const auto product = [&](int64_t M, int64_t K, int hd, const uint32_t* signs) {
@@ -478,6 +479,23 @@ qm::PairChoice gradient_pair(int64_t T, int64_t I, int64_t O, int hd_x, int hd_w
     const qm::ProductChoice cx = choose(x, QM_BF16), cw = choose(w, QM_BF16);
     if (gw_dtype != QM_BF16 && cx.splits == 1 && cw.splits == 1) return qm::choose_pair(x, cx, QM_BF16, w, choose(w, gw_dtype), gw_dtype);
     return qm::choose_pair(x, cx, QM_BF16, w, cw, QM_BF16);
+}
+// Remembered per thread (a small layer's training step is bound by its host): up to 64 layers, 4 KB.  Of the signs only whether they repeat
+// every 32 counts.
+struct PairPlan {
+    int64_t M = -1, N = 0, K = 0;
+    int flags = -1;
+    qm::PairChoice choice{qm::PairChoice::SEPARATE, 0, 0};
+};
+qm::PairChoice gradient_pair(int64_t T, int64_t I, int64_t O, int hd_x, int hd_w, const uint32_t* signs_x, const uint32_t* signs_w, int gw_dtype) {
+    static thread_local qm::ShapeTable<PairPlan, 4> table;
+    const auto form = [](int hd, const uint32_t* signs) {
+        bool repeat = true;
+        for (int j = 1; signs && j < hd / 32; ++j) repeat = repeat && signs[j] == signs[0];
+        return hd / 32 * 2 + (repeat ? 1 : 0);
+    };
+    const int flags = (form(hd_x, signs_x) * 16 + form(hd_w, signs_w)) * 2 + (gw_dtype == QM_BF16 ? 0 : 1);
+    return table.find(T, I, O, flags, [&] { return PairPlan{T, I, O, flags, choose_gradient_pair(T, I, O, hd_x, hd_w, signs_x, signs_w, gw_dtype)}; }).choice;
 }
 }
 }  // namespace
