@@ -424,7 +424,7 @@ __device__ __forceinline__ void big4_step(const Big4Plan& plan, uint8_t* smem_by
 struct RotEpilogue {
     const uint8_t* mask;  // [M][N / 8] clip-mask bits, bit n % 8 of byte n / 8
     uint32_t signs;       // bit n: column n of every 32 of the Hadamard block negated
-    float c;              // 32^-1/2, rounded to the scale dtype
+    float c;              // block^-1/2, rounded to the scale dtype
 };
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -613,7 +613,7 @@ __device__ __forceinline__ unsigned long long shader_clock() {
 // of one fill the gaps of the other.  Every XCD has a contiguous run of either product's tiles, its W = grid / 8 workgroups take the
 // long ones in turn, then `rounds` short ones each, and those that had one long tile fewer take the short ones that are left:
 // the host picks `rounds` so that all end together.  What bounds it is what bounds the kernel with one product (the power limit: 3.4 to
-// 4.1 PFLOP/s); figures at pair_pays().
+// 4.1 PFLOP/s); figures at pair_margin().
 struct Big4Other {   // the short product; the long one is the kernel's first arguments
     const uint8_t* a_codes;
     const uint8_t* a_scales;

@@ -251,7 +251,7 @@ void launch_rowmajor_dense(int mode, const void* x, int64_t rows, int64_t cols, 
 // alone the compiler took 128 to 160 registers (three waves, four for whole tiles of blocks of 32) where 96 do for blocks of 32 and 107
 // and 127 for blocks of 64 and 128; six waves would spill.  The other waves' arithmetic hides one's requests.  us of the grid, before
 // and now: 1824 x 1408 x 2048 18.8 -> 14.5, 20000 x 704 x 704 33.8 -> 30.2, blocks of 64 8192 x 4096 x 4096 83.7 -> 76.3; per step
-// 8192 x 4096 x 4096 285 -> 280, 8192 x 4096 x 11008 693 -> 685, blocks of 128 8192 x 1536 x 4608 194 -> 191.
+// 8192 x 4096 x 4096 279.4 -> 276.1, 8192 x 4096 x 11008 686.6 -> 682.7, blocks of 128 8192 x 1536 x 4608 185.5 -> 183.1.
 constexpr int backward_waves(int hd) { return hd == 32 ? 5 : 4; }
 
 // Tiled code layout ([rows/16][cols/128][16 rows][64 bytes]).  Workgroup b owns block b / chunks of 16 rows and run
