@@ -634,9 +634,9 @@ int qm_linear_swiglu_quantize(const void* packed_x, size_t packed_x_bytes, const
 }
 
 // The same with the rotary split: 0.3 us a tile and CU; the launch of its own 1 us, where it follows its product at once, and 12 bytes an
-// element at 5.0 TB/s.  On 72 sizes of 65 to 32768 tokens and widths 640 to 4096 the two are on the side that the estimate says, but for two
-// that differ by 0.1 us.  us in one launch and in two: 65 x 1536 13.8 / 12.3, 128 x 4096 25.8 / 23.6, 200 x 1280 13.9 / 13.1; 300 x 2048 15.8 / 16.6, 512 x 1536
-// 15.1 / 17.4, 4096 x 640 19.7 / 26.6, 32768 x 1536 310 / 340.
+// element at 5.0 TB/s.  Of 85 sizes of 65 to 32768 tokens and widths 640 to 4096 one is on the other side than the estimate says (256 x 1536, by 0.1
+// us).  us in one launch and in two: 65 x 1536 13.8 / 12.3, 128 x 4096 25.8 / 23.6, 200 x 1280 13.9 / 13.1; 300 x 2048 15.8 / 16.6, 512 x 1536 15.1 / 17.4,
+// 4096 x 640 19.7 / 26.6, 32768 x 1536 310 / 340.
 int qm_linear_rope_serves(int64_t T, int64_t I, int64_t n_embd, int head_dim) {
     qm::TileProduct p;
     if (n_embd <= 0 || n_embd > (1 << 24) || head_dim <= 0 || head_dim % 8 || n_embd % head_dim ||
