@@ -20,6 +20,7 @@
 //                              Persistent, 256x256 macro tile, 4 waves x 128x128, operands global -> LDS directly into a
 //                              4-stage ring, scales in blocks of four K steps, row-major or tiled code bytes, optional split-K.
 //   gemm_tile.hip              tiles from 256x128 down to 64x32 for everything too small or too short for that one.
+//   gemm_two.hip               256x192 tiles, two workgroups to a CU: plain bf16 results whose tiles fill the last round better so.
 //   gemm_mxfp4_tn_kernel       any M, N and K % 32 == 0: 128x128 macro tile, 4 waves x 64x64, operands staged
 //                              global -> registers -> LDS (rows padded from 64 to 80 bytes so the 16-byte fragment
 //                              reads of 16 consecutive rows hit 64 distinct banks), double buffered.
@@ -1013,6 +1014,22 @@ double tile_cost(const KernelCost& k, int64_t M, int64_t N, int64_t K, int split
     const int64_t full = tiles / (k.per_cu * cus), rest = tiles % (k.per_cu * cus);
     return kLaunch + full * round(k.per_cu) + (rest ? round((rest + cus - 1) / cus) : 0.0) + ranges_cost(M, N, splits);
 }
+// 256 x 192 tiles, two to a CU (gemm_two.hip).  Fewer than one a CU leave it to a workgroup that nothing covers; with one on some CUs and two on
+// others the chip runs them faster than with two everywhere.  Fitted to 106 shapes of 0.6 to 370 GF with tiled operands, each launch behind a copy of
+// 32 MiB: rms error 7 %.  Taken where it is below kTwoMargin of the cheapest other kernel, which costs 0.25 % more than the fastest
+// on average and is slower than it by 2 % and more in two of the shapes.  us, the other kernel and this one: 16384 x 1536 x 4096 57.2 and 52.5, 13328 x
+// 1280 x 2176 28.8 and 26.7, 16832 x 9280 x 2176 204.5 and 179.8, 26256 x 4672 x 768 84.6 and 74.1; where the line lies 17152 x 5184 x 1792 92.5 and 95.3,
+// 9120 x 9600 x 1920 99.0 and 99.3; left to the others 8192 x 4096^2 65.4 and 75.4, 4096^3 34.8 and 43.4.
+constexpr double kTwoMargin = 0.95;
+double two_cost(int64_t M, int64_t N, int64_t K, int cus) {
+    const int64_t tiles = ((M + 255) / 256) * ((N + 191) / 192), steps = K / kBK, full = tiles / (2 * cus), rest = tiles % (2 * cus);
+    if (tiles <= cus) return 1e30;
+    const double both = 1.3, one = 0.78, some = 1.1, boundary = 5.5;
+    double cost = kLaunch + 1.0 + full * (steps * both + boundary);
+    if (rest > cus) cost += steps * (some + (both - some) * (double)(rest - cus) / cus) + boundary;
+    else if (rest) cost += steps * one + 3.15;
+    return cost;
+}
 // the masked inverse rotation in the epilogue of a tile kernel, and as a kernel of its own
 double tile_rotate_cost(const KernelCost& k, int64_t M, int64_t N, int hd, int out_bytes, int cus) {
     const int64_t tiles = ((M + k.bm - 1) / k.bm) * ((N + k.bn - 1) / k.bn);
@@ -1182,7 +1199,7 @@ bool gemm_supports_tiled(int64_t M, int64_t N, int64_t K) {
 struct ShapePlan {
     int64_t M = -1, N = 0, K = 0;
     int flags = -1;
-    double persistent = 1e30, tile[5] = {};
+    double persistent = 1e30, two = 1e30, tile[5] = {};
     Cut cut{};
     size_t cut_bytes = 0;       // scratch of the cut, 0 if it would not be made
     size_t scratch_bytes = 0;   // what a caller is asked to provide: at least cut_bytes
@@ -1210,6 +1227,7 @@ ShapePlan make_plan(int64_t M, int64_t N, int64_t K, bool persistent, bool tiles
     p.M = M; p.N = N; p.K = K; p.flags = flags;
     double best = 1e30;
     if (persistent) best = p.persistent = persistent_cost(M, N, K, 1, cus);
+    p.two = two_cost(M, N, K, cus);
     for (int kind = TILE_256x128; kind <= last_tile_kind(e5m2); ++kind) {
         p.tile[kind] = tiles_ok ? tile_cost(tile_costs(e5m2, kind, K, 1), M, N, K, 1, cus) : 1e30;
         best = p.tile[kind] < best ? p.tile[kind] : best;
@@ -1275,6 +1293,7 @@ ProductChoice choose_product(const TileProduct& p, int c_dtype, int rot_out_dtyp
         if (rotate && bf16 && k.bn >= p.hd) consider({ProductChoice::TILE, kind, 1, true}, plan.tile[kind] + tile_rotate_cost(k, M, N, p.hd, rot_out_dtype == BF16 ? 2 : 4, cus));
         consider({ProductChoice::TILE, kind, 1, false}, plan.tile[kind] + separate);
     }
+    if (!rotate && bf16 && plan.two < kTwoMargin * best_cost && gemm_two_serves(p)) consider({ProductChoice::TWO, 0, 1, false}, plan.two);
     return best;
 }
 
@@ -1311,6 +1330,7 @@ hipError_t run_product(const ProductChoice& c, const TileProduct& p, int c_dtype
             splitk_reduce_kernel<float><<<grid, block, 0, stream>>>(part, c.splits, mn, p.alpha, static_cast<float*>(p.c));
         return hipGetLastError();
     }
+    if (c.path == ProductChoice::TWO) return c_dtype == BF16 ? gemm_two(p, stream) : hipErrorInvalidValue;
     if (c.path == ProductChoice::TILE) {
         TileProduct q = p;
         q.splits = 1;

@@ -242,6 +242,10 @@ hipError_t gemm_tile_pair(TileProduct a, int kind_a, bool a_f32, TileProduct b, 
 bool gemm_wide_pair_serves(const TileProduct& a, const TileProduct& b);
 hipError_t gemm_wide_pair(TileProduct a, bool a_f32, TileProduct b, bool b_f32, hipStream_t stream);
 
+// Plain bf16 results of tiled operands on 256 x 192 tiles, two workgroups to a CU (gemm_two.hip): K % 128 == 0, K >= 512, N % 8 == 0, c 16-byte aligned
+bool gemm_two_serves(const TileProduct& p);
+hipError_t gemm_two(const TileProduct& p, hipStream_t stream);
+
 // The product of at most 64 rows with a weight, both tiled (gemm_rows.hip): K % 128 == 0, N % 8 == 0, c 16-byte aligned, no mask.
 // Its sums are in another order than the other kernels'.
 bool gemm_rows_serves(const TileProduct& p);
@@ -257,7 +261,7 @@ hipError_t linear_decode(const void* x, int x_dtype, int64_t T, int64_t I, int64
 // whether that kernel applies it (p.c then holds rot_out_dtype elements: c_dtype, or F32 holding the bf16-rounded result)
 // or the caller has to (p.c then holds the plain product in c_dtype).
 struct ProductChoice {
-    enum Path : int { GENERIC = 0, PERSISTENT = 1, TILE = 2 } path;
+    enum Path : int { GENERIC = 0, PERSISTENT = 1, TILE = 2, TWO = 3 } path;
     int kind;      // TileKind
     int splits;    // K ranges (their fp32 partial sums in the workspace, then one ordered reduction)
     bool rotates;
