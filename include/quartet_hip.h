@@ -440,6 +440,17 @@ int qm_linear_rope(const void* packed_x, size_t packed_x_bytes, const void* pack
 int qm_rmsnorm(const float* x, const void* add, int add_dtype, const float* gain, float eps, int64_t rows, int64_t cols, void* out,
                int out_dtype, void* stream);
 
+/*
+ * The end of an evaluated model (src/models/llama.py:249-256 of the reference under bf16 autocast): h = RMSNorm of (x + add) as qm_rmsnorm, rounded to
+ * bf16; logits [T, V] bf16 = h w^T with the fp32 weight w [V, K] rounded to bf16, fp32 sums; *loss as qm_cross_entropy of those logits, whose
+ * sums of exponentials the product works out beside them.
+ *   workspace   DEVICE scratch of qm_logits_loss_workspace_bytes(T, K, V) bytes (0: not served), 256-byte aligned
+ * K a multiple of 32 in [64, 4096], V a multiple of 8; 16-byte aligned tensors.
+ */
+size_t qm_logits_loss_workspace_bytes(int64_t T, int64_t K, int64_t V);
+int qm_logits_loss(const float* x, const void* add, int add_dtype, const float* gain, float eps, int64_t T, int64_t K, const float* w, int64_t V,
+                   const int64_t* targets, int64_t ignore_index, void* workspace, size_t workspace_bytes, void* logits, float* loss, void* stream);
+
 /* Test aid: silu as the SwiGLU producer evaluates it for bf16 tensors, of every bf16 bit pattern: out[65536] */
 int qm_diag_silu_bf16(uint16_t* out, void* stream);
 

@@ -60,6 +60,8 @@ EXPORTS = (
     "qm_linear_backward_error_in_one_launch",
     "qm_linear_decode",
     "qm_cross_entropy",
+    "qm_logits_loss_workspace_bytes",
+    "qm_logits_loss",
     "qm_diag_silu_bf16",
 )
 
@@ -163,6 +165,10 @@ def lib():
     L.qm_swiglu_quantize_with_weight_mxfp4.argtypes = [vp, i32, i64, i64, vp, vp, ctypes.c_size_t, vp, i64, vp, vp, ctypes.c_size_t, vp]
     L.qm_linear_decode.restype = i32
     L.qm_linear_decode.argtypes = [vp, i32, i64, i64, i64, vp, vp, ctypes.c_size_t, vp, i32, vp]
+    L.qm_logits_loss_workspace_bytes.restype = sz
+    L.qm_logits_loss_workspace_bytes.argtypes = [i64, i64, i64]
+    L.qm_logits_loss.restype = i32
+    L.qm_logits_loss.argtypes = [vp, vp, i32, vp, f32, i64, i64, vp, i64, vp, i64, vp, sz, vp, vp, vp]
     L.qm_cross_entropy.restype = i32
     L.qm_cross_entropy.argtypes = [vp, i32, vp, i64, i64, i64, vp, vp, vp]
     L.qm_rope_merge_qkv_grad.restype = i32

@@ -1128,6 +1128,46 @@ int qm_rmsnorm(const float* x, const void* add, int add_dtype, const float* gain
     return from_hip(qm::rmsnorm_rows(x, add, add_dtype, gain, eps, rows, cols, out, out_dtype, reinterpret_cast<hipStream_t>(stream)), "qm_rmsnorm");
 }
 
+namespace {
+struct LogitsLayout {   // a workspace of qm_logits_loss
+    size_t x, w, parts, losses, total;
+};
+LogitsLayout logits_layout(int64_t T, int64_t K, int64_t V) {
+    LogitsLayout l;
+    l.x = 0;
+    l.w = l.x + up256((size_t)qm::padded_rows(T) * K * 2);
+    l.parts = l.w + up256((size_t)qm::padded_rows(V) * K * 2);
+    l.losses = l.parts + up256((size_t)qm::gemm_logits_segments(V) * T * 8);
+    l.total = l.losses + up256((size_t)T * 4);
+    return l;
+}
+}  // namespace
+
+size_t qm_logits_loss_workspace_bytes(int64_t T, int64_t K, int64_t V) { return qm::gemm_logits_serves(T, V, K) && K <= 4096 ? logits_layout(T, K, V).total : 0; }
+
+int qm_logits_loss(const float* x, const void* add, int add_dtype, const float* gain, float eps, int64_t T, int64_t K, const float* w, int64_t V,
+                   const int64_t* targets, int64_t ignore_index, void* workspace, size_t workspace_bytes, void* logits, float* loss, void* stream) {
+    if (add && !valid_dtype(add_dtype)) return fail(QM_ERR_INVALID, "qm_logits_loss: add_dtype must be QM_BF16/QM_F32");
+    const size_t need = qm_logits_loss_workspace_bytes(T, K, V);
+    if (!need)
+        return fail(QM_ERR_INVALID, "qm_logits_loss: need rows, in_features a multiple of 32 in [64, 4096] and classes a multiple of 8 (got [%lld, %lld] x %lld)", (long long)T,
+                    (long long)K, (long long)V);
+    if (!x || !gain || !w || !targets || !logits || !loss || !workspace || workspace_bytes < need)
+        return fail(QM_ERR_INVALID, "qm_logits_loss: null tensor, or workspace below %zu bytes", need);
+    if (!aligned(x, 16) || !aligned(add, 16) || !aligned(gain, 16) || !aligned(w, 16) || !aligned(logits, 16) || !aligned(workspace, 256) || !aligned(targets, 8) || !aligned(loss, 4))
+        return fail(QM_ERR_UNALIGNED, "qm_logits_loss: tensors need 16-byte, the workspace 256-byte alignment");
+    const LogitsLayout l = logits_layout(T, K, V);
+    uint8_t* ws = static_cast<uint8_t*>(workspace);
+    hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
+    float* losses = reinterpret_cast<float*>(ws + l.losses);
+    hipError_t e = qm::bf16_blocks(w, V, K, ws + l.w, hs);
+    if (e == hipSuccess) e = qm::rmsnorm_rows(x, add, add_dtype, gain, eps, T, K, ws + l.x, QM_BF16, hs, true);
+    if (e == hipSuccess) e = qm::gemm_logits(ws + l.x, ws + l.w, T, V, K, logits, ws + l.parts, hs);
+    if (e == hipSuccess) e = qm::logits_loss_rows(ws + l.parts, qm::gemm_logits_segments(V), T, logits, V, targets, ignore_index, losses, hs);
+    if (e == hipSuccess) e = qm::loss_mean(losses, targets, T, ignore_index, loss, hs);
+    return from_hip(e, "qm_logits_loss");
+}
+
 int qm_diag_silu_bf16(uint16_t* out, void* stream) {
     if (!out) return fail(QM_ERR_INVALID, "qm_diag_silu_bf16: out must be non-null");
     return from_hip(qm::silu_of_bf16_table(out, reinterpret_cast<hipStream_t>(stream)), "qm_diag_silu_bf16");

@@ -1,4 +1,4 @@
-// FP4 x FP4 "TN" product on tiles of 256 x 192, two workgroups to a CU: a plain bf16 result of two tiled operands.
+// FP4 x FP4 and bf16 x bf16 "TN" products on tiles of 256 x 192, two workgroups to a CU: a plain bf16 result of two tiled operands.
 //
 // The persistent kernel of gemm.hip owns a CU with one workgroup and a tile of 256 x 256, and the smaller shapes of gemm_tile.hip read 1.5 times
 // its bytes from LDS per product.  In between, a wave of 128 x 96 holds 192 accumulators, which leaves 64 of the 256 registers that two waves
@@ -12,6 +12,12 @@
 // 75.7; the steps 409.6 -> 409.4, 189.5 -> 185.8 and 438.5 -> 429.8, since part of what a product gains the power limit takes elsewhere.
 // Tried: fragments read a half step ahead across the barrier (scratch memory; 5 % slower), requests ahead of the products instead of among
 // them (4 % slower).
+//
+// The same with bf16 operands makes the logits of an evaluated model, whose workgroups also take the exponentials for their loss while the other one
+// of the CU multiplies: no pass of its own over logits that are larger than the caches.  Bound by the matrix instructions at the power limit and the last,
+// partial round of tiles: 4096 x 32000 x 640 166 us (153 without the exponentials; the library's product 158 and the loss's pass 49), and from 1536
+// on by its two slots (4096 x 32000 x 1536 339; the library's product 300).  An evaluated 30 M model of 8 x 512 tokens 884 -> 847 us.
+// Row-major operands, 64 bytes of a row at a time, took 176 and 380.
 //
 // The order of additions over K is that of gemm.hip and gemm_tile.hip: the same bits.
 #include <hip/hip_runtime.h>
@@ -37,19 +43,24 @@ template <int I>
 __device__ __forceinline__ void two_request(const uint8_t* base, uint32_t lane_off) {
     asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" ::"v"(lane_off), "s"(base), "i"(I * 1024) : "memory");
 }
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+constexpr float kLog2e = 1.44269504088896340736f;
 __device__ __forceinline__ v8i two_operand(const uint4& q) { return v8i{(int)q.x, (int)q.y, (int)q.z, (int)q.w, 0, 0, 0, 0}; }
 
 // EDGES: M or N is no multiple of the tile's.  Rows past the end repeat others, and nothing of theirs is stored.
-template <bool EDGES>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_mxfp4_tn_two_kernel(
-    const uint8_t* __restrict__ a_codes, const uint8_t* __restrict__ a_scales, const uint8_t* __restrict__ b_codes, const uint8_t* __restrict__ b_scales,
-    int M, int N, int K, float alpha, uint16_t* __restrict__ c, int late) {
+// BF16: both operands are bf16 in blocks of 16 rows and 32 elements, [R / 16][K / 32][16][64 bytes]: 32 elements in the place of 128 FP4 codes, no scales,
+// no alpha.  Beside the result it leaves, for every row and 96 columns of it, the largest stored value and the sum of the exponentials
+// relative to that one, in parts [2 ceil(N / 192)][M]: the logits and what their loss needs.
+template <bool BF16, bool EDGES>
+__device__ __forceinline__ void two_run(const uint8_t* __restrict__ a_codes, const uint8_t* __restrict__ a_scales, const uint8_t* __restrict__ b_codes,
+                                        const uint8_t* __restrict__ b_scales, int M, int N, int K, float alpha, uint16_t* __restrict__ c, int late,
+                                        [[maybe_unused]] float2* __restrict__ parts) {
     extern __shared__ uint32_t smem[];
     uint8_t* lds = reinterpret_cast<uint8_t*>(smem);
     const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint32_t*)smem;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int wm = wave >> 1, wn = wave & 1;
-    const int nk = K / kBK, groups = K / 32;
+    const int nk = BF16 ? K / 32 : K / kBK, groups = K / 32;
     const int tiles_m = (M + kTwoM - 1) / kTwoM, tiles_n = (N + kTwoN - 1) / kTwoN, tiles = tiles_m * tiles_n;
     const int64_t block_row = (int64_t)nk * 1024;   // 16 rows of codes
     const int b_unit = wave < 3 ? wave : 2;         // of B's scale rows, 64 at a time: the fourth wave repeats the third's request
@@ -61,6 +72,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
     // The tile that requests go to, its panels and this lane's place in them
     int m0, n0;
+    [[maybe_unused]] int tile_n;
     const uint8_t *pa[4], *pb[3], *psa, *psb;
     uint32_t in_block, lane_sa, lane_sb;
     // scales of the four K steps from ks on; a short last block takes the row's final 16 bytes
@@ -77,6 +89,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         tile_of_run<4>(xcd_run(t, tiles), tiles_m, tiles_n, tm, tn);
         m0 = tm * kTwoM;
         n0 = tn * kTwoN;
+        tile_n = tn;
         // in a 1 KiB block of 16 rows: the 16 bytes that belong at lane * 16 of its LDS image
         in_block = (lane >> 2) * 64 + ((lane & 3) ^ ((lane >> 4) & 3)) * 16;
         const auto block_at = [&](const uint8_t* codes, int b, int rows) {   // 16-row block b, the last one past the end
@@ -87,20 +100,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int j = 0; j < 4; ++j) pa[j] = block_at(a_codes, m0 / 16 + wave * 4 + j, M) - 1024 * j;
 #pragma unroll
         for (int j = 0; j < 3; ++j) pb[j] = block_at(b_codes, n0 / 16 + wave * 3 + j, N) - 1024 * j;
-        psa = a_scales + (int64_t)m0 * groups;
-        psb = b_scales + (int64_t)n0 * groups;
-        int ra = wave * 64 + lane, rb = b_unit * 64 + lane;
-        if (EDGES) {
-            ra = ra < M - 1 - m0 ? ra : M - 1 - m0;
-            rb = rb < N - 1 - n0 ? rb : N - 1 - n0;
-        } else {
-            psa += (int64_t)wave * 64 * groups;
-            psb += (int64_t)b_unit * 64 * groups;
-            ra = rb = lane;
+        if constexpr (!BF16) {
+            psa = a_scales + (int64_t)m0 * groups;
+            psb = b_scales + (int64_t)n0 * groups;
+            int ra = wave * 64 + lane, rb = b_unit * 64 + lane;
+            if (EDGES) {
+                ra = ra < M - 1 - m0 ? ra : M - 1 - m0;
+                rb = rb < N - 1 - n0 ? rb : N - 1 - n0;
+            } else {
+                psa += (int64_t)wave * 64 * groups;
+                psb += (int64_t)b_unit * 64 * groups;
+                ra = rb = lane;
+            }
+            lane_sa = (uint32_t)(ra * groups);
+            lane_sb = (uint32_t)(rb * groups);
+            request_scales(0);
         }
-        lane_sa = (uint32_t)(ra * groups);
-        lane_sb = (uint32_t)(rb * groups);
-        request_scales(0);
         two_lds_base(lds_base + wave * 4096);
         two_request<0>(pa[0], in_block);
         two_request<1>(pa[1], in_block);
@@ -121,7 +136,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         // this lane's 16 bytes of its wave's first A rows, in either half of a K step.  A wave's columns are 64 wn .. + 63 and 128 + 32 wn ..
         // + 31 of the tile, so that two of its blocks make whole lines of the result.
         const int swz = (lrow >> 2) & 3;
-        const uint32_t a_off0 = (wm * 128 + lrow) * kRowBytes + ((2 * half) ^ swz) * 16, a_off1 = (wm * 128 + lrow) * kRowBytes + ((2 * half + 1) ^ swz) * 16;
+        // (a lane's eight bf16 of an instruction are piece half of the row's four, then piece 2 + half)
+        const uint32_t a_off0 = (wm * 128 + lrow) * kRowBytes + ((BF16 ? half : 2 * half) ^ swz) * 16;
+        const uint32_t a_off1 = (wm * 128 + lrow) * kRowBytes + ((BF16 ? 2 + half : 2 * half + 1) ^ swz) * 16;
         const int to_b = kTwoBOff + (wn * 64 - wm * 128) * kRowBytes, to_b2 = kTwoBOff + (128 + wn * 32 - wm * 128) * kRowBytes;   // uniform
         const uint32_t sc_off = (wm * 128 + lrow) * 16 + half * 2;   // the two scale bytes of this lane's half
         v16f acc[kTwoTM][kTwoTN];
@@ -140,14 +157,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             const int next = ks + 1 < nk ? ks + 1 : nk - 1;   // past the end: a repeat that nobody reads
             const uint8_t* cur = lds + slot * kTwoSlot;
             const uint32_t to = lds_base + (slot ^ 1) * kTwoSlot;
-            const uint8_t* sc = lds + kTwoScales + ((ks >> 2) & 1) * kTwoScaleBuf + (ks - scales_at(ks & ~3)) * 4 + sc_off;
-            const uint8_t* sc_b = sc + kTwoM * 16 - wm * 2048;
             uint32_t sca[kTwoTM], scb[kTwoTN];
+            if constexpr (!BF16) {
+                const uint8_t* sc = lds + kTwoScales + ((ks >> 2) & 1) * kTwoScaleBuf + (ks - scales_at(ks & ~3)) * 4 + sc_off;
+                const uint8_t* sc_b = sc + kTwoM * 16 - wm * 2048;
 #pragma unroll
-            for (int i = 0; i < kTwoTM; ++i) sca[i] = *reinterpret_cast<const uint16_t*>(sc + i * 512);
-            scb[0] = *reinterpret_cast<const uint16_t*>(sc_b + wn * 1024);
-            scb[1] = *reinterpret_cast<const uint16_t*>(sc_b + wn * 1024 + 512);
-            scb[2] = *reinterpret_cast<const uint16_t*>(sc_b + 2048 + wn * 512);
+                for (int i = 0; i < kTwoTM; ++i) sca[i] = *reinterpret_cast<const uint16_t*>(sc + i * 512);
+                scb[0] = *reinterpret_cast<const uint16_t*>(sc_b + wn * 1024);
+                scb[1] = *reinterpret_cast<const uint16_t*>(sc_b + wn * 1024 + 512);
+                scb[2] = *reinterpret_cast<const uint16_t*>(sc_b + 2048 + wn * 512);
+            }
             const uint8_t* c0 = cur + a_off0;
             const uint8_t* c1 = cur + a_off1;
             __builtin_amdgcn_s_setprio(2);
@@ -159,7 +178,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             for (int i = 0; i < kTwoTM; ++i) a[i] = *reinterpret_cast<const uint4*>(c0 + i * 2048);
             __builtin_amdgcn_sched_barrier(0);
             // the next block's scales, behind the second step of a block, into the buffer that the block before has left
-            if ((ks & 3) == 1 && ks + 3 < nk) request_scales(ks + 3);
+            if (!BF16 && (ks & 3) == 1 && ks + 3 < nk) request_scales(ks + 3);
             const auto products = [&](auto sub_tag, int i, const uint4 (&bb)[kTwoTN]) {
                 constexpr int SUB = decltype(sub_tag)::value;
 #pragma unroll
@@ -172,7 +191,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                     } else {
                         cin = acc[i][j];
                     }
-                    acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(two_operand(bb[j]), two_operand(a[i]), cin, 4, 4, SUB, (int)scb[j], SUB, (int)sca[i]);
+                    if constexpr (BF16) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, bb[j]), __builtin_bit_cast(v8bf, a[i]), cin, 0, 0, 0);
+                    else acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(two_operand(bb[j]), two_operand(a[i]), cin, 4, 4, SUB, (int)scb[j], SUB, (int)sca[i]);
                 }
             };
 #pragma unroll
@@ -211,6 +231,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
         // the next tile's first step, into the first slot; the result leaves through the second (26576 x 3008 x 1920 86.7 -> 84.5 us)
         const int row0 = m0, col0 = n0;
+        [[maybe_unused]] const int segment = 2 * tile_n + wn;
         t += (int)gridDim.x;
         const bool more = t < tiles;
         if (more) begin(t);
@@ -224,12 +245,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         const int wsw = (ln & 7) * 16;
         const uint8_t* rd = region + rsub * 128 + ((chunk ^ rsub) * 16);
         const int64_t pitch8 = (int64_t)N * 16;   // eight rows, in bytes
-        const auto put_block = [&](const v16f& v, int side) {
+        const auto put_block = [&](v16f& v, int side) {   // BF16: leaves the rounded values in v
+            const float f = BF16 ? 1.0f : alpha;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const v2bf p0 = __builtin_convertvector(v2f{v[4 * q] * alpha, v[4 * q + 1] * alpha}, v2bf);
-                const v2bf p1 = __builtin_convertvector(v2f{v[4 * q + 2] * alpha, v[4 * q + 3] * alpha}, v2bf);
-                *reinterpret_cast<uint2*>(wr + (((side * 4 + q) * 16) ^ wsw)) = make_uint2(__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1));
+                const uint32_t p0 = __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{v[4 * q] * f, v[4 * q + 1] * f}, v2bf));
+                const uint32_t p1 = __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{v[4 * q + 2] * f, v[4 * q + 3] * f}, v2bf));
+                *reinterpret_cast<uint2*>(wr + (((side * 4 + q) * 16) ^ wsw)) = make_uint2(p0, p1);
+                if constexpr (BF16) {
+                    v[4 * q] = u2f(p0 << 16);
+                    v[4 * q + 1] = u2f(p0 & 0xffff0000u);
+                    v[4 * q + 2] = u2f(p1 << 16);
+                    v[4 * q + 3] = u2f(p1 & 0xffff0000u);
+                }
             }
         };
         const auto store_rows = [&](uint8_t* out, int row, bool col_ok) {   // of the lane's first row
@@ -262,8 +290,60 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
+        if constexpr (BF16) {
+            // a lane has 48 of its row's 96 columns (quads of them), the lane of the other half-wave the others
+#pragma unroll
+            for (int i = 0; i < kTwoTM; ++i) {
+                if (EDGES) {
+                    const int half_now = ln >> 5;
+#pragma unroll
+                    for (int j = 0; j < kTwoTN; ++j)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            const bool in = col0 + (j < 2 ? wn * 64 + j * 32 : 128 + wn * 32) + 8 * q + 4 * half_now < N;   // N is a multiple of 8
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) acc[i][j][4 * q + e] = in ? acc[i][j][4 * q + e] : -INFINITY;
+                        }
+                }
+                float top = -INFINITY;
+#pragma unroll
+                for (int j = 0; j < kTwoTN; ++j)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) top = fmaxf(top, acc[i][j][e]);
+                {
+                    const auto r = __builtin_amdgcn_permlane32_swap(f2u(top), f2u(top), false, false);
+                    top = fmaxf(u2f(r[0]), u2f(r[1]));
+                }
+                const float ref = top == -INFINITY ? 0.0f : top * kLog2e;   // nothing but -inf: every term is zero
+                float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int j = 0; j < kTwoTN; ++j)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) sum[e & 3] += __builtin_amdgcn_exp2f(__builtin_fmaf(acc[i][j][e], kLog2e, -ref));
+                float s = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+                {
+                    const auto r = __builtin_amdgcn_permlane32_swap(f2u(s), f2u(s), false, false);
+                    s = u2f(r[0]) + u2f(r[1]);
+                }
+                const int row = row0 + wm * 128 + i * 32 + (ln & 31);
+                if (ln < 32 && (!EDGES || row < M)) parts[(int64_t)segment * M + row] = make_float2(top, s);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
         if (!more) break;
     }
+}
+
+template <bool EDGES>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_mxfp4_tn_two_kernel(
+    const uint8_t* __restrict__ a_codes, const uint8_t* __restrict__ a_scales, const uint8_t* __restrict__ b_codes, const uint8_t* __restrict__ b_scales,
+    int M, int N, int K, float alpha, uint16_t* __restrict__ c, int late) {
+    two_run<false, EDGES>(a_codes, a_scales, b_codes, b_scales, M, N, K, alpha, c, late, nullptr);
+}
+template <bool EDGES>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_bf16_logits_kernel(
+    const uint8_t* __restrict__ a, const uint8_t* __restrict__ b, int M, int N, int K, uint16_t* __restrict__ c, int late, float2* __restrict__ parts) {
+    two_run<true, EDGES>(a, nullptr, b, nullptr, M, N, K, 1.0f, c, late, parts);
 }
 
 }  // namespace
@@ -289,6 +369,28 @@ hipError_t gemm_two(const TileProduct& p, hipStream_t stream) {
         return hipGetLastError();
     };
     return p.M % kTwoM || p.N % kTwoN ? go(std::true_type{}) : go(std::false_type{});
+}
+
+// x [T, K], w [V, K] in blocks of 16 rows and 32 elements (see above), whole blocks of rows; logits 16-byte aligned
+bool gemm_logits_serves(int64_t T, int64_t V, int64_t K) {
+    return T > 0 && V >= 8 && V % 8 == 0 && K % 32 == 0 && K >= 64 && K <= 8192 && T < (1 << 24) && V < (1 << 24) && T * V < (1ll << 38);
+}
+int64_t gemm_logits_segments(int64_t V) { return 2 * ((V + kTwoN - 1) / kTwoN); }
+hipError_t gemm_logits(const void* x, const void* w, int64_t T, int64_t V, int64_t K, void* logits, void* parts, hipStream_t stream) {
+    if (!gemm_logits_serves(T, V, K)) return hipErrorInvalidValue;
+    const int64_t tiles = ((T + kTwoM - 1) / kTwoM) * ((V + kTwoN - 1) / kTwoN);
+    const auto go = [&](auto edges) {
+        const auto kern = gemm_bf16_logits_kernel<decltype(edges)::value>;
+        static std::atomic<bool> lds_allowed[kMaxDevices];
+        const hipError_t e = allow_dynamic_lds(kern, kTwoScales, lds_allowed);
+        if (e != hipSuccess) return e;
+        int64_t grid = tiles < 2 * device_cus() ? tiles : 2 * device_cus();
+        if (grid > 8 && grid < tiles) grid -= grid % 8;
+        kern<<<dim3((unsigned)grid), dim3(256), kTwoScales, stream>>>(static_cast<const uint8_t*>(x), static_cast<const uint8_t*>(w), (int)T, (int)V, (int)K,
+                                                                      static_cast<uint16_t*>(logits), grid < tiles ? 8 : 0, static_cast<float2*>(parts));
+        return hipGetLastError();
+    };
+    return T % kTwoM || V % kTwoN ? go(std::true_type{}) : go(std::false_type{});
 }
 
 }  // namespace qm

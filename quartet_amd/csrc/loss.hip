@@ -149,6 +149,11 @@ __global__ __launch_bounds__(1024) void cross_entropy_mean_kernel(const float* _
 
 }  // namespace
 
+hipError_t loss_mean(const float* losses, const int64_t* targets, int64_t rows, int64_t ignore, float* loss, hipStream_t stream) {
+    cross_entropy_mean_kernel<<<dim3(1), dim3(1024), 0, stream>>>(losses, targets, rows, ignore, loss);
+    return hipGetLastError();
+}
+
 hipError_t cross_entropy_mean(const void* logits, int dtype, const int64_t* targets, int64_t rows, int64_t classes, int64_t ignore,
                               float* losses, float* loss, hipStream_t stream) {
     const auto go = [&](const auto* x, auto past) {
@@ -166,8 +171,7 @@ hipError_t cross_entropy_mean(const void* logits, int dtype, const int64_t* targ
         if (dtype == BF16) by_size(static_cast<const uint16_t*>(logits));
         else by_size(static_cast<const float*>(logits));
     }
-    cross_entropy_mean_kernel<<<dim3(1), dim3(1024), 0, stream>>>(losses, targets, rows, ignore, loss);
-    return hipGetLastError();
+    return loss_mean(losses, targets, rows, ignore, loss, stream);
 }
 
 }  // namespace qm

@@ -22,10 +22,11 @@ typedef float f2 __attribute__((ext_vector_type(2)));
 typedef __bf16 b2 __attribute__((ext_vector_type(2)));
 typedef uint32_t w2 __attribute__((ext_vector_type(2)));
 
+// blocks: the result goes to blocks of 16 rows and 32 elements, [rows / 16][cols / 32][16][32], as the product of the logits reads it (gemm_two.hip).
 // NV: vectors of four per lane, cols <= 256 NV; cols % 4 == 0.  TA: void, uint16_t (bf16) or float
 template <int NV, typename TA, typename TOut>
 __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const float* __restrict__ x, const TA* __restrict__ add, const float* __restrict__ gain, float eps,
-                                                           int64_t rows, int cols, TOut* __restrict__ out) {
+                                                           int64_t rows, int cols, TOut* __restrict__ out, int blocks) {
     const int lane = threadIdx.x & 63;
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;   // a whole wave
@@ -55,11 +56,12 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const float* __restri
         const int c = i * 256 + lane * 4;
         if (c >= cols) continue;
         const f4 r = v[i] * f * *reinterpret_cast<const f4*>(gain + c);
+        const int64_t at = blocks ? (row >> 4) * 16 * cols + (c >> 5) * 512 + (row & 15) * 32 + (c & 31) : row * cols + c;
         if constexpr (sizeof(TOut) == 2)
-            *reinterpret_cast<w2*>(out + row * cols + c) =
+            *reinterpret_cast<w2*>(out + at) =
                 w2{__builtin_bit_cast(uint32_t, __builtin_convertvector(f2{r[0], r[1]}, b2)), __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{r[2], r[3]}, b2))};
         else
-            *reinterpret_cast<f4*>(out + row * cols + c) = r;
+            *reinterpret_cast<f4*>(out + at) = r;
     }
 }
 
@@ -67,7 +69,7 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const float* __restri
 
 // cols % 4 == 0, cols <= 4096; x, gain, out (fp32) and an fp32 summand 16-byte, bf16 ones 8-byte aligned
 hipError_t rmsnorm_rows(const float* x, const void* add, int add_dtype, const float* gain, float eps, int64_t rows, int64_t cols, void* out, int out_dtype,
-                        hipStream_t stream) {
+                        hipStream_t stream, bool blocks) {
     constexpr int64_t kRows = 1 << 25;   // of a launch: a grid has fewer than 2^32 threads, 64 a row
     const auto go = [&](auto nv, const auto* a, auto* o) {
         for (int64_t r = 0; r < rows; r += kRows) {
@@ -75,7 +77,7 @@ hipError_t rmsnorm_rows(const float* x, const void* add, int add_dtype, const fl
             const A* ar = nullptr;
             if constexpr (!std::is_void<A>::value) ar = a + r * cols;
             const int64_t n = rows - r < kRows ? rows - r : kRows;
-            rmsnorm_rows_kernel<decltype(nv)::value><<<dim3((unsigned)((n + 3) / 4)), dim3(256), 0, stream>>>(x + r * cols, ar, gain, eps, n, (int)cols, o + r * cols);
+            rmsnorm_rows_kernel<decltype(nv)::value><<<dim3((unsigned)((n + 3) / 4)), dim3(256), 0, stream>>>(x + r * cols, ar, gain, eps, n, (int)cols, o + r * cols, (int)blocks);
         }
     };
     const auto by_out = [&](auto nv, const auto* a) {

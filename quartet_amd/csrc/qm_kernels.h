@@ -246,6 +246,15 @@ hipError_t gemm_wide_pair(TileProduct a, bool a_f32, TileProduct b, bool b_f32, 
 bool gemm_two_serves(const TileProduct& p);
 hipError_t gemm_two(const TileProduct& p, hipStream_t stream);
 
+// The logits of an evaluated model on the same tiles, bf16 [T, V], and for its loss per row and 96 columns the largest one and the sum of exponentials
+// relative to it, float2 parts [gemm_logits_segments(V)][T]; x and w bf16 in blocks [rows / 16][K / 32][16][64 bytes]
+bool gemm_logits_serves(int64_t T, int64_t V, int64_t K);
+int64_t gemm_logits_segments(int64_t V);
+hipError_t gemm_logits(const void* x, const void* w, int64_t T, int64_t V, int64_t K, void* logits, void* parts, hipStream_t stream);
+hipError_t bf16_blocks(const float* w, int64_t V, int64_t K, void* out, hipStream_t stream);   // fp32 rows into such blocks (lm_head.hip)
+hipError_t logits_loss_rows(const void* parts, int64_t segments, int64_t T, const void* logits, int64_t V, const int64_t* targets, int64_t ignore, float* losses,
+                            hipStream_t stream);
+
 // The product of at most 64 rows with a weight, both tiled (gemm_rows.hip): K % 128 == 0, N % 8 == 0, c 16-byte aligned, no mask.
 // Its sums are in another order than the other kernels'.
 bool gemm_rows_serves(const TileProduct& p);
@@ -300,9 +309,10 @@ hipError_t mfma_only(const uint8_t* operands, float* sink, int iters, hipStream_
 
 // RMSNorm of (x + add) (norm.hip): fp32 x, add null, bf16 or fp32, out bf16 or fp32; cols % 4 == 0, cols <= 4096
 hipError_t rmsnorm_rows(const float* x, const void* add, int add_dtype, const float* gain, float eps, int64_t rows, int64_t cols, void* out, int out_dtype,
-                        hipStream_t stream);
+                        hipStream_t stream, bool blocks = false);
 
 // mean cross-entropy over the rows whose target is not `ignore` (loss.hip); losses: scratch, one float per row
+hipError_t loss_mean(const float* losses, const int64_t* targets, int64_t rows, int64_t ignore, float* loss, hipStream_t stream);   // of the rows not ignored
 hipError_t cross_entropy_mean(const void* logits, int dtype, const int64_t* targets, int64_t rows, int64_t classes, int64_t ignore,
                               float* losses, float* loss, hipStream_t stream);
 

@@ -168,24 +168,54 @@ def rmsnorm_rope_linear(norm, c_attn, x, table, n_head, add=None):
     return (*rope_qkv(qkv, table, n_head), x)
 
 
+def _plain_rows(norm, layer, x, add):
+    """[x, add] as rows, of an RMSNorm module in front of a plain nn.Linear under bf16 autocast that nobody watches, where nothing asks for the norm's
+    gradient and a kernel here takes the tensors; else None."""
+    if not (type(layer) is torch.nn.Linear and not _watched(layer) and type(x) is torch.Tensor and x.is_cuda and x.dtype == torch.float32 and torch.is_autocast_enabled("cuda")
+            and torch.get_autocast_dtype("cuda") == torch.bfloat16 and not (one_node.transformed() or torch.compiler.is_compiling())):
+        return None
+    from .llama import RMSNorm
+    if type(norm) is not RMSNorm or any(_GLOBAL_HOOKS) or _watched(norm):
+        return None
+    gain, cols = norm.weight, x.shape[-1]
+    watched = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, add, gain))
+    if (watched or gain.dtype != torch.float32 or gain.shape != (cols,) or gain.device != x.device or not 0 < cols <= 4096
+            or cols % 4 or not 0 < x.numel() < 1 << 31
+            or not (add is None or (type(add) is torch.Tensor and add.dtype in _KERNEL_DTYPES and add.shape == x.shape and add.device == x.device))):
+        return None
+    rows = [t if t is None else t.reshape(-1, cols).contiguous() for t in (x, add)]
+    return None if any(t is not None and t.data_ptr() % 16 for t in (*rows, gain)) else rows
+
+
 def rmsnorm(norm, layer, x, add=None):
     """norm(x [+ add]) in front of `layer`.  Where that is a plain nn.Linear, in an evaluation under bf16 autocast in one pass, rounded to the
     bf16 that autocast hands the layer."""
-    plain = (type(layer) is torch.nn.Linear and not _watched(layer) and type(x) is torch.Tensor and x.is_cuda and x.dtype == torch.float32 and torch.is_autocast_enabled("cuda")
-             and torch.get_autocast_dtype("cuda") == torch.bfloat16 and not (one_node.transformed() or torch.compiler.is_compiling()))
-    if plain:
-        from .llama import RMSNorm
-        plain = type(norm) is RMSNorm and not (any(_GLOBAL_HOOKS) or _watched(norm))
-    if plain:
-        gain, cols = norm.weight, x.shape[-1]
-        watched = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, add, gain))
-        if (not watched and gain.dtype == torch.float32 and gain.shape == (cols,) and gain.device == x.device and 0 < cols <= 4096
-                and cols % 4 == 0 and 0 < x.numel() < 1 << 31
-                and (add is None or (type(add) is torch.Tensor and add.dtype in _KERNEL_DTYPES and add.shape == x.shape and add.device == x.device))):
-            rows = [t if t is None else t.reshape(-1, cols).contiguous() for t in (x, add)]
-            if not any(t is not None and t.data_ptr() % 16 for t in (*rows, gain)):
-                return kernels.rmsnorm(rows[0], gain.contiguous(), norm.eps, rows[1], torch.bfloat16).view(x.shape)
+    rows = _plain_rows(norm, layer, x, add)
+    if rows is not None:
+        return kernels.rmsnorm(rows[0], norm.weight.contiguous(), norm.eps, rows[1], torch.bfloat16).view(x.shape)
     return norm(x if add is None else x + add)
+
+
+# Contractions that logits_and_loss() takes: the library's product of a longer one is faster by more than the loss's own pass over the logits costs.
+# 32000 classes, us with the weight's conversion and the loss, in one pass and apart: 4096 tokens of 640 189 and 225, of 1536 392 and 404, of 2048 500 and
+# 503, of 3072 737 and 732; 1024 tokens of 640 75 and 84, of 1536 148 and 158, of 2048 216 and 199; 64 of 640 45 either way.
+_MAX_LOGITS_K = 1536
+
+
+def logits_and_loss(norm, layer, x, add, targets, ignore_index=-1):
+    """(layer(norm(x [+ add])), its cross-entropy against `targets`): ``rmsnorm``, a plain nn.Linear without bias and ``cross_entropy``, in an evaluation
+    under bf16 autocast with the loss's sums of exponentials worked out beside the logits."""
+    weight = layer.weight if type(layer) is torch.nn.Linear and layer.bias is None else None
+    if (type(weight) is torch.nn.Parameter and type(targets) is torch.Tensor and targets.dtype == torch.int64 and targets.shape == x.shape[:-1] and targets.is_contiguous()
+            and weight.dtype == torch.float32 and weight.device == x.device == targets.device and weight.dim() == 2 and weight.shape[1] == x.shape[-1] <= _MAX_LOGITS_K
+            and weight.is_contiguous() and weight.data_ptr() % 16 == 0 and not (torch.is_grad_enabled() and weight.requires_grad)):
+        rows = _plain_rows(norm, layer, x, add)
+        if rows is not None:
+            out = kernels.logits_loss(rows[0], norm.weight.contiguous(), norm.eps, rows[1], weight.detach(), targets.view(-1), ignore_index)
+            if out is not None:
+                return out[0].view(*x.shape[:-1], -1), out[1]
+    logits = layer(rmsnorm(norm, layer, x, add))
+    return logits, cross_entropy(logits.view(-1, logits.size(-1)), targets.view(-1), ignore_index=ignore_index)
 
 
 def cross_entropy(logits, targets, ignore_index=-1):

@@ -446,6 +446,28 @@ def linear_backward(e2, packed_x, packed_w, T, I, O, hd_x, signs_x, hd_w, signs_
     return gx, gw
 
 
+def logits_loss(x2, gain, eps, add, weight, targets, ignore_index):
+    """(logits [rows, classes] bf16, mean cross-entropy against int64 targets [rows]) of rmsnorm(x2 [+ add]) * gain and the fp32 `weight`, both
+    rounded to bf16; None for shapes that it does not serve."""
+    _require_cuda(x2, gain, add, weight, targets)
+    assert x2.is_contiguous() and x2.dtype == torch.float32 and gain.is_contiguous() and gain.dtype == torch.float32 and gain.shape == (x2.shape[1],)
+    assert add is None or (add.is_contiguous() and add.shape == x2.shape)
+    assert weight.is_contiguous() and weight.dtype == torch.float32 and weight.shape[1] == x2.shape[1]
+    assert targets.is_contiguous() and targets.dtype == torch.int64 and targets.shape == (x2.shape[0],)
+    T, K, V = *x2.shape, weight.shape[0]
+    size = _lib.lib().qm_logits_loss_workspace_bytes(T, K, V)
+    if not size:
+        return None
+    workspace = torch.empty(size, dtype=torch.uint8, device=x2.device)
+    logits = torch.empty((T, V), dtype=torch.bfloat16, device=x2.device)
+    loss = torch.empty((), dtype=torch.float32, device=x2.device)
+    with torch.cuda.device(x2.device):
+        rc = _lib.lib().qm_logits_loss(_ptr(x2), _ptr(add), _dtype_code(add.dtype) if add is not None else 0, _ptr(gain), float(eps), T, K, _ptr(weight), V,
+                                       _ptr(targets), ignore_index, _ptr(workspace), size, _ptr(logits), _ptr(loss), _stream())
+    _lib.check(rc, "qm_logits_loss")
+    return logits, loss
+
+
 def cross_entropy(logits, targets, ignore_index):
     """Mean cross-entropy of logits [rows, classes] against int64 targets [rows], fp32 scalar (no autograd)."""
     _require_cuda(logits, targets)

@@ -21,7 +21,7 @@ import torch.nn.functional as F
 from torch.nn.attention import SDPBackend, sdpa_kernel
 
 from .backward import BACKWARD_SCHEMES
-from .fused import cross_entropy, rmsnorm, rmsnorm_rope_linear, rmsnorm_swiglu_linear
+from .fused import logits_and_loss, rmsnorm, rmsnorm_rope_linear, rmsnorm_swiglu_linear
 from .linear import QuantizedLinear
 from .quantizers import QUANTIZER_CLASSES
 
@@ -244,11 +244,9 @@ class Llama(nn.Module):
             else:
                 x = block(x if pending is None else x + pending, table)
                 pending = None
-        x = rmsnorm(self.transformer.ln_f, self.lm_head, x, pending)
         if targets is not None:
-            logits = self.lm_head(x)
-            loss = cross_entropy(logits.view(-1, logits.size(-1)), targets.view(-1), ignore_index=-1)
+            logits, loss = logits_and_loss(self.transformer.ln_f, self.lm_head, x, pending, targets)
         else:
-            logits = self.lm_head(x[:, [-1], :])
+            logits = self.lm_head(rmsnorm(self.transformer.ln_f, self.lm_head, x, pending)[:, [-1], :])
             loss = None
         return {"logits": logits if get_logits else None, "loss": loss}

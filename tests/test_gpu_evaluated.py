@@ -219,3 +219,94 @@ def test_rows_that_are_not_the_layer_s_are_refused_as_without_packed_weights():
                 rmsnorm_rope_linear(norm, block.attn.c_attn, torch.randn(3, 96, 1280, device="cuda:0"), table, 5)
             with pytest.raises(RuntimeError):
                 rmsnorm_swiglu_linear(norm, block.mlp.w12, block.mlp.c_proj, torch.randn(3, 96, 1280, device="cuda:0"))
+
+
+def _head(T, K, V, add_dtype, seed):
+    from quartet_amd.llama import RMSNorm
+    norm, head = RMSNorm(K).to("cuda:0"), torch.nn.Linear(K, V, bias=False).to("cuda:0")
+    g = torch.Generator("cuda:0").manual_seed(seed)
+    with torch.no_grad():
+        norm.weight.add_(0.1 * torch.randn(K, generator=g, device="cuda:0"))
+        head.weight.copy_(3 * K ** -0.5 * torch.randn(V, K, generator=g, device="cuda:0"))
+    x = torch.randn(T, K, generator=g, device="cuda:0")
+    add = None if add_dtype is None else torch.randn(T, K, generator=g, device="cuda:0").to(add_dtype)
+    targets = torch.randint(0, V, (T,), generator=g, device="cuda:0")
+    return norm, head, x, add, targets
+
+
+@pytest.mark.parametrize("T,K,V", [(1, 64, 8), (17, 96, 200), (256, 128, 192), (255, 640, 1000), (257, 160, 392),   # edges of tiles, of quads of columns, two K steps
+                                   (3000, 640, 32000),                                                              # several tiles a workgroup
+                                   (700, 1536, 4104)])                                                              # the longest contraction
+@pytest.mark.parametrize("add_dtype", [None, BF16, torch.float32])
+def test_logits_with_their_loss(T, K, V, add_dtype):
+    """The logits are bf16 of fp32 sums of products of the bf16 operands: off by 2^-8 of themselves, and by the sums' own rounding (K
+    additions, below K 2^-24 of sum |h w|).  The loss is that of the stored logits: 2^-24 a term for exponentials, sums and logarithm, 1e-5."""
+    from quartet_amd import kernels as Kn
+    from quartet_amd.fused import logits_and_loss
+    print(f"case logits {T}x{K}x{V}", flush=True)
+    norm, head, x, add, targets = _head(T, K, V, add_dtype, T + K + V)
+    targets[::5] = -1
+    with torch.no_grad(), torch.autocast("cuda", dtype=BF16):
+        assert Kn._lib.lib().qm_logits_loss_workspace_bytes(T, K, V)
+        logits, loss = logits_and_loss(norm, head, x, add, targets)
+        h = Kn.rmsnorm(x, norm.weight, norm.eps, add, BF16)
+    assert logits.dtype == BF16 and logits.shape == (T, V) and loss.dtype == torch.float32
+    h, w = h.double(), head.weight.detach().to(BF16).double()
+    rows = torch.randperm(T, generator=torch.Generator().manual_seed(1))[:64].cuda()
+    want = h[rows] @ w.T
+    assert ((logits[rows].double() - want).abs() <= want.abs() * 2.0 ** -8 + K * 2.0 ** -24 * (h[rows].abs() @ w.abs().T)).all()
+    if T > 1:
+        ref = torch.nn.functional.cross_entropy(logits.double(), targets, ignore_index=-1)
+        assert abs(float(loss) - float(ref)) < 1e-5 * max(1.0, abs(float(ref)))
+    else:   # the only row is ignored: 0 / 0, as the library
+        assert torch.isnan(loss)
+
+
+def test_logits_with_values_that_are_not_finite():
+    """A row with an infinite or NaN logit, a row whose logits are all -inf, a target that is no class: the library's answer (NaN where it asserts)."""
+    from quartet_amd.fused import logits_and_loss
+    norm, head, x, _, targets = _head(300, 64, 400, None, 3)
+    with torch.no_grad():
+        norm.weight.fill_(1.0)
+        head.weight.zero_()
+        head.weight[:, 0] = 1.0
+        x.zero_()
+        x[:, 0] = 1.0
+        head.weight[7, 1] = float("inf")
+        x[5, 1] = -1.0   # class 7 of row 5: -inf; of the others 0 times inf, NaN
+        with torch.autocast("cuda", dtype=BF16):
+            logits, loss = logits_and_loss(norm, head, x, None, targets)
+            assert torch.isnan(loss) and logits[5, 7] == -float("inf")
+            kept = torch.full_like(targets, -1)
+            kept[5] = 3
+            _, loss = logits_and_loss(norm, head, x, None, kept)
+            want = torch.nn.functional.cross_entropy(logits[5:6].double(), kept[5:6])
+            assert abs(float(loss) - float(want)) < 1e-5
+            head.weight[7, 1] = 0.0
+            _, loss = logits_and_loss(norm, head, x, None, torch.full_like(targets, 400))
+            assert torch.isnan(loss)
+
+
+def test_logits_and_loss_take_the_modules_where_somebody_listens_or_asks_for_gradients():
+    import torch.nn.functional as F
+    from quartet_amd.fused import logits_and_loss, rmsnorm
+    norm, head, x, add, targets = _head(70, 64, 96, BF16, 5)
+    x, add, targets = x.view(2, 35, 64), add.view(2, 35, 64), targets.view(2, 35)
+    with torch.autocast("cuda", dtype=BF16):
+        apart = lambda: head(rmsnorm(norm, head, x, add))
+        logits, loss = logits_and_loss(norm, head, x, add, targets)   # the head's weight asks for a gradient
+        assert logits.requires_grad and loss.requires_grad
+        with torch.no_grad():
+            one, one_loss = logits_and_loss(norm, head, x, add, targets)
+            assert one.shape == logits.shape and abs(float(one_loss) - float(F.cross_entropy(one.view(-1, 96).double(), targets.view(-1)))) < 1e-5
+            seen = []
+            handle = head.register_forward_hook(lambda *a: seen.append(1))
+            got, _ = logits_and_loss(norm, head, x, add, targets)
+            assert len(seen) == 1 and torch.equal(got, apart())
+            handle.remove()
+            biased = torch.nn.Linear(64, 96).to("cuda:0")
+            assert torch.equal(logits_and_loss(norm, biased, x, add, targets)[0], biased(rmsnorm(norm, biased, x, add)))
+            with pytest.raises(RuntimeError):
+                logits_and_loss(norm, head, x, add, targets.t().contiguous().t())   # no view of these as one row
+    with torch.no_grad():   # no autocast: fp32 logits
+        assert logits_and_loss(norm, head, x, add, targets)[0].dtype == torch.float32
