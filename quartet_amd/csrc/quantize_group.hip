@@ -36,6 +36,7 @@
 #include <type_traits>
 
 #include "expand_formats.h"
+#include "hadamard_octet.h"
 #include "lds_requests.h"
 #include "qm_jobs.h"
 #include "qm_kernels.h"
@@ -1428,6 +1429,152 @@ struct ProducedRowsJob {
     }
 };
 
+// RMSNorm and quantizer with eight elements to a lane, four lanes to a group: fp32 rows of at most 2048 elements, tiled codes.  The same operations in
+// the same order as RmsNormProducer and quantize_group_regs, sums of a group's or a row's parts by lane exchanges instead of in one lane's registers:
+// the same bits.  A workgroup has as many rows as fit, each in a whole number of sixteen lanes (four groups, whose scale bytes leave together); one
+// barrier, behind the groups' sums of squares.  With a group to a lane, 4096 rows of 640 are 2048 waves of 1400 instructions with 20 of every 32
+// lanes at work; here 5500 waves of 300.  What bounds it at such sizes is latency, and with a summand the sum's way to memory: 4096 x 640 in an
+// evaluated 30 M model 11.1 -> 9.7 us, a pass of it 847 -> 836; past the caches the sum is no faster.  Sizes: octets_serve().
+template <typename TA>
+struct RmsNormOctetsJob {
+    static constexpr int kLds = 256;   // a workgroup's group sums, at most 64
+    static constexpr int kWaves = 0;
+    static constexpr bool kAdd = !std::is_void<TA>::value;
+    using TAdd = typename std::conditional<kAdd, TA, float>::type;
+    RmsNormProducer<float, TA> prod;
+    int64_t rows, cols;
+    float c;
+    uint32_t sign_word;
+    GroupOut out;
+    int groups, groups_p, wg_rows;
+    unsigned blocks;
+
+    RmsNormOctetsJob(const RmsNormProducer<float, TA>& prod_, int64_t rows_, int64_t cols_, uint32_t sign_word_, const GroupOut& out_)
+        : prod(prod_), rows(rows_), cols(cols_), c(hadamard_scale(32, F32)), sign_word(sign_word_), out(out_), groups((int)(cols_ / 32)),
+          groups_p((groups + 3) & ~3), wg_rows(256 / (groups_p * 4)), blocks((unsigned)((rows_ + wg_rows - 1) / wg_rows)) {}
+
+    // the sum over a group's four lanes of what are sums of eight neighbours each: the upper levels of its pairwise tree
+    __device__ __forceinline__ static float over_group(float v) {
+        v = v + lane_xor<1>(v);
+        return v + lane_xor<2>(v);
+    }
+    __device__ __forceinline__ static float tree_sum8(const float (&p)[8]) { return ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7])); }
+
+    __device__ __forceinline__ void run(unsigned bid) const {
+        typedef float v4 __attribute__((ext_vector_type(4)));
+        float* sums = reinterpret_cast<float*>(job_lds);   // [row of the workgroup][group]
+        const int tid = threadIdx.x, lane = tid & 63, per_row = groups_p * 4;
+        const int r = tid / per_row, at = tid - r * per_row, g = at >> 2, octet = at & 3;
+        const int64_t row = (int64_t)bid * wg_rows + r;
+        const bool in_row = r < wg_rows && row < rows, mine = in_row && g < groups;
+        float v[8], gain[8];
+        const int64_t first = row * cols + g * 32 + octet * 8;
+        float s = 0.0f;
+        if (mine) {
+            const v4* src = reinterpret_cast<const v4*>(prod.x + first);
+            v4 lo = src[0], hi = src[1];
+            const v4* gp = reinterpret_cast<const v4*>(prod.gain + g * 32 + octet * 8);
+            const v4 g0 = gp[0], g1 = gp[1];
+            if constexpr (kAdd) {
+                if constexpr (sizeof(TAdd) == 2) {
+                    const uint4 m = *reinterpret_cast<const uint4*>(prod.add + first);
+                    lo = lo + v4{u2f(m.x << 16), u2f(m.x & 0xffff0000u), u2f(m.y << 16), u2f(m.y & 0xffff0000u)};
+                    hi = hi + v4{u2f(m.z << 16), u2f(m.z & 0xffff0000u), u2f(m.w << 16), u2f(m.w & 0xffff0000u)};
+                } else {
+                    const v4* m = reinterpret_cast<const v4*>(prod.add + first);
+                    lo = lo + m[0];
+                    hi = hi + m[1];
+                }
+                v4* dst = reinterpret_cast<v4*>(prod.xsum + first);
+                dst[0] = lo;
+                dst[1] = hi;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[e] = lo[e];
+                v[4 + e] = hi[e];
+                gain[e] = g0[e];
+                gain[4 + e] = g1[e];
+            }
+            float sq[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sq[e] = v[e] * v[e];
+            s = tree_sum8(sq);
+        }
+        job_requests_issued();
+        s = over_group(s);
+        if (mine && octet == 0) sums[r * groups_p + g] = s;
+        __syncthreads();
+        // The row's sum as RmsNormProducer orders it: sixteen partial sums of every sixteenth group, then pairwise.  A wave's lanes are of at most
+        // four rows: sixteen lanes add up each of them.
+        const int r0 = (tid - lane) / per_row;
+        float total;
+        {
+            const int rr = r0 + (lane >> 4);
+            float acc = 0.0f;
+            if (rr < wg_rows)
+                for (int j = lane & 15; j < groups; j += 16) acc = acc + sums[rr * groups_p + j];
+#pragma unroll
+            for (int m = 1; m < 16; m <<= 1) acc = acc + __shfl_xor(acc, m, 64);
+            total = acc;
+        }
+        const float f = __shfl(1.0f / __builtin_sqrtf(total / (float)cols + prod.eps), (r - r0) * 16, 64);
+        if (!in_row) return;
+        if (at == 0) prod.factor[row] = f;
+        const int64_t ci = ((row >> 4) * 16 * groups_p + ((g >> 2) * 64 + (int)(row & 15) * 4 + (g & 3))) * 4 + octet;
+        uint32_t* codes = reinterpret_cast<uint32_t*>(out.codes);
+        uint32_t word = 0u, scale_byte = 0u;
+        if (mine) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = v[e] * f * gain[e];
+#pragma unroll
+            for (int h = 1; h < 8; h <<= 1)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    if (i & h) continue;
+                    const float a = v[i], b = v[i + h];
+                    v[i] = a + b;
+                    v[i + h] = a - b;
+                }
+            octet_cross_lane_stage<1>(v, octet);
+            octet_cross_lane_stage<2>(v, octet);
+            const uint32_t signs = sign_word >> (8 * octet);
+            float sq[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                v[e] = v[e] * u2f(f2u(-c) ^ (((signs >> e) & 1u) << 31));
+                sq[e] = v[e] * v[e];
+            }
+            const float ms = over_group(tree_sum8(sq)) * 0.03125f, m = over_group(tree_sum8(v)) * 0.03125f;
+            float var = ms - m * m;
+            var = var > 0.0f ? var : 0.0f;
+            int E = (int)((f2u(kQuestG * __builtin_sqrtf(var) + 1e-8f) >> 23) & 0xffu) - 127;
+            E = E > 127 ? 127 : E;
+            scale_byte = (uint32_t)(E + 127);
+            const float hw_scale = pow2i(E), thr = 6.0f * hw_scale;
+            uint32_t keep = 0u;
+#pragma unroll
+            for (int e = 7; e >= 0; --e) keep = __builtin_amdgcn_alignbit(keep, f2u(fabsf(v[e]) - thr), 31);
+            const auto convert = [&](auto below) {
+                word = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(word, below(v[0]), below(v[1]), hw_scale, 0);
+                word = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(word, below(v[2]), below(v[3]), hw_scale, 1);
+                word = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(word, below(v[4]), below(v[5]), hw_scale, 2);
+                word = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(word, below(v[6]), below(v[7]), hw_scale, 3) ^ 0x88888888u;
+            };
+            if (__builtin_expect(ms < __builtin_inff(), 1)) convert([](float x) { return below_ties(x); });
+            else convert([](float x) { return below_ties_any(x); });
+            reinterpret_cast<uint8_t*>(out.maskbits)[(row * groups + g) * 4 + octet] = (uint8_t)keep;
+        }
+        job_stores_next();
+        codes[ci] = word;   // zeros in the padding groups
+        // a row's lanes of four groups are sixteen aligned ones: their scale bytes in one dword
+        uint32_t four = scale_byte << (8 * (g & 3));
+        four |= f2u(lane_xor<4>(u2f(four)));
+        four |= f2u(lane_xor<8>(u2f(four)));
+        if ((at & 15) == 0) *reinterpret_cast<uint32_t*>(out.scales + row * groups_p + g) = four;
+    }
+};
+
 // The quantizer of the layer's weight rides in the same grid, behind the rows, where the launch is one of a training step under
 // autocast: fp32 weights, tiled codes of any extents.  By itself it is a launch of a few microseconds that mostly starts and ends
 // (1536 x 4096: 9.6 us, 4608 x 1536 11).  us per training step with the two launches and with one: 16384 x 1536 x 4608 behind its norm 449 ->
@@ -1459,6 +1606,12 @@ void launch_produced(const P& prod, int64_t rows, int64_t cols, uint32_t sign_wo
 
 }  // namespace
 
+namespace {
+// Where RmsNormOctetsJob is the faster one: a row fits a workgroup, and the tensor is small enough for waves to be what is missing.  us behind a copy
+// with a bf16 summand, a group and an octet to a lane: 8192 x 640 14.3 and 12.7, 16384 x 640 22.9 and 20.9, 4096 x 1536 15.7 and 13.7, 8192 x 1536 25.8 and 22.7,
+// 8192 x 2048 30.9 and 30.2; where the line lies 16384 x 1024 29.9 and 30.0, 16384 x 1536 57.7 either way, 32768 x 1536 102.6 and 105.8.
+bool octets_serve(int64_t rows, int64_t cols) { return cols <= 2048 && rows * cols <= 1 << 24; }
+}  // namespace
 bool producer_takes_weight(int dtype, int add_dtype, int w_dtype) { return dtype == F32 && add_dtype == BF16 && w_dtype == F32; }
 bool swiglu_takes_weight(int dtype, int w_dtype) { return dtype == BF16 && w_dtype == F32; }
 
@@ -1469,6 +1622,22 @@ hipError_t rmsnorm_quantize_hd32(const void* x, int dtype, const void* add, int 
                                  float* factor, bool tiled, const RowmajorArgs* weight, hipStream_t stream) {
     if (rows == 0) return hipSuccess;
     if (weight && !(tiled && producer_takes_weight(dtype, add ? add_dtype : BF16, weight->dtype))) return hipErrorInvalidValue;
+    if (tiled && dtype == F32 && octets_serve(rows, cols)) {
+        const float* xp = reinterpret_cast<const float*>(x);
+        float* sp = reinterpret_cast<float*>(xsum);
+        const GroupOut out{reinterpret_cast<uint4*>(codes), scales, reinterpret_cast<uint32_t*>(maskbits), nullptr};
+        const auto go = [&](const auto* summand) {
+            using TA = std::remove_const_t<std::remove_pointer_t<decltype(summand)>>;
+            const RmsNormOctetsJob<TA> job({xp, gain, factor, eps, reinterpret_cast<const typename RmsNormOctetsJob<TA>::TAdd*>(summand), sp}, rows, cols, sign_word, out);
+            if constexpr (!std::is_same<TA, float>::value)
+                if (weight) return launch_jobs(stream, job, weight_job(*weight));
+            launch_job(job, stream);
+        };
+        if (!add) go(static_cast<const void*>(nullptr));
+        else if (add_dtype == BF16) go(static_cast<const uint16_t*>(add));
+        else go(static_cast<const float*>(add));
+        return hipGetLastError();
+    }
     if (add) {
         if (dtype != F32) return hipErrorInvalidValue;
         const float* xp = reinterpret_cast<const float*>(x);

@@ -387,6 +387,46 @@ def test_residual_sum_inside_the_norm_quantizer(q, rows, cols, tiled, add_dtype)
     assert torch.equal(dx, dx2) and torch.equal(dg, dg2) and torch.equal(low, dx.to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("rows,cols", [(33000, 512), (25001, 672), (16400, 1056), (8200, 2048)])
+@pytest.mark.parametrize("add_dtype", [None, torch.bfloat16, torch.float32])
+def test_norm_of_few_rows_and_of_many(q, rows, cols, add_dtype):
+    """A tensor of more than 2^24 elements has a group of 32 to a lane, a few rows by themselves eight elements: the same bits, also of rows with
+    zeros, infinities, NaN and squares that overflow."""
+    from quartet_amd import _lib
+    print(f"case norm {rows}x{cols} {add_dtype}", flush=True)
+    g = torch.Generator(DEV).manual_seed(rows)
+    x = torch.randn(rows, cols, generator=g, device=DEV)
+    add = None if add_dtype is None else torch.randn(rows, cols, generator=g, device=DEV).to(add_dtype)
+    gain = 1 + 0.2 * torch.randn(cols, generator=g, device=DEV)
+    for r, v in ((1, 0.0), (2, 1e25), (3, 1e-30), (4, float("inf"))):
+        x[r] = v
+        if add is not None:
+            add[r] = 0.0
+    x[5, 7], x[6, 3] = float("nan"), -float("inf")
+
+    def run(part):
+        a = None if add is None else add[part].contiguous()
+        xs = x[part].contiguous()
+        n, L = xs.shape[0], _lib.lib()
+        packed = torch.zeros(L.qm_packed_operand_bytes(n, cols), dtype=torch.uint8, device=DEV)
+        factor, total = torch.empty(n, device=DEV), torch.zeros_like(xs)
+        p = lambda t: None if t is None else ctypes.c_void_p(t.data_ptr())
+        rc = L.qm_rmsnorm_quantize_mxfp4(p(xs), _lib.QM_F32, p(a), _lib.QM_BF16 if add_dtype == torch.bfloat16 else _lib.QM_F32, None if a is None else p(total), p(gain),
+                                         1e-5, n, cols, (ctypes.c_uint32 * 4)(0x5a5a1234, 0, 0, 0), p(packed), packed.numel(), p(factor), 2,
+                                         ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        assert rc == 0
+        off, pc = (ctypes.c_size_t * 3)(), (cols + 127) // 128 * 128
+        assert L.qm_packed_operand_offsets(n, cols, off) == 0
+        codes = packed[off[0]:off[0] + (n + 15) // 16 * 16 * pc // 2].view(-1, pc // 128, 16, 64).permute(0, 2, 1, 3).reshape(-1, pc // 2)[:n]
+        scales, mask = packed[off[1]:off[1] + n * pc // 32].view(n, -1), packed[off[2]:off[2] + n * cols // 8].view(n, -1)
+        return codes, scales, mask, factor.view(torch.int32), total.view(torch.int32)
+
+    whole = run(slice(0, rows))
+    for part in (slice(0, 77), slice(rows - 130, rows), slice(3, 4)):
+        for w, few in zip(whole, run(part)):
+            assert torch.equal(w[part], few)
+
+
 def test_block_with_deferred_residual_sums_matches_the_plain_block(q):
     """Two fused blocks chained through `pending` against the same blocks with every residual sum done by torch."""
     print("case fused blocks with pending sums", flush=True)
