@@ -99,8 +99,9 @@ def swiglu_linear(layer, h12):
 
 def _evaluated(norm, layers, x, add):
     """[(weight, its packed form, activation and weight quantizer)] of the layers behind an RMSNorm where nothing asks for a gradient, the
-    products are bf16 ones under autocast, and every weight's packed form is kept and up to date; else None."""
-    if not (x.is_cuda and torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16) or one_node.transformed() or torch.compiler.is_compiling():
+    products are bf16 ones under autocast of more than 64 tokens (up to which the products in question are others), and every weight's packed form is kept
+    and up to date; else None."""
+    if not (x.is_cuda and x.numel() > 64 * x.shape[-1] and torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16) or one_node.transformed() or torch.compiler.is_compiling():
         return None
     gain = getattr(norm, "weight", None)
     tensors = [x, gain] if add is None else [x, gain, add]

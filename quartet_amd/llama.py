@@ -9,7 +9,7 @@ linear is a ``QuantizedLinear`` built from registry names; init N(0, init_std) w
 ``init_std / sqrt(2 n_layer)``; cross-entropy over all positions.  The tokenizer the reference attaches
 (tiktoken) is not part of the numerics and is left out.
 
-Everything here except the block linears and an evaluation's loss is stock PyTorch: this module is plumbing around the hot
+Everything here except the block linears and an evaluation's last norm, logits and loss is stock PyTorch: this module is plumbing around the hot
 path."""
 import contextlib
 import math
@@ -18,8 +18,10 @@ from dataclasses import dataclass, field
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.backends.cuda import SDPAParams, can_use_efficient_attention
 from torch.nn.attention import SDPBackend, sdpa_kernel
 
+from . import one_node
 from .backward import BACKWARD_SCHEMES
 from .fused import logits_and_loss, rmsnorm, rmsnorm_rope_linear, rmsnorm_swiglu_linear
 from .linear import QuantizedLinear
@@ -147,6 +149,16 @@ def _sdpa_choice(mode, q):
     return sdpa_kernel([SDPBackend.EFFICIENT_ATTENTION, SDPBackend.FLASH_ATTENTION, SDPBackend.MATH], set_priority=True)
 
 
+def _first_choice(mode, q, k, v, dropout):
+    """Causal attention of an evaluated model by the kernel that _sdpa_choice() has tried first, called without the choice, which is 12 us of the
+    28 that a call costs the host; the same kernel, the same bits.  None where that kernel does not take the tensors or somebody asks for a gradient."""
+    if (mode != "auto" or dropout or not (type(q) is type(k) is type(v) is torch.Tensor) or not q.is_cuda or not (q.dtype == k.dtype == v.dtype == torch.bfloat16)
+            or (torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad)) or one_node.transformed() or torch.compiler.is_compiling()
+            or (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.bfloat16) or not can_use_efficient_attention(SDPAParams(q, k, v, None, 0.0, True, False))):
+        return None
+    return torch._scaled_dot_product_efficient_attention(q, k, v, None, False, 0.0, True)[0]
+
+
 class LlamaAttention(nn.Module):
     def __init__(self, config):
         super().__init__()
@@ -169,8 +181,10 @@ class LlamaAttention(nn.Module):
         q, k, v = q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2)
         if not torch.is_autocast_enabled() and v.dtype != q.dtype:
             v = v.to(q.dtype)
-        with _sdpa_choice(self.sdpa_backend, q):
-            y = F.scaled_dot_product_attention(q, k, v, attn_mask=None, dropout_p=self.dropout, is_causal=True)
+        y = _first_choice(self.sdpa_backend, q, k, v, self.dropout)
+        if y is None:
+            with _sdpa_choice(self.sdpa_backend, q):
+                y = F.scaled_dot_product_attention(q, k, v, attn_mask=None, dropout_p=self.dropout, is_causal=True)
         y = y.transpose(1, 2).contiguous().view(B, T, C)
         out = self.resid_dropout(self.c_proj(y))
         return out if norm is None else (out, x)   # with the fused norm: also x for the residual sum

@@ -310,3 +310,21 @@ def test_logits_and_loss_take_the_modules_where_somebody_listens_or_asks_for_gra
                 logits_and_loss(norm, head, x, add, targets.t().contiguous().t())   # no view of these as one row
     with torch.no_grad():   # no autocast: fp32 logits
         assert logits_and_loss(norm, head, x, add, targets)[0].dtype == torch.float32
+
+
+@pytest.mark.parametrize("B,S,heads,hs", [(1, 1, 5, 128), (3, 65, 2, 64), (2, 512, 5, 128), (1, 130, 12, 32)])
+def test_attention_called_directly_is_the_chosen_one(B, S, heads, hs):
+    import torch.nn.functional as F
+    from quartet_amd.llama import _first_choice, _sdpa_choice
+    g = torch.Generator("cuda:0").manual_seed(S)
+    q, k, v = (torch.randn(B, S, heads, hs, generator=g, device="cuda:0").to(BF16).transpose(1, 2) for _ in range(3))
+    with torch.no_grad():
+        with _sdpa_choice("auto", q):
+            want = F.scaled_dot_product_attention(q, k, v, attn_mask=None, dropout_p=0.0, is_causal=True)
+        got = _first_choice("auto", q, k, v, 0.0)
+        assert got is not None and got.shape == want.shape and got.stride() == want.stride() and torch.equal(got, want)
+        assert _first_choice("default", q, k, v, 0.0) is None and _first_choice("auto", q, k, v, 0.1) is None
+        assert _first_choice("auto", q.float(), k.float(), v.float(), 0.0) is None
+        with torch.autocast("cuda", dtype=torch.float16):
+            assert _first_choice("auto", q, k, v, 0.0) is None
+    assert _first_choice("auto", q.requires_grad_(True), k, v, 0.0) is None
