@@ -259,6 +259,9 @@ constexpr int backward_waves(int hd) { return hd == 32 ? 5 : 4; }
 // b % chunks of 512 columns (four code tiles); wave w owns rows 4w..4w+3 of the block, lane l its row l / 16 and
 // group l % 16 of the run: the wave reads four contiguous KiB (bf16) and writes, per tile, four rows' 64-byte pieces
 // = 256 contiguous bytes.  The four scale bytes of four adjacent groups are gathered into one dword store.
+// A last run of one or two code tiles would leave three quarters or half of such a workgroup idle: its workgroups own 64 or 32 rows of that
+// run instead, a lane per group.  us per training step with idle lanes and without: 16480 x 1728 x 640 111.6 -> 107.0, 24576 x 1152 x 640 113.7 -> 108.3,
+// 16384 x 640 x 1920 115.5 -> 112.4; widths of whole runs the same.
 // PADDED: any number of rows; columns that are not a multiple of 128 are completed with zero codes and scales.  (Whole tiles
 // have instantiations of their own: the edge tests cost the kernel 5 to 10 %.)
 template <typename T, int MODE, bool WANT_MASK, int HD = 32, bool PADDED = false>
@@ -266,29 +269,44 @@ struct RowmajorTiledJob {
     static constexpr int kLds = 0;
     static constexpr int kWaves = MODE == QUEST_RTN ? 8 : 0;   // forward: 62 registers; with padded extents 70 without the bound
     const T* x;
-    int rows, groups, groups_p, chunks;   // groups of 32 per row: of the tensor, of its padded code tiles
+    int rows, groups, groups_p, chunks;   // groups of 32 per row: of the tensor, of its padded code tiles; runs of up to 16 in workgroups of 16 rows
+    int narrow;                           // groups of the last run, 4 or 8, if it has workgroups of its own, or 0
     Rotation rot;
     uint64_t seed;
     const uint64_t* seed_base = nullptr;  // device memory, or null: a value the kernel adds to `seed` when it runs
     GroupOut out;
-    unsigned blocks;
+    unsigned wide_blocks, blocks;
 
     RowmajorTiledJob(const void* x_, int64_t rows_, int64_t cols_, const Rotation& rot_, uint64_t seed_, const GroupOut& out_)
         : x(reinterpret_cast<const T*>(x_)), rows((int)rows_), groups((int)(cols_ / 32)), groups_p((int)(padded_cols(cols_) / 32)),
-          chunks((groups_p + 15) / 16), rot(rot_), seed(seed_), out(out_), blocks((unsigned)(padded_rows(rows_) / 16 * chunks)) {}
+          chunks((groups_p + 15) / 16), narrow(groups_p % 16 == 12 ? 0 : groups_p % 16), rot(rot_), seed(seed_), out(out_) {
+        if (narrow) --chunks;
+        wide_blocks = (unsigned)(padded_rows(rows_) / 16 * chunks);
+        blocks = wide_blocks + (narrow ? (unsigned)((rows_ * narrow + 255) / 256) : 0u);
+    }
 
     __device__ __forceinline__ void run(unsigned bid) const {
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        const unsigned rb = bid / (unsigned)chunks;
-        const int g = (int)(bid - rb * chunks) * 16 + (lane & 15);  // group within the row
-        const int rin = wave * 4 + (lane >> 4);  // row within the block
+        unsigned rb;   // first block of 16 rows
+        int g, rin;    // group within the row, row within the block
+        const bool wide = bid < wide_blocks;
+        if (wide) {
+            rb = bid / (unsigned)chunks;
+            g = (int)(bid - rb * chunks) * 16 + (lane & 15);
+            rin = wave * 4 + (lane >> 4);
+        } else {
+            const int shift = narrow == 4 ? 2 : 3;
+            rb = (bid - wide_blocks) << (narrow == 4 ? 2 : 1);
+            g = chunks * 16 + ((int)threadIdx.x & (narrow - 1));
+            rin = (int)threadIdx.x >> shift;
+        }
         // groups_p is a multiple of four: quads of lanes leave together, but for the padding lanes of a row's last quad
         if (g >= (PADDED ? groups_p : groups)) return;
-        if (PADDED && (int)rb * 16 + rin >= rows) return;
+        if ((PADDED || !wide) && (int)rb * 16 + rin >= rows) return;
         // uniform 64-bit block bases + small per-lane offsets
         const int pitch = PADDED ? groups_p : groups;   // groups per row of the code and scale arrays
         const int64_t gi = (int64_t)rb * 16 * groups + (rin * groups + g);
-        const int64_t ci = (int64_t)rb * 16 * pitch + ((g >> 2) * 64 + rin * 4 + (g & 3));
+        const int64_t ci = (int64_t)rb * 16 * pitch + ((rin >> 4) * 16 * pitch + (g >> 2) * 64 + (rin & 15) * 4 + (g & 3));
         if (PADDED && g >= groups) {
             out.codes[ci] = make_uint4(0u, 0u, 0u, 0u);
             return;
