@@ -3,8 +3,8 @@
 // What bounds it: W has to come in once (4096 x 4096: 8.9 MB, 1.8 us at this card's copy rate); everything else is latency.
 // The tile kernels of gemm_tile.hip walk K through a ring in LDS with one barrier per 128 indices and put one workgroup on 32
 // columns: 9.6 us at 8 x 4096 x 4096 and 19.6 us at 1 x 4096 x 11008, a chain of 32 (86) steps on half of the CUs.  Here a
-// workgroup owns 16 columns (256 workgroups at N = 4096) and its waves share K among them, each with its own run of K steps
-// whose operands go straight from memory into the registers of v_mfma_scale_f32_16x16x128_f8f6f4, four steps ahead and
+// workgroup owns 16 columns (256 workgroups at N = 4096; more rows or columns: rows_tile()) and its waves share K among them, each with its own run of K steps
+// whose operands go straight from memory into the registers of v_mfma_scale_f32_16x16x128_f8f6f4, four to eight steps ahead and
 // without a barrier: in the tiled layout one K step of 16 rows is 1 KiB in exactly that instruction's order (lane l: row
 // l % 16, block l / 16 of 32 codes).  The waves' partial sums meet in LDS and are added in wave order, so results are
 // reproducible; they differ from the tile kernels' in the order of the fp32 additions, which shows where a row's group scales
@@ -19,26 +19,38 @@
 
 namespace qm {
 
+// With scales requested a step at a time, which touch as many cache lines as the codes do, and each request behind a condition (waits below), it
+// took, us MxNxK: 16x4096x4096 5.2 (now 3.9), 16x11008x4096 10.3 (6.4), 32x4096x4096 6.5 (4.4), 64x4096x4096 9.3 (5.3), 64x4096x11008 14.6 (8.9), 64x1536x8192
+// 15.7 (6.5); with the quantizer in it 1x11008x4096 8.2 (7.3), 8x4096x4096 6.7 (6.4).
 namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-constexpr int kRowsDepth = 4;   // K steps requested ahead of the products
+constexpr int kRowsDepth = 4;   // K steps requested at a time
+struct Scales {   // of a row's groups in that many steps: 4-byte aligned, as rows of a multiple of 128 have them
+    uint32_t w[kRowsDepth];
+};
+__device__ __forceinline__ Scales moved(const Scales& v, int by) {   // `by` steps on
+    const uint32_t w0 = v.w[0], w1 = v.w[1], w2 = v.w[2], w3 = v.w[3];
+    return Scales{{by == 0 ? w0 : by == 1 ? w1 : by == 2 ? w2 : w3, by == 0 ? w1 : by == 1 ? w2 : w3, by == 0 ? w2 : w3, w3}};
+}
 
-// The waves' partial sums in wave order.  Element e of a lane is column n0 + 4 * (lane / 16) + e of row lane % 16.
-template <int TM, int WAVES, typename OutT>
-__device__ __forceinline__ void add_waves(v4f (&partial)[WAVES][TM][64], const v4f (&acc)[TM], int wave, int lane, int n0, int M, int N, float alpha,
-                                          OutT* __restrict__ c) {
+// The waves' partial sums in wave order.  Element e of a lane of tile (i, j) is column n0 + 16 j + 4 * (lane / 16) + e of row m0 + 16 i + lane % 16.
+template <int TM, int TN, int WAVES, typename OutT>
+__device__ __forceinline__ void add_waves(v4f (&partial)[WAVES][TM * TN][64], const v4f (&acc)[TM][TN], int wave, int lane, int m0, int n0, int M, int N,
+                                          float alpha, OutT* __restrict__ c) {
     if (wave < WAVES) {
 #pragma unroll
-        for (int i = 0; i < TM; ++i) partial[wave][i][lane] = acc[i];
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) partial[wave][i * TN + j][lane] = acc[i][j];
     }
     __syncthreads();
-    for (int t = (int)threadIdx.x; t < TM * 64; t += WAVES * 64) {
-        const int i = t >> 6, l = t & 63, m = i * 16 + (l & 15), n = n0 + 4 * (l >> 4);
-        v4f sum = partial[0][i][l];
+    for (int t = (int)threadIdx.x; t < TM * TN * 64; t += WAVES * 64) {
+        const int tile = t >> 6, l = t & 63, m = m0 + tile / TN * 16 + (l & 15), n = n0 + tile % TN * 16 + 4 * (l >> 4);
+        v4f sum = partial[0][tile][l];
 #pragma unroll
-        for (int w = 1; w < WAVES; ++w) sum += partial[w][i][l];
+        for (int w = 1; w < WAVES; ++w) sum += partial[w][tile][l];
         if (m >= M || n >= N) continue;   // N is a multiple of 8
         OutT* dst = c + (int64_t)m * N + n;
         const v4f v = v4f{sum[0] * alpha, sum[1] * alpha, sum[2] * alpha, sum[3] * alpha};
@@ -52,73 +64,109 @@ __device__ __forceinline__ void add_waves(v4f (&partial)[WAVES][TM][64], const v
 }
 
 // W's rows are the instruction's first operand: a lane ends up with four consecutive columns of c, of row l % 16
-template <int TM, int WAVES, typename OutT>
+template <int TM, int TN, int WAVES, typename OutT>
 __global__ __launch_bounds__(WAVES * 64) void gemm_mxfp4_tn_rows_kernel(const uint8_t* __restrict__ a_codes, const uint8_t* __restrict__ a_scales,
                                                                          const uint8_t* __restrict__ b_codes, const uint8_t* __restrict__ b_scales,
                                                                          int M, int N, int K, float alpha, OutT* __restrict__ c) {
-    __shared__ v4f partial[WAVES][TM][64];
+    __shared__ v4f partial[WAVES][TM * TN][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int row = lane & 15, block = lane >> 4, shift = 8 * block;
     const int nk = K / kBK, groups = K / 32;
-    const int n0 = (int)blockIdx.x * 16;
+    const int n0 = (int)blockIdx.x * 16 * TN, m0 = (int)blockIdx.y * 16 * TM;
     const int first = wave * nk / WAVES, end = (wave + 1) * nk / WAVES;   // this wave's K steps
 
-    // rows past the end are read as the last one (a tiled operand's code rows exist up to the next multiple of 16)
-    const int b_row = n0 + row < N ? n0 + row : N - 1;
-    const uint8_t* b_code = b_codes + (int64_t)n0 * (K / 2) + row * 64 + block * 16;
-    const uint8_t* b_scale = b_scales + (int64_t)b_row * groups;
-    const uint8_t *a_code[TM], *a_scale[TM];
+    // A tiled operand's code rows exist up to the next multiple of 16: blocks of 16 rows past that are read as the last one, and of scales
+    // rows past the end as the last row.
+    const uint32_t in_block = (uint32_t)(row * 64 + block * 16);
+    const uint8_t *a_code[TM], *a_scale[TM], *b_code[TN], *b_scale[TN];   // uniform
+    uint32_t a_row[TM], b_row[TN];                                       // the lane's row of scales behind them
+    const auto block_of = [&](int from, int rows, const uint8_t* codes, const uint8_t* scales, const uint8_t*& code, const uint8_t*& scale, uint32_t& at) {
+        from = from < rows ? from : (rows - 1) & ~15;
+        code = codes + (int64_t)from * (K / 2);
+        scale = scales + (int64_t)from * groups;
+        at = (uint32_t)(from + row < rows ? row : rows - 1 - from) * (uint32_t)groups;
+    };
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
-        const int r = i * 16 + row < M ? i * 16 + row : M - 1;
-        a_code[i] = a_codes + (int64_t)(r & ~15) * (K / 2) + (r & 15) * 64 + block * 16;
-        a_scale[i] = a_scales + (int64_t)r * groups;
-    }
+    for (int i = 0; i < TM; ++i) block_of(m0 + i * 16, M, a_codes, a_scales, a_code[i], a_scale[i], a_row[i]);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) block_of(n0 + j * 16, N, b_codes, b_scales, b_code[j], b_scale[j], b_row[j]);
     struct Steps {
-        uint4 b[kRowsDepth], a[kRowsDepth][TM];
-        uint32_t sb[kRowsDepth], sa[kRowsDepth][TM];
+        Scales sa[TM], sb[TN];
+        uint4 a[kRowsDepth][TM], b[kRowsDepth][TN];
     };
-    // steps s .. s + depth - 1 of this wave; past its end a repeat of the last one, which is not multiplied
+    // Steps s .. s + depth - 1 of this wave; past its end sixteen bytes of the last one for all lanes, which cost one request and are not multiplied.
+    // Their scales in one request, which at a row's end begins up to three steps earlier (multiply_last): in rows of fewer steps in front of the
+    // row, which in a packed operand's first row is among its codes.
     const auto request = [&](Steps& f, int s) {
+        const int from = 4 * (s + kRowsDepth <= nk ? s : nk - kRowsDepth);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) f.sb[j] = *reinterpret_cast<const Scales*>(b_scale[j] + from + b_row[j]);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) f.sa[i] = *reinterpret_cast<const Scales*>(a_scale[i] + from + a_row[i]);
 #pragma unroll
         for (int d = 0; d < kRowsDepth; ++d) {
-            const int k = s + d < end ? s + d : end - 1;
-            f.b[d] = *reinterpret_cast<const uint4*>(b_code + (int64_t)k * 1024);
-            f.sb[d] = *reinterpret_cast<const uint32_t*>(b_scale + k * 4);
+            const int64_t at = (int64_t)(s + d < end ? s + d : end - 1) * 1024;
+            const uint32_t off = s + d < end ? in_block : 0u;
 #pragma unroll
-            for (int i = 0; i < TM; ++i) {
-                f.a[d][i] = *reinterpret_cast<const uint4*>(a_code[i] + (int64_t)k * 1024);
-                f.sa[d][i] = *reinterpret_cast<const uint32_t*>(a_scale[i] + k * 4);
-            }
+            for (int j = 0; j < TN; ++j) f.b[d][j] = *reinterpret_cast<const uint4*>(b_code[j] + at + off);
+#pragma unroll
+            for (int i = 0; i < TM; ++i) f.a[d][i] = *reinterpret_cast<const uint4*>(a_code[i] + at + off);
         }
+        __builtin_amdgcn_sched_barrier(0);
     };
-    v4f acc[TM];
+    v4f acc[TM][TN];
 #pragma unroll
-    for (int i = 0; i < TM; ++i) acc[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-    const auto multiply = [&](const Steps& f, int s) {
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    const auto multiply = [&](const Steps& f, int steps) {
 #pragma unroll
         for (int d = 0; d < kRowsDepth; ++d) {
-            if (s + d >= end) break;   // uniform
-            const v8i bv = v8i{(int)f.b[d].x, (int)f.b[d].y, (int)f.b[d].z, (int)f.b[d].w, 0, 0, 0, 0};
-            const int sb = (int)(f.sb[d] >> shift);
+            if (d >= steps) break;   // uniform
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
                 const v8i av = v8i{(int)f.a[d][i].x, (int)f.a[d][i].y, (int)f.a[d][i].z, (int)f.a[d][i].w, 0, 0, 0, 0};
-                acc[i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bv, av, acc[i], 4, 4, 0, sb, 0, (int)(f.sa[d][i] >> shift));
+                const int sa = (int)(f.sa[i].w[d] >> shift);
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    const v8i bv = v8i{(int)f.b[d][j].x, (int)f.b[d][j].y, (int)f.b[d][j].z, (int)f.b[d][j].w, 0, 0, 0, 0};
+                    acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bv, av, acc[i][j], 4, 4, 0, (int)(f.sb[j].w[d] >> shift), 0, sa);
+                }
             }
         }
+        __builtin_amdgcn_sched_barrier(0);
     };
+    const auto multiply_last = [&](Steps& f, int s) {
+        const int by = s + kRowsDepth <= nk ? 0 : s + kRowsDepth - nk;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) f.sb[j] = moved(f.sb[j], by);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) f.sa[i] = moved(f.sa[i], by);
+        multiply(f, end - s);
+    };
+    // Requests without a condition of their own: behind one that may or may not have been made, the compiler waits for what is older as if it had not
+    // been, which is for everything.
     if (first < end) {   // fewer K steps than waves: some have none
         Steps f0, f1;
-        request(f0, first);
-        for (int s = first; s < end; s += 2 * kRowsDepth) {
-            if (s + kRowsDepth < end) request(f1, s + kRowsDepth);
-            multiply(f0, s);
-            if (s + 2 * kRowsDepth < end) request(f0, s + 2 * kRowsDepth);
-            if (s + kRowsDepth < end) multiply(f1, s + kRowsDepth);
+        if (end - first <= kRowsDepth) {
+            request(f0, first);
+            multiply_last(f0, first);
+        } else {
+            request(f0, first);
+            request(f1, first + kRowsDepth);
+            int s = first;
+#pragma unroll 1
+            for (; s + 2 * kRowsDepth < end; s += 2 * kRowsDepth) {
+                multiply(f0, kRowsDepth);
+                request(f0, s + 2 * kRowsDepth);
+                multiply(f1, kRowsDepth);
+                request(f1, s + 3 * kRowsDepth);
+            }
+            multiply_last(f0, s);
+            multiply_last(f1, s + kRowsDepth);
         }
     }
-    add_waves<TM, WAVES>(partial, acc, wave, lane, n0, M, N, alpha, c);
+    add_waves<TM, TN, WAVES>(partial, acc, wave, lane, m0, n0, M, N, alpha, c);
 }
 
 // The same with the forward quantizer of x (Hadamard block 32, quest RTN) in front of the product, in every workgroup: the
@@ -126,7 +174,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_mxfp4_tn_rows_kernel(const ui
 // and a layer call is one launch.  The codes lie in LDS as [K step][row][64 bytes], the scales as one byte per group; the
 // weight's first eight K steps are on their way meanwhile.  Up to sixteen waves quantize, a group to a lane where that is enough
 // for all; WAVES of them multiply.  With WAVES alone, 8 x 4096 x 4096 took its 1024 groups four to a lane, one after the other, each
-// with its own wait for memory: 9.1 us, now 7.0.  Bit-identical to the two launches.
+// with its own wait for memory: 9.1 us, now 6.4.  Bit-identical to the two launches.
 constexpr int kDecodeThreads = 1024;
 template <int WAVES, typename T, typename OutT>
 __global__ __launch_bounds__(kDecodeThreads) void linear_decode_kernel(const T* __restrict__ x, float rot_c, uint32_t sign_word,
@@ -142,20 +190,20 @@ __global__ __launch_bounds__(kDecodeThreads) void linear_decode_kernel(const T* 
     const int first = multiplies ? wave * nk / WAVES : 0, end = multiplies ? (wave + 1) * nk / WAVES : 0;
     uint8_t* const x_scales = reinterpret_cast<uint8_t*>(x_codes + M * groups);
 
-    const int b_row = n0 + row < N ? n0 + row : N - 1;
-    const uint8_t* b_code = b_codes + (int64_t)n0 * (K / 2) + row * 64 + block * 16;
-    const uint8_t* b_scale = b_scales + (int64_t)b_row * groups;
+    const uint32_t in_block = (uint32_t)(row * 64 + block * 16);
+    const uint8_t* b_code = b_codes + (int64_t)n0 * (K / 2);
+    b_scales += (int64_t)n0 * groups;
+    const uint32_t b_scale = (uint32_t)(n0 + row < N ? row : N - 1 - n0) * (uint32_t)groups;
     struct Steps {
+        Scales sb;
         uint4 b[kRowsDepth];
-        uint32_t sb[kRowsDepth];
     };
-    const auto request = [&](Steps& f, int s) {
+    const auto request = [&](Steps& f, int s) {   // as above
+        f.sb = *reinterpret_cast<const Scales*>(b_scales + 4 * (s + kRowsDepth <= nk ? s : nk - kRowsDepth) + b_scale);
 #pragma unroll
-        for (int d = 0; d < kRowsDepth; ++d) {
-            const int k = s + d < end ? s + d : end - 1;
-            f.b[d] = *reinterpret_cast<const uint4*>(b_code + (int64_t)k * 1024);
-            f.sb[d] = *reinterpret_cast<const uint32_t*>(b_scale + k * 4);
-        }
+        for (int d = 0; d < kRowsDepth; ++d)
+            f.b[d] = *reinterpret_cast<const uint4*>(b_code + (int64_t)(s + d < end ? s + d : end - 1) * 1024 + (s + d < end ? in_block : 0u));
+        __builtin_amdgcn_sched_barrier(0);
     };
     Steps f0, f1;
     if (first < end) {
@@ -175,60 +223,94 @@ __global__ __launch_bounds__(kDecodeThreads) void linear_decode_kernel(const T* 
         x_scales[at] = (uint8_t)o.scale_byte;
     }
     __syncthreads();
-    v4f acc[1] = {v4f{0.0f, 0.0f, 0.0f, 0.0f}};
+    v4f acc[1][1] = {{v4f{0.0f, 0.0f, 0.0f, 0.0f}}};
     const int a_row = row < M ? row : M - 1;
-    const auto multiply = [&](const Steps& f, int s) {
+    const auto multiply = [&](const Steps& f, int s, int steps) {
 #pragma unroll
         for (int d = 0; d < kRowsDepth; ++d) {
-            if (s + d >= end) break;   // uniform
+            if (d >= steps) break;   // uniform
             const int at = ((s + d) * M + a_row) * 4 + block;
             const uint4 a = x_codes[at];
             const v8i bv = v8i{(int)f.b[d].x, (int)f.b[d].y, (int)f.b[d].z, (int)f.b[d].w, 0, 0, 0, 0};
             const v8i av = v8i{(int)a.x, (int)a.y, (int)a.z, (int)a.w, 0, 0, 0, 0};
-            acc[0] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bv, av, acc[0], 4, 4, 0, (int)(f.sb[d] >> shift), 0, (int)x_scales[at]);
+            acc[0][0] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bv, av, acc[0][0], 4, 4, 0, (int)(f.sb.w[d] >> shift), 0, (int)x_scales[at]);
         }
+        __builtin_amdgcn_sched_barrier(0);
     };
-    for (int s = first; s < end; s += 2 * kRowsDepth) {
-        multiply(f0, s);
-        if (s + 2 * kRowsDepth < end) request(f0, s + 2 * kRowsDepth);
-        if (s + kRowsDepth < end) multiply(f1, s + kRowsDepth);
-        if (s + 3 * kRowsDepth < end) request(f1, s + 3 * kRowsDepth);
+    const auto multiply_last = [&](Steps& f, int s) {
+        f.sb = moved(f.sb, s + kRowsDepth <= nk ? 0 : s + kRowsDepth - nk);
+        multiply(f, s, end - s);
+    };
+    int s = first;
+#pragma unroll 1
+    for (; s + 2 * kRowsDepth < end; s += 2 * kRowsDepth) {
+        multiply(f0, s, kRowsDepth);
+        request(f0, s + 2 * kRowsDepth);
+        multiply(f1, s + kRowsDepth, kRowsDepth);
+        request(f1, s + 3 * kRowsDepth);
     }
-    add_waves<1, WAVES>(partial, acc, wave, lane, n0, M, N, 1.0f, c);
+    multiply_last(f0, s);
+    multiply_last(f1, s + kRowsDepth);
+    add_waves<1, 1, WAVES>(partial, acc, wave, lane, 0, n0, M, N, 1.0f, c);
 }
-template <int TM, int WAVES>
+template <int TM, int TN, int WAVES>
 hipError_t launch_rows(const TileProduct& p, int c_dtype, hipStream_t stream) {
-    const dim3 grid((unsigned)((p.N + 15) / 16)), block(WAVES * 64);
+    const dim3 grid((unsigned)((p.N + 16 * TN - 1) / (16 * TN)), (unsigned)((p.M + 16 * TM - 1) / (16 * TM))), block(WAVES * 64);
     if (c_dtype == BF16)
-        gemm_mxfp4_tn_rows_kernel<TM, WAVES, uint16_t><<<grid, block, 0, stream>>>(p.a_codes, p.a_scales, p.b_codes, p.b_scales, p.M, p.N, p.K,
+        gemm_mxfp4_tn_rows_kernel<TM, TN, WAVES, uint16_t><<<grid, block, 0, stream>>>(p.a_codes, p.a_scales, p.b_codes, p.b_scales, p.M, p.N, p.K,
                                                                                    p.alpha, static_cast<uint16_t*>(p.c));
     else
-        gemm_mxfp4_tn_rows_kernel<TM, WAVES, float><<<grid, block, 0, stream>>>(p.a_codes, p.a_scales, p.b_codes, p.b_scales, p.M, p.N, p.K, p.alpha,
+        gemm_mxfp4_tn_rows_kernel<TM, TN, WAVES, float><<<grid, block, 0, stream>>>(p.a_codes, p.a_scales, p.b_codes, p.b_scales, p.M, p.N, p.K, p.alpha,
                                                                                 static_cast<float*>(p.c));
     return hipGetLastError();
 }
 
 }  // namespace
 
-// Which products run here rather than on the tile kernels; us, tile kernel -> this one, weights cycled through memory.
-// Up to 16 rows always: 1x4096x11008 20.1 -> 8.2, 8x4096x4096 9.6 -> 4.9, 16x512x8192 15.2 -> 7.2, 16x640x640 4.3 -> 4.2,
-// 16x11008x4096 11.0 -> 10.6, 16x11008x11008 23.8 -> 21.1.
-// More rows while every CU has at most one workgroup (each reads all of A): 17x4096x4096 9.6 -> 5.6, 64x4096x4096 10.4 -> 9.4,
-// 64x2048x11008 22.3 -> 18.6, but 32x6144x4096 9.8 -> 10.5, 64x6144x4096 10.6 -> 17.4.  Up to 32 rows also where K is short
-// enough for that not to matter: 32x8192x1536 6.0 -> 4.9, but 64x8192x1536 6.2 -> 7.5.
+// Tiles of 16 TM rows and 16 TN columns for four waves.  A workgroup requests (TM + TN) KiB a K step and little else bounds it, so the best tile is
+// the one whose workgroups bring in least per CU, in whole rounds of one to a CU: 24 ns a KiB, and beyond that what larger tiles take to start and
+// end.  us, by tile (1 x 1, 2 x 1, 2 x 2, 2 x 4; MxNxK): 32x2048x2048 2.7, 3.0, 3.3, 4.5; 32x4096x4096 5.2, 4.5, 5.2, 7.1; 64x4096x4096 -, 6.5, 5.3, 7.1;
+// 64x4096x11008 -, 12.7, 9.3, 13.2; 64x8192x4096 -, 10.5, 8.5, 7.3; 32x11008x4096 10.6, 8.5, 8.6, 7.6.  16x11008x4096 with 1 x 1 6.7, with 1 x 4 6.1.
+enum RowsTile : int { ROWS_1x1, ROWS_2x1, ROWS_2x2, ROWS_1x4, ROWS_2x4 };
+RowsTile rows_tile(const TileProduct& p) {
+    constexpr struct { int tm, tn; double start; } kTiles[] = {{1, 1, 0.0}, {2, 1, 0.15}, {2, 2, 0.25}, {1, 4, 0.25}, {2, 4, 0.55}};
+    const int64_t cus = device_cus();
+    int best = 0;
+    double least = 1e30;
+    for (int t = 0; t < 5; ++t) {
+        const int64_t workgroups = (int64_t)((p.M + 16 * kTiles[t].tm - 1) / (16 * kTiles[t].tm)) * ((p.N + 16 * kTiles[t].tn - 1) / (16 * kTiles[t].tn));
+        const double us = kTiles[t].start + 0.024 * (double)((workgroups + cus - 1) / cus * (kTiles[t].tm + kTiles[t].tn)) * (p.K / kBK);
+        if (us < least) {
+            least = us;
+            best = t;
+        }
+    }
+    return (RowsTile)best;
+}
+
+// Which products (MxNxK) run here rather than on the tile kernels: up to 16 rows all; up to 32 while their 2 x 4 tiles are at most three on four CUs, or
+// K is short; up to 64 while those are at most one on a CU.  us, tile kernel -> this one: 1x4096x11008 20.1 -> 5.9, 16x11008x4096 11.0 -> 6.4,
+// 17x4096x4096 9.6 -> 4.3, 32x8192x4096 7.8 -> 5.7, 32x11008x11008 15.9 -> 15.1, 64x8192x1536 4.9 -> 4.5, 64x8192x4096 7.9 -> 7.2; but 32x16384x4096
+// 8.7 -> 9.1, 64x11008x4096 8.3 -> 9.4.
 bool gemm_rows_serves(const TileProduct& p) {
     const bool kind = p.M > 0 && p.M <= 64 && p.N >= 8 && p.N % 8 == 0 && p.K > 0 && p.K % kBK == 0 && p.a_tiled && p.b_tiled && !p.mask &&
                       !p.b_e5m2 && (reinterpret_cast<uintptr_t>(p.c) & 15) == 0;
-    return kind && (p.M <= 16 || p.N <= 16 * device_cus() || (p.M <= 32 && p.K <= 2048));
+    const int64_t tiles = ((int64_t)p.N + 63) / 64;
+    return kind && (p.M <= 16 || (p.M <= 32 ? p.K <= 2048 || 4 * tiles <= 3 * device_cus() : 2 * tiles <= device_cus()));
 }
 
-// Waves: four, one per SIMD (8x8192x1536: 4.3 against 5.2 with eight, 64x4096x4096 9.4 / 10.8); eight where a long K leaves each
-// of them enough steps and few rows enough registers (1x4096x11008 8.2 against 8.7, 16x11008x11008 21.1 / 22.3)
+// Waves: four, one per SIMD (8x8192x1536 3.5, with eight 3.6; 64x4096x4096 5.3 and 5.6); eight where few rows meet a long K, whose sums are then of
+// shorter chains (16x4096x11008 6.4 and, with four, 6.0)
 hipError_t gemm_rows(const TileProduct& p, int c_dtype, hipStream_t stream) {
     if (!gemm_rows_serves(p)) return hipErrorInvalidValue;
-    if (p.M <= 16) return p.K >= 64 * kBK ? launch_rows<1, 8>(p, c_dtype, stream) : launch_rows<1, 4>(p, c_dtype, stream);
-    if (p.M <= 32) return launch_rows<2, 4>(p, c_dtype, stream);
-    return launch_rows<4, 4>(p, c_dtype, stream);
+    if (p.M <= 16 && p.K >= 64 * kBK) return launch_rows<1, 1, 8>(p, c_dtype, stream);
+    switch (rows_tile(p)) {
+        case ROWS_1x1: return launch_rows<1, 1, 4>(p, c_dtype, stream);
+        case ROWS_2x1: return launch_rows<2, 1, 4>(p, c_dtype, stream);
+        case ROWS_2x2: return launch_rows<2, 2, 4>(p, c_dtype, stream);
+        case ROWS_1x4: return launch_rows<1, 4, 4>(p, c_dtype, stream);
+        default: return launch_rows<2, 4, 4>(p, c_dtype, stream);
+    }
 }
 
 // One launch instead of two while a CU's share of quantizing is no more than 1024 groups, four per lane (about 5 us, what the

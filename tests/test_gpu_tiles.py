@@ -111,6 +111,31 @@ def test_decode_in_one_launch_is_the_same_layer(T, I, O, one_launch):
                 assert torch.equal(layer(xt[None, :, :])[0], want)
 
 
+# (T, I, O): K steps from fewer than a request's four to several rounds of eight a wave, with remainders of every kind at a wave's and at a row's end; a tile's
+# rows and columns past the end, for tiles of 16 x 16, 32 x 16, 32 x 32, 16 x 64 and 32 x 64; on both sides of the bounds of the kernel
+@pytest.mark.parametrize("T,I,O", [(3, 64, 24), (20, 352, 40), (40, 384, 24), (5, 640, 8), (16, 1056, 200), (33, 2176, 40), (24, 4480, 72), (64, 4736, 136), (16, 8960, 24),
+                                   (9, 12416, 40), (40, 6400, 56), (17, 8448, 4104), (33, 1152, 4088), (49, 1184, 4104), (64, 1664, 8184), (64, 128, 8200), (31, 2304, 12264),
+                                   (32, 2304, 12296), (15, 1152, 11000), (30, 672, 20008)])
+def test_product_of_few_rows_with_scales_apart(oracle, T, I, O):
+    """The layer's forward product of few tokens where neighbouring groups' scales are up to 2^12 apart, so that a scale taken from another K step shows
+    (one group of 400 too large or too small by a factor of two: 10^-2 of the norm and more).  fp32 output against the oracle's float64 sums of the same
+    packed operands, within K additions (1e-5 of the norm)."""
+    print(f"case few rows, scales apart T={T} I={I} O={O}", flush=True)
+    import quartet_amd as q
+    g = torch.Generator().manual_seed(T + I + O)
+    apart = lambda r: torch.exp2(torch.randint(-3, 4, (r, I // 32), generator=g).float()).repeat_interleave(32, 1)
+    x = make_input(T, I, torch.bfloat16, seed=1, outlier_frac=0).float() * apart(T)
+    w = (make_input(O, I, torch.bfloat16, seed=2, outlier_frac=0, scale=0.02).float() * apart(O)).to(torch.bfloat16)
+    layer = q.QuantizedLinear(I, O, bias=False, weight_quantizer=q.QuestMXFP4Quantizer(), activation_quantizer=q.QuestMXFP4Quantizer(),
+                              gradient_quantizer=q.AlbertTsengQuantizer(), backward_scheme=q.BACKWARD_SCHEMES["Q(E)Q(Wt)t_Q(Et)Q(Xt)t"]()).to("cuda:0", torch.bfloat16)
+    with torch.no_grad():
+        layer.weight.copy_(w.to("cuda:0"))
+        y = layer(x.to("cuda:0"))
+    qx, qw = (oracle.quantize(to_oracle(t), 32, mode=oracle.QUEST_RTN) for t in (x, w))
+    want = oracle.gemm_tn(qx["codes"], qx["scales"], qw["codes"], qw["scales"])
+    assert y.dtype == torch.float32 and rel(y.cpu().numpy(), want) < 1e-5
+
+
 # groups between the multiplying waves' lanes and sixteen waves' (320, 432, 1020 of them), behind four and eight multiplying waves
 @pytest.mark.parametrize("T,I,O", [(5, 2048, 264), (9, 1536, 40), (15, 2176, 520), (2, 9216, 24)])
 def test_decode_with_quantizing_waves_beside_the_multiplying_ones(T, I, O):
