@@ -106,16 +106,19 @@ struct TilePlan {
 // lanes request the row's final two 16-byte pieces in place of all four, and the scale dword that ends with the row's last
 // byte (two bytes early), so that no request leaves the row; the consumer shifts that dword down by 16 bits, which puts
 // the two real scale bytes first and zeros (2^-127: products vanish) where the missing half of the step would be.
+// live: all ones, or zero for a request that nobody reads, whose lanes then all ask for the panel's first sixteen bytes: one line instead of eight
+// (and of 64 for scales).  They keep a wave's counts of outstanding requests uniform, STAGES steps and a block of scales at the end of every tile: of K = 640
+// a third of all lines.  us per training step with repeats of the last step and now: 16480 x 1728 x 640 107.2 -> 105.2, 16384 x 640 x 1920 113.5 -> 112.3.
 template <class S>
-__device__ __forceinline__ void tile_issue(const TilePlan<S>& p, int stage, int ks, bool half) {
+__device__ __forceinline__ void tile_issue(const TilePlan<S>& p, int stage, int ks, bool half, uint32_t live = ~0u) {
     const uint32_t off = (uint32_t)stage * S::kStageBytes;
     const uint32_t back = half ? p.half_back : 0u;
     const uint8_t* a = p.a + (int64_t)ks * p.kstep_a;
     const uint8_t* b = p.b + (int64_t)ks * p.kstep_b;
 #pragma unroll
-    for (int j = 0; j < S::kALoads; ++j) load_lds_b128_s(a, p.voff_a[j] - back, p.lds_a + off + j * 1024);
+    for (int j = 0; j < S::kALoads; ++j) load_lds_b128_s(a, (p.voff_a[j] - back) & live, p.lds_a + off + j * 1024);
 #pragma unroll
-    for (int j = 0; j < S::kBLoads; ++j) load_lds_b128_s(b, p.voff_b[j] - back, p.lds_b + off + j * 1024);
+    for (int j = 0; j < S::kBLoads; ++j) load_lds_b128_s(b, (p.voff_b[j] - back) & live, p.lds_b + off + j * 1024);
     const int sback = half ? 2 : 0;
 #pragma unroll
     for (int u = 0; u < S::kSLoads; ++u)
@@ -123,9 +126,9 @@ __device__ __forceinline__ void tile_issue(const TilePlan<S>& p, int stage, int 
 }
 // BLOCKS: the 16 bytes of every row from K step ks on
 template <class S>
-__device__ __forceinline__ void tile_issue_scales(const TilePlan<S>& p, int ks) {
+__device__ __forceinline__ void tile_issue_scales(const TilePlan<S>& p, int ks, uint32_t live = ~0u) {
 #pragma unroll
-    for (int u = 0; u < S::kSLoads; ++u) load_lds_b128_s(p.s[u] + ks * 4, p.voff_s[u], p.lds_s[u]);
+    for (int u = 0; u < S::kSLoads; ++u) load_lds_b128_s(p.s[u] + ks * 4, p.voff_s[u] & live, p.lds_s[u]);
 }
 // the scale dwords of a lane's rows for four K steps
 template <class S>
@@ -357,6 +360,7 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
     if constexpr (ROT && S::kMaskEarly) issue_mask(S::kMaskOff);
 
     const auto issue = [&](int stage, int ks) { tile_issue<S>(plan, stage, ks, ks == half_step); };
+    const auto live_until = [&](int ks) { return ks < nk ? ~0u : 0u; };
     // the scale dwords of a half step arrive two bytes early (see tile_issue).  Without a branch: a K step is one basic block.
     const auto settle_scales = [&](uint32_t (&a)[S::TM], uint32_t (&b)[S::TN], int ks) {
         const uint32_t down = ks == half_step ? 16u : 0u;
@@ -508,7 +512,7 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
         const auto block_at = [&](int ks) { return ks + 4 <= nk ? ks : nk - 4; };
         tile_issue_scales<S>(plan, 0);
 #pragma unroll
-        for (int s = 0; s < S::STAGES; ++s) issue(s, s < nk ? s : nk - 1);
+        for (int s = 0; s < S::STAGES; ++s) tile_issue<S>(plan, s, s < nk ? s : nk - 1, false, live_until(s));   // whole steps: K is a multiple of 128
         __builtin_amdgcn_s_waitcnt(vmcnt_imm((S::STAGES - 1) * S::kLoads));  // the scales and step 0 are in; later ones may be pending
         __syncthreads();
         TileScales<S> sc;
@@ -537,9 +541,9 @@ __device__ __forceinline__ void tile_run(const TileProduct& g, int t, uint32_t* 
             __builtin_amdgcn_s_waitcnt(vmcnt_imm(Q == 3 && kPending > 2 * S::kLoads ? 2 * S::kLoads : kPending));
             __syncthreads();
             __builtin_amdgcn_sched_barrier(0);
-            // past the end: a repeat nobody reads keeps the counts of outstanding requests uniform
-            issue(stage, s + S::STAGES < nk ? s + S::STAGES : nk - 1);
-            if constexpr (Q == 0) tile_issue_scales<S>(plan, block_at(s + 4));   // every wave has taken this block's scales
+            // past the end: a request nobody reads
+            tile_issue<S>(plan, stage, s + S::STAGES < nk ? s + S::STAGES : nk - 1, false, live_until(s + S::STAGES));
+            if constexpr (Q == 0) tile_issue_scales<S>(plan, block_at(s + 4), live_until(s + 4));   // every wave has taken this block's scales
             if constexpr (Q == 3) tile_read_scales<S>(smem_bytes, a_sc_off, b_sc_off, sc);
             tile_read<S>(nxt, a_off0, b_off0, f0);
             tile_mfma<S, 1, SWAP, false>(f1, sca, scb, acc);
