@@ -623,7 +623,7 @@ def counters_to_json(fetch_dir, write_dir, sq_dir=None):
               "gemm_mxfp4_tn_rotated": lambda k: product(k) is not None and product(k)[2] != "0",
               "quantize_x_quest_rtn_mask_alone": lambda k: jobs(k) == ["RowmajorTiledJob"],
               "forward_quantizer_pair": lambda k: jobs(k) == ["RowmajorTiledJob"] * 2,
-              "backward_quantizers": lambda k: jobs(k) == ["TransposedJob", "RowmajorTiledJob"] + ["RequantTiledJob"] * 2,
+              "backward_quantizers": lambda k: jobs(k) == ["RequantTiledJob"] * 2 + ["TransposedJob", "RowmajorTiledJob"],
               "inverse_rotation_pair": lambda k: jobs(k) == ["HadamardBwdJob"] * 2}
     out = {}
     for name, match in groups.items():
