@@ -37,16 +37,9 @@ __device__ __forceinline__ Scales moved(const Scales& v, int by) {   // `by` ste
 
 // The waves' partial sums in wave order.  Element e of a lane of tile (i, j) is column n0 + 16 j + 4 * (lane / 16) + e of row m0 + 16 i + lane % 16.
 template <int TM, int TN, int WAVES, typename OutT>
-__device__ __forceinline__ void add_waves(v4f (&partial)[WAVES][TM * TN][64], const v4f (&acc)[TM][TN], int wave, int lane, int m0, int n0, int M, int N,
-                                          float alpha, OutT* __restrict__ c) {
-    if (wave < WAVES) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j) partial[wave][i * TN + j][lane] = acc[i][j];
-    }
+__device__ __forceinline__ void add_waves(const v4f (&partial)[WAVES][TM * TN][64], int threads, int m0, int n0, int M, int N, float alpha, OutT* __restrict__ c) {
     __syncthreads();
-    for (int t = (int)threadIdx.x; t < TM * TN * 64; t += WAVES * 64) {
+    for (int t = (int)threadIdx.x; t < TM * TN * 64; t += threads) {
         const int tile = t >> 6, l = t & 63, m = m0 + tile / TN * 16 + (l & 15), n = n0 + tile % TN * 16 + 4 * (l >> 4);
         v4f sum = partial[0][tile][l];
 #pragma unroll
@@ -166,34 +159,43 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_mxfp4_tn_rows_kernel(const ui
             multiply_last(f1, s + kRowsDepth);
         }
     }
-    add_waves<TM, TN, WAVES>(partial, acc, wave, lane, m0, n0, M, N, alpha, c);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) partial[wave][i * TN + j][lane] = acc[i][j];
+    add_waves<TM, TN, WAVES>(partial, WAVES * 64, m0, n0, M, N, alpha, c);
 }
 
 // The same with the forward quantizer of x (Hadamard block 32, quest RTN) in front of the product, in every workgroup: the
 // decoded batch is so small that quantizing it 256 times over costs no more time than doing it once in a launch of its own,
 // and a layer call is one launch.  The codes lie in LDS as [K step][row][64 bytes], the scales as one byte per group; the
 // weight's first eight K steps are on their way meanwhile.  Up to sixteen waves quantize, a group to a lane where that is enough
-// for all; WAVES of them multiply.  With WAVES alone, 8 x 4096 x 4096 took its 1024 groups four to a lane, one after the other, each
+// for all; WAVES x TN of them multiply.  With WAVES alone, 8 x 4096 x 4096 took its 1024 groups four to a lane, one after the other, each
 // with its own wait for memory: 9.1 us, now 6.4.  Bit-identical to the two launches.
+// TN: 16 columns each, with waves of their own, so that what a wave holds and adds is the same for any TN.  Wide layers have as many as leave one
+// workgroup to a CU (decode_columns()): with 16 columns a workgroup their CUs quantize all of x two to four times over.
 constexpr int kDecodeThreads = 1024;
-template <int WAVES, typename T, typename OutT>
+template <int WAVES, int TN, typename T, typename OutT>
 __global__ __launch_bounds__(kDecodeThreads) void linear_decode_kernel(const T* __restrict__ x, float rot_c, uint32_t sign_word,
                                                                     const uint8_t* __restrict__ b_codes, const uint8_t* __restrict__ b_scales, int M, int N,
                                                                     int I, int K, OutT* __restrict__ c) {
-    __shared__ v4f partial[WAVES][1][64];
+    __shared__ v4f partial[WAVES][TN][64];
     extern __shared__ uint4 x_codes[];   // [K / 128][M][4], then M * K / 32 scale bytes in the same order
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int row = lane & 15, block = lane >> 4, shift = 8 * block;
     const int nk = K / kBK, groups = K / 32, real_groups = I / 32;
-    const int n0 = (int)blockIdx.x * 16;
-    const bool multiplies = wave < WAVES;
-    const int first = multiplies ? wave * nk / WAVES : 0, end = multiplies ? (wave + 1) * nk / WAVES : 0;
+    const int n0 = (int)blockIdx.x * 16 * TN;
+    const bool multiplies = wave < WAVES * TN;
+    const int share = wave % WAVES, column = wave / WAVES;   // of K, and which 16 columns
+    const int first = multiplies ? share * nk / WAVES : 0, end = multiplies ? (share + 1) * nk / WAVES : 0;
     uint8_t* const x_scales = reinterpret_cast<uint8_t*>(x_codes + M * groups);
 
     const uint32_t in_block = (uint32_t)(row * 64 + block * 16);
-    const uint8_t* b_code = b_codes + (int64_t)n0 * (K / 2);
-    b_scales += (int64_t)n0 * groups;
-    const uint32_t b_scale = (uint32_t)(n0 + row < N ? row : N - 1 - n0) * (uint32_t)groups;
+    int from = n0 + 16 * column;   // past the end the last 16 rows of W, which are not stored
+    from = from < N ? from : (N - 1) & ~15;
+    const uint8_t* b_code = b_codes + (int64_t)from * (K / 2);
+    b_scales += (int64_t)from * groups;
+    const uint32_t b_scale = (uint32_t)(from + row < N ? row : N - 1 - from) * (uint32_t)groups;
     struct Steps {
         Scales sb;
         uint4 b[kRowsDepth];
@@ -223,7 +225,7 @@ __global__ __launch_bounds__(kDecodeThreads) void linear_decode_kernel(const T* 
         x_scales[at] = (uint8_t)o.scale_byte;
     }
     __syncthreads();
-    v4f acc[1][1] = {{v4f{0.0f, 0.0f, 0.0f, 0.0f}}};
+    v4f acc = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     const int a_row = row < M ? row : M - 1;
     const auto multiply = [&](const Steps& f, int s, int steps) {
 #pragma unroll
@@ -233,7 +235,7 @@ __global__ __launch_bounds__(kDecodeThreads) void linear_decode_kernel(const T* 
             const uint4 a = x_codes[at];
             const v8i bv = v8i{(int)f.b[d].x, (int)f.b[d].y, (int)f.b[d].z, (int)f.b[d].w, 0, 0, 0, 0};
             const v8i av = v8i{(int)a.x, (int)a.y, (int)a.z, (int)a.w, 0, 0, 0, 0};
-            acc[0][0] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bv, av, acc[0][0], 4, 4, 0, (int)(f.sb.w[d] >> shift), 0, (int)x_scales[at]);
+            acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bv, av, acc, 4, 4, 0, (int)(f.sb.w[d] >> shift), 0, (int)x_scales[at]);
         }
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -251,7 +253,8 @@ __global__ __launch_bounds__(kDecodeThreads) void linear_decode_kernel(const T* 
     }
     multiply_last(f0, s);
     multiply_last(f1, s + kRowsDepth);
-    add_waves<1, 1, WAVES>(partial, acc, wave, lane, 0, n0, M, N, 1.0f, c);
+    if (multiplies) partial[share][column][lane] = acc;
+    add_waves<1, TN, WAVES>(partial, (int)blockDim.x, 0, n0, M, N, 1.0f, c);
 }
 template <int TM, int TN, int WAVES>
 hipError_t launch_rows(const TileProduct& p, int c_dtype, hipStream_t stream) {
@@ -313,35 +316,53 @@ hipError_t gemm_rows(const TileProduct& p, int c_dtype, hipStream_t stream) {
     }
 }
 
-// One launch instead of two while a CU's share of quantizing is no more than 1024 groups, four per lane (about 5 us, what the
-// quantizer's own launch takes): 8x4096x4096 7.0 us against 4.2 + 4.2 and 1x4096x11008 7.2 against 4.4 + 5.6, where a call's
-// host time, which is what bounds both, falls from 12.5 to 10.3 us (and from 8.9 to 7.2 with fewer attribute look-ups)
+// Columns of a workgroup, in sixteens: as many as it takes for one workgroup to a CU, of which sixteen waves are the most.  us by columns / 16 (1, 2, 3, 4;
+// MxNxK): 8x4096x4096 6.7, 6.4, 6.8, 7.3; 8x8192x2048 6.6, 5.1, 5.3, 5.4; 12x4608x2048 8.4, 5.3, 6.0, 6.2; 8x11008x4096 15.8, 12.2, 8.1, 8.5; 16x11008x1152 11.5,
+// 8.5, 5.8, 5.9; 1x16384x2048 6.3, 6.0, 7.9, 5.7; 4x8192x8192 (eight waves to K) 13.1, 9.7.  Of few groups equal: 1x11008x640 4.2, 4.5, 4.3, 4.5.
+int decode_columns(int64_t O, int64_t K) {
+    const int64_t blocks = (O + 15) / 16, most = K >= 64 * kBK ? 2 : 4, need = (blocks + device_cus() - 1) / device_cus();
+    return (int)(need < most ? need : most);
+}
+
+// One launch instead of two while a CU's share of quantizing is no more than 1024 groups, one to a lane (about 3 us; the quantizer's own
+// launch takes 4): us in two launches and in one, 8x4096x4096 6.7 and 6.4 to 6.7, 8x11008x4096 9.8 and 8.1, 4x11008x4096 9.5 and 6.9, 16x11008x2048 8.1 and
+// 6.6, 1x4096x4096 6.7 and 4.7, 2x11008x11008 (1376 groups) 17.9 and 17.4; a call's host time, which bounds most of these, falls from 10.6 to 7.2
 bool linear_decode_serves(int64_t T, int64_t I, int64_t O) {
     if (!(T > 0 && T <= 16 && I > 0 && I % 32 == 0 && I < (1 << 20) && O >= 8 && O % 8 == 0 && O < (1 << 24))) return false;
-    const int64_t per_cu = ((O + 15) / 16 + device_cus() - 1) / device_cus();
-    return T * (padded_cols(I) / 32) * per_cu <= 1024;
+    const int64_t K = padded_cols(I), columns = 16 * decode_columns(O, K);
+    const int64_t per_cu = ((O + columns - 1) / columns + device_cus() - 1) / device_cus();
+    return T * (K / 32) * per_cu <= 1024;
 }
 
 hipError_t linear_decode(const void* x, int x_dtype, int64_t T, int64_t I, int64_t O, uint32_t sign_word, const uint8_t* w_codes,
                          const uint8_t* w_scales, void* y, int y_dtype, hipStream_t stream) {
     if (!linear_decode_serves(T, I, O)) return hipErrorInvalidValue;
-    const int K = (int)padded_cols(I);
+    const int K = (int)padded_cols(I), columns = decode_columns(O, K);
     const unsigned lds = (unsigned)(T * (K / 32) * 17);
     const float c = hadamard_scale(32, x_dtype);
-    const dim3 grid((unsigned)((O + 15) / 16));
-    const auto go = [&](auto waves, auto tx, auto ty) {   // as many waves as gemm_rows() takes: the same sums in the same order
-        constexpr int W = decltype(waves)::value;
+    const dim3 grid((unsigned)((O + 16 * columns - 1) / (16 * columns)));
+    const auto go = [&](auto waves, auto tn, auto tx, auto ty) {   // as many waves to K as gemm_rows() takes: the same sums in the same order
+        constexpr int W = decltype(waves)::value, TN = decltype(tn)::value;
         const int64_t lanes = (T * (K / 32) + 63) / 64 * 64;
-        const unsigned threads = (unsigned)(lanes < W * 64 ? W * 64 : lanes < kDecodeThreads ? lanes : kDecodeThreads);
-        linear_decode_kernel<W, decltype(tx), decltype(ty)><<<grid, dim3(threads), lds, stream>>>(
+        const unsigned threads = (unsigned)(lanes < W * TN * 64 ? W * TN * 64 : lanes < kDecodeThreads ? lanes : kDecodeThreads);
+        linear_decode_kernel<W, TN, decltype(tx), decltype(ty)><<<grid, dim3(threads), lds, stream>>>(
             static_cast<const decltype(tx)*>(x), c, sign_word, w_codes, w_scales, (int)T, (int)O, (int)I, K, static_cast<decltype(ty)*>(y));
     };
-    const auto typed = [&](auto waves) {
-        if (x_dtype == BF16) { if (y_dtype == BF16) go(waves, uint16_t{}, uint16_t{}); else go(waves, uint16_t{}, float{}); }
-        else { if (y_dtype == BF16) go(waves, float{}, uint16_t{}); else go(waves, float{}, float{}); }
+    const auto typed = [&](auto waves, auto tn) {
+        if (x_dtype == BF16) { if (y_dtype == BF16) go(waves, tn, uint16_t{}, uint16_t{}); else go(waves, tn, uint16_t{}, float{}); }
+        else { if (y_dtype == BF16) go(waves, tn, float{}, uint16_t{}); else go(waves, tn, float{}, float{}); }
     };
-    if (K >= 64 * kBK) typed(std::integral_constant<int, 8>{});
-    else typed(std::integral_constant<int, 4>{});
+    if (K >= 64 * kBK) {
+        const std::integral_constant<int, 8> waves;
+        if (columns == 1) typed(waves, std::integral_constant<int, 1>{});
+        else typed(waves, std::integral_constant<int, 2>{});
+    } else {
+        const std::integral_constant<int, 4> waves;
+        if (columns == 1) typed(waves, std::integral_constant<int, 1>{});
+        else if (columns == 2) typed(waves, std::integral_constant<int, 2>{});
+        else if (columns == 3) typed(waves, std::integral_constant<int, 3>{});
+        else typed(waves, std::integral_constant<int, 4>{});
+    }
     return hipGetLastError();
 }
 

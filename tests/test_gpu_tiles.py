@@ -142,6 +142,12 @@ def test_decode_with_quantizing_waves_beside_the_multiplying_ones(T, I, O):
     test_decode_in_one_launch_is_the_same_layer(T, I, O, True)
 
 
+# workgroups of two, three and four times 16 columns, of which the last one has one, none past the end, or a partial one; more than one to a CU; eight waves to K
+@pytest.mark.parametrize("T,I,O", [(16, 640, 4104), (16, 2048, 8192), (9, 1152, 8200), (16, 2048, 8216), (8, 4096, 11008), (5, 96, 12296), (16, 1024, 16408), (4, 8192, 4104), (1, 8320, 8232)])
+def test_decode_of_wide_layers(T, I, O):
+    test_decode_in_one_launch_is_the_same_layer(T, I, O, True)
+
+
 @pytest.mark.parametrize("T,I,O,hd", [(32, 32, 32, 32), (4128, 96, 160, 32), (4160, 192, 128, 64), (4224, 128, 256, 128), (96, 160, 96, 32), (288, 192, 320, 32), (544, 1728, 352, 32), (1056, 640, 1088, 32),
                                       (64, 64, 64, 64), (192, 320, 128, 64), (128, 128, 128, 128), (384, 256, 640, 128), (1280, 384, 896, 128)])
 def test_layer_on_padded_operands(oracle, T, I, O, hd):
