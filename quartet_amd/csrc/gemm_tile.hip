@@ -906,6 +906,12 @@ hipError_t launch_after(TileProduct g, const TileAfter& after, hipStream_t strea
 
 using Tile256x128 = TileShape<256, 128, 128, 64, 3, 2>;
 using Tile128x128 = TileShape<128, 128, 64, 64, 3, 3>;
+// One more stage where no CU has a second workgroup, which would cover a request's latency.  Plain results, us with three stages and with four: 1024 x 4096^2
+// 13.7 and 12.9, 768 x 4096 x 11008 36.0 and 32.3, 2048 x 1536 x 4096 12.3 and 11.3, 512 x 8192 x 1536 7.9 and 7.5, 1024 x 3072 x 8192 23.9 and 18.8, 1024 x 3456 x
+// 640 5.6 either way.  Up to two workgroups to a CU neither gains (1280 x 4096 x 11008 46.0 and 46.4, 640 x 8192 x 1536 10.3 and 10.0, 1792 x 4096 x 11008 47.9 and
+// 49.9).  Eight waves of 64 x 32 instead of four 13.8 -> 14.5 at 1024 x 4096^2, six stages 13.7: the next block's scales, asked for three steps ahead, hold a ring at
+// four.
+using Deep128x128 = TileShape<128, 128, 64, 64, 4, 2>;
 using Tile128x64 = TileShape<128, 64, 64, 32, 4, 3>;
 using Tile64x64 = TileShape<64, 64, 32, 32, 4, 4>;
 using Tile64x32 = TileShape<64, 32, 32, 32, 6, 4>;
@@ -991,10 +997,13 @@ hipError_t gemm_tile(int shape, const TileProduct& g, int c_dtype, hipStream_t s
     // blocks of scales: every K range has at least four steps, all whole, and scale rows start at multiples of four bytes
     const bool blocks = g.K % kBK == 0 && g.K / kBK / g.splits >= 4 &&
                         ((reinterpret_cast<uintptr_t>(g.a_scales) | reinterpret_cast<uintptr_t>(g.b_scales)) & 3) == 0;
+    const auto run_plain = [&](auto s) {
+        using S = decltype(s);
+        return c_dtype == BF16 ? launch_tiles<S, uint16_t>(g, stream) : launch_tiles<S, float>(g, stream);
+    };
     const auto run = [&](auto s) {
         using S = decltype(s);
-        if (c_dtype != BF16) return launch_tiles<S, float>(g, stream);
-        return g.mask ? launch_tiles<S, uint16_t, true>(g, stream) : launch_tiles<S, uint16_t>(g, stream);
+        return c_dtype == BF16 && g.mask ? launch_tiles<S, uint16_t, true>(g, stream) : run_plain(s);
     };
     // 256 x 128 over fewer than eight steps: its two blocks of 384 rows are more in front of the first step than they save behind it
     // (4096 x 3456 x 640 in an evaluated model 14 us, 16 with blocks)
@@ -1015,7 +1024,7 @@ hipError_t gemm_tile(int shape, const TileProduct& g, int c_dtype, hipStream_t s
     }
     switch (shape) {
         case TILE_256x128: return go(Tile256x128{});
-        case TILE_128x128: return go(Tile128x128{});
+        case TILE_128x128: return blocks && !g.mask && (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) * g.splits <= device_cus() ? run_plain(Deep128x128{}) : go(Tile128x128{});
         case TILE_128x64: return go(Tile128x64{});
         case TILE_64x64: return go(Tile64x64{});
         default: return go(Tile64x32{});

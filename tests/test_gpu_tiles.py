@@ -142,6 +142,25 @@ def test_decode_with_quantizing_waves_beside_the_multiplying_ones(T, I, O):
     test_decode_in_one_launch_is_the_same_layer(T, I, O, True)
 
 
+# 128 x 128 tiles, at most one to a CU: whole and short last blocks of four K steps (5, 6, 9, 12, 17, 20 steps), one row or eight columns past a tile, 256 of them
+@pytest.mark.parametrize("T,I,O", [(641, 1056, 4104), (1000, 2560, 2560), (1537, 1504, 1544), (1025, 640, 3336), (2047, 2176, 1992), (900, 704, 4096)])
+def test_products_on_one_large_tile_to_a_cu(T, I, O):
+    """A frozen layer's output, whole and by 100 rows (smaller tiles, the same order of additions), in bf16 and in fp32: the same bits."""
+    print(f"case one tile to a CU {T}x{I}x{O}", flush=True)
+    import quartet_amd as q
+    layer = q.QuantizedLinear(I, O, bias=False, device="cuda", dtype=torch.bfloat16, weight_quantizer=q.QuestMXFP4Quantizer(), activation_quantizer=q.QuestMXFP4Quantizer(),
+                              gradient_quantizer=q.AlbertTsengQuantizer(), backward_scheme=q.BACKWARD_SCHEMES["Q(E)Q(Wt)t_Q(Et)Q(Xt)t"]())
+    with torch.no_grad():
+        layer.weight.copy_(make_input(O, I, torch.bfloat16, 1, scale=0.02).cuda())
+        x = make_input(T, I, torch.bfloat16, 2).cuda()
+        for xt in (x, x.float()):
+            whole = layer(xt)
+            assert whole.dtype == xt.dtype and torch.isfinite(whole).all()
+            for at in range(0, T - 100, 100):
+                rows = slice(at, at + 100 if at + 200 <= T else T)
+                assert torch.equal(whole[rows], layer(xt[rows].contiguous()))
+
+
 # workgroups of two, three and four times 16 columns, of which the last one has one, none past the end, or a partial one; more than one to a CU; eight waves to K
 @pytest.mark.parametrize("T,I,O", [(16, 640, 4104), (16, 2048, 8192), (9, 1152, 8200), (16, 2048, 8216), (8, 4096, 11008), (5, 96, 12296), (16, 1024, 16408), (4, 8192, 4104), (1, 8320, 8232)])
 def test_decode_of_wide_layers(T, I, O):
