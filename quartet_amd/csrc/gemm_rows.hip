@@ -21,7 +21,7 @@ namespace qm {
 
 // With scales requested a step at a time, which touch as many cache lines as the codes do, and each request behind a condition (waits below), it
 // took, us MxNxK: 16x4096x4096 5.2 (now 3.9), 16x11008x4096 10.3 (6.4), 32x4096x4096 6.5 (4.4), 64x4096x4096 9.3 (5.3), 64x4096x11008 14.6 (8.9), 64x1536x8192
-// 15.7 (6.5); with the quantizer in it 1x11008x4096 8.2 (7.3), 8x4096x4096 6.7 (6.4).
+// 15.7 (6.5); with the quantizer in it 1x11008x4096 8.2 (7.3, in wider workgroups 6.7), 8x4096x4096 6.7 (6.4).
 namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
