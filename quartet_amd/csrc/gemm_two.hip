@@ -314,12 +314,14 @@ __device__ __forceinline__ void two_run(const uint8_t* __restrict__ a_codes, con
                     const auto r = __builtin_amdgcn_permlane32_swap(f2u(top), f2u(top), false, false);
                     top = fmaxf(u2f(r[0]), u2f(r[1]));
                 }
-                const float ref = top == -INFINITY ? 0.0f : top * kLog2e;   // nothing but -inf: every term is zero
+                // Differences first: they are exact where a term counts, however large the logits are, and the largest element's term is one.  (With the
+                // product top * log2 e, rounded, taken off in one fma, its rounding error is in every term: 3e-5 of a loss at logits of 1000, no finite one at 1e10.)
+                const float ref = top == -INFINITY ? 0.0f : top;   // nothing but -inf: every term is zero
                 float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int j = 0; j < kTwoTN; ++j)
 #pragma unroll
-                    for (int e = 0; e < 16; ++e) sum[e & 3] += __builtin_amdgcn_exp2f(__builtin_fmaf(acc[i][j][e], kLog2e, -ref));
+                    for (int e = 0; e < 16; ++e) sum[e & 3] += __builtin_amdgcn_exp2f((acc[i][j][e] - ref) * kLog2e);
                 float s = (sum[0] + sum[1]) + (sum[2] + sum[3]);
                 {
                     const auto r = __builtin_amdgcn_permlane32_swap(f2u(s), f2u(s), false, false);

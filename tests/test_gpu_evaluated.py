@@ -262,6 +262,32 @@ def test_logits_with_their_loss(T, K, V, add_dtype):
         assert torch.isnan(loss)
 
 
+@pytest.mark.parametrize("size", [20.0, 128.0, 1000.0, 1e5, 1e10, 1e38])
+@pytest.mark.parametrize("T,V", [(64, 200), (256, 384)])   # edges, and whole tiles
+def test_loss_of_large_logits(T, V, size):
+    """Row by row, and whether the target is a row's largest class or not, the loss of the stored logits: differences to a row's largest logit round to
+    2^-24 of themselves, as the terms and the sums do (1e-5 in all), however large the logits are.  Never negative beyond that."""
+    from quartet_amd import kernels as Kn
+    print(f"case large logits {T}x{V} {size}", flush=True)
+    K, g = 64, torch.Generator("cuda:0").manual_seed(V)
+    x, gain = torch.randn(T, K, generator=g, device="cuda:0"), torch.ones(K, device="cuda:0")
+    weight = torch.randn(V, K, generator=g, device="cuda:0")
+    weight[V // 2:] *= 0.999   # near ties, too
+    weight[V // 2:] += 1e-3 * weight[: V - V // 2]
+    top = (Kn.rmsnorm(x, gain, 1e-5, None, BF16).double() @ weight.to(BF16).double().T).abs().max()
+    weight = (weight * (size / float(top))).contiguous()
+    one = torch.full((T,), -1, dtype=torch.int64, device="cuda:0")
+    logits, _ = Kn.logits_loss(x, gain, 1e-5, None, weight, one, -1)
+    assert torch.isfinite(logits).all() and logits.double().abs().max() > 0.9 * size
+    for row in (0, 1, 17, T - 1):
+        for target in (int(logits[row].argmax()), int(logits[row].argmin()), 5):
+            one.fill_(-1)
+            one[row] = target
+            again, loss = Kn.logits_loss(x, gain, 1e-5, None, weight, one, -1)
+            want = float(torch.nn.functional.cross_entropy(logits[row:row + 1].double(), one[row:row + 1]))
+            assert torch.equal(again, logits) and abs(float(loss) - want) <= 1e-5 * max(1.0, abs(want)), (row, target, float(loss), want)
+
+
 def test_logits_with_values_that_are_not_finite():
     """A row with an infinite or NaN logit, a row whose logits are all -inf, a target that is no class: the library's answer (NaN where it asserts)."""
     from quartet_amd.fused import logits_and_loss
