@@ -197,10 +197,18 @@ def rmsnorm(norm, layer, x, add=None):
     return norm(x if add is None else x + add)
 
 
-# Contractions that logits_and_loss() takes: the library's product of a longer one is faster by more than the loss's own pass over the logits costs.
-# 32000 classes, us with the weight's conversion and the loss, in one pass and apart: 4096 tokens of 640 189 and 225, of 1536 392 and 404, of 2048 500 and
-# 503, of 3072 737 and 732; 1024 tokens of 640 75 and 84, of 1536 148 and 158, of 2048 216 and 199; 64 of 640 45 either way.
-_MAX_LOGITS_K = 1536
+def _one_pass(T, K, V):
+    """Whether logits_and_loss() makes the logits of T tokens x K x V classes and their loss in one pass, which saves the loss's own pass over the logits and
+    24 us of a call's host time (44 instead of 68; 36 where the library rounds the weight, too) but rounds the whole weight to bf16 on every call; the library does
+    that once per autocast region.  Longer contractions the library multiplies faster by more than the pass costs.
+
+    A weight that takes no longer to round than that (3 * 2^23 elements, 20 us): any number of tokens.  us a pass of an evaluated model of six layers, 32000
+    classes, in one pass and apart, batch after batch in one region: 640 wide 64 tokens 657 and 711, 1024 604 and 666, 2048 623 and 677, 4096 791 and 818; 768 wide 64 tokens 640 and
+    703, 1024 594 and 654, 4096 873 and 865, 8192 1473 and 1512; but 1536 wide 1024 tokens 782 and 725, 4096 1807 and 1766.  A region for each batch: 768 wide 4096 tokens 879 and 914, 1536
+    wide 791 and 786.  (Replayed from a graph, where host time is nothing, 64 tokens of 640 take 300 and 293, 512 475 and 480, 4096 793 and 838.)
+    Larger weights, up to 2^26 elements: enough tokens for the pass to cost more than the rounding.  us on the GPU, the library's weight rounded before: 1024 tokens x 384 x
+    128000 198 and 190, 2048 320 and 385; 2048 x 640 x 64000 220 and 214, 4096 378 and 406; 4096 x 768 x 64000 438 and 446; past that 4096 x 640 x 128000 904 and 822, 8192 1680 and 1663."""
+    return K <= 768 and V * K <= 1 << 26 and (V * K <= 3 << 23 or T >= 6 * K)
 
 
 def logits_and_loss(norm, layer, x, add, targets, ignore_index=-1):
@@ -208,8 +216,8 @@ def logits_and_loss(norm, layer, x, add, targets, ignore_index=-1):
     under bf16 autocast with the loss's sums of exponentials worked out beside the logits."""
     weight = layer.weight if type(layer) is torch.nn.Linear and layer.bias is None else None
     if (type(weight) is torch.nn.Parameter and type(targets) is torch.Tensor and targets.dtype == torch.int64 and targets.shape == x.shape[:-1] and targets.is_contiguous()
-            and weight.dtype == torch.float32 and weight.device == x.device == targets.device and weight.dim() == 2 and weight.shape[1] == x.shape[-1] <= _MAX_LOGITS_K
-            and weight.is_contiguous() and weight.data_ptr() % 16 == 0 and not (torch.is_grad_enabled() and weight.requires_grad)):
+            and weight.dtype == torch.float32 and weight.device == x.device == targets.device and weight.dim() == 2 and weight.shape[1] == x.shape[-1]
+            and _one_pass(targets.numel(), weight.shape[1], weight.shape[0]) and weight.is_contiguous() and weight.data_ptr() % 16 == 0 and not (torch.is_grad_enabled() and weight.requires_grad)):
         rows = _plain_rows(norm, layer, x, add)
         if rows is not None:
             out = kernels.logits_loss(rows[0], norm.weight.contiguous(), norm.eps, rows[1], weight.detach(), targets.view(-1), ignore_index)

@@ -288,6 +288,22 @@ def test_loss_of_large_logits(T, V, size):
             assert torch.equal(again, logits) and abs(float(loss) - want) <= 1e-5 * max(1.0, abs(want)), (row, target, float(loss), want)
 
 
+@pytest.mark.parametrize("T,K,V,one_pass", [(1, 64, 8, True), (40, 768, 32768, True), (40, 768, 32776, False), (4607, 768, 32776, False), (4608, 768, 32776, True),
+                                            (1536, 256, 262144, True), (1536, 256, 262152, False), (40, 800, 256, False), (300, 1536, 400, False)])
+def test_which_logits_have_their_loss_in_the_same_pass(monkeypatch, T, K, V, one_pass):
+    """Large weights, which the library rounds once per autocast region, and long contractions are the library's: its logits, bit for bit."""
+    from quartet_amd import fused
+    print(f"case route logits {T}x{K}x{V}", flush=True)
+    calls, logits_loss = [], fused.kernels.logits_loss
+    monkeypatch.setattr(fused.kernels, "logits_loss", lambda *a: calls.append(a) or logits_loss(*a))
+    norm, head, x, add, targets = _head(T, K, V, BF16, V)
+    with torch.no_grad(), torch.autocast("cuda", dtype=BF16):
+        logits, loss = fused.logits_and_loss(norm, head, x, add, targets)
+        assert len(calls) == one_pass and torch.isfinite(loss)
+        if not one_pass:
+            assert torch.equal(logits, head(fused.rmsnorm(norm, head, x, add)))
+
+
 def test_logits_with_values_that_are_not_finite():
     """A row with an infinite or NaN logit, a row whose logits are all -inf, a target that is no class: the library's answer (NaN where it asserts)."""
     from quartet_amd.fused import logits_and_loss
