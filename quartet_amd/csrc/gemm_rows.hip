@@ -16,6 +16,7 @@
 
 #include "gemm_common.h"
 #include "quantize_group.h"
+#include "scale_requests.h"
 
 namespace qm {
 
@@ -89,7 +90,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_mxfp4_tn_rows_kernel(const ui
     };
     // Steps s .. s + depth - 1 of this wave; past its end sixteen bytes of the last one for all lanes, which cost one request and are not multiplied.
     // Their scales in one request, which at a row's end begins up to three steps earlier (multiply_last): in rows of fewer steps in front of the
-    // row, which in a packed operand's first row is among its codes.
+    // row, which in a packed operand's first row is among its codes (scale_requests.h; what is not packed so does not come here).
     const auto request = [&](Steps& f, int s) {
         const int from = 4 * (s + kRowsDepth <= nk ? s : nk - kRowsDepth);
 #pragma unroll
@@ -297,7 +298,8 @@ RowsTile rows_tile(const TileProduct& p) {
 // 8.7 -> 9.1, 64x11008x4096 8.3 -> 9.4.
 bool gemm_rows_serves(const TileProduct& p) {
     const bool kind = p.M > 0 && p.M <= 64 && p.N >= 8 && p.N % 8 == 0 && p.K > 0 && p.K % kBK == 0 && p.a_tiled && p.b_tiled && !p.mask &&
-                      !p.b_e5m2 && (reinterpret_cast<uintptr_t>(p.c) & 15) == 0;
+                      !p.b_e5m2 && (reinterpret_cast<uintptr_t>(p.c) & 15) == 0 && scale_requests_in_operand(p.a_codes, p.a_scales, p.M, p.K) &&
+                      scale_requests_in_operand(p.b_codes, p.b_scales, p.N, p.K);
     const int64_t tiles = ((int64_t)p.N + 63) / 64;
     return kind && (p.M <= 16 || (p.M <= 32 ? p.K <= 2048 || 4 * tiles <= 3 * device_cus() : 2 * tiles <= device_cus()));
 }
@@ -336,7 +338,7 @@ bool linear_decode_serves(int64_t T, int64_t I, int64_t O) {
 
 hipError_t linear_decode(const void* x, int x_dtype, int64_t T, int64_t I, int64_t O, uint32_t sign_word, const uint8_t* w_codes,
                          const uint8_t* w_scales, void* y, int y_dtype, hipStream_t stream) {
-    if (!linear_decode_serves(T, I, O)) return hipErrorInvalidValue;
+    if (!linear_decode_serves(T, I, O) || !scale_requests_in_operand(w_codes, w_scales, O, padded_cols(I))) return hipErrorInvalidValue;
     const int K = (int)padded_cols(I), columns = decode_columns(O, K);
     const unsigned lds = (unsigned)(T * (K / 32) * 17);
     const float c = hadamard_scale(32, x_dtype);

@@ -255,13 +255,14 @@ hipError_t bf16_blocks(const float* w, int64_t V, int64_t K, void* out, hipStrea
 hipError_t logits_loss_rows(const void* parts, int64_t segments, int64_t T, const void* logits, int64_t V, const int64_t* targets, int64_t ignore, float* losses,
                             hipStream_t stream);
 
-// The product of at most 64 rows with a weight, both tiled (gemm_rows.hip): K % 128 == 0, N % 8 == 0, c 16-byte aligned, no mask.
+// The product of at most 64 rows with a weight, both tiled (gemm_rows.hip): K % 128 == 0, N % 8 == 0, c 16-byte aligned, no mask, scales 4-byte aligned and,
+// for K < 512, behind their codes as in a packed operand (scale_requests.h).
 // Its sums are in another order than the other kernels'.
 bool gemm_rows_serves(const TileProduct& p);
 hipError_t gemm_rows(const TileProduct& p, int c_dtype, hipStream_t stream);
 
 // The forward pass of a layer for a decoded batch in one launch (gemm_rows.hip): quest RTN of x under Hadamard blocks of 32, times
-// the packed weight (padded tiled codes); x 16-byte, y 8-byte aligned
+// the packed weight (padded tiled codes, the scales behind them as above); x 16-byte, y 8-byte aligned
 bool linear_decode_serves(int64_t T, int64_t I, int64_t O);
 hipError_t linear_decode(const void* x, int x_dtype, int64_t T, int64_t I, int64_t O, uint32_t sign_word, const uint8_t* w_codes,
                          const uint8_t* w_scales, void* y, int y_dtype, hipStream_t stream);

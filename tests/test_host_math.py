@@ -40,3 +40,12 @@ def test_remembered_shapes_on_the_host(tmp_path):
                     os.path.join(ROOT, "tests", "shape_table_check.cpp"), "-o", str(exe)], check=True)
     run = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
     assert run.returncode == 0 and run.stdout.strip().endswith("ok"), run.stdout[-2000:]
+
+
+def test_scale_requests_stay_in_their_operand(tmp_path):
+    """Requests for four K steps of a row's scales, in rows of fewer than four steps and of more, of scales behind their codes and elsewhere."""
+    exe = tmp_path / "scale_requests_check"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", "-Werror", "-I", os.path.join(ROOT, "quartet_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "scale_requests_check.cpp"), "-o", str(exe)], check=True)
+    run = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert run.returncode == 0, run.stdout[-2000:]
