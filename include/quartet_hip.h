@@ -445,7 +445,7 @@ int qm_rmsnorm(const float* x, const void* add, int add_dtype, const float* gain
  * bf16; logits [T, V] bf16 = h w^T with the fp32 weight w [V, K] rounded to bf16, fp32 sums; *loss as qm_cross_entropy of those logits, whose
  * sums of exponentials the product works out beside them.
  *   workspace   DEVICE scratch of qm_logits_loss_workspace_bytes(T, K, V) bytes (0: not served), 256-byte aligned
- * K a multiple of 32 in [64, 4096], V a multiple of 8; 16-byte aligned tensors.
+ * K a multiple of 32 in [64, 4096], V a multiple of 8; T and V below 2^24, T V below 2^38, V K below 2^35 - 2^17; 16-byte aligned tensors.
  */
 size_t qm_logits_loss_workspace_bytes(int64_t T, int64_t K, int64_t V);
 int qm_logits_loss(const float* x, const void* add, int add_dtype, const float* gain, float eps, int64_t T, int64_t K, const float* w, int64_t V,

@@ -375,7 +375,8 @@ hipError_t gemm_two(const TileProduct& p, hipStream_t stream) {
 
 // x [T, K], w [V, K] in blocks of 16 rows and 32 elements (see above), whole blocks of rows; logits 16-byte aligned
 bool gemm_logits_serves(int64_t T, int64_t V, int64_t K) {
-    return T > 0 && V >= 8 && V % 8 == 0 && K % 32 == 0 && K >= 64 && K <= 8192 && T < (1 << 24) && V < (1 << 24) && T * V < (1ll << 38);
+    return T > 0 && V >= 8 && V % 8 == 0 && K % 32 == 0 && K >= 64 && K <= 8192 && T < (1 << 24) && V < (1 << 24) && T * V < (1ll << 38) &&
+           padded_rows(V) * K < (1ll << 35) - 2048;   // bf16_blocks' grid has an eighth as many threads, in whole workgroups, and fewer than 2^32
 }
 int64_t gemm_logits_segments(int64_t V) { return 2 * ((V + kTwoN - 1) / kTwoN); }
 hipError_t gemm_logits(const void* x, const void* w, int64_t T, int64_t V, int64_t K, void* logits, void* parts, hipStream_t stream) {

@@ -50,6 +50,14 @@ def test_host_only_entry_points():
     assert L.qm_gemm_workspace_bytes(256, 256, 100) == 0                # K not a multiple of 32
 
 
+def test_extents_of_the_logits_with_their_loss():
+    """Every launch behind qm_logits_loss has fewer than 2^32 threads; the one that rounds the weight has an eighth of its elements."""
+    serves = lambda T, K, V: _lib.lib().qm_logits_loss_workspace_bytes(T, K, V) > 0
+    assert serves(1, 4096, (1 << 23) - 16) and not serves(1, 4096, 1 << 23) and not serves(1, 4096, (1 << 23) - 8)
+    assert serves(1, 2048, (1 << 24) - 16) and not serves(1, 2048, (1 << 24) - 8) and serves(1, 2016, (1 << 24) - 8) and not serves(1, 64, 1 << 24)
+    assert not any(serves(*s) for s in ((0, 64, 8), (1, 64, 0), (1, 64, 12), (1, 32, 8), (1, 72, 8), (1, 4128, 8), (1 << 24, 64, 8), (1 << 20, 64, 1 << 18)))
+
+
 @pytest.mark.parametrize("call,needle", [
     (lambda L: L.qm_quantize_mxfp4(None, 0, 4, 30, 32, None, 0, 0, None, 0, None, None, None, None, 0, None), b"multiple of hadamard_dim"),
     (lambda L: L.qm_quantize_mxfp4(None, 5, 4, 32, 32, None, 0, 0, None, 0, None, None, None, None, 0, None), b"x_dtype"),
