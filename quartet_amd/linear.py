@@ -155,9 +155,9 @@ class QuantizedLinear(nn.Linear):
     """nn.Linear whose forward is scheme(act_q(x), weight_q(W)); the bias parameter, if requested,
     is never applied -- exactly as in the reference (the scheme calls F.linear(x, w, None)).
 
-    A call's results can depend on how many tokens it has: on the packed path the product of at most 16 tokens, and of 17
-    to 64 where out_features <= 16 per compute unit (4096) or, up to 32, in_features <= 2048, adds its terms in another
-    order than that of more tokens.  FP4 codes times powers of two add up exactly in fp32 in any order as long as the
+    A call's results can depend on how many tokens it has: on the packed path the product of at most 16 tokens, of 17 to 32
+    where out_features <= 48 per compute unit (12288) or in_features <= 2048, and of 33 to 64 where out_features <= 32 per
+    compute unit (8192), adds its terms in another order than that of more tokens.  FP4 codes times powers of two add up exactly in fp32 in any order as long as the
     group scales of a row span few octaves -- no result differed for normal, heavy-tailed and outlier-ridden activations --
     but with columns whose scales span 2^16 about one bf16 value in 3 * 10^4 rounds differently than the same row's in a
     larger batch, and behind a further quantizer such a difference can become another FP4 code.  Calls of one token count
