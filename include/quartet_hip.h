@@ -451,6 +451,10 @@ size_t qm_logits_loss_workspace_bytes(int64_t T, int64_t K, int64_t V);
 int qm_logits_loss(const float* x, const void* add, int add_dtype, const float* gain, float eps, int64_t T, int64_t K, const float* w, int64_t V,
                    const int64_t* targets, int64_t ignore_index, void* workspace, size_t workspace_bytes, void* logits, float* loss, void* stream);
 
+/* Test aid: the kernel that qm_linear_forward's product of operands in QM_LAYOUT_PADDED runs on.  1: that of few rows, 2: persistent, 3: 256 x 192 tiles, 16 to 20: tiles of
+ * 256 x 128, 128 x 128, 128 x 64, 64 x 64, 64 x 32, 32: 128 x 128 with a fourth stage; 0: none of these */
+int qm_diag_forward_kernel(int64_t T, int64_t I, int64_t O, int y_dtype);
+
 /* Test aid: silu as the SwiGLU producer evaluates it for bf16 tensors, of every bf16 bit pattern: out[65536] */
 int qm_diag_silu_bf16(uint16_t* out, void* stream);
 

@@ -62,6 +62,7 @@ EXPORTS = (
     "qm_cross_entropy",
     "qm_logits_loss_workspace_bytes",
     "qm_logits_loss",
+    "qm_diag_forward_kernel",
     "qm_diag_silu_bf16",
 )
 
@@ -139,6 +140,8 @@ def lib():
     L.qm_swiglu_backward.argtypes = [vp, i32, vp, i32, i64, i64, vp, vp, i32, vp, vp]
     L.qm_rope_split_qkv.restype = i32
     L.qm_rope_split_qkv.argtypes = [vp, i32, i64, i64, i64, i32, vp, vp, vp, vp, i32, vp]
+    L.qm_diag_forward_kernel.restype = i32
+    L.qm_diag_forward_kernel.argtypes = [i64, i64, i64, i32]
     L.qm_diag_silu_bf16.restype = i32
     L.qm_diag_silu_bf16.argtypes = [vp, vp]
     L.qm_linear_decode_serves.restype = i32

@@ -1168,6 +1168,17 @@ int qm_logits_loss(const float* x, const void* add, int add_dtype, const float* 
     return from_hip(e, "qm_logits_loss");
 }
 
+int qm_diag_forward_kernel(int64_t T, int64_t I, int64_t O, int y_dtype) {
+    if (T <= 0 || I <= 0 || O <= 0 || I % 32 || O % 8 || T >= (1 << 30) || I >= (1 << 23) || O >= (1 << 30) || !valid_dtype(y_dtype)) return 0;
+    const PackedLayout lx = packed_layout(T, I), lw = packed_layout(O, I);
+    const uint8_t *px = reinterpret_cast<const uint8_t*>((uintptr_t)256), *pw = px + lx.total;   // nothing is read
+    const qm::TileProduct p = qm::make_product(px + lx.c, px + lx.s, pw + lw.c, pw + lw.s, T, O, qm::padded_cols(I), 1.0f, const_cast<uint8_t*>(px), QM_LAYOUT_TILED, QM_LAYOUT_TILED);
+    if (T <= 64 && qm::gemm_rows_serves(p)) return 1;
+    const qm::ProductChoice c = qm::choose_product(p, y_dtype, y_dtype, nullptr, 0);
+    if (c.path == qm::ProductChoice::TILE) return c.kind == qm::TILE_128x128 && qm::gemm_tile_deep(p) ? 32 : 16 + c.kind;
+    return c.path == qm::ProductChoice::PERSISTENT ? 2 : c.path == qm::ProductChoice::TWO ? 3 : 0;
+}
+
 int qm_diag_silu_bf16(uint16_t* out, void* stream) {
     if (!out) return fail(QM_ERR_INVALID, "qm_diag_silu_bf16: out must be non-null");
     return from_hip(qm::silu_of_bf16_table(out, reinterpret_cast<hipStream_t>(stream)), "qm_diag_silu_bf16");

@@ -993,10 +993,18 @@ hipError_t gemm_tile_rope(const TileProduct& g, const TileAfter& after, hipStrea
     return g.K / kBK >= 4 ? launch_after<Tile128x128, END_ROPE>(g, after, stream) : launch_after<Tile128x128::Narrow, END_ROPE>(g, after, stream);
 }
 
+namespace {
+// blocks of scales: every K range has at least four steps, all whole, and scale rows start at multiples of four bytes
+bool scales_in_blocks(const TileProduct& g) {
+    return g.K % kBK == 0 && g.K / kBK / g.splits >= 4 && ((reinterpret_cast<uintptr_t>(g.a_scales) | reinterpret_cast<uintptr_t>(g.b_scales)) & 3) == 0;
+}
+}  // namespace
+bool gemm_tile_deep(const TileProduct& g) {
+    return !g.b_e5m2 && !g.mask && scales_in_blocks(g) && (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) * g.splits <= device_cus();
+}
+
 hipError_t gemm_tile(int shape, const TileProduct& g, int c_dtype, hipStream_t stream) {
-    // blocks of scales: every K range has at least four steps, all whole, and scale rows start at multiples of four bytes
-    const bool blocks = g.K % kBK == 0 && g.K / kBK / g.splits >= 4 &&
-                        ((reinterpret_cast<uintptr_t>(g.a_scales) | reinterpret_cast<uintptr_t>(g.b_scales)) & 3) == 0;
+    const bool blocks = scales_in_blocks(g);
     const auto run_plain = [&](auto s) {
         using S = decltype(s);
         return c_dtype == BF16 ? launch_tiles<S, uint16_t>(g, stream) : launch_tiles<S, float>(g, stream);
@@ -1024,7 +1032,7 @@ hipError_t gemm_tile(int shape, const TileProduct& g, int c_dtype, hipStream_t s
     }
     switch (shape) {
         case TILE_256x128: return go(Tile256x128{});
-        case TILE_128x128: return blocks && !g.mask && (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) * g.splits <= device_cus() ? run_plain(Deep128x128{}) : go(Tile128x128{});
+        case TILE_128x128: return gemm_tile_deep(g) ? run_plain(Deep128x128{}) : go(Tile128x128{});
         case TILE_128x64: return go(Tile128x64{});
         case TILE_64x64: return go(Tile64x64{});
         default: return go(Tile64x32{});

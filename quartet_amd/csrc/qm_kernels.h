@@ -235,6 +235,7 @@ constexpr int kShortTallSteps = 8;   // see gemm_tile()
 enum TileKind : int { TILE_256x128 = 0, WIDE_256x256 = 0, TILE_128x128 = 1, TILE_128x64 = 2, TILE_64x64 = 3, TILE_64x32 = 4 };
 bool gemm_tile_serves(int64_t M, int64_t N, int64_t K, int a_tiled, int b_tiled, const void* c);
 hipError_t gemm_tile(int kind, const TileProduct& g, int c_dtype, hipStream_t stream);
+bool gemm_tile_deep(const TileProduct& g);   // TILE_128x128 with a fourth stage
 // two products (bf16 results, or with a mask and *_f32 widened ones) in one grid; TileKinds 128x128 and 64x64
 bool gemm_tile_pair_serves(const TileProduct& a, int kind_a, const TileProduct& b, int kind_b);
 hipError_t gemm_tile_pair(TileProduct a, int kind_a, bool a_f32, TileProduct b, int kind_b, bool b_f32, hipStream_t stream);

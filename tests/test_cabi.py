@@ -50,6 +50,13 @@ def test_host_only_entry_points():
     assert L.qm_gemm_workspace_bytes(256, 256, 100) == 0                # K not a multiple of 32
 
 
+def test_token_counts_whose_sums_are_in_another_order():
+    """Those that QuantizedLinear names for 256 compute units, which a host without a GPU assumes too."""
+    few = lambda T, I, O: _lib.lib().qm_diag_forward_kernel(T, I, O, _lib.QM_BF16) == 1
+    assert few(16, 11008, 65536) and few(17, 4096, 12288) and few(32, 11008, 12288) and few(32, 2048, 65536) and few(33, 11008, 8192) and few(64, 4096, 8192)
+    assert not any((few(17, 4096, 12296), few(32, 2176, 12352), few(33, 2048, 8256), few(64, 4096, 8200), few(65, 512, 512)))
+
+
 def test_extents_of_the_logits_with_their_loss():
     """Every launch behind qm_logits_loss has fewer than 2^32 threads; the one that rounds the weight has an eighth of its elements."""
     serves = lambda T, K, V: _lib.lib().qm_logits_loss_workspace_bytes(T, K, V) > 0

@@ -148,6 +148,9 @@ def test_products_on_one_large_tile_to_a_cu(T, I, O):
     """A frozen layer's output, whole and by 100 rows (smaller tiles, the same order of additions), in bf16 and in fp32: the same bits."""
     print(f"case one tile to a CU {T}x{I}x{O}", flush=True)
     import quartet_amd as q
+    from quartet_amd import _lib
+    kernel = lambda rows, dtype: _lib.lib().qm_diag_forward_kernel(rows, I, O, dtype)
+    assert kernel(T, _lib.QM_BF16) == kernel(T, _lib.QM_F32) == 32 and kernel(100, _lib.QM_BF16) != 32 and kernel(100, _lib.QM_F32) != 32
     layer = q.QuantizedLinear(I, O, bias=False, device="cuda", dtype=torch.bfloat16, weight_quantizer=q.QuestMXFP4Quantizer(), activation_quantizer=q.QuestMXFP4Quantizer(),
                               gradient_quantizer=q.AlbertTsengQuantizer(), backward_scheme=q.BACKWARD_SCHEMES["Q(E)Q(Wt)t_Q(Et)Q(Xt)t"]())
     with torch.no_grad():

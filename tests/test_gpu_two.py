@@ -18,6 +18,9 @@ def test_products_on_two_workgroups_to_a_cu(T, I, O):
     """A frozen layer's output, whole and by 500 rows (another kernel, the same order of additions): the same bits."""
     print(f"case two {T}x{I}x{O}", flush=True)
     import quartet_amd as q
+    from quartet_amd import _lib
+    kernel = lambda rows: _lib.lib().qm_diag_forward_kernel(rows, I, O, _lib.QM_BF16)
+    assert kernel(T) == 3 and kernel(500) != 3
     layer = q.QuantizedLinear(I, O, bias=False, device="cuda", dtype=torch.bfloat16, weight_quantizer=q.QuestMXFP4Quantizer(),
                               activation_quantizer=q.QuestMXFP4Quantizer(), gradient_quantizer=q.AlbertTsengQuantizer(stochastic=True),
                               backward_scheme=q.BACKWARD_SCHEMES["Q(E)Q(Wt)t_Q(Et)Q(Xt)t"]())
@@ -40,6 +43,7 @@ def test_two_workgroups_against_the_product_in_float64():
     from quartet_amd import kernels as K
     g = torch.Generator().manual_seed(5)
     M, N, Kd = 8192, 4608, 1536
+    assert K._lib.lib().qm_diag_forward_kernel(M, Kd, N, K._lib.QM_BF16) == 3
     mk = lambda r: (torch.randint(0, 256, (r, Kd // 2), generator=g, dtype=torch.uint8).cuda(), torch.randint(124, 129, (r, Kd // 32), generator=g, dtype=torch.uint8).cuda())
     (ac, as_), (bc, bs) = mk(M), mk(N)
     got = K.gemm_mxfp4_tn(K.tile_codes(ac), as_, K.tile_codes(bc), bs, 1.5, a_tiled=True, b_tiled=True)
