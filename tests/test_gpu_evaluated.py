@@ -305,7 +305,7 @@ def test_which_logits_have_their_loss_in_the_same_pass(monkeypatch, T, K, V, one
 
 
 def test_logits_with_values_that_are_not_finite():
-    """A row with an infinite or NaN logit, a row whose logits are all -inf, a target that is no class: the library's answer (NaN where it asserts)."""
+    """A row with an infinite and NaN logits, a target that is no class: the library's answer (NaN where it asserts)."""
     from quartet_amd.fused import logits_and_loss
     norm, head, x, _, targets = _head(300, 64, 400, None, 3)
     with torch.no_grad():
@@ -327,6 +327,58 @@ def test_logits_with_values_that_are_not_finite():
             head.weight[7, 1] = 0.0
             _, loss = logits_and_loss(norm, head, x, None, torch.full_like(targets, 400))
             assert torch.isnan(loss)
+
+
+@pytest.mark.parametrize("T,V", [(64, 200), (256, 384)])   # edges, and whole tiles
+def test_loss_of_rows_with_infinite_logits(T, V):
+    """Rows of nothing but -inf, with a segment of -inf beside finite logits, with one +inf and one -inf, and a finite one, each by itself: the library's loss of the
+    stored logits (NaN where it is NaN), within the 1e-5 of finite ones."""
+    from quartet_amd import kernels as Kn
+    print(f"case infinite logits {T}x{V}", flush=True)
+    K, inf = 64, float("inf")
+    x, gain, weight = torch.zeros(T, K, device="cuda:0"), torch.ones(K, device="cuda:0"), torch.zeros(V, K, device="cuda:0")
+    g = torch.Generator("cuda:0").manual_seed(V)
+    weight[:, :4] = torch.randn(V, 4, generator=g, device="cuda:0")
+    x[:, 0] = 1.0
+    big = 3e38   # finite in bf16; times the normalised x of 8 it overflows the fp32 sum
+    weight[:, 4] = -big            # column 4: every class to -inf
+    part = torch.arange(V, device="cuda:0") % 192 // 32
+    first = (part == 0) | (part == 1) | (part == 4)   # the 96 columns of a tile that one wave has, whose sum is one part of the row's; the others
+    weight[first, 5] = -big        # column 5: every first part of a row
+    weight[~first, 6] = -big       # column 6: every second one
+    weight[7, 7], weight[9, 8] = big, -big
+    for row, column in ((1, 4), (2, 5), (3, 6), (4, 7), (5, 8)):
+        x[row, 0], x[row, column] = 0.0, 1.0
+    for row in (2, 3, 5):
+        x[row, 1] = 1.0
+    one = torch.full((T,), -1, dtype=torch.int64, device="cuda:0")
+    logits, _ = Kn.logits_loss(x, gain, 1e-5, None, weight, one, -1)
+    assert (logits[1] == -inf).all()
+    for row, gone in ((2, first), (3, ~first)):
+        assert (logits[row, gone] == -inf).all() and torch.isfinite(logits[row, ~gone]).all()
+    assert logits[4, 7] == inf and logits[5, 9] == -inf and torch.isfinite(logits[6]).all() and not torch.isnan(logits).any()
+    for row in range(1, 7):
+        for target in (0, 7, 9, 100, V - 1):
+            one.fill_(-1)
+            one[row] = target
+            _, loss = Kn.logits_loss(x, gain, 1e-5, None, weight, one, -1)
+            want = torch.nn.functional.cross_entropy(logits[row:row + 1].double(), one[row:row + 1]).float()
+            assert torch.allclose(loss, want, rtol=1e-5, atol=1e-5, equal_nan=True), (row, target, float(loss), float(want))
+
+
+@pytest.mark.parametrize("T,K,V", [(300, 1536, 4104), (130, 4096, 1000)])
+def test_longer_contractions_of_the_logits(T, K, V):
+    """What the entry point takes beyond what the model is sent there with, to the bounds of ``test_logits_with_their_loss``."""
+    from quartet_amd import kernels as Kn
+    print(f"case logits {T}x{K}x{V}", flush=True)
+    norm, head, x, add, targets = _head(T, K, V, BF16, K)
+    with torch.no_grad():
+        logits, loss = Kn.logits_loss(x, norm.weight, norm.eps, add, head.weight, targets, -1)
+        h, w = Kn.rmsnorm(x, norm.weight, norm.eps, add, BF16).double(), head.weight.to(BF16).double()
+    want = h @ w.T
+    assert ((logits.double() - want).abs() <= want.abs() * 2.0 ** -8 + K * 2.0 ** -24 * (h.abs() @ w.abs().T)).all()
+    ref = float(torch.nn.functional.cross_entropy(logits.double(), targets))
+    assert abs(float(loss) - ref) < 1e-5 * max(1.0, abs(ref))
 
 
 def test_logits_and_loss_take_the_modules_where_somebody_listens_or_asks_for_gradients():

@@ -39,6 +39,16 @@ def test_products_keep_nothing_in_memory(kernels):
     assert {n: v for n, v in {**tiles, **persistent}.items() if v[1]} == {}
 
 
+@pytest.mark.parametrize("name", ["gemm_mxfp4_tn_two_kernel<", "gemm_bf16_logits_kernel<", "gemm_mxfp4_tn_rows_kernel<", "linear_decode_kernel<", "gemm_mxfp4_tn_pair_kernel<",
+                                  "gemm_mxfp4_e5m2_pair_kernel<", "gemm_mxfp4_tn_after_kernel<"])
+def test_other_products_keep_nothing_in_memory(kernels, name):
+    """The first two are within ten of the registers that two workgroups to a CU leave a lane."""
+    found = {n: v for n, v in kernels.items() if name in n}
+    assert found and {n: v for n, v in found.items() if v[1]} == {}
+    if "two_kernel" in name or "logits" in name:
+        assert all(v[0] <= 256 for v in found.values()), found
+
+
 def test_a_rotation_in_the_epilogue_holds_no_registers_through_the_product(kernels):
     """The last template argument is the rotation.  Its lane constants belong to the epilogue: a few registers' difference, not 16."""
     tiles = {n: v[0] for n, v in kernels.items() if "tile_kernel<" in n}
@@ -58,8 +68,18 @@ def test_backward_quantizers_fit_their_waves_without_scratch(kernels):
         assert scratch == 0 and registers <= (96 if block == 32 else 128), (n, registers, scratch)
 
 
+def test_norm_producers_of_eight_elements_a_lane_have_no_scratch(kernels):
+    """The RMSNorm in front of a quantizer of rows of up to 2048 elements, 2^24 in all: latency is what bounds it, so waves are what it wants, eight to a SIMD."""
+    found = {n: v for n, v in kernels.items() if "RmsNormOctetsJob<" in n}
+    assert len(found) >= 3
+    for n, (registers, scratch) in found.items():
+        assert scratch == 0, (n, scratch)
+        if "RowmajorTiledJob" not in n:   # the weight's quantizer in the same grid has its own need
+            assert registers <= 64, (n, registers)
+
+
 def test_norm_producers_fit_four_waves_without_scratch(kernels):
-    """The RMSNorm in front of a quantizer, fp32 rows with a bf16 residual summand, as the model calls it."""
+    """The RMSNorm in front of a quantizer, fp32 rows with a bf16 residual summand, wider or more of them than eight elements a lane serve."""
     found = {n: v for n, v in kernels.items() if "RmsNormProducer<float, unsigned short>, true" in n}
     assert len(found) >= 6
     for n, (registers, scratch) in found.items():
