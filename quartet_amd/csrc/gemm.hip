@@ -973,6 +973,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 // Estimated durations in microseconds, fitted to 70 shapes of 0.2 to 740 GF with tiled operands: every kernel that serves the
 // shape and cuts into 2 to 4 K ranges, each launch between two 8192 x 4096 x 4096 products (alone and back to back the kernels run at
 // another clock and in another order of speed): mean error 6 %, and the choice costs 0.3 % more than the fastest on average.
+// The 128 x 128 line is that of three stages: with one tile to a CU the kernel has a fourth (gemm_tile.hip) and is up to a fifth faster than it says.
 // All kernels chosen from here give the same bits except a cut into K ranges, so nothing but time hangs on the choice.  (A
 // layer's forward product of at most 64 tokens may run on gemm_rows.hip instead, before this choice; its sums are in another
 // order.)

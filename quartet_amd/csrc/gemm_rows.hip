@@ -22,7 +22,7 @@ namespace qm {
 
 // With scales requested a step at a time, which touch as many cache lines as the codes do, and each request behind a condition (waits below), it
 // took, us MxNxK: 16x4096x4096 5.2 (now 3.9), 16x11008x4096 10.3 (6.4), 32x4096x4096 6.5 (4.4), 64x4096x4096 9.3 (5.3), 64x4096x11008 14.6 (8.9), 64x1536x8192
-// 15.7 (6.5); with the quantizer in it 1x11008x4096 8.2 (7.3, in wider workgroups 6.7), 8x4096x4096 6.7 (6.4).
+// 15.7 (6.5); with the quantizer in it 1x11008x4096 8.2 (7.3, in wider workgroups 6.7), 8x4096x4096 6.3 (6.1).
 namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -172,7 +172,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_mxfp4_tn_rows_kernel(const ui
 // and a layer call is one launch.  The codes lie in LDS as [K step][row][64 bytes], the scales as one byte per group; the
 // weight's first eight K steps are on their way meanwhile.  Up to sixteen waves quantize, a group to a lane where that is enough
 // for all; WAVES x TN of them multiply.  With WAVES alone, 8 x 4096 x 4096 took its 1024 groups four to a lane, one after the other, each
-// with its own wait for memory: 9.1 us, now 6.4.  Bit-identical to the two launches.
+// with its own wait for memory: 9.1 us, now 6.1 behind another one and 6.7 to 7 by itself.  Bit-identical to the two launches.
 // TN: 16 columns each, with waves of their own, so that what a wave holds and adds is the same for any TN.  Wide layers have as many as leave one
 // workgroup to a CU (decode_columns()): with 16 columns a workgroup their CUs quantize all of x two to four times over.
 constexpr int kDecodeThreads = 1024;
@@ -327,7 +327,7 @@ int decode_columns(int64_t O, int64_t K) {
 }
 
 // One launch instead of two while a CU's share of quantizing is no more than 1024 groups, one to a lane (about 3 us; the quantizer's own
-// launch takes 4): us in two launches and in one, 8x4096x4096 6.7 and 6.4 to 6.7, 8x11008x4096 9.8 and 8.1, 4x11008x4096 9.5 and 6.9, 16x11008x2048 8.1 and
+// launch takes 4): us in two launches and in one, 8x4096x4096 6.7 and 6.1 to 6.7, 8x11008x4096 9.8 and 8.1, 4x11008x4096 9.5 and 6.9, 16x11008x2048 8.1 and
 // 6.6, 1x4096x4096 6.7 and 4.7, 2x11008x11008 (1376 groups) 17.9 and 17.4; a call's host time, which bounds most of these, falls from 10.6 to 7.2
 bool linear_decode_serves(int64_t T, int64_t I, int64_t O) {
     if (!(T > 0 && T <= 16 && I > 0 && I % 32 == 0 && I < (1 << 20) && O >= 8 && O % 8 == 0 && O < (1 << 24))) return false;

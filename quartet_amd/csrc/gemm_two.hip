@@ -16,7 +16,9 @@
 // The same with bf16 operands makes the logits of an evaluated model, whose workgroups also take the exponentials for their loss while the other one
 // of the CU multiplies: no pass of its own over logits that are larger than the caches.  Bound by the matrix instructions at the power limit and the last,
 // partial round of tiles: 4096 x 32000 x 640 166 us (153 without the exponentials; the library's product 158 and the loss's pass 49), and from 1536
-// on by its two slots (4096 x 32000 x 1536 339; the library's product 300).  An evaluated 30 M model of 8 x 512 tokens 884 -> 847 us.
+// on by its two slots (4096 x 32000 x 1536 339; the library's product 300), which the model leaves to the library, as it does weights that cost more to round
+// than that pass (fused.py).  An evaluated 30 M model of 8 x 512 tokens 884 -> 847 us when it came; exponentials of differences, for the loss of large
+// logits, take 3 us of that back.
 // Row-major operands, 64 bytes of a row at a time, took 176 and 380.
 //
 // The order of additions over K is that of gemm.hip and gemm_tile.hip: the same bits.
